@@ -274,4 +274,28 @@ __device__ __forceinline__ float eps_of(const Rules& R, const float* __restrict_
   return tab[i];
 }
 
+// How a launch tells the host that it is through: the last workgroup stores `seq` into
+// pinned host memory that the host looks at.  flag null: nobody is waiting.
+struct HostSignal {
+  unsigned* flag;   // host memory
+  unsigned seq;
+  unsigned* count;  // device memory, zero between launches
+};
+
+// Last thing in the kernel, reached by all threads of all workgroups.  What a thread
+// stored before it is in host memory before the flag is.
+__device__ __forceinline__ void signal_host(const HostSignal h) {
+  if (!h.flag) return;
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    bool last = true;
+    if (gridDim.x > 1) {
+      last = atomicAdd(h.count, 1u) == gridDim.x - 1;
+      if (last) __hip_atomic_store(h.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (last) __hip_atomic_store(h.flag, h.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 }  // namespace crl

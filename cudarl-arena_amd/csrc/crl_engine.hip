@@ -6,6 +6,8 @@
 #include <cstdarg>
 #include <cstdio>
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cstdlib>
 #include <cstring>
 #include <exception>
@@ -19,6 +21,7 @@
 #include "crl_host.h"
 #include "crl_kernels.h"
 #include "crl_persist.h"
+#include "crl_pinned.h"
 
 namespace {
 
@@ -58,19 +61,28 @@ template <class T>
 struct DevBuf {
   T* p = nullptr;
   size_t n = 0;
+  bool owned = false;
   hipError_t alloc(size_t count) {
     release();
     if (count == 0) return hipSuccess;
     hipError_t e = hipMalloc(reinterpret_cast<void**>(&p), count * sizeof(T));
     if (e == hipSuccess) n = count;
     else p = nullptr;
+    owned = p != nullptr;
     return e;
   }
   hipError_t ensure(size_t count) { return count <= n ? hipSuccess : alloc(count); }
+  // a piece of somebody else's allocation
+  void adopt(void* at, size_t count) {
+    release();
+    p = static_cast<T*>(at);
+    n = count;
+  }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p && owned) (void)hipFree(p);
     p = nullptr;
     n = 0;
+    owned = false;
   }
   ~DevBuf() { release(); }
   DevBuf() = default;
@@ -113,7 +125,14 @@ int scratch_of_device(int device, unsigned char** out) {
 
 }  // namespace
 
+// Keeps the pool of pinned blocks alive; the engine's first member, so the last one to go.
+struct PoolUser {
+  PoolUser() { crl::PinnedPool::get().add_user(); }
+  ~PoolUser() { crl::PinnedPool::get().drop_user(); }
+};
+
 struct crl_engine {
+  PoolUser pool_user;
   crl_config cfg{};
   int device = 0;
   hipStream_t stream = nullptr;
@@ -146,6 +165,33 @@ struct crl_engine {
   bool persist_refused = false;  // the device refused the co-resident launch once: not tried again
   bool persist_clocks = false;   // run the instantiation that keeps phase clocks
   int persist_spin_limit = crl::kPersistSpinLimit;  // polls a thread waits for its peers before it gives up
+
+  // One allocation holds every array below that crl_create() makes, in the order it lists
+  // them: what is read out together lies together (state_at: s, ep_step, episode, reward,
+  // done, action; stats_at: the four statistics) and goes out in one piece.
+  DevBuf<unsigned char> arena;
+  unsigned char* state_at = nullptr;
+  size_t state_bytes = 0;
+  unsigned char* stats_at = nullptr;
+  size_t stats_bytes = 0;
+
+  // Pinned memory this engine and its kernels talk through.
+  crl::PinBuf flag_page;        // word 0: number of the last signalled launch that is through; word 16: give-up word
+  DevBuf<unsigned> flag_count;  // workgroups of a signalling launch that are through
+  unsigned seq = 0;             // number of the last signalled launch
+  crl::PinBuf out_page;         // what kernels hand to the host: state, statistics, actions, tables
+  struct InSlot {
+    crl::PinBuf page;
+    unsigned last_seq = 0;  // the launch that reads it
+  };
+  static constexpr int kInSlots = 4;
+  InSlot in_slot[kInSlots];     // what the host hands to kernels, taken in turn
+  int in_next = 0;
+  bool state_shared = false;    // device pointers to the state are out: it may change between calls
+  bool mirror_steps = false;    // crl_step's kernel also writes the state to out_page ...
+  bool mirror_read = false;     // ... because the state was read after the step before
+  bool stepped = false;         // crl_step was the last call that changed the state
+  unsigned mirror_seq = 0;      // != 0: out_page holds the state as of this launch
 
   DevBuf<int32_t> s, ep_step, episode, start, act;
   DevBuf<float> reward;
@@ -782,6 +828,106 @@ int run_persist(crl_engine* e, int n_steps, bool* launched) {
   return CRL_OK;
 }
 
+// ---- pinned memory between host and kernels --------------------------------------------
+
+constexpr size_t kLinkLimitBytes = (size_t)4 << 20;  // larger transfers: hipMemcpyAsync straight to and from the caller's memory
+constexpr int kFlagErrWord = 16;                     // of flag_page; in another 64-byte line than the flag
+
+// the next launch that tells the host when it is through
+crl::HostSignal next_signal(crl_engine* e) {
+  if (++e->seq == 0) ++e->seq;
+  crl::HostSignal sig;
+  sig.flag = reinterpret_cast<unsigned*>(e->flag_page.p);
+  sig.seq = e->seq;
+  sig.count = e->flag_count.p;
+  return sig;
+}
+
+bool seq_passed(const crl_engine* e, unsigned seq) {
+  const volatile unsigned* flag = reinterpret_cast<const volatile unsigned*>(e->flag_page.p);
+  return (int)(*flag - seq) >= 0;
+}
+
+// Waits until launch `seq` is through: looks at the flag for a while (a small call is over
+// in microseconds), then leaves the waiting, and finding out about errors, to the runtime.
+int wait_seq(crl_engine* e, unsigned seq) {
+  if (!seq_passed(e, seq)) {
+    const auto give_up = std::chrono::steady_clock::now() + std::chrono::microseconds(300);
+    bool passed = false;
+    do {
+      for (int i = 0; i < 64 && !passed; ++i) {
+        passed = seq_passed(e, seq);
+        if (!passed) __builtin_ia32_pause();
+      }
+    } while (!passed && std::chrono::steady_clock::now() < give_up);
+    if (!passed) {
+      HIP_TRY(hipStreamSynchronize(e->stream));
+      if (!seq_passed(e, seq)) return fail(CRL_E_DEVICE, "a launch ended without telling the host so");
+    }
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  return CRL_OK;
+}
+
+// out_page with room for `bytes`; what it held is no longer there
+int claim_out_page(crl_engine* e, size_t bytes) {
+  e->mirror_seq = 0;
+  if (bytes <= e->out_page.n) return CRL_OK;
+  HIP_TRY(hipStreamSynchronize(e->stream));  // nobody may still be writing to the smaller one
+  if (!e->out_page.ensure(bytes)) return fail(CRL_E_ALLOC, "pinned host memory: %zu bytes", bytes);
+  return CRL_OK;
+}
+
+// a page for `bytes` that no earlier launch still reads
+int claim_in_slot(crl_engine* e, size_t bytes, crl_engine::InSlot** out) {
+  crl_engine::InSlot& slot = e->in_slot[e->in_next];
+  e->in_next = (e->in_next + 1) % crl_engine::kInSlots;
+  if (slot.last_seq != 0) {
+    const int rc = wait_seq(e, slot.last_seq);
+    if (rc) return rc;
+    slot.last_seq = 0;
+  }
+  if (!slot.page.ensure(bytes)) return fail(CRL_E_ALLOC, "pinned host memory: %zu bytes", bytes);
+  *out = &slot;
+  return CRL_OK;
+}
+
+int persist_result(crl_engine* e, unsigned gave_up);
+
+// `bytes` of device memory (a multiple of 16, as all arrays of the arena are padded to) in
+// out_page once this returns
+int fetch_pinned(crl_engine* e, const void* src, size_t bytes) {
+  int rc = claim_out_page(e, bytes);
+  if (rc) return rc;
+  const crl::HostSignal sig = next_signal(e);
+  const size_t n16 = (bytes + 15) / 16;
+  const int grid = (int)std::min<size_t>((n16 + 255) / 256, 256);
+  const bool check = e->persist_unchecked;
+  unsigned* flags = reinterpret_cast<unsigned*>(e->flag_page.p);
+  hipLaunchKernelGGL(crl::k_export, dim3(grid), dim3(n16 < 256 ? 64 : 256), 0, e->stream,
+                     static_cast<const uint4*>(src), reinterpret_cast<uint4*>(e->out_page.p), n16,
+                     check ? reinterpret_cast<const unsigned*>(e->pdiag.p) : nullptr, flags + kFlagErrWord, sig);
+  HIP_TRY(hipGetLastError());
+  rc = wait_seq(e, sig.seq);
+  if (rc) return rc;
+  if (!check) return CRL_OK;
+  e->persist_unchecked = false;
+  return persist_result(e, static_cast<volatile unsigned*>(flags)[kFlagErrWord]);
+}
+
+// out_page as the engine's state arrays are laid out
+crl::StateMirror state_mirror(const crl_engine* e) {
+  crl::StateMirror M{};
+  auto at = [&](const void* p) { return e->out_page.p + (static_cast<const unsigned char*>(p) - e->state_at); };
+  M.s = reinterpret_cast<int32_t*>(at(e->s.p));
+  M.ep_step = reinterpret_cast<int32_t*>(at(e->ep_step.p));
+  M.episode = reinterpret_cast<int32_t*>(at(e->episode.p));
+  M.reward = reinterpret_cast<float*>(at(e->reward.p));
+  M.done = at(e->done.p);
+  M.action = at(e->action.p);
+  return M;
+}
+
 // Did a one-launch kernel give up waiting for its peers?  Called by the entry points
 // that synchronise; reports a give-up once.  The give-up word stays set on the device
 // (the kernel's later launches see it and return at once), and until the caller has set
@@ -792,6 +938,10 @@ int check_persist(crl_engine* e) {
   unsigned gave_up = 0;
   HIP_TRY(hipMemcpyAsync(&gave_up, e->pdiag.p, sizeof gave_up, hipMemcpyDeviceToHost, e->stream));
   HIP_TRY(hipStreamSynchronize(e->stream));
+  return persist_result(e, gave_up);
+}
+
+int persist_result(crl_engine* e, unsigned gave_up) {
   if (!gave_up) return CRL_OK;
   e->persist_failed = true;
   return fail(CRL_E_DEVICE, "the one-launch shared-table kernel gave up waiting for its workgroups "
@@ -912,36 +1062,65 @@ int create_engine(const crl_config* cfg, int device, crl_engine** out) {
   auto acc = [&](hipError_t x) {
     if (a == hipSuccess) a = x;
   };
-  acc(e->s.alloc(N));
-  acc(e->ep_step.alloc(N));
-  acc(e->episode.alloc(N));
-  acc(e->start.alloc(N));
-  acc(e->act.alloc(N));
-  acc(e->reward.alloc(N));
-  acc(e->done.alloc(N));
-  acc(e->action.alloc(N));
-  acc(e->map.alloc((size_t)e->n_maps * e->map_words));
-  acc(e->moves.alloc((size_t)e->n_maps * e->mv_words));  // move codes of every map, for the fused loops
-  if (cells) acc(e->cell_reward.alloc((size_t)e->n_maps * e->S));
-  acc(e->Q.alloc((size_t)e->n_tables * e->K));
-  acc(e->eps_tab.alloc(eps.size()));
-  acc(e->tr_s.alloc(N));
-  acc(e->tr_a.alloc(N));
-  acc(e->tr_s2.alloc(N));
-  acc(e->tr_r.alloc(N));
-  acc(e->tr_done.alloc(N));
-  if (cfg->table_mode == CRL_TABLE_PER_ENV) acc(e->split.alloc(3));
-  if (cfg->table_mode == CRL_TABLE_SHARED) {
-    acc(e->key.alloc(N));
-    acc(e->delta.alloc(N));
-    acc(e->pdiag.alloc(1 + crl::kPersistClockWords));
-  }
-  if (cfg->track_returns) {
-    acc(e->ret_acc.alloc(N));
-    acc(e->ret_last.alloc(N));
-    acc(e->ret_sum.alloc(N));
-    acc(e->len_last.alloc(N));
-    acc(e->len_sum.alloc(N));
+  // One allocation and one clearing pass for everything (each hipMalloc and hipMemsetAsync
+  // on its own costs microseconds to tens of them, and there are two dozen arrays).
+  unsigned char* base = nullptr;
+  size_t used = 0;
+  auto carve = [&](auto& buf, size_t count) {
+    if (base) buf.adopt(base + used, count);
+    used += (count * sizeof(*buf.p) + 255) & ~(size_t)255;
+  };
+  size_t cleared = 0;  // what comes first is cleared
+  auto lay_out = [&]() {
+    used = 0;
+    carve(e->s, N);
+    carve(e->ep_step, N);
+    carve(e->episode, N);
+    carve(e->reward, N);
+    carve(e->done, N);
+    carve(e->action, N);
+    e->state_at = base;
+    e->state_bytes = used;
+    if (cfg->track_returns) {
+      e->stats_at = base + used;
+      const size_t from = used;
+      carve(e->ret_last, N);
+      carve(e->len_last, N);
+      carve(e->ret_sum, N);
+      carve(e->len_sum, N);
+      e->stats_bytes = used - from;
+      carve(e->ret_acc, N);
+    }
+    carve(e->start, N);
+    carve(e->act, N);
+    carve(e->flag_count, 1);
+    if (cfg->table_mode == CRL_TABLE_PER_ENV) {
+      carve(e->ticket, 3);
+      carve(e->split, 3);
+    } else {
+      carve(e->pdiag, 1 + crl::kPersistClockWords);
+    }
+    carve(e->map, (size_t)e->n_maps * e->map_words);
+    carve(e->Q, (size_t)e->n_tables * e->K);
+    cleared = used;
+    carve(e->moves, (size_t)e->n_maps * e->mv_words);  // move codes of every map, for the fused loops
+    if (cells) carve(e->cell_reward, (size_t)e->n_maps * e->S);
+    carve(e->eps_tab, eps.size());
+    carve(e->tr_s, N);
+    carve(e->tr_a, N);
+    carve(e->tr_s2, N);
+    carve(e->tr_r, N);
+    carve(e->tr_done, N);
+    if (cfg->table_mode == CRL_TABLE_SHARED) {
+      carve(e->key, N);
+      carve(e->delta, N);
+    }
+  };
+  lay_out();
+  acc(e->arena.alloc(used));
+  if (a == hipSuccess) {
+    base = e->arena.p;
+    lay_out();
   }
   if (a != hipSuccess) {
     const int code = a == hipErrorOutOfMemory ? CRL_E_ALLOC : CRL_E_DEVICE;
@@ -951,23 +1130,9 @@ int create_engine(const crl_config* cfg, int device, crl_engine** out) {
     return fail(CRL_E_DEVICE, "%s: %s", what, hipGetErrorString(x));
   };
   hipError_t h;
-  if ((h = hipMemsetAsync(e->Q.p, 0, e->Q.n * sizeof(float), e->stream)) != hipSuccess)
-    return bail(h, "clear Q");
-  if ((h = hipMemsetAsync(e->s.p, 0, N * 4, e->stream)) != hipSuccess) return bail(h, "clear s");
-  if ((h = hipMemsetAsync(e->ep_step.p, 0, N * 4, e->stream)) != hipSuccess) return bail(h, "clear");
-  if ((h = hipMemsetAsync(e->episode.p, 0, N * 4, e->stream)) != hipSuccess) return bail(h, "clear");
-  if ((h = hipMemsetAsync(e->start.p, 0, N * 4, e->stream)) != hipSuccess) return bail(h, "clear");
-  if ((h = hipMemsetAsync(e->act.p, 0, N * 4, e->stream)) != hipSuccess) return bail(h, "clear");
-  if ((h = hipMemsetAsync(e->reward.p, 0, N * 4, e->stream)) != hipSuccess) return bail(h, "clear");
-  if ((h = hipMemsetAsync(e->done.p, 0, N, e->stream)) != hipSuccess) return bail(h, "clear");
-  if ((h = hipMemsetAsync(e->action.p, 0, N, e->stream)) != hipSuccess) return bail(h, "clear");
-  if ((h = hipMemsetAsync(e->map.p, 0, e->map.n * 4, e->stream)) != hipSuccess) return bail(h, "clear");
-  if (e->pdiag.p && (h = hipMemsetAsync(e->pdiag.p, 0, e->pdiag.n * 8, e->stream)) != hipSuccess) return bail(h, "clear");
-  if (cfg->track_returns) {
-    void* bufs[] = {e->ret_acc.p, e->ret_last.p, e->ret_sum.p, e->len_last.p, e->len_sum.p};
-    for (void* b : bufs)
-      if ((h = hipMemsetAsync(b, 0, N * 4, e->stream)) != hipSuccess) return bail(h, "clear");
-  }
+  if (!e->flag_page.ensure(128)) return fail(CRL_E_ALLOC, "pinned host memory for the engine's flag");
+  std::memset(e->flag_page.p, 0, 128);
+  if ((h = hipMemsetAsync(e->arena.p, 0, cleared, e->stream)) != hipSuccess) return bail(h, "clear the arena");
   if ((h = hipMemcpyAsync(e->eps_tab.p, eps.data(), eps.size() * sizeof(float), hipMemcpyHostToDevice,
                           e->stream)) != hipSuccess)
     return bail(h, "upload eps table");
@@ -979,6 +1144,8 @@ int create_engine(const crl_config* cfg, int device, crl_engine** out) {
                        reinterpret_cast<unsigned*>(e->cell_reward.p), bits, n);
     if ((h = hipGetLastError()) != hipSuccess) return bail(h, "fill cell rewards");
   }
+  rc = build_moves(e, 0, e->n_maps);  // of the all-free maps that stand until crl_set_maps
+  if (rc != CRL_OK) return rc;
   if ((h = hipStreamSynchronize(e->stream)) != hipSuccess) return bail(h, "sync");
   // set-up that crl_run_fused_noalloc must not have left to do: this device's copy
   // of the scratch array, and the kernels that may use the whole LDS
@@ -997,6 +1164,8 @@ int reset_envs(crl_engine* e, int32_t first, int32_t count) {
   if (first < 0 || count < 0 || (int64_t)first + count > e->N)
     return fail(CRL_E_RANGE, "env range [%d,%d) outside [0,%d)", first, first + count, e->N);
   if (count == 0) return CRL_OK;
+  e->mirror_seq = 0;
+  e->stepped = false;
   hipLaunchKernelGGL(crl::k_reset, dim3((count + 255) / 256), dim3(256), 0, e->stream, e->ptrs(), first,
                      count);
   HIP_TRY(hipGetLastError());
@@ -1092,6 +1261,8 @@ int run_fused(crl_engine* e, int32_t n_steps, bool no_alloc) {
     ~Restore() { e->no_alloc = false; }
   } restore{e};
   e->no_alloc = no_alloc;
+  e->mirror_seq = 0;
+  e->stepped = false;
   if (e->cfg.table_mode == CRL_TABLE_PER_ENV) {
     const FusedPlan p = plan_fused(e, n_steps);
     if (p.lds > kLdsPerWorkgroup)
@@ -1221,37 +1392,83 @@ int crl_reset(crl_engine* e, int32_t first, int32_t count) { return reset_envs(e
 int crl_step(crl_engine* e, const int32_t* actions) {
   int rc = check_usable(e);
   if (rc) return rc;
-  if (actions) {
-    HIP_TRY(hipMemcpyAsync(e->act.p, actions, (size_t)e->N * 4, hipMemcpyHostToDevice, e->stream));
+  const size_t bytes = (size_t)e->N * 4;
+  const int32_t* act = e->act.p;
+  int act0 = -1;
+  crl::HostSignal sig{};
+  crl::StateMirror mirror{};
+  crl_engine::InSlot* slot = nullptr;
+  if (!actions) {
+    if (!e->have_actions) return fail(CRL_E_STATE, "crl_step(NULL) needs a preceding crl_select");
+  } else if (e->N == 1) {
+    act = nullptr;
+    act0 = actions[0];
+  } else if (bytes <= kLinkLimitBytes) {
+    // the kernel reads the actions where they are put now, and the caller's buffer is free
+    rc = claim_in_slot(e, bytes, &slot);
+    if (rc) return rc;
+    std::memcpy(slot->page.p, actions, bytes);
+    act = reinterpret_cast<const int32_t*>(slot->page.p);
+  } else {
+    HIP_TRY(hipMemcpyAsync(e->act.p, actions, bytes, hipMemcpyHostToDevice, e->stream));
     // the host buffer may be reused as soon as we return
     HIP_TRY(hipStreamSynchronize(e->stream));
-  } else if (!e->have_actions) {
-    return fail(CRL_E_STATE, "crl_step(NULL) needs a preceding crl_select");
   }
-  hipLaunchKernelGGL(crl::k_step, dim3((e->N + 255) / 256), dim3(256), 0, e->stream, e->rules(),
-                     e->ptrs(), e->transition(), e->act.p);
+  // A caller that looks at the state after every step gets it from the step's own kernel
+  // instead of from a second launch: 6 us of launch and answer saved, 18 bytes per env
+  // over the link added, so it stops with the first step whose state nobody asked for.
+  // (Not in a call that a stream capture may record: a replay has no number of its own.)
+  if (!e->mirror_read) e->mirror_steps = false;
+  e->mirror_read = false;
+  e->mirror_seq = 0;
+  const bool mirrors = actions && e->mirror_steps && !e->state_shared && e->state_bytes <= kLinkLimitBytes;
+  if (mirrors) {
+    rc = claim_out_page(e, e->state_bytes);
+    if (rc) return rc;
+    mirror = state_mirror(e);
+  }
+  if (slot || mirrors) sig = next_signal(e);
+  const int block = e->N <= 64 ? 64 : 256;
+  hipLaunchKernelGGL(crl::k_step, dim3((e->N + block - 1) / block), dim3(block), 0, e->stream, e->rules(),
+                     e->ptrs(), e->transition(), act, act0, mirror, sig);
   HIP_TRY(hipGetLastError());
+  if (slot) slot->last_seq = sig.seq;
+  if (mirrors) e->mirror_seq = sig.seq;
   if (e->trace_n > 0 && e->trace_cursor < e->trace_cap) e->trace_cursor += 1;
   e->have_transition = true;
   e->have_actions = false;
+  e->stepped = true;
   return CRL_OK;
 }
 
 int crl_select(crl_engine* e, int32_t* actions_out) {
   int rc = check_usable(e);
   if (rc) return rc;
-  const long long threads = (long long)e->N * e->A;
-  const int grid = (int)((threads + 255) / 256);
+  const size_t bytes = (size_t)e->N * 4;
+  const bool direct = actions_out && bytes <= kLinkLimitBytes;
+  int32_t* host_out = nullptr;
+  crl::HostSignal sig{};
+  if (direct) {
+    rc = claim_out_page(e, bytes);
+    if (rc) return rc;
+    host_out = reinterpret_cast<int32_t*>(e->out_page.p);
+    sig = next_signal(e);
+  }
+  const dim3 block(e->N <= 64 ? 64 : 256), grid((e->N + block.x - 1) / block.x);
   if (e->A == 4)
-    hipLaunchKernelGGL((crl::k_select<4>), dim3(grid), dim3(256), 0, e->stream, e->rules(), e->ptrs(),
-                       e->t, e->act.p);
+    hipLaunchKernelGGL((crl::k_select<4>), grid, block, 0, e->stream, e->rules(), e->ptrs(), e->t, e->act.p,
+                       host_out, sig);
   else
-    hipLaunchKernelGGL((crl::k_select<8>), dim3(grid), dim3(256), 0, e->stream, e->rules(), e->ptrs(),
-                       e->t, e->act.p);
+    hipLaunchKernelGGL((crl::k_select<8>), grid, block, 0, e->stream, e->rules(), e->ptrs(), e->t, e->act.p,
+                       host_out, sig);
   HIP_TRY(hipGetLastError());
   e->have_actions = true;
-  if (actions_out) {
-    HIP_TRY(hipMemcpyAsync(actions_out, e->act.p, (size_t)e->N * 4, hipMemcpyDeviceToHost, e->stream));
+  if (direct) {
+    rc = wait_seq(e, sig.seq);
+    if (rc) return rc;
+    std::memcpy(actions_out, host_out, bytes);
+  } else if (actions_out) {
+    HIP_TRY(hipMemcpyAsync(actions_out, e->act.p, bytes, hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
   }
   return CRL_OK;
@@ -1344,6 +1561,25 @@ int crl_get_state(crl_engine* e, int32_t* s, float* reward, uint8_t* done, uint8
   int rc = check_usable(e);
   if (rc) return rc;
   const size_t N = (size_t)e->N;
+  if (e->state_bytes <= kLinkLimitBytes) {
+    if (e->mirror_seq != 0) {
+      rc = wait_seq(e, e->mirror_seq);
+      if (rc == CRL_OK) rc = check_persist(e);
+    } else {
+      rc = fetch_pinned(e, e->state_at, e->state_bytes);
+      if (rc == CRL_OK && e->stepped) e->mirror_steps = true;
+    }
+    if (rc) return rc;
+    e->mirror_read = true;
+    const crl::StateMirror M = state_mirror(e);
+    if (s) std::memcpy(s, M.s, N * 4);
+    if (reward) std::memcpy(reward, M.reward, N * 4);
+    if (done) std::memcpy(done, M.done, N);
+    if (action) std::memcpy(action, M.action, N);
+    if (ep_step) std::memcpy(ep_step, M.ep_step, N * 4);
+    if (episode) std::memcpy(episode, M.episode, N * 4);
+    return CRL_OK;
+  }
   if (s) HIP_TRY(hipMemcpyAsync(s, e->s.p, N * 4, hipMemcpyDeviceToHost, e->stream));
   if (reward) HIP_TRY(hipMemcpyAsync(reward, e->reward.p, N * 4, hipMemcpyDeviceToHost, e->stream));
   if (done) HIP_TRY(hipMemcpyAsync(done, e->done.p, N, hipMemcpyDeviceToHost, e->stream));
@@ -1360,6 +1596,8 @@ int crl_set_state(crl_engine* e, const int32_t* s, const int32_t* ep_step, const
   rc = clear_persist_failure(e);
   if (rc) return rc;
   const size_t N = (size_t)e->N;
+  e->mirror_seq = 0;
+  e->stepped = false;
   if (s) {
     for (int i = 0; i < e->N; ++i)
       if (s[i] < 0 || (size_t)s[i] >= e->S) return fail(CRL_E_RANGE, "s[%d] = %d outside [0,%zu)", i, s[i], e->S);
@@ -1379,6 +1617,18 @@ int crl_get_episode_stats(crl_engine* e, float* last_return, int32_t* last_lengt
   if (rc) return rc;
   if (!e->cfg.track_returns) return fail(CRL_E_STATE, "the engine was created without track_returns");
   const size_t b = (size_t)e->N * 4;
+  if (e->stats_bytes <= kLinkLimitBytes) {
+    rc = fetch_pinned(e, e->stats_at, e->stats_bytes);
+    if (rc) return rc;
+    auto out = [&](void* to, const void* from) {
+      if (to) std::memcpy(to, e->out_page.p + (static_cast<const unsigned char*>(from) - e->stats_at), b);
+    };
+    out(last_return, e->ret_last.p);
+    out(last_length, e->len_last.p);
+    out(return_sum, e->ret_sum.p);
+    out(length_sum, e->len_sum.p);
+    return CRL_OK;
+  }
   if (last_return) HIP_TRY(hipMemcpyAsync(last_return, e->ret_last.p, b, hipMemcpyDeviceToHost, e->stream));
   if (last_length) HIP_TRY(hipMemcpyAsync(last_length, e->len_last.p, b, hipMemcpyDeviceToHost, e->stream));
   if (return_sum) HIP_TRY(hipMemcpyAsync(return_sum, e->ret_sum.p, b, hipMemcpyDeviceToHost, e->stream));
@@ -1405,8 +1655,14 @@ int crl_q_get_range(crl_engine* e, int32_t first_table, int32_t count, float* ou
   if (!out) return fail(CRL_E_ARG, "out is null");
   if (first_table < 0 || count < 0 || (int64_t)first_table + count > e->n_tables)
     return fail(CRL_E_RANGE, "table range [%d,%d) outside [0,%d)", first_table, first_table + count, e->n_tables);
-  HIP_TRY(hipMemcpyAsync(out, e->Q.p + (size_t)first_table * e->K, (size_t)count * e->K * sizeof(float),
-                         hipMemcpyDeviceToHost, e->stream));
+  const size_t bytes = (size_t)count * e->K * sizeof(float);
+  if (bytes > 0 && bytes <= kLinkLimitBytes) {  // (K is a multiple of 4: 16-byte words)
+    rc = fetch_pinned(e, e->Q.p + (size_t)first_table * e->K, bytes);
+    if (rc) return rc;
+    std::memcpy(out, e->out_page.p, bytes);
+    return CRL_OK;
+  }
+  HIP_TRY(hipMemcpyAsync(out, e->Q.p + (size_t)first_table * e->K, bytes, hipMemcpyDeviceToHost, e->stream));
   HIP_TRY(hipStreamSynchronize(e->stream));
   return check_persist(e);
 }
@@ -1506,6 +1762,7 @@ int crl_device_ptr(crl_engine* e, int32_t which, void** out) {
     case CRL_PTR_Q: *out = e->Q.p; break;
     default: return fail(CRL_E_ARG, "unknown pointer id %d", which);
   }
+  if (which != CRL_PTR_Q) e->state_shared = true;
   return CRL_OK;
 }
 

@@ -723,39 +723,31 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
 // called in that order and back the reference-shaped host classes.
 // ---------------------------------------------------------------------------
 
-// Epsilon-greedy select with A lanes per env: lane a holds Q[s][a] (one
-// coalesced read of the row), and the argmax runs over the lane group with
-// cross-lane shuffles on (value, index) so that the lowest index wins ties
-// (src/q_learning.cu:200-206).  The group's first lane draws and writes.
+// Epsilon-greedy select, one lane per env: the row is one 16-byte load (two with 8
+// actions), the lowest index wins ties (src/q_learning.cu:200-206).  `host_out` (may be
+// null): the actions also go to pinned host memory, 256 bytes in a row per wave - with A
+// lanes per env only every A-th lane had one to store.
 template <int A>
 __global__ __launch_bounds__(256) void k_select(const Rules R, const Ptrs P, const uint64_t t,
-                                                 int32_t* __restrict__ act_out) {
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int env = gid / A;
-  const int a = gid - env * A;
-  const bool live = env < P.N;
-  const int e = live ? env : P.N - 1;  // keep whole groups active for the shuffles
-  const int s = P.s[e];
-  const float* Qe = P.Q + (P.table_shared ? 0 : (size_t)e * P.S * A);
-  float v = Qe[(size_t)s * A + a];
-  int idx = a;
-#pragma unroll
-  for (int m = 1; m < A; m <<= 1) {
-    const float ov = __shfl_xor(v, m);
-    const int oi = __shfl_xor(idx, m);
-    const bool take = (ov > v) || (ov == v && oi < idx);
-    v = take ? ov : v;
-    idx = take ? oi : idx;
+                                                 int32_t* __restrict__ act_out,
+                                                 int32_t* __restrict__ host_out, const HostSignal sig) {
+  const int env = blockIdx.x * blockDim.x + threadIdx.x;
+  if (env < P.N) {
+    const int s = P.s[env];
+    const int episode = P.episode[env];
+    const float* Qe = P.Q + (P.table_shared ? 0 : (size_t)env * P.S * A);
+    const int greedy = row_argmax(load_row<A>(Qe + (size_t)s * A));
+    Draw d = pick_draw(explore_block(R.seed, (uint32_t)env, t >> 1), t, A);
+    if (P.u_sup && t >= P.sup_t0 && t - P.sup_t0 < (uint64_t)P.sup_n) {
+      const size_t o = (size_t)(t - P.sup_t0) * P.N + env;
+      d.u = P.u_sup[o];
+      d.a = P.a_sup[o];
+    }
+    const int a = (d.u < eps_of(R, P.eps_tab, t, episode)) ? d.a : greedy;
+    act_out[env] = a;
+    if (host_out) host_out[env] = a;
   }
-  if (!live || a != 0) return;
-  Draw d = pick_draw(explore_block(R.seed, (uint32_t)env, t >> 1), t, A);
-  if (P.u_sup && t >= P.sup_t0 && t - P.sup_t0 < (uint64_t)P.sup_n) {
-    const size_t o = (size_t)(t - P.sup_t0) * P.N + env;
-    d.u = P.u_sup[o];
-    d.a = P.a_sup[o];
-  }
-  const float eps = eps_of(R, P.eps_tab, t, P.episode[env]);
-  act_out[env] = (d.u < eps) ? d.a : idx;
+  signal_host(sig);
 }
 
 // transition left behind by k_step for k_update_* : (s, a, r, s', done)
@@ -767,33 +759,59 @@ struct Transition {
   uint8_t* done;
 };
 
+// The state arrays' copies in pinned host memory (all null: none is kept), laid out as the
+// engine's own are.
+struct StateMirror {
+  int32_t* s;
+  int32_t* ep_step;
+  int32_t* episode;
+  float* reward;
+  uint8_t* done;
+  uint8_t* action;
+  __device__ __forceinline__ void put(int env, int s_, int ep_step_, int episode_, float reward_, int done_, int action_) const {
+    if (!s) return;
+    s[env] = s_;
+    ep_step[env] = ep_step_;
+    episode[env] = episode_;
+    reward[env] = reward_;
+    done[env] = (uint8_t)done_;
+    action[env] = (uint8_t)action_;
+  }
+};
+
 // One move for every env with supplied actions (src/environment.cu:113-125,
 // rules of src/kernels.cu:13-66), then the restart of finished envs.
-__global__ __launch_bounds__(256) void k_step(const Rules R, const Ptrs P, const Transition T,
-                                               const int32_t* __restrict__ act) {
-  const int env = blockIdx.x * blockDim.x + threadIdx.x;
-  if (env >= P.N) return;
+// `act` may be host memory the device can read; for a single env the action comes as `act0`
+// (act null): one trip over the link less in a call of 6 us.
+// The new state also goes to `mirror` (may be null).
+__device__ __forceinline__ void step_env(const Rules& R, const Ptrs& P, const Transition& T,
+                                         const int32_t* __restrict__ act, const int act0,
+                                         const StateMirror& M, const int env) {
   const uint32_t* gmap = P.map + (P.map_shared ? 0 : (size_t)env * P.map_words);
   auto cls = [&](int cell) -> int { return cell_class_of(gmap[cell >> 4], cell); };
   const float* cr = P.cell_reward ? P.cell_reward + (P.map_shared ? 0 : (size_t)env * P.S) : nullptr;
-  const int s0 = P.s[env];
-  if (R.max_episodes > 0 && P.episode[env] >= R.max_episodes) {
+  // (everything that depends on nothing is asked for at once, before the first store)
+  const int s0 = P.s[env], start = P.start[env], ep_step0 = P.ep_step[env];
+  int episode = P.episode[env];
+  const bool done0 = P.done[env] != 0;
+  const int a = act ? act[env] : act0;
+  if (R.max_episodes > 0 && episode >= R.max_episodes) {
     T.s[env] = s0;  // budget used up: no move and, with action -1, no update
     T.a[env] = -1;
     T.r[env] = 0.0f;
     T.s2[env] = s0;
     T.done[env] = 0;
     trace_idle(P, env, P.trace_cursor, s0);
+    M.put(env, s0, ep_step0, episode, P.reward[env], P.done[env], P.action[env]);
     return;
   }
   int x = s0 % R.W, y = s0 / R.W;
-  const int a = act[env];
   float reward;
   bool hit;
   step_rule(R, ClassRewards{R.step_reward, R.goal_reward, R.trap_reward}, cls, cr, x, y, a, reward, hit);
   const int s2 = y * R.W + x;
-  const bool done = hit || (!R.auto_reset && P.done[env] != 0);
-  int ep_step = P.ep_step[env] + 1;
+  const bool done = hit || (!R.auto_reset && done0);
+  int ep_step = ep_step0 + 1;
   const float ret = P.ret_acc ? P.ret_acc[env] + reward : 0.0f;
   T.s[env] = s0;
   T.a[env] = a;
@@ -810,19 +828,35 @@ __global__ __launch_bounds__(256) void k_step(const Rules R, const Ptrs P, const
     P.tr_r[o] = reward;
     P.tr_d[o] = done ? 1 : 0;
   }
-  if (R.auto_reset && (done || (R.episode_len > 0 && ep_step >= R.episode_len))) {
-    if (P.ret_acc) {
-      record_episode(P, env, ret, ep_step);
-      P.ret_acc[env] = 0.0f;
-    }
-    P.s[env] = P.start[env];
-    P.ep_step[env] = 0;
-    P.episode[env] += 1;
-  } else {
-    if (P.ret_acc) P.ret_acc[env] = ret;
-    P.s[env] = s2;
-    P.ep_step[env] = ep_step;
+  const bool ends = R.auto_reset && (done || (R.episode_len > 0 && ep_step >= R.episode_len));
+  if (P.ret_acc) {
+    if (ends) record_episode(P, env, ret, ep_step);
+    P.ret_acc[env] = ends ? 0.0f : ret;
   }
+  const int s_new = ends ? start : s2;
+  ep_step = ends ? 0 : ep_step;
+  P.s[env] = s_new;
+  P.ep_step[env] = ep_step;
+  if (ends) P.episode[env] = ++episode;
+  M.put(env, s_new, ep_step, episode, reward, done ? 1 : 0, (uint8_t)a);
+}
+__global__ __launch_bounds__(256) void k_step(const Rules R, const Ptrs P, const Transition T,
+                                               const int32_t* __restrict__ act, const int act0,
+                                               const StateMirror M, const HostSignal sig) {
+  const int env = blockIdx.x * blockDim.x + threadIdx.x;
+  if (env < P.N) step_env(R, P, T, act, act0, M, env);
+  signal_host(sig);
+}
+
+// n16 16-byte words from device memory to pinned host memory, and one word on its own
+// (may be null)
+__global__ __launch_bounds__(256) void k_export(const uint4* __restrict__ src, uint4* __restrict__ dst,
+                                                 const size_t n16, const unsigned* __restrict__ word,
+                                                 unsigned* __restrict__ word_out, const HostSignal sig) {
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride) dst[i] = src[i];
+  if (word && blockIdx.x == 0 && threadIdx.x == 0) *word_out = *word;
+  signal_host(sig);
 }
 
 // Environment::reset for envs [first, first+count) (src/environment.cu:6-14)

@@ -34,10 +34,13 @@ BatchedEnvironment::State BatchedEnvironment::state() const {
   st.reward.resize(n);
   st.done.resize(n);
   st.action.resize(n);
-  check(crl_get_state(engine, st.s.data(), st.reward.data(), st.done.data(), st.action.data(),
-                      st.ep_step.data(), st.episode.data()),
-        "state");
+  stateInto(st.s.data(), st.reward.data(), st.done.data(), st.action.data(), st.ep_step.data(), st.episode.data());
   return st;
+}
+
+void BatchedEnvironment::stateInto(int32_t* s, float* reward, uint8_t* done, uint8_t* action, int32_t* ep_step,
+                                   int32_t* episode) const {
+  check(crl_get_state(engine, s, reward, done, action, ep_step, episode), "state");
 }
 
 BatchedEnvironment::EpisodeStats BatchedEnvironment::episodeStats() const {

@@ -39,6 +39,8 @@ class BatchedEnvironment {
     std::vector<uint8_t> done, action;
   };
   State state() const;
+  // the same into the caller's arrays of numEnvs() entries
+  void stateInto(int32_t* s, float* reward, uint8_t* done, uint8_t* action, int32_t* ep_step, int32_t* episode) const;
   // needs config().track_returns
   struct EpisodeStats {
     std::vector<float> last_return, return_sum;

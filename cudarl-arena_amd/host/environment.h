@@ -42,6 +42,8 @@ class Environment {
 
   float getCellValue(int x, int y) const;
   std::vector<float> getGrid() const;
+  // the same without a copy, row-major [y][x]; valid as long as the Environment
+  const std::vector<float>& gridValues() const { return grid_store; }
 
   // Additive: write one cell of the float grid.  The value is classified with
   // the thresholds of src/kernels.cu:30-63 unless `trap` forces a TRAP cell

@@ -97,13 +97,6 @@ crl_config make_config(int n_envs, int width, int height, int n_actions, bool sh
   return c;
 }
 
-template <class T>
-py::array_t<T> to_array(const std::vector<T>& v) {
-  py::array_t<T> a((py::ssize_t)v.size());
-  std::memcpy(a.mutable_data(), v.data(), v.size() * sizeof(T));
-  return a;
-}
-
 // The reference's other Python surface (src/bindings/python_bindings.cpp:9-63,
 // class PyEnvironment bound as `Environment` there): observations as an (H, W)
 // numpy array, a dict for info, width / height / env_id as read-only properties.
@@ -125,7 +118,7 @@ class PyEnvironment {
     return std::make_tuple(observation(), env_.getReward(), env_.isDone(), info);
   }
   py::array_t<float> observation() const {
-    const std::vector<float> grid = env_.getGrid();  // row-major [y][x]: already the (H, W) layout
+    const std::vector<float>& grid = env_.gridValues();  // row-major [y][x]: already the (H, W) layout
     py::array_t<float> obs({(py::ssize_t)height_, (py::ssize_t)width_});
     std::memcpy(obs.mutable_data(), grid.data(), grid.size() * sizeof(float));
     return obs;
@@ -259,14 +252,19 @@ PYBIND11_MODULE(cudarl_core, m) {
       .def("sync", &BatchedEnvironment::sync)
       .def("state",
            [](const BatchedEnvironment& self) {
-             const BatchedEnvironment::State st = self.state();
+             const py::ssize_t n = self.numEnvs();
+             py::array_t<int32_t> s(n), ep_step(n), episode(n);
+             py::array_t<float> reward(n);
+             py::array_t<uint8_t> done(n), action(n);
+             self.stateInto(s.mutable_data(), reward.mutable_data(), done.mutable_data(), action.mutable_data(),
+                            ep_step.mutable_data(), episode.mutable_data());
              py::dict d;
-             d["s"] = to_array(st.s);
-             d["ep_step"] = to_array(st.ep_step);
-             d["episode"] = to_array(st.episode);
-             d["reward"] = to_array(st.reward);
-             d["done"] = to_array(st.done);
-             d["action"] = to_array(st.action);
+             d["s"] = s;
+             d["ep_step"] = ep_step;
+             d["episode"] = episode;
+             d["reward"] = reward;
+             d["done"] = done;
+             d["action"] = action;
              return d;
            })
       .def("q_table",

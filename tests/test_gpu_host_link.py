@@ -1,0 +1,80 @@
+"""What goes between host and kernels through pinned memory: actions in, actions, state and
+tables out, at the sizes where the way they take changes (one env, one and several
+workgroups, past the size that goes through pinned memory at all), and the state copy that
+the step kernel keeps while the state is read after every step."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+NAMES = ("s", "ep_step", "episode", "reward", "done", "action")
+
+
+def same(a, b):
+    return all(np.array_equal(a[k], b[k]) for k in NAMES)
+
+
+@pytest.mark.parametrize("N", [1, 2, 64, 65, 256, 257, 4099, 240001])
+def test_rounds_with_the_state_read_in_every_order(gpu, N):
+    W, H = 6, 5
+    cls, start = gpu.gen_maps_bernoulli(5, N, N, W, H, 0.1, 0.05)
+    cfg = gpu.make_config(N, W, H, episode_len=7, eps0=0.4, seed=9)
+    with gpu.Engine(cfg, 0) as want, gpu.Engine(cfg, 0) as eng:
+        want.set_maps(cls, start)
+        eng.set_maps(cls, start)
+        assert same(want.get_state(), eng.get_state())
+        for k in range(12):
+            want.run_fused(1)
+            # actions through the host, or left on the device
+            eng.step(eng.select() if k % 3 != 2 else (eng.select(fetch=False), None)[1])
+            if k not in (4, 5, 8):  # read after every step but these: the copy stops and starts again
+                if k == 6:
+                    eng.q_get(0, 1)  # (takes the page that held the copy)
+                assert same(want.get_state(), eng.get_state()), k
+            eng.update()
+            if k in (1, 7):  # the update leaves the state as it is
+                assert same(want.get_state(), eng.get_state()), k
+        assert np.array_equal(want.q_get(0, N), eng.q_get(0, N))
+        eng.reset(0, 1)
+        want.reset(0, 1)
+        assert same(want.get_state(), eng.get_state())
+
+
+def test_state_written_by_the_caller_is_what_the_next_read_returns(gpu):
+    """Views of the state are out: no copy of it may be handed out in its place."""
+    hip = C.CDLL("libamdhip64.so")
+    N = 70
+    mine = np.full(N, 7, np.int32)
+    with gpu.Engine(gpu.make_config(N, 6, 5, seed=1), 0) as eng:
+        eng.set_maps(np.zeros((N, 30), np.uint8), np.arange(N, dtype=np.int32) % 30)
+        for _ in range(3):
+            eng.step(np.zeros(N, np.int32))
+            eng.get_state()
+        view = eng.device_ptr(0)
+        eng.step(np.zeros(N, np.int32))
+        assert hip.hipMemcpy(C.c_void_p(view), C.c_void_p(mine.ctypes.data), C.c_size_t(4 * N), 1) == 0  # host to device
+        assert np.array_equal(eng.get_state()["s"], mine)
+
+
+def test_actions_may_be_overwritten_once_step_has_returned(gpu):
+    N = 5000
+    acts = np.zeros((20, N), np.int32)
+    rng = np.random.default_rng(0)
+    acts[:] = rng.integers(0, 4, acts.shape)
+    cls = np.zeros((N, 99), np.uint8)
+    start = np.full(N, 49, np.int32)
+    with gpu.Engine(gpu.make_config(N, 11, 9, seed=1), 0) as eng:
+        eng.set_maps(cls, start)
+        buf = np.empty(N, np.int32)
+        for a in acts:
+            buf[:] = a
+            eng.step(buf)
+            buf[:] = -1
+        st = eng.get_state()
+    x, y = np.full(N, 5), np.full(N, 4)
+    for a in acts:
+        x = np.clip(x + (a == 1) - (a == 3), 0, 10)
+        y = np.clip(y + (a == 2) - (a == 0), 0, 8)
+    assert np.array_equal(st["s"], y * 11 + x)
