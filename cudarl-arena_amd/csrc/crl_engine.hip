@@ -216,10 +216,6 @@ struct crl_engine {
   DevBuf<float> delta;
   DevBuf<unsigned long long> handoff;
   bool lds_opt_in = false;
-  // scratch of crl_td_update
-  DevBuf<int32_t> b_s, b_a, b_s2;
-  DevBuf<float> b_r;
-  DevBuf<uint8_t> b_done;
   // trace
   DevBuf<int32_t> trace_s;
   DevBuf<uint8_t> trace_a, trace_d;
@@ -547,12 +543,22 @@ int ceil_log2(size_t v) {
   return b;
 }
 
+int own_keys(const crl::ReduceGeom& G) {  // keys of the owner that has most
+  const int rows = G.K >> G.a_shift;
+  return ((rows + (1 << G.own_shift) - 1) >> G.own_shift) << G.a_shift;
+}
+
+// Owners of the two-launch reduction: 256, one per compute unit, also where the table has
+// few keys for each (a block's 256 samples then fall into cells of a record or two, and the
+// cells of 8 records are read 16 blocks at a time); more where an owner would have more keys
+// than its LDS rows hold.
 crl::ReduceGeom reduce_geom(const crl_engine* e, int n) {
   crl::ReduceGeom G{};
   G.K = (int)e->K;
   G.a_shift = e->A == 8 ? 3 : 2;
-  G.own_shift = ceil_log2((e->K + crl::kOwnKeys - 1) / crl::kOwnKeys);
   G.n_blocks = (n + crl::kBlockSamples - 1) / crl::kBlockSamples;
+  G.own_shift = crl::kPersistOwnShift;
+  while (own_keys(G) > crl::kMaxOwnKeys) ++G.own_shift;
   G.cell_shift = crl::cell_shift_for(G.own_shift);
   G.main_shift = crl::main_shift_for(G.own_shift);
   return G;
@@ -562,14 +568,21 @@ size_t handoff_records(const crl::ReduceGeom& G) {
   return (((size_t)1 << G.own_shift) * (size_t)G.n_blocks) << G.cell_shift;
 }
 
-// the two-pass reduction needs the dense LDS table (K <= 16384) and a bounded hand-off buffer
-bool reduce_fast(const crl_engine* e, const crl::ReduceGeom& G) {
-  return e->K <= (size_t)crl::kDenseKeys && handoff_records(G) * sizeof(uint2) <= kHandoffLimitBytes;
+// Small tables need less room with as many owners as 64 keys each make: for a call whose
+// hand-off cells have to fit into `limit`.
+crl::ReduceGeom reduce_geom_within(const crl_engine* e, int n, size_t limit) {
+  crl::ReduceGeom G = reduce_geom(e, n);
+  if (handoff_records(G) * sizeof(unsigned long long) <= limit || e->K > (size_t)crl::kDenseKeys) return G;
+  G.own_shift = ceil_log2((e->K + crl::kOwnKeys - 1) / crl::kOwnKeys);
+  G.cell_shift = crl::cell_shift_for(G.own_shift);
+  G.main_shift = crl::main_shift_for(G.own_shift);
+  return G;
 }
 
-constexpr size_t kOwnersLds = (size_t)(crl::kTileBlocks + crl::kTileBlocks / crl::kGroupBlocks) *
-                              crl::kOwnKeys * sizeof(float) +
-                              crl::kBlockSamples * sizeof(float);  // tile, group sums, a word per thread that nobody reads
+// the two-pass reduction needs a bounded number of owners and a bounded hand-off buffer
+bool reduce_fast(const crl::ReduceGeom& G) {
+  return 1 << G.own_shift <= crl::kMaxOwners && handoff_records(G) * sizeof(unsigned long long) <= kHandoffLimitBytes;
+}
 
 template <class Kern>
 hipError_t allow_lds(Kern kern, size_t bytes) {
@@ -581,8 +594,16 @@ hipError_t allow_lds(Kern kern, size_t bytes) {
 int opt_in_lds(crl_engine* e) {
   if (e->lds_opt_in) return CRL_OK;
   const size_t act = kLdsPerWorkgroup;  // what a launch asks for is checked against this
-  HIP_TRY(allow_lds(crl::k_reduce_blocks, crl::kReduceLdsBytes));
-  HIP_TRY(allow_lds(crl::k_reduce_owners, kOwnersLds));
+  HIP_TRY(allow_lds(crl::k_reduce_owners<false>, act));
+  HIP_TRY(allow_lds(crl::k_reduce_owners<true>, act));
+  HIP_TRY(allow_lds(crl::k_td_blocks<4, crl::PackedSamples>, act));
+  HIP_TRY(allow_lds(crl::k_td_blocks<8, crl::PackedSamples>, act));
+  HIP_TRY(allow_lds(crl::k_td_blocks<4, crl::Transition>, act));
+  HIP_TRY(allow_lds(crl::k_td_blocks<8, crl::Transition>, act));
+  HIP_TRY(allow_lds(crl::k_td_small<4, 4, crl::PackedSamples>, act));
+  HIP_TRY(allow_lds(crl::k_td_small<8, 4, crl::PackedSamples>, act));
+  HIP_TRY(allow_lds(crl::k_td_small<4, 4, crl::Transition>, act));
+  HIP_TRY(allow_lds(crl::k_td_small<8, 4, crl::Transition>, act));
   HIP_TRY(allow_lds(crl::k_shared_act<4, 1, true>, act - kStaticLdsReserve));
   HIP_TRY(allow_lds(crl::k_shared_act<4, 2, true>, act - kStaticLdsReserve));
   HIP_TRY(allow_lds(crl::k_shared_act<8, 1, true>, act - kStaticLdsReserve));
@@ -628,31 +649,65 @@ int ensure_handoff(crl_engine* e, const crl::ReduceGeom& G) {
   return opt_in_lds(e);
 }
 
-int reduce_owners(crl_engine* e, const crl::ReduceGeom& G, float* Q, const int32_t* key,
-                  const float* delta, int n) {
-  hipLaunchKernelGGL(crl::k_reduce_owners, dim3(1 << G.own_shift), dim3(256), kOwnersLds, e->stream, G,
-                     Q, key, delta, n, e->ho);
+int reduce_owners(crl_engine* e, const crl::ReduceGeom& G, float* Q, int n, const crl::HostSignal& sig) {
+  const int groups = (G.n_blocks + crl::kGroupBlocks - 1) / crl::kGroupBlocks;
+  const int keys = own_keys(G), waves = std::min(groups, crl::kOwnerWaves);
+  const dim3 grid(1 << G.own_shift), block(64 * waves);
+  const size_t lds = crl::owners_lds_bytes(waves, keys);
+  if (keys <= crl::kTileKeys)
+    hipLaunchKernelGGL(crl::k_reduce_owners<true>, grid, block, lds, e->stream, G, keys, Q, e->key.p, e->delta.p, n, e->ho, sig);
+  else
+    hipLaunchKernelGGL(crl::k_reduce_owners<false>, grid, block, lds, e->stream, G, keys, Q, e->key.p, e->delta.p, n, e->ho, sig);
   HIP_TRY(hipGetLastError());
   return CRL_OK;
 }
 
-// Q[k] += ordered sum of delta[i] with key[i] == k, for n samples on one table
-int reduce_apply(crl_engine* e, float* Q, const int32_t* key, const float* delta, int n) {
-  const crl::ReduceGeom G = reduce_geom(e, n);
-  e->no_alloc = false;  // crl_update / crl_td_update: the engine's own hand-off buffer
-  if (!reduce_fast(e, G)) {
-    const int grid = (int)((e->K + crl::kOwnKeys - 1) / crl::kOwnKeys);
-    hipLaunchKernelGGL(crl::k_reduce_scan, dim3(grid), dim3(256), 0, e->stream, Q, (int)e->K, key,
-                       delta, n);
+// Q[k] += ordered sum of the deltas of the n samples with key k, on one table.
+// `changed`, `sig`: see k_td_small, for at most 1024 samples; with more, `sig` says that the
+// samples have been read.
+template <int A, class Samples>
+int td_apply_a(crl_engine* e, float* Q, const Samples& X, int n, int2* changed, const crl::HostSignal& sig) {
+  const float lr = e->cfg.lr, gamma = e->cfg.gamma;
+  const int max_mode = e->cfg.max_mode;
+  int rc = opt_in_lds(e);
+  if (rc) return rc;
+  if (n <= crl::kSmallSamples) {
+#define CRL_TD_SMALL(NB)                                                                                      \
+  hipLaunchKernelGGL((crl::k_td_small<A, NB, Samples>), dim3(1), dim3(crl::kBlockSamples * NB),               \
+                     sizeof(crl::SmallLds<NB>), e->stream, X, n, Q, lr, gamma, max_mode, changed, sig)
+    if (n <= crl::kBlockSamples) CRL_TD_SMALL(1);
+    else if (n <= 2 * crl::kBlockSamples) CRL_TD_SMALL(2);
+    else CRL_TD_SMALL(4);
+#undef CRL_TD_SMALL
     HIP_TRY(hipGetLastError());
     return CRL_OK;
   }
-  int rc = ensure_handoff(e, G);
-  if (rc) return rc;
-  hipLaunchKernelGGL(crl::k_reduce_blocks, dim3(G.n_blocks), dim3(crl::kBlockSamples),
-                     crl::kReduceLdsBytes, e->stream, G, key, delta, n, e->ho);
+  hipError_t h = e->key.ensure((size_t)n);
+  if (h == hipSuccess) h = e->delta.ensure((size_t)n);
+  if (h != hipSuccess) return fail(CRL_E_ALLOC, "scratch allocation failed: %s", hipGetErrorString(h));
+  const crl::ReduceGeom G = reduce_geom(e, n);
+  const int grid = G.n_blocks;
+  if (reduce_fast(G)) {
+    e->no_alloc = false;  // crl_update / crl_td_update: the engine's own hand-off buffer
+    rc = ensure_handoff(e, G);
+    if (rc) return rc;
+    hipLaunchKernelGGL((crl::k_td_blocks<A, Samples>), dim3(grid), dim3(crl::kBlockSamples),
+                       crl::block_lds_bytes(G.own_shift), e->stream, G, X, n, Q, lr, gamma, max_mode, e->key.p,
+                       e->delta.p, e->ho);
+    HIP_TRY(hipGetLastError());
+    return reduce_owners(e, G, Q, n, sig);
+  }
+  hipLaunchKernelGGL((crl::k_delta<A, Samples>), dim3(grid), dim3(256), 0, e->stream, Q, X, n, lr, gamma, max_mode,
+                     e->key.p, e->delta.p);
   HIP_TRY(hipGetLastError());
-  return reduce_owners(e, G, Q, key, delta, n);
+  hipLaunchKernelGGL(crl::k_reduce_scan, dim3((unsigned)((e->K + crl::kOwnKeys - 1) / crl::kOwnKeys)), dim3(256), 0,
+                     e->stream, Q, (int)e->K, e->key.p, e->delta.p, n, sig);
+  HIP_TRY(hipGetLastError());
+  return CRL_OK;
+}
+template <class Samples>
+int td_apply(crl_engine* e, float* Q, const Samples& X, int n, int2* changed, const crl::HostSignal& sig) {
+  return e->A == 4 ? td_apply_a<4>(e, Q, X, n, changed, sig) : td_apply_a<8>(e, Q, X, n, changed, sig);
 }
 
 template <int A, int MAP>
@@ -660,7 +715,7 @@ void launch_shared_act(crl_engine* e, bool reduce, const crl::ReduceGeom& G, uin
   const crl::Rules R = e->rules();
   const crl::Ptrs P = e->ptrs();
   const int block = 256, grid = (e->N + block - 1) / block;
-  const size_t lds = (reduce ? crl::kReduceLdsBytes : 0) + (MAP == 1 ? (size_t)e->map_words * 4 : 0);
+  const size_t lds = (reduce ? crl::block_lds_bytes(G.own_shift) : 0) + (MAP == 1 ? (size_t)e->map_words * 4 : 0);
   if (reduce)
     hipLaunchKernelGGL((crl::k_shared_act<A, MAP, true>), dim3(grid), dim3(block), lds, e->stream, R, P,
                        t, trace_row, e->key.p, e->delta.p, G, e->ho);
@@ -671,8 +726,8 @@ void launch_shared_act(crl_engine* e, bool reduce, const crl::ReduceGeom& G, uin
 
 // one shared-table step: act (select + move + delta + block sums), then the key owners
 int shared_step(crl_engine* e, uint64_t t, int trace_row) {
-  const crl::ReduceGeom G = reduce_geom(e, e->N);
-  const bool fast = reduce_fast(e, G);
+  const crl::ReduceGeom G = e->no_alloc ? reduce_geom_within(e, e->N, kScratchExchangeBytes) : reduce_geom(e, e->N);
+  const bool fast = reduce_fast(G);
   if (fast) {
     int rc = ensure_handoff(e, G);
     if (rc) return rc;
@@ -681,7 +736,7 @@ int shared_step(crl_engine* e, uint64_t t, int trace_row) {
   // shared table itself stays in L2: streaming its 64 KB into every workgroup's
   // LDS each step measured slower than the row reads it saves (12.4 against 12.05 us
   // per step on 65,536 envs, also against the five speculative reads per env).
-  size_t lds = fast ? crl::kReduceLdsBytes : 0;
+  size_t lds = fast ? crl::block_lds_bytes(G.own_shift) : 0;
   const size_t limit = fast ? kLdsPerWorkgroup - kStaticLdsReserve : (size_t)64 * 1024;
   const size_t map_bytes = (size_t)e->map_words * 4;
   const bool lds_map = e->cfg.map_mode == CRL_MAP_SHARED && map_bytes <= (size_t)kLdsMapLimitBytes &&
@@ -695,10 +750,10 @@ int shared_step(crl_engine* e, uint64_t t, int trace_row) {
     else launch_shared_act<8, 2>(e, fast, G, t, trace_row);
   }
   HIP_TRY(hipGetLastError());
-  if (fast) return reduce_owners(e, G, e->Q.p, e->key.p, e->delta.p, e->N);
+  if (fast) return reduce_owners(e, G, e->Q.p, e->N, crl::HostSignal{});
   const int grid = (int)((e->K + crl::kOwnKeys - 1) / crl::kOwnKeys);
   hipLaunchKernelGGL(crl::k_reduce_scan, dim3(grid), dim3(256), 0, e->stream, e->Q.p, (int)e->K,
-                     e->key.p, e->delta.p, e->N);
+                     e->key.p, e->delta.p, e->N, crl::HostSignal{});
   HIP_TRY(hipGetLastError());
   return CRL_OK;
 }
@@ -831,6 +886,7 @@ int run_persist(crl_engine* e, int n_steps, bool* launched) {
 // ---- pinned memory between host and kernels --------------------------------------------
 
 constexpr size_t kLinkLimitBytes = (size_t)4 << 20;  // larger transfers: hipMemcpyAsync straight to and from the caller's memory
+constexpr size_t kInSlotKeepBytes = (size_t)32 << 20;
 constexpr int kFlagErrWord = 16;                     // of flag_page; in another 64-byte line than the flag
 
 // the next launch that tells the host when it is through
@@ -1244,6 +1300,66 @@ int opt_in_ticket_kernels(crl_engine* e) {
   return CRL_OK;
 }
 
+// crl_td_update and, with `keys`, crl_td_update_collect.  The transitions are packed into
+// pinned memory, 12 bytes each, in the pass that checks them, and the kernel reads them
+// there: the call returns without waiting for anything (65,536 transitions: five copies from
+// pageable memory and a wait took 125 us).
+int td_update(crl_engine* e, int32_t table, int32_t n, const int32_t* s, const int32_t* a, const float* r,
+              const int32_t* s_next, const uint8_t* done, int32_t* keys, float* values) {
+  int rc = check_usable(e);
+  if (rc) return rc;
+  if (table < 0 || table >= e->n_tables) return fail(CRL_E_RANGE, "table %d outside [0,%d)", table, e->n_tables);
+  if (n < 0) return fail(CRL_E_ARG, "negative sample count");
+  if (n == 0) return CRL_OK;
+  if (!s || !a || !r || !s_next || !done) return fail(CRL_E_ARG, "null transition array");
+  const size_t nn = (size_t)n;
+  crl_engine::InSlot* slot = nullptr;
+  rc = claim_in_slot(e, 12 * nn, &slot);
+  if (rc) return rc;
+  crl::PackedSamples X;
+  int32_t* key = reinterpret_cast<int32_t*>(slot->page.p);
+  uint32_t* s2d = reinterpret_cast<uint32_t*>(key + nn);
+  X.key = key;
+  X.s2d = s2d;
+  X.r = reinterpret_cast<const float*>(s2d + nn);
+  if (!crl::pack_transitions(n, (int)e->S, e->A, s, a, s_next, done, key, s2d))
+    for (int i = 0; i < n; ++i) {
+      if (s[i] < 0 || (size_t)s[i] >= e->S) return fail(CRL_E_RANGE, "s[%d] = %d outside [0,%zu)", i, s[i], e->S);
+      if (s_next[i] < 0 || (size_t)s_next[i] >= e->S)
+        return fail(CRL_E_RANGE, "s_next[%d] = %d outside [0,%zu)", i, s_next[i], e->S);
+    }
+  std::memcpy(s2d + nn, r, nn * 4);
+  int2* changed = nullptr;
+  if (keys) {
+    rc = claim_out_page(e, nn * sizeof(int2));
+    if (rc) return rc;
+    changed = reinterpret_cast<int2*>(e->out_page.p);
+  }
+  const crl::HostSignal sig = next_signal(e);
+  rc = td_apply(e, e->Q.p + (size_t)table * e->K, X, n, changed, sig);
+  if (rc) {
+    // nothing may be left that works on the page or waits for a number that never comes
+    (void)hipStreamSynchronize(e->stream);
+    return rc;
+  }
+  slot->last_seq = sig.seq;
+  if (keys) {
+    rc = wait_seq(e, sig.seq);
+    if (rc) return rc;
+    for (int i = 0; i < n; ++i) {
+      keys[i] = changed[i].x;
+      std::memcpy(values + i, &changed[i].y, 4);
+    }
+  }
+  if (slot->page.n > kInSlotKeepBytes) {  // a page that large is not kept
+    rc = wait_seq(e, sig.seq);
+    slot->last_seq = 0;
+    if (rc) return rc;
+    slot->page.release();
+  }
+  return CRL_OK;
+}
+
 // crl_run_fused and its allocation-free variant: with `no_alloc` the ticket
 // counters and the hand-off cells live in the device's static scratch array and
 // nothing below allocates or frees
@@ -1489,16 +1605,7 @@ int crl_update(crl_engine* e) {
                          e->transition());
     HIP_TRY(hipGetLastError());
   } else {
-    if (e->A == 4)
-      hipLaunchKernelGGL((crl::k_delta<4>), dim3(grid), dim3(256), 0, e->stream, e->Q.p, e->N, e->tr_s.p,
-                         e->tr_a.p, e->tr_r.p, e->tr_s2.p, e->tr_done.p, R.lr, R.gamma, R.max_mode,
-                         e->key.p, e->delta.p);
-    else
-      hipLaunchKernelGGL((crl::k_delta<8>), dim3(grid), dim3(256), 0, e->stream, e->Q.p, e->N, e->tr_s.p,
-                         e->tr_a.p, e->tr_r.p, e->tr_s2.p, e->tr_done.p, R.lr, R.gamma, R.max_mode,
-                         e->key.p, e->delta.p);
-    HIP_TRY(hipGetLastError());
-    rc = reduce_apply(e, e->Q.p, e->key.p, e->delta.p, e->N);
+    rc = td_apply(e, e->Q.p, e->transition(), e->N, nullptr, crl::HostSignal{});
     if (rc) return rc;
   }
   e->have_transition = false;
@@ -1508,48 +1615,15 @@ int crl_update(crl_engine* e) {
 
 int crl_td_update(crl_engine* e, int32_t table, int32_t n, const int32_t* s, const int32_t* a,
                   const float* r, const int32_t* s_next, const uint8_t* done) {
-  int rc = check_usable(e);
-  if (rc) return rc;
-  if (table < 0 || table >= e->n_tables) return fail(CRL_E_RANGE, "table %d outside [0,%d)", table, e->n_tables);
-  if (n < 0) return fail(CRL_E_ARG, "negative sample count");
-  if (n == 0) return CRL_OK;
-  if (!s || !a || !r || !s_next || !done) return fail(CRL_E_ARG, "null transition array");
-  for (int i = 0; i < n; ++i) {
-    if (s[i] < 0 || (size_t)s[i] >= e->S) return fail(CRL_E_RANGE, "s[%d] = %d outside [0,%zu)", i, s[i], e->S);
-    if (s_next[i] < 0 || (size_t)s_next[i] >= e->S)
-      return fail(CRL_E_RANGE, "s_next[%d] = %d outside [0,%zu)", i, s_next[i], e->S);
-  }
-  const size_t nn = (size_t)n;
-  hipError_t h = hipSuccess;
-  auto acc = [&](hipError_t x) {
-    if (h == hipSuccess) h = x;
-  };
-  acc(e->b_s.ensure(nn));
-  acc(e->b_a.ensure(nn));
-  acc(e->b_s2.ensure(nn));
-  acc(e->b_r.ensure(nn));
-  acc(e->b_done.ensure(nn));
-  acc(e->key.ensure(nn > (size_t)e->N ? nn : (size_t)e->N));
-  acc(e->delta.ensure(nn > (size_t)e->N ? nn : (size_t)e->N));
-  if (h != hipSuccess) return fail(CRL_E_ALLOC, "scratch allocation failed: %s", hipGetErrorString(h));
-  HIP_TRY(hipMemcpyAsync(e->b_s.p, s, nn * 4, hipMemcpyHostToDevice, e->stream));
-  HIP_TRY(hipMemcpyAsync(e->b_a.p, a, nn * 4, hipMemcpyHostToDevice, e->stream));
-  HIP_TRY(hipMemcpyAsync(e->b_r.p, r, nn * 4, hipMemcpyHostToDevice, e->stream));
-  HIP_TRY(hipMemcpyAsync(e->b_s2.p, s_next, nn * 4, hipMemcpyHostToDevice, e->stream));
-  HIP_TRY(hipMemcpyAsync(e->b_done.p, done, nn, hipMemcpyHostToDevice, e->stream));
-  HIP_TRY(hipStreamSynchronize(e->stream));
-  float* Q = e->Q.p + (size_t)table * e->K;
-  const int grid = (n + 255) / 256;
-  if (e->A == 4)
-    hipLaunchKernelGGL((crl::k_delta<4>), dim3(grid), dim3(256), 0, e->stream, Q, n, e->b_s.p, e->b_a.p,
-                       e->b_r.p, e->b_s2.p, e->b_done.p, e->cfg.lr, e->cfg.gamma, e->cfg.max_mode,
-                       e->key.p, e->delta.p);
-  else
-    hipLaunchKernelGGL((crl::k_delta<8>), dim3(grid), dim3(256), 0, e->stream, Q, n, e->b_s.p, e->b_a.p,
-                       e->b_r.p, e->b_s2.p, e->b_done.p, e->cfg.lr, e->cfg.gamma, e->cfg.max_mode,
-                       e->key.p, e->delta.p);
-  HIP_TRY(hipGetLastError());
-  return reduce_apply(e, Q, e->key.p, e->delta.p, n);
+  return td_update(e, table, n, s, a, r, s_next, done, nullptr, nullptr);
+}
+
+int crl_td_update_collect(crl_engine* e, int32_t table, int32_t n, const int32_t* s, const int32_t* a,
+                          const float* r, const int32_t* s_next, const uint8_t* done, int32_t* keys,
+                          float* values) {
+  if (n > crl::kSmallSamples) return fail(CRL_E_RANGE, "%d samples, at most %d are collected", n, crl::kSmallSamples);
+  if (n > 0 && (!keys || !values)) return fail(CRL_E_ARG, "null output array");
+  return td_update(e, table, n, s, a, r, s_next, done, keys, values);
 }
 
 int crl_run_fused(crl_engine* e, int32_t n_steps) { return run_fused(e, n_steps, false); }

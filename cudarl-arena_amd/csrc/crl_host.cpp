@@ -96,6 +96,24 @@ void pack_classes(const uint8_t* cls, size_t n_cells, uint32_t* words) {
   }
 }
 
+// (wider vectors where the host has them: the loop is the larger half of an update of
+// 65,536 recorded transitions that the caller sees)
+#if defined(__x86_64__) && !defined(__SANITIZE_ADDRESS__)
+__attribute__((target_clones("avx512f", "avx2", "default")))
+#endif
+bool pack_transitions(int n, int S, int A, const int32_t* s, const int32_t* a, const int32_t* s_next,
+                      const uint8_t* done, int32_t* key, uint32_t* s2d) {
+  const int shift = A == 8 ? 3 : 2;
+  uint32_t bad = 0;
+  for (int i = 0; i < n; ++i) {
+    bad |= (uint32_t)((uint32_t)s[i] >= (uint32_t)S) | (uint32_t)((uint32_t)s_next[i] >= (uint32_t)S);
+    const uint32_t k = ((uint32_t)s[i] << shift) | ((uint32_t)a[i] & (uint32_t)(A - 1));
+    key[i] = (uint32_t)a[i] < (uint32_t)A ? (int32_t)k : -1;
+    s2d[i] = (uint32_t)s_next[i] | (done[i] != 0 ? 0x80000000u : 0u);
+  }
+  return bad == 0;
+}
+
 namespace {
 
 // word `i` of the stream (seed; a, stream id): counter (a, id, i/4, 0), lane i%4

@@ -26,4 +26,10 @@ std::vector<float> build_eps_table(const crl_config& cfg);
 // 16 cells per word, cell c in bits [2*(c%16), 2*(c%16)+1] of word c/16
 void pack_classes(const uint8_t* cls, size_t n_cells, uint32_t* words);
 
+// n transitions as the update kernels read them: key = s * A + a (-1 for an action outside
+// [0, A)), s2d = s' with done in the top bit.  -> false if a state lies outside [0, S); what
+// was written is then worthless.  A is 4 or 8, S at most 2^24.
+bool pack_transitions(int n, int S, int A, const int32_t* s, const int32_t* a, const int32_t* s_next,
+                      const uint8_t* done, int32_t* key, uint32_t* s2d);
+
 }  // namespace crl

@@ -750,15 +750,6 @@ __global__ __launch_bounds__(256) void k_select(const Rules R, const Ptrs P, con
   signal_host(sig);
 }
 
-// transition left behind by k_step for k_update_* : (s, a, r, s', done)
-struct Transition {
-  int32_t* s;
-  int32_t* a;
-  float* r;
-  int32_t* s2;
-  uint8_t* done;
-};
-
 // The state arrays' copies in pinned host memory (all null: none is kept), laid out as the
 // engine's own are.
 struct StateMirror {
@@ -888,31 +879,20 @@ __global__ __launch_bounds__(256) void k_update_per_env(const Rules R, const Ptr
   Qe[k] = td_value(Qe[k], T.r[env], m, R.lr, R.gamma);
 }
 
-// (key, delta) of n transitions against ONE table Q (K = S*A entries), all
-// reads before any write.  key = s*A + a, or -1 for an invalid action.
-template <int A>
-__global__ __launch_bounds__(256) void k_delta(const float* __restrict__ Q, const int n,
-                                                const int32_t* __restrict__ s,
-                                                const int32_t* __restrict__ a,
-                                                const float* __restrict__ r,
-                                                const int32_t* __restrict__ s2,
-                                                const uint8_t* __restrict__ done, const float lr,
-                                                const float gamma, const int max_mode,
-                                                int32_t* __restrict__ key,
-                                                float* __restrict__ delta) {
+// (key, delta) of n samples against ONE table (K = S*A entries), all reads before any
+// write, for the reduction that scans them.
+template <int A, class Samples>
+__global__ __launch_bounds__(256) void k_delta(const float* __restrict__ Q, const Samples X, const int n,
+                                                const float lr, const float gamma, const int max_mode,
+                                                int32_t* __restrict__ key, float* __restrict__ delta) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int ai = a[i];
-  if ((unsigned)ai >= (unsigned)A) {
-    key[i] = -1;
-    delta[i] = 0.0f;
-    return;
+  int k;
+  float d;
+  sample_delta<A>(X, i, n, Q, lr, gamma, max_mode, k, d);
+  if (i < n) {
+    key[i] = k;
+    delta[i] = d;
   }
-  const Row<A> row2 = load_row<A>(Q + (size_t)s2[i] * A);
-  const float m = row_max(row2, done[i] != 0, max_mode);
-  const int k = s[i] * A + ai;
-  key[i] = k;
-  delta[i] = td_delta(Q[k], r[i], m, lr, gamma);
 }
 
 // Shared table, first half of a fused step: every env selects, moves and emits
@@ -927,13 +907,13 @@ __global__ __launch_bounds__(256) void k_shared_act(const Rules R, const Ptrs P,
                                                      float* __restrict__ delta, const ReduceGeom G,
                                                      unsigned long long* __restrict__ handoff) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  uint32_t* lds_map = reinterpret_cast<uint32_t*>(lds_raw + (REDUCE ? kReduceLdsBytes : 0));
+  uint32_t* lds_map = reinterpret_cast<uint32_t*>(lds_raw + (REDUCE ? block_lds_bytes(G.own_shift) : 0));
   const int tid = threadIdx.x;
   const int env = blockIdx.x * blockDim.x + tid;
   bool live = env < P.N;
   // the env's cell is fetched while the map streams into LDS
   const int s_in = live ? P.s[env] : 0;
-  if (REDUCE) reduce_block_init(*reinterpret_cast<ReduceLds*>(lds_raw));
+  if (REDUCE) block_lds_init(lds_raw, G);
   if (MAP == 1)
     for (int i = tid; i < P.map_words; i += blockDim.x) lds_map[i] = P.map[i];
   if (MAP == 1 || REDUCE) __syncthreads();
@@ -1021,10 +1001,7 @@ __global__ __launch_bounds__(256) void k_shared_act(const Rules R, const Ptrs P,
       P.ep_step[env] = ep_step;
     }
   }
-  if (REDUCE) {
-    ReduceLds& L = *reinterpret_cast<ReduceLds*>(lds_raw);
-    reduce_block<false>(L, G, blockIdx.x, my_key, my_delta, live, handoff, 0u, reinterpret_cast<float*>(lds_raw + sizeof(ReduceLds)));
-  }
+  if (REDUCE) reduce_block_wide(lds_raw, G, blockIdx.x, my_key, my_delta, live, handoff);
 }
 
 // Move codes of maps [first, first + count) from their class maps: one thread per

@@ -374,9 +374,8 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
     // ---- block sums to the owners' cells ------------------------------------------------
     const int half = k & 1;  // cells and raw samples: two buffers, taken in turn
     // (`sorted`: the upper half of the tile, which is free until the block sums are through)
-    const bool over = reduce_block<true>(L.red, G, wg, my_key, my_delta, live, B.cells, want, L.tile + kTileBlocks * kOwnKeys / 2,
-                                         L.stage, &w_cells,
-                                         (uint32_t)((size_t)half * cells_half * 8), B.cells + (2 + half) * cells_half, true);
+    const bool over = reduce_block(L.red, G, wg, my_key, my_delta, live, want, L.tile + kTileBlocks * kOwnKeys / 2, L.stage,
+                                   w_cells, (uint32_t)((size_t)half * cells_half * 8), B.cells + (2 + half) * cells_half);
     if (over && has_env)
       st_dev64(B.raw + (size_t)half * P.N + env, tagged(__float_as_uint(my_delta),
                                    (uint32_t)my_key | (live ? kRawValid : 0u) | (want << kRawTagShift)));

@@ -8,33 +8,35 @@
 //
 // Two passes over the chip:
 //   1. one workgroup per block: the lowest thread that holds a key becomes the
-//      key's leader (LDS atomic min on a dense table), the other holders mark
+//      key's leader (LDS atomic min on a table of keys), the other holders mark
 //      themselves in the leader's 256-bit member set (LDS atomic or) and line
 //      their deltas up by their place in it, and the leader adds them in that
 //      order = thread order = sample order; every distinct key's block sum goes
 //      to the workgroup that owns the key;
-//   2. one workgroup per 64 keys lays the block sums it was handed out as a
-//      dense [block][key] tile in LDS and adds the columns in the tree order.
+//   2. one workgroup per owner of keys adds the block sums it was handed, a wave
+//      to a group, and then the groups.
+// Up to 1024 samples (four blocks, one group) are one workgroup's work and one launch.
 // Empty blocks add +0.0f, which changes nothing, so the result is a pure
 // function of (keys, deltas) whatever the occupancy.
 #pragma once
-#include <hip/hip_runtime.h>
-#include <stdint.h>
+#include "crl_device.h"
 
 namespace crl {
 
 constexpr int kBlockSamples = 256;   // level 0
 constexpr int kGroupBlocks = 16;     // level 1
-constexpr int kOwnKeys = 64;         // keys per owner workgroup: 64 / A whole table rows
-constexpr int kMinCellRecs = 8;      // records of a hand-off cell: 8 ... 64, see cell_shift_for()
+constexpr int kOwnKeys = 64;         // one-launch kernel: keys per owner workgroup, 64 / A whole table rows
+constexpr int kMaxOwnKeys = 1024;    // two launches: keys per owner at most
+constexpr int kMaxOwners = 4096;     // ... and owners
 constexpr int kSlotOverflow = 127;   // count value: more distinct keys than records, read the block's raw samples instead
 constexpr int kStagePieces = 512;    // 16-byte pieces of the main halves of one block's cells in the one-launch kernel
-constexpr int kDenseKeys = 16384;    // keys the dense LDS table of pass 1 can hold
+constexpr int kDenseKeys = 16384;    // one-launch kernel: keys of its LDS table, one entry per key
+constexpr int kHashSlots = 2048;     // two launches: entries of the LDS table of the keys a block holds
 constexpr int kTileBlocks = 256;     // blocks per LDS tile of pass 2
 constexpr uint32_t kOwnerMix = 37;   // odd: spreads cells a power of two apart over owners
 constexpr uint32_t kNoLead = 0xFFFFFFFFu;
 
-// A hand-off record is 64 bits, written and read as one unit:
+// A hand-off record is 64 bits, written and read as one unit.  One-launch kernel:
 //   bits  0..5   slot of the key among its owner's 64
 //   bits  6..12  record 0 of a cell only: how many records the cell holds
 //                (0: none, kSlotOverflow: more distinct keys than the cell has records)
@@ -47,6 +49,13 @@ __device__ __forceinline__ unsigned long long make_rec(uint32_t slot, uint32_t c
   const uint32_t meta = slot | (count << kRecCountShift) | (tag << kRecTagShift);
   return (unsigned long long)meta | ((unsigned long long)__float_as_uint(v) << 32);
 }
+// Two launches: slot in bits 0..15, count in bits 16..22, no tag.
+__device__ __forceinline__ unsigned long long make_wide_rec(uint32_t slot, uint32_t count, float v) {
+  return (unsigned long long)(slot | (count << 16)) | ((unsigned long long)__float_as_uint(v) << 32);
+}
+__device__ __forceinline__ int wide_slot(uint32_t meta) { return (int)(meta & 0xffffu); }
+__device__ __forceinline__ int wide_count(uint32_t meta) { return (int)(meta >> 16); }
+static_assert(kMaxOwnKeys <= 0x10000, "a record's slot has 16 bits");
 __device__ __forceinline__ int rec_slot(uint32_t meta) { return (int)(meta & 63u); }
 __device__ __forceinline__ int rec_count(uint32_t meta) { return (int)((meta >> kRecCountShift) & 127u); }
 __device__ __forceinline__ uint32_t rec_tag(uint32_t meta) { return meta >> kRecTagShift; }
@@ -54,7 +63,7 @@ __device__ __forceinline__ uint32_t rec_tag(uint32_t meta) { return meta >> kRec
 struct ReduceGeom {
   int K;          // keys of the table, key = cell * A + action
   int a_shift;    // log2(A)
-  int own_shift;  // log2(number of owners); owners = 1 << own_shift, (K >> own_shift) <= 64
+  int own_shift;  // log2(number of owners); an owner has (whole rows of) K >> own_shift keys or a row more
   int n_blocks;   // ceil(n / 256)
   int cell_shift; // log2(records of a hand-off cell), cell_shift_for(own_shift)
   int main_shift; // one-launch kernel: log2(records in the part of a cell that is written every step), main_shift_for()
@@ -147,25 +156,29 @@ __device__ __forceinline__ void st_dev128(DevWindow w, uint32_t byte_offset, con
 }
 __device__ __forceinline__ void poll_fence() { asm volatile("" ::: "memory"); }
 
-struct alignas(16) ReduceLds {  // (lead and members are also accessed 16 bytes at a time)
-  alignas(16) uint32_t lead[kDenseKeys];                     // lowest thread of the block that holds the key; kNoLead between uses
+// `Entries` = entries of the table in which the leader of a key is found: one per key of
+// the table, or (kHashSlots) one per distinct key of the block, found by hashing.
+template <int Entries>
+struct alignas(16) ReduceLdsT {  // (lead and members are also accessed 16 bytes at a time)
+  alignas(16) uint32_t lead[Entries];                        // lowest thread of the block that holds the key; kNoLead between uses
   alignas(16) unsigned long long members[kBlockSamples][4];  // per leader: the threads that hold its key; zero between uses
   float delta[kBlockSamples];
-  int handed[256];                               // block sums handed to each owner
+  int handed[256];                               // block sums handed to each owner (one-launch kernel)
   int over;                                      // some owner was handed more than a cell holds
 };
+using ReduceLds = ReduceLdsT<kDenseKeys>;
 
 // Besides ReduceLds, reduce_block() needs kSortBytes of LDS for `sorted`: the deltas of a
 // key's further holders, lined up for its leader ([place among the holders][leader]).
 constexpr int kSortRows = 32;
 constexpr size_t kSortBytes = (size_t)kSortRows * kBlockSamples * sizeof(float);
-constexpr size_t kReduceLdsBytes = sizeof(ReduceLds) + kSortBytes;  // ReduceLds, then `sorted`
 
 // Once per kernel, before the first reduce_block() and separated from it by a barrier.
-__device__ __forceinline__ void reduce_block_init(ReduceLds& L) {
+template <int Entries>
+__device__ __forceinline__ void reduce_block_init(ReduceLdsT<Entries>& L) {
   const int tid = threadIdx.x;
   uint4* lead4 = reinterpret_cast<uint4*>(L.lead);
-  for (int i = tid; i < kDenseKeys / 4; i += kBlockSamples) lead4[i] = make_uint4(kNoLead, kNoLead, kNoLead, kNoLead);
+  for (int i = tid; i < Entries / 4; i += kBlockSamples) lead4[i] = make_uint4(kNoLead, kNoLead, kNoLead, kNoLead);
   L.members[tid][0] = 0ull;
   L.members[tid][1] = 0ull;
   L.members[tid][2] = 0ull;
@@ -173,52 +186,25 @@ __device__ __forceinline__ void reduce_block_init(ReduceLds& L) {
   if (tid == 0) L.over = 0;
 }
 
-// Pass 1 for one block.  All 256 threads of the workgroup call it with their
-// sample (valid = false: no sample / no delta); key < K <= kDenseKeys.  Leaves the
-// LDS state as reduce_block_init() did, so it can be called again and again.
-// DEV = false: the records go straight to memory with plain stores, for a reader in a
-// later launch; the cell of (owner, block) is at handoff[(owner * blocks + block) << cell_shift],
-// so that an owner reads its cells side by side.
-// DEV = true: for readers on other XCDs in the same launch.  All cells of the block
-// main halves are put together in LDS (`stage`, owners << main_shift records, free again
-// on return) and go out as whole lines (that of (block, owner) at (block * owners + owner)
-// << main_shift behind `window_offset`), 16 bytes to a store and lane, every record
-// carrying `tag`; a record beyond the main half goes straight to
-// ext[(owner * blocks + block) << main_shift]:
-// scattered 8-byte stores are partial line writes, and some 350 of them per workgroup
-// took 1.6 us to be acknowledged.  `window` is a buffer window on `handoff`.
-// Returns (to every thread) whether some owner was handed more distinct keys than a
-// cell has records: its cell then says kSlotOverflow and the owner needs the block's
-// raw samples.
-// DEV = true: before each reduce_block(), separated from it by a barrier (and from the
-// one before by another): every record of every cell starts as "nothing, of this step".
-// Thread t touches the 16-byte pieces t, t + 256, ... of `stage` here and on the way out
-// of reduce_block(), and no others.
-__device__ __forceinline__ void reduce_stage_init(unsigned long long* stage, const ReduceGeom G, const uint32_t tag) {
-  const unsigned long long none = make_rec(0u, 0u, tag, 0.0f);
-  ulonglong2* stage2 = reinterpret_cast<ulonglong2*>(stage);
-  for (int i = threadIdx.x; i < 1 << (G.main_shift - 1 + G.own_shift); i += kBlockSamples) stage2[i] = make_ulonglong2(none, none);
-}
-
-template <bool DEV>
-__device__ __forceinline__ bool reduce_block(ReduceLds& L, const ReduceGeom G, const int block,
-                                             const int key, const float delta, const bool valid,
-                                             unsigned long long* handoff, const uint32_t tag, float* sorted,
-                                             unsigned long long* stage = nullptr, const DevWindow* window = nullptr,
-                                             const uint32_t window_offset = 0, unsigned long long* ext = nullptr,
-                                             const bool elected = false) {
+// What both forms of pass 1 share: the ordered sum of each distinct key of a block, in its
+// leader.  All 256 threads call it with their sample (valid = false: none); `at` is the
+// key's entry of L.lead, where the caller has entered its thread with an atomic min.  On
+// return (behind a barrier that only the last lines of the function follow) *sum is the
+// leader's block sum, and L.lead and L.members are as reduce_block_init() left them, so it
+// can be called again and again.  -> whether this thread is a leader.
+// (Written without branches: one wave to a SIMD has nothing to hide them behind.  A thread
+// without a sample reads its own, empty member set; a thread that has nothing to line up
+// writes its delta where it already is.)
+template <int Entries, class Between>
+__device__ __forceinline__ bool block_sums(ReduceLdsT<Entries>& L, const int at, const float delta, const bool valid,
+                                           float* sorted, Between between, float* sum) {
   const int tid = threadIdx.x;
-  const int n_own = 1 << G.own_shift;
-  const int cap = 1 << G.cell_shift;  // records of a cell
-  const int cap_main = 1 << G.main_shift;  // DEV: of its main half
-  if (valid && !elected) atomicMin(&L.lead[key], (uint32_t)tid);  // (elected: the caller has done this already)
   L.delta[tid] = delta;
   __syncthreads();
-  L.handed[tid] = 0;  // (256 >= owners; the last call's readers are past the barrier above)
-  if (tid == 0) L.over = 0;
+  between();  // (what the last call left to its readers: they are past the barrier above)
   uint32_t ld = (uint32_t)tid;
   if (valid) {
-    ld = L.lead[key];
+    ld = L.lead[at];
     if (ld != (uint32_t)tid) atomicOr(&L.members[ld][tid >> 6], 1ull << (tid & 63));
   }
   __syncthreads();
@@ -228,9 +214,6 @@ __device__ __forceinline__ bool reduce_block(ReduceLds& L, const ReduceGeom G, c
   // leader's walk is loads from known addresses, several in flight, instead of one bit
   // scan, load and add after the other (envs that crowd on a few cells: 14 holders of
   // one key in most blocks, 1 us of such a walk).
-  // (Written without branches: one wave to a SIMD has nothing to hide them behind.  A thread
-  // without a sample reads its own, empty member set; a thread that has nothing to line up
-  // writes its delta where it already is.)
   const bool leader = valid && ld == (uint32_t)tid;
   unsigned long long mw[4];
   int holders;  // leader: the key's further holders
@@ -251,7 +234,6 @@ __device__ __forceinline__ bool reduce_block(ReduceLds& L, const ReduceGeom G, c
   }
   __syncthreads();
   float acc = 0.0f;
-  int slot = 0, owner = 0;
   if (leader) {
     acc = acc + delta;  // the leader is the key's first sample; the other holders come after it
     if (holders != 0) {
@@ -280,172 +262,522 @@ __device__ __forceinline__ bool reduce_block(ReduceLds& L, const ReduceGeom G, c
         }
       }
     }
-    L.lead[key] = kNoLead;
+    L.lead[at] = kNoLead;
+  }
+  *sum = acc;
+  return leader;
+}
+
+// Before each reduce_block(), separated from it by a barrier (and from the
+// one before by another): every record of every cell starts as "nothing, of this step".
+// Thread t touches the 16-byte pieces t, t + 256, ... of `stage` here and on the way out
+// of reduce_block(), and no others.
+__device__ __forceinline__ void reduce_stage_init(unsigned long long* stage, const ReduceGeom G, const uint32_t tag) {
+  const unsigned long long none = make_rec(0u, 0u, tag, 0.0f);
+  ulonglong2* stage2 = reinterpret_cast<ulonglong2*>(stage);
+  for (int i = threadIdx.x; i < 1 << (G.main_shift - 1 + G.own_shift); i += kBlockSamples) stage2[i] = make_ulonglong2(none, none);
+}
+
+// One-launch kernel: pass 1 for one block.  All 256 threads of the workgroup call it with
+// their sample (valid = false: no sample / no delta), having entered their thread number in
+// L.lead[key] with an atomic min; key < K <= kDenseKeys.  The main halves of all cells of the
+// block are put together in LDS (`stage`, owners << main_shift records, free again
+// on return) and go out as whole lines (that of (block, owner) at (block * owners + owner)
+// << main_shift behind `window_offset`), 16 bytes to a store and lane, every record
+// carrying `tag`; a record beyond the main half goes straight to
+// ext[(owner * blocks + block) << main_shift]:
+// scattered 8-byte stores are partial line writes, and some 350 of them per workgroup
+// took 1.6 us to be acknowledged.
+// Returns (to every thread) whether some owner was handed more distinct keys than a
+// cell has records: its cell then says kSlotOverflow and the owner needs the block's
+// raw samples.
+__device__ __forceinline__ bool reduce_block(ReduceLds& L, const ReduceGeom G, const int block,
+                                             const int key, const float delta, const bool valid,
+                                             const uint32_t tag, float* sorted,
+                                             unsigned long long* stage, const DevWindow window,
+                                             const uint32_t window_offset, unsigned long long* ext) {
+  const int tid = threadIdx.x;
+  const int n_own = 1 << G.own_shift;
+  const int cap = 1 << G.cell_shift;  // records of a cell
+  const int cap_main = 1 << G.main_shift;  // of its main half
+  float acc;
+  const bool leader = block_sums(L, key, delta, valid, sorted, [&] {
+    L.handed[tid] = 0;  // (256 owners)
+    if (tid == 0) L.over = 0;
+  }, &acc);
+  int slot = 0, owner = 0;
+  if (leader) {
     owner = owner_of(key, G);
     slot = atomicAdd(&L.handed[owner], 1);  // slot order is free: records carry the key
     if (slot >= cap) L.over = 1;
     // (record 0's count is added on the way out, when every leader has drawn its slot)
-    if (DEV && slot < cap_main) stage[(owner << G.main_shift) + slot] = make_rec((uint32_t)slot_of(key, G), 0u, tag, acc);
+    if (slot < cap_main) stage[(owner << G.main_shift) + slot] = make_rec((uint32_t)slot_of(key, G), 0u, tag, acc);
   }
   __syncthreads();
   const bool over = L.over != 0;
   // (behind the barrier: a barrier waits for the stores before it to be acknowledged)
-  if (DEV && leader && slot >= cap_main && slot < cap)
+  if (leader && slot >= cap_main && slot < cap)
     st_dev64(ext + ((((size_t)owner * G.n_blocks + block) << G.main_shift) + (slot - cap_main)),
              make_rec((uint32_t)slot_of(key, G), 0u, tag, acc));
 
-  if (DEV) {
-    // (the one-launch kernel always has 256 owners and main halves of 4 records: 512 pieces,
-    // two to a thread, both asked for before the first is used)
-    const ulonglong2* stage2 = reinterpret_cast<const ulonglong2*>(stage);
-    const int piece_shift = G.main_shift - 1;  // log2(pieces of a cell's main half)
-    const int pieces = n_own << piece_shift;
-    constexpr int kPer = kStagePieces / kBlockSamples;
-    static_assert(kPer == 2, "two pieces of the stage to a thread");
-    ulonglong2 v[kPer];
-    int c[kPer];
+  // (the one-launch kernel always has 256 owners and main halves of 4 records: 512 pieces,
+  // two to a thread, both asked for before the first is used)
+  const ulonglong2* stage2 = reinterpret_cast<const ulonglong2*>(stage);
+  const int piece_shift = G.main_shift - 1;  // log2(pieces of a cell's main half)
+  const int pieces = n_own << piece_shift;
+  constexpr int kPer = kStagePieces / kBlockSamples;
+  static_assert(kPer == 2, "two pieces of the stage to a thread");
+  ulonglong2 v[kPer];
+  int c[kPer];
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int i = tid + j * kBlockSamples;
-      v[j] = i < pieces ? stage2[i] : make_ulonglong2(0ull, 0ull);
-      c[j] = (i < pieces && (i & ((1 << piece_shift) - 1)) == 0) ? L.handed[i >> piece_shift] : 0;
-    }
+  for (int j = 0; j < kPer; ++j) {
+    const int i = tid + j * kBlockSamples;
+    v[j] = i < pieces ? stage2[i] : make_ulonglong2(0ull, 0ull);
+    c[j] = (i < pieces && (i & ((1 << piece_shift) - 1)) == 0) ? L.handed[i >> piece_shift] : 0;
+  }
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int i = tid + j * kBlockSamples;
-      v[j].x |= (unsigned long long)(uint32_t)(c[j] > cap ? kSlotOverflow : c[j]) << kRecCountShift;
-      if (i < pieces)
-        st_dev128(*window, window_offset + (uint32_t)((((size_t)block * n_own) << (G.main_shift + 3)) + (size_t)i * 16),
-                  make_uint4((uint32_t)v[j].x, (uint32_t)(v[j].x >> 32), (uint32_t)v[j].y, (uint32_t)(v[j].y >> 32)));
-    }
-  } else {
-    if (leader && slot < cap) {
-      uint32_t count = 0;
-      if (slot == 0) {
-        const int c = L.handed[owner];  // final: every leader has drawn its slot
-        count = (uint32_t)(c > cap ? kSlotOverflow : c);
-      }
-      handoff[((((size_t)owner * G.n_blocks) + block) << G.cell_shift) + slot] = make_rec((uint32_t)slot_of(key, G), count, tag, acc);
-    }
-    if (tid < n_own && L.handed[tid] == 0) handoff[(((size_t)tid * G.n_blocks) + block) << G.cell_shift] = make_rec(0u, 0u, tag, 0.0f);
+  for (int j = 0; j < kPer; ++j) {
+    const int i = tid + j * kBlockSamples;
+    v[j].x |= (unsigned long long)(uint32_t)(c[j] > cap ? kSlotOverflow : c[j]) << kRecCountShift;
+    if (i < pieces)
+      st_dev128(window, window_offset + (uint32_t)((((size_t)block * n_own) << (G.main_shift + 3)) + (size_t)i * 16),
+                make_uint4((uint32_t)v[j].x, (uint32_t)(v[j].x >> 32), (uint32_t)v[j].y, (uint32_t)(v[j].y >> 32)));
   }
   return over;
 }
 
-// Pass 1 over (key, delta) arrays already in memory.
-__global__ __launch_bounds__(kBlockSamples) void k_reduce_blocks(const ReduceGeom G,
-                                                                 const int32_t* __restrict__ key,
-                                                                 const float* __restrict__ delta,
-                                                                 const int n,
-                                                                 unsigned long long* __restrict__ handoff) {
-  extern __shared__ __align__(16) unsigned char lds_raw[];
-  ReduceLds& L = *reinterpret_cast<ReduceLds*>(lds_raw);
-  reduce_block_init(L);
-  const int i = blockIdx.x * kBlockSamples + threadIdx.x;
-  const int k = i < n ? key[i] : -1;
-  const bool valid = k >= 0;
-  const float d = valid ? delta[i] : 0.0f;
-  __syncthreads();
-  reduce_block<false>(L, G, blockIdx.x, valid ? k : 0, d, valid, handoff, 0u, reinterpret_cast<float*>(lds_raw + sizeof(ReduceLds)));
+// ---- two launches: pass 1 ---------------------------------------------------------------
+
+// Where the samples of an update come from: packed by the host (which has checked the
+// states), or left behind by k_step.
+struct PackedSamples {
+  const int32_t* key;    // s * A + a, or -1: an action outside [0, A)
+  const uint32_t* s2d;   // s' and, in the top bit, done
+  const float* r;
+  template <int A>
+  __device__ __forceinline__ void get(int i, int& k, int& s2, float& r_, bool& done) const {
+    k = key[i];
+    const uint32_t v = s2d[i];
+    r_ = r[i];
+    s2 = (int)(v & 0x7fffffffu);
+    done = (v >> 31) != 0u;
+  }
+};
+// transition left behind by k_step for k_update_* : (s, a, r, s', done)
+struct Transition {
+  int32_t* s;
+  int32_t* a;
+  float* r;
+  int32_t* s2;
+  uint8_t* done;
+  template <int A>
+  __device__ __forceinline__ void get(int i, int& k, int& s2_, float& r_, bool& done_) const {
+    const int ai = a[i];
+    k = (unsigned)ai < (unsigned)A ? s[i] * A + ai : -1;
+    s2_ = s2[i];
+    r_ = r[i];
+    done_ = done[i] != 0;
+  }
+};
+
+// (key, delta) of sample i of n against ONE table, all reads before any write; key = -1 and
+// delta = 0 without a sample or for an invalid action.
+template <int A, class Samples>
+__device__ __forceinline__ void sample_delta(const Samples& X, const int i, const int n, const float* __restrict__ Q,
+                                             const float lr, const float gamma, const int max_mode, int& k, float& d) {
+  k = -1;
+  d = 0.0f;
+  int s2 = 0;
+  float r = 0.0f;
+  bool done = false;
+  if (i < n) X.template get<A>(i, k, s2, r, done);
+  if (k >= 0) {
+    const float q = Q[k];
+    const Row<A> row2 = load_row<A>(Q + (size_t)s2 * A);
+    d = td_delta(q, r, row_max(row2, done, max_mode), lr, gamma);
+  }
 }
 
-// Pass 2: one workgroup per owner (64 keys).
-__global__ __launch_bounds__(256) void k_reduce_owners(const ReduceGeom G, float* __restrict__ Q,
-                                                        const int32_t* __restrict__ key,
-                                                        const float* __restrict__ delta, const int n,
-                                                        const unsigned long long* __restrict__ handoff) {
-  extern __shared__ __align__(16) float tile[];  // [kTileBlocks][64] block sums, then [16][64] group sums, then a word per thread
-  float* gsum = tile + kTileBlocks * kOwnKeys;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int owner = blockIdx.x;
-  float total = 0.0f;
-  // the table entry this lane will update: fetched now, needed last
-  const int my_key = key_of(owner, lane, G);
-  const float q_old = (wave == 0 && my_key < G.K) ? Q[my_key] : 0.0f;
+// The entry of `key` in a table of `mask` + 1 keys (-1: free) that has room for it.
+__device__ __forceinline__ int hash_enter(int* keys, const int mask, const int key) {
+  unsigned h = ((unsigned)key * 0x9E3779B1u) >> 16;
+  for (;;) {
+    h &= (unsigned)mask;
+    const int old = atomicCAS(&keys[h], -1, key);
+    if (old == -1 || old == key) return (int)h;
+    ++h;
+  }
+}
 
-  for (int b0 = 0; b0 < G.n_blocks; b0 += kTileBlocks) {
-    const int b = b0 + tid;
-    // the first eight records of the hand-off cell in one go: no load depends on
-    // another (a cell with more records has the rest fetched below, when it holds them)
-    uint4 cell[kMinCellRecs / 2];
-    const uint4* src = reinterpret_cast<const uint4*>(handoff + ((((size_t)owner * G.n_blocks) + b) << G.cell_shift));
-    if (b < G.n_blocks) {
-#pragma unroll
-      for (int i = 0; i < kMinCellRecs / 2; ++i) cell[i] = src[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < kMinCellRecs / 2; ++i) cell[i] = make_uint4(0, 0, 0, 0);
+// LDS of pass 1, then handed[owners] (block sums handed to each owner), then `sorted`.
+// A block's 256 keys at most in a table of 2048: a probe or two, also for the unluckiest
+// lane of a wave; tables of up to 2048 keys have an entry per key.
+struct BlockLds {
+  ReduceLdsT<kHashSlots> red;
+  int keys[kHashSlots];
+};
+inline __host__ __device__ size_t block_lds_bytes(int own_shift) {
+  return sizeof(BlockLds) + ((size_t)4 << own_shift) + kSortBytes;
+}
+
+// Before reduce_block_wide(), separated from it by a barrier.
+__device__ __forceinline__ void block_lds_init(unsigned char* lds, const ReduceGeom G) {
+  BlockLds& L = *reinterpret_cast<BlockLds*>(lds);
+  int* handed = reinterpret_cast<int*>(lds + sizeof(BlockLds));
+  reduce_block_init(L.red);
+  for (int i = threadIdx.x; i < kHashSlots; i += kBlockSamples) L.keys[i] = -1;
+  for (int i = threadIdx.x; i < 1 << G.own_shift; i += kBlockSamples) handed[i] = 0;
+}
+
+// Pass 1 for one block of 256 threads, once per launch.  The records go straight to memory,
+// for a reader in a later launch; the cell of (owner, block) is at
+// handoff[(owner * blocks + block) << cell_shift], so that an owner reads its cells side by side.
+__device__ __forceinline__ void reduce_block_wide(unsigned char* lds, const ReduceGeom G, const int block,
+                                                  const int key, const float delta, const bool valid,
+                                                  unsigned long long* handoff) {
+  BlockLds& L = *reinterpret_cast<BlockLds*>(lds);
+  int* handed = reinterpret_cast<int*>(lds + sizeof(BlockLds));
+  float* sorted = reinterpret_cast<float*>(lds + sizeof(BlockLds) + ((size_t)4 << G.own_shift));
+  const int tid = threadIdx.x;
+  const int cap = 1 << G.cell_shift;
+  int at = 0;
+  if (valid) {
+    at = G.K <= kHashSlots ? key : hash_enter(L.keys, kHashSlots - 1, key);
+    atomicMin(&L.red.lead[at], (uint32_t)tid);
+  }
+  float acc;
+  const bool leader = block_sums(L.red, at, delta, valid, sorted, [] {}, &acc);
+  int slot = 0, owner = 0;
+  if (leader) {
+    owner = owner_of(key, G);
+    slot = atomicAdd(&handed[owner], 1);  // slot order is free: records carry the key
+  }
+  __syncthreads();
+  if (leader && slot < cap) {
+    uint32_t count = 0;
+    if (slot == 0) {
+      const int c = handed[owner];  // final: every leader has drawn its slot
+      count = (uint32_t)(c > cap ? kSlotOverflow : c);
     }
-    // the tile is cleared by all threads side by side (a thread clearing its own row
-    // would put all 64 lanes of a store on the same LDS banks)
-    float4* tile4 = reinterpret_cast<float4*>(tile);
-#pragma unroll
-    for (int i = 0; i < kTileBlocks * kOwnKeys / 4 / 256; ++i) tile4[i * 256 + tid] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    __syncthreads();
-    const int c = rec_count(cell[0].x);
-    if (c != kSlotOverflow) {
-      float* row = tile + tid * kOwnKeys;
-      // (no branches: a record that is not there goes to a word that nobody reads)
-      float* none = gsum + 16 * kOwnKeys + tid;
-#pragma unroll
-      for (int i = 0; i < kMinCellRecs / 2; ++i) {
-        *(c > 2 * i ? &row[rec_slot(cell[i].x)] : none) = __uint_as_float(cell[i].y);
-        *(c > 2 * i + 1 ? &row[rec_slot(cell[i].z)] : none) = __uint_as_float(cell[i].w);
+    handoff[((((size_t)owner * G.n_blocks) + block) << G.cell_shift) + slot] =
+        make_wide_rec((uint32_t)slot_of(key, G), count, acc);
+  }
+  for (int o = tid; o < 1 << G.own_shift; o += kBlockSamples)
+    if (handed[o] == 0) handoff[(((size_t)o * G.n_blocks) + block) << G.cell_shift] = 0ull;
+}
+
+// Pass 1 over samples in memory (which may be the host's: each is read once).
+template <int A, class Samples>
+__global__ __launch_bounds__(kBlockSamples) void k_td_blocks(const ReduceGeom G, const Samples X, const int n,
+                                                             const float* __restrict__ Q, const float lr,
+                                                             const float gamma, const int max_mode,
+                                                             int32_t* __restrict__ key, float* __restrict__ delta,
+                                                             unsigned long long* __restrict__ handoff) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  const int i = blockIdx.x * kBlockSamples + threadIdx.x;
+  int k;
+  float d;
+  block_lds_init(lds_raw, G);
+  sample_delta<A>(X, i, n, Q, lr, gamma, max_mode, k, d);
+  if (i < n) {
+    key[i] = k;
+    delta[i] = d;
+  }
+  __syncthreads();
+  reduce_block_wide(lds_raw, G, blockIdx.x, k >= 0 ? k : 0, d, k >= 0, handoff);
+}
+
+// ---- two launches: pass 2 ---------------------------------------------------------------
+
+constexpr int kOwnerWaves = 16;  // at most
+constexpr int kTileKeys = 64;    // keys of an owner up to which a wave lays its group out as a tile
+// 32-bit words of LDS per wave of k_reduce_owners besides its row of group sums: the tile,
+// or the claims; and the list of 256 samples
+inline __host__ __device__ int owner_wave_words(int own_keys) {
+  return (own_keys <= kTileKeys ? kGroupBlocks * kTileKeys : own_keys) + kBlockSamples + kBlockSamples / 2;
+}
+inline __host__ __device__ size_t owners_lds_bytes(int waves, int own_keys) {
+  return ((size_t)(waves + 1) * own_keys + (size_t)waves * owner_wave_words(own_keys)) * 4;
+}
+
+// One workgroup per owner, one wave per group of 16 blocks (in turn where there are more
+// groups than waves): no barrier before the groups are added up.  With cells of 8 records a
+// lane has the 16 bytes it needs of all 16 cells in one load.
+// Owners with up to 64 keys (TILE): the wave lays the records out as a dense [block][key] tile
+// of 4 KB and adds its columns, a lane to a key, 16 loads in flight - the same time whatever
+// the records.  Owners with more keys: 16 blocks hand them some 20 records, so the work goes
+// by the records.  All that are left enter their block number with a minimum under their
+// key, the lowest block of each key adds its record to the key's sum and is done: as many
+// rounds as the most crowded key of the group has blocks, two or three when the keys are
+// spread, and never more than 16.
+// Measured, both launches of a step of a shared table: 65,536 envs on 64x64x4 10.5 us (four
+// waves of four groups each 12.5), 20,000 envs on 101x99x8 12.6 us and 65,536 on 128x128x8
+// 15.0 us (every owner scanning all samples for its range of keys: 40-60 and 164 us).
+// `sig`: tells the host that the launch before this one is through (block 0, at once).
+template <bool TILE>
+__global__ __launch_bounds__(kOwnerWaves * 64) void k_reduce_owners(const ReduceGeom G, const int own_keys,
+                                                                    float* __restrict__ Q,
+                                                                    const int32_t* __restrict__ key,
+                                                                    const float* __restrict__ delta, const int n,
+                                                                    const unsigned long long* __restrict__ handoff,
+                                                                    const HostSignal sig) {
+  extern __shared__ __align__(16) float sums[];  // [waves][own_keys] group sums, [own_keys] totals, the waves' own words
+  const int tid = threadIdx.x, n_threads = blockDim.x;
+  const int lane = tid & 63, wave = tid >> 6, n_waves = n_threads >> 6;
+  const int owner = blockIdx.x;
+  float* gs = sums + wave * own_keys;
+  float* total = sums + n_waves * own_keys;
+  float* own = total + own_keys + wave * owner_wave_words(own_keys);
+  float* tile = own;                                       // TILE: [16 blocks][64 keys]
+  uint32_t* claim = reinterpret_cast<uint32_t*>(own);      // else: [own_keys]
+  float* list_v = own + (TILE ? kGroupBlocks * kTileKeys : own_keys);
+  uint16_t* list_s = reinterpret_cast<uint16_t*>(list_v + kBlockSamples);
+  if (sig.flag && owner == 0 && tid == 0) __hip_atomic_store(sig.flag, sig.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  // the table entry this thread will update first: fetched now, needed last
+  const int key0 = tid < own_keys ? key_of(owner, tid, G) : G.K;
+  const float q0 = key0 < G.K ? Q[key0] : 0.0f;
+  for (int k = tid; k < own_keys; k += n_threads) total[k] = 0.0f;
+  auto wave_fence = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+
+  // block `blk` has more distinct keys for this owner than a cell holds: its part again,
+  // from the samples, the first holder of a key adding up all of them in order
+  auto from_samples = [&](int blk, auto put) {
+    int m = 0;
+    for (int j = 0; j < kBlockSamples; j += 64) {
+      const int i = blk * kBlockSamples + j + lane;
+      const int k = i < n ? key[i] : -1;
+      const bool mine = k >= 0 && owner_of(k, G) == owner;
+      const unsigned long long who = __builtin_amdgcn_ballot_w64(mine);
+      if (mine) {
+        const int at = m + __popcll(who & ((1ull << lane) - 1ull));
+        list_s[at] = (uint16_t)slot_of(k, G);
+        list_v[at] = delta[i];
       }
-      for (int i = kMinCellRecs / 2; 2 * i < c; ++i) {
-        const uint4 more = src[i];
-        row[rec_slot(more.x)] = __uint_as_float(more.y);
-        if (c > 2 * i + 1) row[rec_slot(more.z)] = __uint_as_float(more.w);
+      m += __popcll(who);
+    }
+    wave_fence();
+    for (int e = lane; e < m; e += 64) {
+      const int slot = list_s[e];
+      bool first = true;
+      for (int f = 0; f < e; ++f) first = first && list_s[f] != slot;
+      if (first) {
+        float acc = 0.0f;
+        for (int f = e; f < m; ++f)
+          if (list_s[f] == slot) acc = acc + list_v[f];
+        put(slot, acc);
       }
+    }
+    wave_fence();
+  };
+
+  const int n_groups = (G.n_blocks + kGroupBlocks - 1) / kGroupBlocks;
+  for (int g0 = 0; g0 < n_groups; g0 += n_waves) {
+    const int b0 = (g0 + wave) * kGroupBlocks;
+    const unsigned long long* cells = handoff + (((size_t)owner * G.n_blocks + b0) << G.cell_shift);
+    // lane l: records 2 (l & 3) and the next of block l >> 2
+    const int b = lane >> 2, pair = lane & 3;
+    uint4 rec = make_uint4(0, 0, 0, 0);
+    if (G.cell_shift == 3 && b0 + b < G.n_blocks) rec = reinterpret_cast<const uint4*>(cells)[lane];
+    if (TILE) {
+      float4* tile4 = reinterpret_cast<float4*>(tile);
+#pragma unroll
+      for (int i = 0; i < kGroupBlocks * kTileKeys / 4 / 64; ++i) tile4[i * 64 + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     } else {
-      // more distinct keys than slots: redo the block's part from its samples, in order
-      const int lo = b * kBlockSamples, hi = min(n, lo + kBlockSamples);
-      for (int i = lo; i < hi; ++i) {
-        const int k = key[i];
-        if (k >= 0 && owner_of(k, G) == owner) {
-          float& acc = tile[tid * kOwnKeys + slot_of(k, G)];
-          acc = acc + delta[i];
+      for (int k = lane; k < own_keys; k += 64) {
+        gs[k] = 0.0f;
+        claim[k] = kNoLead;
+      }
+    }
+    if (G.cell_shift == 3) {
+      const int c = wide_count((uint32_t)__builtin_amdgcn_mov_dpp((int)rec.x, 0x00, 0xf, 0xf, true));  // of the quad's lane 0
+      const bool over = c == kSlotOverflow;
+      bool has0 = !over && 2 * pair < c, has1 = !over && 2 * pair + 1 < c;
+      const int slot0 = wide_slot(rec.x), slot1 = wide_slot(rec.z);
+      const float v0 = __uint_as_float(rec.y), v1 = __uint_as_float(rec.w);
+      unsigned long long overs = __builtin_amdgcn_ballot_w64(over);
+      if (TILE) {
+        if (has0) tile[b * kTileKeys + slot0] = v0;
+        if (has1) tile[b * kTileKeys + slot1] = v1;
+        while (overs != 0ull) {
+          const int bb = __builtin_ctzll(overs) >> 2;
+          overs &= ~(0xfull << (4 * bb));
+          from_samples(b0 + bb, [&](int slot, float acc) { tile[bb * kTileKeys + slot] = acc; });
+        }
+      } else if (overs != 0ull) {  // (rare) block after block
+        for (int bb = 0; bb < kGroupBlocks; ++bb) {
+          if ((overs >> (4 * bb)) & 1ull) {
+            from_samples(b0 + bb, [&](int slot, float acc) { gs[slot] = gs[slot] + acc; });
+          } else if (b == bb) {
+            if (has0) gs[slot0] = gs[slot0] + v0;
+            if (has1) gs[slot1] = gs[slot1] + v1;
+          }
+          wave_fence();
+        }
+      } else {
+        while (__builtin_amdgcn_ballot_w64(has0 || has1) != 0ull) {  // (the lowest block of a key always gets through)
+          if (has0) atomicMin(&claim[slot0], (uint32_t)b);
+          if (has1) atomicMin(&claim[slot1], (uint32_t)b);
+          wave_fence();
+          const bool go0 = has0 && claim[slot0] == (uint32_t)b, go1 = has1 && claim[slot1] == (uint32_t)b;
+          wave_fence();
+          if (go0) {
+            gs[slot0] = gs[slot0] + v0;
+            claim[slot0] = kNoLead;
+          }
+          if (go1) {
+            gs[slot1] = gs[slot1] + v1;
+            claim[slot1] = kNoLead;
+          }
+          wave_fence();
+          has0 = has0 && !go0;
+          has1 = has1 && !go1;
         }
       }
-    }
-    __syncthreads();
-    // group sums: 16 groups of 16 blocks in this tile, four per wave; a lane takes four
-    // keys of one group (16 LDS loads of 16 bytes instead of 64 of 4)
-    {
-      const int grp = wave * 4 + (lane >> 4);
-      const float4* rows = reinterpret_cast<const float4*>(tile + grp * kGroupBlocks * kOwnKeys) + (lane & 15);
-      float4 v[kGroupBlocks];
-#pragma unroll
-      for (int bb = 0; bb < kGroupBlocks; ++bb) v[bb] = rows[bb * (kOwnKeys / 4)];
-      float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll
-      for (int bb = 0; bb < kGroupBlocks; ++bb) {
-        acc.x = acc.x + v[bb].x;
-        acc.y = acc.y + v[bb].y;
-        acc.z = acc.z + v[bb].z;
-        acc.w = acc.w + v[bb].w;
+    } else {  // few owners with large cells (and at most 64 keys each): lane l takes record l of one block after the other
+      for (int bb = 0; bb < kGroupBlocks && b0 + bb < G.n_blocks; ++bb) {
+        const unsigned long long r = lane < 1 << G.cell_shift ? cells[((size_t)bb << G.cell_shift) + lane] : 0ull;
+        const int c = wide_count((uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)r));
+        auto put = [&](int slot, float v) {
+          if (TILE) tile[bb * kTileKeys + slot] = v;
+          else gs[slot] = gs[slot] + v;
+        };
+        if (c == kSlotOverflow) from_samples(b0 + bb, put);
+        else if (lane < c) put(wide_slot((uint32_t)r), __uint_as_float((uint32_t)(r >> 32)));
       }
-      reinterpret_cast<float4*>(gsum + grp * kOwnKeys)[lane & 15] = acc;
+    }
+    if (TILE) {
+      wave_fence();
+      float v[kGroupBlocks];
+#pragma unroll
+      for (int bb = 0; bb < kGroupBlocks; ++bb) v[bb] = tile[bb * kTileKeys + lane];
+      float acc = 0.0f;
+#pragma unroll
+      for (int bb = 0; bb < kGroupBlocks; ++bb) acc = acc + v[bb];
+      if (lane < own_keys) gs[lane] = acc;
     }
     __syncthreads();
-    if (wave == 0) {
-#pragma unroll
-      for (int grp = 0; grp < kTileBlocks / kGroupBlocks; ++grp) total = total + gsum[grp * kOwnKeys + lane];
+    const int here = min(n_waves, n_groups - g0);
+    for (int k = tid; k < own_keys; k += n_threads) {
+      float t = total[k];
+      for (int w = 0; w < here; ++w) t = t + sums[w * own_keys + k];
+      total[k] = t;
     }
     __syncthreads();
   }
-  if (wave == 0 && my_key < G.K) Q[my_key] = q_old + total;
+  if (key0 < G.K) Q[key0] = q0 + total[tid];
+  for (int k = tid + n_threads; k < own_keys; k += n_threads) {
+    const int kk = key_of(owner, k, G);
+    if (kk < G.K) Q[kk] = Q[kk] + total[k];
+  }
 }
 
-// Fallback for tables with more than kDenseKeys keys (or too many blocks for the
-// hand-off buffer): one workgroup per 64 consecutive keys scans all samples,
+// ---- up to 1024 samples: one launch --------------------------------------------------------
+
+constexpr int kSmallSamples = 1024;
+// One workgroup, 256 threads to a block of the tree.  A key has one entry in LDS with a
+// leader per block; the leader of a key's first block adds the block sums (all in one
+// group) and applies them.  Costs one launch and a trip for the samples instead of two
+// launches with 256 owners, most of which are handed nothing.
+// `changed` (host memory, may be null): per sample {key, new value} where its thread applied
+// a total, {-1, 0} elsewhere.
+template <int NB>
+struct SmallLds {
+  static constexpr int kSlots = 512 * NB;
+  int keys[kSlots];
+  uint32_t lead[NB][kSlots];
+  unsigned long long members[NB * kBlockSamples][4];
+  float delta[NB * kBlockSamples];
+  float sum[NB * kBlockSamples];
+};
+template <int A, int NB, class Samples>
+__global__ __launch_bounds__(kBlockSamples* NB) void k_td_small(const Samples X, const int n, float* __restrict__ Q,
+                                                                const float lr, const float gamma, const int max_mode,
+                                                                int2* __restrict__ changed, const HostSignal sig) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  using Lds = SmallLds<NB>;
+  Lds& L = *reinterpret_cast<Lds*>(lds_raw);
+  const int tid = threadIdx.x, blk = tid >> 8;
+  int k;
+  float d;
+  sample_delta<A>(X, tid, n, Q, lr, gamma, max_mode, k, d);
+  for (int i = tid; i < Lds::kSlots; i += kBlockSamples * NB) {
+    L.keys[i] = -1;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) L.lead[b][i] = kNoLead;
+  }
+#pragma unroll
+  for (int w = 0; w < 4; ++w) L.members[tid][w] = 0ull;
+  L.delta[tid] = d;
+  __syncthreads();
+  const bool valid = k >= 0;
+  int at = 0;
+  if (valid) {
+    at = hash_enter(L.keys, Lds::kSlots - 1, k);
+    atomicMin(&L.lead[blk][at], (uint32_t)tid);
+  }
+  __syncthreads();
+  uint32_t ld = kNoLead;
+  if (valid) {
+    ld = L.lead[blk][at];
+    if (ld != (uint32_t)tid) atomicOr(&L.members[ld][(tid >> 6) & 3], 1ull << (tid & 63));
+  }
+  const bool leader = ld == (uint32_t)tid;
+  __syncthreads();
+  if (leader) {
+    float acc = 0.0f + d;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      unsigned long long m = L.members[tid][w];
+      const float* from = L.delta + blk * kBlockSamples + w * 64;
+      while (m != 0ull) {  // thread order = sample order, four loads in flight
+        float v[4];
+        int have = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v[j] = m != 0ull ? from[__builtin_ctzll(m)] : 0.0f;
+          have += m != 0ull ? 1 : 0;
+          m &= m - 1ull;  // (0 stays 0)
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (j < have) acc = acc + v[j];
+      }
+    }
+    L.sum[tid] = acc;
+  }
+  __syncthreads();  // (also: every thread has read the table)
+  int2 out = make_int2(-1, 0);
+  if (leader) {
+    bool first = true;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) first = first && (b >= blk || L.lead[b][at] == kNoLead);
+    if (first) {
+      float group = 0.0f;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const uint32_t l = L.lead[b][at];
+        if (l != kNoLead) group = group + L.sum[l];
+      }
+      const float q = Q[k] + (0.0f + group);
+      Q[k] = q;
+      out = make_int2(k, __float_as_int(q));
+    }
+  }
+  if (changed && tid < n) changed[tid] = out;
+  signal_host(sig);
+}
+
+// Fallback for what needs too many owners or too large a hand-off buffer: one workgroup per 64 consecutive keys scans all samples,
 // group by group (4096 samples), compacting its matches in order, and wave 0
 // then folds them through the same tree.  Slow, same result.
 __global__ __launch_bounds__(256) void k_reduce_scan(float* __restrict__ Q, const int K,
                                                       const int32_t* __restrict__ key,
-                                                      const float* __restrict__ delta, const int n) {
+                                                      const float* __restrict__ delta, const int n,
+                                                      const HostSignal sig) {
   constexpr int kSpan = 1024;  // samples one wave scans per group: 4 blocks
   __shared__ float l_d[4][kSpan];
   __shared__ uint8_t l_k[4][kSpan];
@@ -456,6 +788,7 @@ __global__ __launch_bounds__(256) void k_reduce_scan(float* __restrict__ Q, cons
   const int wave = tid >> 6;
   const int owner = blockIdx.x;
   float total = 0.0f;
+  if (sig.flag && owner == 0 && tid == 0) __hip_atomic_store(sig.flag, sig.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 
   for (int g0 = 0; g0 < n; g0 += 4 * kSpan) {
     int cnt = 0;

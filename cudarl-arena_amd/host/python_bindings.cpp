@@ -5,6 +5,7 @@
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
 
+#include <climits>
 #include <cstring>
 #include <memory>
 #include <stdexcept>
@@ -16,6 +17,65 @@
 #include "q_learning.h"
 
 namespace py = pybind11;
+
+// Arguments of update_batch.  A list of exact ints / floats / bools / 2-tuples of ints is
+// read item by item straight into its array (256 transitions: 5 us; the generic casters
+// build and destroy a caster per element); anything else takes the generic caster, with
+// its conversions and its errors.
+struct PairList { std::vector<std::pair<int, int>> v; };
+struct IntList { std::vector<int> v; };
+struct FloatList { std::vector<float> v; };
+struct BoolList { std::vector<uint8_t> v; };
+
+inline bool exact_int(PyObject* o, int& out) {
+  if (!PyLong_CheckExact(o)) return false;
+  int overflow = 0;
+  const long v = PyLong_AsLongAndOverflow(o, &overflow);
+  if (overflow != 0 || v < INT_MIN || v > INT_MAX) return false;
+  out = (int)v;
+  return true;
+}
+inline bool exact_item(PyObject* o, int& out) { return exact_int(o, out); }
+inline bool exact_item(PyObject* o, float& out) {
+  if (!PyFloat_CheckExact(o)) return false;
+  out = (float)PyFloat_AS_DOUBLE(o);
+  return true;
+}
+inline bool exact_item(PyObject* o, uint8_t& out) {
+  out = o == Py_True ? 1 : 0;
+  return o == Py_True || o == Py_False;
+}
+inline bool exact_item(PyObject* o, std::pair<int, int>& out) {
+  return PyTuple_CheckExact(o) && PyTuple_GET_SIZE(o) == 2 && exact_int(PyTuple_GET_ITEM(o, 0), out.first) &&
+         exact_int(PyTuple_GET_ITEM(o, 1), out.second);
+}
+
+namespace pybind11 {
+namespace detail {
+template <class List, class Generic>
+struct list_reader {
+  PYBIND11_TYPE_CASTER(List, make_caster<Generic>::name);
+  bool load(handle src, bool convert) {
+    if (PyList_CheckExact(src.ptr())) {
+      const Py_ssize_t n = PyList_GET_SIZE(src.ptr());
+      value.v.resize((size_t)n);
+      bool exact = true;
+      for (Py_ssize_t i = 0; i < n && exact; ++i) exact = exact_item(PyList_GET_ITEM(src.ptr(), i), value.v[(size_t)i]);
+      if (exact) return true;
+    }
+    make_caster<Generic> generic;
+    if (!generic.load(src, convert)) return false;
+    const Generic& g = cast_op<const Generic&>(generic);
+    value.v.assign(g.begin(), g.end());
+    return true;
+  }
+};
+template <> struct type_caster<PairList> : list_reader<PairList, std::vector<std::pair<int, int>>> {};
+template <> struct type_caster<IntList> : list_reader<IntList, std::vector<int>> {};
+template <> struct type_caster<FloatList> : list_reader<FloatList, std::vector<float>> {};
+template <> struct type_caster<BoolList> : list_reader<BoolList, std::vector<bool>> {};
+}  // namespace detail
+}  // namespace pybind11
 
 namespace {
 
@@ -162,8 +222,24 @@ PYBIND11_MODULE(cudarl_core, m) {
       .def(py::init<int, int, int, float, float, int>(), py::arg("width"), py::arg("height"),
            py::arg("action_space_size"), py::arg("learning_rate") = 0.1f,
            py::arg("discount_factor") = 0.99f, py::arg("max_mode") = 1)
-      .def("update_batch", &CudaQLearning::update_batch)
-      .def("get_q_table", &CudaQLearning::get_q_table)
+      .def("update_batch",
+           [](CudaQLearning& self, const PairList& states, const IntList& actions, const FloatList& rewards,
+              const PairList& next_states, const BoolList& dones) {
+             self.update_batch(states.v.data(), states.v.size(), actions.v.data(), actions.v.size(), rewards.v.data(),
+                               rewards.v.size(), next_states.v.data(), next_states.v.size(), dones.v.data(),
+                               dones.v.size());
+           })
+      .def("get_q_table",
+           [](const CudaQLearning& self) {
+             const std::vector<float>& q = self.q_values();
+             py::list out(q.size());
+             for (size_t i = 0; i < q.size(); ++i) {
+               PyObject* f = PyFloat_FromDouble((double)q[i]);
+               if (!f) throw py::error_already_set();
+               PyList_SET_ITEM(out.ptr(), (Py_ssize_t)i, f);
+             }
+             return out;
+           })
       .def("set_q_table", &CudaQLearning::set_q_table)
       .def("get_best_action", &CudaQLearning::get_best_action)
       .def("get_q_value", &CudaQLearning::get_q_value);

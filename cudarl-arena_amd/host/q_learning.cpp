@@ -47,15 +47,25 @@ void CudaQLearning::update_batch(const std::vector<std::pair<int, int>>& states,
                                  const std::vector<int>& actions, const std::vector<float>& rewards,
                                  const std::vector<std::pair<int, int>>& next_states,
                                  const std::vector<bool>& dones) {
-  const size_t batch_size = states.size();
+  std::vector<uint8_t> d(dones.size());
+  for (size_t i = 0; i < dones.size(); ++i) d[i] = dones[i] ? 1 : 0;
+  update_batch(states.data(), states.size(), actions.data(), actions.size(), rewards.data(), rewards.size(),
+               next_states.data(), next_states.size(), d.data(), d.size());
+}
+
+void CudaQLearning::update_batch(const std::pair<int, int>* states, size_t batch_size, const int* actions,
+                                 size_t n_actions, const float* rewards, size_t n_rewards,
+                                 const std::pair<int, int>* next_states, size_t n_next, const uint8_t* dones,
+                                 size_t n_dones) {
   if (batch_size > (size_t)max_batch_size)  // src/q_learning.cu:117-119
     throw std::runtime_error("Batch size exceeds maximum batch size");
-  if (batch_size != actions.size() || batch_size != rewards.size() || batch_size != next_states.size() ||
-      batch_size != dones.size())  // src/q_learning.cu:121-124
+  if (batch_size != n_actions || batch_size != n_rewards || batch_size != n_next ||
+      batch_size != n_dones)  // src/q_learning.cu:121-124
     throw std::runtime_error("Inconsistent batch sizes");
   if (batch_size == 0) return;
-  std::vector<int32_t> s(batch_size), a(batch_size), s2(batch_size);
-  std::vector<uint8_t> d(batch_size);
+  batch.resize(4 * batch_size);
+  changed.resize(batch_size);
+  int32_t *s = batch.data(), *s2 = s + batch_size, *a = s2 + batch_size, *keys = a + batch_size;
   for (size_t i = 0; i < batch_size; ++i) {
     const int x = states[i].first, y = states[i].second;
     const int nx = next_states[i].first, ny = next_states[i].second;
@@ -67,13 +77,12 @@ void CudaQLearning::update_batch(const std::vector<std::pair<int, int>>& states,
     s[i] = y * width + x;  // src/kernels.cu:96
     s2[i] = ny * width + nx;
     a[i] = actions[i];
-    d[i] = dones[i] ? 1 : 0;
   }
-  if (crl_td_update(engine, 0, (int32_t)batch_size, s.data(), a.data(), rewards.data(), s2.data(), d.data()) != CRL_OK)
+  if (crl_td_update_collect(engine, 0, (int32_t)batch_size, s, a, rewards, s2, dones, keys, changed.data()) != CRL_OK)
     throw std::runtime_error(std::string("update_batch: ") + crl_last_error());
   // src/q_learning.cu:173: the host mirror follows every update
-  if (crl_q_get(engine, 0, h_q_table.data()) != CRL_OK)
-    throw std::runtime_error(std::string("update_batch: ") + crl_last_error());
+  for (size_t i = 0; i < batch_size; ++i)
+    if (keys[i] >= 0) h_q_table[(size_t)keys[i]] = changed[i];
 }
 
 std::vector<float> CudaQLearning::get_q_table() const { return h_q_table; }

@@ -1,6 +1,8 @@
 // CudaQLearning: the reference's tabular Q-learning host class
 // (src/q_learning.cuh:8-95), same public signatures, on the HIP engine.
 #pragma once
+#include <cstddef>
+#include <cstdint>
 #include <utility>
 #include <vector>
 
@@ -23,7 +25,13 @@ class CudaQLearning {
                     const std::vector<float>& rewards,
                     const std::vector<std::pair<int, int>>& next_states,
                     const std::vector<bool>& dones);
+  // the same from arrays, each with its length
+  void update_batch(const std::pair<int, int>* states, size_t batch_size, const int* actions, size_t n_actions,
+                    const float* rewards, size_t n_rewards, const std::pair<int, int>* next_states, size_t n_next,
+                    const uint8_t* dones, size_t n_dones);
   std::vector<float> get_q_table() const;
+  // the same without a copy; valid until the next call that changes the table
+  const std::vector<float>& q_values() const { return h_q_table; }
   void set_q_table(const std::vector<float>& q_table);
   int get_best_action(int x, int y) const;
   float get_q_value(int x, int y, int action) const;
@@ -37,4 +45,6 @@ class CudaQLearning {
   std::vector<float> h_q_table;  // host mirror, refreshed after every update
   crl_engine* engine;
   int max_batch_size;
+  std::vector<int32_t> batch;  // scratch of update_batch: s, s', a, changed keys
+  std::vector<float> changed;  // ... and their new values
 };

@@ -86,7 +86,7 @@ _lib = None
 EXPORTS = [
     "crl_last_error", "crl_version", "crl_device_count", "crl_create", "crl_destroy",
     "crl_set_stream", "crl_sync", "crl_set_resident_envs", "crl_set_fused_variant", "crl_get_fused_split", "crl_set_maps", "crl_set_cell", "crl_classify_grid", "crl_reset",
-    "crl_step", "crl_select", "crl_update", "crl_td_update", "crl_run_fused", "crl_run_fused_noalloc", "crl_get_state",
+    "crl_step", "crl_select", "crl_update", "crl_td_update", "crl_td_update_collect", "crl_run_fused", "crl_run_fused_noalloc", "crl_get_state",
     "crl_set_state", "crl_get_episode_stats", "crl_get_step_count", "crl_set_step_count", "crl_q_get", "crl_q_set",
     "crl_q_get_range", "crl_set_trace", "crl_get_trace", "crl_set_exploration_stream", "crl_set_persist_spin_limit",
     "crl_device_ptr", "crl_fused_kernel_info", "crl_fused_plan_for_config", "crl_philox4x32_10", "crl_explore_draw",
@@ -121,6 +121,7 @@ def load():
     lib.crl_select.argtypes = [vp, vp]
     lib.crl_update.argtypes = [vp]
     lib.crl_td_update.argtypes = [vp, i32, i32, vp, vp, vp, vp, vp]
+    lib.crl_td_update_collect.argtypes = [vp, i32, i32, vp, vp, vp, vp, vp, vp, vp]
     lib.crl_run_fused.argtypes = [vp, i32]
     lib.crl_run_fused_noalloc.argtypes = [vp, i32]
     lib.crl_get_state.argtypes = [vp, vp, vp, vp, vp, vp, vp]
@@ -287,6 +288,19 @@ class Engine:
         if not (a.size == r.size == s2.size == d.size == n):
             raise ValueError("Inconsistent batch sizes")
         _check(self.lib.crl_td_update(self.h, table, n, _ptr(s), _ptr(a), _ptr(r), _ptr(s2), _ptr(d)))
+
+    def td_update_collect(self, table, s, a, r, s_next, done):
+        """td_update of at most 1024 transitions -> (keys, values) of the entries it changed
+        (key -1: none)."""
+        s, a = _arr(s, np.int32), _arr(a, np.int32)
+        r, s2, d = _arr(r, np.float32), _arr(s_next, np.int32), _arr(done, np.uint8)
+        n = s.size
+        if not (a.size == r.size == s2.size == d.size == n):
+            raise ValueError("Inconsistent batch sizes")
+        keys, values = np.empty(n, np.int32), np.empty(n, np.float32)
+        _check(self.lib.crl_td_update_collect(self.h, table, n, _ptr(s), _ptr(a), _ptr(r), _ptr(s2), _ptr(d),
+                                              _ptr(keys), _ptr(values)))
+        return keys, values
 
     def run_fused(self, n_steps):
         _check(self.lib.crl_run_fused(self.h, n_steps))

@@ -197,6 +197,15 @@ int crl_update(crl_engine* e);
 int crl_td_update(crl_engine* e, int32_t table, int32_t n, const int32_t* s, const int32_t* a,
                   const float* r, const int32_t* s_next, const uint8_t* done);
 
+/* The same for at most 1024 transitions, and what it changed: for every sample i either
+ * keys[i] = s*A + a and values[i] = the new Q of that entry, or keys[i] = -1; every entry
+ * that the call changed is named by exactly one sample.  Lets a caller that keeps a
+ * host copy of the table (h_q_table, src/q_learning.cu:173) follow it without fetching the
+ * whole table. */
+int crl_td_update_collect(crl_engine* e, int32_t table, int32_t n, const int32_t* s, const int32_t* a,
+                          const float* r, const int32_t* s_next, const uint8_t* done, int32_t* keys,
+                          float* values);
+
 /* n_steps of select -> step -> update for every env, fused on the device
  * (the loop body of src/train.py:198-222).  Same results as n_steps rounds of
  * crl_select; crl_step(NULL); crl_update. */
