@@ -165,6 +165,11 @@ __device__ __forceinline__ Row<8> load_row8(const float* __restrict__ p) {
   const float4 u = reinterpret_cast<const float4*>(p)[1];
   return Row<8>{t.x, t.y, t.z, t.w, u.x, u.y, u.z, u.w};
 }
+__device__ __forceinline__ void store_row(float* p, const Row<4> r) { *reinterpret_cast<float4*>(p) = make_float4(r.q0, r.q1, r.q2, r.q3); }
+__device__ __forceinline__ void store_row(float* p, const Row<8> r) {
+  reinterpret_cast<float4*>(p)[0] = make_float4(r.q0, r.q1, r.q2, r.q3);
+  reinterpret_cast<float4*>(p)[1] = make_float4(r.q4, r.q5, r.q6, r.q7);
+}
 template <int A>
 __device__ __forceinline__ Row<A> load_row(const float* __restrict__ p);
 template <>

@@ -320,10 +320,13 @@ struct FusedPlan {
   bool fast;       // the folded loop for the common configuration
   bool moves;      // ... whose table waves read pre-built move codes from LDS
   bool fixed;      // tickets dealt by position, round after round: no counter
-  bool pair;       // per-env kernel: two lanes per env
-  int pair_envs;   // ticket kernel: envs per thin table wave (32, 16, 8), 0: 64-env waves
+  bool lanes;      // an env to A lanes, a wave to 2^log_envs envs, draws taped tape_steps ahead
+  int log_envs, tape_steps;
   bool rich;       // ticket kernel: the folded loop's variant with per-cell rewards / per-episode epsilon
   int tab_stride;  // floats between two tables in LDS
+  bool in_lds;     // ... with all tables in LDS
+  bool words;      // ... beside their move words
+  int env_bytes;   // ... bytes per env
 };
 
 constexpr size_t kLdsPerWorkgroup = 160 * 1024;  // gfx950
@@ -336,9 +339,67 @@ constexpr size_t kStaticLdsReserve = 1024;
 // 32: 2.4e10 / 2.1e10, 48: 2.8e10 / 2.75e10, 64: 3.0e10 / 3.3e10, 100: 3.6e10 / 4.2e10).
 constexpr int kHybridMinSteps = 64;
 constexpr int kStagedMovesMinSteps = 128;
+constexpr int kLdsMinSteps = 16;
+constexpr int kLongLaunchSteps = 4096;
+
+// Configurations that run_lanes() steps: no goal test on the resulting cell, no sticky done,
+// no trace and no supplied stream.
+bool lanes_rules(const crl_engine* e) {
+  const crl_config& c = e->cfg;
+  return c.goal_mode == CRL_GOAL_ON_TARGET && c.auto_reset == 1 && e->trace_n == 0 && e->sup_n == 0;
+}
+// steps of a tape: enough that all 64 lanes have a Philox block to work out
+int tape_steps_for(int log_envs) { return std::max(16, 128 >> log_envs); }
+size_t tape_bytes(int log_envs) { return ((size_t)(tape_steps_for(log_envs) + 1) << log_envs) * 4; }
+// as few envs to a wave as leaves no more than `waves` of them, and as many as it has lanes for
+int lanes_log_envs(const crl_engine* e, long waves) {
+  const int most = e->A == 8 ? 3 : 4;
+  int log_envs = 0;
+  while (log_envs < most && ((long)e->N + (1L << log_envs) - 1) >> log_envs > waves) ++log_envs;
+  return log_envs;
+}
+
+// All tables in LDS, if they fit there with the envs spread over every SIMD of the chip.
+// Not for launches so short that moving the tables in and out costs more than it saves.
+bool plan_fused_lds(const crl_engine* e, int n_steps, FusedPlan* p) {
+  const crl_config& c = e->cfg;
+  if (!lanes_rules(e) || c.reward_flags != 0 || e->fused_variant != 0 || e->resident_envs != 0 || n_steps < kLdsMinSteps)
+    return false;
+  const bool shared = c.map_mode == CRL_MAP_SHARED;
+  if (!shared && (size_t)e->map_words * 4 * 64 > (size_t)kLdsMapLimitBytes) return false;
+  const int log_envs = lanes_log_envs(e, 4L * kComputeUnits);
+  const long waves = ((long)e->N + (1L << log_envs) - 1) >> log_envs;
+  const size_t per_unit = (size_t)((waves + kComputeUnits - 1) / kComputeUnits);
+  // (an env's pieces in whole rows of 16 bytes, and a row more against bank conflicts)
+  const size_t code_bytes = (size_t)e->mv_words * 4;
+  const size_t env_bytes[2] = {((4 * e->K + (shared ? 0 : code_bytes) + 15) & ~(size_t)15) + 16, 8 * e->K + 16};
+  for (int words = 1; words >= 0; --words) {
+    const size_t bytes = 16 + (env_bytes[words] << log_envs) + tape_bytes(log_envs) + (shared && !words ? code_bytes : 0);
+    if (((bytes + 1023) & ~(size_t)1023) * per_unit > kLdsPerWorkgroup) continue;
+    p->in_lds = p->lanes = p->fast = true;
+    p->words = words != 0;
+    p->rich = c.eps_mode >= CRL_EPS_EPISODE_MULT;
+    p->log_envs = log_envs;
+    p->tape_steps = tape_steps_for(log_envs);
+    p->env_bytes = (int)env_bytes[words];
+    p->block = 64;
+    p->grid = (int)waves;
+    p->lds = bytes;
+    p->map_kind = shared ? 1 : 0;
+    static const char* names[2][2][2] = {
+        {{"k_fused_tickets_lds<4,fast>", "k_fused_tickets_lds<4,fast+>"},
+         {"k_fused_per_env_lds<4,fast>", "k_fused_per_env_lds<4,fast+>"}},
+        {{"k_fused_tickets_lds<8,fast>", "k_fused_tickets_lds<8,fast+>"},
+         {"k_fused_per_env_lds<8,fast>", "k_fused_per_env_lds<8,fast+>"}}};
+    p->name = names[e->A == 8][shared][p->rich];
+    return true;
+  }
+  return false;
+}
 
 FusedPlan plan_fused(const crl_engine* e, int n_steps) {
   FusedPlan p{};
+  if (plan_fused_lds(e, n_steps, &p)) return p;
   // small batches spread over more compute units with one-wave blocks
   p.block = e->N >= 256 * 512 ? 256 : 64;
   if (e->cfg.map_mode == CRL_MAP_SHARED) {
@@ -390,10 +451,19 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     p.grid = (int)std::min<long>((e->N + p.block - 1) / p.block, std::max<long>(1, resident / p.block));
     // ... its variant for large or shared maps takes per-cell rewards and per-episode epsilon
     p.fast = foldable && c.eps_mode != CRL_EPS_STEP_MULT && c.table_mode != CRL_TABLE_SHARED;
-    // two lanes per env while that still leaves the batch with at most two waves per
-    // compute unit (config 5 with 8192 / 16,384 / 32,768 envs: +4 % / +6 % / -4 %)
-    p.pair = p.fast && (e->N + 63) / 64 <= kComputeUnits;
-    if (p.pair) p.grid = (int)std::min<long>((e->N + p.block / 2 - 1) / (p.block / 2), std::max<long>(1, 2 * resident / p.block));
+    // An env to A lanes while that leaves the chip a wave or two per SIMD.
+    const int log_envs = lanes_log_envs(e, 4L * kComputeUnits);
+    const long waves = ((long)e->N + (1L << log_envs) - 1) >> log_envs;
+    if (lanes_rules(e) && c.table_mode != CRL_TABLE_SHARED && (e->N + 63) / 64 <= kComputeUnits && resident >= e->N &&
+        (e->K * sizeof(float)) << log_envs < (size_t)1 << 32) {
+      p.fast = p.lanes = true;
+      p.log_envs = log_envs;
+      p.tape_steps = tape_steps_for(log_envs);
+      const int per_block = waves > 2 * kComputeUnits ? 4 : waves > kComputeUnits ? 2 : 1;
+      p.block = 64 * per_block;
+      p.grid = (int)((waves + per_block - 1) / per_block);
+      p.lds = 16 + per_block * tape_bytes(log_envs) + (p.map_kind == 1 ? (size_t)e->mv_words * 4 : 0);
+    }
   } else {
     p.rich = foldable && c.eps_mode != CRL_EPS_STEP_MULT && !(c.eps_mode == CRL_EPS_FIXED && c.reward_flags == 0);
     p.fast = foldable && c.eps_mode != CRL_EPS_STEP_MULT;
@@ -447,26 +517,34 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       // staging the codes (four times the class map) pays off over a long launch only:
       // 1M envs of config 4, one step per launch 7.7e9 -> 1.4e10 with class maps, 48 steps 3.6e10 -> 3.7e10
       p.moves = p.fast && waves * mv_lds <= kLdsPerWorkgroup && n_steps >= kStagedMovesMinSteps;
-      // Few enough envs that 32-env waves still find a SIMD each: one ticket per wave,
-      // two lanes per env - half the distinct addresses per request and the Philox
-      // rounds shared by the pair (32x32 maps: 4096 envs +10 %, 8192 +8 %, 16,384 +0 %)
+      // Few enough envs that a wave of 16 (8 actions: 8) still finds a SIMD that has at most
+      // one other: A lanes to an env - or fewer envs to a wave while that gives more compute
+      // units a wave of their own.
       long units = tickets;  // tickets as the kernel counts them
-      if (p.moves && waves == 1 && tickets <= 2 * kComputeUnits) {
-        p.pair = true;
-        // ... and thinner still while that gives more compute units a wave of their own
-        // (4096 envs of 32x32: 128 waves of 32 envs 1.165e10 env-steps/s, 256 of 16 1.25e10,
-        // 512 of 8 - two to a unit - 1.16e10)
-        p.pair_envs = crl::kTicketEnvs;
-        while (p.pair_envs > 8 && (e->N + p.pair_envs - 1) / p.pair_envs < kComputeUnits) p.pair_envs /= 2;
-        units = (e->N + p.pair_envs - 1) / p.pair_envs;
-        p.grid = (int)std::min<long>(std::max<long>(1, resident / p.pair_envs), units);
+      if (lanes_rules(e) && waves == 1 && tickets <= 2 * kComputeUnits) {
+        // (one wave to a compute unit in long launches, whose rows are in the caches most of the
+        // time; a wave to a SIMD in shorter ones, where most steps wait for a first use of a line,
+        // and the fewer envs a wave has the less often: 4096 envs of 32x32, 256 steps 108 / 98 us)
+        const long spread = n_steps > kLongLaunchSteps ? kComputeUnits : 4L * kComputeUnits;
+        int log_envs = e->A == 8 ? 3 : 4;
+        while (log_envs > 0 && (e->N + (1L << log_envs) - 1) >> log_envs < spread) --log_envs;
+        const size_t lds = 16 + tape_bytes(log_envs) + ((size_t)e->mv_words * 4 << log_envs);
+        if (lds <= kLdsPerWorkgroup && (e->K * sizeof(float)) << log_envs < (size_t)1 << 32) {
+          p.fast = p.moves = p.lanes = true;
+          p.rich = c.eps_mode >= CRL_EPS_EPISODE_MULT || c.reward_flags != 0;
+          p.log_envs = log_envs;
+          p.tape_steps = tape_steps_for(log_envs);
+          units = (e->N + (1L << log_envs) - 1) >> log_envs;
+          p.grid = (int)std::min<long>(std::max<long>(1, resident >> log_envs), units);
+          // (where there is a compute unit for every workgroup, LDS for no second one beside it)
+          p.lds = p.grid <= kComputeUnits ? std::max(lds, std::min<size_t>(mv_lds, kLdsMapLimitBytes)) : lds;
+        }
       }
       // Tickets dealt by position instead of drawn from a counter: the workers of this plan
       // all take the same time, and 16,384 draws from one counter take 0.38 ms however short
       // the launch (1M envs: the whole of a 4-step launch, half of a 20-step one).
-      p.fixed = n_steps < kHybridMinSteps;
-      (void)units;
-      p.lds = waves * (p.moves ? mv_lds : map_lds);
+      p.fixed = n_steps < kHybridMinSteps || (p.lanes && p.grid >= units);
+      if (!p.lanes) p.lds = waves * (p.moves ? mv_lds : map_lds);
     }
   }
   static const char* names[2][3][3] = {
@@ -476,7 +554,7 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       {{"k_fused_per_env<8,0>", "k_fused_per_env<8,1,general>", "k_fused_per_env<8,2,general>"},
        {"k_fused_per_env<8,0>", "k_fused_per_env<8,1,fast>", "k_fused_per_env<8,2,fast>"},
        {"k_fused_per_env<8,0>", "k_fused_per_env<8,1,fast,pairs>", "k_fused_per_env<8,2,fast,pairs>"}}};
-  p.name = names[e->A == 8][!p.fast ? 0 : p.pair ? 2 : 1][p.map_kind];
+  p.name = names[e->A == 8][!p.fast ? 0 : p.lanes ? 2 : 1][p.map_kind];
   if (p.tickets) {
     static const char* tnames[2][3][2] = {
         {{"k_fused_tickets<4,general,hbm>", "k_fused_tickets<4,general,hbm+lds>"},
@@ -494,6 +572,23 @@ template <int A>
 void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n) {
   const crl::Rules R = e->rules();
   const crl::Ptrs P = e->ptrs();
+  if (p.in_lds) {
+    const bool events = crl::lane_events(R, P);
+#define CRL_LAUNCH_LDS(KERN)                                                                                              \
+  do {                                                                                                                    \
+    auto go = [&](auto kern) {                                                                                            \
+      hipLaunchKernelGGL(kern, dim3(p.grid), dim3(64), p.lds, e->stream, R, P, t0, n, p.log_envs, p.env_bytes, p.tape_steps); \
+    };                                                                                                                    \
+    if (p.words && events) go(crl::KERN<A, true, true>);                                                                  \
+    else if (p.words) go(crl::KERN<A, true, false>);                                                                      \
+    else if (events) go(crl::KERN<A, false, true>);                                                                       \
+    else go(crl::KERN<A, false, false>);                                                                                  \
+  } while (0)
+    if (p.map_kind == 1) CRL_LAUNCH_LDS(k_fused_per_env_lds);
+    else CRL_LAUNCH_LDS(k_fused_tickets_lds);
+#undef CRL_LAUNCH_LDS
+    return;
+  }
   if (p.tickets) {
     // (tickets dealt by position use no counter; the kernel itself notes who did how much)
     if (!p.fixed) hipLaunchKernelGGL(crl::k_fill_u32, dim3(1), dim3(64), 0, e->stream, e->tk, 0u, 3);
@@ -501,7 +596,7 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
     unsigned* tk = e->tk;
 #define CRL_LAUNCH_TICKETS(MODE, LDSW, MOVES)                                                       \
   hipLaunchKernelGGL((crl::k_fused_tickets<A, MODE, LDSW, MOVES>), g, b, p.lds, e->stream, R, P, t0, n, \
-                     tk, p.tab_stride, p.fixed ? 1 : 0, p.pair ? p.pair_envs : 0)
+                     tk, p.tab_stride, p.fixed ? 1 : 0, p.lanes ? 1 << p.log_envs : 0, p.tape_steps)
     if (p.rich && p.moves)
       CRL_LAUNCH_TICKETS(2, false, true);
     else if (p.rich)
@@ -521,8 +616,8 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
   }
 #define CRL_LAUNCH_PER_ENV(MAP, MODE)                                                                 \
   hipLaunchKernelGGL((crl::k_fused_per_env<A, MAP, MODE>), dim3(p.grid), dim3(p.block),               \
-                     MAP == 1 ? p.lds : 0, e->stream, R, P, t0, n)
-  const int mode = !p.fast ? 0 : p.pair ? 2 : 1;
+                     MAP == 1 || MODE == 2 ? p.lds : 0, e->stream, R, P, t0, n, p.log_envs, p.tape_steps)
+  const int mode = !p.fast ? 0 : p.lanes ? 2 : 1;
   if (p.map_kind == 1) {
     if (mode == 2) CRL_LAUNCH_PER_ENV(1, 2);
     else if (mode == 1) CRL_LAUNCH_PER_ENV(1, 1);
@@ -1290,9 +1385,16 @@ int opt_in_ticket_kernels(crl_engine* e) {
       reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 0, true, false>),         \
       reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, true, false>),         \
       reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, false, true>),         \
-      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 2, false, true>)
+      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 2, false, true>),         \
+      reinterpret_cast<const void*>(&crl::k_fused_per_env<A, 1, 2>),                    \
+      CRL_LDS_KERNELS(A, false, false), CRL_LDS_KERNELS(A, false, true),               \
+      CRL_LDS_KERNELS(A, true, false), CRL_LDS_KERNELS(A, true, true)
+#define CRL_LDS_KERNELS(A, WORDS, EVENTS)                                              \
+  reinterpret_cast<const void*>(&crl::k_fused_tickets_lds<A, WORDS, EVENTS>),          \
+      reinterpret_cast<const void*>(&crl::k_fused_per_env_lds<A, WORDS, EVENTS>)
       CRL_TICKET_KERNELS(4), CRL_TICKET_KERNELS(8)
 #undef CRL_TICKET_KERNELS
+#undef CRL_LDS_KERNELS
   };
   for (const void* fn : fns)
     HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsPerWorkgroup));

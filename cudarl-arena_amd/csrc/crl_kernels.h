@@ -474,47 +474,597 @@ __device__ __forceinline__ void run_env_fast(const Rules& R, const Ptrs& P, cons
   P.action[env] = (uint8_t)action;
 }
 
+// ---------------------------------------------------------------------------
+// One env to A lanes of a wave, a lane to an action, for batches that leave lanes to spare.
+// A lone wave issues an instruction every six cycles whatever its lanes do (measured: 2.4 GHz,
+// dependent or not), an LDS read is back after 50 and an L2 hit after 220, so a step's time
+// is mostly its number of instructions.  With an action to a lane the row is one register:
+//   - the maximum over the row is two (A = 8: three) cross-lane operations, and so is the
+//     choice of the first lane that holds it: every lane offers what its own action would do
+//     - action, resulting cell, class of the target, one word - and the smallest word of
+//     those that qualify wins, the action being its top bits;
+//   - no value is looked up by a run-time action: the lane whose word won computes the
+//     update on its own value, and all lanes write their values back;
+//   - the row of the start cell is read only in the steps in which an episode of the wave ends.
+// The exploration draws of the next steps are worked out ahead by all 64 lanes into a tape
+// in LDS (a Philox block is 75 instructions; with E envs to a wave a step's share is 75 E / 128).
+// ---------------------------------------------------------------------------
+
+// u01(w) < eps  <=>  (w >> 8) < eps * 2^24, both sides exact: an integer compare
+__device__ __forceinline__ uint32_t explore_threshold(float eps) {
+  const float scaled = ceilf(eps * 16777216.0f);
+  return !(scaled > 0.0f) ? 0u : scaled >= 16777216.0f ? (1u << 24) : (uint32_t)scaled;
+}
+
+// A word of the tape: explore iff it is below the env's limit, and then the action is its low
+// byte.  Epsilon by episode: the upper 24 bits are the draw's and the limit the threshold.
+// Else whether to explore is settled when the word is written: the action, or kTapeGreedy.
+constexpr uint32_t kTapeGreedy = 0xffffffffu, kTapeLimit = 0x80000000u;
+__device__ __forceinline__ uint32_t tape_limit(float eps) {
+  const uint32_t th = explore_threshold(eps);
+  return th >= (1u << 24) ? 0xffffffffu : th << 8;  // (no word with the upper 24 bits set has all the lower ones)
+}
+
+// The tape of steps [tb, tb + steps) of a wave's 1 << log_envs envs from env0 on, a Philox
+// block to a lane and pair of steps; tb and steps are even.  [step][env].
+template <int A>
+__device__ __forceinline__ void write_tape(const Rules& R, const Ptrs& P, const int env0, const int log_envs,
+                                           const uint64_t tb, const int steps, uint32_t* tape, const int lane) {
+  const int E = 1 << log_envs;
+  const bool by_episode = R.eps_mode >= 2;
+  for (int i = lane; i < (steps >> 1) << log_envs; i += 64) {
+    const int e = i & (E - 1), b = i >> log_envs;
+    const uint64_t t = tb + (uint64_t)(2 * b);
+    const Philox4 blk = explore_block(R.seed, (uint32_t)(env0 + e), t >> 1);
+    uint32_t w0 = below(blk.w1, (uint32_t)A), w1 = below(blk.w3, (uint32_t)A);
+    if (by_episode) {
+      w0 |= blk.w0 & 0xffffff00u;
+      w1 |= blk.w2 & 0xffffff00u;
+    } else {
+      w0 = (blk.w0 >> 8) < explore_threshold(eps_of(R, P.eps_tab, t, 0)) ? w0 : kTapeGreedy;
+      w1 = (blk.w2 >> 8) < explore_threshold(eps_of(R, P.eps_tab, t + 1, 0)) ? w1 : kTapeGreedy;
+    }
+    tape[((2 * b) << log_envs) + e] = w0;
+    tape[((2 * b + 1) << log_envs) + e] = w1;
+  }
+}
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The cross-lane steps of run_lanes, written out.  v_max_f32 is fmaxf (a number beats none),
+// but the compiler puts a v_max_f32 x, x in front of each operand and cannot fold the lane
+// move into it then; and a lane move, like the use of a comparison's mask, has to stay two
+// instructions away from the one that wrote its operand, which the compiler does not see
+// inside an asm statement, so each block keeps that distance itself (also from what comes
+// before it), with work that is due anyway where there is some: s_nop 1 costs nine cycles,
+// any other instruction five.  Masks of comparisons go from vector
+// instruction to vector instruction: a scalar instruction between them waits for 13 cycles,
+// a branch on one for 28.
+#define CRL_PAIRS "quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+#define CRL_HALVES "quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+#define CRL_EIGHT "row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+
+// Maximum of q over the env's lanes, but at least `floor` (no number: no floor).  On the
+// way, for the draw of the next step: named = c in the lane of its action (low byte) and all
+// ones elsewhere, explore = the lanes whose draw is below their limit.
+template <int A>
+__device__ __forceinline__ float row_top(float q, float floor, uint32_t draw, uint32_t limit, uint32_t mine, uint32_t c,
+                                         uint32_t& named, unsigned long long& explore) {
+  float m;
+  if (A == 4)
+    asm("v_cmp_eq_u32_sdwa vcc, %[draw], %[mine] src0_sel:BYTE_0 src1_sel:DWORD\n\t"
+        "v_cmp_lt_u32 %[explore], %[draw], %[limit]\n\t"
+        "v_max_f32_dpp %[m], %[q], %[q] " CRL_PAIRS
+        "v_cndmask_b32 %[named], -1, %[c], vcc\n\t"
+        "s_nop 0\n\t"
+        "v_max_f32_dpp %[m], %[m], %[m] " CRL_HALVES
+        "v_max_f32 %[m], %[m], %[floor]"
+        : [m] "=&v"(m), [named] "=&v"(named), [explore] "=&s"(explore)
+        : [q] "v"(q), [floor] "v"(floor), [draw] "v"(draw), [limit] "v"(limit), [mine] "v"(mine), [c] "v"(c)
+        : "vcc");
+  else
+    asm("v_cmp_eq_u32_sdwa vcc, %[draw], %[mine] src0_sel:BYTE_0 src1_sel:DWORD\n\t"
+        "v_cmp_lt_u32 %[explore], %[draw], %[limit]\n\t"
+        "v_max_f32_dpp %[m], %[q], %[q] " CRL_PAIRS
+        "v_cndmask_b32 %[named], -1, %[c], vcc\n\t"
+        "s_nop 0\n\t"
+        "v_max_f32_dpp %[m], %[m], %[m] " CRL_HALVES
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %[m], %[m], %[m] " CRL_EIGHT
+        "v_max_f32 %[m], %[m], %[floor]"
+        : [m] "=&v"(m), [named] "=&v"(named), [explore] "=&s"(explore)
+        : [q] "v"(q), [floor] "v"(floor), [draw] "v"(draw), [limit] "v"(limit), [mine] "v"(mine), [c] "v"(c)
+        : "vcc");
+  return m;
+}
+// The smallest word of the lanes that qualify: those of `named` that are not all ones where
+// the env explores, else those whose q no other beats - where `unless` is the value that a q
+// that is no number counts as: in the first lane it stays one, and then nothing beats it
+// (src/q_learning.cu:200-206: strict >, from action 0 on).  On the way: word += next_word,
+// left -= 1.
+template <int A>
+__device__ __forceinline__ uint32_t row_pick_word(float q, float unless, uint32_t c, uint32_t named, unsigned long long explore,
+                                                  uint32_t& word, uint32_t next_word, int& left) {
+  float v, m;
+  uint32_t w;
+  if (A == 4)
+    asm("v_max_f32 %[v], %[q], %[unless]\n\t"
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %[m], %[v], %[v] " CRL_PAIRS
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %[m], %[m], %[m] " CRL_HALVES
+        "v_cmp_nlt_f32 vcc, %[v], %[m]\n\t"
+        "v_add_u32 %[word], %[next_word], %[word]\n\t"
+        "v_add_u32 %[left], -1, %[left]\n\t"
+        "v_cndmask_b32 %[w], -1, %[c], vcc\n\t"
+        "v_cndmask_b32 %[w], %[w], %[named], %[explore]\n\t"
+        "s_nop 1\n\t"
+        "v_min_u32_dpp %[w], %[w], %[w] " CRL_PAIRS
+        "s_nop 1\n\t"
+        "v_min_u32_dpp %[w], %[w], %[w] " CRL_HALVES
+        : [v] "=&v"(v), [m] "=&v"(m), [w] "=&v"(w), [word] "+v"(word), [left] "+v"(left)
+        : [q] "v"(q), [unless] "v"(unless), [c] "v"(c), [named] "v"(named), [explore] "s"(explore), [next_word] "s"(next_word)
+        : "vcc");
+  else
+    asm("v_max_f32 %[v], %[q], %[unless]\n\t"
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %[m], %[v], %[v] " CRL_PAIRS
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %[m], %[m], %[m] " CRL_HALVES
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %[m], %[m], %[m] " CRL_EIGHT
+        "v_cmp_nlt_f32 vcc, %[v], %[m]\n\t"
+        "v_add_u32 %[word], %[next_word], %[word]\n\t"
+        "v_add_u32 %[left], -1, %[left]\n\t"
+        "v_cndmask_b32 %[w], -1, %[c], vcc\n\t"
+        "v_cndmask_b32 %[w], %[w], %[named], %[explore]\n\t"
+        "s_nop 1\n\t"
+        "v_min_u32_dpp %[w], %[w], %[w] " CRL_PAIRS
+        "s_nop 1\n\t"
+        "v_min_u32_dpp %[w], %[w], %[w] " CRL_HALVES
+        "s_nop 1\n\t"
+        "v_min_u32_dpp %[w], %[w], %[w] " CRL_EIGHT
+        : [v] "=&v"(v), [m] "=&v"(m), [w] "=&v"(w), [word] "+v"(word), [left] "+v"(left)
+        : [q] "v"(q), [unless] "v"(unless), [c] "v"(c), [named] "v"(named), [explore] "s"(explore), [next_word] "s"(next_word)
+        : "vcc");
+  return w;
+}
+#undef CRL_PAIRS
+#undef CRL_HALVES
+#undef CRL_EIGHT
+
+// What an action does from a cell, as one word: the action in the top three bits, the
+// resulting cell as the byte offset of its row (a multiple of 16), the class of the target
+// (kWall outside the grid) in bits 2 and 3.
+constexpr uint32_t kMoveOffset = 0x1ffffff0u, kMoveClass = 0xcu;
+__device__ __forceinline__ uint32_t move_word(uint32_t a, uint32_t offset, uint32_t cls) { return (a << 29) | offset | (cls << 2); }
+
+// LDS by address
+template <class T>
+using LdsPtr = __attribute__((address_space(3))) T*;
+template <class T>
+__device__ __forceinline__ LdsPtr<T> lds_at(uint32_t address) { return reinterpret_cast<LdsPtr<T>>(address); }
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return (uint32_t)reinterpret_cast<uintptr_t>((LdsPtr<const void>)p);
+}
+
+// Table and move words of an env in LDS, cell by cell: A values, then A words - one
+// instruction reads both of a lane's.  At most 2^29 bytes per table.
+template <int A>
+struct LaneLds {
+  static constexpr uint32_t kRow = 8 * A;
+  uint32_t first;  // LDS address of the lane's value of the env's first cell
+  using At = uint32_t;
+  __device__ __forceinline__ At at(uint32_t offset) const { return first + offset; }
+  __device__ __forceinline__ uint32_t offset(At p) const { return p - first; }
+  static __device__ __forceinline__ float value(At p) { return *lds_at<float>(p); }
+  static __device__ __forceinline__ void fetch(At p, float& q, uint32_t& c) {
+    q = value(p);
+    c = *lds_at<uint32_t>(p + 4 * A);
+  }
+  static __device__ __forceinline__ void store(At p, float v) { *lds_at<float>(p) = v; }
+};
+
+// Values in LDS (QL) or in HBM and the caches, the cells' move codes in LDS (CL) or global
+// memory, a byte per cell (two with 8 actions): the move word is worked out when the code
+// has arrived, seven instructions.
+template <int A, bool QL, bool CL>
+struct LaneCodes {
+  static constexpr uint32_t kRow = 4 * A;
+  unsigned char* values;       // QL: the lane's value of the env's first cell; else the wave's first table
+  uint32_t values_at;          // QL: 0; else from there to the lane's value of its env's first cell
+  const unsigned char* codes;  // CL: the env's codes; else the wave's first env's
+  uint32_t codes_at;           // CL: 0; else from there to the env's
+  uint32_t action;
+  int step;                    // bytes from a row to the one the lane's action leads to
+  using At = uint32_t;
+  __device__ __forceinline__ At at(uint32_t offset) const { return offset; }
+  __device__ __forceinline__ uint32_t offset(At p) const { return p; }
+  __device__ __forceinline__ float value(At p) const { return *reinterpret_cast<const float*>(values + (QL ? p : values_at + p)); }
+  __device__ __forceinline__ void fetch(At p, float& q, uint32_t& c) const {
+    q = value(p);
+    const uint32_t i = codes_at + p / (A == 4 ? kRow : kRow / 2);
+    const uint32_t code = A == 4 ? (uint32_t)codes[i] : (uint32_t)*reinterpret_cast<const uint16_t*>(codes + i);
+    const uint32_t cls = __builtin_amdgcn_ubfe(code, 2 * action, 2u);
+    c = move_word(action, cls < (uint32_t)kTrap ? p + (uint32_t)step : p, cls);
+  }
+  __device__ __forceinline__ void store(At p, float v) const { *reinterpret_cast<float*>(values + (QL ? p : values_at + p)) = v; }
+};
+
+// The steps.  Every lane of the wave calls it; env e of the wave is lanes e A ... e A + A - 1
+// and `live` tells whether there is one.  The rewards by class - step, goal, trap, step - lie
+// at LDS address 0, where dynamic LDS starts in a kernel without any other; CELLS: `cell_rewards` of the env's cells also count.  EVENTS: an episode's end changes more
+// than where the env stands - epsilon by episode, episode statistics, an episode budget.
+// The row of the cell the move ends on (for the TD target) and that of the cell the env acts
+// from next - another one only where its episode ended - are asked for together.
+template <int A, bool CELLS, bool EVENTS, class Mem>
+__device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const int env0, const bool live,
+                                          const uint64_t t0, const int n_steps, const Mem mem, uint32_t* tape,
+                                          const int log_envs, const int tape_steps,
+                                          const float* __restrict__ cell_rewards) {
+  const int lane = (int)__lane_id();
+  const uint32_t mine = (uint32_t)lane & (A - 1);  // this lane's action
+  const int slot = live ? lane / A : 0, env = env0 + slot;
+  const int whole = R.episode_len > 0 ? R.episode_len : 0x7fffffff;
+  const float lr = R.lr, gamma = R.gamma;
+  const float nan = __uint_as_float(0x7fc00000u);
+  const float floor = R.max_mode == 1 ? 0.0f : nan;
+  const float unless = mine == 0 ? nan : -__builtin_inff();
+  const typename Mem::At at_start = mem.at((uint32_t)P.start[env] * Mem::kRow);
+  typename Mem::At at = mem.at((uint32_t)P.s[env] * Mem::kRow);
+  int left = whole - P.ep_step[env];  // steps of the episode that are left
+  int episode = P.episode[env];
+  float reward = P.reward[env];
+  uint32_t won = ((uint32_t)P.action[env] << 29) | (P.done[env] != 0 ? (uint32_t)kGoal << 2 : 0u);  // the last step's word
+  const bool by_episode = EVENTS && R.eps_mode >= 2, track = EVENTS && P.ret_acc != nullptr;
+  const bool base_cells = CELLS && (R.reward_flags & 2) != 0;
+  uint32_t limit = by_episode ? tape_limit(eps_of(R, P.eps_tab, t0, episode)) : kTapeLimit;
+  float eps_next = by_episode ? eps_of(R, P.eps_tab, t0, episode + 1) : 0.0f;  // of the next episode: asked for ahead
+  float ret = 0.0f, ret_last = 0.0f, ret_sum = 0.0f;
+  int len_last = 0, len_sum = 0;
+  if (track) {
+    ret = P.ret_acc[env];
+    ret_last = P.ret_last[env];
+    ret_sum = P.ret_sum[env];
+    len_last = P.len_last[env];
+    len_sum = P.len_sum[env];
+  }
+  const int budget = EVENTS && R.max_episodes > 0 ? R.max_episodes : 0x7fffffff;
+  bool going = live && episode < budget;
+  float q;
+  uint32_t c;
+  mem.fetch(at, q, c);
+  // (arrived before the loop starts: a value that may be in flight there makes every round
+  // wait for everything, the last store's answer included)
+  asm volatile("" : "+v"(q), "+v"(c), "+v"(reward), "+v"(left), "+v"(episode), "+v"(won), "+v"(limit), "+v"(eps_next));
+  if (EVENTS) asm volatile("" : "+v"(ret), "+v"(ret_last), "+v"(ret_sum), "+v"(len_last), "+v"(len_sum));
+
+  const uint64_t t_end = t0 + (uint64_t)n_steps;
+  for (uint64_t tb = t0 & ~(uint64_t)1; tb < t_end; tb += (uint64_t)tape_steps) {
+    wave_fence();
+    write_tape<A>(R, P, env0, log_envs, tb, tape_steps, tape, lane);
+    wave_fence();
+    const int k0 = tb < t0 ? 1 : 0;  // (the first block may start with a step of the launch before)
+    const int k1 = (int)min((uint64_t)tape_steps, t_end - tb);
+    // (leaving the loop is the same for all lanes that are in it: an env that has used up its
+    // budget ends the loop for its wave, and the others enter it again without it)
+    for (int k = k0; k < k1;) {
+      const unsigned long long who = __builtin_amdgcn_ballot_w64(going);
+      if (who == 0ull) break;
+      int kk = k;
+      if (going) {
+        uint32_t word = lds_address(tape) + 4u * (uint32_t)((kk << log_envs) + slot);
+        const uint32_t first = *lds_at<uint32_t>(word);
+        uint32_t named = (first & 0xffu) == mine ? c : 0xffffffffu;
+        unsigned long long explore = __builtin_amdgcn_ballot_w64(first < limit);
+        for (int end = k1; kk < end;) {
+          const int before = left;
+          won = row_pick_word<A>(q, unless, c, named, explore, word, 4u << log_envs, left);
+          const typename Mem::At at2 = mem.at(won & kMoveOffset);
+          const uint32_t cls = won & kMoveClass;
+          const bool hit = cls == (uint32_t)kGoal << 2;
+          left = hit ? 0 : left;
+          const bool ends = left <= 0;
+          typename Mem::At at_next = ends ? at_start : at2;
+          asm("" : "+v"(at_next));  // (one address, not one per use)
+          const float q2 = mem.value(at2);
+          float q_next;
+          uint32_t c_next;
+          mem.fetch(at_next, q_next, c_next);
+          reward = *lds_at<float>(cls);
+          float by_cell = 0.0f;
+          if (CELLS) {
+            // the goal pays on the goal cell (where the move ends), a trap on the cell it
+            // guards, anything else where the move ends
+            int pays = (int)(mem.offset(at2) / Mem::kRow);
+            if (__builtin_amdgcn_ballot_w64(cls == (uint32_t)kTrap << 2) != 0ull) {
+              int dx, dy;
+              action_delta((int)(won >> 29), A, dx, dy);
+              pays = cls == (uint32_t)kTrap << 2 ? pays + __mul24(dy, R.W) + dx : pays;
+            }
+            by_cell = cell_rewards[pays];
+          }
+          const uint32_t draw = *lds_at<uint32_t>(word);  // (the one behind the tape's end is not used)
+          ++kk;
+          const bool me = c == won, stays = at_next == at;
+          const int len = whole - before + 1;
+          left = ends ? whole : left;
+          episode += ends ? 1 : 0;
+          __builtin_amdgcn_sched_barrier(0);  // all of the above while the values are on their way
+          if (CELLS) reward = (base_cells || (cls - 4u) < 8u) ? by_cell : reward;  // (goal or trap, or any)
+          if (EVENTS) {
+            ret = ret + reward;
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(ends) != 0ull, 0)) {
+              if (track) {
+                ret_last = ends ? ret : ret_last;
+                ret_sum = ends ? ret_sum + ret : ret_sum;
+                len_last = ends ? len : len_last;
+                len_sum += ends ? len : 0;
+              }
+              ret = ends ? 0.0f : ret;
+              if (by_episode) {
+                limit = ends ? tape_limit(eps_next) : limit;
+                eps_next = eps_of(R, P.eps_tab, t0, episode + 1);
+              }
+              if (__builtin_amdgcn_ballot_w64(episode >= budget) != 0ull) end = kk;
+            }
+          }
+          float m = row_top<A>(q2, floor, draw, limit, mine, c_next, named, explore);
+          m = hit ? 0.0f : m;
+          q = me ? td_value(q, reward, m, lr, gamma) : q;
+          mem.store(at, q);
+          q = stays ? q : q_next;
+          c = c_next;
+          at = at_next;
+        }
+        going = episode < budget;
+      }
+      k = __builtin_amdgcn_readlane(kk, __builtin_ctzll(who));
+    }
+  }
+
+  if (live && mine == 0) {
+    P.s[env] = (int)(mem.offset(at) / Mem::kRow);
+    P.ep_step[env] = whole - left;
+    P.episode[env] = episode;
+    P.reward[env] = reward;
+    P.done[env] = (won & kMoveClass) == (uint32_t)kGoal << 2 ? 1 : 0;
+    P.action[env] = (uint8_t)(won >> 29);
+    if (track) {
+      P.ret_acc[env] = ret;
+      P.ret_last[env] = ret_last;
+      P.ret_sum[env] = ret_sum;
+      P.len_last[env] = len_last;
+      P.len_sum[env] = len_sum;
+    }
+  }
+}
+
+// whether run_lanes needs its EVENTS form
+__host__ __device__ inline bool lane_events(const Rules& R, const Ptrs& P) {
+  return R.eps_mode >= 2 || R.max_episodes > 0 || P.ret_acc != nullptr;
+}
+// the rewards by class, where run_lanes looks them up; word i of n, by one wave
+__device__ __forceinline__ void write_rewards(const Rules& R, float* rewards, int lane) {
+  if (lane < 4) rewards[lane] = lane == kGoal ? R.goal_reward : lane == kTrap ? R.trap_reward : R.step_reward;
+}
+// n consecutive words into LDS by one wave, eight loads in flight per lane
+__device__ __forceinline__ void copy_words(const uint32_t* __restrict__ src, const int n, uint32_t* dst, const int lane) {
+  for (int i = lane; i < n; i += 64 * 8) {
+    uint32_t v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (i + 64 * u < n) v[u] = src[i + 64 * u];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (i + 64 * u < n) dst[i + 64 * u] = v[u];
+  }
+}
+// bytes from a row to the one that action `a` leads to
+template <int A>
+__device__ __forceinline__ int row_step(const Rules& R, uint32_t a, uint32_t row_bytes) {
+  int dx, dy;
+  action_delta((int)a, A, dx, dy);
+  return (dy * R.W + dx) * (int)row_bytes;
+}
+
+// Batches whose tables all fit the chip's LDS: a wave of 1 << log_envs envs, alone in its
+// workgroup, keeps them there for the whole launch.
+// LDS: the rewards by class (at address 0: their index is their address), [env][env_bytes],
+// the tape.  WORDS: an env is rows of values and move words side by side (8 bytes per
+// key); else rows of values, then the move codes (4 bytes and a quarter; a shared map's
+// codes only once, behind the tape).
+template <int A, bool MAP_SHARED, bool WORDS, bool EVENTS>
+__device__ __forceinline__ void fused_lds(const Rules& R, const Ptrs& P, const uint64_t t0, const int n_steps,
+                                          const int log_envs, const int env_bytes, const int tape_steps) {
+  extern __shared__ __align__(16) unsigned char lds_bytes[];
+  constexpr uint32_t kRow = WORDS ? LaneLds<A>::kRow : LaneCodes<A, true, true>::kRow;
+  const int lane = threadIdx.x;
+  const int E = 1 << log_envs;
+  const int env0 = blockIdx.x << log_envs;
+  const int n_here = min(E, P.N - env0);
+  const int S = (int)P.S;
+  float* rewards = reinterpret_cast<float*>(lds_bytes);
+  unsigned char* envs = lds_bytes + 16;
+  uint32_t* tape = reinterpret_cast<uint32_t*>(envs + (size_t)E * env_bytes);
+  uint32_t* shared_codes = tape + ((tape_steps + 1) << log_envs);
+  write_rewards(R, rewards, lane);
+  if (!WORDS) {
+    if (MAP_SHARED) {
+      copy_words(P.moves, P.mv_words, shared_codes, lane);
+    } else {
+      for (int e = 0; e < n_here; ++e)
+        copy_words(P.moves + (size_t)(env0 + e) * P.mv_words, P.mv_words,
+                   reinterpret_cast<uint32_t*>(envs + (size_t)e * env_bytes + (size_t)S * kRow), lane);
+    }
+  }
+
+  // a lane takes a cell at a time: its row (and its codes) in, its row (and its move words) out
+  const float* Q = P.Q + (size_t)env0 * S * A;
+  const int cells = n_here * S;
+  int e = 0, cell = lane;
+  for (int i0 = lane; i0 < cells; i0 += 64 * 4) {
+    Row<A> row[4];
+    uint32_t codes[4];
+    int ee[4], cc[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {  // (four rows in flight)
+      while (cell >= S) {
+        cell -= S;
+        ++e;
+      }
+      ee[u] = e;
+      cc[u] = cell;
+      cell += 64;
+      if (i0 + 64 * u < cells) {
+        row[u] = load_row<A>(Q + (size_t)(i0 + 64 * u) * A);
+        if (WORDS) {
+          const unsigned char* map = reinterpret_cast<const unsigned char*>(P.moves + (MAP_SHARED ? 0 : (size_t)(env0 + ee[u]) * P.mv_words));
+          codes[u] = A == 4 ? map[cc[u]] : reinterpret_cast<const uint16_t*>(map)[cc[u]];
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (i0 + 64 * u >= cells) break;
+      unsigned char* to = envs + (size_t)ee[u] * env_bytes + (size_t)cc[u] * kRow;
+      store_row(reinterpret_cast<float*>(to), row[u]);
+      if (WORDS) {
+        uint32_t w[A];
+#pragma unroll
+        for (int a = 0; a < A; ++a) {
+          const uint32_t cls = (codes[u] >> (2 * a)) & 3u;
+          const uint32_t from = (uint32_t)cc[u] * kRow;
+          w[a] = move_word((uint32_t)a, cls < (uint32_t)kTrap ? from + (uint32_t)row_step<A>(R, a, kRow) : from, cls);
+        }
+#pragma unroll
+        for (int a = 0; a < A; a += 4)
+          *reinterpret_cast<uint4*>(to + 4 * A + 4 * a) = make_uint4(w[a], w[a + 1], w[a + 2], w[a + 3]);
+      }
+    }
+  }
+  wave_fence();
+  const int slot = lane / A;
+  const bool live = slot < n_here;
+  const uint32_t action = (uint32_t)lane & (A - 1);
+  unsigned char* mine = envs + (size_t)(live ? slot : 0) * env_bytes;
+  if (WORDS) {
+    run_lanes<A, false, EVENTS>(R, P, env0, live, t0, n_steps, LaneLds<A>{lds_address(mine) + 4 * action}, tape, log_envs, tape_steps, nullptr);
+  } else {
+    const unsigned char* codes = MAP_SHARED ? reinterpret_cast<const unsigned char*>(shared_codes) : mine + (size_t)S * kRow;
+    const LaneCodes<A, true, true> mem{mine + 4 * action, 0u, codes, 0u, action, row_step<A>(R, action, kRow)};
+    run_lanes<A, false, EVENTS>(R, P, env0, live, t0, n_steps, mem, tape, log_envs, tape_steps, nullptr);
+  }
+  wave_fence();
+  float* out = P.Q + (size_t)env0 * S * A;
+  e = 0;
+  cell = lane;
+  for (int i = lane; i < cells; i += 64, cell += 64) {
+    while (cell >= S) {
+      cell -= S;
+      ++e;
+    }
+    store_row(out + (size_t)i * A, load_row<A>(reinterpret_cast<const float*>(envs + (size_t)e * env_bytes + (size_t)cell * kRow)));
+  }
+}
+template <int A, bool WORDS, bool EVENTS>
+__global__ __launch_bounds__(64) void k_fused_tickets_lds(const Rules R, const Ptrs P, const uint64_t t0,
+                                                           const int n_steps, const int log_envs,
+                                                           const int env_bytes, const int tape_steps) {
+  fused_lds<A, false, WORDS, EVENTS>(R, P, t0, n_steps, log_envs, env_bytes, tape_steps);
+}
+template <int A, bool WORDS, bool EVENTS>
+__global__ __launch_bounds__(64) void k_fused_per_env_lds(const Rules R, const Ptrs P, const uint64_t t0,
+                                                           const int n_steps, const int log_envs,
+                                                           const int env_bytes, const int tape_steps) {
+  fused_lds<A, true, WORDS, EVENTS>(R, P, t0, n_steps, log_envs, env_bytes, tape_steps);
+}
+
+// Tables in HBM and the caches, an env to A lanes, a wave to 1 << log_envs envs from env0 on.
+// `codes` are the move codes of the map (shared) or of the wave's first env, in LDS (CL) or
+// global memory; `code_bytes` from one env's to the next (0: shared).
+template <int A, bool CELLS, bool CL>
+__device__ __forceinline__ void fused_lanes_hbm(const Rules& R, const Ptrs& P, const int env0, const uint64_t t0,
+                                                const int n_steps, const unsigned char* codes, const uint32_t code_bytes,
+                                                uint32_t* tape, const int log_envs, const int tape_steps) {
+  constexpr uint32_t kRow = LaneCodes<A, false, CL>::kRow;
+  const int lane = (int)__lane_id();
+  const int slot = lane / A;
+  const bool live = slot < min(1 << log_envs, P.N - env0);
+  const uint32_t at = live ? (uint32_t)slot : 0u, action = (uint32_t)lane & (A - 1);
+  const LaneCodes<A, false, CL> mem{reinterpret_cast<unsigned char*>(P.Q + (size_t)env0 * P.S * A),
+                                    at * (uint32_t)P.S * kRow + 4u * action,
+                                    CL ? codes + at * code_bytes : codes,
+                                    CL ? 0u : at * code_bytes,
+                                    action, row_step<A>(R, action, kRow)};
+  const float* cr = CELLS ? P.cell_reward + (P.map_shared ? 0 : (size_t)(env0 + at) * P.S) : nullptr;
+  if (lane_events(R, P))
+    run_lanes<A, CELLS, true>(R, P, env0, live, t0, n_steps, mem, tape, log_envs, tape_steps, cr);
+  else
+    run_lanes<A, CELLS, false>(R, P, env0, live, t0, n_steps, mem, tape, log_envs, tape_steps, cr);
+}
+
 // Per-env tables whose maps are shared (MAP = 1: the one map's move codes staged
 // in LDS) or too large for LDS (MAP = 2: move codes read from global memory, one
 // load per step).  A block takes chunks blockIdx, blockIdx + gridDim, ... and runs
-// each for all n_steps.  MODE 0: the general loop, 1: the folded loop, 2: the
-// folded loop with two lanes per env (a batch too small to give every SIMD a wave
-// of 64 envs: twice the waves, each with half the distinct addresses per request,
-// and the Philox rounds shared between the lanes of a pair).
+// each for all n_steps.  MODE 0: the general loop, 1: the folded loop, 2: an env to A
+// lanes, for batches that then still leave the chip at most a wave or two per SIMD
+// (`log_envs` envs to a wave; LDS: rewards, a tape per wave, the shared map's codes).
 template <int A, int MAP, int MODE>
 __global__ __launch_bounds__(256) void k_fused_per_env(const Rules R, const Ptrs P,
-                                                        const uint64_t t0, const int n_steps) {
-  constexpr bool FAST = MODE >= 1;
-  constexpr bool PAIR = MODE == 2;  // two lanes per env: lanes l and l + 32 of a wave
-  extern __shared__ uint32_t lds[];
+                                                        const uint64_t t0, const int n_steps,
+                                                        const int log_envs, const int tape_steps) {
+  extern __shared__ __align__(16) uint32_t lds[];
   const int tid = threadIdx.x;
   const int bdim = blockDim.x;
-  const int envs_per_block = PAIR ? bdim >> 1 : bdim;
-  const int n_chunks = (P.N + envs_per_block - 1) / envs_per_block;
-  const int slot = PAIR ? ((tid >> 6) << 5) + (tid & 31) : tid;
-
-  if (MAP == 1) {
-    for (int i = tid; i < P.mv_words; i += bdim) lds[i] = P.moves[i];
+  if constexpr (MODE == 2) {
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), n_waves = bdim >> 6;
+    const int tape_words = (tape_steps + 1) << log_envs;
+    float* rewards = reinterpret_cast<float*>(lds);
+    uint32_t* codes = lds + 4 + n_waves * tape_words;
+    write_rewards(R, rewards, tid);
+    if (MAP == 1)
+      for (int i = tid; i < P.mv_words; i += bdim) codes[i] = P.moves[i];
     __syncthreads();
-  }
-  for (int chunk = blockIdx.x; chunk < n_chunks; chunk += gridDim.x) {
-    const int env = chunk * envs_per_block + slot;
-    if (env >= P.N) continue;
-    const float* cr =
-        P.cell_reward ? P.cell_reward + (P.map_shared ? 0 : (size_t)env * P.S) : nullptr;
-    const uint32_t* own_map = P.map + (P.map_shared ? 0 : (size_t)env * P.map_words);
-    const GlobalTable<A> tab{P.Q + (size_t)env * P.S * A};
+    const int env0 = (blockIdx.x * n_waves + wave) << log_envs;
+    if (env0 >= P.N) return;
+    uint32_t* tape = lds + 4 + wave * tape_words;
+    const uint32_t code_bytes = P.map_shared ? 0u : (uint32_t)P.mv_words * 4u;
+    const unsigned char* from = reinterpret_cast<const unsigned char*>(
+        MAP == 1 ? codes : P.moves + (P.map_shared ? 0 : (size_t)env0 * P.mv_words));
+    if (P.cell_reward)
+      fused_lanes_hbm<A, true, MAP == 1>(R, P, env0, t0, n_steps, from, code_bytes, tape, log_envs, tape_steps);
+    else
+      fused_lanes_hbm<A, false, MAP == 1>(R, P, env0, t0, n_steps, from, code_bytes, tape, log_envs, tape_steps);
+  } else {
+    constexpr bool FAST = MODE == 1;
+    const int n_chunks = (P.N + bdim - 1) / bdim;
     if (MAP == 1) {
-      if (FAST)
-        run_env_fast<A, PAIR, true>(R, P, env, t0, n_steps, MovesLds<A>{lds, 1}, cr, tab);
-      else
-        run_env_steps<A>(R, P, env, t0, n_steps, MovesLds<A>{lds, 1}, own_map, cr, tab);
-    } else {
-      const MovesGlobal<A> moves{P.moves + (P.map_shared ? 0 : (size_t)env * P.mv_words)};
-      if (FAST)
-        run_env_fast<A, PAIR, true>(R, P, env, t0, n_steps, moves, cr, tab);
-      else
-        run_env_steps<A>(R, P, env, t0, n_steps, moves, own_map, cr, tab);
+      for (int i = tid; i < P.mv_words; i += bdim) lds[i] = P.moves[i];
+      __syncthreads();
+    }
+    for (int chunk = blockIdx.x; chunk < n_chunks; chunk += gridDim.x) {
+      const int env = chunk * bdim + tid;
+      if (env >= P.N) continue;
+      const float* cr =
+          P.cell_reward ? P.cell_reward + (P.map_shared ? 0 : (size_t)env * P.S) : nullptr;
+      const uint32_t* own_map = P.map + (P.map_shared ? 0 : (size_t)env * P.map_words);
+      const GlobalTable<A> tab{P.Q + (size_t)env * P.S * A};
+      if (MAP == 1) {
+        if (FAST)
+          run_env_fast<A, false, true>(R, P, env, t0, n_steps, MovesLds<A>{lds, 1}, cr, tab);
+        else
+          run_env_steps<A>(R, P, env, t0, n_steps, MovesLds<A>{lds, 1}, own_map, cr, tab);
+      } else {
+        const MovesGlobal<A> moves{P.moves + (P.map_shared ? 0 : (size_t)env * P.mv_words)};
+        if (FAST)
+          run_env_fast<A, false, true>(R, P, env, t0, n_steps, moves, cr, tab);
+        else
+          run_env_steps<A>(R, P, env, t0, n_steps, moves, own_map, cr, tab);
+      }
     }
   }
 }
@@ -537,10 +1087,9 @@ __global__ __launch_bounds__(256) void k_fused_per_env(const Rules R, const Ptrs
 // variant with per-cell rewards and per-episode epsilon), which works on move
 // codes: the LDS wave always stages the pre-built codes of its envs; the table
 // waves stage them too with MOVES, and otherwise stage the (four times smaller)
-// class maps and derive the codes while their row loads are in flight.  With
-// staged codes and `pair_tables` a table wave takes one ticket instead of two and
-// gives every env two lanes, like the LDS wave: for batches too small to fill the
-// chip with 64-env waves.
+// class maps and derive the codes while their row loads are in flight.
+// `lane_envs`: the batch is too small to fill the chip with 64-env waves, and the (one) wave
+// of a workgroup takes that many envs a ticket with A lanes to each.
 constexpr int kTicketEnvs = 32;
 
 // `count` envs' words (`wpe` per env, contiguous in HBM) into [word][lane]; eight
@@ -571,10 +1120,11 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
                                                                      unsigned* __restrict__ ticket,
                                                                      const int tab_stride,
                                                                      const int fixed_tickets,
-                                                                     const int pair_envs) {
+                                                                     const int lane_envs,
+                                                                     const int tape_steps) {
   constexpr bool FAST = MODE >= 1;  // the folded loop ...
   constexpr bool RICH = MODE == 2;  // ... in its variant with per-cell rewards and per-episode epsilon
-  extern __shared__ uint32_t lds[];
+  extern __shared__ __align__(16) uint32_t lds[];
   const int n_waves = (int)(blockDim.x >> 6);  // with LDSW the last one works on LDS tables
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -586,10 +1136,9 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
   uint32_t* my_words = lds + wave * slice;  // (the LDS wave is the last one)
   float* tabs = reinterpret_cast<float*>(lds + (n_waves - 1) * slice + lds_slice);
   // envs per ticket: 32, or what a thin table wave steps (never with an LDS wave beside it)
-  const int unit = (FAST && MOVES && pair_envs) ? pair_envs : kTicketEnvs;
+  const int unit = (FAST && MOVES && lane_envs) ? lane_envs : kTicketEnvs;
   const unsigned n_tickets = (unsigned)((P.N + unit - 1) / unit);
-  // (pair_envs: the table waves, too, take one ticket and give every env several lanes)
-  const bool thin = lds_worker || (FAST && MOVES && pair_envs);
+  const bool thin = lds_worker || (FAST && MOVES && lane_envs);
   const int cap = thin ? unit : 64;
   const unsigned take = thin ? 1u : 2u;
   const size_t table = P.S * A;  // floats per table
@@ -606,10 +1155,10 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
   for (unsigned round = 0;; ++round) {
     unsigned base = 0;
     if (fixed_tickets) {
-      base = ((round * gridDim.x + blockIdx.x) * (unsigned)n_waves + (unsigned)wave) * take;
+      base = ((round * gridDim.x + blockIdx.x) * (unsigned)n_waves + (unsigned)__builtin_amdgcn_readfirstlane(wave)) * take;
     } else {
       if (lane == 0) base = atomicAdd(ticket, take);
-      base = __shfl(base, 0);
+      base = (unsigned)__builtin_amdgcn_readfirstlane((int)base);
     }
     if (base >= n_tickets) break;  // every worker gets here: the counter only grows
     const int env0 = (int)base * unit;
@@ -621,6 +1170,22 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
     // this worker's maps: contiguous in HBM, transposed into [word][lane]
     __builtin_amdgcn_wave_barrier();
     const bool codes = FAST && (MOVES || lds_worker);
+    if (kTableMoves && lane_envs) {
+      // LDS: rewards, tape, the codes env by env
+      const int log_envs = 31 - __builtin_clz((unsigned)lane_envs);
+      uint32_t* tape = lds + 4;
+      uint32_t* words = tape + ((tape_steps + 1) << log_envs);
+      write_rewards(R, reinterpret_cast<float*>(lds), lane);
+      copy_words(P.moves + (size_t)env0 * P.mv_words, n_here * P.mv_words, words, lane);
+      wave_fence();
+      const unsigned char* from = reinterpret_cast<const unsigned char*>(words);
+      const uint32_t code_bytes = (uint32_t)P.mv_words * 4u;
+      if (RICH && P.cell_reward)
+        fused_lanes_hbm<A, RICH, true>(R, P, env0, t0, n_steps, from, code_bytes, tape, log_envs, tape_steps);
+      else
+        fused_lanes_hbm<A, false, true>(R, P, env0, t0, n_steps, from, code_bytes, tape, log_envs, tape_steps);
+      continue;
+    }
     if (codes)
       stage_words(P.moves + (size_t)env0 * P.mv_words, n_here, P.mv_words, cap, my_words, lane);
     else
@@ -630,17 +1195,7 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
     if (!lds_worker) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
-      if (kTableMoves && pair_envs) {
-        // lanes l, l + unit, ... step env l; the halves of the wave share the Philox rounds
-        const int l = lane & (unit - 1);
-        if (l < n_here) {
-          const GlobalTable<A> tab{P.Q + (size_t)(env0 + l) * table};
-          if (n_steps >= kTouchMinSteps) tab.touch((int)table);
-          run_env_fast<A, true, RICH>(R, P, env0 + l, t0, n_steps, MovesLds<A>{my_words + l, unit},
-                                      RICH && P.cell_reward ? P.cell_reward + (size_t)(env0 + l) * P.S : nullptr,
-                                      tab);
-        }
-      } else if (live) {
+      if (live) {
         const GlobalTable<A> tab{P.Q + (size_t)env * table};
         if (n_steps >= kTouchMinSteps) tab.touch((int)table);
         if (kTableMoves)
