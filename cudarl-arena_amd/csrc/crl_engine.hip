@@ -327,6 +327,7 @@ struct FusedPlan {
   bool in_lds;     // ... with all tables in LDS
   bool words;      // ... beside their move words
   int env_bytes;   // ... bytes per env
+  int lds_waves;   // hybrid: waves of a workgroup that work on LDS tables ...
 };
 
 constexpr size_t kLdsPerWorkgroup = 160 * 1024;  // gfx950
@@ -340,7 +341,11 @@ constexpr size_t kStaticLdsReserve = 1024;
 constexpr int kHybridMinSteps = 64;
 constexpr int kStagedMovesMinSteps = 128;
 constexpr int kLdsMinSteps = 16;
+constexpr size_t kLdsBytesPerStep = 640;
 constexpr int kLongLaunchSteps = 4096;
+constexpr int kLaneWavesMinSteps = 8;
+constexpr int kLaneRoundsMinSteps = 384;
+constexpr size_t kTableBytesAtOnce = (size_t)512 << 20;
 
 // Configurations that run_lanes() steps: no goal test on the resulting cell, no sticky done,
 // no trace and no supplied stream.
@@ -376,6 +381,10 @@ bool plan_fused_lds(const crl_engine* e, int n_steps, FusedPlan* p) {
   for (int words = 1; words >= 0; --words) {
     const size_t bytes = 16 + (env_bytes[words] << log_envs) + tape_bytes(log_envs) + (shared && !words ? code_bytes : 0);
     if (((bytes + 1023) & ~(size_t)1023) * per_unit > kLdsPerWorkgroup) continue;
+    // (what a wave's tables take to move in and out, 640 bytes to a step saved: tables in LDS / in
+    // HBM, 4096 envs of 16x16, 16 KB to a wave, 16 / 32 steps 11.4 / 13.6, 10.7 / 14.1 us; 100 of
+    // 48x48 with 8 actions, 72 KB, 16 / 100 steps 17.5 / 31.0, 11.0 / 29.1)
+    if ((size_t)n_steps * kLdsBytesPerStep < (4 * e->K) << log_envs) return false;
     p->in_lds = p->lanes = p->fast = true;
     p->words = words != 0;
     p->rich = c.eps_mode >= CRL_EPS_EPISODE_MULT;
@@ -467,33 +476,79 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
   } else {
     p.rich = foldable && c.eps_mode != CRL_EPS_STEP_MULT && !(c.eps_mode == CRL_EPS_FIXED && c.reward_flags == 0);
     p.fast = foldable && c.eps_mode != CRL_EPS_STEP_MULT;
-    // Hybrid workgroups when 32 whole tables (padded by one row against bank
-    // conflicts), the LDS wave's maps and at least one table wave's maps fit into
-    // LDS.  One workgroup per compute unit (the LDS holds no second one); the envs
-    // in flight on HBM tables set how many 64-env waves work beside the LDS wave.
-    p.tab_stride = (int)e->K + 4;
+    // Hybrid workgroups: some waves work on HBM tables, the others on whole tables in LDS.
+    // One workgroup per compute unit (the LDS holds no second one).
     const size_t map_lds = (size_t)e->map_words * 64 * 4;
     const size_t mv_lds = (size_t)e->mv_words * 64 * 4;
-    const size_t lds_wave = p.fast ? (size_t)e->mv_words * crl::kTicketEnvs * 4 : map_lds;
-    const size_t tables_lds = (size_t)crl::kTicketEnvs * p.tab_stride * 4;
+    const int most_log_envs = e->A == 8 ? 3 : 4;  // an env to A lanes: the most that a wave has lanes for
     const long tickets = (e->N + crl::kTicketEnvs - 1) / crl::kTicketEnvs;
     // (not with per-cell rewards: they would stay in HBM, one request per step, and
     // a worker that waits for memory every step has no use for tables in LDS)
-    const bool fits = e->K % 4 == 0 && map_lds + lds_wave + tables_lds <= kLdsPerWorkgroup && !p.rich;
-    // ... and (automatic) when the tables outgrow the caches: while they all fit,
-    // plain waves on every SIMD are faster (16x16 maps, env-steps/s plain / hybrid:
-    // 32,768 envs 5.7e10 / 4.6e10, 65,536 envs 5.5e10 / 6.3e10, 262,144 envs 6.1e10 / 8.1e10)
-    const bool outgrown = (size_t)e->N * e->K * sizeof(float) > kTableBytesInFlight;
+    bool fits = !p.rich;
+    int hbm_waves = 0;
+    if (p.fast) {
+      // The folded loop's LDS waves give an env A lanes: two table waves, and beside them as
+      // many LDS waves as there is room for up to three.  1M envs, 16x16 maps, table + LDS
+      // waves: 3 + 1 7.7e10, 2 + 2 9.0e10, 3 + 2 8.4e10; 8x8: 2 + 2 1.16e11, 2 + 3 1.27e11;
+      // 8 actions, 16x16: 2 + 1 4.2e10, 2 + 2 4.7e10, 3 + 2 4.2e10.
+      hbm_waves = 2;
+      p.log_envs = most_log_envs;
+      p.tape_steps = tape_steps_for(p.log_envs);
+      p.env_bytes = (int)(((4 * e->K + (size_t)e->mv_words * 4 + 15) & ~(size_t)15) + 16);
+      const size_t wave_lds = ((size_t)p.env_bytes << p.log_envs) + tape_bytes(p.log_envs);
+      p.lds_waves = 3;
+      while (p.lds_waves > 0 && 16 + hbm_waves * map_lds + p.lds_waves * wave_lds > kLdsPerWorkgroup) --p.lds_waves;
+      fits = fits && p.lds_waves > 0;
+      p.lds = 16 + hbm_waves * map_lds + p.lds_waves * wave_lds;
+      // (asked for beyond that: what keeps a second workgroup off the compute unit, and the room
+      // that 32 padded tables with their codes and three waves' maps take, the same for all
+      // plans of a table size where it fits)
+      const size_t alone = kLdsPerWorkgroup / 2 + 1024;
+      const size_t room = 3 * map_lds + (size_t)crl::kTicketEnvs * 4 * (e->K + 4 + (size_t)e->mv_words);
+      p.lds = std::max({p.lds, alone, room <= kLdsPerWorkgroup ? room : 0});
+    } else {
+      // The general loop's: 32 whole tables (padded by one row against bank conflicts), the
+      // LDS wave's maps and at least one table wave's.
+      p.tab_stride = (int)e->K + 4;
+      p.lds_waves = 1;
+      const size_t rest = map_lds + (size_t)crl::kTicketEnvs * p.tab_stride * 4;
+      fits = fits && e->K % 4 == 0 && map_lds + rest <= kLdsPerWorkgroup;
+      // at most three, so that the LDS wave has a SIMD to itself
+      hbm_waves = (int)std::min<long>(3, std::max<long>(1, resident / (64L * kComputeUnits)));
+      while (hbm_waves > 1 && hbm_waves * map_lds + rest > kLdsPerWorkgroup) --hbm_waves;
+      p.lds = hbm_waves * map_lds + rest;
+    }
+    // Lane waves: an env to A lanes, one wave to a workgroup.
+    // (one wave to a compute unit in long launches of small batches, whose rows are in the caches
+    // most of the time; a wave to a SIMD in shorter ones, where most steps wait for a first use of
+    // a line, and the fewer envs a wave has the less often: 4096 envs of 32x32, 256 steps 108 / 98 us)
+    const long spread = n_steps > kLongLaunchSteps ? kComputeUnits : 4L * kComputeUnits;
+    int lane_log_envs = most_log_envs;
+    while (lane_log_envs > 0 && (e->N + (1L << lane_log_envs) - 1) >> lane_log_envs < spread) --lane_log_envs;
+    const size_t lane_lds = 16 + tape_bytes(lane_log_envs) + ((size_t)e->mv_words * 4 << lane_log_envs);
+    const long lane_fit = lane_lds <= kLdsPerWorkgroup ? (long)(kLdsPerWorkgroup / ((lane_lds + 1023) & ~(size_t)1023)) : 0;  // waves of a compute unit
+    const long lane_units = (e->N + (1L << lane_log_envs) - 1) >> lane_log_envs;
+    const bool lanes_can = lanes_rules(e) && (e->K * sizeof(float)) << lane_log_envs < (size_t)1 << 32;
+    const size_t all_tables = (size_t)e->N * e->K * sizeof(float);
+    const bool outgrown = all_tables > kTableBytesInFlight;
+    // All envs at once: 24 waves to a compute unit are what the registers hold (80,000 envs of
+    // 5x5 in one round 266 us, in two 361), 20 where the tables outgrow the caches - there 24
+    // lose to the hybrid (98,000 envs of 16x16, 500 steps: 1294 / 650 us) and 15 to 20 win over
+    // it and over 64-env waves (60,000 of 16x16, 64 / 500 steps: 143 / 566 hybrid, 86 / 420;
+    // 40,000 of 20x20 with 8 actions, 130 steps: 212, 163) up to about 512 MB (65,536 of 32x32,
+    // 1 GB, 300 steps: 503, 506).
+    const bool lanes_at_once = lanes_can && lane_units <= kComputeUnits * std::min(lane_fit, outgrown ? 20L : 24L) &&
+                               all_tables <= kTableBytesAtOnce;
+    // ... (automatic) when the tables outgrow the caches: while they all fit, other plans are
+    // faster (16x16 maps, 30,000 envs: 3.5e10 hybrid, 5.9e10 with lane waves); and where lane
+    // waves could step what is left to the general loop, they are faster too (262,144 envs of
+    // 16x16 with a zero-floored maximum: 5.1e10 general hybrid, 6.4e10)
     p.hybrid = fits && (e->fused_variant == 2 ||
-                        (e->fused_variant == 0 && outgrown && n_steps >= kHybridMinSteps));
+                        (e->fused_variant == 0 && outgrown && n_steps >= kHybridMinSteps &&
+                         (lanes_can ? p.fast && (!lanes_at_once || e->resident_envs > 0) : true)));
     if (p.hybrid) {
       p.grid = (int)std::min<long>(kComputeUnits, (tickets + 8) / 9);
-      // at most three, so that the LDS wave has a SIMD to itself (1M envs, 8x8 / 12x12
-      // maps: 1.11e11 / 1.00e11 env-steps/s with three table waves, 1.00e11 / 8.4e10 with four)
-      long hbm_waves = std::min<long>(3, std::max<long>(1, resident / (64L * p.grid)));
-      while (hbm_waves * map_lds + lds_wave + tables_lds > kLdsPerWorkgroup) --hbm_waves;
-      p.block = 64 * ((int)hbm_waves + 1);
-      p.lds = hbm_waves * map_lds + lds_wave + tables_lds;
+      p.block = 64 * (hbm_waves + p.lds_waves);
     } else {
       long waves = 4, workers;  // waves per workgroup, 64-env workers in flight
       if (tickets / 2 < 4 * kComputeUnits) {
@@ -517,33 +572,39 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       // staging the codes (four times the class map) pays off over a long launch only:
       // 1M envs of config 4, one step per launch 7.7e9 -> 1.4e10 with class maps, 48 steps 3.6e10 -> 3.7e10
       p.moves = p.fast && waves * mv_lds <= kLdsPerWorkgroup && n_steps >= kStagedMovesMinSteps;
-      // Few enough envs that a wave of 16 (8 actions: 8) still finds a SIMD that has at most
-      // one other: A lanes to an env - or fewer envs to a wave while that gives more compute
-      // units a wave of their own.
-      long units = tickets;  // tickets as the kernel counts them
-      if (lanes_rules(e) && waves == 1 && tickets <= 2 * kComputeUnits) {
-        // (one wave to a compute unit in long launches, whose rows are in the caches most of the
-        // time; a wave to a SIMD in shorter ones, where most steps wait for a first use of a line,
-        // and the fewer envs a wave has the less often: 4096 envs of 32x32, 256 steps 108 / 98 us)
-        const long spread = n_steps > kLongLaunchSteps ? kComputeUnits : 4L * kComputeUnits;
-        int log_envs = e->A == 8 ? 3 : 4;
-        while (log_envs > 0 && (e->N + (1L << log_envs) - 1) >> log_envs < spread) --log_envs;
-        const size_t lds = 16 + tape_bytes(log_envs) + ((size_t)e->mv_words * 4 << log_envs);
-        if (lds <= kLdsPerWorkgroup && (e->K * sizeof(float)) << log_envs < (size_t)1 << 32) {
-          p.fast = p.moves = p.lanes = true;
-          p.rich = c.eps_mode >= CRL_EPS_EPISODE_MULT || c.reward_flags != 0;
-          p.log_envs = log_envs;
-          p.tape_steps = tape_steps_for(log_envs);
-          units = (e->N + (1L << log_envs) - 1) >> log_envs;
-          p.grid = (int)std::min<long>(std::max<long>(1, resident >> log_envs), units);
-          // (where there is a compute unit for every workgroup, LDS for no second one beside it)
-          p.lds = p.grid <= kComputeUnits ? std::max(lds, std::min<size_t>(mv_lds, kLdsMapLimitBytes)) : lds;
-        }
+      // Few envs: A lanes to each, in as many waves as leave no more than two to a SIMD.  More:
+      // all at once in lane waves, for launches of some steps (30,000 envs of 16x16, 4 / 8 / 16
+      // steps: 15 / 28 / 35 us, 15 / 26 / 28).  Else lane waves in even rounds, of as many waves as
+      // leave their rows in the caches most of the time (16x16 maps, waves per compute unit:
+      // 4 actions, 524,288 envs 4: 4.8e10, 8: 6.2e10, 12: 5.7e10, 16: 5.0e10; 8 actions, 262,144
+      // envs 8: 3.7e10, 12: 4.2e10, 16: 4.0e10) - not with fewer of them because the codes take
+      // too much LDS (50,000 envs of 48x48, 4 waves: 643 / 700 us), and where the folded loop would
+      // do as well in launches long enough only (4 actions, 64-env / lane waves: 65,536 envs of
+      // 32x32, 64 / 300 / 1000 steps 131 / 503 / 1487, 179 / 517 / 1471; 30,000 of 24x24 - half
+      // the SIMDs without a 64-env wave - 130 steps 116, 99).
+      const bool small = waves == 1 && tickets <= 2 * kComputeUnits;
+      const long per_round = kComputeUnits * (!outgrown ? 16L : e->A == 8 ? 12L : 8L);
+      const long rounds = small || lanes_at_once ? 1 : (lane_units + per_round - 1) / per_round;
+      const long lane_waves = (lane_units + rounds - 1) / rounds;
+      const int rounds_min_steps = !(p.fast && outgrown)                                ? kLaneWavesMinSteps
+                                   : e->A == 4 && (long)e->N <= kMinEnvsInFlight ? kStagedMovesMinSteps
+                                                                                 : kLaneRoundsMinSteps;
+      const bool rounds_ok = lane_waves <= kComputeUnits * lane_fit && n_steps >= rounds_min_steps;
+      if (lanes_can && (small ? lane_fit > 0 : lanes_at_once ? n_steps >= kLaneWavesMinSteps : rounds_ok)) {
+        p.fast = p.moves = p.lanes = true;
+        p.rich = c.eps_mode >= CRL_EPS_EPISODE_MULT || c.reward_flags != 0;
+        p.log_envs = lane_log_envs;
+        p.tape_steps = tape_steps_for(lane_log_envs);
+        const long most = e->resident_envs > 0 ? std::max<long>(1, resident >> lane_log_envs) : lane_waves;
+        p.grid = (int)std::min<long>(lane_units, most);
+        p.block = 64;
+        // (where there is a compute unit for every workgroup, LDS for no second one beside it)
+        p.lds = p.grid <= kComputeUnits ? std::max(lane_lds, std::min<size_t>(mv_lds, kLdsMapLimitBytes)) : lane_lds;
       }
       // Tickets dealt by position instead of drawn from a counter: the workers of this plan
       // all take the same time, and 16,384 draws from one counter take 0.38 ms however short
       // the launch (1M envs: the whole of a 4-step launch, half of a 20-step one).
-      p.fixed = n_steps < kHybridMinSteps || (p.lanes && p.grid >= units);
+      p.fixed = n_steps < kHybridMinSteps || (p.lanes && p.grid >= lane_units);
       if (!p.lanes) p.lds = waves * (p.moves ? mv_lds : map_lds);
     }
   }
@@ -596,8 +657,12 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
     unsigned* tk = e->tk;
 #define CRL_LAUNCH_TICKETS(MODE, LDSW, MOVES)                                                       \
   hipLaunchKernelGGL((crl::k_fused_tickets<A, MODE, LDSW, MOVES>), g, b, p.lds, e->stream, R, P, t0, n, \
-                     tk, p.tab_stride, p.fixed ? 1 : 0, p.lanes ? 1 << p.log_envs : 0, p.tape_steps)
-    if (p.rich && p.moves)
+                     tk, p.tab_stride, p.fixed ? 1 : 0, p.tape_steps, p.lds_waves, p.env_bytes)
+    if (p.lanes && P.cell_reward)
+      hipLaunchKernelGGL((crl::k_fused_lanes<A, true>), g, b, p.lds, e->stream, R, P, t0, n, tk, p.fixed ? 1 : 0, p.log_envs, p.tape_steps);
+    else if (p.lanes)
+      hipLaunchKernelGGL((crl::k_fused_lanes<A, false>), g, b, p.lds, e->stream, R, P, t0, n, tk, p.fixed ? 1 : 0, p.log_envs, p.tape_steps);
+    else if (p.rich && p.moves)
       CRL_LAUNCH_TICKETS(2, false, true);
     else if (p.rich)
       CRL_LAUNCH_TICKETS(2, false, false);
@@ -1386,7 +1451,9 @@ int opt_in_ticket_kernels(crl_engine* e) {
       reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, true, false>),         \
       reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, false, true>),         \
       reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 2, false, true>),         \
-      reinterpret_cast<const void*>(&crl::k_fused_per_env<A, 1, 2>),                    \
+      reinterpret_cast<const void*>(&crl::k_fused_lanes<A, false>),                    \
+      reinterpret_cast<const void*>(&crl::k_fused_lanes<A, true>),                     \
+      reinterpret_cast<const void*>(&crl::k_fused_per_env<A, 1, 2>),                   \
       CRL_LDS_KERNELS(A, false, false), CRL_LDS_KERNELS(A, false, true),               \
       CRL_LDS_KERNELS(A, true, false), CRL_LDS_KERNELS(A, true, true)
 #define CRL_LDS_KERNELS(A, WORDS, EVENTS)                                              \

@@ -661,16 +661,15 @@ struct LaneLds {
   __device__ __forceinline__ At at(uint32_t offset) const { return first + offset; }
   __device__ __forceinline__ uint32_t offset(At p) const { return p - first; }
   static __device__ __forceinline__ float value(At p) { return *lds_at<float>(p); }
-  static __device__ __forceinline__ void fetch(At p, float& q, uint32_t& c) {
-    q = value(p);
-    c = *lds_at<uint32_t>(p + 4 * A);
-  }
+  // asks for what `word` needs / the lane's move word from that, when it has arrived
+  static __device__ __forceinline__ uint32_t code(At p) { return *lds_at<uint32_t>(p + 4 * A); }
+  static __device__ __forceinline__ uint32_t word(At, uint32_t code) { return code; }
   static __device__ __forceinline__ void store(At p, float v) { *lds_at<float>(p) = v; }
 };
 
 // Values in LDS (QL) or in HBM and the caches, the cells' move codes in LDS (CL) or global
 // memory, a byte per cell (two with 8 actions): the move word is worked out when the code
-// has arrived, seven instructions.
+// has arrived, four or five instructions.
 template <int A, bool QL, bool CL>
 struct LaneCodes {
   static constexpr uint32_t kRow = 4 * A;
@@ -684,12 +683,17 @@ struct LaneCodes {
   __device__ __forceinline__ At at(uint32_t offset) const { return offset; }
   __device__ __forceinline__ uint32_t offset(At p) const { return p; }
   __device__ __forceinline__ float value(At p) const { return *reinterpret_cast<const float*>(values + (QL ? p : values_at + p)); }
-  __device__ __forceinline__ void fetch(At p, float& q, uint32_t& c) const {
-    q = value(p);
+  __device__ __forceinline__ uint32_t code(At p) const {
     const uint32_t i = codes_at + p / (A == 4 ? kRow : kRow / 2);
-    const uint32_t code = A == 4 ? (uint32_t)codes[i] : (uint32_t)*reinterpret_cast<const uint16_t*>(codes + i);
+    return A == 4 ? (uint32_t)codes[i] : (uint32_t)*reinterpret_cast<const uint16_t*>(codes + i);
+  }
+  __device__ __forceinline__ uint32_t word(At p, uint32_t code) const {
+    // (classes from kTrap on leave the env where it is: that is the class's upper bit)
     const uint32_t cls = __builtin_amdgcn_ubfe(code, 2 * action, 2u);
-    c = move_word(action, cls < (uint32_t)kTrap ? p + (uint32_t)step : p, cls);
+    const uint32_t there = p + (uint32_t)step + (action << 29);
+    const uint32_t w = QL ? there - (uint32_t)__mul24((int)__builtin_amdgcn_ubfe(code, 2 * action + 1, 1u), step)  // (a table in LDS is small)
+                          : there - ((uint32_t)__builtin_amdgcn_sbfe((int)code, 2 * action + 1, 1u) & (uint32_t)step);
+    return w + (cls << 2);
   }
   __device__ __forceinline__ void store(At p, float v) const { *reinterpret_cast<float*>(values + (QL ? p : values_at + p)) = v; }
 };
@@ -734,9 +738,8 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
   }
   const int budget = EVENTS && R.max_episodes > 0 ? R.max_episodes : 0x7fffffff;
   bool going = live && episode < budget;
-  float q;
-  uint32_t c;
-  mem.fetch(at, q, c);
+  float q = mem.value(at);
+  uint32_t c = mem.word(at, mem.code(at));
   // (arrived before the loop starts: a value that may be in flight there makes every round
   // wait for everything, the last store's answer included)
   asm volatile("" : "+v"(q), "+v"(c), "+v"(reward), "+v"(left), "+v"(episode), "+v"(won), "+v"(limit), "+v"(eps_next));
@@ -770,10 +773,9 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
           const bool ends = left <= 0;
           typename Mem::At at_next = ends ? at_start : at2;
           asm("" : "+v"(at_next));  // (one address, not one per use)
+          const uint32_t code = mem.code(at_next);
           const float q2 = mem.value(at2);
-          float q_next;
-          uint32_t c_next;
-          mem.fetch(at_next, q_next, c_next);
+          float q_next = mem.value(at_next);
           reward = *lds_at<float>(cls);
           float by_cell = 0.0f;
           if (CELLS) {
@@ -793,7 +795,12 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
           const int len = whole - before + 1;
           left = ends ? whole : left;
           episode += ends ? 1 : 0;
-          __builtin_amdgcn_sched_barrier(0);  // all of the above while the values are on their way
+          // All of the above while the values are on their way.  (Without the barrier the move
+          // word's arithmetic moves up and waits for its code before the other reads are asked
+          // for: two trips to LDS in a row.  1M envs of 16x16 on LDS waves alone, with the codes
+          // staged eight loads at a time as well: 3.18e10 -> 3.60e10 env-steps/s.)
+          __builtin_amdgcn_sched_barrier(0);
+          const uint32_t c_next = mem.word(at_next, code);
           if (CELLS) reward = (base_cells || (cls - 4u) < 8u) ? by_cell : reward;  // (goal or trap, or any)
           if (EVENTS) {
             ret = ret + reward;
@@ -1069,6 +1076,55 @@ __global__ __launch_bounds__(256) void k_fused_per_env(const Rules R, const Ptrs
   }
 }
 
+// The same with per-env maps: one wave to a workgroup, which draws 1 << log_envs envs at a
+// time from a ticket counter (or is dealt them by position: fixed_tickets), stages their move
+// codes into its LDS and steps them for all n_steps, A lanes to an env.  What bounds it is the
+// wave's dependent chain - 45 instructions and a trip to the row, 0.26 us per step alone on its
+// SIMD, of which a wave with 64 envs pays the slowest of 64 trips and 150 instructions.
+// LDS: the rewards by class, the tape, the codes env by env.
+template <int A, bool CELLS>
+__global__ __launch_bounds__(64) void k_fused_lanes(const Rules R, const Ptrs P, const uint64_t t0, const int n_steps,
+                                                    unsigned* __restrict__ ticket, const int fixed_tickets,
+                                                    const int log_envs, const int tape_steps) {
+  extern __shared__ __align__(16) uint32_t lds[];
+  const int lane = threadIdx.x;
+  const unsigned n_tickets = (unsigned)(((long)P.N + (1 << log_envs) - 1) >> log_envs);
+  const size_t table = P.S * A;  // floats per table
+  uint32_t* tape = lds + 4;
+  uint32_t* words = tape + ((tape_steps + 1) << log_envs);
+  write_rewards(R, reinterpret_cast<float*>(lds), lane);
+  if (fixed_tickets && blockIdx.x == 0 && lane == 0) {
+    ticket[1] = (unsigned)P.N;
+    ticket[2] = 0u;
+  }
+  unsigned stepped = 0;  // envs this worker has stepped
+  for (unsigned round = 0;; ++round) {
+    unsigned base = round * gridDim.x + blockIdx.x;
+    if (!fixed_tickets) {
+      if (lane == 0) base = atomicAdd(ticket, 1u);
+      base = (unsigned)__builtin_amdgcn_readfirstlane((int)base);
+    }
+    if (base >= n_tickets) break;  // every worker gets here: the number only grows
+    const int env0 = (int)base << log_envs;
+    const int n_here = min(1 << log_envs, P.N - env0);
+    stepped += (unsigned)n_here;
+    wave_fence();
+    copy_words(P.moves + (size_t)env0 * P.mv_words, n_here * P.mv_words, words, lane);
+    // (GlobalTable::touch for all of the wave's envs, whose tables are one run in HBM: where
+    // they go through the chip in rounds, a launch meets most lines for the first time)
+    if (!fixed_tickets && n_steps >= kTouchMinSteps && table <= (size_t)kTouchFloats) {
+      const float* q = P.Q + (size_t)env0 * table;
+      float acc = 0.0f;
+      for (int i = lane * 32; i < n_here * (int)table; i += 64 * 32) acc += q[i];
+      asm volatile("" ::"v"(acc));
+    }
+    wave_fence();
+    fused_lanes_hbm<A, CELLS, true>(R, P, env0, t0, n_steps, reinterpret_cast<const unsigned char*>(words),
+                                    (uint32_t)P.mv_words * 4u, tape, log_envs, tape_steps);
+  }
+  if (!fixed_tickets && lane == 0 && stepped != 0u) atomicAdd(ticket + 1, stepped);
+}
+
 // Per-env tables with per-env maps small enough for LDS: every wave is an
 // independent worker that draws env ranges from one ticket counter (32 envs per
 // ticket), stages its envs' maps into its own LDS slice ([word][lane]: conflict
@@ -1076,20 +1132,20 @@ __global__ __launch_bounds__(256) void k_fused_per_env(const Rules R, const Ptrs
 // how many bytes of their tables - are live on the chip at once: few enough and
 // the rows an env keeps returning to are still in the last-level cache.
 //
-// All waves of a workgroup but the last step 64 envs each against tables in HBM /
-// the caches, and spend most of their time waiting for one row per step.  With
-// LDSW the last wave uses the idle issue slots and the LDS: it stages the WHOLE
-// tables of 32 envs into LDS, steps them there and writes the tables back.  The
-// split between the two kinds follows their speed; which worker steps an env does
-// not change its results.
+// All waves of a workgroup but the LDS waves step 64 envs each against tables in HBM / the
+// caches, and spend most of their time waiting for one row per step.  With LDSW the last
+// `lds_waves` waves use the idle issue slots and the LDS: they stage the WHOLE tables of their
+// envs into LDS, step them there and write the tables back.  The split between the two kinds
+// follows their speed; which worker steps an env does not change its results.
 //
-// MODE 0 is the general loop; 1 and 2 select the folded loop (run_env_fast; 2: its
-// variant with per-cell rewards and per-episode epsilon), which works on move
-// codes: the LDS wave always stages the pre-built codes of its envs; the table
-// waves stage them too with MOVES, and otherwise stage the (four times smaller)
-// class maps and derive the codes while their row loads are in flight.
-// `lane_envs`: the batch is too small to fill the chip with 64-env waves, and the (one) wave
-// of a workgroup takes that many envs a ticket with A lanes to each.
+// MODE 0 is the general loop (LDSW: one LDS wave of 32 envs); 1 and 2 select the folded loop
+// (run_env_fast; 2: its variant with per-cell rewards and per-episode epsilon), which works on
+// move codes: with MOVES the table waves stage the pre-built codes, otherwise the (four times
+// smaller) class maps, and derive the codes while their row loads are in flight.  MODE 1's LDS
+// waves take 64 / A envs, A lanes to each (run_lanes; what bounds them is one env's dependent
+// chain, 0.21 us per step on a SIMD of its own).  Three table waves and one LDS wave of 32 envs
+// with two lanes each / two table waves and the LDS waves of 64 / A envs that fit, launch after
+// launch: 1M envs of 16x16, 1000 steps 12.46 / 12.23 ms, of 8x8 8.83 / 8.26 ms.
 constexpr int kTicketEnvs = 32;
 
 // `count` envs' words (`wpe` per env, contiguous in HBM) into [word][lane]; eight
@@ -1113,6 +1169,42 @@ __device__ __forceinline__ void stage_words(const uint32_t* __restrict__ src, co
   for (int i = i0 + lane; i < total; i += 64) put(i, __builtin_nontemporal_load(src + i));
 }
 
+// `per` pieces each of n consecutive envs - one contiguous run in HBM - into LDS, env_bytes
+// apart, or out again, by one wave.  Read once and written once per launch: marked
+// non-temporal so that they do not push the table waves' rows out of the L2.
+__device__ __forceinline__ uint32_t stream_load(const uint32_t* p) { return __builtin_nontemporal_load(p); }
+__device__ __forceinline__ float4 stream_load(const float4* p) { return stream_load4(p); }
+__device__ __forceinline__ void stream_store(const uint32_t v, uint32_t* p) { __builtin_nontemporal_store(v, p); }
+__device__ __forceinline__ void stream_store(const float4 v, float4* p) { stream_store4(v, p); }
+template <bool IN, class T>
+__device__ __forceinline__ void strided_copy(T* __restrict__ g, const int per, const int n, unsigned char* envs,
+                                             const int env_bytes, const int lane) {
+  const int total = n * per;
+  const int de = 64 / per, dp = 64 - de * per;  // 64 pieces on: that many envs and pieces
+  int e = lane / per, piece = lane - e * per;
+  constexpr int kFlight = 8;
+  for (int i0 = lane; i0 < total; i0 += 64 * kFlight) {
+    T v[kFlight];
+    T* at[kFlight];
+#pragma unroll
+    for (int u = 0; u < kFlight; ++u) {
+      at[u] = reinterpret_cast<T*>(envs + (size_t)e * env_bytes) + piece;
+      if (i0 + 64 * u < total) v[u] = IN ? stream_load(g + i0 + 64 * u) : *at[u];
+      e += de;
+      piece += dp;
+      const bool wrap = piece >= per;
+      piece -= wrap ? per : 0;
+      e += wrap ? 1 : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < kFlight; ++u)
+      if (i0 + 64 * u < total) {
+        if (IN) *at[u] = v[u];
+        else stream_store(v[u], g + i0 + 64 * u);
+      }
+  }
+}
+
 template <int A, int MODE, bool LDSW, bool MOVES>
 __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules R, const Ptrs P,
                                                                      const uint64_t t0,
@@ -1120,27 +1212,29 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
                                                                      unsigned* __restrict__ ticket,
                                                                      const int tab_stride,
                                                                      const int fixed_tickets,
-                                                                     const int lane_envs,
-                                                                     const int tape_steps) {
+                                                                     const int tape_steps,
+                                                                     const int lds_waves,
+                                                                     const int env_bytes) {
   constexpr bool FAST = MODE >= 1;  // the folded loop ...
   constexpr bool RICH = MODE == 2;  // ... in its variant with per-cell rewards and per-episode epsilon
+  constexpr bool kLaneTables = LDSW && FAST;  // the LDS waves give an env A lanes
   extern __shared__ __align__(16) uint32_t lds[];
-  const int n_waves = (int)(blockDim.x >> 6);  // with LDSW the last one works on LDS tables
+  const int n_waves = (int)(blockDim.x >> 6);  // with LDSW the last `lds_waves` work on LDS tables
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const bool lds_worker = LDSW && wave == n_waves - 1;
-  // LDS: one slice per table wave, the LDS wave's slice, the tables
+  const bool lds_worker = LDSW && wave >= n_waves - lds_waves;
+  // LDS: (kLaneTables) the rewards by class; one slice per table wave; then kLaneTables:
+  // [LDS wave][its envs: rows, then move codes; its tape], else the LDS wave's slice, the tables
   constexpr bool kTableMoves = FAST && MOVES;
   const int slice = (kTableMoves ? P.mv_words : P.map_words) * 64;
-  const int lds_slice = !LDSW ? 0 : FAST ? P.mv_words * kTicketEnvs : P.map_words * 64;
-  uint32_t* my_words = lds + wave * slice;  // (the LDS wave is the last one)
-  float* tabs = reinterpret_cast<float*>(lds + (n_waves - 1) * slice + lds_slice);
-  // envs per ticket: 32, or what a thin table wave steps (never with an LDS wave beside it)
-  const int unit = (FAST && MOVES && lane_envs) ? lane_envs : kTicketEnvs;
+  uint32_t* my_words = lds + (kLaneTables ? 4 : 0) + wave * slice;  // (the LDS waves are the last ones)
+  float* tabs = reinterpret_cast<float*>(lds + (n_waves - 1) * slice + P.map_words * 64);
+  // envs per ticket: 32, or what a wave that gives an env A lanes steps
+  constexpr int unit = kLaneTables ? 64 / A : kTicketEnvs;
   const unsigned n_tickets = (unsigned)((P.N + unit - 1) / unit);
-  const bool thin = lds_worker || (FAST && MOVES && lane_envs);
-  const int cap = thin ? unit : 64;
-  const unsigned take = thin ? 1u : 2u;
+  const int cap = lds_worker ? unit : 64;
+  const unsigned take = lds_worker ? 1u : 64u / (unsigned)unit;
+  if (kLaneTables && lds_worker) write_rewards(R, reinterpret_cast<float*>(lds), lane);  // (every one of them, the same)
   const size_t table = P.S * A;  // floats per table
 
   // fixed_tickets: the tickets are dealt by position, wave after wave, round after round
@@ -1155,10 +1249,10 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
   for (unsigned round = 0;; ++round) {
     unsigned base = 0;
     if (fixed_tickets) {
-      base = ((round * gridDim.x + blockIdx.x) * (unsigned)n_waves + (unsigned)__builtin_amdgcn_readfirstlane(wave)) * take;
+      base = ((round * gridDim.x + blockIdx.x) * (unsigned)n_waves + (unsigned)wave) * take;
     } else {
       if (lane == 0) base = atomicAdd(ticket, take);
-      base = (unsigned)__builtin_amdgcn_readfirstlane((int)base);
+      base = __shfl(base, 0);
     }
     if (base >= n_tickets) break;  // every worker gets here: the counter only grows
     const int env0 = (int)base * unit;
@@ -1169,21 +1263,24 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
 
     // this worker's maps: contiguous in HBM, transposed into [word][lane]
     __builtin_amdgcn_wave_barrier();
-    const bool codes = FAST && (MOVES || lds_worker);
-    if (kTableMoves && lane_envs) {
-      // LDS: rewards, tape, the codes env by env
-      const int log_envs = 31 - __builtin_clz((unsigned)lane_envs);
-      uint32_t* tape = lds + 4;
-      uint32_t* words = tape + ((tape_steps + 1) << log_envs);
-      write_rewards(R, reinterpret_cast<float*>(lds), lane);
-      copy_words(P.moves + (size_t)env0 * P.mv_words, n_here * P.mv_words, words, lane);
+    const bool codes = kTableMoves;
+    if (kLaneTables && lds_worker) {
+      constexpr int log_envs = A == 8 ? 3 : 4;
+      unsigned char* envs = reinterpret_cast<unsigned char*>(lds + 4 + (n_waves - lds_waves) * slice) +
+                            (size_t)(wave - (n_waves - lds_waves)) * (((size_t)env_bytes + 4u * (tape_steps + 1)) << log_envs);
+      strided_copy<true>(reinterpret_cast<uint32_t*>(const_cast<uint32_t*>(P.moves)) + (size_t)env0 * P.mv_words, P.mv_words,
+                         n_here, envs + table * 4, env_bytes, lane);
+      float4* tables = reinterpret_cast<float4*>(P.Q + (size_t)env0 * table);
+      strided_copy<true>(tables, (int)(table / 4), n_here, envs, env_bytes, lane);
       wave_fence();
-      const unsigned char* from = reinterpret_cast<const unsigned char*>(words);
-      const uint32_t code_bytes = (uint32_t)P.mv_words * 4u;
-      if (RICH && P.cell_reward)
-        fused_lanes_hbm<A, RICH, true>(R, P, env0, t0, n_steps, from, code_bytes, tape, log_envs, tape_steps);
-      else
-        fused_lanes_hbm<A, false, true>(R, P, env0, t0, n_steps, from, code_bytes, tape, log_envs, tape_steps);
+      const int slot = lane / A;
+      const uint32_t action = (uint32_t)lane & (A - 1);
+      unsigned char* mine = envs + (size_t)(slot < n_here ? slot : 0) * env_bytes;
+      const LaneCodes<A, true, true> mem{mine + 4 * action, 0u, mine + table * 4, 0u, action, row_step<A>(R, action, 4 * A)};
+      run_lanes<A, false, false>(R, P, env0, slot < n_here, t0, n_steps, mem,
+                                 reinterpret_cast<uint32_t*>(envs + ((size_t)env_bytes << log_envs)), log_envs, tape_steps, nullptr);
+      wave_fence();
+      strided_copy<false>(tables, (int)(table / 4), n_here, envs, env_bytes, lane);
       continue;
     }
     if (codes)
@@ -1235,16 +1332,7 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
       for (int i = i0 + lane; i < total4; i += 64) put(i, ld(i));
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
-      if (FAST) {
-        // lanes l and l + 32 both step env l of the ticket
-        const int l = lane & (kTicketEnvs - 1);
-        if (l < n_here) {
-          const LdsTable<A> tab{tabs + l * tab_stride};
-          run_env_fast<A, true, RICH>(R, P, env0 + l, t0, n_steps, MovesLds<A>{my_words + l, kTicketEnvs},
-                                      RICH && P.cell_reward ? P.cell_reward + (size_t)(env0 + l) * P.S : nullptr,
-                                      tab);
-        }
-      } else if (live) {
+      if (live) {
         const LdsTable<A> tab{tabs + lane * tab_stride};
         run_env_steps<A>(R, P, env, t0, n_steps, MovesFromMap<A>{my_words + lane, R.W, R.H},
                          P.map + (size_t)env * P.map_words, cr, tab);

@@ -132,9 +132,10 @@ int crl_sync(crl_engine* e);
 int crl_set_resident_envs(crl_engine* e, int32_t n_envs);
 /* Tuning (no reference counterpart): kernel of crl_run_fused.  0 = automatic.
  * Per-env tables: 1 = plain (every wave steps envs against tables in HBM),
- * 2 = hybrid (the last wave of each workgroup steps envs whose whole tables it holds
- * in LDS; used only when 32 tables fit; automatic picks it for launches of at
- * least 64 steps).  Shared table: 1 = two launches per step; 2 = all steps of a
+ * 2 = hybrid (the last waves of each workgroup step envs whose whole tables they hold
+ * in LDS; used only where the tables of 64 / actions envs fit, with the general loop 32;
+ * automatic picks it for launches of at least 64 steps on tables that outgrow the
+ * caches).  Shared table: 1 = two launches per step; 2 = all steps of a
  * call in one launch whose 256 workgroups exchange block sums and table values
  * through device-scope loads and stores (needs every workgroup resident at once:
  * at most 65,536 envs and 16,384 table entries, else two launches per step);

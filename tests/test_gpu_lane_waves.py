@@ -1,0 +1,63 @@
+"""Waves that give an env A lanes beside and instead of waves of 64 envs: batches past the
+small ones all at once and in rounds, and hybrid workgroups of table waves and one to three
+LDS waves.  At batch sizes that leave the last wave and the last ticket part-filled, on maps
+whose codes end inside a word, against the oracle bit for bit."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+STATE = ("s", "ep_step", "episode", "reward", "done", "action")
+
+
+def check(gpu, oracle, N, W, H, A, chunks, resident=0, variant=0, hybrid=False, cells=0, block=None, **kw):
+    cr = None
+    if cells:
+        cls, start, cr = gpu.gen_maps_noise(3, N, W, H, 4, 0.2, 0.3, 5.0)
+    else:
+        cls, start = gpu.gen_maps_bernoulli(7, N, N, W, H, 0.12, 0.08)
+    cfg = gpu.make_config(N, W, H, n_actions=A, reward_flags=cells, lr=0.3, gamma=0.9, seed=N + A, trap_reward=-0.5,
+                          **{"eps0": 0.4, "episode_len": 9, **kw})
+    with gpu.Engine(cfg, 0) as eng:
+        eng.set_maps(cls, start, cr)
+        eng.set_resident_envs(resident)
+        eng.set_fused_variant(variant)
+        for c in chunks:
+            plan = eng.fused_kernel_info(c)
+            assert ("hbm+lds" in plan["name"]) == hybrid, plan
+            assert block is None or plan["block"] == block, plan
+            eng.run_fused(c)
+            assert sum(eng.fused_split()) == N
+        q, st = eng.q_get(0, N), eng.get_state()
+        stats = eng.episode_stats() if cfg.track_returns else None
+    Q = np.zeros((N, W * H, A), np.float32)
+    ost = oracle.new_state(cfg, start)
+    ostats = oracle.new_stats(N) if cfg.track_returns else None
+    oracle.run(cfg, cls, cr, start, Q, ost, 0, sum(chunks), stats=ostats)
+    for k in STATE:
+        assert np.array_equal(st[k], ost[k]), k
+    assert np.array_equal(q.reshape(Q.shape), Q)
+    for k in stats or ():
+        assert np.array_equal(stats[k], ostats[k]), k
+
+
+# one wave to a workgroup; `resident`: in rounds drawn from the counter (from 64 steps on) or
+# dealt by position
+@pytest.mark.parametrize("N,W,H,A,chunks,resident,kw", [
+    (16387, 13, 11, 4, (8, 9, 64), 0, dict()),
+    (16385, 9, 7, 8, (8, 31), 0, dict(eps_mode=3, eps0=1.0, eps_end=0.1, eps_span=4, max_mode=1)),
+    (33001, 5, 3, 4, (65, 20), 3000, dict()),
+    (33001, 5, 3, 8, (65, 20), 3000, dict(track_returns=1, max_episodes=3)),
+    (20003, 7, 5, 4, (130, 12), 4096, dict(cells=1, eps_mode=3, eps0=0.9, eps_end=0.2, eps_span=5)),
+    (20003, 7, 5, 8, (130, 12), 0, dict(cells=3, max_mode=1)),
+    (99001, 9, 7, 4, (70,), 0, dict(max_mode=1)),  # more than the registers hold at once: two even rounds
+])
+def test_lane_waves(gpu, oracle, N, W, H, A, chunks, resident, kw):
+    check(gpu, oracle, N, W, H, A, chunks, resident, block=64, **kw)
+
+
+# table waves and LDS waves: three, two and one of them, fewer envs than a wave, than a round
+@pytest.mark.parametrize("N,W,H,A,lds_waves", [(4099, 6, 5, 4, 3), (4099, 6, 5, 8, 3), (2051, 16, 16, 4, 2), (1033, 16, 16, 8, 2),
+                                               (1037, 20, 19, 4, 1), (521, 23, 21, 8, 1), (1, 16, 16, 4, 2), (7, 3, 3, 8, 3)])
+def test_hybrid_workgroups(gpu, oracle, N, W, H, A, lds_waves):
+    check(gpu, oracle, N, W, H, A, (67, 130, 1), variant=2, hybrid=True, block=64 * (2 + lds_waves))
