@@ -573,8 +573,9 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       // 1M envs of config 4, one step per launch 7.7e9 -> 1.4e10 with class maps, 48 steps 3.6e10 -> 3.7e10
       p.moves = p.fast && waves * mv_lds <= kLdsPerWorkgroup && n_steps >= kStagedMovesMinSteps;
       // Few envs: A lanes to each, in as many waves as leave no more than two to a SIMD.  More:
-      // all at once in lane waves, for launches of some steps (30,000 envs of 16x16, 4 / 8 / 16
-      // steps: 15 / 28 / 35 us, 15 / 26 / 28).  Else lane waves in even rounds, of as many waves as
+      // all at once in lane waves, in place of the folded loop for launches of some steps (30,000
+      // envs of 16x16, 4 / 8 / 16 steps: 23 / 28 / 35 us, 23 / 26 / 28), of the general loop always
+      // (30,000 of 16x16, one step: 12.5 us, 8.9; in rounds 200,000, 2 / 6 steps: 34 / 75, 50 / 74).  Else lane waves in even rounds, of as many waves as
       // leave their rows in the caches most of the time (16x16 maps, waves per compute unit:
       // 4 actions, 524,288 envs 4: 4.8e10, 8: 6.2e10, 12: 5.7e10, 16: 5.0e10; 8 actions, 262,144
       // envs 8: 3.7e10, 12: 4.2e10, 16: 4.0e10) - not with fewer of them because the codes take
@@ -586,11 +587,12 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       const long per_round = kComputeUnits * (!outgrown ? 16L : e->A == 8 ? 12L : 8L);
       const long rounds = small || lanes_at_once ? 1 : (lane_units + per_round - 1) / per_round;
       const long lane_waves = (lane_units + rounds - 1) / rounds;
-      const int rounds_min_steps = !(p.fast && outgrown)                                ? kLaneWavesMinSteps
+      const int at_once_min_steps = p.fast ? kLaneWavesMinSteps : 1;
+      const int rounds_min_steps = !(p.fast && outgrown)                         ? kLaneWavesMinSteps
                                    : e->A == 4 && (long)e->N <= kMinEnvsInFlight ? kStagedMovesMinSteps
                                                                                  : kLaneRoundsMinSteps;
       const bool rounds_ok = lane_waves <= kComputeUnits * lane_fit && n_steps >= rounds_min_steps;
-      if (lanes_can && (small ? lane_fit > 0 : lanes_at_once ? n_steps >= kLaneWavesMinSteps : rounds_ok)) {
+      if (lanes_can && (small ? lane_fit > 0 : lanes_at_once ? n_steps >= at_once_min_steps : rounds_ok)) {
         p.fast = p.moves = p.lanes = true;
         p.rich = c.eps_mode >= CRL_EPS_EPISODE_MULT || c.reward_flags != 0;
         p.log_envs = lane_log_envs;
@@ -695,6 +697,7 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
 #undef CRL_LAUNCH_PER_ENV
 }
 
+constexpr int kScanBlocks = 2;
 constexpr size_t kHandoffLimitBytes = (size_t)128 << 20;
 
 int ceil_log2(size_t v) {
@@ -739,8 +742,11 @@ crl::ReduceGeom reduce_geom_within(const crl_engine* e, int n, size_t limit) {
   return G;
 }
 
-// the two-pass reduction needs a bounded number of owners and a bounded hand-off buffer
+// the two-pass reduction needs a bounded number of owners and a bounded hand-off buffer; and
+// two blocks against a large table are scanned faster than their keys are handed over (10 steps
+// of 256 / 512 / 1000 envs on 120x120 with 8 actions: 132 / 146 / 167 us, two passes 145 / 146 / 148)
 bool reduce_fast(const crl::ReduceGeom& G) {
+  if (G.n_blocks <= kScanBlocks && G.K > crl::kDenseKeys) return false;
   return 1 << G.own_shift <= crl::kMaxOwners && handoff_records(G) * sizeof(unsigned long long) <= kHandoffLimitBytes;
 }
 
@@ -932,15 +938,19 @@ struct PersistPlan {
 };
 
 // Shortest call worth the set-up of the one-launch kernel (clearing what its workgroups
-// exchange, one co-resident launch) instead of two plain launches per step.
-constexpr int kPersistMinSteps = 4;
+// exchange, one co-resident launch: 28 us) instead of two plain launches per step, which cost
+// more the more envs there are (4 / 8 / 10 / 12 steps, one launch against two: 3000 envs of
+// 16x16 52 / 75 / 86 / 97 us, 31 / 60 / 74 / 89; 20,000 of 32x32 with 8 actions 57 / 84 / 96 / 109,
+// 40 / 75 / 93 / 112; 65,536 of 64x64 57 / 85 / 99 / 113, 45 / 86 / 107 / 128).  With a few
+// thousand envs the two cross at 16 steps only; calls of ten keep the one launch.
+int persist_min_steps(int n_envs) { return n_envs <= 32768 ? 10 : 8; }
 
 // The one-launch kernel needs every workgroup resident at once (one per compute
 // unit), the dense LDS table of the block pass and one tile of the owners' pass.
 PersistPlan plan_persist(const crl_engine* e, int n_steps) {
   PersistPlan p{};
   if (e->cfg.table_mode != CRL_TABLE_SHARED || e->fused_variant == 1 || e->persist_refused) return p;
-  if (e->fused_variant == 0 && n_steps < kPersistMinSteps) return p;
+  if (e->fused_variant == 0 && n_steps < persist_min_steps(e->N)) return p;
   const int n_blocks = (e->N + crl::kBlockSamples - 1) / crl::kBlockSamples;
   if (e->K > (size_t)crl::kDenseKeys || n_blocks > crl::kPersistMaxGroups || crl::kPersistMaxGroups > kComputeUnits) return p;
   // always 256 workgroups, each a block (with or without envs) and an owner (with or
