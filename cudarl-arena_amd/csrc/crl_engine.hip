@@ -1479,6 +1479,16 @@ int opt_in_ticket_kernels(crl_engine* e) {
   return CRL_OK;
 }
 
+// For calls whose kernel reads what the host has just put down - in pages that are taken in
+// turn, or as an argument: a replay of a recorded launch would read another call's.
+int refuse_capture(const crl_engine* e) {
+  if (!e->stream) return CRL_OK;  // (the null stream cannot be captured)
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(e->stream, &status));
+  if (status == hipStreamCaptureStatusNone) return CRL_OK;
+  return fail(CRL_E_DEVICE, "a call that takes host data cannot be recorded: its stream is being captured");
+}
+
 // crl_td_update and, with `keys`, crl_td_update_collect.  The transitions are packed into
 // pinned memory, 12 bytes each, in the pass that checks them, and the kernel reads them
 // there: the call returns without waiting for anything (65,536 transitions: five copies from
@@ -1491,6 +1501,8 @@ int td_update(crl_engine* e, int32_t table, int32_t n, const int32_t* s, const i
   if (n < 0) return fail(CRL_E_ARG, "negative sample count");
   if (n == 0) return CRL_OK;
   if (!s || !a || !r || !s_next || !done) return fail(CRL_E_ARG, "null transition array");
+  rc = refuse_capture(e);
+  if (rc) return rc;
   const size_t nn = (size_t)n;
   crl_engine::InSlot* slot = nullptr;
   rc = claim_in_slot(e, 12 * nn, &slot);
@@ -1686,6 +1698,7 @@ int crl_reset(crl_engine* e, int32_t first, int32_t count) { return reset_envs(e
 
 int crl_step(crl_engine* e, const int32_t* actions) {
   int rc = check_usable(e);
+  if (rc == CRL_OK && actions) rc = refuse_capture(e);
   if (rc) return rc;
   const size_t bytes = (size_t)e->N * 4;
   const int32_t* act = e->act.p;

@@ -78,3 +78,26 @@ def test_actions_may_be_overwritten_once_step_has_returned(gpu):
         x = np.clip(x + (a == 1) - (a == 3), 0, 10)
         y = np.clip(y + (a == 2) - (a == 0), 0, 8)
     assert np.array_equal(st["s"], y * 11 + x)
+
+
+def test_calls_that_take_host_data_are_refused_under_capture(gpu):
+    """Their kernels read pages that are taken in turn: a replay would read another call's."""
+    import torch
+    cfg = gpu.make_config(8, 5, 5, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED)
+    one = np.zeros(8, np.int32)
+    stream = torch.cuda.Stream()
+    with gpu.Engine(cfg, 0) as eng:
+        assert eng.lib.crl_set_stream(eng.h, C.c_void_p(stream.cuda_stream)) == 0
+        eng.td_update(0, one, one, np.ones(8, np.float32), one, one.astype(np.uint8))
+        before = eng.q_get(0).copy()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(stream):
+            graph.capture_begin()
+            for call in (lambda: eng.td_update(0, one, one, np.ones(8, np.float32), one, one.astype(np.uint8)),
+                         lambda: eng.step(one)):
+                with pytest.raises(gpu.CrlError, match="captured"):
+                    call()
+            graph.capture_end()
+        assert np.array_equal(eng.q_get(0), before)
+        eng.step(one)
+        assert eng.lib.crl_set_stream(eng.h, None) == 0
