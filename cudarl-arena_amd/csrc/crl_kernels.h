@@ -307,6 +307,12 @@ __device__ __forceinline__ void run_env_steps(const Rules& R, const Ptrs& P, con
   P.action[env] = (uint8_t)action;
 }
 
+// u01(w) < eps  <=>  (w >> 8) < eps * 2^24, both sides exact: an integer compare
+__device__ __forceinline__ uint32_t explore_threshold(float eps) {
+  const float scaled = ceilf(eps * 16777216.0f);
+  return !(scaled > 0.0f) ? 0u : scaled >= 16777216.0f ? (1u << 24) : (uint32_t)scaled;
+}
+
 // The same loop for the common configuration, with everything that is fixed
 // there folded away: fixed epsilon, class rewards (no per-cell array), goal test
 // on the target cell, auto-reset, true max, no trace and no supplied stream.
@@ -317,30 +323,18 @@ __device__ __forceinline__ void run_env_steps(const Rules& R, const Ptrs& P, con
 // argmax, the draw and one shift of the cell's move codes; the codes of the next
 // cell, the Philox rounds and the bookkeeping run while the row is in flight.
 //
-// PAIR: lanes l and l + 32 of the wave step the SAME env (a wave that can hold
-// only 32 envs, because their tables fill the LDS, has half its lanes to spare).
-// Both do everything twice - same addresses, same values - except the Philox
-// rounds, the most expensive stretch of a step that waits for no memory: one
-// lane computes the block of the next two steps, the other the block after, and
-// they swap, so the rounds run every fourth step instead of every second.
-//
 // RICH adds the two things that configurations with large maps bring along and
 // that cost one more request per step at most: per-cell rewards (`cr`, may be
 // null) and an epsilon that follows the env's episode count.  The threshold
 // stays in a register and is looked up again only when an episode of the wave
 // ends, and so is the row of the start cell: with long episodes both are rare.
-template <int A, bool PAIR, bool RICH, class Table, class Moves>
+template <int A, bool RICH, class Table, class Moves>
 __device__ __forceinline__ void run_env_fast(const Rules& R, const Ptrs& P, const int env,
                                              const uint64_t t0, const int n_steps, const Moves moves,
                                              const float* __restrict__ cr, const Table tab) {
   const int W = R.W, T = R.episode_len;
   const float lr = R.lr, gamma = R.gamma;
-  // u01(w) < eps  <=>  (w >> 8) < eps * 2^24, both sides exact: an integer compare
-  auto threshold = [](float eps) -> uint32_t {
-    const float scaled = ceilf(eps * 16777216.0f);
-    return !(scaled > 0.0f) ? 0u : scaled >= 16777216.0f ? (1u << 24) : (uint32_t)scaled;
-  };
-  uint32_t explore_below = threshold(R.eps0);
+  uint32_t explore_below = explore_threshold(R.eps0);
   float r_step = R.step_reward, r_goal = R.goal_reward, r_trap = R.trap_reward;
   if (RICH) asm volatile("" : "+v"(r_step), "+v"(r_goal), "+v"(r_trap));  // plain values: no select of loads
   const bool cells = RICH && cr != nullptr;
@@ -357,35 +351,9 @@ __device__ __forceinline__ void run_env_fast(const Rules& R, const Ptrs& P, cons
   bool hit = false;
   Row<A> row = tab.load(s);
   uint32_t mv = moves.at(s, x, y);
-  if (scheduled) explore_below = threshold(eps_of(R, P.eps_tab, t0, episode));
-  const int lane = (int)__lane_id();
-  const bool upper = PAIR && lane >= 32;
-  // own block, and (PAIR) the partner lane's: {blk, nxt} = the next two blocks
-  auto two_blocks = [&](uint64_t b, Philox4& first, Philox4& second) {
-    const Philox4 own = explore_block(R.seed, (uint32_t)env, b + (upper ? 1 : 0));
-    // v_permlane32_swap exchanges the upper 32 lanes of its first operand with the
-    // lower 32 of its second: given the same value twice it returns the lower
-    // half's words in both halves (block b) and the upper half's (block b + 1)
-    const auto w0 = __builtin_amdgcn_permlane32_swap(own.w0, own.w0, false, false);
-    const auto w1 = __builtin_amdgcn_permlane32_swap(own.w1, own.w1, false, false);
-    const auto w2 = __builtin_amdgcn_permlane32_swap(own.w2, own.w2, false, false);
-    const auto w3 = __builtin_amdgcn_permlane32_swap(own.w3, own.w3, false, false);
-    first.w0 = w0[0];
-    first.w1 = w1[0];
-    first.w2 = w2[0];
-    first.w3 = w3[0];
-    second.w0 = w0[1];
-    second.w1 = w1[1];
-    second.w2 = w2[1];
-    second.w3 = w3[1];
-  };
-  Philox4 blk, nxt{};
-  bool have_nxt = PAIR;
-  uint64_t next_block = (t0 >> 1) + (PAIR ? 2 : 1);
-  if (PAIR)
-    two_blocks(t0 >> 1, blk, nxt);
-  else
-    blk = explore_block(R.seed, (uint32_t)env, t0 >> 1);
+  if (scheduled) explore_below = explore_threshold(eps_of(R, P.eps_tab, t0, episode));
+  uint64_t next_block = (t0 >> 1) + 1;
+  Philox4 blk = explore_block(R.seed, (uint32_t)env, t0 >> 1);
   bool odd = (t0 & 1) != 0;
   // everything loaded above has arrived before the loop starts: a value still in
   // flight at the loop's entry makes the loop's first instruction wait for ALL
@@ -436,18 +404,7 @@ __device__ __forceinline__ void run_env_fast(const Rules& R, const Ptrs& P, cons
     x = ends ? sx : x + dx;
     y = ends ? sy : y + dy;
     mv = moves.at(s_next, x, y);
-    if (odd) {  // in the loads' shadow
-      if (!PAIR) {
-        blk = explore_block(R.seed, (uint32_t)env, next_block++);
-      } else if (have_nxt) {
-        blk = nxt;
-        have_nxt = false;
-      } else {
-        two_blocks(next_block, blk, nxt);
-        next_block += 2;
-        have_nxt = true;
-      }
-    }
+    if (odd) blk = explore_block(R.seed, (uint32_t)env, next_block++);  // in the loads' shadow
     if (RICH) reward = (cells && (hit || trap || base_cells)) ? by_cell : reward;
     const float m = row_max(row2, hit, 0);
     const float qn = td_value(row_get(row, a), reward, m, lr, gamma);
@@ -461,7 +418,7 @@ __device__ __forceinline__ void run_env_fast(const Rules& R, const Ptrs& P, cons
     action = a;
     odd = !odd;
     if (RICH && scheduled && any_ends) {
-      explore_below = threshold(eps_of(R, P.eps_tab, t0, episode));
+      explore_below = explore_threshold(eps_of(R, P.eps_tab, t0, episode));
       asm volatile("" : "+v"(explore_below));  // arrived before the loop goes round
     }
   }
@@ -489,12 +446,6 @@ __device__ __forceinline__ void run_env_fast(const Rules& R, const Ptrs& P, cons
 // The exploration draws of the next steps are worked out ahead by all 64 lanes into a tape
 // in LDS (a Philox block is 75 instructions; with E envs to a wave a step's share is 75 E / 128).
 // ---------------------------------------------------------------------------
-
-// u01(w) < eps  <=>  (w >> 8) < eps * 2^24, both sides exact: an integer compare
-__device__ __forceinline__ uint32_t explore_threshold(float eps) {
-  const float scaled = ceilf(eps * 16777216.0f);
-  return !(scaled > 0.0f) ? 0u : scaled >= 16777216.0f ? (1u << 24) : (uint32_t)scaled;
-}
 
 // A word of the tape: explore iff it is below the env's limit, and then the action is its low
 // byte.  Epsilon by episode: the upper 24 bits are the draw's and the limit the threshold.
@@ -1062,13 +1013,13 @@ __global__ __launch_bounds__(256) void k_fused_per_env(const Rules R, const Ptrs
       const GlobalTable<A> tab{P.Q + (size_t)env * P.S * A};
       if (MAP == 1) {
         if (FAST)
-          run_env_fast<A, false, true>(R, P, env, t0, n_steps, MovesLds<A>{lds, 1}, cr, tab);
+          run_env_fast<A, true>(R, P, env, t0, n_steps, MovesLds<A>{lds, 1}, cr, tab);
         else
           run_env_steps<A>(R, P, env, t0, n_steps, MovesLds<A>{lds, 1}, own_map, cr, tab);
       } else {
         const MovesGlobal<A> moves{P.moves + (P.map_shared ? 0 : (size_t)env * P.mv_words)};
         if (FAST)
-          run_env_fast<A, false, true>(R, P, env, t0, n_steps, moves, cr, tab);
+          run_env_fast<A, true>(R, P, env, t0, n_steps, moves, cr, tab);
         else
           run_env_steps<A>(R, P, env, t0, n_steps, moves, own_map, cr, tab);
       }
@@ -1296,9 +1247,9 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
         const GlobalTable<A> tab{P.Q + (size_t)env * table};
         if (n_steps >= kTouchMinSteps) tab.touch((int)table);
         if (kTableMoves)
-          run_env_fast<A, false, RICH>(R, P, env, t0, n_steps, MovesLds<A>{my_words + lane, 64}, RICH ? cr : nullptr, tab);
+          run_env_fast<A, RICH>(R, P, env, t0, n_steps, MovesLds<A>{my_words + lane, 64}, RICH ? cr : nullptr, tab);
         else if (FAST)
-          run_env_fast<A, false, RICH>(R, P, env, t0, n_steps, MovesFromMap<A>{my_words + lane, R.W, R.H}, RICH ? cr : nullptr, tab);
+          run_env_fast<A, RICH>(R, P, env, t0, n_steps, MovesFromMap<A>{my_words + lane, R.W, R.H}, RICH ? cr : nullptr, tab);
         else
           run_env_steps<A>(R, P, env, t0, n_steps, MovesFromMap<A>{my_words + lane, R.W, R.H},
                            P.map + (size_t)env * P.map_words, cr, tab);
