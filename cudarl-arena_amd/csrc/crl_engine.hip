@@ -1326,9 +1326,18 @@ int create_engine(const crl_config* cfg, int device, crl_engine** out) {
     } else {
       carve(e->pdiag, 1 + crl::kPersistClockWords);
     }
+    // (large arrays where an allocation of their own would start them: 1M tables of 4 KB that
+    // start 256 bytes into a page each, 20 steps 631 -> 635 us, 1000 steps 12.17 -> 12.23 ms)
+    auto page = [&](size_t bytes) {
+      const size_t at = bytes >= (size_t)32 << 20 ? (size_t)2 << 20 : 256;
+      used = (used + at - 1) & ~(at - 1);
+    };
+    page((size_t)e->n_maps * e->map_words * 4);
     carve(e->map, (size_t)e->n_maps * e->map_words);
+    page((size_t)e->n_tables * e->K * 4);
     carve(e->Q, (size_t)e->n_tables * e->K);
     cleared = used;
+    page((size_t)e->n_maps * e->mv_words * 4);
     carve(e->moves, (size_t)e->n_maps * e->mv_words);  // move codes of every map, for the fused loops
     if (cells) carve(e->cell_reward, (size_t)e->n_maps * e->S);
     carve(e->eps_tab, eps.size());
