@@ -187,7 +187,8 @@ struct crl_engine {
   static constexpr int kInSlots = 4;
   InSlot in_slot[kInSlots];     // what the host hands to kernels, taken in turn
   int in_next = 0;
-  bool state_shared = false;    // device pointers to the state are out: it may change between calls
+  bool state_shared = false;    // the state may change between calls: device pointers to it are out,
+                                // or a call that changes it has been recorded and may be replayed
   bool mirror_steps = false;    // crl_step's kernel also writes the state to out_page ...
   bool mirror_read = false;     // ... because the state was read after the step before
   bool stepped = false;         // crl_step was the last call that changed the state
@@ -1209,6 +1210,28 @@ void set_geometry(crl_engine* e, const crl_config& cfg) {
   e->mv_words = (int)((e->S + cells_per_word - 1) / cells_per_word);
 }
 
+// Is the engine's stream being captured, so that what is launched now is recorded?
+int query_capture(const crl_engine* e, bool* active) {
+  *active = false;
+  if (!e->stream) return CRL_OK;  // (the null stream cannot be captured)
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(e->stream, &status));
+  *active = status != hipStreamCaptureStatusNone;
+  return CRL_OK;
+}
+
+// For calls that change the state: no copy of it that the host holds is good any more, and
+// once such a call has been recorded none ever is, as its replays change the state unseen.
+int state_changes(crl_engine* e) {
+  bool active;
+  const int rc = query_capture(e, &active);
+  if (rc) return rc;
+  if (active) e->state_shared = true;
+  e->mirror_seq = 0;
+  e->stepped = false;
+  return CRL_OK;
+}
+
 int check_engine(const crl_engine* e) {
   if (!e) return fail(CRL_E_ARG, "null engine");
   hipError_t err = hipSetDevice(e->device);
@@ -1399,8 +1422,8 @@ int reset_envs(crl_engine* e, int32_t first, int32_t count) {
   if (first < 0 || count < 0 || (int64_t)first + count > e->N)
     return fail(CRL_E_RANGE, "env range [%d,%d) outside [0,%d)", first, first + count, e->N);
   if (count == 0) return CRL_OK;
-  e->mirror_seq = 0;
-  e->stepped = false;
+  rc = state_changes(e);
+  if (rc) return rc;
   hipLaunchKernelGGL(crl::k_reset, dim3((count + 255) / 256), dim3(256), 0, e->stream, e->ptrs(), first,
                      count);
   HIP_TRY(hipGetLastError());
@@ -1491,10 +1514,9 @@ int opt_in_ticket_kernels(crl_engine* e) {
 // For calls whose kernel reads what the host has just put down - in pages that are taken in
 // turn, or as an argument: a replay of a recorded launch would read another call's.
 int refuse_capture(const crl_engine* e) {
-  if (!e->stream) return CRL_OK;  // (the null stream cannot be captured)
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  HIP_TRY(hipStreamIsCapturing(e->stream, &status));
-  if (status == hipStreamCaptureStatusNone) return CRL_OK;
+  bool active;
+  const int rc = query_capture(e, &active);
+  if (rc || !active) return rc;
   return fail(CRL_E_DEVICE, "a call that takes host data cannot be recorded: its stream is being captured");
 }
 
@@ -1577,8 +1599,8 @@ int run_fused(crl_engine* e, int32_t n_steps, bool no_alloc) {
     ~Restore() { e->no_alloc = false; }
   } restore{e};
   e->no_alloc = no_alloc;
-  e->mirror_seq = 0;
-  e->stepped = false;
+  rc = state_changes(e);
+  if (rc) return rc;
   if (e->cfg.table_mode == CRL_TABLE_PER_ENV) {
     const FusedPlan p = plan_fused(e, n_steps);
     if (p.lds > kLdsPerWorkgroup)
@@ -1735,9 +1757,10 @@ int crl_step(crl_engine* e, const int32_t* actions) {
   // instead of from a second launch: 6 us of launch and answer saved, 18 bytes per env
   // over the link added, so it stops with the first step whose state nobody asked for.
   // (Not in a call that a stream capture may record: a replay has no number of its own.)
+  rc = state_changes(e);
+  if (rc) return rc;
   if (!e->mirror_read) e->mirror_steps = false;
   e->mirror_read = false;
-  e->mirror_seq = 0;
   const bool mirrors = actions && e->mirror_steps && !e->state_shared && e->state_bytes <= kLinkLimitBytes;
   if (mirrors) {
     rc = claim_out_page(e, e->state_bytes);
@@ -1870,9 +1893,9 @@ int crl_set_state(crl_engine* e, const int32_t* s, const int32_t* ep_step, const
   if (rc) return rc;
   rc = clear_persist_failure(e);
   if (rc) return rc;
+  rc = state_changes(e);
+  if (rc) return rc;
   const size_t N = (size_t)e->N;
-  e->mirror_seq = 0;
-  e->stepped = false;
   if (s) {
     for (int i = 0; i < e->N; ++i)
       if (s[i] < 0 || (size_t)s[i] >= e->S) return fail(CRL_E_RANGE, "s[%d] = %d outside [0,%zu)", i, s[i], e->S);
@@ -2037,7 +2060,10 @@ int crl_device_ptr(crl_engine* e, int32_t which, void** out) {
     case CRL_PTR_Q: *out = e->Q.p; break;
     default: return fail(CRL_E_ARG, "unknown pointer id %d", which);
   }
-  if (which != CRL_PTR_Q) e->state_shared = true;
+  if (which != CRL_PTR_Q) {  // the caller may write through it from now on
+    e->state_shared = true;
+    e->mirror_seq = 0;
+  }
   return CRL_OK;
 }
 

@@ -58,6 +58,78 @@ def test_state_written_by_the_caller_is_what_the_next_read_returns(gpu):
         assert np.array_equal(eng.get_state()["s"], mine)
 
 
+@pytest.mark.parametrize("which,key", [(0, "s"), (1, "ep_step"), (2, "episode"), (3, "reward")])
+def test_state_written_through_a_pointer_taken_after_the_step(gpu, which, key):
+    """The step has left a copy of the state already when the pointer is asked for."""
+    hip = C.CDLL("libamdhip64.so")
+    N = 70
+    mine = np.full(N, 7, np.float32 if key == "reward" else np.int32)
+    with gpu.Engine(gpu.make_config(N, 6, 5, seed=1), 0) as eng:
+        eng.set_maps(np.zeros((N, 30), np.uint8), np.arange(N, dtype=np.int32) % 30)
+        for _ in range(3):
+            eng.step(np.zeros(N, np.int32))
+            eng.get_state()
+        eng.step(np.zeros(N, np.int32))
+        view = eng.device_ptr(which)
+        for value in (7, 9):  # ... and once more through the pointer that is out
+            mine[:] = value
+            eng.sync()
+            assert hip.hipMemcpy(C.c_void_p(view), C.c_void_p(mine.ctypes.data), C.c_size_t(4 * N), 1) == 0
+            assert np.array_equal(eng.get_state()[key], mine)
+        eng.step(np.zeros(N, np.int32))
+        assert eng.get_state()["ep_step"][0] == (10 if key == "ep_step" else 5)
+
+
+@pytest.mark.parametrize("recorded", ["run", "step", "reset"])
+def test_state_after_the_replay_of_a_recorded_call(gpu, recorded):
+    """A replay moves the state without a call of the engine: no copy that an earlier step
+    left may be handed out."""
+    import torch
+    N, W, H = 300, 9, 7
+    cls, start = gpu.gen_maps_bernoulli(3, N, N, W, H, 0.1, 0.02)
+    cfg = gpu.make_config(N, W, H, eps0=0.4, episode_len=11, seed=5)
+    rng = np.random.default_rng(1)
+    stream = torch.cuda.Stream()
+
+    def call(e):
+        e.step_count = 0  # a replay draws what the recorded call drew
+        if recorded == "run":
+            e.run_fused(3)
+        elif recorded == "step":
+            e.select(fetch=False)
+            e.step()
+        else:
+            e.reset(0, N)
+
+    with gpu.Engine(cfg, 0) as want, gpu.Engine(cfg, 0) as eng:
+        for e in (want, eng):
+            e.set_maps(cls, start)
+            assert e.lib.crl_set_stream(e.h, C.c_void_p(stream.cuda_stream)) == 0
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(stream):
+            graph.capture_begin()
+            call(eng)
+            graph.capture_end()
+        eng.reset(0, N)
+        for _ in range(3):
+            for _ in range(3):
+                acts = rng.integers(0, 4, N).astype(np.int32)
+                for e in (want, eng):
+                    e.step(acts)
+                assert same(want.get_state(), eng.get_state())
+            acts = rng.integers(0, 4, N).astype(np.int32)
+            for e in (want, eng):
+                e.step(acts)
+            with torch.cuda.stream(stream):
+                graph.replay()
+            call(want)
+            assert same(want.get_state(), eng.get_state())
+        assert np.array_equal(want.q_get(0, N), eng.q_get(0, N))
+        for e in (want, eng):
+            assert e.lib.crl_set_stream(e.h, None) == 0
+        del graph
+
+
 def test_actions_may_be_overwritten_once_step_has_returned(gpu):
     N = 5000
     acts = np.zeros((20, N), np.int32)
