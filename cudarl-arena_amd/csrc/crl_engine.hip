@@ -800,6 +800,12 @@ bool handoff_fits(const crl_engine* e, const crl::ReduceGeom& G) {
   return !e->no_alloc || handoff_records(G) * sizeof(unsigned long long) <= kScratchExchangeBytes;
 }
 
+// Does this call sum in two passes, or by the scan?  A larger table than 16,384 keys whose cells
+// have no room is scanned (ensure_handoff refuses a smaller one).
+bool two_passes(const crl_engine* e, const crl::ReduceGeom& G) {
+  return reduce_fast(G) && (G.K <= crl::kDenseKeys || handoff_fits(e, G));
+}
+
 int ensure_handoff(crl_engine* e, const crl::ReduceGeom& G) {
   const size_t recs = handoff_records(G);
   if (e->no_alloc) {
@@ -894,7 +900,7 @@ void launch_shared_act(crl_engine* e, bool reduce, const crl::ReduceGeom& G, uin
 // one shared-table step: act (select + move + delta + block sums), then the key owners
 int shared_step(crl_engine* e, uint64_t t, int trace_row) {
   const crl::ReduceGeom G = e->no_alloc ? reduce_geom_within(e, e->N, kScratchExchangeBytes) : reduce_geom(e, e->N);
-  const bool fast = reduce_fast(G);
+  const bool fast = two_passes(e, G);
   if (fast) {
     int rc = ensure_handoff(e, G);
     if (rc) return rc;

@@ -220,11 +220,12 @@ int crl_run_fused(crl_engine* e, int32_t n_steps);
  * the exchange buffers of the one-launch shared-table kernel - lives in a
  * static device array of 10 MB + 4 KB that each GPU the library runs on holds
  * until the process ends, and the call allocates and frees nothing (device or
- * host).  CRL_E_RANGE if the engine's ordered reduction needs more hand-off cells
- * than the array holds (65,536 envs on a 64x64x4 table need 4 MB with two launches
- * per step, 9.7 MB of exchange buffers in the one-launch kernel; an engine whose
- * one-launch buffers do not fit takes two launches per step).  All engines on one GPU share that GPU's
- * array: calls that overlap in time on one GPU (different streams or threads)
+ * host).  CRL_E_RANGE if the ordered reduction of a table of at most 16,384 entries
+ * needs more hand-off cells than the array holds (65,536 envs on a 64x64x4 table need
+ * 4 MB with two launches per step, 9.7 MB of exchange buffers in the one-launch kernel;
+ * an engine whose one-launch buffers do not fit takes two launches per step); a larger
+ * table whose cells do not fit is summed by a scan of all samples that needs none
+ * and is slower.  All engines on one GPU share that GPU's array: calls that overlap in time on one GPU (different streams or threads)
  * race; calls in stream order do not. */
 int crl_run_fused_noalloc(crl_engine* e, int32_t n_steps);
 

@@ -77,3 +77,13 @@ def test_noalloc_rejects_a_reduction_larger_than_the_scratch(gpu):
         assert eng.step_count == 0
         eng.run_fused(2)  # the allocating entry point still takes it
         assert eng.step_count == 2
+
+
+@pytest.mark.parametrize("N,W,H,A", [(20000, 1024, 1024, 4), (65536, 512, 512, 4), (200000, 101, 99, 8)])
+def test_noalloc_shared_tables_whose_hand_off_cells_outgrow_the_scratch(gpu, N, W, H, A):
+    """More than 16,384 keys: the scan, which needs no cells, takes the step instead."""
+    cls, start = gpu.gen_maps_bernoulli(2, 1, N, W, H, 0.15)
+    cfg = gpu.make_config(N, W, H, n_actions=A, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=0.01,
+                          eps0=0.3, episode_len=3, seed=6)
+    st, q = run_pair(gpu, cfg, cls, start, (3, 2), 1)
+    assert np.isfinite(q).all() and np.count_nonzero(q) > 1000 and st["episode"].min() >= 1
