@@ -800,10 +800,31 @@ bool handoff_fits(const crl_engine* e, const crl::ReduceGeom& G) {
   return !e->no_alloc || handoff_records(G) * sizeof(unsigned long long) <= kScratchExchangeBytes;
 }
 
+// Is the engine's stream being captured, so that what is launched now is recorded?
+int query_capture(const crl_engine* e, bool* active) {
+  *active = false;
+  if (!e->stream) return CRL_OK;  // (the null stream cannot be captured)
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(e->stream, &status));
+  *active = status != hipStreamCaptureStatusNone;
+  return CRL_OK;
+}
+
 // Does this call sum in two passes, or by the scan?  A larger table than 16,384 keys whose cells
-// have no room is scanned (ensure_handoff refuses a smaller one).
-bool two_passes(const crl_engine* e, const crl::ReduceGeom& G) {
-  return reduce_fast(G) && (G.K <= crl::kDenseKeys || handoff_fits(e, G));
+// have no room is scanned, also where they would have to be allocated now and the stream is
+// being captured, which allows no allocation.  (A smaller one is refused by ensure_handoff.)
+int choose_passes(const crl_engine* e, const crl::ReduceGeom& G, bool* two) {
+  *two = reduce_fast(G);
+  if (!*two || G.K <= crl::kDenseKeys) return CRL_OK;
+  bool recorded = false;
+  if (e->no_alloc) {
+    *two = handoff_fits(e, G);
+  } else if (handoff_records(G) > e->handoff.n) {
+    const int rc = query_capture(e, &recorded);
+    if (rc) return rc;
+    *two = !recorded;
+  }
+  return CRL_OK;
 }
 
 int ensure_handoff(crl_engine* e, const crl::ReduceGeom& G) {
@@ -860,8 +881,11 @@ int td_apply_a(crl_engine* e, float* Q, const Samples& X, int n, int2* changed, 
   if (h != hipSuccess) return fail(CRL_E_ALLOC, "scratch allocation failed: %s", hipGetErrorString(h));
   const crl::ReduceGeom G = reduce_geom(e, n);
   const int grid = G.n_blocks;
-  if (reduce_fast(G)) {
-    e->no_alloc = false;  // crl_update / crl_td_update: the engine's own hand-off buffer
+  e->no_alloc = false;  // crl_update / crl_td_update: the engine's own hand-off buffer
+  bool two;
+  rc = choose_passes(e, G, &two);
+  if (rc) return rc;
+  if (two) {
     rc = ensure_handoff(e, G);
     if (rc) return rc;
     hipLaunchKernelGGL((crl::k_td_blocks<A, Samples>), dim3(grid), dim3(crl::kBlockSamples),
@@ -900,11 +924,10 @@ void launch_shared_act(crl_engine* e, bool reduce, const crl::ReduceGeom& G, uin
 // one shared-table step: act (select + move + delta + block sums), then the key owners
 int shared_step(crl_engine* e, uint64_t t, int trace_row) {
   const crl::ReduceGeom G = e->no_alloc ? reduce_geom_within(e, e->N, kScratchExchangeBytes) : reduce_geom(e, e->N);
-  const bool fast = two_passes(e, G);
-  if (fast) {
-    int rc = ensure_handoff(e, G);
-    if (rc) return rc;
-  }
+  bool fast;
+  int rc = choose_passes(e, G, &fast);
+  if (rc == CRL_OK && fast) rc = ensure_handoff(e, G);
+  if (rc) return rc;
   // LDS plan of the act kernel: reduction table (fast path), then the map.  The
   // shared table itself stays in L2: streaming its 64 KB into every workgroup's
   // LDS each step measured slower than the row reads it saves (12.4 against 12.05 us
@@ -1214,16 +1237,6 @@ void set_geometry(crl_engine* e, const crl_config& cfg) {
   e->map_words = (int)((e->S + 15) / 16);
   const size_t cells_per_word = 16 / (size_t)e->A;
   e->mv_words = (int)((e->S + cells_per_word - 1) / cells_per_word);
-}
-
-// Is the engine's stream being captured, so that what is launched now is recorded?
-int query_capture(const crl_engine* e, bool* active) {
-  *active = false;
-  if (!e->stream) return CRL_OK;  // (the null stream cannot be captured)
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  HIP_TRY(hipStreamIsCapturing(e->stream, &status));
-  *active = status != hipStreamCaptureStatusNone;
-  return CRL_OK;
 }
 
 // For calls that change the state: no copy of it that the host holds is good any more, and

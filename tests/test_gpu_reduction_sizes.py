@@ -94,6 +94,56 @@ def test_update_of_a_shared_table_from_the_last_step(gpu, oracle):
         assert np.array_equal(q, Q[0]) and np.array_equal(st["s"], ost["s"]), N
 
 
+@pytest.mark.parametrize("call", ["run", "update"])
+def test_large_table_recorded_before_anything_has_run(gpu, call):
+    """A stream being captured allows no allocation: past 16,384 keys a first call is recorded
+    all the same, without the cells that the two passes need."""
+    import ctypes as C
+    import torch
+    N, W, H = 5000, 90, 70  # 25,200 keys
+    cls, start = gpu.gen_maps_bernoulli(2, 1, N, W, H, 0.15)
+    cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=0.02, eps0=0.3,
+                          episode_len=5, seed=3)
+    stream = torch.cuda.Stream()
+
+    def go(e):
+        e.step_count = 0  # a replay draws what the recorded call drew
+        if call == "run":
+            e.run_fused(2)
+        else:
+            e.select(fetch=False)
+            e.step()
+            e.update()
+
+    with gpu.Engine(cfg, 0) as want, gpu.Engine(cfg, 0) as eng:
+        for e in (want, eng):
+            e.set_maps(cls, start)
+            assert e.lib.crl_set_stream(e.h, C.c_void_p(stream.cuda_stream)) == 0
+        graph, failed = torch.cuda.CUDAGraph(), None
+        with torch.cuda.stream(stream):
+            graph.capture_begin()
+            try:
+                go(eng)
+            except gpu.CrlError as x:
+                failed = x
+            finally:
+                graph.capture_end()
+        assert failed is None
+        for _ in range(3):
+            with torch.cuda.stream(stream):
+                graph.replay()
+            go(want)
+            assert np.array_equal(want.q_get(0), eng.q_get(0))
+            assert np.array_equal(want.get_state()["s"], eng.get_state()["s"])
+            for e in (want, eng):  # eager work between the replays, which allocates the cells
+                e.step_count = 7
+                e.run_fused(3)
+        assert np.array_equal(want.q_get(0), eng.q_get(0))
+        for e in (want, eng):
+            assert e.lib.crl_set_stream(e.h, None) == 0
+        del graph
+
+
 @pytest.mark.parametrize("items", [
     lambda v: v,                                                   # exact ints, floats, bools and tuples
     lambda v: tuple(v),
