@@ -72,6 +72,21 @@ struct DevBuf {
     return e;
   }
   hipError_t ensure(size_t count) { return count <= n ? hipSuccess : alloc(count); }
+  // `count` elements in a new allocation, the old one handed over to `keep` instead of freed (at
+  // least twice as many as now, so that what is kept never exceeds what is in use)
+  hipError_t replace(size_t count, std::vector<void*>& keep) {
+    if (count <= n) return hipSuccess;
+    count = std::max(count, 2 * n);
+    if (owned) {
+      try {
+        keep.push_back(p);
+      } catch (...) {
+        return hipErrorOutOfMemory;
+      }
+      owned = false;
+    }
+    return alloc(count);
+  }
   // a piece of somebody else's allocation
   void adopt(void* at, size_t count) {
     release();
@@ -187,6 +202,19 @@ struct crl_engine {
   static constexpr int kInSlots = 4;
   InSlot in_slot[kInSlots];     // what the host hands to kernels, taken in turn
   int in_next = 0;
+  // A call of this engine has been recorded into a graph: what its launches work on stays
+  // allocated until the engine goes, also where a later call needs a larger buffer.
+  bool recorded = false;
+  struct Outgrown {
+    std::vector<void*> p;
+    ~Outgrown() {
+      for (void* x : p) (void)hipFree(x);
+    }
+  } outgrown;
+  template <class T>
+  hipError_t grow(DevBuf<T>& buf, size_t count) {
+    return recorded ? buf.replace(count, outgrown.p) : buf.ensure(count);
+  }
   bool state_shared = false;    // the state may change between calls: device pointers to it are out,
                                 // or a call that changes it has been recorded and may be replayed
   bool mirror_steps = false;    // crl_step's kernel also writes the state to out_page ...
@@ -836,7 +864,7 @@ int ensure_handoff(crl_engine* e, const crl::ReduceGeom& G) {
                   kScratchExchangeBytes);
     e->ho = reinterpret_cast<unsigned long long*>(e->static_scratch + kScratchTicketBytes);
   } else {
-    hipError_t h = e->handoff.ensure(recs);
+    hipError_t h = e->grow(e->handoff, recs);
     if (h != hipSuccess) return fail(CRL_E_ALLOC, "hand-off buffer allocation failed: %s", hipGetErrorString(h));
     e->ho = e->handoff.p;
   }
@@ -876,8 +904,8 @@ int td_apply_a(crl_engine* e, float* Q, const Samples& X, int n, int2* changed, 
     HIP_TRY(hipGetLastError());
     return CRL_OK;
   }
-  hipError_t h = e->key.ensure((size_t)n);
-  if (h == hipSuccess) h = e->delta.ensure((size_t)n);
+  hipError_t h = e->grow(e->key, (size_t)n);
+  if (h == hipSuccess) h = e->grow(e->delta, (size_t)n);
   if (h != hipSuccess) return fail(CRL_E_ALLOC, "scratch allocation failed: %s", hipGetErrorString(h));
   const crl::ReduceGeom G = reduce_geom(e, n);
   const int grid = G.n_blocks;
@@ -1239,13 +1267,20 @@ void set_geometry(crl_engine* e, const crl_config& cfg) {
   e->mv_words = (int)((e->S + cells_per_word - 1) / cells_per_word);
 }
 
+// For calls that may be recorded: note it where this one is.
+int note_recording(crl_engine* e) {
+  bool active;
+  const int rc = query_capture(e, &active);
+  if (rc == CRL_OK && active) e->recorded = true;
+  return rc;
+}
+
 // For calls that change the state: no copy of it that the host holds is good any more, and
 // once such a call has been recorded none ever is, as its replays change the state unseen.
 int state_changes(crl_engine* e) {
-  bool active;
-  const int rc = query_capture(e, &active);
+  const int rc = note_recording(e);
   if (rc) return rc;
-  if (active) e->state_shared = true;
+  if (e->recorded) e->state_shared = true;
   e->mirror_seq = 0;
   e->stepped = false;
   return CRL_OK;
@@ -1802,6 +1837,7 @@ int crl_step(crl_engine* e, const int32_t* actions) {
 
 int crl_select(crl_engine* e, int32_t* actions_out) {
   int rc = check_usable(e);
+  if (rc == CRL_OK) rc = note_recording(e);
   if (rc) return rc;
   const size_t bytes = (size_t)e->N * 4;
   const bool direct = actions_out && bytes <= kLinkLimitBytes;
@@ -1837,6 +1873,8 @@ int crl_update(crl_engine* e) {
   int rc = check_usable(e);
   if (rc) return rc;
   if (!e->have_transition) return fail(CRL_E_STATE, "crl_update needs a preceding crl_step");
+  rc = note_recording(e);
+  if (rc) return rc;
   const crl::Rules R = e->rules();
   const int grid = (e->N + 255) / 256;
   if (e->cfg.table_mode == CRL_TABLE_PER_ENV) {
@@ -2013,10 +2051,10 @@ int crl_set_trace(crl_engine* e, int32_t n_envs, int32_t max_steps) {
   auto acc = [&](hipError_t x) {
     if (h == hipSuccess) h = x;
   };
-  acc(e->trace_s.ensure(cells));
-  acc(e->trace_a.ensure(cells));
-  acc(e->trace_r.ensure(cells));
-  acc(e->trace_d.ensure(cells));
+  acc(e->grow(e->trace_s, cells));
+  acc(e->grow(e->trace_a, cells));
+  acc(e->grow(e->trace_r, cells));
+  acc(e->grow(e->trace_d, cells));
   if (h != hipSuccess) return fail(CRL_E_ALLOC, "trace allocation failed: %s", hipGetErrorString(h));
   e->trace_n = n_envs;
   e->trace_cap = max_steps;
@@ -2056,8 +2094,8 @@ int crl_set_exploration_stream(crl_engine* e, int32_t n_steps, const float* u, c
   const size_t cells = (size_t)n_steps * e->N;
   for (size_t i = 0; i < cells; ++i)
     if (a_rand[i] < 0 || a_rand[i] >= e->A) return fail(CRL_E_RANGE, "a_rand[%zu] = %d outside [0,%d)", i, a_rand[i], e->A);
-  hipError_t h = e->u_sup.ensure(cells);
-  if (h == hipSuccess) h = e->a_sup.ensure(cells);
+  hipError_t h = e->grow(e->u_sup, cells);
+  if (h == hipSuccess) h = e->grow(e->a_sup, cells);
   if (h != hipSuccess) return fail(CRL_E_ALLOC, "stream allocation failed: %s", hipGetErrorString(h));
   HIP_TRY(hipMemcpyAsync(e->u_sup.p, u, cells * 4, hipMemcpyHostToDevice, e->stream));
   HIP_TRY(hipMemcpyAsync(e->a_sup.p, a_rand, cells * 4, hipMemcpyHostToDevice, e->stream));

@@ -262,3 +262,46 @@ def gpu(pycrl):
     n = lib.crl_device_count()
     assert n >= 1, "no HIP device: %s" % lib.crl_last_error().decode()
     return pycrl
+
+
+class HipGraphs:
+    """Streams and graphs of the HIP runtime that the engine library itself uses."""
+
+    def __init__(self):
+        self.lib = C.CDLL("libamdhip64.so.7")
+
+    def ok(self, rc):
+        assert rc == 0, "HIP error %d" % rc
+
+    def stream(self):
+        s = C.c_void_p()
+        self.ok(self.lib.hipStreamCreate(C.byref(s)))
+        return s
+
+    def destroy_stream(self, stream):
+        self.ok(self.lib.hipStreamDestroy(stream))
+
+    def record(self, stream, call):
+        """What call() launches on `stream`, as a graph; an exception of call() goes on to the caller."""
+        graph, runnable = C.c_void_p(), C.c_void_p()
+        self.ok(self.lib.hipStreamBeginCapture(stream, 0))
+        try:
+            call()
+        finally:
+            rc = self.lib.hipStreamEndCapture(stream, C.byref(graph))
+            self.lib.hipGetLastError()
+        self.ok(rc)
+        self.ok(self.lib.hipGraphInstantiate(C.byref(runnable), graph, None, None, C.c_size_t(0)))
+        self.ok(self.lib.hipGraphDestroy(graph))
+        return runnable
+
+    def replay(self, runnable, stream):
+        self.ok(self.lib.hipGraphLaunch(runnable, stream))
+
+    def destroy(self, runnable):
+        self.ok(self.lib.hipGraphExecDestroy(runnable))
+
+
+@pytest.fixture(scope="session")
+def graphs(gpu):
+    return HipGraphs()

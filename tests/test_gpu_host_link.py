@@ -81,15 +81,14 @@ def test_state_written_through_a_pointer_taken_after_the_step(gpu, which, key):
 
 
 @pytest.mark.parametrize("recorded", ["run", "step", "reset"])
-def test_state_after_the_replay_of_a_recorded_call(gpu, recorded):
+def test_state_after_the_replay_of_a_recorded_call(gpu, graphs, recorded):
     """A replay moves the state without a call of the engine: no copy that an earlier step
     left may be handed out."""
-    import torch
     N, W, H = 300, 9, 7
     cls, start = gpu.gen_maps_bernoulli(3, N, N, W, H, 0.1, 0.02)
     cfg = gpu.make_config(N, W, H, eps0=0.4, episode_len=11, seed=5)
     rng = np.random.default_rng(1)
-    stream = torch.cuda.Stream()
+    stream = graphs.stream()
 
     def call(e):
         e.step_count = 0  # a replay draws what the recorded call drew
@@ -104,12 +103,8 @@ def test_state_after_the_replay_of_a_recorded_call(gpu, recorded):
     with gpu.Engine(cfg, 0) as want, gpu.Engine(cfg, 0) as eng:
         for e in (want, eng):
             e.set_maps(cls, start)
-            assert e.lib.crl_set_stream(e.h, C.c_void_p(stream.cuda_stream)) == 0
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.stream(stream):
-            graph.capture_begin()
-            call(eng)
-            graph.capture_end()
+            assert e.lib.crl_set_stream(e.h, stream) == 0
+        graph = graphs.record(stream, lambda: call(eng))
         eng.reset(0, N)
         for _ in range(3):
             for _ in range(3):
@@ -120,14 +115,14 @@ def test_state_after_the_replay_of_a_recorded_call(gpu, recorded):
             acts = rng.integers(0, 4, N).astype(np.int32)
             for e in (want, eng):
                 e.step(acts)
-            with torch.cuda.stream(stream):
-                graph.replay()
+            graphs.replay(graph, stream)
             call(want)
             assert same(want.get_state(), eng.get_state())
         assert np.array_equal(want.q_get(0, N), eng.q_get(0, N))
         for e in (want, eng):
             assert e.lib.crl_set_stream(e.h, None) == 0
-        del graph
+        graphs.destroy(graph)
+    graphs.destroy_stream(stream)
 
 
 def test_actions_may_be_overwritten_once_step_has_returned(gpu):

@@ -95,16 +95,14 @@ def test_update_of_a_shared_table_from_the_last_step(gpu, oracle):
 
 
 @pytest.mark.parametrize("call", ["run", "update"])
-def test_large_table_recorded_before_anything_has_run(gpu, call):
+def test_large_table_recorded_before_anything_has_run(gpu, graphs, call):
     """A stream being captured allows no allocation: past 16,384 keys a first call is recorded
     all the same, without the cells that the two passes need."""
-    import ctypes as C
-    import torch
     N, W, H = 5000, 90, 70  # 25,200 keys
     cls, start = gpu.gen_maps_bernoulli(2, 1, N, W, H, 0.15)
     cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=0.02, eps0=0.3,
                           episode_len=5, seed=3)
-    stream = torch.cuda.Stream()
+    stream = graphs.stream()
 
     def go(e):
         e.step_count = 0  # a replay draws what the recorded call drew
@@ -118,20 +116,10 @@ def test_large_table_recorded_before_anything_has_run(gpu, call):
     with gpu.Engine(cfg, 0) as want, gpu.Engine(cfg, 0) as eng:
         for e in (want, eng):
             e.set_maps(cls, start)
-            assert e.lib.crl_set_stream(e.h, C.c_void_p(stream.cuda_stream)) == 0
-        graph, failed = torch.cuda.CUDAGraph(), None
-        with torch.cuda.stream(stream):
-            graph.capture_begin()
-            try:
-                go(eng)
-            except gpu.CrlError as x:
-                failed = x
-            finally:
-                graph.capture_end()
-        assert failed is None
+            assert e.lib.crl_set_stream(e.h, stream) == 0
+        graph = graphs.record(stream, lambda: go(eng))
         for _ in range(3):
-            with torch.cuda.stream(stream):
-                graph.replay()
+            graphs.replay(graph, stream)
             go(want)
             assert np.array_equal(want.q_get(0), eng.q_get(0))
             assert np.array_equal(want.get_state()["s"], eng.get_state()["s"])
@@ -141,7 +129,49 @@ def test_large_table_recorded_before_anything_has_run(gpu, call):
         assert np.array_equal(want.q_get(0), eng.q_get(0))
         for e in (want, eng):
             assert e.lib.crl_set_stream(e.h, None) == 0
-        del graph
+        graphs.destroy(graph)
+    graphs.destroy_stream(stream)
+
+
+@pytest.mark.parametrize("W,H", [(40, 30), (90, 70)])
+@pytest.mark.parametrize("call", ["run", "update"])
+def test_recorded_calls_keep_the_buffers_they_were_recorded_with(gpu, graphs, call, W, H):
+    """A larger td_update between two replays needs larger buffers than the recorded launches have."""
+    N = 5000
+    cls, start = gpu.gen_maps_bernoulli(2, 1, N, W, H, 0.15)
+    cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=0.02, eps0=0.3,
+                          episode_len=5, seed=3)
+    stream = graphs.stream()
+    rng = np.random.default_rng(W)
+    small, large, larger = (transitions(rng, W * H, 4, n) for n in (6000, 40000, 90000))
+
+    def go(e):
+        e.step_count = 0
+        if call == "run":
+            e.run_fused(2)
+        else:
+            e.select(fetch=False)
+            e.step()
+            e.update()
+
+    with gpu.Engine(cfg, 0) as want, gpu.Engine(cfg, 0) as eng:
+        for e in (want, eng):
+            e.set_maps(cls, start)
+            assert e.lib.crl_set_stream(e.h, stream) == 0
+            e.td_update(0, *small)
+            go(e)
+        graph = graphs.record(stream, lambda: go(eng))
+        for batch in (small, large, larger):
+            for e in (want, eng):
+                e.td_update(0, *batch)
+            graphs.replay(graph, stream)
+            go(want)
+            assert np.array_equal(want.q_get(0), eng.q_get(0))
+            assert np.array_equal(want.get_state()["s"], eng.get_state()["s"])
+        for e in (want, eng):
+            assert e.lib.crl_set_stream(e.h, None) == 0
+        graphs.destroy(graph)
+    graphs.destroy_stream(stream)
 
 
 @pytest.mark.parametrize("items", [
