@@ -639,13 +639,14 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       if (!p.lanes) p.lds = waves * (p.moves ? mv_lds : map_lds);
     }
   }
+  // (as launch_fused_a() picks the kernel)
   static const char* names[2][3][3] = {
       {{"k_fused_per_env<4,0>", "k_fused_per_env<4,1,general>", "k_fused_per_env<4,2,general>"},
        {"k_fused_per_env<4,0>", "k_fused_per_env<4,1,fast>", "k_fused_per_env<4,2,fast>"},
-       {"k_fused_per_env<4,0>", "k_fused_per_env<4,1,fast,pairs>", "k_fused_per_env<4,2,fast,pairs>"}},
+       {"k_fused_per_env<4,0>", "k_fused_per_env<4,1,fast,lanes>", "k_fused_per_env<4,2,fast,lanes>"}},
       {{"k_fused_per_env<8,0>", "k_fused_per_env<8,1,general>", "k_fused_per_env<8,2,general>"},
        {"k_fused_per_env<8,0>", "k_fused_per_env<8,1,fast>", "k_fused_per_env<8,2,fast>"},
-       {"k_fused_per_env<8,0>", "k_fused_per_env<8,1,fast,pairs>", "k_fused_per_env<8,2,fast,pairs>"}}};
+       {"k_fused_per_env<8,0>", "k_fused_per_env<8,1,fast,lanes>", "k_fused_per_env<8,2,fast,lanes>"}}};
   p.name = names[e->A == 8][!p.fast ? 0 : p.lanes ? 2 : 1][p.map_kind];
   if (p.tickets) {
     static const char* tnames[2][3][2] = {
@@ -655,7 +656,10 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
         {{"k_fused_tickets<8,general,hbm>", "k_fused_tickets<8,general,hbm+lds>"},
          {"k_fused_tickets<8,fast,hbm>", "k_fused_tickets<8,fast,hbm+lds>"},
          {"k_fused_tickets<8,fast+,hbm>", "k_fused_tickets<8,fast+,hbm>"}}};
-    p.name = tnames[e->A == 8][p.rich ? 2 : p.fast ? 1 : 0][p.hybrid];
+    static const char* lnames[2][2] = {{"k_fused_lanes<4,fast>", "k_fused_lanes<4,fast,cells>"},
+                                       {"k_fused_lanes<8,fast>", "k_fused_lanes<8,fast,cells>"}};
+    p.name = p.lanes ? lnames[e->A == 8][(c.reward_flags & CRL_REWARD_CELLS) != 0]
+                     : tnames[e->A == 8][p.rich ? 2 : p.fast ? 1 : 0][p.hybrid];
   }
   return p;
 }
@@ -935,46 +939,57 @@ int td_apply(crl_engine* e, float* Q, const Samples& X, int n, int2* changed, co
   return e->A == 4 ? td_apply_a<4>(e, Q, X, n, changed, sig) : td_apply_a<8>(e, Q, X, n, changed, sig);
 }
 
+// one shared-table step of two launches
+struct SharedPlan {
+  crl::ReduceGeom G;
+  bool two;      // block sums and key owners; else one scan of the samples
+  bool lds_map;  // the map in LDS
+  size_t lds;    // of the act kernel: reduction table (two passes), then the map
+};
+
+int plan_shared_step(const crl_engine* e, SharedPlan* p) {
+  p->G = e->no_alloc ? reduce_geom_within(e, e->N, kScratchExchangeBytes) : reduce_geom(e, e->N);
+  const int rc = choose_passes(e, p->G, &p->two);
+  if (rc) return rc;
+  // The shared table itself stays in L2: streaming its 64 KB into every workgroup's
+  // LDS each step measured slower than the row reads it saves (12.4 against 12.05 us
+  // per step on 65,536 envs, also against the five speculative reads per env).
+  p->lds = p->two ? crl::block_lds_bytes(p->G.own_shift) : 0;
+  const size_t limit = p->two ? kLdsPerWorkgroup - kStaticLdsReserve : (size_t)64 * 1024;
+  const size_t map_bytes = (size_t)e->map_words * 4;
+  p->lds_map = e->cfg.map_mode == CRL_MAP_SHARED && map_bytes <= (size_t)kLdsMapLimitBytes && p->lds + map_bytes <= limit;
+  if (p->lds_map) p->lds += map_bytes;
+  return CRL_OK;
+}
+
 template <int A, int MAP>
-void launch_shared_act(crl_engine* e, bool reduce, const crl::ReduceGeom& G, uint64_t t, int trace_row) {
+void launch_shared_act(crl_engine* e, const SharedPlan& p, uint64_t t, int trace_row) {
   const crl::Rules R = e->rules();
   const crl::Ptrs P = e->ptrs();
   const int block = 256, grid = (e->N + block - 1) / block;
-  const size_t lds = (reduce ? crl::block_lds_bytes(G.own_shift) : 0) + (MAP == 1 ? (size_t)e->map_words * 4 : 0);
-  if (reduce)
-    hipLaunchKernelGGL((crl::k_shared_act<A, MAP, true>), dim3(grid), dim3(block), lds, e->stream, R, P,
-                       t, trace_row, e->key.p, e->delta.p, G, e->ho);
+  if (p.two)
+    hipLaunchKernelGGL((crl::k_shared_act<A, MAP, true>), dim3(grid), dim3(block), p.lds, e->stream, R, P,
+                       t, trace_row, e->key.p, e->delta.p, p.G, e->ho);
   else
-    hipLaunchKernelGGL((crl::k_shared_act<A, MAP, false>), dim3(grid), dim3(block), lds, e->stream, R,
-                       P, t, trace_row, e->key.p, e->delta.p, G, e->ho);
+    hipLaunchKernelGGL((crl::k_shared_act<A, MAP, false>), dim3(grid), dim3(block), p.lds, e->stream, R,
+                       P, t, trace_row, e->key.p, e->delta.p, p.G, e->ho);
 }
 
-// one shared-table step: act (select + move + delta + block sums), then the key owners
+// act (select + move + delta + block sums), then the key owners or the scan
 int shared_step(crl_engine* e, uint64_t t, int trace_row) {
-  const crl::ReduceGeom G = e->no_alloc ? reduce_geom_within(e, e->N, kScratchExchangeBytes) : reduce_geom(e, e->N);
-  bool fast;
-  int rc = choose_passes(e, G, &fast);
-  if (rc == CRL_OK && fast) rc = ensure_handoff(e, G);
+  SharedPlan p{};
+  int rc = plan_shared_step(e, &p);
+  if (rc == CRL_OK && p.two) rc = ensure_handoff(e, p.G);
   if (rc) return rc;
-  // LDS plan of the act kernel: reduction table (fast path), then the map.  The
-  // shared table itself stays in L2: streaming its 64 KB into every workgroup's
-  // LDS each step measured slower than the row reads it saves (12.4 against 12.05 us
-  // per step on 65,536 envs, also against the five speculative reads per env).
-  size_t lds = fast ? crl::block_lds_bytes(G.own_shift) : 0;
-  const size_t limit = fast ? kLdsPerWorkgroup - kStaticLdsReserve : (size_t)64 * 1024;
-  const size_t map_bytes = (size_t)e->map_words * 4;
-  const bool lds_map = e->cfg.map_mode == CRL_MAP_SHARED && map_bytes <= (size_t)kLdsMapLimitBytes &&
-                       lds + map_bytes <= limit;
-  if (lds_map) lds += map_bytes;
   if (e->A == 4) {
-    if (lds_map) launch_shared_act<4, 1>(e, fast, G, t, trace_row);
-    else launch_shared_act<4, 2>(e, fast, G, t, trace_row);
+    if (p.lds_map) launch_shared_act<4, 1>(e, p, t, trace_row);
+    else launch_shared_act<4, 2>(e, p, t, trace_row);
   } else {
-    if (lds_map) launch_shared_act<8, 1>(e, fast, G, t, trace_row);
-    else launch_shared_act<8, 2>(e, fast, G, t, trace_row);
+    if (p.lds_map) launch_shared_act<8, 1>(e, p, t, trace_row);
+    else launch_shared_act<8, 2>(e, p, t, trace_row);
   }
   HIP_TRY(hipGetLastError());
-  if (fast) return reduce_owners(e, G, e->Q.p, e->N, crl::HostSignal{});
+  if (p.two) return reduce_owners(e, p.G, e->Q.p, e->N, crl::HostSignal{});
   const int grid = (int)((e->K + crl::kOwnKeys - 1) / crl::kOwnKeys);
   hipLaunchKernelGGL(crl::k_reduce_scan, dim3(grid), dim3(256), 0, e->stream, e->Q.p, (int)e->K,
                      e->key.p, e->delta.p, e->N, crl::HostSignal{});
@@ -2142,10 +2157,13 @@ int crl_fused_kernel_info(crl_engine* e, int32_t n_steps, char* name, size_t nam
       if (lds_bytes) *lds_bytes = (int32_t)pp.lds;
       return CRL_OK;
     }
-    if (name && name_len) snprintf(name, name_len, "k_shared_act+k_reduce_owners");
-    if (grid) *grid = (e->N + 255) / 256;
+    SharedPlan sp{};
+    const int rc = plan_shared_step(e, &sp);
+    if (rc) return rc;
+    if (name && name_len) snprintf(name, name_len, sp.two ? "k_shared_act+k_reduce_owners" : "k_shared_act+k_reduce_scan");
+    if (grid) *grid = (e->N + 255) / 256;  // (of the first of the two)
     if (block) *block = 256;
-    if (lds_bytes) *lds_bytes = e->map_words * 4;
+    if (lds_bytes) *lds_bytes = (int32_t)sp.lds;
   }
   return CRL_OK;
 }

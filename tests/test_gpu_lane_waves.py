@@ -25,6 +25,7 @@ def check(gpu, oracle, N, W, H, A, chunks, resident=0, variant=0, hybrid=False, 
         for c in chunks:
             plan = eng.fused_kernel_info(c)
             assert ("hbm+lds" in plan["name"]) == hybrid, plan
+            assert hybrid or plan["name"] == "k_fused_lanes<%d,fast%s>" % (A, ",cells" if cells else ""), plan
             assert block is None or plan["block"] == block, plan
             eng.run_fused(c)
             assert sum(eng.fused_split()) == N

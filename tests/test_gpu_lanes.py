@@ -60,14 +60,14 @@ def test_tables_in_lds_beside_words_or_codes(gpu, oracle, A, N, W, H, shared):
 
 
 @pytest.mark.parametrize("A,N,W,H,shared,cells,kernel", [
-    (4, 5000, 24, 21, False, 0, "k_fused_tickets<4,fast,hbm>"),      # codes in LDS
-    (8, 2049, 24, 21, False, 0, "k_fused_tickets<8,fast,hbm>"),
-    (4, 700, 9, 7, False, 3, "k_fused_tickets<4,fast+,hbm>"),        # rewards by cell
-    (8, 700, 9, 7, False, 1, "k_fused_tickets<8,fast+,hbm>"),
-    (4, 300, 70, 66, False, 3, "k_fused_per_env<4,2,fast,pairs>"),   # codes in global memory
-    (8, 300, 70, 66, False, 1, "k_fused_per_env<8,2,fast,pairs>"),
-    (4, 9000, 24, 31, True, 0, "k_fused_per_env<4,1,fast,pairs>"),   # one map's codes in LDS, four waves to a workgroup
-    (8, 4000, 24, 31, True, 3, "k_fused_per_env<8,1,fast,pairs>"),
+    (4, 5000, 24, 21, False, 0, "k_fused_lanes<4,fast>"),      # codes in LDS
+    (8, 2049, 24, 21, False, 0, "k_fused_lanes<8,fast>"),
+    (4, 700, 9, 7, False, 3, "k_fused_lanes<4,fast,cells>"),        # rewards by cell
+    (8, 700, 9, 7, False, 1, "k_fused_lanes<8,fast,cells>"),
+    (4, 300, 70, 66, False, 3, "k_fused_per_env<4,2,fast,lanes>"),   # codes in global memory
+    (8, 300, 70, 66, False, 1, "k_fused_per_env<8,2,fast,lanes>"),
+    (4, 9000, 24, 31, True, 0, "k_fused_per_env<4,1,fast,lanes>"),   # one map's codes in LDS, four waves to a workgroup
+    (8, 4000, 24, 31, True, 3, "k_fused_per_env<8,1,fast,lanes>"),
 ])
 def test_tables_in_hbm(gpu, oracle, A, N, W, H, shared, cells, kernel):
     check(gpu, oracle, N, W, H, A, (129, 70, 1), kernel, shared_map=shared, cells=cells, episode_len=40)

@@ -787,14 +787,14 @@ def test_config5_shape_untraced_pairs_kernel(gpu, oracle):
     """Config 5 at its own shape - 256x256 value-noise maps, 8 actions, per-cell
     rewards, T = 1024, epsilon 1.0 -> 0.05 over 100 episodes - for a few hundred
     envs and more than two episodes, untraced, so that the kernel the benchmark
-    times runs (folded loop, two lanes per env, move codes from global memory):
+    times runs (an env to eight lanes, move codes from global memory):
     every table and all state bit-exact against the oracle."""
     N, steps = 320, 2 * 1024 + 77
     cls, start, cr = gpu.gen_maps_noise(0, N, 256, 256, 16, 0.25, 0.05, 10.0)
     cfg = config5(gpu, N)
     with gpu.Engine(cfg, 0) as eng:
         eng.set_maps(cls, start, cr)
-        assert eng.fused_kernel_info(steps)["name"] == "k_fused_per_env<8,2,fast,pairs>"
+        assert eng.fused_kernel_info(steps)["name"] == "k_fused_per_env<8,2,fast,lanes>"
         eng.run_fused(1024)  # in two launches: the second starts mid-way with trained tables
         eng.run_fused(steps - 1024)
         st, q = eng.get_state(), eng.q_get(0, N)
@@ -827,7 +827,7 @@ def test_full_size_config5(gpu, oracle):
             q = eng.q_get(lo, chunk).reshape(chunk, S, 8)
             same = (q == Q[lo:lo + chunk]).all(axis=(1, 2))
             bad_tables += int(chunk - np.count_nonzero(same))
-    assert info["name"] == "k_fused_per_env<8,2,fast,pairs>"
+    assert info["name"] == "k_fused_per_env<8,2,fast,lanes>"
     for k in ("s", "ep_step", "episode", "reward", "done", "action"):
         assert np.array_equal(st[k], ost[k]), (k, int(np.count_nonzero(st[k] != ost[k])))
     assert bad_tables == 0
