@@ -66,8 +66,12 @@ struct DevBuf {
     release();
     if (count == 0) return hipSuccess;
     hipError_t e = hipMalloc(reinterpret_cast<void**>(&p), count * sizeof(T));
-    if (e == hipSuccess) n = count;
-    else p = nullptr;
+    if (e == hipSuccess) {
+      n = count;
+    } else {
+      p = nullptr;
+      (void)hipGetLastError();  // reported here, not by the next launch's check
+    }
     owned = p != nullptr;
     return e;
   }
@@ -169,11 +173,12 @@ struct crl_engine {
   unsigned* tk = nullptr;  // ticket counters {next ticket, envs on HBM tables, envs on LDS tables}
   bool split_valid = false;  // the last fused launch drew tickets
   unsigned long long* ho = nullptr;  // hand-off cells of the ordered reduction
-  // one-launch shared-table kernel: what its workgroups exchange (the tagged views of
-  // the table's cells, raw samples, hand-off cells), the engine's own give-up word
-  // followed by the phase clocks, and whether a launch has not been checked for
-  // having given up yet
-  DevBuf<unsigned long long> pbuf;
+  // what the workgroups of a shared-table step exchange: the hand-off cells of the ordered
+  // reduction, or all buffers of the one-launch kernel (the tagged views of the table's
+  // cells, raw samples, hand-off cells)
+  DevBuf<unsigned long long> exchange;
+  // one-launch shared-table kernel: the engine's own give-up word followed by the phase
+  // clocks, and whether a launch has not been checked for having given up yet
   DevBuf<unsigned long long> pdiag;  // [0] give-up word, [1..16] phase clocks; allocated at crl_create
   bool persist_unchecked = false;
   bool persist_failed = false;   // a launch gave up: state and table are not valid until they are set again
@@ -239,11 +244,9 @@ struct crl_engine {
   DevBuf<float> tr_r;
   DevBuf<uint8_t> tr_done;
   bool have_transition = false, have_actions = false;
-  // (key, delta) scratch of the ordered reduction, and the block sums its
-  // first pass hands to the key owners
+  // (key, delta) scratch of the ordered reduction
   DevBuf<int32_t> key;
   DevBuf<float> delta;
-  DevBuf<unsigned long long> handoff;
   bool lds_opt_in = false;
   // trace
   DevBuf<int32_t> trace_s;
@@ -851,7 +854,7 @@ int choose_passes(const crl_engine* e, const crl::ReduceGeom& G, bool* two) {
   bool recorded = false;
   if (e->no_alloc) {
     *two = handoff_fits(e, G);
-  } else if (handoff_records(G) > e->handoff.n) {
+  } else if (handoff_records(G) > e->exchange.n) {
     const int rc = query_capture(e, &recorded);
     if (rc) return rc;
     *two = !recorded;
@@ -859,7 +862,8 @@ int choose_passes(const crl_engine* e, const crl::ReduceGeom& G, bool* two) {
   return CRL_OK;
 }
 
-int ensure_handoff(crl_engine* e, const crl::ReduceGeom& G) {
+// (`words`: the engine's own buffer gets at least that many 64-bit words)
+int ensure_handoff(crl_engine* e, const crl::ReduceGeom& G, size_t words = 0) {
   const size_t recs = handoff_records(G);
   if (e->no_alloc) {
     if (!handoff_fits(e, G))
@@ -868,9 +872,9 @@ int ensure_handoff(crl_engine* e, const crl::ReduceGeom& G) {
                   kScratchExchangeBytes);
     e->ho = reinterpret_cast<unsigned long long*>(e->static_scratch + kScratchTicketBytes);
   } else {
-    hipError_t h = e->grow(e->handoff, recs);
+    hipError_t h = e->grow(e->exchange, std::max(recs, words));
     if (h != hipSuccess) return fail(CRL_E_ALLOC, "hand-off buffer allocation failed: %s", hipGetErrorString(h));
-    e->ho = e->handoff.p;
+    e->ho = e->exchange.p;
   }
   return opt_in_lds(e);
 }
@@ -975,11 +979,15 @@ void launch_shared_act(crl_engine* e, const SharedPlan& p, uint64_t t, int trace
                        P, t, trace_row, e->key.p, e->delta.p, p.G, e->ho);
 }
 
+size_t persist_words(const crl_engine* e);
+
 // act (select + move + delta + block sums), then the key owners or the scan
 int shared_step(crl_engine* e, uint64_t t, int trace_row) {
   SharedPlan p{};
   int rc = plan_shared_step(e, &p);
-  if (rc == CRL_OK && p.two) rc = ensure_handoff(e, p.G);
+  // (with room for the one-launch kernel where a longer call would run it: whichever runs first,
+  // no later call allocates, so that it can be recorded)
+  if (rc == CRL_OK && p.two) rc = ensure_handoff(e, p.G, persist_words(e));
   if (rc) return rc;
   if (e->A == 4) {
     if (p.lds_map) launch_shared_act<4, 1>(e, p, t, trace_row);
@@ -1020,32 +1028,45 @@ int persist_min_steps(int n_envs) { return n_envs <= 32768 ? 10 : 8; }
 
 // The one-launch kernel needs every workgroup resident at once (one per compute
 // unit), the dense LDS table of the block pass and one tile of the owners' pass.
-PersistPlan plan_persist(const crl_engine* e, int n_steps) {
-  PersistPlan p{};
-  if (e->cfg.table_mode != CRL_TABLE_SHARED || e->fused_variant == 1 || e->persist_refused) return p;
-  if (e->fused_variant == 0 && n_steps < persist_min_steps(e->N)) return p;
+bool persist_shape(const crl_engine* e, PersistPlan* p) {
   const int n_blocks = (e->N + crl::kBlockSamples - 1) / crl::kBlockSamples;
-  if (e->K > (size_t)crl::kDenseKeys || n_blocks > crl::kPersistMaxGroups || crl::kPersistMaxGroups > kComputeUnits) return p;
+  if (e->cfg.table_mode != CRL_TABLE_SHARED || e->K > (size_t)crl::kDenseKeys || n_blocks > crl::kPersistMaxGroups ||
+      crl::kPersistMaxGroups > kComputeUnits)
+    return false;
   // always 256 workgroups, each a block (with or without envs) and an owner (with or
   // without keys): 16,384 keys at most are 64 to an owner
-  p.G = reduce_geom(e, e->N);
-  p.G.own_shift = crl::kPersistOwnShift;
-  p.G.cell_shift = crl::cell_shift_for(p.G.own_shift);
-  p.G.main_shift = crl::main_shift_for(p.G.own_shift);
-  p.grid = crl::kPersistMaxGroups;
-  p.G.n_blocks = p.grid;  // workgroups without envs hand over empty cells
+  p->G = reduce_geom(e, e->N);
+  p->G.own_shift = crl::kPersistOwnShift;
+  p->G.cell_shift = crl::cell_shift_for(p->G.own_shift);
+  p->G.main_shift = crl::main_shift_for(p->G.own_shift);
+  p->grid = crl::kPersistMaxGroups;
+  p->G.n_blocks = p->grid;  // workgroups without envs hand over empty cells
+  const int n_own = 1 << p->G.own_shift;
+  auto pad = [](size_t words) { return (words + 31) & ~(size_t)31; };  // 256-byte pieces
+  p->at_table = 0;
+  p->at_raw = p->at_table + pad(2 * (size_t)e->K);  // a cell's view: its A values and A neighbours' maxima
+  p->at_cells = p->at_raw + pad(2 * (size_t)e->N);  // raw samples and cells: two buffers each
+  p->words = p->at_cells + 2 * (((size_t)n_own * p->grid) << p->G.cell_shift);
+  return true;
+}
+
+// 64-bit words that the one-launch kernel's workgroups exchange through; 0: it cannot run
+size_t persist_words(const crl_engine* e) {
+  PersistPlan p{};
+  return persist_shape(e, &p) ? p.words : 0;
+}
+
+PersistPlan plan_persist(const crl_engine* e, int n_steps) {
+  PersistPlan p{};
+  if (e->fused_variant == 1 || e->persist_refused) return p;
+  if (e->fused_variant == 0 && n_steps < persist_min_steps(e->N)) return p;
+  if (!persist_shape(e, &p)) return p;
   const crl_config& c = e->cfg;
   p.fold = c.goal_mode == CRL_GOAL_ON_TARGET && c.auto_reset == 1 && c.max_mode == CRL_MAX_TRUE && c.reward_flags == 0 &&
            e->trace_n == 0 && e->sup_n == 0 && c.max_episodes == 0 && c.track_returns == 0;
-  const int n_own = 1 << p.G.own_shift;
   const size_t map_bytes = (size_t)e->map_words * 4;
   p.lds_map = e->cfg.map_mode == CRL_MAP_SHARED && sizeof(crl::PersistLds) + map_bytes <= kLdsPerWorkgroup - kStaticLdsReserve;
   p.lds = sizeof(crl::PersistLds) + (p.lds_map ? map_bytes : 0);
-  auto pad = [](size_t words) { return (words + 31) & ~(size_t)31; };  // 256-byte pieces
-  p.at_table = 0;
-  p.at_raw = p.at_table + pad(2 * (size_t)e->K);  // a cell's view: its A values and A neighbours' maxima
-  p.at_cells = p.at_raw + pad(2 * (size_t)e->N);  // raw samples and cells: two buffers each
-  p.words = p.at_cells + 2 * (((size_t)n_own * p.grid) << p.G.cell_shift);
   if (e->no_alloc && p.words * sizeof(unsigned long long) > kScratchExchangeBytes) return p;
   p.ok = true;
   return p;
@@ -1084,8 +1105,8 @@ int run_persist(crl_engine* e, int n_steps, bool* launched) {
   if (e->no_alloc) {
     buf = reinterpret_cast<unsigned long long*>(e->static_scratch + kScratchTicketBytes);
   } else {
-    if (e->pbuf.ensure(p.words) != hipSuccess) return fail(CRL_E_ALLOC, "allocation of the exchange buffers failed");
-    buf = e->pbuf.p;
+    if (e->grow(e->exchange, p.words) != hipSuccess) return fail(CRL_E_ALLOC, "allocation of the exchange buffers failed");
+    buf = e->exchange.p;
   }
   rc = opt_in_lds(e);
   if (rc) return rc;

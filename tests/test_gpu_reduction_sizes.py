@@ -133,6 +133,40 @@ def test_large_table_recorded_before_anything_has_run(gpu, graphs, call):
     graphs.destroy_stream(stream)
 
 
+@pytest.mark.parametrize("first,recorded", [(60, 6), (6, 60), (60, 60), (6, 6)])
+def test_calls_of_any_length_are_recorded_once_one_has_run(gpu, graphs, first, recorded):
+    """Short calls take two launches to a step, long ones one launch in all: what either needs is
+    there after the first call of any length."""
+    N, W, H = 3000, 16, 16
+    cls, start = gpu.gen_maps_bernoulli(9, 1, N, W, H, 0.12, 0.03)
+    cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=0.003, eps0=0.3,
+                          episode_len=30, seed=4)
+    stream = graphs.stream()
+    with gpu.Engine(cfg, 0) as want, gpu.Engine(cfg, 0) as eng:
+        for e in (want, eng):
+            e.set_maps(cls, start)
+            assert e.lib.crl_set_stream(e.h, stream) == 0
+            e.run_fused(first)
+            e.step_count = 0
+        names = [eng.fused_kernel_info(n)["name"] for n in (6, 60)]
+        assert names == ["k_shared_act+k_reduce_owners", "k_shared_persist<4,1,folded>"]
+        graph = graphs.record(stream, lambda: eng.run_fused(recorded))
+        for _ in range(3):
+            graphs.replay(graph, stream)
+            want.step_count = 0
+            want.run_fused(recorded)
+            assert np.array_equal(want.q_get(0), eng.q_get(0))
+            assert np.array_equal(want.get_state()["s"], eng.get_state()["s"])
+            for e in (want, eng):
+                e.step_count = 9
+                e.run_fused(first)
+        assert np.array_equal(want.q_get(0), eng.q_get(0))
+        for e in (want, eng):
+            assert e.lib.crl_set_stream(e.h, None) == 0
+        graphs.destroy(graph)
+    graphs.destroy_stream(stream)
+
+
 @pytest.mark.parametrize("W,H", [(40, 30), (90, 70)])
 @pytest.mark.parametrize("call", ["run", "update"])
 def test_recorded_calls_keep_the_buffers_they_were_recorded_with(gpu, graphs, call, W, H):
