@@ -531,13 +531,10 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       p.lds_waves = 3;
       while (p.lds_waves > 0 && 16 + hbm_waves * map_lds + p.lds_waves * wave_lds > kLdsPerWorkgroup) --p.lds_waves;
       fits = fits && p.lds_waves > 0;
+      // (no more than it uses: there is a compute unit for every workgroup, and LDS asked for so
+      // that no second one fits beside it gains nothing - 1M envs of 8x8, 300 steps, 81 KB / 57 KB
+      // 2.74 / 2.75 ms; 1M of 16x16, 1000 steps, 148.5 / 146.6 KB 11.75 / 11.75 ms)
       p.lds = 16 + hbm_waves * map_lds + p.lds_waves * wave_lds;
-      // (asked for beyond that: what keeps a second workgroup off the compute unit, and the room
-      // that 32 padded tables with their codes and three waves' maps take, the same for all
-      // plans of a table size where it fits)
-      const size_t alone = kLdsPerWorkgroup / 2 + 1024;
-      const size_t room = 3 * map_lds + (size_t)crl::kTicketEnvs * 4 * (e->K + 4 + (size_t)e->mv_words);
-      p.lds = std::max({p.lds, alone, room <= kLdsPerWorkgroup ? room : 0});
     } else {
       // The general loop's: 32 whole tables (padded by one row against bank conflicts), the
       // LDS wave's maps and at least one table wave's.
@@ -632,8 +629,9 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
         const long most = e->resident_envs > 0 ? std::max<long>(1, resident >> lane_log_envs) : lane_waves;
         p.grid = (int)std::min<long>(lane_units, most);
         p.block = 64;
-        // (where there is a compute unit for every workgroup, LDS for no second one beside it)
-        p.lds = p.grid <= kComputeUnits ? std::max(lane_lds, std::min<size_t>(mv_lds, kLdsMapLimitBytes)) : lane_lds;
+        // (no more than it uses, also where there is a compute unit for every workgroup: 4096 envs
+        // of 32x32, 10,000 steps, 17 / 64 / 81 KB 2.78 / 2.76 / 2.80 ms)
+        p.lds = lane_lds;
       }
       // Tickets dealt by position instead of drawn from a counter: the workers of this plan
       // all take the same time, and 16,384 draws from one counter take 0.38 ms however short
