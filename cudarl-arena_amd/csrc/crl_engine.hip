@@ -1018,11 +1018,14 @@ struct PersistPlan {
 
 // Shortest call worth the set-up of the one-launch kernel (clearing what its workgroups
 // exchange, one co-resident launch: 28 us) instead of two plain launches per step, which cost
-// more the more envs there are (4 / 8 / 10 / 12 steps, one launch against two: 3000 envs of
-// 16x16 52 / 75 / 86 / 97 us, 31 / 60 / 74 / 89; 20,000 of 32x32 with 8 actions 57 / 84 / 96 / 109,
-// 40 / 75 / 93 / 112; 65,536 of 64x64 57 / 85 / 99 / 113, 45 / 86 / 107 / 128).  With a few
-// thousand envs the two cross at 16 steps only; calls of ten keep the one launch.
-int persist_min_steps(int n_envs) { return n_envs <= 32768 ? 10 : 8; }
+// more the more envs there are.  Where the two cross (us per call, one launch / two, at 8, 12 and
+// 16 steps): 3000 envs of 16x16 75/58, 97/88, 119/118; 8000 of 32x32 77/61, 100/91, 123/122;
+// 12,000 of 64x64 78/66, 102/98, 125/131; 16,000 of 32x32 77/64, 100/95, 122/126; 24,000 of 64x64
+// 78/68, 102/102, 126/137; 32,768 of 64x64 82/71, 106/106, 130/141; 40,000 of 32x32 79/73, 103/109,
+// 126/145; 65,536 of 64x64 85/85, 113/127, 139/168.
+int persist_min_steps(int n_envs) {
+  return n_envs <= 8192 ? 16 : n_envs <= 16384 ? 14 : n_envs <= 32768 ? 12 : n_envs <= 49152 ? 10 : 9;
+}
 
 // The one-launch kernel needs every workgroup resident at once (one per compute
 // unit), the dense LDS table of the block pass and one tile of the owners' pass.

@@ -387,7 +387,8 @@ def test_shared_table_one_launch_kernel_shapes(gpu, oracle):
     cfg = gpu.make_config(300, 16, 16, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=0.01, eps0=0.3,
                           episode_len=25, seed=3, trap_reward=-0.5)
     with gpu.Engine(cfg, 0) as eng:
-        assert eng.fused_kernel_info(10)["name"] == "k_shared_persist<4,1,folded>"  # (automatic; the common rules)
+        assert eng.fused_kernel_info(16)["name"] == "k_shared_persist<4,1,folded>"  # (automatic; the common rules)
+        assert eng.fused_kernel_info(15)["name"] == "k_shared_act+k_reduce_owners"
         eng.set_fused_variant(1)
         assert eng.fused_kernel_info(10)["name"] == "k_shared_act+k_reduce_owners"
         eng.set_fused_variant(2)

@@ -133,6 +133,25 @@ def test_large_table_recorded_before_anything_has_run(gpu, graphs, call):
     graphs.destroy_stream(stream)
 
 
+@pytest.mark.parametrize("N,steps", [(8192, 16), (8193, 14), (16385, 12), (32769, 10), (49153, 9)])
+def test_calls_on_either_side_of_the_shortest_one_launch_call(gpu, oracle, N, steps):
+    W, H = 24, 21
+    cls, start = gpu.gen_maps_bernoulli(9, 1, N, W, H, 0.12, 0.03)
+    cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=0.003, eps0=0.3,
+                          episode_len=30, seed=4)
+    with gpu.Engine(cfg, 0) as eng:
+        eng.set_maps(cls, start)
+        assert eng.fused_kernel_info(steps)["name"].startswith("k_shared_persist")
+        assert eng.fused_kernel_info(steps - 1)["name"] == "k_shared_act+k_reduce_owners"
+        for n in (steps, steps - 1, steps):
+            eng.run_fused(n)
+        q, st = eng.q_get(0), eng.get_state()
+    Q = np.zeros((1, W * H, 4), np.float32)
+    ost = oracle.new_state(cfg, start)
+    oracle.run(cfg, cls, None, start, Q, ost, 0, 3 * steps - 1)
+    assert np.array_equal(q, Q[0]) and np.array_equal(st["s"], ost["s"])
+
+
 @pytest.mark.parametrize("first,recorded", [(60, 6), (6, 60), (60, 60), (6, 6)])
 def test_calls_of_any_length_are_recorded_once_one_has_run(gpu, graphs, first, recorded):
     """Short calls take two launches to a step, long ones one launch in all: what either needs is
