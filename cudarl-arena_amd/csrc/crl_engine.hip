@@ -891,54 +891,83 @@ int reduce_owners(crl_engine* e, const crl::ReduceGeom& G, float* Q, int n, cons
 }
 
 // Q[k] += ordered sum of the deltas of the n samples with key k, on one table.
-// `changed`, `sig`: see k_td_small, for at most 1024 samples; with more, `sig` says that the
-// samples have been read.
-template <int A, class Samples>
-int td_apply_a(crl_engine* e, float* Q, const Samples& X, int n, int2* changed, const crl::HostSignal& sig) {
-  const float lr = e->cfg.lr, gamma = e->cfg.gamma;
-  const int max_mode = e->cfg.max_mode;
-  int rc = opt_in_lds(e);
+// Up to kSmallSamples in one launch; `changed`, `sig`: see k_td_small.
+template <class Samples>
+int td_small(crl_engine* e, float* Q, const Samples& X, int n, int2* changed, const crl::HostSignal& sig) {
+  const int rc = opt_in_lds(e);
   if (rc) return rc;
-  if (n <= crl::kSmallSamples) {
-#define CRL_TD_SMALL(NB)                                                                                      \
-  hipLaunchKernelGGL((crl::k_td_small<A, NB, Samples>), dim3(1), dim3(crl::kBlockSamples * NB),               \
-                     sizeof(crl::SmallLds<NB>), e->stream, X, n, Q, lr, gamma, max_mode, changed, sig)
-    if (n <= crl::kBlockSamples) CRL_TD_SMALL(1);
-    else if (n <= 2 * crl::kBlockSamples) CRL_TD_SMALL(2);
-    else CRL_TD_SMALL(4);
+#define CRL_TD_SMALL(A, NB)                                                                                        \
+  hipLaunchKernelGGL((crl::k_td_small<A, NB, Samples>), dim3(1), dim3(crl::kBlockSamples * NB),                    \
+                     sizeof(crl::SmallLds<NB>), e->stream, X, n, Q, e->cfg.lr, e->cfg.gamma, e->cfg.max_mode, changed, sig)
+#define CRL_TD_SMALL_A(NB)              \
+  do {                                  \
+    if (e->A == 4) CRL_TD_SMALL(4, NB); \
+    else CRL_TD_SMALL(8, NB);           \
+  } while (0)
+  if (n <= crl::kBlockSamples) CRL_TD_SMALL_A(1);
+  else if (n <= 2 * crl::kBlockSamples) CRL_TD_SMALL_A(2);
+  else CRL_TD_SMALL_A(4);
+#undef CRL_TD_SMALL_A
 #undef CRL_TD_SMALL
-    HIP_TRY(hipGetLastError());
-    return CRL_OK;
-  }
-  hipError_t h = e->grow(e->key, (size_t)n);
-  if (h == hipSuccess) h = e->grow(e->delta, (size_t)n);
-  if (h != hipSuccess) return fail(CRL_E_ALLOC, "scratch allocation failed: %s", hipGetErrorString(h));
-  const crl::ReduceGeom G = reduce_geom(e, n);
-  const int grid = G.n_blocks;
-  e->no_alloc = false;  // crl_update / crl_td_update: the engine's own hand-off buffer
-  bool two;
-  rc = choose_passes(e, G, &two);
-  if (rc) return rc;
-  if (two) {
-    rc = ensure_handoff(e, G);
-    if (rc) return rc;
-    hipLaunchKernelGGL((crl::k_td_blocks<A, Samples>), dim3(grid), dim3(crl::kBlockSamples),
-                       crl::block_lds_bytes(G.own_shift), e->stream, G, X, n, Q, lr, gamma, max_mode, e->key.p,
-                       e->delta.p, e->ho);
-    HIP_TRY(hipGetLastError());
-    return reduce_owners(e, G, Q, n, sig);
-  }
-  hipLaunchKernelGGL((crl::k_delta<A, Samples>), dim3(grid), dim3(256), 0, e->stream, Q, X, n, lr, gamma, max_mode,
-                     e->key.p, e->delta.p);
-  HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(crl::k_reduce_scan, dim3((unsigned)((e->K + crl::kOwnKeys - 1) / crl::kOwnKeys)), dim3(256), 0,
-                     e->stream, Q, (int)e->K, e->key.p, e->delta.p, n, sig);
   HIP_TRY(hipGetLastError());
   return CRL_OK;
 }
+
+// More: a begin, the samples in one piece or several (whole blocks but for the last), an end.
+struct TdPlan {
+  crl::ReduceGeom G;
+  int n;
+  bool two;  // two passes, or the scan
+};
+
+int td_begin(crl_engine* e, int n, TdPlan* p) {
+  hipError_t h = e->grow(e->key, (size_t)n);
+  if (h == hipSuccess) h = e->grow(e->delta, (size_t)n);
+  if (h != hipSuccess) return fail(CRL_E_ALLOC, "scratch allocation failed: %s", hipGetErrorString(h));
+  p->n = n;
+  p->G = reduce_geom(e, n);
+  e->no_alloc = false;  // crl_update / crl_td_update: the engine's own hand-off buffer
+  const int rc = choose_passes(e, p->G, &p->two);
+  if (rc) return rc;
+  return p->two ? ensure_handoff(e, p->G) : opt_in_lds(e);
+}
+
+// samples [at, at + m), which are X's first; `before`: says that the pieces before have been read
 template <class Samples>
-int td_apply(crl_engine* e, float* Q, const Samples& X, int n, int2* changed, const crl::HostSignal& sig) {
-  return e->A == 4 ? td_apply_a<4>(e, Q, X, n, changed, sig) : td_apply_a<8>(e, Q, X, n, changed, sig);
+int td_piece(crl_engine* e, const TdPlan& p, const float* Q, const Samples& X, size_t at, int m,
+             const crl::HostSignal& before) {
+  const float lr = e->cfg.lr, gamma = e->cfg.gamma;
+  const int max_mode = e->cfg.max_mode;
+  const size_t block = at / crl::kBlockSamples;
+  const dim3 grid((m + crl::kBlockSamples - 1) / crl::kBlockSamples);
+  int32_t* key = e->key.p + at;
+  float* delta = e->delta.p + at;
+  if (p.two) {
+    unsigned long long* cells = e->ho + (block << p.G.cell_shift);
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, dim3(crl::kBlockSamples), crl::block_lds_bytes(p.G.own_shift), e->stream, p.G, X, m, Q,
+                         lr, gamma, max_mode, key, delta, cells, before);
+    };
+    if (e->A == 4) go(crl::k_td_blocks<4, Samples>);
+    else go(crl::k_td_blocks<8, Samples>);
+  } else {
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, dim3(256), 0, e->stream, Q, X, m, lr, gamma, max_mode, key, delta, before);
+    };
+    if (e->A == 4) go(crl::k_delta<4, Samples>);
+    else go(crl::k_delta<8, Samples>);
+  }
+  HIP_TRY(hipGetLastError());
+  return CRL_OK;
+}
+
+// `read`: says that the samples have been read
+int td_end(crl_engine* e, const TdPlan& p, float* Q, const crl::HostSignal& read) {
+  if (p.two) return reduce_owners(e, p.G, Q, p.n, read);
+  hipLaunchKernelGGL(crl::k_reduce_scan, dim3((unsigned)((e->K + crl::kOwnKeys - 1) / crl::kOwnKeys)), dim3(256), 0,
+                     e->stream, Q, (int)e->K, e->key.p, e->delta.p, p.n, read);
+  HIP_TRY(hipGetLastError());
+  return CRL_OK;
 }
 
 // one shared-table step of two launches
@@ -1151,7 +1180,11 @@ int run_persist(crl_engine* e, int n_steps, bool* launched) {
 // ---- pinned memory between host and kernels --------------------------------------------
 
 constexpr size_t kLinkLimitBytes = (size_t)4 << 20;  // larger transfers: hipMemcpyAsync straight to and from the caller's memory
-constexpr size_t kInSlotKeepBytes = (size_t)32 << 20;
+// Transitions of a crl_td_update that go through one page.  Larger pieces cost more to pin, smaller
+// ones more launches (one page of their own for all / pieces of 65,536 / 131,072 / 262,144, us per
+// call among others: 262,144 82 / 97 / 84 / 83, 1 million 400 / 375 / 325 / 300, 6 million 39,900 /
+// 13,000 / 12,400 / 12,300; alone: 262,144 157 / 126 / 127 / 155).
+constexpr int kPieceSamples = 1 << 17;
 constexpr int kFlagErrWord = 16;                     // of flag_page; in another 64-byte line than the flag
 
 // the next launch that tells the host when it is through
@@ -1611,6 +1644,59 @@ int refuse_capture(const crl_engine* e) {
   return fail(CRL_E_DEVICE, "a call that takes host data cannot be recorded: its stream is being captured");
 }
 
+// Transitions [at, at + n) of a call packed into a page.
+int pack_page(const crl_engine* e, size_t at, int n, const int32_t* s, const int32_t* a, const float* r,
+              const int32_t* s_next, const uint8_t* done, unsigned char* page, crl::PackedSamples* X) {
+  int32_t* key = reinterpret_cast<int32_t*>(page);
+  uint32_t* s2d = reinterpret_cast<uint32_t*>(key + n);
+  if (!crl::pack_transitions(n, (int)e->S, e->A, s + at, a + at, s_next + at, done + at, key, s2d))
+    for (size_t i = at; i < at + n; ++i) {
+      if (s[i] < 0 || (size_t)s[i] >= e->S) return fail(CRL_E_RANGE, "s[%zu] = %d outside [0,%zu)", i, s[i], e->S);
+      if (s_next[i] < 0 || (size_t)s_next[i] >= e->S)
+        return fail(CRL_E_RANGE, "s_next[%zu] = %d outside [0,%zu)", i, s_next[i], e->S);
+    }
+  std::memcpy(s2d + n, r + at, (size_t)n * 4);
+  X->key = key;
+  X->s2d = s2d;
+  X->r = reinterpret_cast<const float*>(s2d + n);
+  return CRL_OK;
+}
+
+// Even pieces of at most kPieceSamples, each a page and a launch of the first pass of its own:
+// a piece is packed while the kernels read the ones before.  A page is free again when the
+// launch after the one that reads it starts.
+int td_pieces(crl_engine* e, float* Q, int n, const int32_t* s, const int32_t* a, const float* r, const int32_t* s_next,
+              const uint8_t* done) {
+  TdPlan p;
+  int rc = td_begin(e, n, &p);
+  if (rc) return rc;
+  const size_t pieces = ((size_t)n + kPieceSamples - 1) / kPieceSamples;
+  const size_t even = ((n + pieces - 1) / pieces + crl::kBlockSamples - 1) & ~(size_t)(crl::kBlockSamples - 1);
+  crl_engine::InSlot* unread = nullptr;  // the page of the last launch
+  auto read = [&]() {
+    crl::HostSignal sig{};
+    if (unread) sig = next_signal(e);
+    return sig;
+  };
+  for (size_t at = 0; at < (size_t)n; at += even) {
+    const int m = (int)std::min(even, n - at);
+    crl_engine::InSlot* slot;
+    crl::PackedSamples X;
+    rc = claim_in_slot(e, 12 * even, &slot);
+    if (rc == CRL_OK) rc = pack_page(e, at, m, s, a, r, s_next, done, slot->page.p, &X);
+    if (rc) return rc;
+    const crl::HostSignal sig = read();
+    rc = td_piece(e, p, Q, X, at, m, sig);
+    if (rc) return rc;
+    if (unread) unread->last_seq = sig.seq;
+    unread = slot;
+  }
+  const crl::HostSignal sig = read();
+  rc = td_end(e, p, Q, sig);
+  if (rc == CRL_OK) unread->last_seq = sig.seq;
+  return rc;
+}
+
 // crl_td_update and, with `keys`, crl_td_update_collect.  The transitions are packed into
 // pinned memory, 12 bytes each, in the pass that checks them, and the kernel reads them
 // there: the call returns without waiting for anything (65,536 transitions: five copies from
@@ -1625,33 +1711,28 @@ int td_update(crl_engine* e, int32_t table, int32_t n, const int32_t* s, const i
   if (!s || !a || !r || !s_next || !done) return fail(CRL_E_ARG, "null transition array");
   rc = refuse_capture(e);
   if (rc) return rc;
-  const size_t nn = (size_t)n;
-  crl_engine::InSlot* slot = nullptr;
-  rc = claim_in_slot(e, 12 * nn, &slot);
-  if (rc) return rc;
+  float* Q = e->Q.p + (size_t)table * e->K;
+  if (n > crl::kSmallSamples) {
+    rc = td_pieces(e, Q, n, s, a, r, s_next, done);
+    // nothing may be left that works on a page or waits for a number that never comes (nothing has
+    // been applied: what is launched before the end only reads the table)
+    if (rc) (void)hipStreamSynchronize(e->stream);
+    return rc;
+  }
+  crl_engine::InSlot* slot;
   crl::PackedSamples X;
-  int32_t* key = reinterpret_cast<int32_t*>(slot->page.p);
-  uint32_t* s2d = reinterpret_cast<uint32_t*>(key + nn);
-  X.key = key;
-  X.s2d = s2d;
-  X.r = reinterpret_cast<const float*>(s2d + nn);
-  if (!crl::pack_transitions(n, (int)e->S, e->A, s, a, s_next, done, key, s2d))
-    for (int i = 0; i < n; ++i) {
-      if (s[i] < 0 || (size_t)s[i] >= e->S) return fail(CRL_E_RANGE, "s[%d] = %d outside [0,%zu)", i, s[i], e->S);
-      if (s_next[i] < 0 || (size_t)s_next[i] >= e->S)
-        return fail(CRL_E_RANGE, "s_next[%d] = %d outside [0,%zu)", i, s_next[i], e->S);
-    }
-  std::memcpy(s2d + nn, r, nn * 4);
+  rc = claim_in_slot(e, 12 * (size_t)n, &slot);
+  if (rc == CRL_OK) rc = pack_page(e, 0, n, s, a, r, s_next, done, slot->page.p, &X);
+  if (rc) return rc;
   int2* changed = nullptr;
   if (keys) {
-    rc = claim_out_page(e, nn * sizeof(int2));
+    rc = claim_out_page(e, n * sizeof(int2));
     if (rc) return rc;
     changed = reinterpret_cast<int2*>(e->out_page.p);
   }
   const crl::HostSignal sig = next_signal(e);
-  rc = td_apply(e, e->Q.p + (size_t)table * e->K, X, n, changed, sig);
+  rc = td_small(e, Q, X, n, changed, sig);
   if (rc) {
-    // nothing may be left that works on the page or waits for a number that never comes
     (void)hipStreamSynchronize(e->stream);
     return rc;
   }
@@ -1663,12 +1744,6 @@ int td_update(crl_engine* e, int32_t table, int32_t n, const int32_t* s, const i
       keys[i] = changed[i].x;
       std::memcpy(values + i, &changed[i].y, 4);
     }
-  }
-  if (slot->page.n > kInSlotKeepBytes) {  // a page that large is not kept
-    rc = wait_seq(e, sig.seq);
-    slot->last_seq = 0;
-    if (rc) return rc;
-    slot->page.release();
   }
   return CRL_OK;
 }
@@ -1923,7 +1998,15 @@ int crl_update(crl_engine* e) {
                          e->transition());
     HIP_TRY(hipGetLastError());
   } else {
-    rc = td_apply(e, e->Q.p, e->transition(), e->N, nullptr, crl::HostSignal{});
+    const crl::Transition X = e->transition();
+    if (e->N <= crl::kSmallSamples) {
+      rc = td_small(e, e->Q.p, X, e->N, nullptr, crl::HostSignal{});
+    } else {
+      TdPlan p;
+      rc = td_begin(e, e->N, &p);
+      if (rc == CRL_OK) rc = td_piece(e, p, e->Q.p, X, 0, e->N, crl::HostSignal{});
+      if (rc == CRL_OK) rc = td_end(e, p, e->Q.p, crl::HostSignal{});
+    }
     if (rc) return rc;
   }
   e->have_transition = false;

@@ -1474,12 +1474,14 @@ __global__ __launch_bounds__(256) void k_update_per_env(const Rules R, const Ptr
 }
 
 // (key, delta) of n samples against ONE table (K = S*A entries), all reads before any
-// write, for the reduction that scans them.
+// write, for the reduction that scans them.  `before`: see signal_reached.
 template <int A, class Samples>
 __global__ __launch_bounds__(256) void k_delta(const float* __restrict__ Q, const Samples X, const int n,
                                                 const float lr, const float gamma, const int max_mode,
-                                                int32_t* __restrict__ key, float* __restrict__ delta) {
+                                                int32_t* __restrict__ key, float* __restrict__ delta,
+                                                const HostSignal before) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  signal_reached(before);
   int k;
   float d;
   sample_delta<A>(X, i, n, Q, lr, gamma, max_mode, k, d);

@@ -466,15 +466,18 @@ __device__ __forceinline__ void reduce_block_wide(unsigned char* lds, const Redu
     if (handed[o] == 0) handoff[(((size_t)o * G.n_blocks) + block) << G.cell_shift] = 0ull;
 }
 
-// Pass 1 over samples in memory (which may be the host's: each is read once).
+// Pass 1 over samples in memory (which may be the host's: each is read once).  `before`: see
+// signal_reached.
 template <int A, class Samples>
 __global__ __launch_bounds__(kBlockSamples) void k_td_blocks(const ReduceGeom G, const Samples X, const int n,
                                                              const float* __restrict__ Q, const float lr,
                                                              const float gamma, const int max_mode,
                                                              int32_t* __restrict__ key, float* __restrict__ delta,
-                                                             unsigned long long* __restrict__ handoff) {
+                                                             unsigned long long* __restrict__ handoff,
+                                                             const HostSignal before) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int i = blockIdx.x * kBlockSamples + threadIdx.x;
+  signal_reached(before);
   int k;
   float d;
   block_lds_init(lds_raw, G);
@@ -532,7 +535,7 @@ __global__ __launch_bounds__(kOwnerWaves * 64) void k_reduce_owners(const Reduce
   uint32_t* claim = reinterpret_cast<uint32_t*>(own);      // else: [own_keys]
   float* list_v = own + (TILE ? kGroupBlocks * kTileKeys : own_keys);
   uint16_t* list_s = reinterpret_cast<uint16_t*>(list_v + kBlockSamples);
-  if (sig.flag && owner == 0 && tid == 0) __hip_atomic_store(sig.flag, sig.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  signal_reached(sig);
   // the table entry this thread will update first: fetched now, needed last
   const int key0 = tid < own_keys ? key_of(owner, tid, G) : G.K;
   const float q0 = key0 < G.K ? Q[key0] : 0.0f;
@@ -788,7 +791,7 @@ __global__ __launch_bounds__(256) void k_reduce_scan(float* __restrict__ Q, cons
   const int wave = tid >> 6;
   const int owner = blockIdx.x;
   float total = 0.0f;
-  if (sig.flag && owner == 0 && tid == 0) __hip_atomic_store(sig.flag, sig.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  signal_reached(sig);
 
   for (int g0 = 0; g0 < n; g0 += 4 * kSpan) {
     int cnt = 0;

@@ -37,6 +37,40 @@ def test_sample_counts(gpu, oracle, n, W, H, A):
     check(gpu, oracle, W, H, A, [transitions(rng, W * H, A, n) for _ in range(6)], mode=n & 1)
 
 
+PIECE = 1 << 17  # transitions of a call that go through one page
+
+
+@pytest.mark.parametrize("n", [PIECE - 1, PIECE, PIECE + 1, 2 * PIECE + 257, 5 * PIECE - 300])
+@pytest.mark.parametrize("W,H,A", [(8, 8, 4), (101, 99, 8), (1025, 1024, 4)])  # 1.05 million cells: the scan
+def test_batches_of_several_pieces(gpu, oracle, n, W, H, A):
+    """Calls large and small in turn, so that pages of one call's pieces are another's."""
+    if W > 1000 and n > PIECE + 1:
+        n = 2 * PIECE + 1
+    rng = np.random.default_rng(n)
+    big = transitions(rng, W * H, A, n)
+    check(gpu, oracle, W, H, A, [big, transitions(rng, W * H, A, 5000), transitions(rng, W * H, A, 700), big])
+
+
+def test_a_late_piece_that_is_refused_leaves_the_table_alone(gpu, oracle):
+    W, H, A = 12, 10, 4
+    S, n = W * H, 3 * PIECE
+    rng = np.random.default_rng(3)
+    good = transitions(rng, S, A, n)
+    cfg = gpu.make_config(1, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED)
+    want = rng.normal(0, 1, S * A).astype(np.float32)
+    with gpu.Engine(cfg, 0) as eng:
+        eng.q_set(0, want)
+        for at, which in ((n - 1, 0), (PIECE + 5, 3), (0, 0)):
+            bad = [x.copy() for x in good]
+            bad[which][at] = S if which else -1
+            with pytest.raises(gpu.CrlError, match=r"\[%d\]" % at):
+                eng.td_update(0, *bad)
+            assert np.array_equal(eng.q_get(0).reshape(-1), want)
+        eng.td_update(0, *good)
+        oracle.td_update_batch(want, S, A, *good, 0.1, 0.99, 0)
+        assert np.array_equal(eng.q_get(0).reshape(-1), want)
+
+
 @pytest.mark.parametrize("W,H,A", [(16, 16, 8), (16, 17, 8), (64, 65, 4), (181, 181, 8), (400, 400, 8)])
 def test_table_sizes(gpu, oracle, W, H, A):
     rng = np.random.default_rng(W)
