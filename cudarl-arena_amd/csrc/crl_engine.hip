@@ -200,13 +200,16 @@ struct crl_engine {
   DevBuf<unsigned> flag_count;  // workgroups of a signalling launch that are through
   unsigned seq = 0;             // number of the last signalled launch
   crl::PinBuf out_page;         // what kernels hand to the host: state, statistics, actions, tables
+  // What the host hands to kernels: one pinned block cut into pages that are taken in turn.
+  crl::PinBuf in_block;
   struct InSlot {
-    crl::PinBuf page;
+    unsigned char* page = nullptr;
     unsigned last_seq = 0;  // the launch that reads it
   };
   static constexpr int kInSlots = 4;
-  InSlot in_slot[kInSlots];     // what the host hands to kernels, taken in turn
-  int in_next = 0;
+  InSlot in_slot[kInSlots];
+  int in_slots = 0, in_next = 0;  // pages there are, the one taken next
+  size_t in_page_bytes = 0;
   // A call of this engine has been recorded into a graph: what its launches work on stays
   // allocated until the engine goes, also where a later call needs a larger buffer.
   bool recorded = false;
@@ -1180,6 +1183,7 @@ int run_persist(crl_engine* e, int n_steps, bool* launched) {
 // ---- pinned memory between host and kernels --------------------------------------------
 
 constexpr size_t kLinkLimitBytes = (size_t)4 << 20;  // larger transfers: hipMemcpyAsync straight to and from the caller's memory
+constexpr size_t kInPageBytesOfFour = (size_t)128 << 10;  // larger pages are two
 // Transitions of a crl_td_update that go through one page.  Larger pieces cost more to pin, smaller
 // ones more launches (one page of their own for all / pieces of 65,536 / 131,072 / 262,144, us per
 // call among others: 262,144 82 / 97 / 84 / 83, 1 million 400 / 375 / 325 / 300, 6 million 39,900 /
@@ -1232,16 +1236,37 @@ int claim_out_page(crl_engine* e, size_t bytes) {
   return CRL_OK;
 }
 
-// a page for `bytes` that no earlier launch still reads
+// The launch that reads this page is through.
+int wait_slot(crl_engine* e, crl_engine::InSlot& slot) {
+  if (slot.last_seq == 0) return CRL_OK;
+  const int rc = wait_seq(e, slot.last_seq);
+  if (rc == CRL_OK) slot.last_seq = 0;
+  return rc;
+}
+
+// A page for `bytes` that no earlier launch still reads.  The pages grow together, and are two
+// where they are large: what they cost is the first touch of their memory (0.37 ms per MB), paid
+// by the first call that takes each of them.
 int claim_in_slot(crl_engine* e, size_t bytes, crl_engine::InSlot** out) {
-  crl_engine::InSlot& slot = e->in_slot[e->in_next];
-  e->in_next = (e->in_next + 1) % crl_engine::kInSlots;
-  if (slot.last_seq != 0) {
-    const int rc = wait_seq(e, slot.last_seq);
-    if (rc) return rc;
-    slot.last_seq = 0;
+  if (bytes > e->in_page_bytes) {
+    for (auto& slot : e->in_slot) {
+      const int rc = wait_slot(e, slot);
+      if (rc) return rc;
+    }
+    size_t page = 4096;
+    while (page < bytes) page *= 2;
+    const int slots = page > kInPageBytesOfFour ? 2 : crl_engine::kInSlots;
+    e->in_page_bytes = 0;
+    if (!e->in_block.ensure(page * slots)) return fail(CRL_E_ALLOC, "pinned host memory: %zu bytes", page * slots);
+    e->in_page_bytes = page;
+    e->in_slots = slots;
+    e->in_next = 0;
+    for (int i = 0; i < slots; ++i) e->in_slot[i].page = e->in_block.p + page * i;
   }
-  if (!slot.page.ensure(bytes)) return fail(CRL_E_ALLOC, "pinned host memory: %zu bytes", bytes);
+  crl_engine::InSlot& slot = e->in_slot[e->in_next];
+  e->in_next = (e->in_next + 1) % e->in_slots;
+  const int rc = wait_slot(e, slot);
+  if (rc) return rc;
   *out = &slot;
   return CRL_OK;
 }
@@ -1683,7 +1708,7 @@ int td_pieces(crl_engine* e, float* Q, int n, const int32_t* s, const int32_t* a
     crl_engine::InSlot* slot;
     crl::PackedSamples X;
     rc = claim_in_slot(e, 12 * even, &slot);
-    if (rc == CRL_OK) rc = pack_page(e, at, m, s, a, r, s_next, done, slot->page.p, &X);
+    if (rc == CRL_OK) rc = pack_page(e, at, m, s, a, r, s_next, done, slot->page, &X);
     if (rc) return rc;
     const crl::HostSignal sig = read();
     rc = td_piece(e, p, Q, X, at, m, sig);
@@ -1722,7 +1747,7 @@ int td_update(crl_engine* e, int32_t table, int32_t n, const int32_t* s, const i
   crl_engine::InSlot* slot;
   crl::PackedSamples X;
   rc = claim_in_slot(e, 12 * (size_t)n, &slot);
-  if (rc == CRL_OK) rc = pack_page(e, 0, n, s, a, r, s_next, done, slot->page.p, &X);
+  if (rc == CRL_OK) rc = pack_page(e, 0, n, s, a, r, s_next, done, slot->page, &X);
   if (rc) return rc;
   int2* changed = nullptr;
   if (keys) {
@@ -1912,8 +1937,8 @@ int crl_step(crl_engine* e, const int32_t* actions) {
     // the kernel reads the actions where they are put now, and the caller's buffer is free
     rc = claim_in_slot(e, bytes, &slot);
     if (rc) return rc;
-    std::memcpy(slot->page.p, actions, bytes);
-    act = reinterpret_cast<const int32_t*>(slot->page.p);
+    std::memcpy(slot->page, actions, bytes);
+    act = reinterpret_cast<const int32_t*>(slot->page);
   } else {
     HIP_TRY(hipMemcpyAsync(e->act.p, actions, bytes, hipMemcpyHostToDevice, e->stream));
     // the host buffer may be reused as soon as we return

@@ -147,6 +147,26 @@ def test_actions_may_be_overwritten_once_step_has_returned(gpu):
     assert np.array_equal(st["s"], y * 11 + x)
 
 
+def test_pages_grow_while_earlier_calls_still_read_them(gpu, oracle):
+    """Batches of growing and shrinking size one after the other, without a wait between: four
+    pages of a small size, two of a large one, all of one block."""
+    W, H, A = 30, 20, 4
+    S = W * H
+    rng = np.random.default_rng(2)
+    sizes = [1, 300, 900, 341, 342, 1025, 10922, 10923, 5, 40000, 3, 3, 3, 131072, 1500, 131073, 7, 200000, 64, 64, 64, 64, 64]
+    want = rng.normal(0, 1, S * A).astype(np.float32)
+    cfg = gpu.make_config(1, W, H, n_actions=A, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=1e-3)
+    with gpu.Engine(cfg, 0) as eng:
+        eng.q_set(0, want)
+        batches = [(rng.integers(0, S, n), rng.integers(0, A, n), rng.normal(0, 1, n).astype(np.float32),
+                    rng.integers(0, S, n), (rng.random(n) < 0.2).astype(np.uint8)) for n in sizes]
+        for b in batches:
+            eng.td_update(0, *b)
+        for b in batches:
+            oracle.td_update_batch(want, S, A, *b, 1e-3, 0.99, 0)
+        assert np.array_equal(eng.q_get(0).reshape(-1), want)
+
+
 def test_calls_that_take_host_data_are_refused_under_capture(gpu):
     """Their kernels read pages that are taken in turn: a replay would read another call's."""
     import torch
