@@ -735,7 +735,11 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
 }
 
 constexpr int kScanBlocks = 2;
-constexpr size_t kHandoffLimitBytes = (size_t)128 << 20;
+// 8.4 million envs' cells for 256 owners, 524,288 envs' for 4096.  Two passes against the scan, us
+// per step: 4 million envs of 16x16 310 / 36,300, 8 million 632 / 74,000, 140,000 envs of 1024x1024
+// 179 / 5160, 500,000 668 / 18,000.
+constexpr size_t kHandoffLimitBytes = (size_t)512 << 20;
+constexpr size_t kNoAllocScanBytes = (size_t)128 << 20;
 
 int ceil_log2(size_t v) {
   int b = 0;
@@ -769,7 +773,8 @@ size_t handoff_records(const crl::ReduceGeom& G) {
 }
 
 // Small tables need less room with as many owners as 64 keys each make: for a call whose
-// hand-off cells have to fit into `limit`.
+// hand-off cells have to fit into `limit` (4 million envs of 16x16: 581 us per step with 16 owners,
+// 310 with 256).
 crl::ReduceGeom reduce_geom_within(const crl_engine* e, int n, size_t limit) {
   crl::ReduceGeom G = reduce_geom(e, n);
   if (handoff_records(G) * sizeof(unsigned long long) <= limit || e->K > (size_t)crl::kDenseKeys) return G;
@@ -846,16 +851,19 @@ int query_capture(const crl_engine* e, bool* active) {
   return CRL_OK;
 }
 
-// Does this call sum in two passes, or by the scan?  A larger table than 16,384 keys whose cells
-// have no room is scanned, also where they would have to be allocated now and the stream is
-// being captured, which allows no allocation.  (A smaller one is refused by ensure_handoff.)
+// Does this call sum in two passes, or by the scan?  The scan also takes what has no room for its
+// cells: in the static scratch tables of more than 16,384 keys and batches of millions (cells past
+// kNoAllocScanBytes; what is between is refused by ensure_handoff), and the larger tables where the
+// cells would have to be allocated now and the stream is being captured, which allows none.
 int choose_passes(const crl_engine* e, const crl::ReduceGeom& G, bool* two) {
+  const size_t bytes = handoff_records(G) * sizeof(unsigned long long);
+  const bool large = G.K > crl::kDenseKeys;
   *two = reduce_fast(G);
-  if (!*two || G.K <= crl::kDenseKeys) return CRL_OK;
-  bool recorded = false;
+  if (!*two) return CRL_OK;
   if (e->no_alloc) {
-    *two = handoff_fits(e, G);
-  } else if (handoff_records(G) > e->exchange.n) {
+    *two = handoff_fits(e, G) || (!large && bytes <= kNoAllocScanBytes);
+  } else if (large && handoff_records(G) > e->exchange.n) {
+    bool recorded;
     const int rc = query_capture(e, &recorded);
     if (rc) return rc;
     *two = !recorded;
@@ -928,7 +936,7 @@ int td_begin(crl_engine* e, int n, TdPlan* p) {
   if (h == hipSuccess) h = e->grow(e->delta, (size_t)n);
   if (h != hipSuccess) return fail(CRL_E_ALLOC, "scratch allocation failed: %s", hipGetErrorString(h));
   p->n = n;
-  p->G = reduce_geom(e, n);
+  p->G = reduce_geom_within(e, n, kHandoffLimitBytes);
   e->no_alloc = false;  // crl_update / crl_td_update: the engine's own hand-off buffer
   const int rc = choose_passes(e, p->G, &p->two);
   if (rc) return rc;
@@ -982,7 +990,7 @@ struct SharedPlan {
 };
 
 int plan_shared_step(const crl_engine* e, SharedPlan* p) {
-  p->G = e->no_alloc ? reduce_geom_within(e, e->N, kScratchExchangeBytes) : reduce_geom(e, e->N);
+  p->G = reduce_geom_within(e, e->N, e->no_alloc ? kScratchExchangeBytes : kHandoffLimitBytes);
   const int rc = choose_passes(e, p->G, &p->two);
   if (rc) return rc;
   // The shared table itself stays in L2: streaming its 64 KB into every workgroup's

@@ -224,8 +224,8 @@ int crl_run_fused(crl_engine* e, int32_t n_steps);
  * needs more hand-off cells than the array holds (65,536 envs on a 64x64x4 table need
  * 4 MB with two launches per step, 9.7 MB of exchange buffers in the one-launch kernel;
  * an engine whose one-launch buffers do not fit takes two launches per step); a larger
- * table whose cells do not fit is summed by a scan of all samples that needs none
- * and is slower.  All engines on one GPU share that GPU's array: calls that overlap in time on one GPU (different streams or threads)
+ * table, or a batch of millions, whose cells do not fit is summed by a scan of all
+ * samples that needs none and is slower.  All engines on one GPU share that GPU's array: calls that overlap in time on one GPU (different streams or threads)
  * race; calls in stream order do not. */
 int crl_run_fused_noalloc(crl_engine* e, int32_t n_steps);
 

@@ -51,6 +51,24 @@ def test_batches_of_several_pieces(gpu, oracle, n, W, H, A):
     check(gpu, oracle, W, H, A, [big, transitions(rng, W * H, A, 5000), transitions(rng, W * H, A, 700), big])
 
 
+@pytest.mark.parametrize("N,W,H,A", [((1 << 21) + 300, 8, 8, 4),   # 2.1 million samples
+                                     ((1 << 23) + 300, 16, 16, 4),  # 256 owners' cells outgrow their limit: 16 owners
+                                     (140000, 1024, 1024, 4)])      # 4096 owners
+def test_very_large_batches_take_two_passes(gpu, oracle, N, W, H, A):
+    cls, start = gpu.gen_maps_bernoulli(2, 1, N, W, H, 0.15)
+    cfg = gpu.make_config(N, W, H, n_actions=A, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=1e-6, eps0=0.3,
+                          episode_len=2, seed=6)
+    with gpu.Engine(cfg, 0) as eng:
+        eng.set_maps(cls, start)
+        assert eng.fused_kernel_info(3)["name"] == "k_shared_act+k_reduce_owners"
+        eng.run_fused(3)
+        q, st = eng.q_get(0), eng.get_state()
+    Q = np.zeros((1, W * H, A), np.float32)
+    ost = oracle.new_state(cfg, start)
+    oracle.run(cfg, cls, None, start, Q, ost, 0, 3)
+    assert np.array_equal(q, Q[0]) and np.array_equal(st["s"], ost["s"])
+
+
 def test_a_late_piece_that_is_refused_leaves_the_table_alone(gpu, oracle):
     W, H, A = 12, 10, 4
     S, n = W * H, 3 * PIECE

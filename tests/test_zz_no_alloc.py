@@ -79,11 +79,22 @@ def test_noalloc_rejects_a_reduction_larger_than_the_scratch(gpu):
         assert eng.step_count == 2
 
 
-@pytest.mark.parametrize("N,W,H,A", [(20000, 1024, 1024, 4), (65536, 512, 512, 4), (200000, 101, 99, 8)])
-def test_noalloc_shared_tables_whose_hand_off_cells_outgrow_the_scratch(gpu, N, W, H, A):
-    """More than 16,384 keys: the scan, which needs no cells, takes the step instead."""
+@pytest.mark.parametrize("W,H,A", [(3, 3, 4), (16, 16, 4), (16, 16, 8), (32, 32, 4)])
+def test_noalloc_small_shared_tables_with_as_many_owners_as_the_scratch_holds(gpu, W, H, A):
+    N = 200000  # 256 owners: 12.5 MB of cells
     cls, start = gpu.gen_maps_bernoulli(2, 1, N, W, H, 0.15)
-    cfg = gpu.make_config(N, W, H, n_actions=A, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=0.01,
+    cfg = gpu.make_config(N, W, H, n_actions=A, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=1e-5,
                           eps0=0.3, episode_len=3, seed=6)
     st, q = run_pair(gpu, cfg, cls, start, (3, 2), 1)
-    assert np.isfinite(q).all() and np.count_nonzero(q) > 1000 and st["episode"].min() >= 1
+    assert np.isfinite(q).all() and st["episode"].min() >= 1
+
+
+@pytest.mark.parametrize("N,W,H,A", [(20000, 1024, 1024, 4), (65536, 512, 512, 4), (200000, 101, 99, 8), (4300000, 16, 16, 4)])
+def test_noalloc_shared_tables_whose_hand_off_cells_outgrow_the_scratch(gpu, N, W, H, A):
+    """More than 16,384 keys, or millions of envs: the scan, which needs no cells, takes the step
+    instead."""
+    cls, start = gpu.gen_maps_bernoulli(2, 1, N, W, H, 0.15)
+    cfg = gpu.make_config(N, W, H, n_actions=A, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED,
+                          lr=0.01 if W > 16 else 1e-6, eps0=0.3, episode_len=3, seed=6)
+    st, q = run_pair(gpu, cfg, cls, start, (3, 2), 1)
+    assert np.isfinite(q).all() and np.count_nonzero(q) > min(1000, W * H * A // 2) and st["episode"].min() >= 1
