@@ -678,9 +678,18 @@ def test_td_update_slot_overflow_path(gpu, oracle):
     _td_case(gpu, oracle, W, H, A, s, a, r, s2, np.zeros(n, np.uint8))
 
 
-def test_td_update_large_table_scan_path(gpu, oracle):
-    """More than 16384 keys: the scanning fallback, same tree order."""
-    W, H, A, n = 80, 80, 8, 9000
+# more than 16,384 keys: the two passes with a hash of the block's keys; more than 4 million: the
+# scanning fallback, here over three groups of samples
+LARGE_TABLES = [(80, 80, 8, "k_shared_act+k_reduce_owners"), (1025, 1024, 4, "k_shared_act+k_reduce_scan")]
+
+
+@pytest.mark.parametrize("W,H,A,kernels", LARGE_TABLES)
+def test_td_update_large_table_scan_path(gpu, oracle, W, H, A, kernels):
+    """Same tree order either way."""
+    n = 9000
+    cfg = gpu.make_config(n, W, H, n_actions=A, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED)
+    with gpu.Engine(cfg, 0) as eng:  # (as many envs as samples: the same choice)
+        assert eng.fused_kernel_info(1)["name"] == kernels
     rng = np.random.default_rng(3)
     S = W * H
     hot = rng.integers(0, S, 30)  # few cells: long runs per key across blocks and groups
@@ -689,11 +698,15 @@ def test_td_update_large_table_scan_path(gpu, oracle):
     _td_case(gpu, oracle, W, H, A, s, a, r, s2, (rng.random(n) < 0.1).astype(np.uint8), mode=1)
 
 
-def test_shared_table_large_table_scan_path(gpu, oracle):
-    N, W, H = 6000, 72, 72  # 20736 keys > 16384
+@pytest.mark.parametrize("N,W,H,kernels", [(6000, 72, 72, LARGE_TABLES[0][3]), (6000, 1025, 1024, LARGE_TABLES[1][3])])
+def test_shared_table_large_table_scan_path(gpu, oracle, N, W, H, kernels):
     cls, start = gpu.gen_maps_bernoulli(8, 1, N, W, H, 0.15)
+    if W > 1000:  # crowded: a few thousand envs meet on some cells of the million
+        start = np.resize(start[:40], N).astype(np.int32)
     cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=0.01,
                           eps0=0.2, seed=2)
+    with gpu.Engine(cfg, 0) as eng:
+        assert eng.fused_kernel_info(40)["name"] == kernels
     run_both(gpu, oracle, cfg, cls, start, 40, trace_n=N)
 
 
