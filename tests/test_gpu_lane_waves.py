@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 STATE = ("s", "ep_step", "episode", "reward", "done", "action")
 
 
-def check(gpu, oracle, N, W, H, A, chunks, resident=0, variant=0, hybrid=False, cells=0, block=None, **kw):
+def check(gpu, oracle, N, W, H, A, chunks, resident=0, variant=0, hybrid=False, cells=0, block=None, kernel=None, **kw):
     cr = None
     if cells:
         cls, start, cr = gpu.gen_maps_noise(3, N, W, H, 4, 0.2, 0.3, 5.0)
@@ -25,7 +25,8 @@ def check(gpu, oracle, N, W, H, A, chunks, resident=0, variant=0, hybrid=False, 
         for c in chunks:
             plan = eng.fused_kernel_info(c)
             assert ("hbm+lds" in plan["name"]) == hybrid, plan
-            assert hybrid or plan["name"] == "k_fused_lanes<%d,fast%s>" % (A, ",cells" if cells else ""), plan
+            assert hybrid or kernel or plan["name"] == "k_fused_lanes<%d,fast%s>" % (A, ",cells" if cells else ""), plan
+            assert kernel is None or plan["name"] == kernel, plan
             assert block is None or plan["block"] == block, plan
             eng.run_fused(c)
             assert sum(eng.fused_split()) == N
@@ -62,3 +63,24 @@ def test_lane_waves(gpu, oracle, N, W, H, A, chunks, resident, kw):
                                                (1037, 20, 19, 4, 1), (521, 23, 21, 8, 1), (1, 16, 16, 4, 2), (7, 3, 3, 8, 3)])
 def test_hybrid_workgroups(gpu, oracle, N, W, H, A, lds_waves):
     check(gpu, oracle, N, W, H, A, (67, 130, 1), variant=2, hybrid=True, block=64 * (2 + lds_waves))
+
+
+# waves of 64 envs, which short calls of more envs than lane waves are for take, and longer calls on
+# tables past the caches, then with their move codes staged; the general loop's hybrid workgroups
+LINEAR = dict(eps_mode=3, eps0=0.9, eps_end=0.1, eps_span=4)
+
+
+@pytest.mark.parametrize("N,W,H,A,chunks,variant,kernel,kw", [
+    (17003, 13, 11, 4, (3, 1, 7), 0, "k_fused_tickets<4,fast,hbm>", dict()),
+    (17003, 13, 11, 8, (3, 1, 7), 0, "k_fused_tickets<8,fast,hbm>", dict()),
+    (17003, 13, 11, 4, (3, 1, 7), 0, "k_fused_tickets<4,fast+,hbm>", LINEAR),
+    (17003, 13, 11, 8, (3, 1, 7), 0, "k_fused_tickets<8,fast+,hbm>", dict(cells=3)),
+    (65601, 32, 31, 4, (130, 2), 0, "k_fused_tickets<4,fast,hbm>", dict()),
+    (70003, 16, 16, 8, (130, 2), 1, "k_fused_tickets<8,fast,hbm>", dict()),
+    (65601, 32, 31, 4, (130, 2), 0, "k_fused_tickets<4,fast+,hbm>", LINEAR),
+    (70003, 16, 16, 8, (130, 2), 0, "k_fused_tickets<8,fast+,hbm>", LINEAR),
+    (4099, 6, 5, 4, (67, 30), 2, "k_fused_tickets<4,general,hbm+lds>", dict(goal_mode=1)),
+    (4099, 6, 5, 8, (67, 30), 2, "k_fused_tickets<8,general,hbm+lds>", dict(goal_mode=1)),
+])
+def test_waves_of_64_envs(gpu, oracle, N, W, H, A, chunks, variant, kernel, kw):
+    check(gpu, oracle, N, W, H, A, chunks, variant=variant, hybrid="hbm+lds" in kernel, kernel=kernel, **kw)

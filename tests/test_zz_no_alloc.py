@@ -45,10 +45,11 @@ def run_pair(gpu, cfg, cls, start, chunks, n_tables, variant=0):
 
 def test_noalloc_per_env_tables_two_calls_second_smaller(gpu):
     big = None
-    for N, W, H, chunks in ((70000, 16, 16, (150, 37)), (3000, 12, 9, (90,))):  # hybrid and plain ticket kernels
+    # lane waves, tables in LDS, hybrid workgroups that draw their tickets
+    for N, W, H, chunks, variant in ((70000, 16, 16, (150, 37), 0), (3000, 12, 9, (90,), 0), (5000, 16, 16, (150, 37), 2)):
         cls, start = gpu.gen_maps_bernoulli(3, N, N, W, H, 0.1, 0.02)
         cfg = gpu.make_config(N, W, H, episode_len=64, gamma=0.95, eps0=0.15, seed=11)
-        st, q = run_pair(gpu, cfg, cls, start, chunks, N)
+        st, q = run_pair(gpu, cfg, cls, start, chunks, N, variant)
         assert np.count_nonzero(q) > N and st["episode"].min() >= 1
         big = big or N
     assert big == 70000
@@ -59,7 +60,7 @@ def test_noalloc_shared_table_two_calls_second_smaller(gpu):
         cls, start = gpu.gen_maps_bernoulli(2, 1, N, W, H, 0.15)
         cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=0.002,
                               eps0=0.2, episode_len=50, seed=13)
-        for variant in (0, 2):  # two launches per step; all steps in one launch (its flags, too, come from the scratch)
+        for variant in (0, 1, 2):  # all steps in one launch; two launches per step; one launch again, asked for
             st, q = run_pair(gpu, cfg, cls, start, (steps,), 1, variant)
             assert np.isfinite(q).all() and np.count_nonzero(q) > 100
 
