@@ -1017,15 +1017,12 @@ void launch_shared_act(crl_engine* e, const SharedPlan& p, uint64_t t, int trace
                        P, t, trace_row, e->key.p, e->delta.p, p.G, e->ho);
 }
 
-size_t persist_words(const crl_engine* e);
-
-// act (select + move + delta + block sums), then the key owners or the scan
-int shared_step(crl_engine* e, uint64_t t, int trace_row) {
+// act (select + move + delta + block sums), then the key owners or the scan; `words`: of the
+// exchange buffer, at least
+int shared_step(crl_engine* e, uint64_t t, int trace_row, size_t words) {
   SharedPlan p{};
   int rc = plan_shared_step(e, &p);
-  // (with room for the one-launch kernel where a longer call would run it: whichever runs first,
-  // no later call allocates, so that it can be recorded)
-  if (rc == CRL_OK && p.two) rc = ensure_handoff(e, p.G, persist_words(e));
+  if (rc == CRL_OK && p.two) rc = ensure_handoff(e, p.G, words);
   if (rc) return rc;
   if (e->A == 4) {
     if (p.lds_map) launch_shared_act<4, 1>(e, p, t, trace_row);
@@ -1834,8 +1831,13 @@ int run_fused(crl_engine* e, int32_t n_steps, bool no_alloc) {
     bool launched = false;
     rc = run_persist(e, n_steps, &launched);
     if (rc) return rc;
+    // A call of a few steps takes two launches to a step and a longer one the one-launch kernel:
+    // whichever comes first makes room for both, so that neither allocates later and both can be
+    // recorded.  (Not calls of one to three steps: the larger allocation costs a first call 20 us,
+    // 6 steps of 300 envs 66 / 85.)
+    const size_t words = n_steps > 3 ? persist_words(e) : 0;
     for (int k = 0; !launched && k < n_steps; ++k) {
-      rc = shared_step(e, e->t + (uint64_t)k, e->trace_cursor);
+      rc = shared_step(e, e->t + (uint64_t)k, e->trace_cursor, words);
       if (rc) return rc;
       if (e->trace_n > 0 && e->trace_cursor < e->trace_cap) e->trace_cursor += 1;
     }
