@@ -52,7 +52,7 @@ WORKLOADS = {
     # traffic: bytes per env-step past the L2, from rocprofv3 FETCH_SIZE x2.000 + WRITE_SIZE x1.000
     # in separate --pmc runs of the same launches (profiles/*.md), valid for the
     # workload's own launch length only (traffic_short: c4 at 20 steps per launch)
-    "c4": dict(n=1 << 20, launch_steps=1000, bytes=42.25, traffic=29.8, traffic_short={20: 58.1, 1: 335.0},
+    "c4": dict(n=1 << 20, launch_steps=1000, bytes=42.25, traffic=21.6, traffic_short={20: 58.1, 1: 335.0},
                name="c4: 1048576 envs 16x16, per-env tables 256x4 (4 GB), traps, eps 0.1, T=128, 1000 steps"),
     "c5": dict(n=8192, launch_steps=1024, bytes=70.0, traffic=87.1,
                name="c5: 8192 envs 256x256, 8 actions, per-env tables 65536x8 (16 GB), cell rewards, "

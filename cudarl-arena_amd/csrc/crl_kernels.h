@@ -1030,8 +1030,9 @@ __global__ __launch_bounds__(256) void k_fused_per_env(const Rules R, const Ptrs
 // The same with per-env maps: one wave to a workgroup, which draws 1 << log_envs envs at a
 // time from a ticket counter (or is dealt them by position: fixed_tickets), stages their move
 // codes into its LDS and steps them for all n_steps, A lanes to an env.  What bounds it is the
-// wave's dependent chain - 45 instructions and a trip to the row, 0.26 us per step alone on its
-// SIMD, of which a wave with 64 envs pays the slowest of 64 trips and 150 instructions.
+// wave's dependent chain - 50 vector instructions a step with four envs to a wave, 60 with 16 (by the
+// counters, tape and all), and a trip to the row, 0.28 us per step with a wave to a compute unit -
+// of which a wave with 64 envs pays the slowest of 64 trips and 150 instructions.
 // LDS: the rewards by class, the tape, the codes env by env.
 template <int A, bool CELLS>
 __global__ __launch_bounds__(64) void k_fused_lanes(const Rules R, const Ptrs P, const uint64_t t0, const int n_steps,
