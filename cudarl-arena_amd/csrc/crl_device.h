@@ -303,8 +303,8 @@ __device__ __forceinline__ void signal_host(const HostSignal h) {
   }
 }
 
-// First thing in the kernel: says that the launches before it in its stream are through, what
-// they read has been read.
+// Anywhere in the kernel: says that the launches before it in its stream are through, what they
+// read has been read.
 __device__ __forceinline__ void signal_reached(const HostSignal h) {
   if (h.flag && blockIdx.x == 0 && threadIdx.x == 0)
     __hip_atomic_store(h.flag, h.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);

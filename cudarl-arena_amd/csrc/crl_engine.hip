@@ -1191,10 +1191,9 @@ constexpr size_t kLinkLimitBytes = (size_t)4 << 20;  // larger transfers: hipMem
 constexpr size_t kInPageBytesOfFour = (size_t)128 << 10;  // larger pages are two
 // Transitions of a crl_td_update that go through one page.  Larger pieces cost more to pin, smaller
 // ones more launches (one page of their own for all / pieces of 65,536 / 131,072 / 262,144, us per
-// call among others: 262,144 82 / 97 / 84 / 83, 1 million 400 / 375 / 325 / 300, 2 million 935 / 1010 /
-// 880 / 780; alone: 262,144 157 / 126 / 127 / 155.  6 million in a page of their own 39,000, in pieces
-// of 131,072 3000).
-constexpr int kPieceSamples = 1 << 17;
+// call among others: 200,000 58.8 / - / 62.8 / 58.8, 1 million 400 / 375 / 325 / 300, 2 million 935 /
+// 1010 / 880 / 780; 6 million in a page of their own 39,000, in pieces 3000).
+constexpr int kPieceSamples = 1 << 18;
 constexpr int kFlagErrWord = 16;                     // of flag_page; in another 64-byte line than the flag
 
 // the next launch that tells the host when it is through

@@ -1482,7 +1482,6 @@ __global__ __launch_bounds__(256) void k_delta(const float* __restrict__ Q, cons
                                                 int32_t* __restrict__ key, float* __restrict__ delta,
                                                 const HostSignal before) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  signal_reached(before);
   int k;
   float d;
   sample_delta<A>(X, i, n, Q, lr, gamma, max_mode, k, d);
@@ -1490,6 +1489,7 @@ __global__ __launch_bounds__(256) void k_delta(const float* __restrict__ Q, cons
     key[i] = k;
     delta[i] = d;
   }
+  signal_reached(before);
 }
 
 // Shared table, first half of a fused step: every env selects, moves and emits

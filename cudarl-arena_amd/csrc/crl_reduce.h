@@ -477,7 +477,6 @@ __global__ __launch_bounds__(kBlockSamples) void k_td_blocks(const ReduceGeom G,
                                                              const HostSignal before) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int i = blockIdx.x * kBlockSamples + threadIdx.x;
-  signal_reached(before);
   int k;
   float d;
   block_lds_init(lds_raw, G);
@@ -486,6 +485,7 @@ __global__ __launch_bounds__(kBlockSamples) void k_td_blocks(const ReduceGeom G,
     key[i] = k;
     delta[i] = d;
   }
+  signal_reached(before);  // (not ahead of the samples: 262,144 of them 61.2 -> 60.6 us)
   __syncthreads();
   reduce_block_wide(lds_raw, G, blockIdx.x, k >= 0 ? k : 0, d, k >= 0, handoff);
 }

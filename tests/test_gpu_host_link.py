@@ -153,7 +153,7 @@ def test_pages_grow_while_earlier_calls_still_read_them(gpu, oracle):
     W, H, A = 30, 20, 4
     S = W * H
     rng = np.random.default_rng(2)
-    sizes = [1, 300, 900, 341, 342, 1025, 10922, 10923, 5, 40000, 3, 3, 3, 131072, 1500, 131073, 7, 200000, 64, 64, 64, 64, 64]
+    sizes = [1, 300, 900, 341, 342, 1025, 10922, 10923, 5, 40000, 3, 3, 3, 131072, 1500, 262144, 7, 262145, 64, 64, 64, 64, 64]
     want = rng.normal(0, 1, S * A).astype(np.float32)
     cfg = gpu.make_config(1, W, H, n_actions=A, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=1e-3)
     with gpu.Engine(cfg, 0) as eng:

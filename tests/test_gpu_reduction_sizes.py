@@ -37,7 +37,7 @@ def test_sample_counts(gpu, oracle, n, W, H, A):
     check(gpu, oracle, W, H, A, [transitions(rng, W * H, A, n) for _ in range(6)], mode=n & 1)
 
 
-PIECE = 1 << 17  # transitions of a call that go through one page
+PIECE = 1 << 18  # transitions of a call that go through one page
 
 
 @pytest.mark.parametrize("n", [PIECE - 1, PIECE, PIECE + 1, 2 * PIECE + 257, 5 * PIECE - 300])
