@@ -3,6 +3,7 @@
 // There is no CPU fallback anywhere in this file.
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <cstdarg>
 #include <cstdio>
 #include <algorithm>
@@ -816,22 +817,22 @@ int opt_in_lds(crl_engine* e) {
   HIP_TRY(allow_lds(crl::k_shared_act<4, 2, true>, act - kStaticLdsReserve));
   HIP_TRY(allow_lds(crl::k_shared_act<8, 1, true>, act - kStaticLdsReserve));
   HIP_TRY(allow_lds(crl::k_shared_act<8, 2, true>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<4, 1, false, false>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<4, 1, false, true>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<4, 2, false, false>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<4, 2, false, true>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<8, 1, false, false>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<8, 1, false, true>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<8, 2, false, false>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<8, 2, false, true>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<4, 1, true, false>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<4, 1, true, true>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<4, 2, true, false>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<4, 2, true, true>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<8, 1, true, false>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<8, 1, true, true>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<8, 2, true, false>, act - kStaticLdsReserve));
-  HIP_TRY(allow_lds(crl::k_shared_persist<8, 2, true, true>, act - kStaticLdsReserve));
+#define CRL_ALLOW_PERSIST(A, MAP)                                                                       \
+  do {                                                                                                  \
+    HIP_TRY(allow_lds(crl::k_shared_persist<A, MAP, false, false, false>, act - kStaticLdsReserve));    \
+    HIP_TRY(allow_lds(crl::k_shared_persist<A, MAP, false, true, false>, act - kStaticLdsReserve));     \
+    HIP_TRY(allow_lds(crl::k_shared_persist<A, MAP, true, false, false>, act - kStaticLdsReserve));     \
+    HIP_TRY(allow_lds(crl::k_shared_persist<A, MAP, true, true, false>, act - kStaticLdsReserve));      \
+    HIP_TRY(allow_lds(crl::k_shared_persist<A, MAP, false, false, true>, act - kStaticLdsReserve));     \
+    HIP_TRY(allow_lds(crl::k_shared_persist<A, MAP, false, true, true>, act - kStaticLdsReserve));      \
+    HIP_TRY(allow_lds(crl::k_shared_persist<A, MAP, true, false, true>, act - kStaticLdsReserve));      \
+    HIP_TRY(allow_lds(crl::k_shared_persist<A, MAP, true, true, true>, act - kStaticLdsReserve));       \
+  } while (0)
+  CRL_ALLOW_PERSIST(4, 1);
+  CRL_ALLOW_PERSIST(4, 2);
+  CRL_ALLOW_PERSIST(8, 1);
+  CRL_ALLOW_PERSIST(8, 2);
+#undef CRL_ALLOW_PERSIST
   e->lds_opt_in = true;
   return CRL_OK;
 }
@@ -1047,34 +1048,25 @@ struct PersistPlan {
   int grid;
   bool lds_map;
   bool fold;  // the instantiation with the common configuration's rules folded in
+  bool hashed;  // the form for more than 16,384 keys
   size_t lds;
   crl::ReduceGeom G;
   // what the workgroups exchange, in 64-bit words from the start of one buffer
   size_t at_table, at_raw, at_cells, words;
 };
 
-// Shortest call worth the set-up of the one-launch kernel (clearing what its workgroups
-// exchange, one co-resident launch: 28 us) instead of two plain launches per step, which cost
-// more the more envs there are.  Where the two cross (us per call, one launch / two, at 8, 12 and
-// 16 steps): 3000 envs of 16x16 75/58, 97/88, 119/118; 8000 of 32x32 77/61, 100/91, 123/122;
-// 12,000 of 64x64 78/66, 102/98, 125/131; 16,000 of 32x32 77/64, 100/95, 122/126; 24,000 of 64x64
-// 78/68, 102/102, 126/137; 32,768 of 64x64 82/71, 106/106, 130/141; 40,000 of 32x32 79/73, 103/109,
-// 126/145; 65,536 of 64x64 85/85, 113/127, 139/168.
-int persist_min_steps(int n_envs) {
-  return n_envs <= 8192 ? 16 : n_envs <= 16384 ? 14 : n_envs <= 32768 ? 12 : n_envs <= 49152 ? 10 : 9;
-}
-
-// The one-launch kernel needs every workgroup resident at once (one per compute
-// unit), the dense LDS table of the block pass and one tile of the owners' pass.
+// The one-launch kernel needs every workgroup resident at once (one per compute unit), and an
+// owner's keys in its LDS.
 bool persist_shape(const crl_engine* e, PersistPlan* p) {
   const int n_blocks = (e->N + crl::kBlockSamples - 1) / crl::kBlockSamples;
-  if (e->cfg.table_mode != CRL_TABLE_SHARED || e->K > (size_t)crl::kDenseKeys || n_blocks > crl::kPersistMaxGroups ||
-      crl::kPersistMaxGroups > kComputeUnits)
+  if (e->cfg.table_mode != CRL_TABLE_SHARED || n_blocks > crl::kPersistMaxGroups || crl::kPersistMaxGroups > kComputeUnits)
     return false;
   // always 256 workgroups, each a block (with or without envs) and an owner (with or
-  // without keys): 16,384 keys at most are 64 to an owner
+  // without keys): 16,384 keys at most are 64 to an owner, more up to 512 in the hashed form
   p->G = reduce_geom(e, e->N);
   p->G.own_shift = crl::kPersistOwnShift;
+  p->hashed = e->K > (size_t)crl::kDenseKeys;
+  if (p->hashed && own_keys(p->G) > crl::kOwnKeysHashed) return false;
   p->G.cell_shift = crl::cell_shift_for(p->G.own_shift);
   p->G.main_shift = crl::main_shift_for(p->G.own_shift);
   p->grid = crl::kPersistMaxGroups;
@@ -1088,6 +1080,26 @@ bool persist_shape(const crl_engine* e, PersistPlan* p) {
   return true;
 }
 
+// Shortest call worth the set-up of the one-launch kernel (clearing what its workgroups
+// exchange, one co-resident launch: 28 us) instead of two plain launches per step, which cost
+// more the more envs there are.  Where the two cross (us per call, one launch / two, at 8, 12 and
+// 16 steps): 3000 envs of 16x16 75/58, 97/88, 119/118; 8000 of 32x32 77/61, 100/91, 123/122;
+// 12,000 of 64x64 78/66, 102/98, 125/131; 16,000 of 32x32 77/64, 100/95, 122/126; 24,000 of 64x64
+// 78/68, 102/102, 126/137; 32,768 of 64x64 82/71, 106/106, 130/141; 40,000 of 32x32 79/73, 103/109,
+// 126/145; 65,536 of 64x64 85/85, 113/127, 139/168.
+// With more than 16,384 keys two launches cost 9 to 11 us a step with 4 actions and 13 to 15 with 8
+// (three rows of the neighbourhood instead of one are other lines), the hashed form 6.5 to 10; at 8
+// and 12 steps: 20,000 envs of 101x99, 8 actions 99/100, 133/151; 65,536 of 128x128, 8 actions
+// 121/121, 165/181; 3000 of 90x90 85/77, 112/117; 20,000 of 128x128 95/83, 126/124; 65,536 of
+// 128x128 109/100, 149/152.  Tables of up to 96 keys to an owner under few envs keep two launches,
+// the plan that has always been reported for them (6000 envs of 72x72, 40 steps: 307/401).
+int persist_min_steps(const crl_engine* e, const PersistPlan& p) {
+  const int n_envs = e->N;
+  if (p.hashed && n_envs <= 8192 && own_keys(p.G) <= 96) return INT_MAX;
+  if (p.hashed) return e->A == 8 ? 8 : 12;
+  return n_envs <= 8192 ? 16 : n_envs <= 16384 ? 14 : n_envs <= 32768 ? 12 : n_envs <= 49152 ? 10 : 9;
+}
+
 // 64-bit words that the one-launch kernel's workgroups exchange through; 0: it cannot run
 size_t persist_words(const crl_engine* e) {
   PersistPlan p{};
@@ -1097,20 +1109,20 @@ size_t persist_words(const crl_engine* e) {
 PersistPlan plan_persist(const crl_engine* e, int n_steps) {
   PersistPlan p{};
   if (e->fused_variant == 1 || e->persist_refused) return p;
-  if (e->fused_variant == 0 && n_steps < persist_min_steps(e->N)) return p;
-  if (!persist_shape(e, &p)) return p;
+  if (!persist_shape(e, &p) || (e->fused_variant == 0 && n_steps < persist_min_steps(e, p))) return p;
   const crl_config& c = e->cfg;
   p.fold = c.goal_mode == CRL_GOAL_ON_TARGET && c.auto_reset == 1 && c.max_mode == CRL_MAX_TRUE && c.reward_flags == 0 &&
            e->trace_n == 0 && e->sup_n == 0 && c.max_episodes == 0 && c.track_returns == 0;
   const size_t map_bytes = (size_t)e->map_words * 4;
-  p.lds_map = e->cfg.map_mode == CRL_MAP_SHARED && sizeof(crl::PersistLds) + map_bytes <= kLdsPerWorkgroup - kStaticLdsReserve;
-  p.lds = sizeof(crl::PersistLds) + (p.lds_map ? map_bytes : 0);
+  const size_t lds = p.hashed ? sizeof(crl::PersistLdsHashed) : sizeof(crl::PersistLds);
+  p.lds_map = e->cfg.map_mode == CRL_MAP_SHARED && lds + map_bytes <= kLdsPerWorkgroup - kStaticLdsReserve;
+  p.lds = lds + (p.lds_map ? map_bytes : 0);
   if (e->no_alloc && p.words * sizeof(unsigned long long) > kScratchExchangeBytes) return p;
   p.ok = true;
   return p;
 }
 
-template <int A, int MAP, bool CLK, bool FOLD>
+template <int A, int MAP, bool CLK, bool FOLD, bool HASHED>
 hipError_t launch_persist_kernel(crl_engine* e, const PersistPlan& p, unsigned long long* buf, uint64_t t0,
                                  int n_steps, int trace_row0) {
   crl::Rules R = e->rules();
@@ -1126,7 +1138,7 @@ hipError_t launch_persist_kernel(crl_engine* e, const PersistPlan& p, unsigned l
   void* args[] = {&R, &P, &t0, &n_steps, &trace_row0, &G, &B, &spin_limit};
   // a cooperative launch is refused unless all workgroups can be resident together,
   // which the kernel's waits rely on
-  return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&crl::k_shared_persist<A, MAP, CLK, FOLD>), dim3(p.grid),
+  return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&crl::k_shared_persist<A, MAP, CLK, FOLD, HASHED>), dim3(p.grid),
                                     dim3(256), args, (unsigned)p.lds, e->stream);
 }
 
@@ -1140,6 +1152,13 @@ int run_persist(crl_engine* e, int n_steps, bool* launched) {
   if (!p.ok) return CRL_OK;
   int rc;
   unsigned long long* buf;
+  if (p.hashed && !e->no_alloc && p.words > e->exchange.n) {
+    // (a stream being captured allows no allocation: two launches per step record such a call)
+    bool recorded;
+    rc = query_capture(e, &recorded);
+    if (rc) return rc;
+    if (recorded) return CRL_OK;
+  }
   if (e->no_alloc) {
     buf = reinterpret_cast<unsigned long long*>(e->static_scratch + kScratchTicketBytes);
   } else {
@@ -1153,21 +1172,23 @@ int run_persist(crl_engine* e, int n_steps, bool* launched) {
   // and a call longer than the tags allow goes out as several launches.
   int done = 0;
   while (done < n_steps) {
-    const int n = std::min(n_steps - done, crl::kPersistMaxSteps);
+    const int n = std::min(n_steps - done, p.hashed ? crl::kPersistMaxStepsHashed : crl::kPersistMaxSteps);
     const size_t w32 = p.words * 2;
     hipLaunchKernelGGL(crl::k_fill_u32, dim3((unsigned)((w32 + 255) / 256)), dim3(256), 0, e->stream,
                        reinterpret_cast<unsigned*>(buf), 0u, w32);
     const uint64_t t0 = e->t + (uint64_t)done;
     const int row0 = (int)std::min<long long>((long long)e->trace_cursor + done, e->trace_cap);
     hipError_t h;
-#define CRL_PERSIST(A, MAP) \
-  (e->persist_clocks ? (p.fold ? launch_persist_kernel<A, MAP, true, true>(e, p, buf, t0, n, row0)    \
-                               : launch_persist_kernel<A, MAP, true, false>(e, p, buf, t0, n, row0))  \
-                     : (p.fold ? launch_persist_kernel<A, MAP, false, true>(e, p, buf, t0, n, row0)   \
-                               : launch_persist_kernel<A, MAP, false, false>(e, p, buf, t0, n, row0)))
+#define CRL_PERSIST_FORM(A, MAP, HASHED)                                                                    \
+  (e->persist_clocks ? (p.fold ? launch_persist_kernel<A, MAP, true, true, HASHED>(e, p, buf, t0, n, row0)    \
+                               : launch_persist_kernel<A, MAP, true, false, HASHED>(e, p, buf, t0, n, row0))  \
+                     : (p.fold ? launch_persist_kernel<A, MAP, false, true, HASHED>(e, p, buf, t0, n, row0)   \
+                               : launch_persist_kernel<A, MAP, false, false, HASHED>(e, p, buf, t0, n, row0)))
+#define CRL_PERSIST(A, MAP) (p.hashed ? CRL_PERSIST_FORM(A, MAP, true) : CRL_PERSIST_FORM(A, MAP, false))
     if (e->A == 4) h = p.lds_map ? CRL_PERSIST(4, 1) : CRL_PERSIST(4, 2);
     else h = p.lds_map ? CRL_PERSIST(8, 1) : CRL_PERSIST(8, 2);
 #undef CRL_PERSIST
+#undef CRL_PERSIST_FORM
     if (h != hipSuccess) {
       (void)hipGetLastError();
       if (done > 0) return fail(CRL_E_DEVICE, "the one-launch shared-table kernel was refused after %d steps: %s", done, hipGetErrorString(h));
@@ -2291,7 +2312,8 @@ int crl_fused_kernel_info(crl_engine* e, int32_t n_steps, char* name, size_t nam
   } else {
     const PersistPlan pp = plan_persist(e, n_steps > 0 ? n_steps : 1 << 20);
     if (pp.ok) {
-      if (name && name_len) snprintf(name, name_len, "k_shared_persist<%d,%d%s>", e->A, pp.lds_map ? 1 : 2, pp.fold ? ",folded" : "");
+      if (name && name_len) snprintf(name, name_len, "k_shared_persist<%d,%d%s%s>", e->A, pp.lds_map ? 1 : 2,
+                                      pp.fold ? ",folded" : "", pp.hashed ? ",hashed" : "");
       if (grid) *grid = pp.grid;
       if (block) *block = 256;
       if (lds_bytes) *lds_bytes = (int32_t)pp.lds;

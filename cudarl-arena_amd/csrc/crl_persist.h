@@ -1,8 +1,8 @@
 // Shared table, all steps of a launch in ONE kernel: 256 workgroups, one per compute
 // unit, every one of them a block of the ordered reduction (256 envs, state in
 // registers for the whole launch; fewer envs: blocks without envs) and the owner of up
-// to 64 keys (whole table rows, values in registers), and the two roles hand their
-// data to each other through memory.  Always 256 owners, also where the table would
+// to 64 keys, or in the hashed form 512 (whole table rows, values in registers), and the two
+// roles hand their data to each other through memory.  Always 256 owners, also where the table would
 // fit fewer: an owner's 256 cells are then small ones, every workgroup has a part in
 // both passes, and a table of few cells that many envs crowd on is spread as far as
 // it goes (65,536 envs on a 16x16x4 table: 7.2 us per step with 256 owners of one row
@@ -34,6 +34,10 @@
 //           quarter of the tile -> poll the cells of its blocks -> into the tile -> its
 //           four group sums; one barrier; totals in group order -> new values and row
 //           maxima into the views
+// What bounds a step is the chain of the two exchanges between all compute units and the work
+// between them.  20,000 envs on 101x99x8 (hashed form, phase clocks of a workgroup with envs):
+// views 1.8 us, select and hash 0.5, block sums 1.0, cells and records 2.4, totals 0.8; 200 steps
+// 2655 us with two launches per step, 1713 with this kernel.
 // An owner overwrites its values only after it has every block's cells of the step,
 // which a block writes after all its threads have read theirs: one buffer of views
 // suffices.  Cells and raw samples have two buffers, taken in turn: a workgroup that
@@ -59,10 +63,13 @@ constexpr int kMainShift = 2, kMainRecs = 1 << kMainShift;  // records in the ha
 static_assert(main_shift_for(kPersistOwnShift) == kMainShift && cell_shift_for(kPersistOwnShift) == kMainShift + 1 &&
               (1 << kPersistOwnShift) == kPersistMaxGroups && (kPersistMaxGroups << (kMainShift - 1)) == kStagePieces,
               "the owner's loads are laid out for cells of 4 + 4 records");
-constexpr int kPersistMaxSteps = 65535;     // per launch: the raw samples' tags have 17 bits
+constexpr int kPersistMaxSteps = 65535;     // per launch, dense form: the raw samples' tags have 17 bits
+constexpr int kPersistMaxStepsHashed = 16381;  // ... hashed form: 14 bits
 constexpr int kPersistClockWords = 20 + 8 * 256;  // 2 workgroups x (8 phases + polls of the two waits by thread 0),
                                                   // then the wall clock of every workgroup at the 8 marks of one step
 
+// Dense form, up to 16,384 keys: an entry per key of the table in the block pass, a dense
+// [block][key] tile in the owner's.
 struct alignas(16) PersistLds {
   ReduceLds red;
   alignas(16) float tile[kTileBlocks * kOwnKeys];       // the owner's [block][key] block sums: a quarter (64 blocks) to a wave, which
@@ -75,6 +82,27 @@ struct alignas(16) PersistLds {
   int o_count;
   int dead;  // some thread gave up waiting (never cleared)
 };
+
+// Hashed form, up to 131,072 keys: the keys a block holds are found in a hash of 2048 entries
+// (as with two launches), and the owner's tile has a column not per key but per distinct key
+// that its records name.
+constexpr int kGroups = kTileBlocks / kGroupBlocks;
+constexpr int kMaxColumns = 2 * kMainRecs * kGroupBlocks;  // a group's records at most
+struct alignas(16) PersistLdsHashed {
+  ReduceLdsT<kHashSlots> red;
+  int keys[kHashSlots];                                 // -1 between uses
+  alignas(16) float tile[kTileBlocks * kOwnKeys];       // [block][column], a quarter to a wave; see add_records
+  alignas(16) unsigned long long stage[kPersistMaxGroups << kMainShift];
+  alignas(16) uint32_t sum[kGroups][kOwnKeysHashed];    // a key's group sum, on the way there its column; kNoLead: none
+  alignas(16) float gsum[kGroups][kMaxColumns];
+  float list_v[4][kBlockSamples];                       // a wave's list of one overflowing block's samples
+  uint16_t list_s[4][kBlockSamples];
+  alignas(16) int by_key[4];  // the wave's group sums lie in its tile, [group][key]
+  int o_count;
+  int dead;
+};
+template <bool HASHED>
+using PersistLdsOf = std::conditional_t<HASHED, PersistLdsHashed, PersistLds>;
 
 struct PersistBufs {
   unsigned long long* table;   // view [S][2 A]
@@ -90,12 +118,18 @@ __device__ __forceinline__ unsigned long long tagged(uint32_t bits, uint32_t tag
 __device__ __forceinline__ uint32_t tag_of(unsigned long long v) { return (uint32_t)(v >> 32); }
 __device__ __forceinline__ float value_of(unsigned long long v) { return __uint_as_float((uint32_t)v); }
 
-// raw sample: delta in the low word; key, valid bit and a 17-bit tag in the high word
-constexpr uint32_t kRawKeyMask = 0x3FFFu, kRawValid = 0x4000u;
-constexpr int kRawTagShift = 15;
-static_assert(kDenseKeys - 1 <= (int)kRawKeyMask, "raw samples hold 14-bit keys");
-static_assert(kPersistMaxSteps + 1 < (1 << (32 - kRawTagShift)), "raw tags must be unique within a launch");
-static_assert((uint32_t)kPersistMaxSteps + 1u <= kRecTagMask, "record tags must be unique within a launch");
+// raw sample: delta in the low word; key, valid bit and a tag (17 / 14 bits) in the high word
+template <bool HASHED>
+struct Raw {
+  static constexpr uint32_t kValid = HASHED ? 1u << 17 : 1u << 14, kKeyMask = kValid - 1u;
+  static constexpr int kTagShift = HASHED ? 18 : 15;
+};
+static_assert(kDenseKeys - 1 <= (int)Raw<false>::kKeyMask && kOwnKeysHashed * kPersistMaxGroups - 1 <= (int)Raw<true>::kKeyMask,
+              "raw samples hold a key");
+static_assert(kPersistMaxSteps + 1 < (1 << (32 - Raw<false>::kTagShift)) &&
+              kPersistMaxStepsHashed + 1 < (1 << (32 - Raw<true>::kTagShift)), "raw tags must be unique within a launch");
+static_assert((uint32_t)kPersistMaxSteps + 1u <= Rec<false>::kTagMask &&
+              (uint32_t)kPersistMaxStepsHashed + 1u <= Rec<true>::kTagMask, "record tags must be unique within a launch");
 
 template <int A>
 __device__ __forceinline__ Row<A> row_of_tagged(const unsigned long long (&v)[A]);
@@ -124,6 +158,165 @@ __device__ __forceinline__ Row<8> row_of_tagged<8>(const unsigned long long (&v)
     }                                                                                       \
   } while (0)
 
+// a wave's quarter of an owner's tile
+__device__ __forceinline__ void clear_tile(float* tile, const int lane) {
+  float4* tile4 = reinterpret_cast<float4*>(tile);
+#pragma unroll
+  for (int i = 0; i < kTileBlocks * kOwnKeys / 4 / 256; ++i) tile4[i * 64 + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+}
+
+// Hashed form, owner: the sums of a wave's four groups from the records of its 64 blocks.  Two
+// lanes to a cell: rec[j] is this lane's piece of the main half of block wave * 64 + j * 32 +
+// lane / 2, more[j] of its extension, cnt[j] what its record 0 says.
+// Every record enters its number in the group - its block first - with a minimum under its key:
+// the number of the key's first record is the key's column in the wave's part of the tile, which
+// comes in cleared, and from there it is the dense form's pass: values to [block][column], then
+// the columns added up, whatever the number of blocks that hold a key.  (All that are left
+// entering with a minimum, the lowest of each key adding its value and being done, took as many
+// rounds as the most crowded key of a group has blocks: 4 us in the owner of a key that all hold.)
+// -> false: gave up waiting for raw samples.
+__device__ __forceinline__ bool add_records(PersistLdsHashed& L, const ReduceGeom G, const int n_envs,
+                                            const unsigned long long* raw, const unsigned* err, const uint32_t want,
+                                            const int spin_limit, const uint4 (&rec)[2], const uint4 (&more)[2],
+                                            const int (&cnt)[2]) {
+  using R64 = Rec<true>;
+  constexpr int kTile = kTileBlocks * kOwnKeys / 4;  // words of a wave's part
+  const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6), pair = lane & 1;
+  float* const tile = L.tile + wave * kTile;
+  if (lane == 0) L.by_key[wave] = 0;
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(cnt[0] == kSlotOverflow || cnt[1] == kSlotOverflow) != 0ull, 0)) {
+    // (rare) block after block into sums by key; one with more distinct keys for this owner than
+    // a cell holds again from its raw samples, the first holder of a key adding up all of them
+    // in order
+    static_assert(kOwnKeysHashed <= kTile / 4, "the sums of four groups by key");
+    if (lane == 0) L.by_key[wave] = 1;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      for (int bb = 0; bb < 32; ++bb) {
+        float* sums = tile + (j * 2 + bb / kGroupBlocks) * (kTile / 4);
+        if (__builtin_amdgcn_readlane(cnt[j], 2 * bb) != kSlotOverflow) {
+          if ((lane >> 1) == bb) {
+            auto add = [&](int r, uint32_t meta, uint32_t bits) {
+              if (r < cnt[j]) sums[R64::slot(meta)] = sums[R64::slot(meta)] + __uint_as_float(bits);
+            };
+            add(2 * pair, rec[j].x, rec[j].y);
+            add(2 * pair + 1, rec[j].z, rec[j].w);
+            add(kMainRecs + 2 * pair, more[j].x, more[j].y);
+            add(kMainRecs + 2 * pair + 1, more[j].z, more[j].w);
+          }
+          wave_fence();
+          continue;
+        }
+        int m = 0;
+        for (int q = 0; q < kBlockSamples; q += 64) {
+          const int i = (wave * 64 + j * 32 + bb) * kBlockSamples + q + lane;
+          unsigned long long v = 0ull;
+          bool ok = i >= n_envs;
+          for (int spins = 0; !ok && spins < spin_limit; ++spins) {
+            poll_fence();
+            v = ld_dev64(raw + i);
+            ok = (tag_of(v) >> Raw<true>::kTagShift) == want;
+            if (!ok && (spins & 63) == 63 && ld_dev32(err) != 0u) break;
+          }
+          if (!__all(ok)) return false;
+          const int k = (int)(tag_of(v) & Raw<true>::kKeyMask);
+          const bool mine = i < n_envs && (tag_of(v) & Raw<true>::kValid) != 0u && owner_of(k, G) == (int)blockIdx.x;
+          const unsigned long long who = __builtin_amdgcn_ballot_w64(mine);
+          if (mine) {
+            const int at = m + __popcll(who & ((1ull << lane) - 1ull));
+            L.list_s[wave][at] = (uint16_t)slot_of(k, G);
+            L.list_v[wave][at] = value_of(v);
+          }
+          m += __popcll(who);
+        }
+        wave_fence();
+        for (int e = lane; e < m; e += 64) {
+          const int slot = L.list_s[wave][e];
+          bool first = true;
+          for (int f = 0; f < e; ++f) first = first && L.list_s[wave][f] != slot;
+          if (first) {
+            float acc = 0.0f;
+            for (int f = e; f < m; ++f)
+              if (L.list_s[wave][f] == slot) acc = acc + L.list_v[wave][f];
+            sums[slot] = sums[slot] + acc;
+          }
+        }
+        wave_fence();
+      }
+    }
+    return true;
+  }
+  const uint32_t b = (uint32_t)(lane >> 1) & (kGroupBlocks - 1);  // the block in its group
+  // kJ = 2: both j, four groups of 64 columns; kJ = 1: one j, two groups of 128
+  auto pass = [&](auto n_j, auto n_recs, const int j0) {
+    constexpr int kJ = decltype(n_j)::value, kRecs = decltype(n_recs)::value;
+    constexpr int kColumns = kRecs * kGroupBlocks, kMine = kJ * kRecs / 2;  // records of a lane
+    static_assert(kJ * 32 * kColumns <= kTile && kJ * 2 * kColumns == 256, "one pass: the wave's tile, four columns to a lane");
+    bool has[kMine];
+    uint32_t* col[kMine];
+    uint32_t number[kMine];
+    float v[kMine];
+#pragma unroll
+    for (int c = 0; c < kMine; ++c) {
+      const int j = kJ == 2 ? c & 1 : j0, r = kJ == 2 ? c >> 1 : c;  // (r: 0, 1 of the main half, 2, 3 of the extension)
+      const uint4 m0 = j == 0 ? rec[0] : rec[1], m1 = j == 0 ? more[0] : more[1];
+      const uint4 from = r < 2 ? m0 : m1;
+      const int n = j == 0 ? cnt[0] : cnt[1], record = (r < 2 ? 0 : kMainRecs) + 2 * pair + (r & 1);
+      has[c] = record < n;
+      col[c] = &L.sum[wave * 4 + j * 2 + (lane >> 5)][R64::slot((r & 1) ? from.z : from.x)];
+      v[c] = __uint_as_float((r & 1) ? from.w : from.y);
+      number[c] = b * kRecs + (uint32_t)record;
+      if (has[c]) atomicMin(col[c], number[c]);
+    }
+    wave_fence();
+    uint32_t at[kMine];
+#pragma unroll
+    for (int c = 0; c < kMine; ++c) at[c] = *col[c];
+    wave_fence();
+#pragma unroll
+    for (int c = 0; c < kMine; ++c)
+      if (has[c]) tile[((kJ == 2 ? (c & 1) * 32 : 0) + (lane >> 1)) * kColumns + (int)at[c]] = v[c];
+    wave_fence();
+    constexpr int kLanes = kColumns / 4;  // of a group, four columns to a lane
+    const int grp = lane / kLanes;
+    const float4* rows = reinterpret_cast<const float4*>(tile + grp * kGroupBlocks * kColumns) + lane % kLanes;
+    float4 x[kGroupBlocks];
+#pragma unroll
+    for (int i = 0; i < kGroupBlocks; ++i) x[i] = rows[i * kLanes];
+    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int i = 0; i < kGroupBlocks; ++i) {
+      acc.x = acc.x + x[i].x;
+      acc.y = acc.y + x[i].y;
+      acc.z = acc.z + x[i].z;
+      acc.w = acc.w + x[i].w;
+    }
+    reinterpret_cast<float4*>(L.gsum[wave * 4 + j0 * 2 + grp])[lane % kLanes] = acc;
+    wave_fence();
+    float total[kMine];
+#pragma unroll
+    for (int c = 0; c < kMine; ++c)
+      total[c] = L.gsum[wave * 4 + (kJ == 2 ? (c & 1) * 2 : j0 * 2) + (lane >> 5)][number[c] & (kColumns - 1)];
+#pragma unroll
+    for (int c = 0; c < kMine; ++c) {
+      const uint32_t bits = __float_as_uint(total[c]);
+      if (has[c] && at[c] == number[c]) *col[c] = bits == kNoLead ? 0x7fc00000u : bits;  // (all ones are no number either)
+    }
+  };
+  if (__builtin_amdgcn_ballot_w64(cnt[0] > kMainRecs || cnt[1] > kMainRecs) == 0ull) {
+    pass(std::integral_constant<int, 2>{}, std::integral_constant<int, kMainRecs>{}, 0);
+  } else {  // (few cells have more than the four records of a main half) two groups at a time, with room for eight
+    for (int j = 0; j < 2; ++j) {
+      if (j == 1) {
+        wave_fence();
+        clear_tile(tile, lane);
+      }
+      pass(std::integral_constant<int, 1>{}, std::integral_constant<int, 2 * kMainRecs>{}, j);
+    }
+  }
+  return true;
+}
+
 // MAP = 1: the shared map staged in LDS; MAP = 2: maps read from global memory
 // (they do not change during a launch, so plain loads are fine).
 // G.own_shift = kPersistOwnShift, G.n_blocks = 256 = the number of workgroups (blocks
@@ -134,16 +327,18 @@ __device__ __forceinline__ Row<8> row_of_tagged<8>(const unsigned long long (&v)
 // no supplied stream, no episode budget, no return statistics): the general kernel keeps
 // a dozen lane masks and pointers for them that do not fit the scalar registers and are
 // fetched back again and again (190 lane reads per step).
-template <int A, int MAP, bool CLK, bool FOLD>
+template <int A, int MAP, bool CLK, bool FOLD, bool HASHED>
 __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptrs P, const uint64_t t0,
                                                          const int n_steps, const int trace_row0,
                                                          const ReduceGeom G, const PersistBufs B,
                                                          const int spin_limit) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  PersistLds& L = *reinterpret_cast<PersistLds*>(lds_raw);
-  static_assert(sizeof(PersistLds) % 16 == 0 && offsetof(PersistLds, tile) % 16 == 0, "16-byte LDS accesses");
-  static_assert(kSortBytes <= sizeof(L.tile) / 2, "the holders' line-up borrows the upper half of the tile");
-  uint32_t* lds_map = reinterpret_cast<uint32_t*>(lds_raw + sizeof(PersistLds));
+  using Lds = PersistLdsOf<HASHED>;
+  using R64 = Rec<HASHED>;
+  Lds& L = *reinterpret_cast<Lds*>(lds_raw);
+  static_assert(sizeof(Lds) % 16 == 0, "16-byte LDS accesses");
+  static_assert(kSortBytes <= sizeof(PersistLds::tile) / 2, "the holders' line-up borrows the upper half of the tile");
+  uint32_t* lds_map = reinterpret_cast<uint32_t*>(lds_raw + sizeof(Lds));
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -162,6 +357,10 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
   if (tid == 0) {
     L.o_count = 0;
     L.dead = 0;
+  }
+  if constexpr (HASHED) {
+    for (int i = tid; i < kHashSlots; i += 256) L.keys[i] = -1;
+    for (int i = tid; i < kGroups * kOwnKeysHashed; i += 256) (&L.sum[0][0])[i] = kNoLead;
   }
   if (MAP == 1)
     for (int i = tid; i < P.map_words; i += 256) lds_map[i] = P.map[i];
@@ -183,47 +382,60 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
   const bool cells_flag = !FOLD && (R.reward_flags & 1) != 0;
   const bool base_cells = cells_flag && (R.reward_flags & 2) != 0;
 
-  // owner: lane l of wave 0 keeps the table value of its key in a register; the A lanes
-  // of a row sit side by side, each of them publishes its value and one copy of the row's
-  // maximum
-  const int own_key = key_of(wg, lane, G);
-  const bool own_live = wave == 0 && own_key < G.K;
-  float q_own = own_live ? P.Q[own_key] : 0.0f;
+  // owner: a lane keeps the table value of its key (dense form: lane l of wave 0, key l) or of
+  // its two (hashed: thread t, keys t and t + 256) in registers; the A lanes of a row sit side
+  // by side, each of them publishes its value and one copy of the row's maximum
+  constexpr int kOwn = HASHED ? kOwnKeysHashed / 256 : 1;
+  const bool owns = HASHED || wave == 0;
+  const bool more_keys = HASHED && key_of(wg, 256 + (wave << 6), G) < G.K;  // this wave's second half: any at all
   // where the lane of action a publishes: its value in the view of its cell, and the row's
   // maximum in the view of the cell that reaches this one by action a (and in its own
   // cell's view if action a would leave the grid there)
-  int pub_q = -1, pub_from = -1, pub_self = -1;
-  if (own_live) {
-    const int c = own_key >> G.a_shift, a = own_key & (A - 1);
-    const int x = c % R.W, y = c / R.W;
-    int dx, dy;
-    action_delta(a, A, dx, dy);
-    pub_q = c * 2 * A + a;
-    if ((unsigned)(x - dx) < (unsigned)R.W && (unsigned)(y - dy) < (unsigned)R.H) pub_from = (c - dy * R.W - dx) * 2 * A + A + a;
-    if (!((unsigned)(x + dx) < (unsigned)R.W && (unsigned)(y + dy) < (unsigned)R.H)) pub_self = c * 2 * A + A + a;
-  }
-  auto publish = [&](uint32_t tag) {  // wave 0 of an owner
-    if (own_live) st_dev64(B.table + pub_q, tagged(__float_as_uint(q_own), tag));
-    float qs[A];
-    if constexpr (A == 4) {  // the four lanes of a row are a quad: a move within it, no trip through LDS
-      qs[0] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(q_own), 0x00, 0xf, 0xf, true));
-      qs[1] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(q_own), 0x55, 0xf, 0xf, true));
-      qs[2] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(q_own), 0xaa, 0xf, 0xf, true));
-      qs[3] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(q_own), 0xff, 0xf, 0xf, true));
-    } else {
+  int own_key[kOwn], pub_q[kOwn], pub_from[kOwn], pub_self[kOwn];
+  float q_own[kOwn];
 #pragma unroll
-      for (int i = 0; i < A; ++i) qs[i] = __shfl(q_own, (lane & ~(A - 1)) + i);
+  for (int o = 0; o < kOwn; ++o) {
+    const int slot = HASHED ? o * 256 + tid : lane;
+    own_key[o] = owns ? key_of(wg, slot, G) : G.K;
+    q_own[o] = own_key[o] < G.K ? P.Q[own_key[o]] : 0.0f;
+    pub_q[o] = pub_from[o] = pub_self[o] = -1;
+    if (own_key[o] < G.K) {
+      const int c = own_key[o] >> G.a_shift, a = own_key[o] & (A - 1);
+      const int x = c % R.W, y = c / R.W;
+      int dx, dy;
+      action_delta(a, A, dx, dy);
+      pub_q[o] = c * 2 * A + a;
+      if ((unsigned)(x - dx) < (unsigned)R.W && (unsigned)(y - dy) < (unsigned)R.H) pub_from[o] = (c - dy * R.W - dx) * 2 * A + A + a;
+      if (!((unsigned)(x + dx) < (unsigned)R.W && (unsigned)(y + dy) < (unsigned)R.H)) pub_self[o] = c * 2 * A + A + a;
     }
-    if (own_live) {
-      Row<A> row;
-      if constexpr (A == 4) row = Row<4>{qs[0], qs[1], qs[2], qs[3]};
-      else row = Row<8>{qs[0], qs[1], qs[2], qs[3], qs[4], qs[5], qs[6], qs[7]};
-      const unsigned long long mx = tagged(__float_as_uint(row_max(row, false, 0)), tag);
-      if (pub_from >= 0) st_dev64(B.table + pub_from, mx);
-      if (pub_self >= 0) st_dev64(B.table + pub_self, mx);
+  }
+  auto publish = [&](uint32_t tag) {  // the waves that own keys
+#pragma unroll
+    for (int o = 0; o < kOwn; ++o)
+      if (own_key[o] < G.K) st_dev64(B.table + pub_q[o], tagged(__float_as_uint(q_own[o]), tag));
+#pragma unroll
+    for (int o = 0; o < kOwn; ++o) {
+      float qs[A];
+      if constexpr (A == 4) {  // the four lanes of a row are a quad: a move within it, no trip through LDS
+        qs[0] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(q_own[o]), 0x00, 0xf, 0xf, true));
+        qs[1] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(q_own[o]), 0x55, 0xf, 0xf, true));
+        qs[2] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(q_own[o]), 0xaa, 0xf, 0xf, true));
+        qs[3] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(q_own[o]), 0xff, 0xf, 0xf, true));
+      } else {
+#pragma unroll
+        for (int i = 0; i < A; ++i) qs[i] = __shfl(q_own[o], (lane & ~(A - 1)) + i);
+      }
+      if (own_key[o] < G.K) {
+        Row<A> row;
+        if constexpr (A == 4) row = Row<4>{qs[0], qs[1], qs[2], qs[3]};
+        else row = Row<8>{qs[0], qs[1], qs[2], qs[3], qs[4], qs[5], qs[6], qs[7]};
+        const unsigned long long mx = tagged(__float_as_uint(row_max(row, false, 0)), tag);
+        if (pub_from[o] >= 0) st_dev64(B.table + pub_from[o], mx);
+        if (pub_self[o] >= 0) st_dev64(B.table + pub_self[o], mx);
+      }
     }
   };
-  if (wave == 0) publish(1u);
+  if (owns) publish(1u);
   __syncthreads();
 
   // What a step needs that does not depend on the table: computed at the top of the step,
@@ -264,6 +476,7 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
     }
   };
 
+  const int live_groups = (P.N + kBlockSamples * kGroupBlocks - 1) / (kBlockSamples * kGroupBlocks);
   unsigned long long phase_[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   unsigned long long last_ = CLK ? clock64() : 0ull;
   bool gave_up = false;
@@ -272,7 +485,7 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
     CRL_MARK(7);
     // (the values this workgroup published as an owner are on their way meanwhile)
     prepare(k);
-    reduce_stage_init(L.stage, G, want);
+    reduce_stage_init<HASHED>(L.stage, G, want);
     // (The values published at the end of the last step need about 1 us to be visible, which
     // is what the preparation above takes.  A look that comes too early costs a whole round
     // trip more; while a step was longer than now, a pause of 0.1-0.2 us here and before the
@@ -320,7 +533,7 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
     CRL_MARK(1);
 
     // ---- select, move, (key, delta) ---------------------------------------------------
-    int my_key = 0;
+    int my_key = 0, my_at = 0;
     float my_delta = 0.0f;
     if (live) {
       const Row<A> row = row_of_tagged<A>(rq);
@@ -328,7 +541,14 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
       const int a = (d.u < eps) ? d.a : greedy;
       // (the key is known: its leader is being found while the delta is worked out)
       my_key = s0 * A + a;
-      atomicMin(&L.red.lead[my_key], (uint32_t)tid);
+      int found = -1;
+      if constexpr (HASHED) {
+        my_at = hash_start(kHashSlots - 1, my_key);
+        found = atomicCAS(&L.keys[my_at], -1, my_key);
+      } else {
+        my_at = my_key;
+        atomicMin(&L.red.lead[my_at], (uint32_t)tid);
+      }
       // the rule of step_rule() on the move code of the action: the class of the target
       // cell, or kWall outside the grid
       const int code = (int)((mv >> (2 * a)) & 3u);
@@ -352,6 +572,10 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
       if (!FOLD && R.max_mode == 1) m = fmaxf(0.0f, m);
       m = done ? 0.0f : m;
       my_delta = td_delta(row_get(row, a), reward, m, R.lr, R.gamma);
+      if constexpr (HASHED) {
+        my_at = hash_finish(L.keys, kHashSlots - 1, my_key, my_at, found);
+        atomicMin(&L.red.lead[my_at], (uint32_t)tid);
+      }
       action = a;
       if (!FOLD && env < P.trace_n && trace_row0 + k < P.trace_cap) {
         const size_t o = (size_t)(trace_row0 + k) * P.trace_n + env;
@@ -374,18 +598,20 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
     // ---- block sums to the owners' cells ------------------------------------------------
     const int half = k & 1;  // cells and raw samples: two buffers, taken in turn
     // (`sorted`: the upper half of the tile, which is free until the block sums are through)
-    const bool over = reduce_block(L.red, G, wg, my_key, my_delta, live, want, L.tile + kTileBlocks * kOwnKeys / 2, L.stage,
-                                   w_cells, (uint32_t)((size_t)half * cells_half * 8), B.cells + (2 + half) * cells_half);
+    int* keys = nullptr;
+    if constexpr (HASHED) keys = L.keys;
+    const bool over = reduce_block<HASHED>(L.red, G, wg, my_key, my_at, keys, my_delta, live, want,
+                                           L.tile + kTileBlocks * kOwnKeys / 2, L.stage, w_cells, (uint32_t)((size_t)half * cells_half * 8), B.cells + (2 + half) * cells_half);
     if (over && has_env)
       st_dev64(B.raw + (size_t)half * P.N + env, tagged(__float_as_uint(my_delta),
-                                   (uint32_t)my_key | (live ? kRawValid : 0u) | (want << kRawTagShift)));
+                                   (uint32_t)my_key | (live ? Raw<HASHED>::kValid : 0u) | (want << Raw<HASHED>::kTagShift)));
     CRL_MARK(3);
 
     // ---- while the cells travel: the owner's tile cleared -------------------------------
-    {  // (each wave its own quarter)
-      float4* tile4 = reinterpret_cast<float4*>(L.tile) + wave * (kTileBlocks * kOwnKeys / 4 / 4);
-#pragma unroll
-      for (int i = 0; i < kTileBlocks * kOwnKeys / 4 / 256; ++i) tile4[i * 64 + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    clear_tile(L.tile + wave * (kTileBlocks * kOwnKeys / 4), lane);  // (each wave its own quarter)
+    if constexpr (HASHED) {
+      uint4* sums4 = reinterpret_cast<uint4*>(L.sum[wave * 4]);
+      for (int i = lane; i < 4 * kOwnKeysHashed / 4; i += 64) sums4[i] = make_uint4(kNoLead, kNoLead, kNoLead, kNoLead);
     }
     // (no waiting for the own cells' acknowledgement before the first look at the others':
     // that costs 0.3 us per step; clearing the tile first is pause enough)
@@ -395,7 +621,7 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
     }
     CRL_MARK(4);
 
-    // ---- as owner of 64 keys: all blocks' cells, added in tree order --------------------
+    // ---- as owner: all blocks' cells, added in tree order --------------------------------
     {
       // A wave takes 64 blocks' cells.  A main half is two pieces of 16 bytes = two records
       // each: two lanes read it side by side, so a load of the wave is 32 whole halves, and
@@ -425,12 +651,12 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
           for (int j = 0; j < GS; ++j) {
             // (record 0 of the cell is in the even lane of the two: a move within the quad)
             const uint32_t meta0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)rec[j].x, 0xa0, 0xf, 0xf, true);
-            cnt[j] = rec_count(meta0);
+            cnt[j] = R64::count(meta0);
             // (every record of a main half is written every step)
-            bool mine = rec_tag(meta0) == want && rec_tag(rec[j].x) == want && rec_tag(rec[j].z) == want;
+            bool mine = R64::tag(meta0) == want && R64::tag(rec[j].x) == want && R64::tag(rec[j].z) == want;
             if (cnt[j] != kSlotOverflow) {  // (an extension record: only where the count says so)
-              mine = mine && (kMainRecs + 2 * pair >= cnt[j] || rec_tag(more[j].x) == want) &&
-                     (kMainRecs + 2 * pair + 1 >= cnt[j] || rec_tag(more[j].z) == want);
+              mine = mine && (kMainRecs + 2 * pair >= cnt[j] || R64::tag(more[j].x) == want) &&
+                     (kMainRecs + 2 * pair + 1 >= cnt[j] || R64::tag(more[j].z) == want);
             }
             ok = ok && mine;
           }
@@ -442,7 +668,9 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
           }
         }
         if (CLK) phase_[9] += (unsigned long long)spins + 1ull;
-        if (!stop) {
+        if constexpr (HASHED) {
+          if (!stop && !add_records(L, G, P.N, B.raw + (size_t)half * P.N, B.err, want, spin_limit, rec, more, cnt)) L.dead = 1;
+        } else if (!stop) {
 #pragma unroll
           for (int j = 0; j < GS; ++j) {
             const int blk = wave * 64 + j * 32 + (lane >> 1);
@@ -455,14 +683,55 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
             // nobody reads)
             const int n = too_many ? 0 : cnt[j];
             float* none = &L.o_delta[tid];
-            *(2 * pair < n ? &row[rec_slot(rec[j].x)] : none) = __uint_as_float(rec[j].y);
-            *(2 * pair + 1 < n ? &row[rec_slot(rec[j].z)] : none) = __uint_as_float(rec[j].w);
-            *(kMainRecs + 2 * pair < n ? &row[rec_slot(more[j].x)] : none) = __uint_as_float(more[j].y);
-            *(kMainRecs + 2 * pair + 1 < n ? &row[rec_slot(more[j].z)] : none) = __uint_as_float(more[j].w);
+            *(2 * pair < n ? &row[R64::slot(rec[j].x)] : none) = __uint_as_float(rec[j].y);
+            *(2 * pair + 1 < n ? &row[R64::slot(rec[j].z)] : none) = __uint_as_float(rec[j].w);
+            *(kMainRecs + 2 * pair < n ? &row[R64::slot(more[j].x)] : none) = __uint_as_float(more[j].y);
+            *(kMainRecs + 2 * pair + 1 < n ? &row[R64::slot(more[j].z)] : none) = __uint_as_float(more[j].w);
           }
         }
       }
       CRL_MARK(5);
+      if constexpr (HASHED) {
+        __syncthreads();
+        if (L.dead) {  // some wave gave up waiting for its cells
+          gave_up = true;
+          break;
+        }
+        float total[kOwn];
+#pragma unroll
+        for (int o = 0; o < kOwn; ++o) total[o] = 0.0f;
+        const int4 by_key = *reinterpret_cast<const int4*>(L.by_key);
+        if (__builtin_expect((by_key.x | by_key.y | by_key.z | by_key.w) != 0, 0)) {
+          for (int grp = 0; grp < kGroups; ++grp)
+#pragma unroll
+            for (int o = 0; o < kOwn; ++o) {
+              const uint32_t v = L.sum[grp][o * 256 + tid];
+              const float t = L.tile[grp * (kTileBlocks * kOwnKeys / 4 / 4) + o * 256 + tid];
+              total[o] = total[o] + (L.by_key[grp / 4] ? t : v != kNoLead ? __uint_as_float(v) : 0.0f);
+            }
+        } else {
+          auto add = [&](int o, auto groups) {  // (all asked for at once)
+            uint32_t v[decltype(groups)::value];
+#pragma unroll
+            for (int i = 0; i < decltype(groups)::value; ++i) v[i] = L.sum[i][o * 256 + tid];
+#pragma unroll
+            for (int i = 0; i < decltype(groups)::value; ++i) total[o] = total[o] + (v[i] != kNoLead ? __uint_as_float(v[i]) : 0.0f);
+          };
+          // (the groups without envs add nothing)
+          if (live_groups > kGroups / 2) {
+            add(0, std::integral_constant<int, kGroups>{});
+            if (more_keys) add(1, std::integral_constant<int, kGroups>{});
+          } else {
+            add(0, std::integral_constant<int, kGroups / 2>{});
+            if (more_keys) add(1, std::integral_constant<int, kGroups / 2>{});
+          }
+        }
+#pragma unroll
+        for (int o = 0; o < kOwn; ++o) q_own[o] = q_own[o] + total[o];
+        publish(want + 1u);
+        CRL_MARK(6);
+        continue;
+      } else {
       // the wave's four groups: its own 64 rows of the tile, which only it has written
       auto group_sums = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -515,14 +784,14 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
             for (;;) {
               poll_fence();
               v = ld_dev64(B.raw + (size_t)half * P.N + i);
-              if ((tag_of(v) >> kRawTagShift) == want) break;
+              if ((tag_of(v) >> Raw<false>::kTagShift) == want) break;
               if (++spins >= spin_limit || ((spins & 63) == 0 && ld_dev32(B.err) != 0u)) {
                 raw_failed = true;
                 break;
               }
             }
-            const int kk = (int)(tag_of(v) & kRawKeyMask);
-            if (!raw_failed && (tag_of(v) & kRawValid) && owner_of(kk, G) == wg) {
+            const int kk = (int)(tag_of(v) & Raw<false>::kKeyMask);
+            if (!raw_failed && (tag_of(v) & Raw<false>::kValid) && owner_of(kk, G) == wg) {
               slot = slot_of(kk, G);
               dv = value_of(v);
             }
@@ -550,10 +819,11 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
         total = totals();
       }
       if (wave == 0) {
-        q_own = q_own + total;
+        q_own[0] = q_own[0] + total;
         publish(want + 1u);
       }
       CRL_MARK(6);
+      }
     }
   }
 #undef CRL_MARK
@@ -561,7 +831,9 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
   if (CLK && B.clocks && tid == 0 && (wg == 0 || wg == (int)gridDim.x - 1))
     for (int i = 0; i < 10; ++i) B.clocks[(wg ? 10 : 0) + i] = phase_[i];
 
-  if (own_live) P.Q[own_key] = q_own;
+#pragma unroll
+  for (int o = 0; o < kOwn; ++o)
+    if (own_key[o] < G.K) P.Q[own_key[o]] = q_own[o];
   if (has_env) {
     P.s[env] = s;
     P.ep_step[env] = ep_step;

@@ -25,30 +25,37 @@ namespace crl {
 
 constexpr int kBlockSamples = 256;   // level 0
 constexpr int kGroupBlocks = 16;     // level 1
-constexpr int kOwnKeys = 64;         // one-launch kernel: keys per owner workgroup, 64 / A whole table rows
+constexpr int kOwnKeys = 64;         // one-launch kernel, dense form: keys per owner workgroup, 64 / A whole table rows
+constexpr int kOwnKeysHashed = 512;  // ... hashed form
 constexpr int kMaxOwnKeys = 1024;    // two launches: keys per owner at most
 constexpr int kMaxOwners = 4096;     // ... and owners
 constexpr int kSlotOverflow = 127;   // count value: more distinct keys than records, read the block's raw samples instead
 constexpr int kStagePieces = 512;    // 16-byte pieces of the main halves of one block's cells in the one-launch kernel
-constexpr int kDenseKeys = 16384;    // one-launch kernel: keys of its LDS table, one entry per key
-constexpr int kHashSlots = 2048;     // two launches: entries of the LDS table of the keys a block holds
+constexpr int kDenseKeys = 16384;    // one-launch kernel, dense form: keys of its LDS table, one entry per key
+constexpr int kHashSlots = 2048;     // hashed form, two launches: entries of the LDS table of the keys a block holds
 constexpr int kTileBlocks = 256;     // blocks per LDS tile of pass 2
 constexpr uint32_t kOwnerMix = 37;   // odd: spreads cells a power of two apart over owners
 constexpr uint32_t kNoLead = 0xFFFFFFFFu;
 
-// A hand-off record is 64 bits, written and read as one unit.  One-launch kernel:
-//   bits  0..5   slot of the key among its owner's 64
-//   bits  6..12  record 0 of a cell only: how many records the cell holds
-//                (0: none, kSlotOverflow: more distinct keys than the cell has records)
-//   bits 13..31  step tag (the one-launch kernel: a record is valid once its tag is
-//                the step's; 0 where launches separate the steps)
-//   bits 32..63  the block sum, fp32
-constexpr int kRecCountShift = 6, kRecTagShift = 13;
-constexpr uint32_t kRecTagMask = (1u << (32 - kRecTagShift)) - 1u;
-__device__ __forceinline__ unsigned long long make_rec(uint32_t slot, uint32_t count, uint32_t tag, float v) {
-  const uint32_t meta = slot | (count << kRecCountShift) | (tag << kRecTagShift);
-  return (unsigned long long)meta | ((unsigned long long)__float_as_uint(v) << 32);
-}
+// A hand-off record is 64 bits, written and read as one unit.  One-launch kernel, dense /
+// hashed form (owners of up to 64 / 512 keys):
+//   bits  0..5  / 0..8    slot of the key among its owner's
+//   bits  6..12 / 9..15   record 0 of a cell only: how many records the cell holds
+//                         (0: none, kSlotOverflow: more distinct keys than the cell has records)
+//   bits 13..31 / 16..31  step tag (a record is valid once its tag is the step's)
+//   bits 32..63           the block sum, fp32
+template <bool HASHED>
+struct Rec {
+  static constexpr int kCountShift = HASHED ? 9 : 6, kTagShift = kCountShift + 7;
+  static constexpr uint32_t kTagMask = (1u << (32 - kTagShift)) - 1u;
+  static __device__ __forceinline__ unsigned long long make(uint32_t slot, uint32_t tag, float v) {
+    return (unsigned long long)(slot | (tag << kTagShift)) | ((unsigned long long)__float_as_uint(v) << 32);
+  }
+  static __device__ __forceinline__ int slot(uint32_t meta) { return (int)(meta & ((1u << kCountShift) - 1u)); }
+  static __device__ __forceinline__ int count(uint32_t meta) { return (int)((meta >> kCountShift) & 127u); }
+  static __device__ __forceinline__ uint32_t tag(uint32_t meta) { return meta >> kTagShift; }
+};
+static_assert(kOwnKeys == 1 << Rec<false>::kCountShift && kOwnKeysHashed == 1 << Rec<true>::kCountShift, "a record's slot");
 // Two launches: slot in bits 0..15, count in bits 16..22, no tag.
 __device__ __forceinline__ unsigned long long make_wide_rec(uint32_t slot, uint32_t count, float v) {
   return (unsigned long long)(slot | (count << 16)) | ((unsigned long long)__float_as_uint(v) << 32);
@@ -56,9 +63,6 @@ __device__ __forceinline__ unsigned long long make_wide_rec(uint32_t slot, uint3
 __device__ __forceinline__ int wide_slot(uint32_t meta) { return (int)(meta & 0xffffu); }
 __device__ __forceinline__ int wide_count(uint32_t meta) { return (int)(meta >> 16); }
 static_assert(kMaxOwnKeys <= 0x10000, "a record's slot has 16 bits");
-__device__ __forceinline__ int rec_slot(uint32_t meta) { return (int)(meta & 63u); }
-__device__ __forceinline__ int rec_count(uint32_t meta) { return (int)((meta >> kRecCountShift) & 127u); }
-__device__ __forceinline__ uint32_t rec_tag(uint32_t meta) { return meta >> kRecTagShift; }
 
 struct ReduceGeom {
   int K;          // keys of the table, key = cell * A + action
@@ -92,7 +96,7 @@ __host__ __device__ constexpr int main_shift_for(int own_shift) {
   return m < c ? (m < 2 ? 2 : m) : c;
 }
 
-// key <-> (owner, slot in the owner's 64).  An owner holds whole table rows:
+// key <-> (owner, slot among the owner's).  An owner holds whole table rows:
 // hi = cell >> own_shift, owner = (cell + 37 * hi) mod owners, slot = hi * A + action
 __device__ __forceinline__ int owner_of(int key, const ReduceGeom& G) {
   const uint32_t mask = (1u << G.own_shift) - 1u;
@@ -272,15 +276,17 @@ __device__ __forceinline__ bool block_sums(ReduceLdsT<Entries>& L, const int at,
 // one before by another): every record of every cell starts as "nothing, of this step".
 // Thread t touches the 16-byte pieces t, t + 256, ... of `stage` here and on the way out
 // of reduce_block(), and no others.
+template <bool HASHED>
 __device__ __forceinline__ void reduce_stage_init(unsigned long long* stage, const ReduceGeom G, const uint32_t tag) {
-  const unsigned long long none = make_rec(0u, 0u, tag, 0.0f);
+  const unsigned long long none = Rec<HASHED>::make(0u, tag, 0.0f);
   ulonglong2* stage2 = reinterpret_cast<ulonglong2*>(stage);
   for (int i = threadIdx.x; i < 1 << (G.main_shift - 1 + G.own_shift); i += kBlockSamples) stage2[i] = make_ulonglong2(none, none);
 }
 
 // One-launch kernel: pass 1 for one block.  All 256 threads of the workgroup call it with
 // their sample (valid = false: no sample / no delta), having entered their thread number in
-// L.lead[key] with an atomic min; key < K <= kDenseKeys.  The main halves of all cells of the
+// L.lead[at] with an atomic min: `at` is the key itself, or (hashed form) its entry in `keys`,
+// which is cleared again.  The main halves of all cells of the
 // block are put together in LDS (`stage`, owners << main_shift records, free again
 // on return) and go out as whole lines (that of (block, owner) at (block * owners + owner)
 // << main_shift behind `window_offset`), 16 bytes to a store and lane, every record
@@ -291,9 +297,10 @@ __device__ __forceinline__ void reduce_stage_init(unsigned long long* stage, con
 // Returns (to every thread) whether some owner was handed more distinct keys than a
 // cell has records: its cell then says kSlotOverflow and the owner needs the block's
 // raw samples.
-__device__ __forceinline__ bool reduce_block(ReduceLds& L, const ReduceGeom G, const int block,
-                                             const int key, const float delta, const bool valid,
-                                             const uint32_t tag, float* sorted,
+template <bool HASHED, int Entries>
+__device__ __forceinline__ bool reduce_block(ReduceLdsT<Entries>& L, const ReduceGeom G, const int block,
+                                             const int key, const int at, int* keys, const float delta,
+                                             const bool valid, const uint32_t tag, float* sorted,
                                              unsigned long long* stage, const DevWindow window,
                                              const uint32_t window_offset, unsigned long long* ext) {
   const int tid = threadIdx.x;
@@ -301,7 +308,7 @@ __device__ __forceinline__ bool reduce_block(ReduceLds& L, const ReduceGeom G, c
   const int cap = 1 << G.cell_shift;  // records of a cell
   const int cap_main = 1 << G.main_shift;  // of its main half
   float acc;
-  const bool leader = block_sums(L, key, delta, valid, sorted, [&] {
+  const bool leader = block_sums(L, at, delta, valid, sorted, [&] {
     L.handed[tid] = 0;  // (256 owners)
     if (tid == 0) L.over = 0;
   }, &acc);
@@ -310,15 +317,16 @@ __device__ __forceinline__ bool reduce_block(ReduceLds& L, const ReduceGeom G, c
     owner = owner_of(key, G);
     slot = atomicAdd(&L.handed[owner], 1);  // slot order is free: records carry the key
     if (slot >= cap) L.over = 1;
+    if (HASHED) keys[at] = -1;
     // (record 0's count is added on the way out, when every leader has drawn its slot)
-    if (slot < cap_main) stage[(owner << G.main_shift) + slot] = make_rec((uint32_t)slot_of(key, G), 0u, tag, acc);
+    if (slot < cap_main) stage[(owner << G.main_shift) + slot] = Rec<HASHED>::make((uint32_t)slot_of(key, G), tag, acc);
   }
   __syncthreads();
   const bool over = L.over != 0;
   // (behind the barrier: a barrier waits for the stores before it to be acknowledged)
   if (leader && slot >= cap_main && slot < cap)
     st_dev64(ext + ((((size_t)owner * G.n_blocks + block) << G.main_shift) + (slot - cap_main)),
-             make_rec((uint32_t)slot_of(key, G), 0u, tag, acc));
+             Rec<HASHED>::make((uint32_t)slot_of(key, G), tag, acc));
 
   // (the one-launch kernel always has 256 owners and main halves of 4 records: 512 pieces,
   // two to a thread, both asked for before the first is used)
@@ -338,7 +346,7 @@ __device__ __forceinline__ bool reduce_block(ReduceLds& L, const ReduceGeom G, c
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
     const int i = tid + j * kBlockSamples;
-    v[j].x |= (unsigned long long)(uint32_t)(c[j] > cap ? kSlotOverflow : c[j]) << kRecCountShift;
+    v[j].x |= (unsigned long long)(uint32_t)(c[j] > cap ? kSlotOverflow : c[j]) << Rec<HASHED>::kCountShift;
     if (i < pieces)
       st_dev128(window, window_offset + (uint32_t)((((size_t)block * n_own) << (G.main_shift + 3)) + (size_t)i * 16),
                 make_uint4((uint32_t)v[j].x, (uint32_t)(v[j].x >> 32), (uint32_t)v[j].y, (uint32_t)(v[j].y >> 32)));
@@ -398,15 +406,21 @@ __device__ __forceinline__ void sample_delta(const Samples& X, const int i, cons
   }
 }
 
-// The entry of `key` in a table of `mask` + 1 keys (-1: free) that has room for it.
-__device__ __forceinline__ int hash_enter(int* keys, const int mask, const int key) {
-  unsigned h = ((unsigned)key * 0x9E3779B1u) >> 16;
-  for (;;) {
-    h &= (unsigned)mask;
-    const int old = atomicCAS(&keys[h], -1, key);
-    if (old == -1 || old == key) return (int)h;
-    ++h;
+// The entry of `key` in a table of `mask` + 1 keys (-1: free) that has room for it.  In two
+// halves: `found` is what a compare-and-swap of -1 for the key left at the first entry.
+__device__ __forceinline__ int hash_start(const int mask, const int key) {
+  return (int)(((unsigned)key * 0x9E3779B1u) >> 16) & mask;
+}
+__device__ __forceinline__ int hash_finish(int* keys, const int mask, const int key, int h, int found) {
+  while (found != -1 && found != key) {
+    h = (h + 1) & mask;
+    found = atomicCAS(&keys[h], -1, key);
   }
+  return h;
+}
+__device__ __forceinline__ int hash_enter(int* keys, const int mask, const int key) {
+  const int h = hash_start(mask, key);
+  return hash_finish(keys, mask, key, h, atomicCAS(&keys[h], -1, key));
 }
 
 // LDS of pass 1, then handed[owners] (block sums handed to each owner), then `sorted`.

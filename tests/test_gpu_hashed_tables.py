@@ -1,0 +1,132 @@
+"""A shared table of more than 16,384 keys with all steps of a call in one launch (the hashed
+form of k_shared_persist): the smallest and the largest table, owners with a part of a row more
+than others, one block of envs to all 256, cells with more records than their main half, cells
+that overflow into the raw samples.  Bit for bit against the oracle: every sum has a stated
+order."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def run(gpu, oracle, cfg, cls, start, calls, variant=2, trace=False):
+    W, H, A = cfg.width, cfg.height, cfg.n_actions
+    with gpu.Engine(cfg, 0) as eng:
+        eng.set_maps(cls, start)
+        eng.set_fused_variant(variant)
+        if trace:
+            eng.set_trace(cfg.n_envs, sum(calls))
+        name = eng.fused_kernel_info(max(calls))["name"]
+        for n in calls:
+            eng.run_fused(n)
+        q, st = eng.q_get(0), eng.get_state()
+    Q = np.zeros((1, W * H, A), np.float32)
+    ost = oracle.new_state(cfg, start)
+    oracle.run(cfg, cls, None, start, Q, ost, 0, sum(calls))
+    assert np.array_equal(q, Q[0], equal_nan=True)
+    for k in ("s", "ep_step", "episode", "reward", "done", "action"):
+        assert np.array_equal(st[k], ost[k]), k
+    return name, q
+
+
+@pytest.mark.parametrize("N,W,H,A", [(100, 17, 241, 4),       # 16,388 keys: one row more than the dense form takes
+                                     (257, 46, 46, 8), (4097, 65, 64, 4), (20000, 101, 99, 8),
+                                     (65536, 128, 128, 8),    # 512 keys to every owner
+                                     (65000, 181, 181, 4)])
+def test_sizes(gpu, oracle, N, W, H, A):
+    cls, start = gpu.gen_maps_bernoulli(9, 1, N, W, H, 0.12, 0.03)
+    cfg = gpu.make_config(N, W, H, n_actions=A, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=1e-3, eps0=0.3,
+                          episode_len=11, seed=4, trap_reward=-0.5)
+    name, q = run(gpu, oracle, cfg, cls, start, (20, 3, 17))
+    assert name == "k_shared_persist<%d,1,folded,hashed>" % A and np.count_nonzero(q) > 100
+
+
+@pytest.mark.parametrize("options", [dict(max_mode=1, episode_len=9), dict(goal_mode=1, auto_reset=0),
+                                     dict(eps_mode=1, eps_decay=0.9, eps_span=50, max_episodes=3, episode_len=7, track_returns=1)])
+def test_general_rules(gpu, oracle, options):
+    N, W, H = 5000, 70, 61
+    cls, start = gpu.gen_maps_bernoulli(3, 1, N, W, H, 0.12, 0.03)
+    cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=1e-3, eps0=0.4, seed=8, **options)
+    name, _ = run(gpu, oracle, cfg, cls, start, (30, 20))
+    assert name == "k_shared_persist<4,1,hashed>"
+
+
+@pytest.mark.parametrize("cells,envs", [(1, 20000), (3, 20000), (64, 3000), (64, 65536)])
+def test_crowded_keys_and_cells_that_overflow(gpu, oracle, cells, envs):
+    """Every env acts on one of a few cells of one owner in every step: a key that all blocks hold,
+    cells of up to 8 * 3 keys (the extensions, two groups at a time), cells of hundreds (the raw
+    samples, sums by key)."""
+    W, H, A = 128, 128, 8
+    mine = np.array([(h << 8) | ((5 - 37 * h) & 255) for h in range(64)])[:cells]
+    start = np.random.default_rng(cells).choice(mine, envs).astype(np.int32)
+    start[envs // 2:] = np.random.default_rng(7).integers(0, W * H, envs - envs // 2) if cells == 3 else start[envs // 2:]
+    cls = np.zeros((1, W * H), np.uint8)
+    cfg = gpu.make_config(envs, W, H, n_actions=A, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=1e-4, eps0=1.0,
+                          episode_len=1, seed=6)
+    run(gpu, oracle, cfg, cls, start, (12,))
+
+
+@pytest.mark.parametrize("N,W,H,A,steps,hashed", [(20000, 101, 99, 8, 8, True), (20000, 101, 99, 8, 7, False),
+                                                  (20000, 80, 80, 4, 12, True), (20000, 80, 80, 4, 11, False),
+                                                  (8192, 80, 80, 4, 50, True), (8192, 72, 72, 4, 50, False),
+                                                  (8193, 72, 72, 4, 50, True), (65537, 80, 80, 4, 50, False),
+                                                  (20000, 5, 3277, 8, 50, False)])  # 131,080 keys
+def test_which_calls_take_it(gpu, oracle, N, W, H, A, steps, hashed):
+    cls, start = gpu.gen_maps_bernoulli(9, 1, N, W, H, 0.12, 0.03)
+    cfg = gpu.make_config(N, W, H, n_actions=A, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=1e-3, eps0=0.3,
+                          episode_len=30, seed=4)
+    name, _ = run(gpu, oracle, cfg, cls, start, (steps,), variant=0)
+    assert name == ("k_shared_persist<%d,1,folded,hashed>" % A if hashed else "k_shared_act+k_reduce_owners")
+
+
+def test_a_first_call_that_is_recorded(gpu, graphs):
+    """A stream being captured allows no allocation: the call is recorded step by step instead."""
+    N, W, H = 5000, 90, 70
+    cls, start = gpu.gen_maps_bernoulli(2, 1, N, W, H, 0.15)
+    cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=0.02, eps0=0.3, episode_len=5, seed=3)
+    stream = graphs.stream()
+    with gpu.Engine(cfg, 0) as want, gpu.Engine(cfg, 0) as eng:
+        for e in (want, eng):
+            e.set_maps(cls, start)
+            assert e.lib.crl_set_stream(e.h, stream) == 0
+        graph = graphs.record(stream, lambda: eng.run_fused(20))
+        for _ in range(3):
+            eng.step_count = 0  # (a replay draws what the recorded call drew)
+            graphs.replay(graph, stream)
+            want.step_count = 0
+            want.run_fused(20)
+            assert np.array_equal(want.q_get(0), eng.q_get(0))
+            for e in (want, eng):  # eager work between the replays: one launch, with buffers of its own
+                e.step_count = 20
+                e.run_fused(14)
+            assert np.array_equal(want.q_get(0), eng.q_get(0))
+            assert np.array_equal(want.get_state()["s"], eng.get_state()["s"])
+        for e in (want, eng):
+            assert e.lib.crl_set_stream(e.h, None) == 0
+        graphs.destroy(graph)
+    graphs.destroy_stream(stream)
+
+
+def test_it_gives_up_cleanly(gpu):
+    """With a wait of one poll the threads give up and every workgroup leaves the kernel; once state
+    and table are set again the engine works."""
+    N, W, H = 20000, 90, 70
+    cls, start = gpu.gen_maps_bernoulli(6, 1, N, W, H, 0.15)
+    cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=0.004, eps0=0.2, seed=21)
+    q = []
+    for give_up in (True, False):
+        with gpu.Engine(cfg, 0) as eng:
+            eng.set_maps(cls, start)
+            if give_up:
+                eng.set_persist_spin_limit(1)
+                eng.run_fused(50)
+                with pytest.raises(gpu.CrlError, match="gave up"):
+                    eng.sync()
+                eng.set_persist_spin_limit(1 << 20)
+                eng.reset()
+                eng.q_set(0, np.zeros((W * H, 4), np.float32))
+                eng.set_state(s=start.copy(), ep_step=np.zeros(N, np.int32), episode=np.zeros(N, np.int32))
+                eng.step_count = 0
+            eng.run_fused(50)
+            q.append(eng.q_get(0))
+    assert np.array_equal(q[0], q[1]) and np.isfinite(q[0]).all()
