@@ -181,6 +181,9 @@ struct crl_engine {
   // one-launch shared-table kernel: the engine's own give-up word followed by the phase
   // clocks, and whether a launch has not been checked for having given up yet
   DevBuf<unsigned long long> pdiag;  // [0] give-up word, [1..16] phase clocks; allocated at crl_create
+  // The tags in `exchange` are at most this; 0: something else lies there, or may.  (Not kept once a
+  // call has been recorded: a replay clears and counts from the start.)
+  uint32_t exchange_tag = 0;
   bool persist_unchecked = false;
   bool persist_failed = false;   // a launch gave up: state and table are not valid until they are set again
   bool persist_refused = false;  // the device refused the co-resident launch once: not tried again
@@ -885,6 +888,7 @@ int ensure_handoff(crl_engine* e, const crl::ReduceGeom& G, size_t words = 0) {
     hipError_t h = e->grow(e->exchange, std::max(recs, words));
     if (h != hipSuccess) return fail(CRL_E_ALLOC, "hand-off buffer allocation failed: %s", hipGetErrorString(h));
     e->ho = e->exchange.p;
+    e->exchange_tag = 0;
   }
   return opt_in_lds(e);
 }
@@ -1080,23 +1084,25 @@ bool persist_shape(const crl_engine* e, PersistPlan* p) {
   return true;
 }
 
-// Shortest call worth the set-up of the one-launch kernel (clearing what its workgroups
-// exchange, one co-resident launch: 28 us) instead of two plain launches per step, which cost
-// more the more envs there are.  Where the two cross (us per call, one launch / two, at 8, 12 and
-// 16 steps): 3000 envs of 16x16 75/58, 97/88, 119/118; 8000 of 32x32 77/61, 100/91, 123/122;
-// 12,000 of 64x64 78/66, 102/98, 125/131; 16,000 of 32x32 77/64, 100/95, 122/126; 24,000 of 64x64
-// 78/68, 102/102, 126/137; 32,768 of 64x64 82/71, 106/106, 130/141; 40,000 of 32x32 79/73, 103/109,
-// 126/145; 65,536 of 64x64 85/85, 113/127, 139/168.
+// Shortest call worth the set-up of the one-launch kernel (one co-resident launch and its first
+// values: 25 us) instead of two plain launches per step, which cost more the more envs there are.
+// Where the two cross (us per call, one launch / two, at 8, 10, 12 and 14 steps): 3000 envs of 16x16
+// 68/59, 80/74, 91/94, 102/112; 8000 of 32x32 70/61, 82/76, 94/91, 105/107; 16,000 of 32x32 70/65,
+// 81/81, 94/97, 105/119; 32,768 of 64x64 73/71, 86/88, 99/106, 112/124; 65,536 of 64x64 80/85,
+// 94/106, 109/128, 123/149.  The lines of the dense form lie two or three steps higher, where the two
+// crossed while each call also cleared what is exchanged; callers read them from crl_fused_kernel_info,
+// and they stay.
 // With more than 16,384 keys two launches cost 9 to 11 us a step with 4 actions and 13 to 15 with 8
-// (three rows of the neighbourhood instead of one are other lines), the hashed form 6.5 to 10; at 8
-// and 12 steps: 20,000 envs of 101x99, 8 actions 99/100, 133/151; 65,536 of 128x128, 8 actions
-// 121/121, 165/181; 3000 of 90x90 85/77, 112/117; 20,000 of 128x128 95/83, 126/124; 65,536 of
-// 128x128 109/100, 149/152.  Tables of up to 96 keys to an owner under few envs keep two launches,
-// the plan that has always been reported for them (6000 envs of 72x72, 40 steps: 307/401).
+// (a row of the table is 32 bytes then, and a cell has nine of them to read), the hashed form 6.5 to
+// 10; at 6, 8 and 10 steps: 20,000 envs of 101x99, 8 actions 74/75, 90/100, 106/125; 65,536 of 128x128,
+// 8 actions 90/90, 112/120, 133/150; 3000 of 90x90 64/58, 77/77, 91/97; 20,000 of 128x128 72/62, 86/82,
+// 102/103; 65,536 of 128x128 82/75, 103/100, 121/125.  Tables of up to 96 keys to an owner under few
+// envs keep two launches, the plan that has always been reported for them (6000 envs of 72x72, 40
+// steps: 307/401).
 int persist_min_steps(const crl_engine* e, const PersistPlan& p) {
   const int n_envs = e->N;
   if (p.hashed && n_envs <= 8192 && own_keys(p.G) <= 96) return INT_MAX;
-  if (p.hashed) return e->A == 8 ? 8 : 12;
+  if (p.hashed) return e->A == 8 ? 6 : 10;
   return n_envs <= 8192 ? 16 : n_envs <= 16384 ? 14 : n_envs <= 32768 ? 12 : n_envs <= 49152 ? 10 : 9;
 }
 
@@ -1124,7 +1130,7 @@ PersistPlan plan_persist(const crl_engine* e, int n_steps) {
 
 template <int A, int MAP, bool CLK, bool FOLD, bool HASHED>
 hipError_t launch_persist_kernel(crl_engine* e, const PersistPlan& p, unsigned long long* buf, uint64_t t0,
-                                 int n_steps, int trace_row0) {
+                                 int n_steps, uint32_t tag0, int trace_row0) {
   crl::Rules R = e->rules();
   crl::Ptrs P = e->ptrs();
   crl::ReduceGeom G = p.G;
@@ -1135,7 +1141,7 @@ hipError_t launch_persist_kernel(crl_engine* e, const PersistPlan& p, unsigned l
   B.err = reinterpret_cast<unsigned*>(e->pdiag.p);
   B.clocks = e->pdiag.p + 1;
   int spin_limit = e->persist_spin_limit;
-  void* args[] = {&R, &P, &t0, &n_steps, &trace_row0, &G, &B, &spin_limit};
+  void* args[] = {&R, &P, &t0, &n_steps, &tag0, &trace_row0, &G, &B, &spin_limit};
   // a cooperative launch is refused unless all workgroups can be resident together,
   // which the kernel's waits rely on
   return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&crl::k_shared_persist<A, MAP, CLK, FOLD, HASHED>), dim3(p.grid),
@@ -1162,28 +1168,40 @@ int run_persist(crl_engine* e, int n_steps, bool* launched) {
   if (e->no_alloc) {
     buf = reinterpret_cast<unsigned long long*>(e->static_scratch + kScratchTicketBytes);
   } else {
+    if (p.words > e->exchange.n) e->exchange_tag = 0;
     if (e->grow(e->exchange, p.words) != hipSuccess) return fail(CRL_E_ALLOC, "allocation of the exchange buffers failed");
     buf = e->exchange.p;
   }
   rc = opt_in_lds(e);
   if (rc) return rc;
-  // The kernel's tags count the steps of one launch, so everything the workgroups
-  // exchange starts from tag 0 (a fill kernel, not a memset: a caller may record this),
-  // and a call longer than the tags allow goes out as several launches.
+  // A launch's tags go on from those of the launch before, so that what the workgroups exchange
+  // need not be cleared for it (10 MB, a launch of 6 us and the gap behind it; 12
+  // steps of 3000 envs on 16x16 97 -> 91 us).  It is cleared where the tags start again: in a buffer
+  // that something else was in, in the scratch that all engines share, in a launch that is or has been
+  // recorded (its replays bring its tags back) and when they have all been used; a call longer than
+  // that goes out as several launches.  (A kernel, not a memset: a caller may record this.)
+  const uint32_t max_tag = p.hashed ? crl::kPersistMaxTagHashed : crl::kPersistMaxTag;
+  const bool keep = !e->no_alloc && !e->recorded;
+  uint32_t tag = keep ? e->exchange_tag : 0;
   int done = 0;
   while (done < n_steps) {
-    const int n = std::min(n_steps - done, p.hashed ? crl::kPersistMaxStepsHashed : crl::kPersistMaxSteps);
-    const size_t w32 = p.words * 2;
-    hipLaunchKernelGGL(crl::k_fill_u32, dim3((unsigned)((w32 + 255) / 256)), dim3(256), 0, e->stream,
-                       reinterpret_cast<unsigned*>(buf), 0u, w32);
+    // (tags tag + 1 to tag + n + 1)
+    const uint32_t left = (uint32_t)(n_steps - done);
+    if (tag != 0 && (left >= max_tag || tag + left + 1 > max_tag)) tag = 0;
+    const int n = (int)std::min(left, max_tag - 1);
+    if (tag == 0) {
+      const size_t n16 = p.words / 2;
+      hipLaunchKernelGGL(crl::k_clear16, dim3((unsigned)((n16 + 1023) / 1024)), dim3(256), 0, e->stream,
+                         reinterpret_cast<uint4*>(buf), n16);
+    }
     const uint64_t t0 = e->t + (uint64_t)done;
     const int row0 = (int)std::min<long long>((long long)e->trace_cursor + done, e->trace_cap);
     hipError_t h;
 #define CRL_PERSIST_FORM(A, MAP, HASHED)                                                                    \
-  (e->persist_clocks ? (p.fold ? launch_persist_kernel<A, MAP, true, true, HASHED>(e, p, buf, t0, n, row0)    \
-                               : launch_persist_kernel<A, MAP, true, false, HASHED>(e, p, buf, t0, n, row0))  \
-                     : (p.fold ? launch_persist_kernel<A, MAP, false, true, HASHED>(e, p, buf, t0, n, row0)   \
-                               : launch_persist_kernel<A, MAP, false, false, HASHED>(e, p, buf, t0, n, row0)))
+  (e->persist_clocks ? (p.fold ? launch_persist_kernel<A, MAP, true, true, HASHED>(e, p, buf, t0, n, tag, row0)    \
+                               : launch_persist_kernel<A, MAP, true, false, HASHED>(e, p, buf, t0, n, tag, row0))  \
+                     : (p.fold ? launch_persist_kernel<A, MAP, false, true, HASHED>(e, p, buf, t0, n, tag, row0)   \
+                               : launch_persist_kernel<A, MAP, false, false, HASHED>(e, p, buf, t0, n, tag, row0)))
 #define CRL_PERSIST(A, MAP) (p.hashed ? CRL_PERSIST_FORM(A, MAP, true) : CRL_PERSIST_FORM(A, MAP, false))
     if (e->A == 4) h = p.lds_map ? CRL_PERSIST(4, 1) : CRL_PERSIST(4, 2);
     else h = p.lds_map ? CRL_PERSIST(8, 1) : CRL_PERSIST(8, 2);
@@ -1197,6 +1215,8 @@ int run_persist(crl_engine* e, int n_steps, bool* launched) {
     }
     e->persist_unchecked = true;
     done += n;
+    tag += (uint32_t)n + 1;
+    if (!e->no_alloc) e->exchange_tag = keep ? tag : 0;
   }
   if (e->trace_n > 0) {
     const long long c = (long long)e->trace_cursor + n_steps;

@@ -1629,6 +1629,13 @@ __global__ void k_fill_u32(unsigned* p, const unsigned v, const size_t n) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
+// n16 16-byte words, four to a thread of 256
+__global__ __launch_bounds__(256) void k_clear16(uint4* __restrict__ p, const size_t n16) {
+  const size_t i0 = (size_t)blockIdx.x * 1024 + threadIdx.x;
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    if (i0 + 256 * u < n16) p[i0 + 256 * u] = make_uint4(0u, 0u, 0u, 0u);
+}
 // (a launch instead of a device-to-device copy: a caller may record the call)
 __global__ void k_copy3_u32(const unsigned* __restrict__ src, unsigned* __restrict__ dst) {
   if (threadIdx.x < 3) dst[threadIdx.x] = src[threadIdx.x];

@@ -26,7 +26,7 @@
 //                               block with more than 4 distinct keys for that owner writes into
 //   raw[env]     {delta, key, tag}   only from blocks whose cell for some owner overflowed
 //
-// One step k (tag k + 1 for what the blocks read, k + 2 for the table that results):
+// One step k (tag0 + k + 1 for what the blocks read, tag0 + k + 2 for the table that results):
 //   block:  what does not depend on the table (exploration draw, neighbour cells, move
 //           codes; the owner's stores are on their way meanwhile) -> poll the view of
 //           the env's cell -> select, move, (key, delta) -> ordered block sums -> cells
@@ -63,8 +63,9 @@ constexpr int kMainShift = 2, kMainRecs = 1 << kMainShift;  // records in the ha
 static_assert(main_shift_for(kPersistOwnShift) == kMainShift && cell_shift_for(kPersistOwnShift) == kMainShift + 1 &&
               (1 << kPersistOwnShift) == kPersistMaxGroups && (kPersistMaxGroups << (kMainShift - 1)) == kStagePieces,
               "the owner's loads are laid out for cells of 4 + 4 records");
-constexpr int kPersistMaxSteps = 65535;     // per launch, dense form: the raw samples' tags have 17 bits
-constexpr int kPersistMaxStepsHashed = 16381;  // ... hashed form: 14 bits
+// The tags of what is exchanged only grow, from one launch to the next as well; when they reach
+// what the raw samples' 17 (hashed form: 14) bits hold, everything is cleared and they start again.
+constexpr uint32_t kPersistMaxTag = (1u << 17) - 1u, kPersistMaxTagHashed = (1u << 14) - 1u;
 constexpr int kPersistClockWords = 20 + 8 * 256;  // 2 workgroups x (8 phases + polls of the two waits by thread 0),
                                                   // then the wall clock of every workgroup at the 8 marks of one step
 
@@ -126,10 +127,8 @@ struct Raw {
 };
 static_assert(kDenseKeys - 1 <= (int)Raw<false>::kKeyMask && kOwnKeysHashed * kPersistMaxGroups - 1 <= (int)Raw<true>::kKeyMask,
               "raw samples hold a key");
-static_assert(kPersistMaxSteps + 1 < (1 << (32 - Raw<false>::kTagShift)) &&
-              kPersistMaxStepsHashed + 1 < (1 << (32 - Raw<true>::kTagShift)), "raw tags must be unique within a launch");
-static_assert((uint32_t)kPersistMaxSteps + 1u <= Rec<false>::kTagMask &&
-              (uint32_t)kPersistMaxStepsHashed + 1u <= Rec<true>::kTagMask, "record tags must be unique within a launch");
+static_assert(kPersistMaxTag < (1u << (32 - Raw<false>::kTagShift)) && kPersistMaxTagHashed < (1u << (32 - Raw<true>::kTagShift)) &&
+              kPersistMaxTag <= Rec<false>::kTagMask && kPersistMaxTagHashed <= Rec<true>::kTagMask, "tags must be unique");
 
 template <int A>
 __device__ __forceinline__ Row<A> row_of_tagged(const unsigned long long (&v)[A]);
@@ -321,7 +320,7 @@ __device__ __forceinline__ bool add_records(PersistLdsHashed& L, const ReduceGeo
 // (they do not change during a launch, so plain loads are fine).
 // G.own_shift = kPersistOwnShift, G.n_blocks = 256 = the number of workgroups (blocks
 // without envs hand over empty cells).
-// Everything in B holds tag 0 at launch (cleared by the host), *B.err is zero.
+// Everything in B holds tags of at most tag0 at launch, *B.err is zero.
 // FOLD = the rules of the common configuration are compile-time facts (goal test on the
 // target cell, restart at the end of an episode, true maximum, rewards by class, no trace,
 // no supplied stream, no episode budget, no return statistics): the general kernel keeps
@@ -329,8 +328,8 @@ __device__ __forceinline__ bool add_records(PersistLdsHashed& L, const ReduceGeo
 // fetched back again and again (190 lane reads per step).
 template <int A, int MAP, bool CLK, bool FOLD, bool HASHED>
 __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptrs P, const uint64_t t0,
-                                                         const int n_steps, const int trace_row0,
-                                                         const ReduceGeom G, const PersistBufs B,
+                                                         const int n_steps, const uint32_t tag0,
+                                                         const int trace_row0, const ReduceGeom G, const PersistBufs B,
                                                          const int spin_limit) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   using Lds = PersistLdsOf<HASHED>;
@@ -435,7 +434,7 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
       }
     }
   };
-  if (owns) publish(1u);
+  if (owns) publish(tag0 + 1u);
   __syncthreads();
 
   // What a step needs that does not depend on the table: computed at the top of the step,
@@ -481,7 +480,7 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
   unsigned long long last_ = CLK ? clock64() : 0ull;
   bool gave_up = false;
   for (int k = 0; k < n_steps; ++k) {
-    const uint32_t want = (uint32_t)k + 1u;
+    const uint32_t want = tag0 + (uint32_t)k + 1u;
     CRL_MARK(7);
     // (the values this workgroup published as an owner are on their way meanwhile)
     prepare(k);

@@ -140,7 +140,7 @@ int crl_set_resident_envs(crl_engine* e, int32_t n_envs);
  * through device-scope loads and stores (needs every workgroup resident at once:
  * at most 65,536 envs and 131,072 table entries, else two launches per step);
  * automatic picks the one launch for calls of at least 16 steps, down to 9 with more
- * than 49,152 envs; with more than 16,384 entries for 12 steps, 8 with 8 actions.
+ * than 49,152 envs; with more than 16,384 entries for 10 steps, 6 with 8 actions.
  * Results do not depend on it. */
 int crl_set_fused_variant(crl_engine* e, int32_t variant);
 /* How the last hybrid crl_run_fused split the envs between its two kinds of

@@ -66,8 +66,8 @@ def test_crowded_keys_and_cells_that_overflow(gpu, oracle, cells, envs):
     run(gpu, oracle, cfg, cls, start, (12,))
 
 
-@pytest.mark.parametrize("N,W,H,A,steps,hashed", [(20000, 101, 99, 8, 8, True), (20000, 101, 99, 8, 7, False),
-                                                  (20000, 80, 80, 4, 12, True), (20000, 80, 80, 4, 11, False),
+@pytest.mark.parametrize("N,W,H,A,steps,hashed", [(20000, 101, 99, 8, 6, True), (20000, 101, 99, 8, 5, False),
+                                                  (20000, 80, 80, 4, 10, True), (20000, 80, 80, 4, 9, False),
                                                   (8192, 80, 80, 4, 50, True), (8192, 72, 72, 4, 50, False),
                                                   (8193, 72, 72, 4, 50, True), (65537, 80, 80, 4, 50, False),
                                                   (20000, 5, 3277, 8, 50, False)])  # 131,080 keys
@@ -130,3 +130,78 @@ def test_it_gives_up_cleanly(gpu):
             eng.run_fused(50)
             q.append(eng.q_get(0))
     assert np.array_equal(q[0], q[1]) and np.isfinite(q[0]).all()
+
+
+@pytest.mark.parametrize("N,W,H,calls", [(90, 17, 241, (9000, 7381, 1, 20000, 300)),  # hashed: 16,383 tags, reached exactly by the second call
+                                         (20, 9, 7, (70000, 61069, 1, 300))])         # dense: 131,071
+def test_tags_that_run_out(gpu, oracle, N, W, H, calls):
+    cls, start = gpu.gen_maps_bernoulli(9, 1, N, W, H, 0.12, 0.03)
+    cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=1e-3, eps0=0.3,
+                          episode_len=50, seed=4)
+    run(gpu, oracle, cfg, cls, start, calls)
+
+
+@pytest.mark.parametrize("W,H", [(32, 16), (90, 70)])
+def test_tags_go_on_only_over_what_the_kernel_itself_left(gpu, oracle, W, H):
+    """Between the one-launch calls: steps of two launches, an update from host data, the scratch that
+    engines share, a recorded call and its replays."""
+    N, A = 3000, 4
+    cls, start = gpu.gen_maps_bernoulli(9, 1, N, W, H, 0.12, 0.03)
+    cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=1e-3, eps0=0.3,
+                          episode_len=50, seed=4)
+    rng = np.random.default_rng(1)
+    s, a, s2 = rng.integers(0, W * H, 5000), rng.integers(0, A, 5000), rng.integers(0, W * H, 5000)
+    r, d = rng.normal(0, 1, 5000).astype(np.float32), np.zeros(5000, np.uint8)
+    Q = np.zeros((1, W * H, A), np.float32)
+    ost = oracle.new_state(cfg, start)
+    with gpu.Engine(cfg, 0) as eng:
+        eng.set_maps(cls, start)
+        t = 0
+        for kind, n in [("one", 20), ("one", 5), ("two", 4), ("one", 9), ("td", 0), ("one", 9), ("noalloc", 20), ("one", 20),
+                        ("rounds", 2), ("one", 3), ("one", 1)]:
+            eng.set_fused_variant(1 if kind == "two" else 2)
+            if kind == "td":
+                eng.td_update(0, s, a, r, s2, d)
+                flat = Q[0].reshape(-1).copy()
+                oracle.td_update_batch(flat, W * H, A, s, a, r, s2, d, cfg.lr, cfg.gamma, 0)
+                Q[0] = flat.reshape(W * H, A)
+            elif kind == "rounds":
+                for _ in range(n):
+                    eng.step(eng.select())
+                    eng.update()
+            else:
+                (eng.run_fused_noalloc if kind == "noalloc" else eng.run_fused)(n)
+            oracle.run(cfg, cls, None, start, Q, ost, t, n)
+            t += n
+            assert np.array_equal(eng.q_get(0), Q[0]), (kind, t)
+        assert np.array_equal(eng.get_state()["s"], ost["s"])
+
+
+@pytest.mark.parametrize("W,H", [(32, 16), (90, 70)])
+def test_replays_bring_their_tags_back(gpu, graphs, W, H):
+    N = 3000
+    cls, start = gpu.gen_maps_bernoulli(9, 1, N, W, H, 0.12, 0.03)
+    cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=1e-3, eps0=0.3,
+                          episode_len=50, seed=4)
+    stream = graphs.stream()
+    with gpu.Engine(cfg, 0) as want, gpu.Engine(cfg, 0) as eng:
+        for e, variant in ((want, 1), (eng, 2)):
+            e.set_maps(cls, start)
+            e.set_fused_variant(variant)
+            assert e.lib.crl_set_stream(e.h, stream) == 0
+            e.run_fused(10)
+            e.step_count = 0
+        graph = graphs.record(stream, lambda: eng.run_fused(60))
+        for eager in (30, 30, 3, 100, 7):
+            graphs.replay(graph, stream)
+            want.step_count = 0
+            want.run_fused(60)
+            for e in (want, eng):
+                e.step_count = 60
+                e.run_fused(eager)
+            assert np.array_equal(want.q_get(0), eng.q_get(0))
+            assert np.array_equal(want.get_state()["s"], eng.get_state()["s"])
+        for e in (want, eng):
+            assert e.lib.crl_set_stream(e.h, None) == 0
+        graphs.destroy(graph)
+    graphs.destroy_stream(stream)
