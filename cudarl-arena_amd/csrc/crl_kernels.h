@@ -490,102 +490,153 @@ __device__ __forceinline__ void wave_fence() {
 // move into it then; and a lane move, like the use of a comparison's mask, has to stay two
 // instructions away from the one that wrote its operand, which the compiler does not see
 // inside an asm statement, so each block keeps that distance itself (also from what comes
-// before it), with work that is due anyway where there is some: s_nop 1 costs nine cycles,
-// any other instruction five.  Masks of comparisons go from vector
-// instruction to vector instruction: a scalar instruction between them waits for 13 cycles,
-// a branch on one for 28.
+// before it), with work that is due anyway where there is some.  A lone wave issues an
+// instruction every four cycles (measured; runs of 8-byte encodings every five), s_nop 1 costs
+// two of them.  Masks of comparisons go from vector instruction to vector instruction: a scalar
+// instruction between them waits for 13 cycles, a branch on one for 28, a taken one for 25.
 #define CRL_PAIRS "quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
 #define CRL_HALVES "quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
 #define CRL_EIGHT "row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
 
-// Maximum of q over the env's lanes, but at least `floor` (no number: no floor).  On the
-// way, for the draw of the next step: named = c in the lane of its action (low byte) and all
-// ones elsewhere, explore = the lanes whose draw is below their limit.
+// The update: top = the maximum of the row q2 over the env's lanes, but at least `floor` (no
+// number: no floor), 0 in the lanes of `hit`; q_new = q after the update with that target in the
+// lanes of `me`, elsewhere q; next = q_new in the lanes of `stays`, elsewhere q_next.  On the way,
+// for the draw of the next step: named = c in the lane of its action (low byte) and all ones
+// elsewhere, explore = the lanes whose draw is below their limit; word += next_word.
 template <int A>
-__device__ __forceinline__ float row_top(float q, float floor, uint32_t draw, uint32_t limit, uint32_t mine, uint32_t c,
-                                         uint32_t& named, unsigned long long& explore) {
-  float m;
-  if (A == 4)
-    asm("v_cmp_eq_u32_sdwa vcc, %[draw], %[mine] src0_sel:BYTE_0 src1_sel:DWORD\n\t"
-        "v_cmp_lt_u32 %[explore], %[draw], %[limit]\n\t"
-        "v_max_f32_dpp %[m], %[q], %[q] " CRL_PAIRS
-        "v_cndmask_b32 %[named], -1, %[c], vcc\n\t"
-        "s_nop 0\n\t"
-        "v_max_f32_dpp %[m], %[m], %[m] " CRL_HALVES
-        "v_max_f32 %[m], %[m], %[floor]"
-        : [m] "=&v"(m), [named] "=&v"(named), [explore] "=&s"(explore)
-        : [q] "v"(q), [floor] "v"(floor), [draw] "v"(draw), [limit] "v"(limit), [mine] "v"(mine), [c] "v"(c)
-        : "vcc");
-  else
-    asm("v_cmp_eq_u32_sdwa vcc, %[draw], %[mine] src0_sel:BYTE_0 src1_sel:DWORD\n\t"
-        "v_cmp_lt_u32 %[explore], %[draw], %[limit]\n\t"
-        "v_max_f32_dpp %[m], %[q], %[q] " CRL_PAIRS
-        "v_cndmask_b32 %[named], -1, %[c], vcc\n\t"
-        "s_nop 0\n\t"
-        "v_max_f32_dpp %[m], %[m], %[m] " CRL_HALVES
-        "s_nop 1\n\t"
-        "v_max_f32_dpp %[m], %[m], %[m] " CRL_EIGHT
-        "v_max_f32 %[m], %[m], %[floor]"
-        : [m] "=&v"(m), [named] "=&v"(named), [explore] "=&s"(explore)
-        : [q] "v"(q), [floor] "v"(floor), [draw] "v"(draw), [limit] "v"(limit), [mine] "v"(mine), [c] "v"(c)
-        : "vcc");
-  return m;
+__device__ __forceinline__ float lanes_update(float q, float q2, float q_next, float reward, unsigned long long hit,
+                                              unsigned long long me, unsigned long long stays, float lr, float gamma,
+                                              float floor, uint32_t draw, uint32_t limit, uint32_t mine, uint32_t c,
+                                              uint32_t& named, unsigned long long& explore, uint32_t& word,
+                                              uint32_t next_word, float& q_new) {
+  float m, next;
+#define CRL_UPDATE(MORE)                                                              \
+  asm("v_cmp_eq_u32_sdwa vcc, %[draw], %[mine] src0_sel:BYTE_0 src1_sel:DWORD\n\t"  \
+      "v_cmp_lt_u32 %[explore], %[draw], %[limit]\n\t"                              \
+      "v_max_f32_dpp %[m], %[q2], %[q2] " CRL_PAIRS                                   \
+      "v_cndmask_b32 %[named], -1, %[c], vcc\n\t"                                   \
+      "v_add_u32 %[word], %[next_word], %[word]\n\t"                                \
+      "v_max_f32_dpp %[m], %[m], %[m] " CRL_HALVES MORE                               \
+      "v_max_f32 %[m], %[m], %[floor]\n\t"                                          \
+      "v_cndmask_b32 %[m], %[m], 0, %[hit]\n\t"                                     \
+      "v_fma_f32 %[m], %[gamma], %[m], %[reward]\n\t"                               \
+      "v_sub_f32 %[m], %[m], %[q]\n\t"                                              \
+      "v_fma_f32 %[m], %[lr], %[m], %[q]\n\t"                                       \
+      "v_cndmask_b32 %[q_new], %[q], %[m], %[me]\n\t"                               \
+      "v_cndmask_b32 %[next], %[q_next], %[q_new], %[stays]"                          \
+      : [m] "=&v"(m), [next] "=&v"(next), [named] "=&v"(named), [explore] "=&s"(explore), [word] "+v"(word),      \
+        [q_new] "=&v"(q_new)                                                                                      \
+      : [q] "v"(q), [q2] "v"(q2), [q_next] "v"(q_next), [reward] "v"(reward), [hit] "s"(hit), [me] "s"(me),       \
+        [stays] "s"(stays), [lr] "s"(lr), [gamma] "s"(gamma), [floor] "v"(floor), [draw] "v"(draw),               \
+        [limit] "v"(limit), [mine] "v"(mine), [c] "v"(c), [next_word] "s"(next_word)                              \
+      : "vcc")
+  if (A == 4) CRL_UPDATE("");
+  else CRL_UPDATE("s_nop 1\n\tv_max_f32_dpp %[m], %[m], %[m] " CRL_EIGHT);
+#undef CRL_UPDATE
+  return next;
 }
-// The smallest word of the lanes that qualify: those of `named` that are not all ones where
-// the env explores, else those whose q no other beats - where `unless` is the value that a q
-// that is no number counts as: in the first lane it stays one, and then nothing beats it
-// (src/q_learning.cu:200-206: strict >, from action 0 on).  On the way: word += next_word,
-// left -= 1.
-template <int A>
-__device__ __forceinline__ uint32_t row_pick_word(float q, float unless, uint32_t c, uint32_t named, unsigned long long explore,
-                                                  uint32_t& word, uint32_t next_word, int& left) {
+
+// Episode statistics of an env (in all its lanes).
+struct LaneStats {
+  float ret, ret_last, ret_sum;
+  int len_last, len_sum;
+};
+// The choice: the smallest word of the lanes that qualify - those of `named` that are not all
+// ones where the env explores, else those whose q no other beats, where `unless` is the value
+// that a q that is no number counts as: in the first lane it stays one, and then nothing beats
+// it (src/q_learning.cu:200-206: strict >, from action 0 on).  On the way: last = the lanes
+// whose episode has no step left after this one.  TRACK: the step before had this reward, and in
+// the lanes of `ends` an episode of `len` steps ended with it; the statistics take the places
+// that are idle otherwise.
+template <int A, bool TRACK>
+__device__ __forceinline__ uint32_t lanes_choose(float q, float unless, uint32_t c, uint32_t named, unsigned long long explore,
+                                                 int left, unsigned long long& last, LaneStats& stats, float reward,
+                                                 unsigned long long ends, int len) {
   float v, m;
   uint32_t w;
-  if (A == 4)
-    asm("v_max_f32 %[v], %[q], %[unless]\n\t"
-        "s_nop 1\n\t"
-        "v_max_f32_dpp %[m], %[v], %[v] " CRL_PAIRS
-        "s_nop 1\n\t"
-        "v_max_f32_dpp %[m], %[m], %[m] " CRL_HALVES
-        "v_cmp_nlt_f32 vcc, %[v], %[m]\n\t"
-        "v_add_u32 %[word], %[next_word], %[word]\n\t"
-        "v_add_u32 %[left], -1, %[left]\n\t"
-        "v_cndmask_b32 %[w], -1, %[c], vcc\n\t"
-        "v_cndmask_b32 %[w], %[w], %[named], %[explore]\n\t"
-        "s_nop 1\n\t"
-        "v_min_u32_dpp %[w], %[w], %[w] " CRL_PAIRS
-        "s_nop 1\n\t"
-        "v_min_u32_dpp %[w], %[w], %[w] " CRL_HALVES
-        : [v] "=&v"(v), [m] "=&v"(m), [w] "=&v"(w), [word] "+v"(word), [left] "+v"(left)
-        : [q] "v"(q), [unless] "v"(unless), [c] "v"(c), [named] "v"(named), [explore] "s"(explore), [next_word] "s"(next_word)
-        : "vcc");
-  else
-    asm("v_max_f32 %[v], %[q], %[unless]\n\t"
-        "s_nop 1\n\t"
-        "v_max_f32_dpp %[m], %[v], %[v] " CRL_PAIRS
-        "s_nop 1\n\t"
-        "v_max_f32_dpp %[m], %[m], %[m] " CRL_HALVES
-        "s_nop 1\n\t"
-        "v_max_f32_dpp %[m], %[m], %[m] " CRL_EIGHT
-        "v_cmp_nlt_f32 vcc, %[v], %[m]\n\t"
-        "v_add_u32 %[word], %[next_word], %[word]\n\t"
-        "v_add_u32 %[left], -1, %[left]\n\t"
-        "v_cndmask_b32 %[w], -1, %[c], vcc\n\t"
-        "v_cndmask_b32 %[w], %[w], %[named], %[explore]\n\t"
-        "s_nop 1\n\t"
-        "v_min_u32_dpp %[w], %[w], %[w] " CRL_PAIRS
-        "s_nop 1\n\t"
-        "v_min_u32_dpp %[w], %[w], %[w] " CRL_HALVES
-        "s_nop 1\n\t"
-        "v_min_u32_dpp %[w], %[w], %[w] " CRL_EIGHT
-        : [v] "=&v"(v), [m] "=&v"(m), [w] "=&v"(w), [word] "+v"(word), [left] "+v"(left)
-        : [q] "v"(q), [unless] "v"(unless), [c] "v"(c), [named] "v"(named), [explore] "s"(explore), [next_word] "s"(next_word)
-        : "vcc");
+#define CRL_CHOOSE(G1, G2, G3, G4, G5, MORE1, MORE2)                        \
+  "v_max_f32 %[v], %[q], %[unless]\n\t"                                       \
+  "v_cmp_ge_i32 %[last], 1, %[left]\n\t" G1                                   \
+  "v_max_f32_dpp %[m], %[v], %[v] " CRL_PAIRS G2                                \
+  "v_max_f32_dpp %[m], %[m], %[m] " CRL_HALVES MORE1                            \
+  "v_cmp_nlt_f32 vcc, %[v], %[m]\n\t" G3                                      \
+  "v_cndmask_b32 %[w], -1, %[c], vcc\n\t"                                     \
+  "v_cndmask_b32 %[w], %[w], %[named], %[explore]\n\t" G4                     \
+  "v_min_u32_dpp %[w], %[w], %[w] " CRL_PAIRS G5                                \
+  "v_min_u32_dpp %[w], %[w], %[w] " CRL_HALVES MORE2
+#define CRL_NOP "s_nop 0\n\t"
+#define CRL_NOPS "s_nop 1\n\t"
+#define CRL_CHOOSE_IN                                                                                                     \
+  [q] "v"(q), [unless] "v"(unless), [c] "v"(c), [named] "v"(named), [explore] "s"(explore), [left] "v"(left)
+#define CRL_MAX8 CRL_NOPS "v_max_f32_dpp %[m], %[m], %[m] " CRL_EIGHT
+#define CRL_MIN8 CRL_NOPS "v_min_u32_dpp %[w], %[w], %[w] " CRL_EIGHT
+  if constexpr (TRACK) {
+    float sum;
+#define CRL_TRACKED(MORE1, MORE2)                                                                                         \
+  asm(CRL_CHOOSE("v_add_f32 %[ret], %[ret], %[reward]\n\t",                                                             \
+                 "v_cndmask_b32 %[len_last], %[len_last], %[len], %[ends]\n\t"                                          \
+                 "v_add_f32 %[sum], %[ret_sum], %[ret]\n\t",                                                            \
+                 "v_cndmask_b32 %[ret_last], %[ret_last], %[ret], %[ends]\n\t"                                          \
+                 "v_cndmask_b32 %[ret], %[ret], 0, %[ends]\n\t",                                                        \
+                 "v_cndmask_b32 %[ret_sum], %[ret_sum], %[sum], %[ends]\n\t"                                            \
+                 "v_cndmask_b32 %[sum], 0, %[len], %[ends]\n\t",                                                        \
+                 "v_add_u32 %[len_sum], %[len_sum], %[sum]\n\t" CRL_NOP, MORE1, MORE2)                                \
+      : [v] "=&v"(v), [m] "=&v"(m), [w] "=&v"(w), [last] "=&s"(last), [sum] "=&v"(sum), [ret] "+v"(stats.ret),            \
+        [ret_last] "+v"(stats.ret_last), [ret_sum] "+v"(stats.ret_sum), [len_last] "+v"(stats.len_last),                  \
+        [len_sum] "+v"(stats.len_sum)                                                                                     \
+      : CRL_CHOOSE_IN, [reward] "v"(reward), [ends] "s"(ends), [len] "v"(len)                                             \
+      : "vcc")
+    if (A == 4) CRL_TRACKED("", "");
+    else CRL_TRACKED(CRL_MAX8, CRL_MIN8);
+#undef CRL_TRACKED
+  } else {
+#define CRL_PLAIN(MORE1, MORE2)                                                             \
+  asm(CRL_CHOOSE(CRL_NOP, CRL_NOPS, CRL_NOPS, CRL_NOPS, CRL_NOPS, MORE1, MORE2)           \
+      : [v] "=&v"(v), [m] "=&v"(m), [w] "=&v"(w), [last] "=&s"(last)                        \
+      : CRL_CHOOSE_IN                                                                       \
+      : "vcc")
+    if (A == 4) CRL_PLAIN("", "");
+    else CRL_PLAIN(CRL_MAX8, CRL_MIN8);
+#undef CRL_PLAIN
+  }
+#undef CRL_CHOOSE
+#undef CRL_CHOOSE_IN
+#undef CRL_NOP
+#undef CRL_NOPS
+#undef CRL_MAX8
+#undef CRL_MIN8
   return w;
 }
 #undef CRL_PAIRS
 #undef CRL_HALVES
 #undef CRL_EIGHT
+
+// Where the env acts from next: where the move ends, `at2`, or the start cell in the lanes of
+// `last` and where the target was the goal (hit).
+__device__ __forceinline__ uint32_t lanes_next(uint32_t at2, uint32_t at_start, uint32_t cls, unsigned long long last,
+                                               unsigned long long& hit) {
+  uint32_t at;
+  asm("v_cmp_eq_u32 %[hit], 4, %[cls]\n\t"
+      "v_cndmask_b32 %[at], %[at2], %[start], %[last]\n\t"
+      "s_nop 0\n\t"
+      "v_cndmask_b32 %[at], %[at], %[start], %[hit]"
+      : [at] "=&v"(at), [hit] "=&s"(hit)
+      : [at2] "v"(at2), [start] "v"(at_start), [cls] "v"(cls), [last] "s"(last));
+  return at;
+}
+// Steps left of the episode and episodes so far, after a step that ended one in the lanes returned.
+__device__ __forceinline__ unsigned long long lanes_count(unsigned long long hit, unsigned long long last, int whole, int& left,
+                                                          int& episode) {
+  unsigned long long ends;
+  asm("s_or_b64 %[ends], %[hit], %[last]\n\t"
+      "v_add_u32 %[left], -1, %[left]\n\t"
+      "v_cndmask_b32 %[left], %[left], %[whole], %[ends]\n\t"
+      "v_addc_co_u32 %[episode], vcc, 0, %[episode], %[ends]"
+      : [ends] "=&s"(ends), [left] "+v"(left), [episode] "+v"(episode)
+      : [hit] "s"(hit), [last] "s"(last), [whole] "v"(whole)
+      : "vcc", "scc");
+  return ends;
+}
 
 // What an action does from a cell, as one word: the action in the top three bits, the
 // resulting cell as the byte offset of its row (a multiple of 16), the class of the target
@@ -610,6 +661,7 @@ struct LaneLds {
   uint32_t first;  // LDS address of the lane's value of the env's first cell
   using At = uint32_t;
   __device__ __forceinline__ At at(uint32_t offset) const { return first + offset; }
+  __device__ __forceinline__ At at_word(uint32_t word) const { return first + (word & kMoveOffset); }
   __device__ __forceinline__ uint32_t offset(At p) const { return p - first; }
   static __device__ __forceinline__ float value(At p) { return *lds_at<float>(p); }
   // asks for what `word` needs / the lane's move word from that, when it has arrived
@@ -632,6 +684,7 @@ struct LaneCodes {
   int step;                    // bytes from a row to the one the lane's action leads to
   using At = uint32_t;
   __device__ __forceinline__ At at(uint32_t offset) const { return offset; }
+  __device__ __forceinline__ At at_word(uint32_t word) const { return word & kMoveOffset; }
   __device__ __forceinline__ uint32_t offset(At p) const { return p; }
   __device__ __forceinline__ float value(At p) const { return *reinterpret_cast<const float*>(values + (QL ? p : values_at + p)); }
   __device__ __forceinline__ uint32_t code(At p) const {
@@ -663,7 +716,8 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
   const int lane = (int)__lane_id();
   const uint32_t mine = (uint32_t)lane & (A - 1);  // this lane's action
   const int slot = live ? lane / A : 0, env = env0 + slot;
-  const int whole = R.episode_len > 0 ? R.episode_len : 0x7fffffff;
+  int whole = R.episode_len > 0 ? R.episode_len : 0x7fffffff;
+  asm("" : "+v"(whole));
   const float lr = R.lr, gamma = R.gamma;
   const float nan = __uint_as_float(0x7fc00000u);
   const float floor = R.max_mode == 1 ? 0.0f : nan;
@@ -678,15 +732,8 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
   const bool base_cells = CELLS && (R.reward_flags & 2) != 0;
   uint32_t limit = by_episode ? tape_limit(eps_of(R, P.eps_tab, t0, episode)) : kTapeLimit;
   float eps_next = by_episode ? eps_of(R, P.eps_tab, t0, episode + 1) : 0.0f;  // of the next episode: asked for ahead
-  float ret = 0.0f, ret_last = 0.0f, ret_sum = 0.0f;
-  int len_last = 0, len_sum = 0;
-  if (track) {
-    ret = P.ret_acc[env];
-    ret_last = P.ret_last[env];
-    ret_sum = P.ret_sum[env];
-    len_last = P.len_last[env];
-    len_sum = P.len_sum[env];
-  }
+  LaneStats stats{0.0f, 0.0f, 0.0f, 0, 0};
+  if (track) stats = LaneStats{P.ret_acc[env], P.ret_last[env], P.ret_sum[env], P.len_last[env], P.len_sum[env]};
   const int budget = EVENTS && R.max_episodes > 0 ? R.max_episodes : 0x7fffffff;
   bool going = live && episode < budget;
   float q = mem.value(at);
@@ -694,7 +741,7 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
   // (arrived before the loop starts: a value that may be in flight there makes every round
   // wait for everything, the last store's answer included)
   asm volatile("" : "+v"(q), "+v"(c), "+v"(reward), "+v"(left), "+v"(episode), "+v"(won), "+v"(limit), "+v"(eps_next));
-  if (EVENTS) asm volatile("" : "+v"(ret), "+v"(ret_last), "+v"(ret_sum), "+v"(len_last), "+v"(len_sum));
+  if (EVENTS) asm volatile("" : "+v"(stats.ret), "+v"(stats.ret_last), "+v"(stats.ret_sum), "+v"(stats.len_last), "+v"(stats.len_sum));
 
   const uint64_t t_end = t0 + (uint64_t)n_steps;
   for (uint64_t tb = t0 & ~(uint64_t)1; tb < t_end; tb += (uint64_t)tape_steps) {
@@ -703,6 +750,8 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
     wave_fence();
     const int k0 = tb < t0 ? 1 : 0;  // (the first block may start with a step of the launch before)
     const int k1 = (int)min((uint64_t)tape_steps, t_end - tb);
+    // (whether the end of an episode can mean more to these steps than its statistics)
+    const bool watch = EVENTS && (by_episode || __builtin_amdgcn_ballot_w64(episode >= budget - tape_steps) != 0ull);
     // (leaving the loop is the same for all lanes that are in it: an env that has used up its
     // budget ends the loop for its wave, and the others enter it again without it)
     for (int k = k0; k < k1;) {
@@ -713,17 +762,17 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
         uint32_t word = lds_address(tape) + 4u * (uint32_t)((kk << log_envs) + slot);
         const uint32_t first = *lds_at<uint32_t>(word);
         uint32_t named = (first & 0xffu) == mine ? c : 0xffffffffu;
-        unsigned long long explore = __builtin_amdgcn_ballot_w64(first < limit);
-        for (int end = k1; kk < end;) {
-          const int before = left;
-          won = row_pick_word<A>(q, unless, c, named, explore, word, 4u << log_envs, left);
-          const typename Mem::At at2 = mem.at(won & kMoveOffset);
+        unsigned long long explore = __builtin_amdgcn_ballot_w64(first < limit), last;
+        word += 4u << log_envs;
+        int end = k1, len = 0;
+        unsigned long long ends = 0ull;
+        float paid = -0.0f;  // (nothing to add yet)
+        do {
+          won = lanes_choose<A, EVENTS>(q, unless, c, named, explore, left, last, stats, paid, ends, len);
+          const typename Mem::At at2 = mem.at_word(won);
           const uint32_t cls = won & kMoveClass;
-          const bool hit = cls == (uint32_t)kGoal << 2;
-          left = hit ? 0 : left;
-          const bool ends = left <= 0;
-          typename Mem::At at_next = ends ? at_start : at2;
-          asm("" : "+v"(at_next));  // (one address, not one per use)
+          unsigned long long hit;
+          const typename Mem::At at_next = lanes_next(at2, at_start, cls, last, hit);
           const uint32_t code = mem.code(at_next);
           const float q2 = mem.value(at2);
           float q_next = mem.value(at_next);
@@ -742,10 +791,9 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
           }
           const uint32_t draw = *lds_at<uint32_t>(word);  // (the one behind the tape's end is not used)
           ++kk;
-          const bool me = c == won, stays = at_next == at;
-          const int len = whole - before + 1;
-          left = ends ? whole : left;
-          episode += ends ? 1 : 0;
+          const unsigned long long me = __builtin_amdgcn_ballot_w64(c == won), stays = __builtin_amdgcn_ballot_w64(at_next == at);
+          if (EVENTS) len = whole - left + 1;
+          ends = lanes_count(hit, last, whole, left, episode);
           // All of the above while the values are on their way.  (Without the barrier the move
           // word's arithmetic moves up and waits for its code before the other reads are asked
           // for: two trips to LDS in a row.  1M envs of 16x16 on LDS waves alone, with the codes
@@ -753,30 +801,32 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
           __builtin_amdgcn_sched_barrier(0);
           const uint32_t c_next = mem.word(at_next, code);
           if (CELLS) reward = (base_cells || (cls - 4u) < 8u) ? by_cell : reward;  // (goal or trap, or any)
-          if (EVENTS) {
-            ret = ret + reward;
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(ends) != 0ull, 0)) {
-              if (track) {
-                ret_last = ends ? ret : ret_last;
-                ret_sum = ends ? ret_sum + ret : ret_sum;
-                len_last = ends ? len : len_last;
-                len_sum += ends ? len : 0;
-              }
-              ret = ends ? 0.0f : ret;
+          if (EVENTS && watch) {
+            asm volatile("");  // (two branches: without `watch` nothing waits for the mask)
+            if (__builtin_expect(ends != 0ull, 0)) {
               if (by_episode) {
-                limit = ends ? tape_limit(eps_next) : limit;
+                limit = __builtin_amdgcn_inverse_ballot_w64(ends) ? tape_limit(eps_next) : limit;
                 eps_next = eps_of(R, P.eps_tab, t0, episode + 1);
               }
               if (__builtin_amdgcn_ballot_w64(episode >= budget) != 0ull) end = kk;
             }
           }
-          float m = row_top<A>(q2, floor, draw, limit, mine, c_next, named, explore);
-          m = hit ? 0.0f : m;
-          q = me ? td_value(q, reward, m, lr, gamma) : q;
-          mem.store(at, q);
-          q = stays ? q : q_next;
+          float q_new;
+          q = lanes_update<A>(q, q2, q_next, reward, hit, me, stays, lr, gamma, floor, draw, limit, mine, c_next, named,
+                              explore, word, 4u << log_envs, q_new);
+          mem.store(at, q_new);
           c = c_next;
           at = at_next;
+          paid = reward;
+        } while (kk < end);
+        if (EVENTS) {  // (the last step's)
+          const bool over = __builtin_amdgcn_inverse_ballot_w64(ends);
+          stats.ret = stats.ret + paid;
+          stats.ret_last = over ? stats.ret : stats.ret_last;
+          stats.ret_sum = over ? stats.ret_sum + stats.ret : stats.ret_sum;
+          stats.len_last = over ? len : stats.len_last;
+          stats.len_sum += over ? len : 0;
+          stats.ret = over ? 0.0f : stats.ret;
         }
         going = episode < budget;
       }
@@ -792,11 +842,11 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
     P.done[env] = (won & kMoveClass) == (uint32_t)kGoal << 2 ? 1 : 0;
     P.action[env] = (uint8_t)(won >> 29);
     if (track) {
-      P.ret_acc[env] = ret;
-      P.ret_last[env] = ret_last;
-      P.ret_sum[env] = ret_sum;
-      P.len_last[env] = len_last;
-      P.len_sum[env] = len_sum;
+      P.ret_acc[env] = stats.ret;
+      P.ret_last[env] = stats.ret_last;
+      P.ret_sum[env] = stats.ret_sum;
+      P.len_last[env] = stats.len_last;
+      P.len_sum[env] = stats.len_sum;
     }
   }
 }
