@@ -702,20 +702,32 @@ struct LaneCodes {
   __device__ __forceinline__ void store(At p, float v) const { *reinterpret_cast<float*>(values + (QL ? p : values_at + p)) = v; }
 };
 
-// The steps.  Every lane of the wave calls it; env e of the wave is lanes e A ... e A + A - 1
-// and `live` tells whether there is one.  The rewards by class - step, goal, trap, step - lie
+// Which of the wave's n_here envs (at most 1 << log_envs) a lane works for: env e is lanes
+// e A ... e A + A - 1, and what lanes are left do the same once more, to the same effect.  Waves
+// with up to 32 lanes switched off issue slower, and the slower the more of them a compute unit
+// has (measured; vector instructions alone, 4 lanes, one wave to a SIMD: up to three times the
+// cycles, 64 lanes: none): 1024 envs of 10x10, one to a wave, a step 616 -> 325 cycles;
+// 1000 of 128x128 with 8 actions and cell rewards 0.57 -> 0.35 us.
+template <int A>
+__device__ __forceinline__ int lane_slot(const int lane, const int log_envs, const int n_here) {
+  const int slot = (lane / A) & ((1 << log_envs) - 1);
+  return slot < n_here ? slot : 0;
+}
+
+// The steps.  Every lane of the wave calls it with its env's number in the wave (lane_slot).
+// The rewards by class - step, goal, trap, step - lie
 // at LDS address 0, where dynamic LDS starts in a kernel without any other; CELLS: `cell_rewards` of the env's cells also count.  EVENTS: an episode's end changes more
 // than where the env stands - epsilon by episode, episode statistics, an episode budget.
 // The row of the cell the move ends on (for the TD target) and that of the cell the env acts
 // from next - another one only where its episode ended - are asked for together.
 template <int A, bool CELLS, bool EVENTS, class Mem>
-__device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const int env0, const bool live,
+__device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const int env0, const int slot,
                                           const uint64_t t0, const int n_steps, const Mem mem, uint32_t* tape,
                                           const int log_envs, const int tape_steps,
                                           const float* __restrict__ cell_rewards) {
   const int lane = (int)__lane_id();
   const uint32_t mine = (uint32_t)lane & (A - 1);  // this lane's action
-  const int slot = live ? lane / A : 0, env = env0 + slot;
+  const int env = env0 + slot;
   int whole = R.episode_len > 0 ? R.episode_len : 0x7fffffff;
   asm("" : "+v"(whole));
   const float lr = R.lr, gamma = R.gamma;
@@ -735,7 +747,7 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
   LaneStats stats{0.0f, 0.0f, 0.0f, 0, 0};
   if (track) stats = LaneStats{P.ret_acc[env], P.ret_last[env], P.ret_sum[env], P.len_last[env], P.len_sum[env]};
   const int budget = EVENTS && R.max_episodes > 0 ? R.max_episodes : 0x7fffffff;
-  bool going = live && episode < budget;
+  bool going = episode < budget;
   float q = mem.value(at);
   uint32_t c = mem.word(at, mem.code(at));
   // (arrived before the loop starts: a value that may be in flight there makes every round
@@ -834,7 +846,7 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
     }
   }
 
-  if (live && mine == 0) {
+  if (lane == slot * A) {
     P.s[env] = (int)(mem.offset(at) / Mem::kRow);
     P.ep_step[env] = whole - left;
     P.episode[env] = episode;
@@ -955,16 +967,15 @@ __device__ __forceinline__ void fused_lds(const Rules& R, const Ptrs& P, const u
     }
   }
   wave_fence();
-  const int slot = lane / A;
-  const bool live = slot < n_here;
+  const int slot = lane_slot<A>(lane, log_envs, n_here);
   const uint32_t action = (uint32_t)lane & (A - 1);
-  unsigned char* mine = envs + (size_t)(live ? slot : 0) * env_bytes;
+  unsigned char* mine = envs + (size_t)slot * env_bytes;
   if (WORDS) {
-    run_lanes<A, false, EVENTS>(R, P, env0, live, t0, n_steps, LaneLds<A>{lds_address(mine) + 4 * action}, tape, log_envs, tape_steps, nullptr);
+    run_lanes<A, false, EVENTS>(R, P, env0, slot, t0, n_steps, LaneLds<A>{lds_address(mine) + 4 * action}, tape, log_envs, tape_steps, nullptr);
   } else {
     const unsigned char* codes = MAP_SHARED ? reinterpret_cast<const unsigned char*>(shared_codes) : mine + (size_t)S * kRow;
     const LaneCodes<A, true, true> mem{mine + 4 * action, 0u, codes, 0u, action, row_step<A>(R, action, kRow)};
-    run_lanes<A, false, EVENTS>(R, P, env0, live, t0, n_steps, mem, tape, log_envs, tape_steps, nullptr);
+    run_lanes<A, false, EVENTS>(R, P, env0, slot, t0, n_steps, mem, tape, log_envs, tape_steps, nullptr);
   }
   wave_fence();
   float* out = P.Q + (size_t)env0 * S * A;
@@ -1000,9 +1011,8 @@ __device__ __forceinline__ void fused_lanes_hbm(const Rules& R, const Ptrs& P, c
                                                 uint32_t* tape, const int log_envs, const int tape_steps) {
   constexpr uint32_t kRow = LaneCodes<A, false, CL>::kRow;
   const int lane = (int)__lane_id();
-  const int slot = lane / A;
-  const bool live = slot < min(1 << log_envs, P.N - env0);
-  const uint32_t at = live ? (uint32_t)slot : 0u, action = (uint32_t)lane & (A - 1);
+  const int slot = lane_slot<A>(lane, log_envs, P.N - env0);
+  const uint32_t at = (uint32_t)slot, action = (uint32_t)lane & (A - 1);
   const LaneCodes<A, false, CL> mem{reinterpret_cast<unsigned char*>(P.Q + (size_t)env0 * P.S * A),
                                     at * (uint32_t)P.S * kRow + 4u * action,
                                     CL ? codes + at * code_bytes : codes,
@@ -1010,9 +1020,9 @@ __device__ __forceinline__ void fused_lanes_hbm(const Rules& R, const Ptrs& P, c
                                     action, row_step<A>(R, action, kRow)};
   const float* cr = CELLS ? P.cell_reward + (P.map_shared ? 0 : (size_t)(env0 + at) * P.S) : nullptr;
   if (lane_events(R, P))
-    run_lanes<A, CELLS, true>(R, P, env0, live, t0, n_steps, mem, tape, log_envs, tape_steps, cr);
+    run_lanes<A, CELLS, true>(R, P, env0, slot, t0, n_steps, mem, tape, log_envs, tape_steps, cr);
   else
-    run_lanes<A, CELLS, false>(R, P, env0, live, t0, n_steps, mem, tape, log_envs, tape_steps, cr);
+    run_lanes<A, CELLS, false>(R, P, env0, slot, t0, n_steps, mem, tape, log_envs, tape_steps, cr);
 }
 
 // Per-env tables whose maps are shared (MAP = 1: the one map's move codes staged
@@ -1275,11 +1285,11 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
       float4* tables = reinterpret_cast<float4*>(P.Q + (size_t)env0 * table);
       strided_copy<true>(tables, (int)(table / 4), n_here, envs, env_bytes, lane);
       wave_fence();
-      const int slot = lane / A;
+      const int slot = lane_slot<A>(lane, log_envs, n_here);
       const uint32_t action = (uint32_t)lane & (A - 1);
-      unsigned char* mine = envs + (size_t)(slot < n_here ? slot : 0) * env_bytes;
+      unsigned char* mine = envs + (size_t)slot * env_bytes;
       const LaneCodes<A, true, true> mem{mine + 4 * action, 0u, mine + table * 4, 0u, action, row_step<A>(R, action, 4 * A)};
-      run_lanes<A, false, false>(R, P, env0, slot < n_here, t0, n_steps, mem,
+      run_lanes<A, false, false>(R, P, env0, slot, t0, n_steps, mem,
                                  reinterpret_cast<uint32_t*>(envs + ((size_t)env_bytes << log_envs)), log_envs, tape_steps, nullptr);
       wave_fence();
       strided_copy<false>(tables, (int)(table / 4), n_here, envs, env_bytes, lane);
