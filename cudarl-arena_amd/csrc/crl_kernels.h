@@ -11,6 +11,8 @@
 // Nothing here is a contraction, so there is no MFMA: every kernel is bound by
 // HBM traffic or by dependent-access latency.
 #pragma once
+#include <type_traits>
+
 #include "crl_device.h"
 #include "crl_reduce.h"
 
@@ -433,9 +435,9 @@ __device__ __forceinline__ void run_env_fast(const Rules& R, const Ptrs& P, cons
 
 // ---------------------------------------------------------------------------
 // One env to A lanes of a wave, a lane to an action, for batches that leave lanes to spare.
-// A lone wave issues an instruction every six cycles whatever its lanes do (measured: 2.4 GHz,
-// dependent or not), an LDS read is back after 50 and an L2 hit after 220, so a step's time
-// is mostly its number of instructions.  With an action to a lane the row is one register:
+// A lone wave issues an instruction every four cycles (measured: 2.4 GHz, dependent or not; a
+// taken branch costs 25 to 40), an LDS read is back after 50 and an L2 hit after 220, so a step's
+// time is mostly its number of instructions.  With an action to a lane the row is one register:
 //   - the maximum over the row is two (A = 8: three) cross-lane operations, and so is the
 //     choice of the first lane that holds it: every lane offers what its own action would do
 //     - action, resulting cell, class of the target, one word - and the smallest word of
@@ -444,7 +446,9 @@ __device__ __forceinline__ void run_env_fast(const Rules& R, const Ptrs& P, cons
 //     update on its own value, and all lanes write their values back;
 //   - the row of the start cell is read only in the steps in which an episode of the wave ends.
 // The exploration draws of the next steps are worked out ahead by all 64 lanes into a tape
-// in LDS (a Philox block is 75 instructions; with E envs to a wave a step's share is 75 E / 128).
+// in LDS (a block of two draws is some 80 instructions, 40 of them Philox; with E envs to a wave a
+// step's share is 80 E / 128).  A step with tables in LDS, episode statistics or none: one env to a
+// wave 270 cycles, four 310, 16 400.
 // ---------------------------------------------------------------------------
 
 // A word of the tape: explore iff it is below the env's limit, and then the action is its low
@@ -456,24 +460,43 @@ __device__ __forceinline__ uint32_t tape_limit(float eps) {
   return th >= (1u << 24) ? 0xffffffffu : th << 8;  // (no word with the upper 24 bits set has all the lower ones)
 }
 
+// Where the draws' limits of the next tape come from: one for all steps, or (epsilon by step) the
+// table's, asked for while the steps of the tape before are made.
+struct TapeLimits {
+  uint32_t below;
+  float eps[2][2];  // of this lane's pairs of steps
+  __device__ __forceinline__ void ask(const Rules& R, const Ptrs& P, const int log_envs, const uint64_t tb, const int lane) {
+    if (R.eps_mode != 1) return;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint64_t t = tb + 2u * (unsigned)((lane + 64 * j) >> log_envs);
+      eps[j][0] = eps_of(R, P.eps_tab, t, 0);
+      eps[j][1] = eps_of(R, P.eps_tab, t + 1, 0);
+    }
+  }
+};
+
 // The tape of steps [tb, tb + steps) of a wave's 1 << log_envs envs from env0 on, a Philox
-// block to a lane and pair of steps; tb and steps are even.  [step][env].
+// block to a lane and pair of steps; tb and steps are even, and there are at most two blocks to
+// a lane.  [step][env].
 template <int A>
-__device__ __forceinline__ void write_tape(const Rules& R, const Ptrs& P, const int env0, const int log_envs,
-                                           const uint64_t tb, const int steps, uint32_t* tape, const int lane) {
+__device__ __forceinline__ void write_tape(const Rules& R, const int env0, const int log_envs, const uint64_t tb,
+                                           const int steps, uint32_t* tape, const int lane, const TapeLimits& limits) {
   const int E = 1 << log_envs;
-  const bool by_episode = R.eps_mode >= 2;
-  for (int i = lane; i < (steps >> 1) << log_envs; i += 64) {
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int i = lane + 64 * j;
+    if (i >= (steps >> 1) << log_envs) break;
     const int e = i & (E - 1), b = i >> log_envs;
-    const uint64_t t = tb + (uint64_t)(2 * b);
-    const Philox4 blk = explore_block(R.seed, (uint32_t)(env0 + e), t >> 1);
+    const Philox4 blk = explore_block(R.seed, (uint32_t)(env0 + e), (tb >> 1) + (uint64_t)b);
     uint32_t w0 = below(blk.w1, (uint32_t)A), w1 = below(blk.w3, (uint32_t)A);
-    if (by_episode) {
+    if (R.eps_mode >= 2) {
       w0 |= blk.w0 & 0xffffff00u;
       w1 |= blk.w2 & 0xffffff00u;
     } else {
-      w0 = (blk.w0 >> 8) < explore_threshold(eps_of(R, P.eps_tab, t, 0)) ? w0 : kTapeGreedy;
-      w1 = (blk.w2 >> 8) < explore_threshold(eps_of(R, P.eps_tab, t + 1, 0)) ? w1 : kTapeGreedy;
+      const bool by_step = R.eps_mode == 1;
+      w0 = (blk.w0 >> 8) < (by_step ? explore_threshold(limits.eps[j][0]) : limits.below) ? w0 : kTapeGreedy;
+      w1 = (blk.w2 >> 8) < (by_step ? explore_threshold(limits.eps[j][1]) : limits.below) ? w1 : kTapeGreedy;
     }
     tape[((2 * b) << log_envs) + e] = w0;
     tape[((2 * b + 1) << log_envs) + e] = w1;
@@ -639,8 +662,9 @@ __device__ __forceinline__ unsigned long long lanes_count(unsigned long long hit
 }
 
 // What an action does from a cell, as one word: the action in the top three bits, the
-// resulting cell as the byte offset of its row (a multiple of 16), the class of the target
-// (kWall outside the grid) in bits 2 and 3.
+// resulting cell (where cell rewards count the target cell, whether the env gets there or not)
+// as the byte offset of its row (a multiple of 16), the class of the target (kWall outside the
+// grid) in bits 2 and 3.
 constexpr uint32_t kMoveOffset = 0x1ffffff0u, kMoveClass = 0xcu;
 __device__ __forceinline__ uint32_t move_word(uint32_t a, uint32_t offset, uint32_t cls) { return (a << 29) | offset | (cls << 2); }
 
@@ -661,7 +685,7 @@ struct LaneLds {
   uint32_t first;  // LDS address of the lane's value of the env's first cell
   using At = uint32_t;
   __device__ __forceinline__ At at(uint32_t offset) const { return first + offset; }
-  __device__ __forceinline__ At at_word(uint32_t word) const { return first + (word & kMoveOffset); }
+  __device__ __forceinline__ At at_word(uint32_t word, At) const { return first + (word & kMoveOffset); }
   __device__ __forceinline__ uint32_t offset(At p) const { return p - first; }
   static __device__ __forceinline__ float value(At p) { return *lds_at<float>(p); }
   // asks for what `word` needs / the lane's move word from that, when it has arrived
@@ -673,7 +697,8 @@ struct LaneLds {
 // Values in LDS (QL) or in HBM and the caches, the cells' move codes in LDS (CL) or global
 // memory, a byte per cell (two with 8 actions): the move word is worked out when the code
 // has arrived, four or five instructions.
-template <int A, bool QL, bool CL>
+// TARGET: the words name the target cell.
+template <int A, bool QL, bool CL, bool TARGET>
 struct LaneCodes {
   static constexpr uint32_t kRow = 4 * A;
   unsigned char* values;       // QL: the lane's value of the env's first cell; else the wave's first table
@@ -684,7 +709,10 @@ struct LaneCodes {
   int step;                    // bytes from a row to the one the lane's action leads to
   using At = uint32_t;
   __device__ __forceinline__ At at(uint32_t offset) const { return offset; }
-  __device__ __forceinline__ At at_word(uint32_t word) const { return word & kMoveOffset; }
+  __device__ __forceinline__ At at_word(uint32_t word, At at) const {
+    const uint32_t there = word & kMoveOffset;
+    return TARGET && (word & 8u) != 0u ? at : there;  // (classes from kTrap on leave the env where it is)
+  }
   __device__ __forceinline__ uint32_t offset(At p) const { return p; }
   __device__ __forceinline__ float value(At p) const { return *reinterpret_cast<const float*>(values + (QL ? p : values_at + p)); }
   __device__ __forceinline__ uint32_t code(At p) const {
@@ -692,8 +720,9 @@ struct LaneCodes {
     return A == 4 ? (uint32_t)codes[i] : (uint32_t)*reinterpret_cast<const uint16_t*>(codes + i);
   }
   __device__ __forceinline__ uint32_t word(At p, uint32_t code) const {
-    // (classes from kTrap on leave the env where it is: that is the class's upper bit)
     const uint32_t cls = __builtin_amdgcn_ubfe(code, 2 * action, 2u);
+    if (TARGET) return ((p + (uint32_t)step) & kMoveOffset) | ((cls << 2) | (action << 29));
+    // (a class's upper bit: the env stays where it is)
     const uint32_t there = p + (uint32_t)step + (action << 29);
     const uint32_t w = QL ? there - (uint32_t)__mul24((int)__builtin_amdgcn_ubfe(code, 2 * action + 1, 1u), step)  // (a table in LDS is small)
                           : there - ((uint32_t)__builtin_amdgcn_sbfe((int)code, 2 * action + 1, 1u) & (uint32_t)step);
@@ -716,7 +745,7 @@ __device__ __forceinline__ int lane_slot(const int lane, const int log_envs, con
 
 // The steps.  Every lane of the wave calls it with its env's number in the wave (lane_slot).
 // The rewards by class - step, goal, trap, step - lie
-// at LDS address 0, where dynamic LDS starts in a kernel without any other; CELLS: `cell_rewards` of the env's cells also count.  EVENTS: an episode's end changes more
+// at LDS address 0, where dynamic LDS starts in a kernel without any other; CELLS: `cell_rewards` of the cells of the wave's first env (or of the shared map) also count.  EVENTS: an episode's end changes more
 // than where the env stands - epsilon by episode, episode statistics, an episode budget.
 // The row of the cell the move ends on (for the TD target) and that of the cell the env acts
 // from next - another one only where its episode ended - are asked for together.
@@ -742,6 +771,7 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
   uint32_t won = ((uint32_t)P.action[env] << 29) | (P.done[env] != 0 ? (uint32_t)kGoal << 2 : 0u);  // the last step's word
   const bool by_episode = EVENTS && R.eps_mode >= 2, track = EVENTS && P.ret_acc != nullptr;
   const bool base_cells = CELLS && (R.reward_flags & 2) != 0;
+  const uint32_t rewards_at = CELLS && !P.map_shared ? (uint32_t)slot * (uint32_t)P.S * 4u : 0u;
   uint32_t limit = by_episode ? tape_limit(eps_of(R, P.eps_tab, t0, episode)) : kTapeLimit;
   float eps_next = by_episode ? eps_of(R, P.eps_tab, t0, episode + 1) : 0.0f;  // of the next episode: asked for ahead
   LaneStats stats{0.0f, 0.0f, 0.0f, 0, 0};
@@ -756,14 +786,17 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
   if (EVENTS) asm volatile("" : "+v"(stats.ret), "+v"(stats.ret_last), "+v"(stats.ret_sum), "+v"(stats.len_last), "+v"(stats.len_sum));
 
   const uint64_t t_end = t0 + (uint64_t)n_steps;
+  TapeLimits limits{explore_threshold(R.eps0), {}};
+  limits.ask(R, P, log_envs, t0 & ~(uint64_t)1, lane);
   for (uint64_t tb = t0 & ~(uint64_t)1; tb < t_end; tb += (uint64_t)tape_steps) {
     wave_fence();
-    write_tape<A>(R, P, env0, log_envs, tb, tape_steps, tape, lane);
+    write_tape<A>(R, env0, log_envs, tb, tape_steps, tape, lane, limits);
     wave_fence();
+    limits.ask(R, P, log_envs, tb + (uint64_t)tape_steps, lane);
     const int k0 = tb < t0 ? 1 : 0;  // (the first block may start with a step of the launch before)
     const int k1 = (int)min((uint64_t)tape_steps, t_end - tb);
-    // (whether the end of an episode can mean more to these steps than its statistics)
-    const bool watch = EVENTS && (by_episode || __builtin_amdgcn_ballot_w64(episode >= budget - tape_steps) != 0ull);
+    // (whether an env can use up its budget in these steps)
+    const bool close = EVENTS && __builtin_amdgcn_ballot_w64(episode >= budget - tape_steps) != 0ull;
     // (leaving the loop is the same for all lanes that are in it: an env that has used up its
     // budget ends the loop for its wave, and the others enter it again without it)
     for (int k = k0; k < k1;) {
@@ -779,9 +812,9 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
         int end = k1, len = 0;
         unsigned long long ends = 0ull;
         float paid = -0.0f;  // (nothing to add yet)
-        do {
+        auto step = [&](auto by_end, auto by_budget) {
           won = lanes_choose<A, EVENTS>(q, unless, c, named, explore, left, last, stats, paid, ends, len);
-          const typename Mem::At at2 = mem.at_word(won);
+          const typename Mem::At at2 = mem.at_word(won, at);
           const uint32_t cls = won & kMoveClass;
           unsigned long long hit;
           const typename Mem::At at_next = lanes_next(at2, at_start, cls, last, hit);
@@ -792,17 +825,12 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
           float by_cell = 0.0f;
           if (CELLS) {
             // the goal pays on the goal cell (where the move ends), a trap on the cell it
-            // guards, anything else where the move ends
-            int pays = (int)(mem.offset(at2) / Mem::kRow);
-            if (__builtin_amdgcn_ballot_w64(cls == (uint32_t)kTrap << 2) != 0ull) {
-              int dx, dy;
-              action_delta((int)(won >> 29), A, dx, dy);
-              pays = cls == (uint32_t)kTrap << 2 ? pays + __mul24(dy, R.W) + dx : pays;
-            }
-            by_cell = cell_rewards[pays];
+            // guards, anything else where the move ends: that is the target but for a wall
+            const uint32_t pays = cls == kMoveClass ? mem.offset(at) : won & kMoveOffset;
+            by_cell = *reinterpret_cast<const float*>(reinterpret_cast<const unsigned char*>(cell_rewards) +
+                                                      (rewards_at + pays / (Mem::kRow / 4)));
           }
           const uint32_t draw = *lds_at<uint32_t>(word);  // (the one behind the tape's end is not used)
-          ++kk;
           const unsigned long long me = __builtin_amdgcn_ballot_w64(c == won), stays = __builtin_amdgcn_ballot_w64(at_next == at);
           if (EVENTS) len = whole - left + 1;
           ends = lanes_count(hit, last, whole, left, episode);
@@ -813,14 +841,13 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
           __builtin_amdgcn_sched_barrier(0);
           const uint32_t c_next = mem.word(at_next, code);
           if (CELLS) reward = (base_cells || (cls - 4u) < 8u) ? by_cell : reward;  // (goal or trap, or any)
-          if (EVENTS && watch) {
-            asm volatile("");  // (two branches: without `watch` nothing waits for the mask)
+          if constexpr (decltype(by_end)::value) {
             if (__builtin_expect(ends != 0ull, 0)) {
               if (by_episode) {
                 limit = __builtin_amdgcn_inverse_ballot_w64(ends) ? tape_limit(eps_next) : limit;
                 eps_next = eps_of(R, P.eps_tab, t0, episode + 1);
               }
-              if (__builtin_amdgcn_ballot_w64(episode >= budget) != 0ull) end = kk;
+              if (decltype(by_budget)::value && __builtin_amdgcn_ballot_w64(episode >= budget) != 0ull) end = kk + 1;
             }
           }
           float q_new;
@@ -830,7 +857,26 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
           c = c_next;
           at = at_next;
           paid = reward;
-        } while (kk < end);
+          ++kk;
+        };
+        auto steps = [&](auto by_end) {  // (a taken branch and the moves before it are a tenth of a step)
+          constexpr std::false_type no{};
+          while (kk + 4 <= end) {
+            step(by_end, no);
+            step(by_end, no);
+            step(by_end, no);
+            step(by_end, no);
+          }
+          while (kk < end) step(by_end, no);
+        };
+        if (EVENTS && close) {
+          do step(std::true_type{}, std::true_type{});
+          while (kk < end);
+        } else if (EVENTS && by_episode) {
+          steps(std::true_type{});
+        } else {
+          steps(std::false_type{});
+        }
         if (EVENTS) {  // (the last step's)
           const bool over = __builtin_amdgcn_inverse_ballot_w64(ends);
           stats.ret = stats.ret + paid;
@@ -901,7 +947,7 @@ template <int A, bool MAP_SHARED, bool WORDS, bool EVENTS>
 __device__ __forceinline__ void fused_lds(const Rules& R, const Ptrs& P, const uint64_t t0, const int n_steps,
                                           const int log_envs, const int env_bytes, const int tape_steps) {
   extern __shared__ __align__(16) unsigned char lds_bytes[];
-  constexpr uint32_t kRow = WORDS ? LaneLds<A>::kRow : LaneCodes<A, true, true>::kRow;
+  constexpr uint32_t kRow = WORDS ? LaneLds<A>::kRow : LaneCodes<A, true, true, false>::kRow;
   const int lane = threadIdx.x;
   const int E = 1 << log_envs;
   const int env0 = blockIdx.x << log_envs;
@@ -974,7 +1020,7 @@ __device__ __forceinline__ void fused_lds(const Rules& R, const Ptrs& P, const u
     run_lanes<A, false, EVENTS>(R, P, env0, slot, t0, n_steps, LaneLds<A>{lds_address(mine) + 4 * action}, tape, log_envs, tape_steps, nullptr);
   } else {
     const unsigned char* codes = MAP_SHARED ? reinterpret_cast<const unsigned char*>(shared_codes) : mine + (size_t)S * kRow;
-    const LaneCodes<A, true, true> mem{mine + 4 * action, 0u, codes, 0u, action, row_step<A>(R, action, kRow)};
+    const LaneCodes<A, true, true, false> mem{mine + 4 * action, 0u, codes, 0u, action, row_step<A>(R, action, kRow)};
     run_lanes<A, false, EVENTS>(R, P, env0, slot, t0, n_steps, mem, tape, log_envs, tape_steps, nullptr);
   }
   wave_fence();
@@ -1009,16 +1055,16 @@ template <int A, bool CELLS, bool CL>
 __device__ __forceinline__ void fused_lanes_hbm(const Rules& R, const Ptrs& P, const int env0, const uint64_t t0,
                                                 const int n_steps, const unsigned char* codes, const uint32_t code_bytes,
                                                 uint32_t* tape, const int log_envs, const int tape_steps) {
-  constexpr uint32_t kRow = LaneCodes<A, false, CL>::kRow;
+  constexpr uint32_t kRow = LaneCodes<A, false, CL, CELLS>::kRow;
   const int lane = (int)__lane_id();
   const int slot = lane_slot<A>(lane, log_envs, P.N - env0);
   const uint32_t at = (uint32_t)slot, action = (uint32_t)lane & (A - 1);
-  const LaneCodes<A, false, CL> mem{reinterpret_cast<unsigned char*>(P.Q + (size_t)env0 * P.S * A),
+  const LaneCodes<A, false, CL, CELLS> mem{reinterpret_cast<unsigned char*>(P.Q + (size_t)env0 * P.S * A),
                                     at * (uint32_t)P.S * kRow + 4u * action,
                                     CL ? codes + at * code_bytes : codes,
                                     CL ? 0u : at * code_bytes,
                                     action, row_step<A>(R, action, kRow)};
-  const float* cr = CELLS ? P.cell_reward + (P.map_shared ? 0 : (size_t)(env0 + at) * P.S) : nullptr;
+  const float* cr = CELLS ? P.cell_reward + (P.map_shared ? 0 : (size_t)env0 * P.S) : nullptr;  // of the wave's first env
   if (lane_events(R, P))
     run_lanes<A, CELLS, true>(R, P, env0, slot, t0, n_steps, mem, tape, log_envs, tape_steps, cr);
   else
@@ -1090,9 +1136,9 @@ __global__ __launch_bounds__(256) void k_fused_per_env(const Rules R, const Ptrs
 // The same with per-env maps: one wave to a workgroup, which draws 1 << log_envs envs at a
 // time from a ticket counter (or is dealt them by position: fixed_tickets), stages their move
 // codes into its LDS and steps them for all n_steps, A lanes to an env.  What bounds it is the
-// wave's dependent chain - 50 vector instructions a step with four envs to a wave, 60 with 16 (by the
-// counters, tape and all), and a trip to the row, 0.28 us per step with a wave to a compute unit -
-// of which a wave with 64 envs pays the slowest of 64 trips and 150 instructions.
+// wave's dependent chain - some 60 instructions a step, the tape's not counted, and a trip to the row,
+// 0.26 us per step of 4096 envs on 32x32 maps - of which a wave with 64 envs pays the slowest of 64
+// trips and 150 instructions.
 // LDS: the rewards by class, the tape, the codes env by env.
 template <int A, bool CELLS>
 __global__ __launch_bounds__(64) void k_fused_lanes(const Rules R, const Ptrs P, const uint64_t t0, const int n_steps,
@@ -1288,7 +1334,7 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
       const int slot = lane_slot<A>(lane, log_envs, n_here);
       const uint32_t action = (uint32_t)lane & (A - 1);
       unsigned char* mine = envs + (size_t)slot * env_bytes;
-      const LaneCodes<A, true, true> mem{mine + 4 * action, 0u, mine + table * 4, 0u, action, row_step<A>(R, action, 4 * A)};
+      const LaneCodes<A, true, true, false> mem{mine + 4 * action, 0u, mine + table * 4, 0u, action, row_step<A>(R, action, 4 * A)};
       run_lanes<A, false, false>(R, P, env0, slot, t0, n_steps, mem,
                                  reinterpret_cast<uint32_t*>(envs + ((size_t)env_bytes << log_envs)), log_envs, tape_steps, nullptr);
       wave_fence();
