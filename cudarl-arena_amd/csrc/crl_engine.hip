@@ -694,10 +694,11 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
     return;
   }
   if (p.tickets) {
-    // (tickets dealt by position use no counter; the kernel itself notes who did how much)
+    // (tickets dealt by position use no counter; the kernel itself notes who did how much, and
+    // where it is kept: a launch to copy three words was 3 to 5 us of a call)
     if (!p.fixed) hipLaunchKernelGGL(crl::k_fill_u32, dim3(1), dim3(64), 0, e->stream, e->tk, 0u, 3);
     const dim3 g(p.grid), b(p.block);
-    unsigned* tk = e->tk;
+    unsigned* tk = p.fixed ? e->split.p : e->tk;
 #define CRL_LAUNCH_TICKETS(MODE, LDSW, MOVES)                                                       \
   hipLaunchKernelGGL((crl::k_fused_tickets<A, MODE, LDSW, MOVES>), g, b, p.lds, e->stream, R, P, t0, n, \
                      tk, p.tab_stride, p.fixed ? 1 : 0, p.tape_steps, p.lds_waves, p.env_bytes)
@@ -1858,7 +1859,7 @@ int run_fused(crl_engine* e, int32_t n_steps, bool no_alloc) {
     else
       launch_fused_a<8>(e, p, e->t, n_steps);
     HIP_TRY(hipGetLastError());
-    if (p.tickets) {
+    if (p.tickets && !p.fixed) {
       // the counters may sit in the scratch all engines of this GPU share: kept here
       hipLaunchKernelGGL(crl::k_copy3_u32, dim3(1), dim3(64), 0, e->stream, e->tk, e->split.p);
       HIP_TRY(hipGetLastError());

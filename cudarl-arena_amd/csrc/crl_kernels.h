@@ -812,7 +812,7 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
         int end = k1, len = 0;
         unsigned long long ends = 0ull;
         float paid = -0.0f;  // (nothing to add yet)
-        auto step = [&](auto by_end, auto by_budget) {
+        auto step = [&](auto by_end, auto by_budget) __attribute__((always_inline)) {
           won = lanes_choose<A, EVENTS>(q, unless, c, named, explore, left, last, stats, paid, ends, len);
           const typename Mem::At at2 = mem.at_word(won, at);
           const uint32_t cls = won & kMoveClass;
@@ -1240,7 +1240,7 @@ __device__ __forceinline__ void strided_copy(T* __restrict__ g, const int per, c
   const int total = n * per;
   const int de = 64 / per, dp = 64 - de * per;  // 64 pieces on: that many envs and pieces
   int e = lane / per, piece = lane - e * per;
-  constexpr int kFlight = 8;
+  constexpr int kFlight = 16;  // (1M envs of 16x16, 1000 steps: 8 / 16 / 32 10.71 / 10.59 / 11.05 ms)
   for (int i0 = lane; i0 < total; i0 += 64 * kFlight) {
     T v[kFlight];
     T* at[kFlight];
