@@ -116,6 +116,8 @@ struct PersistBufs {
 __device__ __forceinline__ unsigned long long tagged(uint32_t bits, uint32_t tag) {
   return (unsigned long long)bits | ((unsigned long long)tag << 32);
 }
+// a | (b ^ c)
+__device__ __forceinline__ uint32_t or_xor(uint32_t a, uint32_t b, uint32_t c) { return __builtin_amdgcn_bitop3_b32(a, b, c, 0xf6); }
 __device__ __forceinline__ uint32_t tag_of(unsigned long long v) { return (uint32_t)(v >> 32); }
 __device__ __forceinline__ float value_of(unsigned long long v) { return __uint_as_float((uint32_t)v); }
 
@@ -514,11 +516,12 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
             rn[i + 1] = tagged(r.z, r.w);
           }
         }
-        ok = true;
-        if (live) {
+        // (one value, one comparison: what is wrong with the tags.  A chain of conditions becomes a
+        // chain of branches, which nothing hides here.)
+        uint32_t wrong = 0;
 #pragma unroll
-          for (int i = 0; i < A; ++i) ok = ok && tag_of(rq[i]) == want && tag_of(rn[i]) == want;
-        }
+        for (int i = 0; i < A; ++i) wrong = or_xor(or_xor(wrong, tag_of(rq[i]), want), tag_of(rn[i]), want);
+        ok = !live || wrong == 0u;
         if (!ok && (++spins >= spin_limit || ((spins & 63) == 0 && ld_dev32(B.err) != 0u))) {
           L.dead = 1;
           break;
@@ -645,20 +648,21 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
           for (int j = 0; j < GS; ++j) rec[j] = ld_dev128(w_cells, src[j]);
 #pragma unroll
           for (int j = 0; j < GS; ++j) more[j] = ld_dev128(w_cells, src_more[j]);
-          bool ok = true;
+          uint32_t wrong = 0;
+          const uint32_t tags = want << R64::kTagShift;
 #pragma unroll
           for (int j = 0; j < GS; ++j) {
             // (record 0 of the cell is in the even lane of the two: a move within the quad)
             const uint32_t meta0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)rec[j].x, 0xa0, 0xf, 0xf, true);
             cnt[j] = R64::count(meta0);
-            // (every record of a main half is written every step)
-            bool mine = R64::tag(meta0) == want && R64::tag(rec[j].x) == want && R64::tag(rec[j].z) == want;
-            if (cnt[j] != kSlotOverflow) {  // (an extension record: only where the count says so)
-              mine = mine && (kMainRecs + 2 * pair >= cnt[j] || R64::tag(more[j].x) == want) &&
-                     (kMainRecs + 2 * pair + 1 >= cnt[j] || R64::tag(more[j].z) == want);
-            }
-            ok = ok && mine;
+            // (every record of a main half is written every step, an extension's only where the
+            // count says so)
+            const int more_n = (cnt[j] == kSlotOverflow ? 0 : cnt[j]) - kMainRecs - 2 * pair;
+            wrong = or_xor(or_xor(or_xor(wrong, meta0, tags), rec[j].x, tags), rec[j].z, tags);
+            wrong = or_xor(wrong, more_n > 0 ? more[j].x : tags, tags);
+            wrong = or_xor(wrong, more_n > 1 ? more[j].z : tags, tags);
           }
+          const bool ok = wrong < 1u << R64::kTagShift;
           if (__all(ok)) break;
           if (++spins >= spin_limit || ((spins & 63) == 0 && ld_dev32(B.err) != 0u)) {
             L.dead = 1;
