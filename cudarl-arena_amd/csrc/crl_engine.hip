@@ -1134,7 +1134,7 @@ hipError_t launch_persist_kernel(crl_engine* e, const PersistPlan& p, unsigned l
                                  int n_steps, uint32_t tag0, int trace_row0) {
   crl::Rules R = e->rules();
   crl::Ptrs P = e->ptrs();
-  crl::ReduceGeom G = p.G;
+  int n_keys = p.G.K;
   crl::PersistBufs B{};
   B.table = buf + p.at_table;
   B.raw = buf + p.at_raw;
@@ -1142,7 +1142,7 @@ hipError_t launch_persist_kernel(crl_engine* e, const PersistPlan& p, unsigned l
   B.err = reinterpret_cast<unsigned*>(e->pdiag.p);
   B.clocks = e->pdiag.p + 1;
   int spin_limit = e->persist_spin_limit;
-  void* args[] = {&R, &P, &t0, &n_steps, &tag0, &trace_row0, &G, &B, &spin_limit};
+  void* args[] = {&R, &P, &t0, &n_steps, &tag0, &trace_row0, &n_keys, &B, &spin_limit};
   // a cooperative launch is refused unless all workgroups can be resident together,
   // which the kernel's waits rely on
   return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&crl::k_shared_persist<A, MAP, CLK, FOLD, HASHED>), dim3(p.grid),

@@ -320,8 +320,7 @@ __device__ __forceinline__ bool add_records(PersistLdsHashed& L, const ReduceGeo
 
 // MAP = 1: the shared map staged in LDS; MAP = 2: maps read from global memory
 // (they do not change during a launch, so plain loads are fine).
-// G.own_shift = kPersistOwnShift, G.n_blocks = 256 = the number of workgroups (blocks
-// without envs hand over empty cells).
+// 256 workgroups (blocks without envs hand over empty cells), n_keys keys.
 // Everything in B holds tags of at most tag0 at launch, *B.err is zero.
 // FOLD = the rules of the common configuration are compile-time facts (goal test on the
 // target cell, restart at the end of an episode, true maximum, rewards by class, no trace,
@@ -331,7 +330,7 @@ __device__ __forceinline__ bool add_records(PersistLdsHashed& L, const ReduceGeo
 template <int A, int MAP, bool CLK, bool FOLD, bool HASHED>
 __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptrs P, const uint64_t t0,
                                                          const int n_steps, const uint32_t tag0,
-                                                         const int trace_row0, const ReduceGeom G, const PersistBufs B,
+                                                         const int trace_row0, const int n_keys, const PersistBufs B,
                                                          const int spin_limit) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   using Lds = PersistLdsOf<HASHED>;
@@ -340,6 +339,9 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
   static_assert(sizeof(Lds) % 16 == 0, "16-byte LDS accesses");
   static_assert(kSortBytes <= sizeof(PersistLds::tile) / 2, "the holders' line-up borrows the upper half of the tile");
   uint32_t* lds_map = reinterpret_cast<uint32_t*>(lds_raw + sizeof(Lds));
+  // (shifts that are known here are no scalar registers to run out of)
+  constexpr int kAShift = A == 8 ? 3 : 2;
+  const ReduceGeom G{n_keys, kAShift, kPersistOwnShift, kPersistMaxGroups, kMainShift + 1, kMainShift};
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -478,6 +480,11 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
   };
 
   const int live_groups = (P.N + kBlockSamples * kGroupBlocks - 1) / (kBlockSamples * kGroupBlocks);
+  // (in vector registers: as scalars, or as conditions that hold for the launch, they do not fit and
+  // are fetched back in every step)
+  int whole = R.episode_len > 0 ? R.episode_len : 0x7fffffff;
+  float r_step = R.step_reward, r_goal = R.goal_reward, r_trap = R.trap_reward;
+  asm volatile("" : "+v"(whole), "+v"(r_step), "+v"(r_goal), "+v"(r_trap));
   unsigned long long phase_[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   unsigned long long last_ = CLK ? clock64() : 0ull;
   bool gave_up = false;
@@ -565,7 +572,7 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
       const bool trap = code == kTrap;
       const int s2 = moved ? tgt : s0;
       const bool hit = (FOLD || R.goal_mode == 0) ? code == kGoal : ((moved ? code : cls0) == kGoal);
-      const float by_class = hit ? R.goal_reward : trap ? R.trap_reward : R.step_reward;
+      const float by_class = hit ? r_goal : trap ? r_trap : r_step;
       float by_cell = 0.0f;
       if (cells_flag) by_cell = cr[(trap && !hit) ? tgt : s2];
       reward = (cells_flag && (hit || trap || base_cells)) ? by_cell : by_class;
@@ -588,7 +595,7 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
       }
       ep_step += 1;
       ret = ret + reward;
-      const bool over_now = (FOLD || R.auto_reset) && (done || (R.episode_len > 0 && ep_step >= R.episode_len));
+      const bool over_now = (FOLD || R.auto_reset) && (done || ep_step >= whole);
       if (!FOLD && track && over_now) record_episode(P, env, ret, ep_step);
       ret = over_now ? 0.0f : ret;
       s = over_now ? start : s2;

@@ -169,6 +169,7 @@ struct alignas(16) ReduceLdsT {  // (lead and members are also accessed 16 bytes
   float delta[kBlockSamples];
   int handed[256];                               // block sums handed to each owner (one-launch kernel)
   int over;                                      // some owner was handed more than a cell holds
+  int none;                                      // (written by the others; nobody reads it)
 };
 using ReduceLds = ReduceLdsT<kDenseKeys>;
 
@@ -316,7 +317,7 @@ __device__ __forceinline__ bool reduce_block(ReduceLdsT<Entries>& L, const Reduc
   if (leader) {
     owner = owner_of(key, G);
     slot = atomicAdd(&L.handed[owner], 1);  // slot order is free: records carry the key
-    if (slot >= cap) L.over = 1;
+    *(slot >= cap ? &L.over : &L.none) = 1;
     if (HASHED) keys[at] = -1;
     // (record 0's count is added on the way out, when every leader has drawn its slot)
     if (slot < cap_main) stage[(owner << G.main_shift) + slot] = Rec<HASHED>::make((uint32_t)slot_of(key, G), tag, acc);
