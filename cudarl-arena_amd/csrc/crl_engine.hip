@@ -1716,21 +1716,29 @@ int refuse_capture(const crl_engine* e) {
   return fail(CRL_E_DEVICE, "a call that takes host data cannot be recorded: its stream is being captured");
 }
 
+// Bytes of a packed transition: the key, s' and done fit one word where a key has 16 bits and s' 15.
+size_t sample_bytes(const crl_engine* e) { return e->K < 0xffffu ? 8 : 12; }
+
 // Transitions [at, at + n) of a call packed into a page.
 int pack_page(const crl_engine* e, size_t at, int n, const int32_t* s, const int32_t* a, const float* r,
               const int32_t* s_next, const uint8_t* done, unsigned char* page, crl::PackedSamples* X) {
   int32_t* key = reinterpret_cast<int32_t*>(page);
-  uint32_t* s2d = reinterpret_cast<uint32_t*>(key + n);
-  if (!crl::pack_transitions(n, (int)e->S, e->A, s + at, a + at, s_next + at, done + at, key, s2d))
+  const bool two_words = sample_bytes(e) == 8;
+  uint32_t* s2d = two_words ? nullptr : reinterpret_cast<uint32_t*>(key + n);
+  const bool fine = two_words ? crl::pack_transitions_short(n, (int)e->S, e->A, s + at, a + at, s_next + at, done + at,
+                                                            reinterpret_cast<uint32_t*>(page))
+                              : crl::pack_transitions(n, (int)e->S, e->A, s + at, a + at, s_next + at, done + at, key, s2d);
+  if (!fine)
     for (size_t i = at; i < at + n; ++i) {
       if (s[i] < 0 || (size_t)s[i] >= e->S) return fail(CRL_E_RANGE, "s[%zu] = %d outside [0,%zu)", i, s[i], e->S);
       if (s_next[i] < 0 || (size_t)s_next[i] >= e->S)
         return fail(CRL_E_RANGE, "s_next[%zu] = %d outside [0,%zu)", i, s_next[i], e->S);
     }
-  std::memcpy(s2d + n, r + at, (size_t)n * 4);
+  float* rewards = reinterpret_cast<float*>(key + (two_words ? n : 2 * (size_t)n));
+  std::memcpy(rewards, r + at, (size_t)n * 4);
   X->key = key;
   X->s2d = s2d;
-  X->r = reinterpret_cast<const float*>(s2d + n);
+  X->r = rewards;
   return CRL_OK;
 }
 
@@ -1754,7 +1762,7 @@ int td_pieces(crl_engine* e, float* Q, int n, const int32_t* s, const int32_t* a
     const int m = (int)std::min(even, n - at);
     crl_engine::InSlot* slot;
     crl::PackedSamples X;
-    rc = claim_in_slot(e, 12 * even, &slot);
+    rc = claim_in_slot(e, sample_bytes(e) * even, &slot);
     if (rc == CRL_OK) rc = pack_page(e, at, m, s, a, r, s_next, done, slot->page, &X);
     if (rc) return rc;
     const crl::HostSignal sig = read();
@@ -1770,7 +1778,7 @@ int td_pieces(crl_engine* e, float* Q, int n, const int32_t* s, const int32_t* a
 }
 
 // crl_td_update and, with `keys`, crl_td_update_collect.  The transitions are packed into
-// pinned memory, 12 bytes each, in the pass that checks them, and the kernel reads them
+// pinned memory, 8 or 12 bytes each, in the pass that checks them, and the kernel reads them
 // there: the call returns without waiting for anything (65,536 transitions: five copies from
 // pageable memory and a wait took 125 us).
 int td_update(crl_engine* e, int32_t table, int32_t n, const int32_t* s, const int32_t* a, const float* r,
@@ -1793,7 +1801,7 @@ int td_update(crl_engine* e, int32_t table, int32_t n, const int32_t* s, const i
   }
   crl_engine::InSlot* slot;
   crl::PackedSamples X;
-  rc = claim_in_slot(e, 12 * (size_t)n, &slot);
+  rc = claim_in_slot(e, sample_bytes(e) * (size_t)n, &slot);
   if (rc == CRL_OK) rc = pack_page(e, 0, n, s, a, r, s_next, done, slot->page, &X);
   if (rc) return rc;
   int2* changed = nullptr;

@@ -114,6 +114,22 @@ bool pack_transitions(int n, int S, int A, const int32_t* s, const int32_t* a, c
   return bad == 0;
 }
 
+#if defined(__x86_64__) && !defined(__SANITIZE_ADDRESS__)
+__attribute__((target_clones("avx512f", "avx2", "default")))
+#endif
+bool pack_transitions_short(int n, int S, int A, const int32_t* s, const int32_t* a, const int32_t* s_next,
+                            const uint8_t* done, uint32_t* words) {
+  const int shift = A == 8 ? 3 : 2;
+  uint32_t bad = 0;
+  for (int i = 0; i < n; ++i) {
+    bad |= (uint32_t)((uint32_t)s[i] >= (uint32_t)S) | (uint32_t)((uint32_t)s_next[i] >= (uint32_t)S);
+    const uint32_t outside = (uint32_t)a[i] < (uint32_t)A ? 0u : 0xffffu;
+    const uint32_t k = ((uint32_t)s[i] << shift) | ((uint32_t)a[i] & (uint32_t)(A - 1)) | outside;
+    words[i] = k | ((uint32_t)s_next[i] << 16) | (done[i] != 0 ? 0x80000000u : 0u);
+  }
+  return bad == 0;
+}
+
 namespace {
 
 // word `i` of the stream (seed; a, stream id): counter (a, id, i/4, 0), lane i%4

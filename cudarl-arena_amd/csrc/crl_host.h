@@ -31,5 +31,9 @@ void pack_classes(const uint8_t* cls, size_t n_cells, uint32_t* words);
 // was written is then worthless.  A is 4 or 8, S at most 2^24.
 bool pack_transitions(int n, int S, int A, const int32_t* s, const int32_t* a, const int32_t* s_next,
                       const uint8_t* done, int32_t* key, uint32_t* s2d);
+// The same in one word each: key in bits 0..15 (all ones: an action outside [0, A)), s' in bits
+// 16..30, done in bit 31.  S * A is below 65535.
+bool pack_transitions_short(int n, int S, int A, const int32_t* s, const int32_t* a, const int32_t* s_next,
+                            const uint8_t* done, uint32_t* words);
 
 }  // namespace crl
