@@ -279,6 +279,11 @@ __device__ __forceinline__ float eps_of(const Rules& R, const float* __restrict_
   return tab[i];
 }
 
+// The same with eps_mode >= 2, where a step of a loop asks: no branch, 32 bits.
+__device__ __forceinline__ float eps_of_episode(const Rules& R, const float* __restrict__ tab, int episode) {
+  return tab[min(max(episode, 0), R.eps_len - 1)];
+}
+
 // How a launch tells the host that it is through: the last workgroup stores `seq` into
 // pinned host memory that the host looks at.  flag null: nobody is waiting.
 struct HostSignal {

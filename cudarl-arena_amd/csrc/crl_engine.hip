@@ -361,6 +361,7 @@ struct FusedPlan {
   bool fixed;      // tickets dealt by position, round after round: no counter
   bool lanes;      // an env to A lanes, a wave to 2^log_envs envs, draws taped tape_steps ahead
   int log_envs, tape_steps;
+  bool touch;      // ... whose tables are read ahead whole
   bool rich;       // ticket kernel: the folded loop's variant with per-cell rewards / per-episode epsilon
   int tab_stride;  // floats between two tables in LDS
   bool in_lds;     // ... with all tables in LDS
@@ -379,11 +380,18 @@ constexpr size_t kStaticLdsReserve = 1024;
 // 32: 2.4e10 / 2.1e10, 48: 2.8e10 / 2.75e10, 64: 3.0e10 / 3.3e10, 100: 3.6e10 / 4.2e10).
 constexpr int kHybridMinSteps = 64;
 constexpr int kStagedMovesMinSteps = 128;
-constexpr int kLdsMinSteps = 16;
-constexpr size_t kLdsBytesPerStep = 640;
+constexpr int kLdsMinSteps = 16, kLdsAlwaysSteps = 144;
+constexpr size_t kLdsBytesFree = 8192, kLdsBytesPerStep = 208;
 constexpr int kLongLaunchSteps = 4096;
 constexpr int kLaneWavesMinSteps = 8;
-constexpr int kLaneRoundsMinSteps = 384;
+constexpr int kLaneRoundsMinSteps = 64, kLaneRoundsManyMinSteps = 131;
+constexpr long kLaneRoundsManyEnvs = 65536;
+constexpr int kLaneRoundsFourMinSteps = 64, kLaneRoundsFourLongSteps = 300;
+constexpr int kLaneDrawnMinSteps = 256, kLaneDrawnManyMinSteps = 128;
+constexpr int kLaneTouchMinSteps4 = 90, kLaneTouchMinSteps8 = 160;
+// Hybrid workgroups in place of rounds of lane waves.
+constexpr int kHybridFewRoundsMinSteps = 384;
+constexpr long kHybridEnvStepsSmall = 18000000, kHybridEnvSteps4 = 24000000, kHybridEnvSteps8 = 28000000;
 constexpr size_t kTableBytesAtOnce = (size_t)512 << 20;
 
 // Configurations that run_lanes() steps: no goal test on the resulting cell, no sticky done,
@@ -420,10 +428,13 @@ bool plan_fused_lds(const crl_engine* e, int n_steps, FusedPlan* p) {
   for (int words = 1; words >= 0; --words) {
     const size_t bytes = 16 + (env_bytes[words] << log_envs) + tape_bytes(log_envs) + (shared && !words ? code_bytes : 0);
     if (((bytes + 1023) & ~(size_t)1023) * per_unit > kLdsPerWorkgroup) continue;
-    // (what a wave's tables take to move in and out, 640 bytes to a step saved: tables in LDS / in
-    // HBM, 4096 envs of 16x16, 16 KB to a wave, 16 / 32 steps 11.4 / 13.6, 10.7 / 14.1 us; 100 of
-    // 48x48 with 8 actions, 72 KB, 16 / 100 steps 17.5 / 31.0, 11.0 / 29.1)
-    if ((size_t)n_steps * kLdsBytesPerStep < (4 * e->K) << log_envs) return false;
+    // What a wave's tables, or a quarter of a compute unit's, take to move in and out against the
+    // steps' trips to HBM (tables in LDS / in HBM: 4096 envs of 16x16, 16 KB to a wave, 32 / 48 steps
+    // 12.7 / 11.7, 14.9 / 15.5 us; 2000 of 32x32, 32 KB, 64 / 128 / 200 steps 22.0 / 18.9, 30.5 / 30.6,
+    // 40.3 / 44.4; 30,000 of 8x8, eight waves of 16 KB to a unit, 64 / 128 steps 29.5 / 25.2, 42.9 / 43.3;
+    // 100 of 48x48 with 8 actions, 72 KB, 128 / 200 steps 30.4 / 28.1, 39.6 / 41.4).
+    const size_t moved = std::max<size_t>((4 * e->K) << log_envs, ((4 * e->K) << log_envs) * per_unit / 4);
+    if (n_steps < kLdsAlwaysSteps && (size_t)n_steps * kLdsBytesPerStep + kLdsBytesFree < moved) return false;
     p->in_lds = p->lanes = p->fast = true;
     p->words = words != 0;
     p->rich = c.eps_mode >= CRL_EPS_EPISODE_MULT;
@@ -573,15 +584,45 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     // it and over 64-env waves (60,000 of 16x16, 64 / 500 steps: 143 / 566 hybrid, 86 / 420;
     // 40,000 of 20x20 with 8 actions, 130 steps: 212, 163) up to about 512 MB (65,536 of 32x32,
     // 1 GB, 300 steps: 503, 506).
-    const bool lanes_at_once = lanes_can && lane_units <= kComputeUnits * std::min(lane_fit, outgrown ? 20L : 24L) &&
+    // With 4 actions rather fewer, in launches long enough that rows are used again: a full unit's waves
+    // have less of the L2 each (waves to a unit; in one round / two, 31 / 130 / 300 / 800 steps: 17.1,
+    // 70,000 envs of 6x6 28 / 95 / 208 / 625, 32 / 100 / 210 / 533 us; 19.5, 80,000 of 5x5 29 / 110 / 281 /
+    // 769, 32 / 103 / 216 / 559; 19.8, 81,000 of 12x12 41 / 198 / 461 / 1214, 41 / 136 / 300 / 778; 22,
+    // 90,000 of 7x7 130 steps 182, 117; epsilon by episode: 19.5 111 / 273, 129 / 280, 22 184 / 416, 138 /
+    // 295; with 8 actions 43,662 of 10x10, 21.3, 29 / 90 / 186, 36 / 108 / 234).
+    const bool by_episode = c.eps_mode >= CRL_EPS_EPISODE_MULT;
+    const long at_once_waves = e->A == 4 && n_steps >= kLaneRoundsFourMinSteps
+                                   ? (by_episode ? 20L : n_steps >= kLaneRoundsFourLongSteps ? 16L : 18L)
+                                   : outgrown ? 20L : 24L;
+    const bool lanes_at_once = lanes_can && lane_units <= kComputeUnits * std::min(lane_fit, at_once_waves) &&
                                all_tables <= kTableBytesAtOnce;
+    // Lane waves in even rounds: as many waves as leave their rows in the caches most of the time
+    // (16x16 maps, waves per compute unit: 4 actions, 524,288 envs 4: 4.8e10, 8: 6.2e10, 12: 5.7e10,
+    // 16: 5.0e10; 8 actions, 262,144 envs 8: 3.7e10, 12: 4.2e10, 16: 4.0e10).
+    const long per_round = kComputeUnits * (!outgrown ? 16L : e->A == 8 ? 12L : 8L);
+    const long rounds = (lane_units + per_round - 1) / per_round;
+    // Hybrid workgroups take a while to share out their envs, and their last table waves are late:
+    // they pay over rounds of lane waves once a table's steps are worth its way into LDS and there is
+    // enough to step (lane waves / hybrid, 8x8 maps: 1M envs, 16 / 32 / 64 steps 433 / 703 / 938, 405 / 571 / 776 us; 200,000, 64 / 96 steps 179 / 190,
+    // 249 / 236; 16x16: 1M envs, 64 / 96 steps 1515 / 1682, 2174 / 1945 us; 180,000, 96 / 128 steps 396 / 414, 489 / 469;
+    // 140,000, 160 / 256 steps 385 / 408, 588 / 551; 8 actions, 160,000 of 12x12, 128 / 256 steps
+    // 471 / 503, 874 / 794), and not where the lane waves have few rounds: 95,000, three of them, 256 /
+    // 500 steps 353 / 383, 662 / 634; 8 actions, 73,000, three, 500 / 1000 steps 682 / 830, 1302 / 1484.
+    const bool few_rounds = rounds <= (e->A == 8 ? 4 : 3);
+    const bool hybrid_pays =
+        few_rounds ? e->A == 4 && n_steps >= kHybridFewRoundsMinSteps
+                   : 64L * n_steps >= 5L * (long)e->K &&
+                         (long)e->N * n_steps >= (e->K < 512   ? kHybridEnvStepsSmall
+                                                  : e->A == 8 ? kHybridEnvSteps8
+                                                              : kHybridEnvSteps4);
     // ... (automatic) when the tables outgrow the caches: while they all fit, other plans are
     // faster (16x16 maps, 30,000 envs: 3.5e10 hybrid, 5.9e10 with lane waves); and where lane
     // waves could step what is left to the general loop, they are faster too (262,144 envs of
     // 16x16 with a zero-floored maximum: 5.1e10 general hybrid, 6.4e10)
     p.hybrid = fits && (e->fused_variant == 2 ||
-                        (e->fused_variant == 0 && outgrown && n_steps >= kHybridMinSteps &&
-                         (lanes_can ? p.fast && (!lanes_at_once || e->resident_envs > 0) : true)));
+                        (e->fused_variant == 0 && outgrown &&
+                         (lanes_can && e->resident_envs == 0 ? p.fast && !lanes_at_once && hybrid_pays
+                                                             : (!lanes_can || p.fast) && n_steps >= kHybridMinSteps)));
     if (p.hybrid) {
       p.grid = (int)std::min<long>(kComputeUnits, (tickets + 8) / 9);
       p.block = 64 * (hbm_waves + p.lds_waves);
@@ -605,28 +646,34 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       while (waves > 1 && (size_t)waves * map_lds > kLdsPerWorkgroup) --waves;
       p.grid = (int)((workers + waves - 1) / waves);
       p.block = 64 * (int)waves;
-      // staging the codes (four times the class map) pays off over a long launch only:
-      // 1M envs of config 4, one step per launch 7.7e9 -> 1.4e10 with class maps, 48 steps 3.6e10 -> 3.7e10
-      p.moves = p.fast && waves * mv_lds <= kLdsPerWorkgroup && n_steps >= kStagedMovesMinSteps;
+      // staging the codes (four times the class map) pays off over a long launch only (1M envs of
+      // 16x16, one step per launch 7.7e9 -> 1.4e10 with class maps, 48 steps 3.6e10 -> 3.7e10), and not
+      // where fewer of the workgroups fit a compute unit for it (34,000 of 32x32, 128 steps: 193, 120 us)
+      p.moves = p.fast && (size_t)((p.grid + kComputeUnits - 1) / kComputeUnits) * waves * mv_lds <= kLdsPerWorkgroup &&
+                n_steps >= kStagedMovesMinSteps;
       // Few envs: A lanes to each, in as many waves as leave no more than two to a SIMD.  More:
       // all at once in lane waves, in place of the folded loop for launches of some steps (30,000
       // envs of 16x16, 4 / 8 / 16 steps: 23 / 28 / 35 us, 23 / 26 / 28), of the general loop always
-      // (30,000 of 16x16, one step: 12.5 us, 8.9; in rounds 200,000, 2 / 6 steps: 34 / 75, 50 / 74).  Else lane waves in even rounds, of as many waves as
-      // leave their rows in the caches most of the time (16x16 maps, waves per compute unit:
-      // 4 actions, 524,288 envs 4: 4.8e10, 8: 6.2e10, 12: 5.7e10, 16: 5.0e10; 8 actions, 262,144
-      // envs 8: 3.7e10, 12: 4.2e10, 16: 4.0e10) - not with fewer of them because the codes take
-      // too much LDS (50,000 envs of 48x48, 4 waves: 643 / 700 us), and where the folded loop would
-      // do as well in launches long enough only (4 actions, 64-env / lane waves: 65,536 envs of
-      // 32x32, 64 / 300 / 1000 steps 131 / 503 / 1487, 179 / 517 / 1471; 30,000 of 24x24 - half
-      // the SIMDs without a 64-env wave - 130 steps 116, 99).
+      // (30,000 of 16x16, one step: 12.5 us, 8.9; in rounds 200,000, 2 / 6 steps: 34 / 75, 50 / 74).
+      // Else lane waves in rounds (not with fewer of them because the codes take too much LDS:
+      // 50,000 envs of 48x48, 4 waves: 643 / 700 us): always soon where the tables do not outgrow the
+      // caches or the general loop is the other choice.  Where they do, 64-env / lane waves:
+      //   tables that hybrid workgroups could take, 16 / 48 steps: 1M of 16x16 468 / 1246, 494 / 1177 us;
+      //     70,000 with 8 actions 47.6 / 117, 47.9 / 103; the smaller the sooner: 130,000 of 12x12, 24
+      //     steps 67.0, 64.8; 200,000 of 8x8, 8 / 16 steps 51.6 / 70.6, 44.1 / 64.3
+      //   others, 32 / 64 / 96 steps: 52,000 of 32x32 61 / 114 / 160, 57 / 98 / 139; 40,000 of 24x24 with
+      //     8 actions 49 / 100 / 142, 57 / 97 / 136; 100,000 of 32x32 123 / 229 / 333, 119 / 206 / 291 (the
+      //     larger batches keep their 64-env waves up to 130 steps, a length that their tests hold them to)
+      //   4 actions, not more than three waves of 64 envs to a compute unit: 64-env waves always, 34,000 of
+      //     32x32, 128 / 1000 steps 120 / 727, 146 / 908; 49,000 176 / 1235, 174 / 1240
       const bool small = waves == 1 && tickets <= 2 * kComputeUnits;
-      const long per_round = kComputeUnits * (!outgrown ? 16L : e->A == 8 ? 12L : 8L);
-      const long rounds = small || lanes_at_once ? 1 : (lane_units + per_round - 1) / per_round;
-      const long lane_waves = (lane_units + rounds - 1) / rounds;
+      const long lane_waves = small || lanes_at_once ? lane_units : (lane_units + rounds - 1) / rounds;
       const int at_once_min_steps = p.fast ? kLaneWavesMinSteps : 1;
-      const int rounds_min_steps = !(p.fast && outgrown)                         ? kLaneWavesMinSteps
-                                   : e->A == 4 && (long)e->N <= kMinEnvsInFlight ? kStagedMovesMinSteps
-                                                                                 : kLaneRoundsMinSteps;
+      const int rounds_min_steps = !(p.fast && outgrown)                             ? kLaneWavesMinSteps
+                                   : fits && e->fused_variant == 0                   ? (int)std::min<size_t>(40, std::max<size_t>(kLaneWavesMinSteps, e->K / 24))
+                                   : e->A == 4 && (long)e->N <= kMinEnvsInFlight     ? INT_MAX
+                                   : (long)e->N <= kLaneRoundsManyEnvs               ? kLaneRoundsMinSteps
+                                                                                     : kLaneRoundsManyMinSteps;
       const bool rounds_ok = lane_waves <= kComputeUnits * lane_fit && n_steps >= rounds_min_steps;
       if (lanes_can && (small ? lane_fit > 0 : lanes_at_once ? n_steps >= at_once_min_steps : rounds_ok)) {
         p.fast = p.moves = p.lanes = true;
@@ -636,14 +683,26 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
         const long most = e->resident_envs > 0 ? std::max<long>(1, resident >> lane_log_envs) : lane_waves;
         p.grid = (int)std::min<long>(lane_units, most);
         p.block = 64;
+        const bool many_rounds = p.grid * 5L < lane_units;
+        // (the tables' lines asked for ahead: 300,000 of 16x16, 64 / 96 / 200 / 1000 steps 531 / 682 /
+        // 1196 / 4774 us with, 483 / 701 / 1346 / 5276 without; 200,000 with 8 actions, 128 / 200 steps 841 /
+        // 1142, 808 / 1179; 198,000 of
+        // 10x30, seven rounds, 757 steps 2375, 2740; 120,000 of 16x16, four rounds, 200 / 1000 steps 488 / 1910,
+        // 373 / 1706)
+        p.touch = outgrown && many_rounds && n_steps >= (e->A == 8 ? kLaneTouchMinSteps8 : kLaneTouchMinSteps4) &&
+                  e->K <= (size_t)crl::kTouchFloats;
         // (no more than it uses, also where there is a compute unit for every workgroup: 4096 envs
         // of 32x32, 10,000 steps, 17 / 64 / 81 KB 2.78 / 2.76 / 2.80 ms)
         p.lds = lane_lds;
       }
-      // Tickets dealt by position instead of drawn from a counter: the workers of this plan
-      // all take the same time, and 16,384 draws from one counter take 0.38 ms however short
-      // the launch (1M envs: the whole of a 4-step launch, half of a 20-step one).
-      p.fixed = n_steps < kHybridMinSteps || (p.lanes && p.grid >= lane_units);
+      // Envs dealt by position instead of drawn from a counter: 16,384 draws take 0.38 ms however short
+      // the launch (1M envs: the whole of a 4-step launch, half of a 20-step one).  Lane waves, drawn /
+      // dealt: 120,000 envs of 8x8, two rounds, 128 / 1000 steps 207 / 1315, 176 / 1268 us; 140,000 of 6x6
+      // with 8 actions, five rounds, 128 / 300 / 1000 steps 290 / 563 / 1654, 279 / 609 / 1912; 300,000
+      // of 16x16, ten rounds, 128 / 300 steps 868 / 1523, 879 / 1585; 891,000 of 20x14, 150 steps 2503, 2705.
+      const bool drawn_lanes = n_steps >= kLaneDrawnMinSteps ? e->A == 8 || p.grid * 3L < lane_units
+                                                             : n_steps >= kLaneDrawnManyMinSteps && p.grid * 5L < lane_units;
+      p.fixed = p.lanes ? p.grid >= lane_units || !drawn_lanes : n_steps < kHybridMinSteps;
       if (!p.lanes) p.lds = waves * (p.moves ? mv_lds : map_lds);
     }
   }
@@ -677,16 +736,21 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
   const crl::Rules R = e->rules();
   const crl::Ptrs P = e->ptrs();
   if (p.in_lds) {
-    const bool events = crl::lane_events(R, P);
+    const int events = crl::lane_events(R, P);
 #define CRL_LAUNCH_LDS(KERN)                                                                                              \
   do {                                                                                                                    \
     auto go = [&](auto kern) {                                                                                            \
       hipLaunchKernelGGL(kern, dim3(p.grid), dim3(64), p.lds, e->stream, R, P, t0, n, p.log_envs, p.env_bytes, p.tape_steps); \
     };                                                                                                                    \
-    if (p.words && events) go(crl::KERN<A, true, true>);                                                                  \
-    else if (p.words) go(crl::KERN<A, true, false>);                                                                      \
-    else if (events) go(crl::KERN<A, false, true>);                                                                       \
-    else go(crl::KERN<A, false, false>);                                                                                  \
+    if (p.words) {                                                                                                        \
+      if (events == crl::kNoEvents) go(crl::KERN<A, true, crl::kNoEvents>);                                               \
+      else if (events == crl::kEpsilonEvents) go(crl::KERN<A, true, crl::kEpsilonEvents>);                                \
+      else go(crl::KERN<A, true, crl::kAllEvents>);                                                                       \
+    } else {                                                                                                              \
+      if (events == crl::kNoEvents) go(crl::KERN<A, false, crl::kNoEvents>);                                              \
+      else if (events == crl::kEpsilonEvents) go(crl::KERN<A, false, crl::kEpsilonEvents>);                               \
+      else go(crl::KERN<A, false, crl::kAllEvents>);                                                                      \
+    }                                                                                                                     \
   } while (0)
     if (p.map_kind == 1) CRL_LAUNCH_LDS(k_fused_per_env_lds);
     else CRL_LAUNCH_LDS(k_fused_tickets_lds);
@@ -702,10 +766,20 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
 #define CRL_LAUNCH_TICKETS(MODE, LDSW, MOVES)                                                       \
   hipLaunchKernelGGL((crl::k_fused_tickets<A, MODE, LDSW, MOVES>), g, b, p.lds, e->stream, R, P, t0, n, \
                      tk, p.tab_stride, p.fixed ? 1 : 0, p.tape_steps, p.lds_waves, p.env_bytes)
+    const int events = crl::lane_events(R, P);
+#define CRL_LAUNCH_LANES(CELLS)                                                                                            \
+  do {                                                                                                                     \
+    auto go = [&](auto kern) {                                                                                             \
+      hipLaunchKernelGGL(kern, g, b, p.lds, e->stream, R, P, t0, n, tk, p.fixed ? 1 : 0, p.touch ? 1 : 0, p.log_envs, p.tape_steps); \
+    };                                                                                                                     \
+    if (events == crl::kNoEvents) go(crl::k_fused_lanes<A, CELLS, crl::kNoEvents>);                                        \
+    else if (events == crl::kEpsilonEvents) go(crl::k_fused_lanes<A, CELLS, crl::kEpsilonEvents>);                         \
+    else go(crl::k_fused_lanes<A, CELLS, crl::kAllEvents>);                                                                \
+  } while (0)
     if (p.lanes && P.cell_reward)
-      hipLaunchKernelGGL((crl::k_fused_lanes<A, true>), g, b, p.lds, e->stream, R, P, t0, n, tk, p.fixed ? 1 : 0, p.log_envs, p.tape_steps);
+      CRL_LAUNCH_LANES(true);
     else if (p.lanes)
-      hipLaunchKernelGGL((crl::k_fused_lanes<A, false>), g, b, p.lds, e->stream, R, P, t0, n, tk, p.fixed ? 1 : 0, p.log_envs, p.tape_steps);
+      CRL_LAUNCH_LANES(false);
     else if (p.rich && p.moves)
       CRL_LAUNCH_TICKETS(2, false, true);
     else if (p.rich)
@@ -721,6 +795,7 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
     else
       CRL_LAUNCH_TICKETS(0, false, false);
 #undef CRL_LAUNCH_TICKETS
+#undef CRL_LAUNCH_LANES
     return;
   }
 #define CRL_LAUNCH_PER_ENV(MAP, MODE)                                                                 \
@@ -1689,17 +1764,20 @@ int opt_in_ticket_kernels(crl_engine* e) {
       reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, true, false>),         \
       reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, false, true>),         \
       reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 2, false, true>),         \
-      reinterpret_cast<const void*>(&crl::k_fused_lanes<A, false>),                    \
-      reinterpret_cast<const void*>(&crl::k_fused_lanes<A, true>),                     \
+      CRL_LANE_KERNELS(A, false), CRL_LANE_KERNELS(A, true),                           \
       reinterpret_cast<const void*>(&crl::k_fused_per_env<A, 1, 2>),                   \
-      CRL_LDS_KERNELS(A, false, false), CRL_LDS_KERNELS(A, false, true),               \
-      CRL_LDS_KERNELS(A, true, false), CRL_LDS_KERNELS(A, true, true)
-#define CRL_LDS_KERNELS(A, WORDS, EVENTS)                                              \
-  reinterpret_cast<const void*>(&crl::k_fused_tickets_lds<A, WORDS, EVENTS>),          \
-      reinterpret_cast<const void*>(&crl::k_fused_per_env_lds<A, WORDS, EVENTS>)
+      CRL_LDS_KERNELS(A, false), CRL_LDS_KERNELS(A, true)
+#define CRL_EVENTS(KERN, A, FLAG)                                                      \
+  reinterpret_cast<const void*>(&crl::KERN<A, FLAG, crl::kNoEvents>),                  \
+      reinterpret_cast<const void*>(&crl::KERN<A, FLAG, crl::kEpsilonEvents>),         \
+      reinterpret_cast<const void*>(&crl::KERN<A, FLAG, crl::kAllEvents>)
+#define CRL_LANE_KERNELS(A, CELLS) CRL_EVENTS(k_fused_lanes, A, CELLS)
+#define CRL_LDS_KERNELS(A, WORDS) CRL_EVENTS(k_fused_tickets_lds, A, WORDS), CRL_EVENTS(k_fused_per_env_lds, A, WORDS)
       CRL_TICKET_KERNELS(4), CRL_TICKET_KERNELS(8)
 #undef CRL_TICKET_KERNELS
 #undef CRL_LDS_KERNELS
+#undef CRL_LANE_KERNELS
+#undef CRL_EVENTS
   };
   for (const void* fn : fns)
     HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsPerWorkgroup));

@@ -743,13 +743,19 @@ __device__ __forceinline__ int lane_slot(const int lane, const int log_envs, con
   return slot < n_here ? slot : 0;
 }
 
+constexpr int kNoEvents = 0, kEpsilonEvents = 1, kAllEvents = 2;
+
 // The steps.  Every lane of the wave calls it with its env's number in the wave (lane_slot).
 // The rewards by class - step, goal, trap, step - lie
-// at LDS address 0, where dynamic LDS starts in a kernel without any other; CELLS: `cell_rewards` of the cells of the wave's first env (or of the shared map) also count.  EVENTS: an episode's end changes more
-// than where the env stands - epsilon by episode, episode statistics, an episode budget.
+// at LDS address 0, where dynamic LDS starts in a kernel without any other; CELLS: `cell_rewards` of the cells of the wave's first env (or of the shared map) also count.  EVENTS: an
+// episode's end changes more than where the env stands: epsilon by episode (kEpsilonEvents), or any of
+// that, episode statistics and an episode budget (kAllEvents).  Epsilon alone needs one loop and none of
+// the statistics' registers: 78 in place of 104, six waves to a SIMD in place of four (43,662 envs of
+// 10x10 with 8 actions, 300 steps: 278 -> 218 us; 4096 of
+// 16x16 in LDS, 300 steps 98 -> 72).
 // The row of the cell the move ends on (for the TD target) and that of the cell the env acts
 // from next - another one only where its episode ended - are asked for together.
-template <int A, bool CELLS, bool EVENTS, class Mem>
+template <int A, bool CELLS, int EVENTS, class Mem>
 __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const int env0, const int slot,
                                           const uint64_t t0, const int n_steps, const Mem mem, uint32_t* tape,
                                           const int log_envs, const int tape_steps,
@@ -769,21 +775,22 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
   int episode = P.episode[env];
   float reward = P.reward[env];
   uint32_t won = ((uint32_t)P.action[env] << 29) | (P.done[env] != 0 ? (uint32_t)kGoal << 2 : 0u);  // the last step's word
-  const bool by_episode = EVENTS && R.eps_mode >= 2, track = EVENTS && P.ret_acc != nullptr;
+  constexpr bool kAll = EVENTS == kAllEvents;
+  const bool by_episode = EVENTS == kEpsilonEvents || (kAll && R.eps_mode >= 2), track = kAll && P.ret_acc != nullptr;
   const bool base_cells = CELLS && (R.reward_flags & 2) != 0;
   const uint32_t rewards_at = CELLS && !P.map_shared ? (uint32_t)slot * (uint32_t)P.S * 4u : 0u;
-  uint32_t limit = by_episode ? tape_limit(eps_of(R, P.eps_tab, t0, episode)) : kTapeLimit;
-  float eps_next = by_episode ? eps_of(R, P.eps_tab, t0, episode + 1) : 0.0f;  // of the next episode: asked for ahead
+  uint32_t limit = by_episode ? tape_limit(eps_of_episode(R, P.eps_tab, episode)) : kTapeLimit;
+  float eps_next = by_episode ? eps_of_episode(R, P.eps_tab, episode + 1) : 0.0f;  // of the next episode: asked for ahead
   LaneStats stats{0.0f, 0.0f, 0.0f, 0, 0};
   if (track) stats = LaneStats{P.ret_acc[env], P.ret_last[env], P.ret_sum[env], P.len_last[env], P.len_sum[env]};
-  const int budget = EVENTS && R.max_episodes > 0 ? R.max_episodes : 0x7fffffff;
+  const int budget = kAll && R.max_episodes > 0 ? R.max_episodes : 0x7fffffff;
   bool going = episode < budget;
   float q = mem.value(at);
   uint32_t c = mem.word(at, mem.code(at));
   // (arrived before the loop starts: a value that may be in flight there makes every round
   // wait for everything, the last store's answer included)
   asm volatile("" : "+v"(q), "+v"(c), "+v"(reward), "+v"(left), "+v"(episode), "+v"(won), "+v"(limit), "+v"(eps_next));
-  if (EVENTS) asm volatile("" : "+v"(stats.ret), "+v"(stats.ret_last), "+v"(stats.ret_sum), "+v"(stats.len_last), "+v"(stats.len_sum));
+  if (kAll) asm volatile("" : "+v"(stats.ret), "+v"(stats.ret_last), "+v"(stats.ret_sum), "+v"(stats.len_last), "+v"(stats.len_sum));
 
   const uint64_t t_end = t0 + (uint64_t)n_steps;
   TapeLimits limits{explore_threshold(R.eps0), {}};
@@ -796,7 +803,7 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
     const int k0 = tb < t0 ? 1 : 0;  // (the first block may start with a step of the launch before)
     const int k1 = (int)min((uint64_t)tape_steps, t_end - tb);
     // (whether an env can use up its budget in these steps)
-    const bool close = EVENTS && __builtin_amdgcn_ballot_w64(episode >= budget - tape_steps) != 0ull;
+    const bool close = kAll && __builtin_amdgcn_ballot_w64(episode >= budget - tape_steps) != 0ull;
     // (leaving the loop is the same for all lanes that are in it: an env that has used up its
     // budget ends the loop for its wave, and the others enter it again without it)
     for (int k = k0; k < k1;) {
@@ -813,7 +820,7 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
         unsigned long long ends = 0ull;
         float paid = -0.0f;  // (nothing to add yet)
         auto step = [&](auto by_end, auto by_budget) __attribute__((always_inline)) {
-          won = lanes_choose<A, EVENTS>(q, unless, c, named, explore, left, last, stats, paid, ends, len);
+          won = lanes_choose<A, kAll>(q, unless, c, named, explore, left, last, stats, paid, ends, len);
           const typename Mem::At at2 = mem.at_word(won, at);
           const uint32_t cls = won & kMoveClass;
           unsigned long long hit;
@@ -832,7 +839,7 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
           }
           const uint32_t draw = *lds_at<uint32_t>(word);  // (the one behind the tape's end is not used)
           const unsigned long long me = __builtin_amdgcn_ballot_w64(c == won), stays = __builtin_amdgcn_ballot_w64(at_next == at);
-          if (EVENTS) len = whole - left + 1;
+          if (kAll) len = whole - left + 1;
           ends = lanes_count(hit, last, whole, left, episode);
           // All of the above while the values are on their way.  (Without the barrier the move
           // word's arithmetic moves up and waits for its code before the other reads are asked
@@ -845,7 +852,7 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
             if (__builtin_expect(ends != 0ull, 0)) {
               if (by_episode) {
                 limit = __builtin_amdgcn_inverse_ballot_w64(ends) ? tape_limit(eps_next) : limit;
-                eps_next = eps_of(R, P.eps_tab, t0, episode + 1);
+                eps_next = eps_of_episode(R, P.eps_tab, episode + 1);
               }
               if (decltype(by_budget)::value && __builtin_amdgcn_ballot_w64(episode >= budget) != 0ull) end = kk + 1;
             }
@@ -869,15 +876,17 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
           }
           while (kk < end) step(by_end, no);
         };
-        if (EVENTS && close) {
+        if constexpr (!kAll) {
+          steps(std::integral_constant<bool, EVENTS == kEpsilonEvents>{});
+        } else if (close) {
           do step(std::true_type{}, std::true_type{});
           while (kk < end);
-        } else if (EVENTS && by_episode) {
+        } else if (by_episode) {
           steps(std::true_type{});
         } else {
           steps(std::false_type{});
         }
-        if (EVENTS) {  // (the last step's)
+        if (kAll) {  // (the last step's)
           const bool over = __builtin_amdgcn_inverse_ballot_w64(ends);
           stats.ret = stats.ret + paid;
           stats.ret_last = over ? stats.ret : stats.ret_last;
@@ -909,9 +918,9 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
   }
 }
 
-// whether run_lanes needs its EVENTS form
-__host__ __device__ inline bool lane_events(const Rules& R, const Ptrs& P) {
-  return R.eps_mode >= 2 || R.max_episodes > 0 || P.ret_acc != nullptr;
+// the form of run_lanes that a configuration needs
+__host__ __device__ inline int lane_events(const Rules& R, const Ptrs& P) {
+  return R.max_episodes > 0 || P.ret_acc != nullptr ? kAllEvents : R.eps_mode >= 2 ? kEpsilonEvents : kNoEvents;
 }
 // the rewards by class, where run_lanes looks them up; word i of n, by one wave
 __device__ __forceinline__ void write_rewards(const Rules& R, float* rewards, int lane) {
@@ -943,7 +952,7 @@ __device__ __forceinline__ int row_step(const Rules& R, uint32_t a, uint32_t row
 // the tape.  WORDS: an env is rows of values and move words side by side (8 bytes per
 // key); else rows of values, then the move codes (4 bytes and a quarter; a shared map's
 // codes only once, behind the tape).
-template <int A, bool MAP_SHARED, bool WORDS, bool EVENTS>
+template <int A, bool MAP_SHARED, bool WORDS, int EVENTS>
 __device__ __forceinline__ void fused_lds(const Rules& R, const Ptrs& P, const uint64_t t0, const int n_steps,
                                           const int log_envs, const int env_bytes, const int tape_steps) {
   extern __shared__ __align__(16) unsigned char lds_bytes[];
@@ -1035,13 +1044,13 @@ __device__ __forceinline__ void fused_lds(const Rules& R, const Ptrs& P, const u
     store_row(out + (size_t)i * A, load_row<A>(reinterpret_cast<const float*>(envs + (size_t)e * env_bytes + (size_t)cell * kRow)));
   }
 }
-template <int A, bool WORDS, bool EVENTS>
+template <int A, bool WORDS, int EVENTS>
 __global__ __launch_bounds__(64) void k_fused_tickets_lds(const Rules R, const Ptrs P, const uint64_t t0,
                                                            const int n_steps, const int log_envs,
                                                            const int env_bytes, const int tape_steps) {
   fused_lds<A, false, WORDS, EVENTS>(R, P, t0, n_steps, log_envs, env_bytes, tape_steps);
 }
-template <int A, bool WORDS, bool EVENTS>
+template <int A, bool WORDS, int EVENTS>
 __global__ __launch_bounds__(64) void k_fused_per_env_lds(const Rules R, const Ptrs P, const uint64_t t0,
                                                            const int n_steps, const int log_envs,
                                                            const int env_bytes, const int tape_steps) {
@@ -1051,7 +1060,7 @@ __global__ __launch_bounds__(64) void k_fused_per_env_lds(const Rules R, const P
 // Tables in HBM and the caches, an env to A lanes, a wave to 1 << log_envs envs from env0 on.
 // `codes` are the move codes of the map (shared) or of the wave's first env, in LDS (CL) or
 // global memory; `code_bytes` from one env's to the next (0: shared).
-template <int A, bool CELLS, bool CL>
+template <int A, bool CELLS, bool CL, int EVENTS>
 __device__ __forceinline__ void fused_lanes_hbm(const Rules& R, const Ptrs& P, const int env0, const uint64_t t0,
                                                 const int n_steps, const unsigned char* codes, const uint32_t code_bytes,
                                                 uint32_t* tape, const int log_envs, const int tape_steps) {
@@ -1065,10 +1074,7 @@ __device__ __forceinline__ void fused_lanes_hbm(const Rules& R, const Ptrs& P, c
                                     CL ? 0u : at * code_bytes,
                                     action, row_step<A>(R, action, kRow)};
   const float* cr = CELLS ? P.cell_reward + (P.map_shared ? 0 : (size_t)env0 * P.S) : nullptr;  // of the wave's first env
-  if (lane_events(R, P))
-    run_lanes<A, CELLS, true>(R, P, env0, slot, t0, n_steps, mem, tape, log_envs, tape_steps, cr);
-  else
-    run_lanes<A, CELLS, false>(R, P, env0, slot, t0, n_steps, mem, tape, log_envs, tape_steps, cr);
+  run_lanes<A, CELLS, EVENTS>(R, P, env0, slot, t0, n_steps, mem, tape, log_envs, tape_steps, cr);
 }
 
 // Per-env tables whose maps are shared (MAP = 1: the one map's move codes staged
@@ -1099,10 +1105,18 @@ __global__ __launch_bounds__(256) void k_fused_per_env(const Rules R, const Ptrs
     const uint32_t code_bytes = P.map_shared ? 0u : (uint32_t)P.mv_words * 4u;
     const unsigned char* from = reinterpret_cast<const unsigned char*>(
         MAP == 1 ? codes : P.moves + (P.map_shared ? 0 : (size_t)env0 * P.mv_words));
-    if (P.cell_reward)
-      fused_lanes_hbm<A, true, MAP == 1>(R, P, env0, t0, n_steps, from, code_bytes, tape, log_envs, tape_steps);
-    else
-      fused_lanes_hbm<A, false, MAP == 1>(R, P, env0, t0, n_steps, from, code_bytes, tape, log_envs, tape_steps);
+    auto run = [&](auto cells, auto events) __attribute__((always_inline)) {
+      fused_lanes_hbm<A, decltype(cells)::value, MAP == 1, decltype(events)::value>(R, P, env0, t0, n_steps, from, code_bytes, tape,
+                                                                                   log_envs, tape_steps);
+    };
+    auto with = [&](auto events) __attribute__((always_inline)) {
+      if (P.cell_reward) run(std::true_type{}, events);
+      else run(std::false_type{}, events);
+    };
+    const int events = lane_events(R, P);
+    if (events == kNoEvents) with(std::integral_constant<int, kNoEvents>{});
+    else if (events == kEpsilonEvents) with(std::integral_constant<int, kEpsilonEvents>{});
+    else with(std::integral_constant<int, kAllEvents>{});
   } else {
     constexpr bool FAST = MODE == 1;
     const int n_chunks = (P.N + bdim - 1) / bdim;
@@ -1133,16 +1147,18 @@ __global__ __launch_bounds__(256) void k_fused_per_env(const Rules R, const Ptrs
   }
 }
 
-// The same with per-env maps: one wave to a workgroup, which draws 1 << log_envs envs at a
-// time from a ticket counter (or is dealt them by position: fixed_tickets), stages their move
-// codes into its LDS and steps them for all n_steps, A lanes to an env.  What bounds it is the
+// The same with per-env maps: one wave to a workgroup, which takes 1 << log_envs envs at a
+// time, stages their move codes into its LDS and steps them for all n_steps, A lanes to an env.
+// The first envs, and with `dealt` all of them, come by position; else the next ones by a draw from
+// a counter, which waits 23 ns for each other wave that draws then.  `touch`: see below.
+// What bounds it is the
 // wave's dependent chain - some 60 instructions a step, the tape's not counted, and a trip to the row,
 // 0.26 us per step of 4096 envs on 32x32 maps - of which a wave with 64 envs pays the slowest of 64
 // trips and 150 instructions.
 // LDS: the rewards by class, the tape, the codes env by env.
-template <int A, bool CELLS>
+template <int A, bool CELLS, int EVENTS>
 __global__ __launch_bounds__(64) void k_fused_lanes(const Rules R, const Ptrs P, const uint64_t t0, const int n_steps,
-                                                    unsigned* __restrict__ ticket, const int fixed_tickets,
+                                                    unsigned* __restrict__ ticket, const int dealt, const int touch,
                                                     const int log_envs, const int tape_steps) {
   extern __shared__ __align__(16) uint32_t lds[];
   const int lane = threadIdx.x;
@@ -1151,36 +1167,34 @@ __global__ __launch_bounds__(64) void k_fused_lanes(const Rules R, const Ptrs P,
   uint32_t* tape = lds + 4;
   uint32_t* words = tape + ((tape_steps + 1) << log_envs);
   write_rewards(R, reinterpret_cast<float*>(lds), lane);
-  if (fixed_tickets && blockIdx.x == 0 && lane == 0) {
+  if (blockIdx.x == 0 && lane == 0) {
     ticket[1] = (unsigned)P.N;
     ticket[2] = 0u;
   }
-  unsigned stepped = 0;  // envs this worker has stepped
-  for (unsigned round = 0;; ++round) {
-    unsigned base = round * gridDim.x + blockIdx.x;
-    if (!fixed_tickets) {
-      if (lane == 0) base = atomicAdd(ticket, 1u);
-      base = (unsigned)__builtin_amdgcn_readfirstlane((int)base);
-    }
-    if (base >= n_tickets) break;  // every worker gets here: the number only grows
+  unsigned base = blockIdx.x;
+  while (base < n_tickets) {  // every wave leaves: the number only grows
     const int env0 = (int)base << log_envs;
     const int n_here = min(1 << log_envs, P.N - env0);
-    stepped += (unsigned)n_here;
     wave_fence();
     copy_words(P.moves + (size_t)env0 * P.mv_words, n_here * P.mv_words, words, lane);
     // (GlobalTable::touch for all of the wave's envs, whose tables are one run in HBM: where
     // they go through the chip in rounds, a launch meets most lines for the first time)
-    if (!fixed_tickets && n_steps >= kTouchMinSteps && table <= (size_t)kTouchFloats) {
+    if (touch) {
       const float* q = P.Q + (size_t)env0 * table;
       float acc = 0.0f;
       for (int i = lane * 32; i < n_here * (int)table; i += 64 * 32) acc += q[i];
       asm volatile("" ::"v"(acc));
     }
     wave_fence();
-    fused_lanes_hbm<A, CELLS, true>(R, P, env0, t0, n_steps, reinterpret_cast<const unsigned char*>(words),
+    fused_lanes_hbm<A, CELLS, true, EVENTS>(R, P, env0, t0, n_steps, reinterpret_cast<const unsigned char*>(words),
                                     (uint32_t)P.mv_words * 4u, tape, log_envs, tape_steps);
+    if (dealt) {
+      base += gridDim.x;
+    } else {
+      if (lane == 0) base = gridDim.x + atomicAdd(ticket, 1u);
+      base = (unsigned)__builtin_amdgcn_readfirstlane((int)base);
+    }
   }
-  if (!fixed_tickets && lane == 0 && stepped != 0u) atomicAdd(ticket + 1, stepped);
 }
 
 // Per-env tables with per-env maps small enough for LDS: every wave is an
@@ -1335,7 +1349,7 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
       const uint32_t action = (uint32_t)lane & (A - 1);
       unsigned char* mine = envs + (size_t)slot * env_bytes;
       const LaneCodes<A, true, true, false> mem{mine + 4 * action, 0u, mine + table * 4, 0u, action, row_step<A>(R, action, 4 * A)};
-      run_lanes<A, false, false>(R, P, env0, slot, t0, n_steps, mem,
+      run_lanes<A, false, kNoEvents>(R, P, env0, slot, t0, n_steps, mem,
                                  reinterpret_cast<uint32_t*>(envs + ((size_t)env_bytes << log_envs)), log_envs, tape_steps, nullptr);
       wave_fence();
       strided_copy<false>(tables, (int)(table / 4), n_here, envs, env_bytes, lane);
