@@ -539,7 +539,7 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     if (p.fast) {
       // The folded loop's LDS waves give an env A lanes: two table waves, and beside them as
       // many LDS waves as there is room for up to three.  1M envs, 16x16 maps, table + LDS
-      // waves: 3 + 1 7.7e10, 2 + 2 9.0e10, 3 + 2 8.4e10; 8x8: 2 + 2 1.16e11, 2 + 3 1.27e11;
+      // waves: 1 + 2 7.6e10, 2 + 2 9.8e10, 3 + 2 9.4e10 (8x8, 2 + 3: 1.45e11);
       // 8 actions, 16x16: 2 + 1 4.2e10, 2 + 2 4.7e10, 3 + 2 4.2e10.
       hbm_waves = 2;
       p.log_envs = most_log_envs;

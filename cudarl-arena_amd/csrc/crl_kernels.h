@@ -752,7 +752,7 @@ constexpr int kNoEvents = 0, kEpsilonEvents = 1, kAllEvents = 2;
 // that, episode statistics and an episode budget (kAllEvents).  Epsilon alone needs one loop and none of
 // the statistics' registers: 78 in place of 104, six waves to a SIMD in place of four (43,662 envs of
 // 10x10 with 8 actions, 300 steps: 278 -> 218 us; 4096 of
-// 16x16 in LDS, 300 steps 98 -> 72).
+// 16x16 in LDS, with the look-up that has no branch, 94 -> 72).
 // The row of the cell the move ends on (for the TD target) and that of the cell the env acts
 // from next - another one only where its episode ended - are asked for together.
 template <int A, bool CELLS, int EVENTS, class Mem>
@@ -1151,8 +1151,7 @@ __global__ __launch_bounds__(256) void k_fused_per_env(const Rules R, const Ptrs
 // time, stages their move codes into its LDS and steps them for all n_steps, A lanes to an env.
 // The first envs, and with `dealt` all of them, come by position; else the next ones by a draw from
 // a counter, which waits 23 ns for each other wave that draws then.  `touch`: see below.
-// What bounds it is the
-// wave's dependent chain - some 60 instructions a step, the tape's not counted, and a trip to the row,
+// What bounds it is the wave's dependent chain - 52 vector instructions a step, the tape's counted, and a trip to the row,
 // 0.26 us per step of 4096 envs on 32x32 maps - of which a wave with 64 envs pays the slowest of 64
 // trips and 150 instructions.
 // LDS: the rewards by class, the tape, the codes env by env.
@@ -1215,7 +1214,7 @@ __global__ __launch_bounds__(64) void k_fused_lanes(const Rules R, const Ptrs P,
 // move codes: with MOVES the table waves stage the pre-built codes, otherwise the (four times
 // smaller) class maps, and derive the codes while their row loads are in flight.  MODE 1's LDS
 // waves take 64 / A envs, A lanes to each (run_lanes; what bounds them is one env's dependent
-// chain, 0.21 us per step on a SIMD of its own).  Three table waves and one LDS wave of 32 envs
+// chain, 0.16 us per step where they are alone).  Three table waves and one LDS wave of 32 envs
 // with two lanes each / two table waves and the LDS waves of 64 / A envs that fit, launch after
 // launch: 1M envs of 16x16, 1000 steps 12.46 / 12.23 ms, of 8x8 8.83 / 8.26 ms.
 constexpr int kTicketEnvs = 32;

@@ -5,8 +5,8 @@
 // roles hand their data to each other through memory.  Always 256 owners, also where the table would
 // fit fewer: an owner's 256 cells are then small ones, every workgroup has a part in
 // both passes, and a table of few cells that many envs crowd on is spread as far as
-// it goes (65,536 envs on a 16x16x4 table: 7.2 us per step with 256 owners of one row
-// each, 14.3 with 16 owners of 16 rows).
+// it goes (65,536 envs on a 16x16x4 table: 6.3 us per step with 256 owners of one row
+// each; 16 owners of 16 rows took twice as long).
 //
 // What is exchanged is only ever touched with device-scope accesses (st_dev64 /
 // ld_dev64: coherent between the eight XCDs without fences), and every exchanged
@@ -37,7 +37,7 @@
 // What bounds a step is the chain of the two exchanges between all compute units and the work
 // between them.  20,000 envs on 101x99x8 (hashed form, phase clocks of a workgroup with envs):
 // views 1.8 us, select and hash 0.5, block sums 1.0, cells and records 2.4, totals 0.8; 200 steps
-// 2655 us with two launches per step, 1713 with this kernel.
+// 2609 us with two launches per step, 1660 with this kernel.
 // An owner overwrites its values only after it has every block's cells of the step,
 // which a block writes after all its threads have read theirs: one buffer of views
 // suffices.  Cells and raw samples have two buffers, taken in turn: a workgroup that
