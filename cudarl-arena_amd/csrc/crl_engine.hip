@@ -346,7 +346,10 @@ constexpr int kLdsMapLimitBytes = 64 * 1024;
 constexpr size_t kTableBytesInFlight = (size_t)192 << 20;
 constexpr int kComputeUnits = 256;
 constexpr long kMinEnvsInFlight = kComputeUnits * 3L * 64;  // three waves per compute unit
-constexpr int kInFlightMinSteps = 16;  // shorter launches: 4 steps 6.1e9 -> 6.9e9 with all envs in flight
+// Shorter launches have all envs in flight (all / as many as that, 2 / 4 / 6 / 8 / 12 steps: 1M envs of 16x16
+// 107 / 176 / 251 / 332 / 503 us, 127 / 175 / 225 / 275 / 378; 100,000 of 32x32 27 / 34 / 41 / 48 / 66,
+// 28 / 35 / 42 / 48 / 61; 200,000 of 16x16 with 8 actions 31 / 52 / 73 / 94 / 136, 31 / 46 / 60 / 74 / 104).
+constexpr int kInFlightMinSteps = 6;
 
 // launch geometry of the fused per-env kernel
 struct FusedPlan {
