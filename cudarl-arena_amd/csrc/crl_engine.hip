@@ -388,6 +388,7 @@ constexpr size_t kLdsBytesFree = 8192, kLdsBytesPerStep = 208;
 constexpr int kLongLaunchSteps = 4096;
 constexpr int kLaneWavesMinSteps = 8;
 constexpr int kLaneRoundsMinSteps = 64, kLaneRoundsManyMinSteps = 131;
+constexpr int kLaneFewRoundsMinSteps = 48;
 constexpr long kLaneRoundsManyEnvs = 65536;
 constexpr int kLaneRoundsFourMinSteps = 64, kLaneRoundsFourLongSteps = 300;
 constexpr int kLaneDrawnMinSteps = 256, kLaneDrawnManyMinSteps = 128;
@@ -663,7 +664,8 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       // caches or the general loop is the other choice.  Where they do, 64-env / lane waves:
       //   tables that hybrid workgroups could take, 16 / 48 steps: 1M of 16x16 468 / 1246, 494 / 1177 us;
       //     70,000 with 8 actions 47.6 / 117, 47.9 / 103; the smaller the sooner: 130,000 of 12x12, 24
-      //     steps 67.0, 64.8; 200,000 of 8x8, 8 / 16 steps 51.6 / 70.6, 44.1 / 64.3
+      //     steps 67.0, 64.8; 200,000 of 8x8, 8 / 16 steps 51.6 / 70.6, 44.1 / 64.3; with few rounds later:
+      //     94,000 of 12x12, three, 32 / 48 steps 50.9 / 72.3, 53.6 / 72.7
       //   others, 32 / 64 / 96 steps: 52,000 of 32x32 61 / 114 / 160, 57 / 98 / 139; 40,000 of 24x24 with
       //     8 actions 49 / 100 / 142, 57 / 97 / 136; 100,000 of 32x32 123 / 229 / 333, 119 / 206 / 291 (the
       //     larger batches keep their 64-env waves up to 130 steps, a length that their tests hold them to)
@@ -673,7 +675,7 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       const long lane_waves = small || lanes_at_once ? lane_units : (lane_units + rounds - 1) / rounds;
       const int at_once_min_steps = p.fast ? kLaneWavesMinSteps : 1;
       const int rounds_min_steps = !(p.fast && outgrown)                             ? kLaneWavesMinSteps
-                                   : fits && e->fused_variant == 0                   ? (int)std::min<size_t>(40, std::max<size_t>(kLaneWavesMinSteps, e->K / 24))
+                                   : fits && e->fused_variant == 0                   ? (few_rounds ? kLaneFewRoundsMinSteps : (int)std::min<size_t>(40, std::max<size_t>(kLaneWavesMinSteps, e->K / 24)))
                                    : e->A == 4 && (long)e->N <= kMinEnvsInFlight     ? INT_MAX
                                    : (long)e->N <= kLaneRoundsManyEnvs               ? kLaneRoundsMinSteps
                                                                                      : kLaneRoundsManyMinSteps;

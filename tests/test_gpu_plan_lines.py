@@ -21,6 +21,8 @@ LDS, LANES, PLAIN, HYBRID = "k_fused_tickets_lds<%d,fast>", "k_fused_lanes<%d,fa
     (66001, 28, 28, 4, 130, PLAIN), (66001, 28, 28, 4, 131, LANES),  # of more
     (250001, 8, 8, 4, 9, PLAIN), (250001, 8, 8, 4, 10, LANES),       # in place of hybrid workgroups
     (250001, 8, 8, 4, 71, LANES), (250001, 8, 8, 4, 72, HYBRID),
+    (94001, 12, 12, 4, 47, PLAIN), (94001, 12, 12, 4, 48, LANES),    # ... where they are few rounds
+    (200001, 8, 8, 4, 5, PLAIN), (200001, 8, 8, 4, 6, PLAIN),        # all envs in flight, a limit on them
 ])
 def test_lines(gpu, oracle, N, W, H, A, steps, kernel):
     cls, start = gpu.gen_maps_bernoulli(7, N, N, W, H, 0.12, 0.08)
