@@ -1239,7 +1239,7 @@ int run_persist(crl_engine* e, int n_steps, bool* launched) {
   if (!p.ok) return CRL_OK;
   int rc;
   unsigned long long* buf;
-  if (p.hashed && !e->no_alloc && p.words > e->exchange.n) {
+  if (!e->no_alloc && p.words > e->exchange.n) {
     // (a stream being captured allows no allocation: two launches per step record such a call)
     bool recorded;
     rc = query_capture(e, &recorded);
@@ -1967,8 +1967,12 @@ int run_fused(crl_engine* e, int32_t n_steps, bool no_alloc) {
     // A call of a few steps takes two launches to a step and a longer one the one-launch kernel:
     // whichever comes first makes room for both, so that neither allocates later and both can be
     // recorded.  (Not calls of one to three steps: the larger allocation costs a first call 20 us,
-    // 6 steps of 300 envs 66 / 85.)
-    const size_t words = n_steps > 3 ? persist_words(e) : 0;
+    // 6 steps of 300 envs 66 / 85.  Not a call that is being recorded, which may allocate nothing: it
+    // makes do with the cells that calls before it have left.)
+    bool capturing = false;
+    if (e->recorded) rc = query_capture(e, &capturing);  // (state_changes has noted this call)
+    if (rc) return rc;
+    const size_t words = n_steps > 3 && !capturing ? persist_words(e) : 0;
     for (int k = 0; !launched && k < n_steps; ++k) {
       rc = shared_step(e, e->t + (uint64_t)k, e->trace_cursor, words);
       if (rc) return rc;
