@@ -168,7 +168,8 @@ struct MovesGlobal {
 // resulting cell), `cr` its per-cell rewards (or null), `tab` its table.
 // The step rule is step_rule()'s, restated on move codes: the class of the
 // target cell is two bits of the codes of the cell the env stands on.
-template <int A, class Table, class Moves>
+// THREE: which form of Philox (xor3).
+template <int A, bool THREE, class Table, class Moves>
 __device__ __forceinline__ void run_env_steps(const Rules& R, const Ptrs& P, const int env,
                                               const uint64_t t0, const int n_steps, const Moves moves,
                                               const uint32_t* __restrict__ own_map,
@@ -200,7 +201,7 @@ __device__ __forceinline__ void run_env_steps(const Rules& R, const Ptrs& P, con
     on_goal = cell_class_of(own_map[s >> 4], s) == kGoal;
     start_goal = cell_class_of(own_map[start >> 4], start) == kGoal;
   }
-  Philox4 blk = explore_block(R.seed, (uint32_t)env, t0 >> 1);
+  Philox4 blk = explore_block<THREE>(R.seed, (uint32_t)env, t0 >> 1);
   // Epsilon of a per-episode schedule stays in a register and is looked up again
   // only when an episode of the wave ends: as a load at the top of every step it
   // was a second round trip to memory per step, in front of the action.
@@ -274,7 +275,7 @@ __device__ __forceinline__ void run_env_steps(const Rules& R, const Ptrs& P, con
     mv = moves.at(s, x, y);
     // the next step's draws depend on nothing: the Philox rounds run while the
     // loads are in flight
-    if ((t & 1) == 1) blk = explore_block(R.seed, (uint32_t)env, (t + 1) >> 1);
+    if ((t & 1) == 1) blk = explore_block<THREE>(R.seed, (uint32_t)env, (t + 1) >> 1);
     const float m = row_max(row2, done, R.max_mode);
     const float qn = td_value(row_get(row, a), reward, m, R.lr, R.gamma);
     tab.store(s0, a, qn);
@@ -1135,13 +1136,13 @@ __global__ __launch_bounds__(256) void k_fused_per_env(const Rules R, const Ptrs
         if (FAST)
           run_env_fast<A, true>(R, P, env, t0, n_steps, MovesLds<A>{lds, 1}, cr, tab);
         else
-          run_env_steps<A>(R, P, env, t0, n_steps, MovesLds<A>{lds, 1}, own_map, cr, tab);
+          run_env_steps<A, true>(R, P, env, t0, n_steps, MovesLds<A>{lds, 1}, own_map, cr, tab);
       } else {
         const MovesGlobal<A> moves{P.moves + (P.map_shared ? 0 : (size_t)env * P.mv_words)};
         if (FAST)
           run_env_fast<A, true>(R, P, env, t0, n_steps, moves, cr, tab);
         else
-          run_env_steps<A>(R, P, env, t0, n_steps, moves, own_map, cr, tab);
+          run_env_steps<A, true>(R, P, env, t0, n_steps, moves, own_map, cr, tab);
       }
     }
   }
@@ -1371,7 +1372,7 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
         else if (FAST)
           run_env_fast<A, RICH>(R, P, env, t0, n_steps, MovesFromMap<A>{my_words + lane, R.W, R.H}, RICH ? cr : nullptr, tab);
         else
-          run_env_steps<A>(R, P, env, t0, n_steps, MovesFromMap<A>{my_words + lane, R.W, R.H},
+          run_env_steps<A, false>(R, P, env, t0, n_steps, MovesFromMap<A>{my_words + lane, R.W, R.H},
                            P.map + (size_t)env * P.map_words, cr, tab);
       }
     } else {
@@ -1405,7 +1406,7 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
       __builtin_amdgcn_wave_barrier();
       if (live) {
         const LdsTable<A> tab{tabs + lane * tab_stride};
-        run_env_steps<A>(R, P, env, t0, n_steps, MovesFromMap<A>{my_words + lane, R.W, R.H},
+        run_env_steps<A, false>(R, P, env, t0, n_steps, MovesFromMap<A>{my_words + lane, R.W, R.H},
                          P.map + (size_t)env * P.map_words, cr, tab);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
