@@ -751,9 +751,8 @@ constexpr int kNoEvents = 0, kEpsilonEvents = 1, kAllEvents = 2;
 // at LDS address 0, where dynamic LDS starts in a kernel without any other; CELLS: `cell_rewards` of the cells of the wave's first env (or of the shared map) also count.  EVENTS: an
 // episode's end changes more than where the env stands: epsilon by episode (kEpsilonEvents), or any of
 // that, episode statistics and an episode budget (kAllEvents).  Epsilon alone needs one loop and none of
-// the statistics' registers: 78 in place of 104, six waves to a SIMD in place of four (43,662 envs of
-// 10x10 with 8 actions, 300 steps: 278 -> 218 us; 4096 of
-// 16x16 in LDS, with the look-up that has no branch, 94 -> 72).
+// the statistics' registers (43,662 envs of 10x10 with 8 actions, 300 steps, with a form of its own
+// 278 -> 218 us; 4096 of 16x16 in LDS, with the look-up that has no branch, 94 -> 72).
 // The row of the cell the move ends on (for the TD target) and that of the cell the env acts
 // from next - another one only where its episode ended - are asked for together.
 template <int A, bool CELLS, int EVENTS, class Mem>
@@ -798,9 +797,16 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
   limits.ask(R, P, log_envs, t0 & ~(uint64_t)1, lane);
   for (uint64_t tb = t0 & ~(uint64_t)1; tb < t_end; tb += (uint64_t)tape_steps) {
     wave_fence();
-    write_tape<A>(R, env0, log_envs, tb, tape_steps, tape, lane, limits);
+    // (Where registers are short the lane's places on the tape are worked out anew for every tape, and
+    // its env's places in the state anew at the end: kept over the steps they took 30 registers, and of
+    // the 105 of kAllEvents in k_fused_lanes only four waves fit a SIMD where plan_fused counts on six -
+    // the last of 17 to 24 waves to a compute unit had to wait.  34,816 envs of 10x45 with 8 actions and
+    // statistics, 13 / 100 steps 29.8 / 125 us with them.)
+    int lane_now = lane;
+    if (kAll) asm volatile("" : "+v"(lane_now));
+    write_tape<A>(R, env0, log_envs, tb, tape_steps, tape, lane_now, limits);
     wave_fence();
-    limits.ask(R, P, log_envs, tb + (uint64_t)tape_steps, lane);
+    limits.ask(R, P, log_envs, tb + (uint64_t)tape_steps, lane_now);
     const int k0 = tb < t0 ? 1 : 0;  // (the first block may start with a step of the launch before)
     const int k1 = (int)min((uint64_t)tape_steps, t_end - tb);
     // (whether an env can use up its budget in these steps)
@@ -903,6 +909,8 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
   }
 
   if (lane == slot * A) {
+    int env = env0 + slot;
+    asm volatile("" : "+v"(env));  // (see above)
     P.s[env] = (int)(mem.offset(at) / Mem::kRow);
     P.ep_step[env] = whole - left;
     P.episode[env] = episode;
@@ -1157,7 +1165,7 @@ __global__ __launch_bounds__(256) void k_fused_per_env(const Rules R, const Ptrs
 // trips and 150 instructions.
 // LDS: the rewards by class, the tape, the codes env by env.
 template <int A, bool CELLS, int EVENTS>
-__global__ __launch_bounds__(64) void k_fused_lanes(const Rules R, const Ptrs P, const uint64_t t0, const int n_steps,
+__global__ __launch_bounds__(64, 6) void k_fused_lanes(const Rules R, const Ptrs P, const uint64_t t0, const int n_steps,
                                                     unsigned* __restrict__ ticket, const int dealt, const int touch,
                                                     const int log_envs, const int tape_steps) {
   extern __shared__ __align__(16) uint32_t lds[];
