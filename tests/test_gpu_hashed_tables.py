@@ -9,23 +9,34 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def run(gpu, oracle, cfg, cls, start, calls, variant=2, trace=False):
-    W, H, A = cfg.width, cfg.height, cfg.n_actions
+def run(gpu, oracle, cfg, cls, start, calls, variant=2, trace=False, cell_reward=None, stream=None):
+    N, W, H, A, total = cfg.n_envs, cfg.width, cfg.height, cfg.n_actions, sum(calls)
     with gpu.Engine(cfg, 0) as eng:
-        eng.set_maps(cls, start)
+        eng.set_maps(cls, start, cell_reward)
         eng.set_fused_variant(variant)
         if trace:
-            eng.set_trace(cfg.n_envs, sum(calls))
+            eng.set_trace(N, total)
+        if stream is not None:
+            eng.set_exploration_stream(*stream)
         name = eng.fused_kernel_info(max(calls))["name"]
         for n in calls:
             eng.run_fused(n)
         q, st = eng.q_get(0), eng.get_state()
+        rows = eng.get_trace(total) if trace else None
+        stats = eng.episode_stats() if cfg.track_returns else None
     Q = np.zeros((1, W * H, A), np.float32)
     ost = oracle.new_state(cfg, start)
-    oracle.run(cfg, cls, None, start, Q, ost, 0, sum(calls))
+    ostats = oracle.new_stats(N) if cfg.track_returns else None
+    u, a_rand = stream if stream is not None else (None, None)
+    want = oracle.run(cfg, cls, cell_reward, start, Q, ost, 0, total, u=u, a_rand=a_rand, trace_n=N if trace else 0,
+                      stats=ostats)
     assert np.array_equal(q, Q[0], equal_nan=True)
     for k in ("s", "ep_step", "episode", "reward", "done", "action"):
         assert np.array_equal(st[k], ost[k]), k
+    for k in rows or ():
+        assert np.array_equal(rows[k], want[k]), k
+    for k in stats or ():
+        assert np.array_equal(stats[k], ostats[k]), k
     return name, q
 
 
@@ -49,6 +60,38 @@ def test_general_rules(gpu, oracle, options):
     cfg = gpu.make_config(N, W, H, table_mode=gpu.TABLE_SHARED, map_mode=gpu.MAP_SHARED, lr=1e-3, eps0=0.4, seed=8, **options)
     name, _ = run(gpu, oracle, cfg, cls, start, (30, 20))
     assert name == "k_shared_persist<4,1,hashed>"
+
+
+@pytest.mark.parametrize("A", [4, 8])
+@pytest.mark.parametrize("shared_map", [True, False])
+@pytest.mark.parametrize("form", ["plain", "trace", "cells", "cells for all", "stream", "all"])
+def test_maps_and_every_output(gpu, oracle, A, shared_map, form):
+    """The map staged in LDS and a map per env from global memory, with what the other tests leave out:
+    trace rows (also of envs whose budget is used up), rewards by cell, supplied draws, statistics."""
+    N, W, H, calls = 700, 67, 63 if A == 4 else 40, (21, 12)
+    cells = {"cells": 1, "cells for all": 3, "all": 3}.get(form, 0)
+    options = dict(max_episodes=2, episode_len=6, track_returns=1) if form in ("trace", "all") else dict(episode_len=13)
+    n_maps = 1 if shared_map else N
+    if cells:
+        cls, start, cr = gpu.gen_maps_noise(5, n_maps, W, H, 8, 0.2, 0.3, 5.0)
+        if shared_map:
+            start = np.random.default_rng(5).choice(np.flatnonzero(cls[0] == 0), N).astype(np.int32)
+    else:
+        (cls, start), cr = gpu.gen_maps_bernoulli(5, n_maps, N, W, H, 0.12, 0.05), None
+    start[N // 2:] = start[:N - N // 2]  # (keys that several blocks hold)
+    if not shared_map:
+        cls[N // 2:] = cls[:N - N // 2]
+        if cells:
+            cr[N // 2:] = cr[:N - N // 2]
+    stream = None
+    if form in ("stream", "all"):
+        rng = np.random.default_rng(A)
+        stream = rng.random((sum(calls), N), dtype=np.float32), rng.integers(0, A, (sum(calls), N)).astype(np.int32)
+    cfg = gpu.make_config(N, W, H, n_actions=A, table_mode=gpu.TABLE_SHARED, reward_flags=cells, lr=0.02, eps0=0.4, seed=12,
+                          map_mode=gpu.MAP_SHARED if shared_map else gpu.MAP_PER_ENV, trap_reward=-0.5, **options)
+    name, q = run(gpu, oracle, cfg, cls, start, calls, trace=form in ("trace", "all"), cell_reward=cr, stream=stream)
+    folded = ",folded" if form == "plain" else ""
+    assert name == "k_shared_persist<%d,%d%s,hashed>" % (A, 1 if shared_map else 2, folded) and np.count_nonzero(q) > 100
 
 
 @pytest.mark.parametrize("cells,envs", [(1, 20000), (3, 20000), (64, 3000), (64, 65536)])
