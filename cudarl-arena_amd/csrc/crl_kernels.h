@@ -797,16 +797,9 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
   limits.ask(R, P, log_envs, t0 & ~(uint64_t)1, lane);
   for (uint64_t tb = t0 & ~(uint64_t)1; tb < t_end; tb += (uint64_t)tape_steps) {
     wave_fence();
-    // (Where registers are short the lane's places on the tape are worked out anew for every tape, and
-    // its env's places in the state anew at the end: kept over the steps they took 30 registers, and of
-    // the 105 of kAllEvents in k_fused_lanes only four waves fit a SIMD where plan_fused counts on six -
-    // the last of 17 to 24 waves to a compute unit had to wait.  34,816 envs of 10x45 with 8 actions and
-    // statistics, 13 / 100 steps 29.8 / 125 us with them.)
-    int lane_now = lane;
-    if (kAll) asm volatile("" : "+v"(lane_now));
-    write_tape<A>(R, env0, log_envs, tb, tape_steps, tape, lane_now, limits);
+    write_tape<A>(R, env0, log_envs, tb, tape_steps, tape, lane, limits);
     wave_fence();
-    limits.ask(R, P, log_envs, tb + (uint64_t)tape_steps, lane_now);
+    limits.ask(R, P, log_envs, tb + (uint64_t)tape_steps, lane);
     const int k0 = tb < t0 ? 1 : 0;  // (the first block may start with a step of the launch before)
     const int k1 = (int)min((uint64_t)tape_steps, t_end - tb);
     // (whether an env can use up its budget in these steps)
@@ -909,8 +902,13 @@ __device__ __forceinline__ void run_lanes(const Rules& R, const Ptrs& P, const i
   }
 
   if (lane == slot * A) {
+    // (The addresses of the env's state worked out anew: kept over the steps they take 12 registers, and
+    // of the 105 of kAllEvents in k_fused_lanes only four waves fit a SIMD - the last of 17 to 24 waves
+    // to a compute unit wait.  34,816 envs of 9x8 with 8 actions, statistics, epsilon by episode, 13 / 100
+    // steps 21.0 / 88.7 us with them.  Working the lane's places on the tape out anew as well makes it 75, six
+    // waves, and costs 2 to 4 per cent of every launch.)
     int env = env0 + slot;
-    asm volatile("" : "+v"(env));  // (see above)
+    if (kAll || (CELLS && EVENTS != kNoEvents)) asm volatile("" : "+v"(env));
     P.s[env] = (int)(mem.offset(at) / Mem::kRow);
     P.ep_step[env] = whole - left;
     P.episode[env] = episode;
@@ -1165,7 +1163,7 @@ __global__ __launch_bounds__(256) void k_fused_per_env(const Rules R, const Ptrs
 // trips and 150 instructions.
 // LDS: the rewards by class, the tape, the codes env by env.
 template <int A, bool CELLS, int EVENTS>
-__global__ __launch_bounds__(64, 6) void k_fused_lanes(const Rules R, const Ptrs P, const uint64_t t0, const int n_steps,
+__global__ __launch_bounds__(64, EVENTS == kAllEvents ? 5 : 6) void k_fused_lanes(const Rules R, const Ptrs P, const uint64_t t0, const int n_steps,
                                                     unsigned* __restrict__ ticket, const int dealt, const int touch,
                                                     const int log_envs, const int tape_steps) {
   extern __shared__ __align__(16) uint32_t lds[];

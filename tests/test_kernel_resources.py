@@ -35,10 +35,11 @@ def kernels(tmp_path_factory):
     return found
 
 
-def test_lane_waves_fit_six_to_a_simd(kernels):
-    """plan_fused puts up to 24 lane waves on a compute unit: 512 / 6 registers, in eights."""
+def test_lane_waves_to_a_simd(kernels):
+    """plan_fused puts up to 24 lane waves on a compute unit, 20 with episode statistics or a budget (the
+    third form): 512 / 6 and 512 / 5 registers, in eights."""
     lanes = {k: v for k, v in kernels.items() if "k_fused_lanes" in k}
     assert len(lanes) == 12
     for name, got in lanes.items():
-        assert got["vgpr_count"] <= 80, (name, got)
+        assert got["vgpr_count"] <= (96 if "ELi2EEE" in name else 80), (name, got)
         assert got["private_segment_fixed_size"] == 0 and got["vgpr_spill_count"] == 0, (name, got)
