@@ -384,7 +384,7 @@ constexpr size_t kStaticLdsReserve = 1024;
 constexpr int kHybridMinSteps = 64;
 constexpr int kStagedMovesMinSteps = 128;
 constexpr int kLdsMinSteps = 16, kLdsAlwaysSteps = 144;
-constexpr size_t kLdsBytesFree = 8192, kLdsBytesPerStep = 208;
+constexpr size_t kLdsBytesFree = 8192, kLdsBytesPerStep = 208, kLdsSmallWaveBytes = 5120, kLdsSmallMoved = 17000;
 constexpr int kLongLaunchSteps = 4096;
 constexpr int kLaneWavesMinSteps = 8;
 constexpr int kLaneRoundsMinSteps = 64, kLaneRoundsManyMinSteps = 131;
@@ -437,7 +437,13 @@ bool plan_fused_lds(const crl_engine* e, int n_steps, FusedPlan* p) {
     // 12.7 / 11.7, 14.9 / 15.5 us; 2000 of 32x32, 32 KB, 64 / 128 / 200 steps 22.0 / 18.9, 30.5 / 30.6,
     // 40.3 / 44.4; 30,000 of 8x8, eight waves of 16 KB to a unit, 64 / 128 steps 29.5 / 25.2, 42.9 / 43.3;
     // 100 of 48x48 with 8 actions, 72 KB, 128 / 200 steps 30.4 / 28.1, 39.6 / 41.4).
-    const size_t moved = std::max<size_t>((4 * e->K) << log_envs, ((4 * e->K) << log_envs) * per_unit / 4);
+    // The smallest tables of 4 actions (up to 5 KB to a wave) cross sooner, beside their move words at
+    // once (15.5 waves to a unit, 4x4, 16 / 32 steps: 13.1 / 17.6, 15.4 / 23.3 us; 12 waves, 5x4, 32 steps 16.4,
+    // 20.2), beside move codes at some 40 steps (24 waves, 4x4, 32 / 64 steps 32.6 / 48.2, 34.9 / 62.6; 20 waves,
+    // 5x4 29.9 / 43.3, 33.3 / 54.7).
+    const size_t wave_bytes = (4 * e->K) << log_envs;
+    size_t moved = std::max<size_t>(wave_bytes, wave_bytes * per_unit / 4);
+    if (e->A == 4 && wave_bytes <= kLdsSmallWaveBytes) moved = words ? wave_bytes : std::min(moved, kLdsSmallMoved);
     if (n_steps < kLdsAlwaysSteps && (size_t)n_steps * kLdsBytesPerStep + kLdsBytesFree < moved) return false;
     p->in_lds = p->lanes = p->fast = true;
     p->words = words != 0;
