@@ -349,7 +349,10 @@ constexpr long kMinEnvsInFlight = kComputeUnits * 3L * 64;  // three waves per c
 // Shorter launches have all envs in flight (all / as many as that, 2 / 4 / 6 / 8 / 12 steps: 1M envs of 16x16
 // 107 / 176 / 251 / 332 / 503 us, 127 / 175 / 225 / 275 / 378; 100,000 of 32x32 27 / 34 / 41 / 48 / 66,
 // 28 / 35 / 42 / 48 / 61; 200,000 of 16x16 with 8 actions 31 / 52 / 73 / 94 / 136, 31 / 46 / 60 / 74 / 104).
-constexpr int kInFlightMinSteps = 6;
+// The general loop on a shared map, 4 actions, loses by two shifts (20x20, 80,000 envs, statistics and epsilon by
+// episode, 6 / 14 steps 21.0 / 42.7, 24.4 / 47.1; three shifts of 16x16, 14 steps 80.9, 69.5; with 8 actions, two of
+// 20x20, 55.1, 51.0; two of 60x60, 9 steps 29.7, 28.5).
+constexpr int kInFlightMinSteps = 6, kInFlightMinStepsTwoShifts = 16;
 
 // launch geometry of the fused per-env kernel
 struct FusedPlan {
@@ -487,6 +490,11 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       p.map_kind = 2;
     }
   }
+  const crl_config& c = e->cfg;
+  // what the folded loop leaves out altogether ...
+  const bool foldable = c.goal_mode == CRL_GOAL_ON_TARGET && c.auto_reset == 1 && c.max_mode == CRL_MAX_TRUE &&
+                        e->trace_n == 0 && e->sup_n == 0 && c.max_episodes == 0 && c.track_returns == 0 &&
+                        e->mv_words > 0;
   // Envs live on the chip at once.  A worker steps its envs for all n steps
   // before it takes the next ones, so a smaller grid means fewer tables in
   // flight: when all tables together exceed what the last-level cache holds well,
@@ -497,8 +505,11 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     resident = e->N;
     // (a launch of a few steps re-uses no row often enough for that to matter: it
     // runs with every env in flight)
-    if ((size_t)e->N * table_bytes > kTableBytesInFlight && n_steps >= kInFlightMinSteps)
-      resident = std::max<long>(kMinEnvsInFlight, (long)(kTableBytesInFlight / table_bytes));
+    const long fits = std::max<long>(kMinEnvsInFlight, (long)(kTableBytesInFlight / table_bytes));
+    const bool general = !foldable || c.eps_mode == CRL_EPS_STEP_MULT;
+    const bool two_shifts = p.map_kind == 1 && general && e->A == 4 && e->K < 4096 && e->N <= 2 * fits;
+    if ((size_t)e->N * table_bytes > kTableBytesInFlight && n_steps >= (two_shifts ? kInFlightMinStepsTwoShifts : kInFlightMinSteps))
+      resident = fits;
     // The batch goes through the chip in shifts of that many envs; a last shift that
     // fills a fraction of the chip costs a whole one.  Even the shifts out, in whole
     // waves per compute unit (65,536 envs with 32x32 maps: 3.5e10 env-steps/s as one
@@ -511,11 +522,6 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     }
   }
   p.tickets = p.map_kind == 0;
-  const crl_config& c = e->cfg;
-  // what the folded loop leaves out altogether ...
-  const bool foldable = c.goal_mode == CRL_GOAL_ON_TARGET && c.auto_reset == 1 && c.max_mode == CRL_MAX_TRUE &&
-                        e->trace_n == 0 && e->sup_n == 0 && c.max_episodes == 0 && c.track_returns == 0 &&
-                        e->mv_words > 0;
   if (!p.tickets) {
     p.grid = (int)std::min<long>((e->N + p.block - 1) / p.block, std::max<long>(1, resident / p.block));
     // ... its variant for large or shared maps takes per-cell rewards and per-episode epsilon
