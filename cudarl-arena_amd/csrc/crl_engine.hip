@@ -398,7 +398,7 @@ constexpr int kLaneDrawnMinSteps = 256, kLaneDrawnManyMinSteps = 128;
 constexpr int kLaneTouchMinSteps4 = 90, kLaneTouchMinSteps8 = 160;
 // Hybrid workgroups in place of rounds of lane waves.
 constexpr int kHybridFewRoundsMinSteps = 384;
-constexpr long kHybridEnvStepsSmall = 18000000, kHybridEnvSteps4 = 24000000, kHybridEnvSteps8 = 28000000;
+constexpr long kHybridEnvStepsSmall = 18000000, kHybridEnvSteps4 = 24000000, kHybridEnvSteps8 = 28000000, kHybridEnvSteps8FewRounds = 20000000;
 constexpr size_t kTableBytesAtOnce = (size_t)512 << 20;
 
 // Configurations that run_lanes() steps: no goal test on the resulting cell, no sticky done,
@@ -622,15 +622,21 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     // enough to step (lane waves / hybrid, 8x8 maps: 1M envs, 16 / 32 / 64 steps 433 / 703 / 938, 405 / 571 / 776 us; 200,000, 64 / 96 steps 179 / 190,
     // 249 / 236; 16x16: 1M envs, 64 / 96 steps 1515 / 1682, 2174 / 1945 us; 180,000, 96 / 128 steps 396 / 414, 489 / 469;
     // 140,000, 160 / 256 steps 385 / 408, 588 / 551; 8 actions, 160,000 of 12x12, 128 / 256 steps
-    // 471 / 503, 874 / 794), and not where the lane waves have few rounds: 95,000, three of them, 256 /
-    // 500 steps 353 / 383, 662 / 634; 8 actions, 73,000, three, 500 / 1000 steps 682 / 830, 1302 / 1484.
-    const bool few_rounds = rounds <= (e->A == 8 ? 4 : 3);
+    // 471 / 503, 874 / 794; four rounds of 8 actions from 20 million env-steps on: 94,000 of 19x12, 200 / 440 steps
+    // 546 / 1128, 520 / 892; 98,000 of 9x9, 256 steps 420, 404).  Where the lane waves have at most three rounds
+    // they are late by less, and the larger a table the sooner hybrid workgroups pay: 95,000 of 12x12, 256 / 500 steps
+    // 322 / 546, 316 / 541, of 16x16 429, 375; 73,000 of 26x18, 256 / 367 steps 465 / 657, 465 / 602; 80,000 of 20x20, 200 /
+    // 256 steps 379 / 477, 383 / 450; 8 actions, 73,000 of 12x12, 500 / 1000 steps 644 / 1189, 722 / 1354, of 16x16 960 / 1729,
+    // 898 / 1574; 70,000 of 19x12, 440 steps 782, 745.
+    const bool few_rounds = rounds <= 3;
+    const int few_rounds_min_steps = e->A == 8 ? (e->K >= 1536 ? 400 : INT_MAX) : e->K >= 1024 ? 256 : kHybridFewRoundsMinSteps;
     const bool hybrid_pays =
-        few_rounds ? e->A == 4 && n_steps >= kHybridFewRoundsMinSteps
+        few_rounds ? n_steps >= few_rounds_min_steps
                    : 64L * n_steps >= 5L * (long)e->K &&
                          (long)e->N * n_steps >= (e->K < 512   ? kHybridEnvStepsSmall
-                                                  : e->A == 8 ? kHybridEnvSteps8
-                                                              : kHybridEnvSteps4);
+                                                  : e->A == 4 ? kHybridEnvSteps4
+                                                  : rounds > 4 ? kHybridEnvSteps8
+                                                               : kHybridEnvSteps8FewRounds);
     // ... (automatic) when the tables outgrow the caches: while they all fit, other plans are
     // faster (16x16 maps, 30,000 envs: 3.5e10 hybrid, 5.9e10 with lane waves); and where lane
     // waves could step what is left to the general loop, they are faster too (262,144 envs of
