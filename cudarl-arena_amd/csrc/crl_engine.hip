@@ -380,6 +380,12 @@ constexpr size_t kLdsPerWorkgroup = 160 * 1024;  // gfx950
 // static LDS of kernels that call the workgroup-wide "or" (the device library keeps a few
 // words there), rounded up: their dynamic LDS can be at most the rest
 constexpr size_t kStaticLdsReserve = 1024;
+// How many workgroups that ask for `bytes` fit a compute unit: LDS is given out in pieces of 1280 bytes.
+// (Counted in 1024, lane waves of 45x19 maps, 8 actions, 14,240 bytes, were put 11 to a unit where 10 fit, and the
+// eleventh ran after the others: 131 steps, 10 / 11 to a unit 96 / 150 us; of 24x20, 8240 bytes, 17 / 18 / 19
+// 132 / 142 / 190; of 28x25, 11,760 bytes, 12 / 13 105 / 157.)
+constexpr size_t kLdsPiece = 1280;
+constexpr long lds_fit(size_t bytes) { return (long)(kLdsPerWorkgroup / ((bytes + kLdsPiece - 1) / kLdsPiece * kLdsPiece)); }
 
 // Launches shorter than this do not repay moving whole tables into LDS and back
 // (1M envs of config 4, steps per launch -> env-steps/s, plain / hybrid:
@@ -393,6 +399,7 @@ constexpr int kLaneWavesMinSteps = 8;
 constexpr int kLaneRoundsMinSteps = 64, kLaneRoundsManyMinSteps = 131;
 constexpr int kLaneFewRoundsMinSteps = 48;
 constexpr long kLaneRoundsManyEnvs = 65536;
+constexpr int kLaneLateWavesMinSteps = 384;
 constexpr int kLaneRoundsFourMinSteps = 64, kLaneRoundsFourLongSteps = 300;
 constexpr int kLaneDrawnMinSteps = 256, kLaneDrawnManyMinSteps = 128;
 constexpr int kLaneTouchMinSteps4 = 90, kLaneTouchMinSteps8 = 160;
@@ -434,6 +441,9 @@ bool plan_fused_lds(const crl_engine* e, int n_steps, FusedPlan* p) {
   const size_t env_bytes[2] = {((4 * e->K + (shared ? 0 : code_bytes) + 15) & ~(size_t)15) + 16, 8 * e->K + 16};
   for (int words = 1; words >= 0; --words) {
     const size_t bytes = 16 + (env_bytes[words] << log_envs) + tape_bytes(log_envs) + (shared && !words ? code_bytes : 0);
+    // (pieces of 1024 bytes, not the 1280 of lds_fit: a unit's last wave may run after the others.  With the smallest
+    // tables that is better than lane waves on HBM - 77,524 envs of 4x6, 160 / 500 steps 107 / 297 us, 120 / 357 - with
+    // larger ones worse: 20,180 of 19x6 94 / 223, 54 / 153.)
     if (((bytes + 1023) & ~(size_t)1023) * per_unit > kLdsPerWorkgroup) continue;
     // What a wave's tables, or a quarter of a compute unit's, take to move in and out against the
     // steps' trips to HBM (tables in LDS / in HBM: 4096 envs of 16x16, 16 KB to a wave, 32 / 48 steps
@@ -589,7 +599,7 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     int lane_log_envs = most_log_envs;
     while (lane_log_envs > 0 && (e->N + (1L << lane_log_envs) - 1) >> lane_log_envs < spread) --lane_log_envs;
     const size_t lane_lds = 16 + tape_bytes(lane_log_envs) + ((size_t)e->mv_words * 4 << lane_log_envs);
-    const long lane_fit = lane_lds <= kLdsPerWorkgroup ? (long)(kLdsPerWorkgroup / ((lane_lds + 1023) & ~(size_t)1023)) : 0;  // waves of a compute unit
+    const long lane_fit = lds_fit(lane_lds);  // waves of a compute unit
     const long lane_units = (e->N + (1L << lane_log_envs) - 1) >> lane_log_envs;
     const bool lanes_can = lanes_rules(e) && (e->K * sizeof(float)) << lane_log_envs < (size_t)1 << 32;
     const size_t all_tables = (size_t)e->N * e->K * sizeof(float);
@@ -697,7 +707,12 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
                                    : e->A == 4 && (long)e->N <= kMinEnvsInFlight     ? INT_MAX
                                    : (long)e->N <= kLaneRoundsManyEnvs               ? kLaneRoundsMinSteps
                                                                                      : kLaneRoundsManyMinSteps;
-      const bool rounds_ok = lane_waves <= kComputeUnits * lane_fit && n_steps >= rounds_min_steps;
+      // (one wave more to a compute unit than fits, which runs when another has ended: 67,000 envs of 45x19 with 8
+      // actions, 131 / 400 / 800 steps, 64-env waves 380 / 1052 / 2053, lane waves 502 / 1002 / 1890, in a fourth round
+      // instead 384 / 1050 / 1977; 45,000, fewer than three 64-env waves to a unit, 227 / 594 / 1175, 327 / 718 / 1340)
+      const bool late_waves = lane_waves > kComputeUnits * lane_fit;
+      const bool late_pay = !p.fast || (outgrown && (long)e->N > kLaneRoundsManyEnvs && n_steps >= kLaneLateWavesMinSteps);
+      const bool rounds_ok = (late_waves ? late_pay && lane_waves <= kComputeUnits * (lane_fit + 1) : true) && n_steps >= rounds_min_steps;
       if (lanes_can && (small ? lane_fit > 0 : lanes_at_once ? n_steps >= at_once_min_steps : rounds_ok)) {
         p.fast = p.moves = p.lanes = true;
         p.rich = c.eps_mode >= CRL_EPS_EPISODE_MULT || c.reward_flags != 0;

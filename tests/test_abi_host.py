@@ -228,6 +228,19 @@ def test_every_valid_configuration_has_a_launch_plan_that_fits(pycrl):
         pycrl.fused_plan_for_config(pycrl.make_config(64, 8, 8, table_mode=pycrl.TABLE_SHARED), 10)
 
 
+@pytest.mark.parametrize("N,W,H,A,n_steps,name,grid", [
+    # 14,240 bytes of LDS to a wave: 12 pieces of 1280, ten waves to a compute unit
+    (67000, 45, 19, 8, 131, "k_fused_tickets<8,fast,hbm>", 256), (67000, 45, 19, 8, 383, "k_fused_tickets<8,fast,hbm>", 256),
+    (67000, 45, 19, 8, 384, "k_fused_lanes<8,fast>", 2792),  # long calls: an eleventh that runs late
+    (100000, 45, 19, 8, 131, "k_fused_lanes<8,fast>", 2500), (45000, 45, 19, 8, 800, "k_fused_tickets<8,fast,hbm>", 704),
+    # 8272 bytes: seven pieces, eighteen to a unit
+    (73728, 21, 21, 4, 131, "k_fused_lanes<4,fast>", 4608), (73729, 21, 21, 4, 131, "k_fused_lanes<4,fast>", 1537),
+])
+def test_lane_waves_are_as_many_as_fit_a_compute_unit(pycrl, N, W, H, A, n_steps, name, grid):
+    plan = pycrl.fused_plan_for_config(pycrl.make_config(N, W, H, n_actions=A, episode_len=128), n_steps)
+    assert (plan["name"], plan["grid"]) == (name, grid)
+
+
 def test_npy_agent_files_match_numpy(pycrl, tmp_path):
     """QTableAgent.save / load files (src/train.py:150-168): float64 (W, H, A)
     indexed [x, y, a], exchanged with numpy in both directions."""
