@@ -402,7 +402,7 @@ constexpr long kLaneRoundsManyEnvs = 65536;
 constexpr int kLaneLateWavesMinSteps = 384;
 constexpr int kLaneRoundsFourMinSteps = 64, kLaneRoundsFourLongSteps = 300;
 constexpr int kLaneDrawnMinSteps = 256, kLaneDrawnManyMinSteps = 128;
-constexpr int kLaneTouchMinSteps4 = 90, kLaneTouchMinSteps8 = 160;
+constexpr int kLaneTouchMinSteps4 = 90, kLaneTouchMinSteps8 = 160, kLaneTouchFourRoundsMinSteps = 200;
 // Hybrid workgroups in place of rounds of lane waves.
 constexpr int kHybridFewRoundsMinSteps = 384;
 constexpr long kHybridEnvStepsSmall = 18000000, kHybridEnvSteps4 = 24000000, kHybridEnvSteps8 = 28000000, kHybridEnvSteps8FewRounds = 20000000;
@@ -726,9 +726,14 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
         // 1196 / 4774 us with, 483 / 701 / 1346 / 5276 without; 200,000 with 8 actions, 128 / 200 steps 841 /
         // 1142, 808 / 1179; 198,000 of
         // 10x30, seven rounds, 757 steps 2375, 2740; 120,000 of 16x16, four rounds, 200 / 1000 steps 488 / 1910,
-        // 373 / 1706)
-        p.touch = outgrown && many_rounds && n_steps >= (e->A == 8 ? kLaneTouchMinSteps8 : kLaneTouchMinSteps4) &&
-                  e->K <= (size_t)crl::kTouchFloats;
+        // 373 / 1706.  In four or five rounds where envs explore for long, epsilon by episode, tables of 4 KB on, with /
+        // without: 150,000 of 16x16, 131 / 200 / 329 / 700 steps 430 / 590 / 903 / 1804, 451 / 677 / 1075 / 2143; 149,286 of
+        // 27x11, 700 steps 1831, 2165; 110,000 of 21x21, 131 / 200 / 329 413 / 546 / 803, 368 / 545 / 875; 90,000 of 16x16 with 8
+        // actions 381 / 544 / 812, 384 / 569 / 901; not of 12x12: 4 actions 700 steps 1662, 1675, 8 actions 200 steps 472, 422)
+        const bool explores = by_episode && e->K >= (e->A == 8 ? 1536 : 1024) && 8L * n_steps >= (long)e->K &&
+                              n_steps >= kLaneTouchFourRoundsMinSteps && p.grid * 3L < lane_units;
+        p.touch = outgrown && e->K <= (size_t)crl::kTouchFloats &&
+                  (explores || (many_rounds && n_steps >= (e->A == 8 ? kLaneTouchMinSteps8 : kLaneTouchMinSteps4)));
         // (no more than it uses, also where there is a compute unit for every workgroup: 4096 envs
         // of 32x32, 10,000 steps, 17 / 64 / 81 KB 2.78 / 2.76 / 2.80 ms)
         p.lds = lane_lds;

@@ -65,3 +65,26 @@ def test_tables_read_ahead(gpu):
         assert all(np.array_equal(a[k], b[k]) for k in STATE)
         for at in range(0, N, 29500):
             assert np.array_equal(one.q_get(at, 29500), two.q_get(at, 29500))
+
+
+@pytest.mark.parametrize("N,W,H,A", [(98500, 16, 16, 4), (74000, 12, 16, 8)])
+def test_tables_read_ahead_in_four_rounds(gpu, N, W, H, A):
+    """Four rounds of lane waves, epsilon by episode: tables read ahead from 200 steps on, not in shorter calls."""
+    cls, start = gpu.gen_maps_bernoulli(7, N, N, W, H, 0.1, 0.02)
+    cfg = gpu.make_config(N, W, H, n_actions=A, episode_len=40, eps0=0.9, eps_mode=gpu.EPS_EPISODE_LINEAR, eps_end=0.1,
+                          eps_span=9, seed=3)
+    with gpu.Engine(cfg, 0) as one, gpu.Engine(cfg, 0) as two:
+        for e in (one, two):
+            e.set_maps(cls, start)
+        plan = one.fused_kernel_info(200)
+        assert plan["name"] == "k_fused_lanes<%d,fast>" % A
+        waves = -(-N // (64 // A))
+        assert 3 * plan["grid"] < waves <= 4 * plan["grid"]
+        for _ in range(2):
+            one.run_fused(200)
+            two.run_fused(199)
+            two.run_fused(1)
+        a, b = one.get_state(), two.get_state()
+        assert all(np.array_equal(a[k], b[k]) for k in STATE)
+        for at in range(0, N, N // 2):
+            assert np.array_equal(one.q_get(at, N // 2), two.q_get(at, N // 2))
