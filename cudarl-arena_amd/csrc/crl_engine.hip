@@ -404,7 +404,7 @@ constexpr int kLaneRoundsFourMinSteps = 64, kLaneRoundsFourLongSteps = 300;
 constexpr int kLaneDrawnMinSteps = 256, kLaneDrawnManyMinSteps = 128;
 constexpr int kLaneTouchMinSteps4 = 90, kLaneTouchMinSteps8 = 160, kLaneTouchFourRoundsMinSteps = 200;
 // Hybrid workgroups in place of rounds of lane waves.
-constexpr int kHybridFewRoundsMinSteps = 384;
+constexpr int kHybridFewRoundsMinSteps = 384, kHybridOneWaveMinSteps = 96;
 constexpr long kHybridEnvStepsSmall = 18000000, kHybridEnvSteps4 = 24000000, kHybridEnvSteps8 = 28000000, kHybridEnvSteps8FewRounds = 20000000;
 constexpr size_t kTableBytesAtOnce = (size_t)512 << 20;
 
@@ -627,26 +627,36 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     // 16: 5.0e10; 8 actions, 262,144 envs 8: 3.7e10, 12: 4.2e10, 16: 4.0e10).
     const long per_round = kComputeUnits * (!outgrown ? 16L : e->A == 8 ? 12L : 8L);
     const long rounds = (lane_units + per_round - 1) / per_round;
-    // Hybrid workgroups take a while to share out their envs, and their last table waves are late:
-    // they pay over rounds of lane waves once a table's steps are worth its way into LDS and there is
-    // enough to step (lane waves / hybrid, 8x8 maps: 1M envs, 16 / 32 / 64 steps 433 / 703 / 938, 405 / 571 / 776 us; 200,000, 64 / 96 steps 179 / 190,
-    // 249 / 236; 16x16: 1M envs, 64 / 96 steps 1515 / 1682, 2174 / 1945 us; 180,000, 96 / 128 steps 396 / 414, 489 / 469;
-    // 140,000, 160 / 256 steps 385 / 408, 588 / 551; 8 actions, 160,000 of 12x12, 128 / 256 steps
-    // 471 / 503, 874 / 794; four rounds of 8 actions from 20 million env-steps on: 94,000 of 19x12, 200 / 440 steps
-    // 546 / 1128, 520 / 892; 98,000 of 9x9, 256 steps 420, 404).  Where the lane waves have at most three rounds
-    // they are late by less, and the larger a table the sooner hybrid workgroups pay: 95,000 of 12x12, 256 / 500 steps
-    // 322 / 546, 316 / 541, of 16x16 429, 375; 73,000 of 26x18, 256 / 367 steps 465 / 657, 465 / 602; 80,000 of 20x20, 200 /
-    // 256 steps 379 / 477, 383 / 450; 8 actions, 73,000 of 12x12, 500 / 1000 steps 644 / 1189, 722 / 1354, of 16x16 960 / 1729,
-    // 898 / 1574; 70,000 of 19x12, 440 steps 782, 745.
+    // Hybrid workgroups take a while to share out their envs, and their last table waves are late: they pay
+    // over rounds of lane waves once a table's steps are worth its way into LDS and there is enough to step
+    // (lane waves / hybrid, us; launch after launch, from the first on):
+    //   8x8, 4 actions: 1M envs, 16 / 32 / 64 steps 433 / 703 / 938, 405 / 571 / 776; 200,000, 64 / 96 179 / 190, 249 / 236
+    //   up to 6 KB, 4 actions: 150,000 of 12x12, 96 / 131 235 / 305, 247 / 294; 200,000, 64 / 96 273 / 380, 261 / 325;
+    //     150,000 of 16x16, 96 / 131 329 / 440, 325 / 377; 140,000, 160 520, 420; 180,000, 96 / 131 409 / 498, 413 / 482;
+    //     8 actions, six rounds and more: 130,000 of 8x8, 96 / 131 246 / 327, 262 / 321; 200,000 96 / 131 380 / 491, 362 /
+    //     445; 150,000 of 12x12, 96 / 131 394 / 494, 388 / 462; five rounds: 110,000 of 12x12, 131 / 220 327 / 507, 394 / 552
+    //   larger, 4 actions: 150,000 of 20x20, 131 / 170 485 / 652, 557 / 654; 110,000 of 25x20, 170 / 220 480 / 643, 547 / 642
+    //   8 actions, two LDS waves: 150,000 of 16x16, 131 / 170 / 220 639 / 739 / 871, 657 / 752 / 872; 220,000, 131 / 170
+    //     865 / 1141, 991 / 1138; one, five rounds and more: 100,000 of 24x12, 64 / 96 / 131 / 220 228 / 326 / 435 / 699,
+    //     226 / 314 / 412 / 648; 150,000, 64 / 96 / 131 340 / 484 / 643, 370 / 459 / 592; 110,000 of 23x23, 96 / 131 / 300 380 /
+    //     503 / 1075, 380 / 491 / 996; four rounds: 80,000 of 19x18, 131 / 200 362 / 534, 413 / 585
+    //   four rounds of 8 actions from 20 million env-steps on: 94,000 of 19x12, 200 / 440 steps 546 / 1128, 520 / 892;
+    //     98,000 of 9x9, 256 steps 420, 404
+    // Where the lane waves have at most three rounds they are late by less, and the larger a table the sooner
+    // hybrid workgroups pay: 95,000 of 12x12, 256 / 500 steps 322 / 546, 316 / 541, of 16x16 429, 375; 73,000 of 26x18, 256 /
+    // 367 steps 465 / 657, 465 / 602; 80,000 of 20x20, 200 / 256 steps 379 / 477, 383 / 450; 8 actions, 73,000 of 12x12, 500 /
+    // 1000 steps 644 / 1189, 722 / 1354, of 16x16 960 / 1729, 898 / 1574; 70,000 of 19x12, 440 steps 782, 745.
     const bool few_rounds = rounds <= 3;
     const int few_rounds_min_steps = e->A == 8 ? (e->K >= 1536 ? 400 : INT_MAX) : e->K >= 1024 ? 256 : kHybridFewRoundsMinSteps;
     const bool hybrid_pays =
         few_rounds ? n_steps >= few_rounds_min_steps
-                   : 64L * n_steps >= 5L * (long)e->K &&
-                         (long)e->N * n_steps >= (e->K < 512   ? kHybridEnvStepsSmall
-                                                  : e->A == 4 ? kHybridEnvSteps4
-                                                  : rounds > 4 ? kHybridEnvSteps8
-                                                               : kHybridEnvSteps8FewRounds);
+        : e->A == 8 && p.lds_waves == 1 && rounds > 4
+            ? n_steps >= kHybridOneWaveMinSteps
+            : 64L * n_steps >= 5L * (long)e->K &&
+                  (long)e->N * n_steps >= (e->K < 512 || (e->K < 1536 && (e->A == 4 || rounds > 5)) ? kHybridEnvStepsSmall
+                                           : e->A == 4                                              ? kHybridEnvSteps4
+                                           : rounds > 4                                             ? kHybridEnvSteps8
+                                                                                                    : kHybridEnvSteps8FewRounds);
     // ... (automatic) when the tables outgrow the caches: while they all fit, other plans are
     // faster (16x16 maps, 30,000 envs: 3.5e10 hybrid, 5.9e10 with lane waves); and where lane
     // waves could step what is left to the general loop, they are faster too (262,144 envs of

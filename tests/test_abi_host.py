@@ -241,6 +241,21 @@ def test_lane_waves_are_as_many_as_fit_a_compute_unit(pycrl, N, W, H, A, n_steps
     assert (plan["name"], plan["grid"]) == (name, grid)
 
 
+@pytest.mark.parametrize("N,W,H,A,n_steps,hybrid", [
+    (150000, 16, 16, 4, 119, False), (150000, 16, 16, 4, 120, True),  # 18 million env-steps
+    (200000, 12, 12, 4, 89, False), (200000, 12, 12, 4, 90, True),
+    (150000, 20, 20, 4, 159, False), (150000, 20, 20, 4, 160, True),  # 24: larger tables
+    (150000, 12, 12, 8, 119, False), (150000, 12, 12, 8, 120, True),  # seven rounds of lane waves
+    (110000, 12, 12, 8, 254, False), (110000, 12, 12, 8, 255, True),  # five: 28
+    (150000, 16, 16, 8, 186, False), (150000, 16, 16, 8, 187, True),
+    (100000, 24, 12, 8, 95, False), (100000, 24, 12, 8, 96, True),    # one wave on LDS tables beside the others
+    (80000, 19, 18, 8, 249, False), (80000, 19, 18, 8, 250, True),    # ... four rounds
+])
+def test_hybrid_workgroups_or_rounds_of_lane_waves(pycrl, N, W, H, A, n_steps, hybrid):
+    name = pycrl.fused_plan_for_config(pycrl.make_config(N, W, H, n_actions=A, episode_len=128), n_steps)["name"]
+    assert name == ("k_fused_tickets<%d,fast,hbm+lds>" if hybrid else "k_fused_lanes<%d,fast>") % A
+
+
 def test_npy_agent_files_match_numpy(pycrl, tmp_path):
     """QTableAgent.save / load files (src/train.py:150-168): float64 (W, H, A)
     indexed [x, y, a], exchanged with numpy in both directions."""
