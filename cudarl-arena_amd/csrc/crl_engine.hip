@@ -399,7 +399,7 @@ constexpr int kLaneWavesMinSteps = 8;
 constexpr int kLaneRoundsMinSteps = 64, kLaneRoundsManyMinSteps = 131;
 constexpr int kLaneFewRoundsMinSteps = 48;
 constexpr long kLaneRoundsManyEnvs = 65536;
-constexpr int kLaneLateWavesMinSteps = 384;
+constexpr int kLaneLateWavesMinSteps = 384, kLaneLateWavesManyMinSteps = 192;
 constexpr int kLaneRoundsFourMinSteps = 64, kLaneRoundsFourLongSteps = 300;
 constexpr int kLaneDrawnMinSteps = 256, kLaneDrawnManyMinSteps = 128;
 constexpr int kLaneTouchMinSteps4 = 90, kLaneTouchMinSteps8 = 160, kLaneTouchFourRoundsMinSteps = 200;
@@ -719,9 +719,10 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
                                                                                      : kLaneRoundsManyMinSteps;
       // (one wave more to a compute unit than fits, which runs when another has ended: 67,000 envs of 45x19 with 8
       // actions, 131 / 400 / 800 steps, 64-env waves 380 / 1052 / 2053, lane waves 502 / 1002 / 1890, in a fourth round
-      // instead 384 / 1050 / 1977; 45,000, fewer than three 64-env waves to a unit, 227 / 594 / 1175, 327 / 718 / 1340)
+      // instead 384 / 1050 / 1977; where there are many rounds sooner, 150,000, seven, 131 / 250 / 400 steps 752 / 1411 / 2231,
+      // 760 / 1352 / 2070; 45,000, fewer than three 64-env waves to a unit, 227 / 594 / 1175, 327 / 718 / 1340)
       const bool late_waves = lane_waves > kComputeUnits * lane_fit;
-      const bool late_pay = !p.fast || (outgrown && (long)e->N > kLaneRoundsManyEnvs && n_steps >= kLaneLateWavesMinSteps);
+      const bool late_pay = !p.fast || (outgrown && (long)e->N > kLaneRoundsManyEnvs && n_steps >= (rounds > 6 ? kLaneLateWavesManyMinSteps : kLaneLateWavesMinSteps));
       const bool rounds_ok = (late_waves ? late_pay && lane_waves <= kComputeUnits * (lane_fit + 1) : true) && n_steps >= rounds_min_steps;
       if (lanes_can && (small ? lane_fit > 0 : lanes_at_once ? n_steps >= at_once_min_steps : rounds_ok)) {
         p.fast = p.moves = p.lanes = true;

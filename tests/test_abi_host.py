@@ -233,6 +233,7 @@ def test_every_valid_configuration_has_a_launch_plan_that_fits(pycrl):
     (67000, 45, 19, 8, 131, "k_fused_tickets<8,fast,hbm>", 256), (67000, 45, 19, 8, 383, "k_fused_tickets<8,fast,hbm>", 256),
     (67000, 45, 19, 8, 384, "k_fused_lanes<8,fast>", 2792),  # long calls: an eleventh that runs late
     (100000, 45, 19, 8, 131, "k_fused_lanes<8,fast>", 2500), (45000, 45, 19, 8, 800, "k_fused_tickets<8,fast,hbm>", 704),
+    (150000, 45, 19, 8, 191, "k_fused_tickets<8,fast,hbm>", 256), (150000, 45, 19, 8, 192, "k_fused_lanes<8,fast>", 2679),
     # 8272 bytes: seven pieces, eighteen to a unit
     (73728, 21, 21, 4, 131, "k_fused_lanes<4,fast>", 4608), (73729, 21, 21, 4, 131, "k_fused_lanes<4,fast>", 1537),
 ])
