@@ -387,8 +387,9 @@ constexpr size_t kStaticLdsReserve = 1024;
 constexpr size_t kLdsPiece = 1280;
 constexpr long lds_fit(size_t bytes) { return (long)(kLdsPerWorkgroup / ((bytes + kLdsPiece - 1) / kLdsPiece * kLdsPiece)); }
 
-// Launches shorter than this do not repay moving whole tables into LDS and back
-// (1M envs of config 4, steps per launch -> env-steps/s, plain / hybrid:
+// Where lane waves are no choice (rules they leave out, a caller that sets the envs in flight), launches shorter
+// than this do not repay moving whole tables into LDS and back (beside lane waves: hybrid_pays in plan_fused).
+// (1M envs of 16x16, steps per launch -> env-steps/s, 64-env waves / hybrid:
 // 32: 2.4e10 / 2.1e10, 48: 2.8e10 / 2.75e10, 64: 3.0e10 / 3.3e10, 100: 3.6e10 / 4.2e10).
 constexpr int kHybridMinSteps = 64;
 constexpr int kStagedMovesMinSteps = 128;

@@ -53,7 +53,6 @@ struct Rec {
   }
   static __device__ __forceinline__ int slot(uint32_t meta) { return (int)(meta & ((1u << kCountShift) - 1u)); }
   static __device__ __forceinline__ int count(uint32_t meta) { return (int)((meta >> kCountShift) & 127u); }
-  static __device__ __forceinline__ uint32_t tag(uint32_t meta) { return meta >> kTagShift; }
 };
 static_assert(kOwnKeys == 1 << Rec<false>::kCountShift && kOwnKeysHashed == 1 << Rec<true>::kCountShift, "a record's slot");
 // Two launches: slot in bits 0..15, count in bits 16..22, no tag.

@@ -133,14 +133,15 @@ int crl_set_resident_envs(crl_engine* e, int32_t n_envs);
 /* Tuning (no reference counterpart): kernel of crl_run_fused.  0 = automatic.
  * Per-env tables: 1 = plain (every wave steps envs against tables in HBM),
  * 2 = hybrid (the last waves of each workgroup step envs whose whole tables they hold
- * in LDS; used only where the tables of 64 / actions envs fit, with the general loop 32;
- * automatic picks it for launches of at least 64 steps on tables that outgrow the
- * caches).  Shared table: 1 = two launches per step; 2 = all steps of a
+ * in LDS; used only where the tables of 64 / actions envs fit, with the general loop 32);
+ * automatic chooses by the sizes, the rules and the length of the call, and
+ * crl_fused_kernel_info tells what it chose.  Shared table: 1 = two launches per step; 2 = all steps of a
  * call in one launch whose 256 workgroups exchange block sums and table values
  * through device-scope loads and stores (needs every workgroup resident at once:
  * at most 65,536 envs and 131,072 table entries, else two launches per step);
  * automatic picks the one launch for calls of at least 16 steps, down to 9 with more
- * than 49,152 envs; with more than 16,384 entries for 10 steps, 6 with 8 actions.
+ * than 49,152 envs; with more than 16,384 entries for 10 steps, 6 with 8 actions, but
+ * not for up to 8192 envs on a table of up to 24,576 entries.
  * Results do not depend on it. */
 int crl_set_fused_variant(crl_engine* e, int32_t variant);
 /* How the last hybrid crl_run_fused split the envs between its two kinds of
