@@ -352,7 +352,12 @@ constexpr long kMinEnvsInFlight = kComputeUnits * 3L * 64;  // three waves per c
 // The general loop on a shared map, 4 actions, loses by two shifts (20x20, 80,000 envs, statistics and epsilon by
 // episode, 6 / 14 steps 21.0 / 42.7, 24.4 / 47.1; three shifts of 16x16, 14 steps 80.9, 69.5; with 8 actions, two of
 // 20x20, 55.1, 51.0; two of 60x60, 9 steps 29.7, 28.5).
-constexpr int kInFlightMinSteps = 6, kInFlightMinStepsTwoShifts = 16;
+// Maps of their own and of some 1000 cells, whose tables' lines a few steps meet once, lose longer by three shifts
+// and more, or two with 8 actions (105,108 envs of 43x23, 6 / 9 / 11 steps 43.1 / 56.0 / 66.9, 47.5 / 57.4 / 64.0; 200,000
+// 66.0 / 87.9 / 105.0, 78.2 / 96.0 / 107.8; 105,000 of 32x32, epsilon by episode, 6 / 8 38.9 / 46.8, 44.6 / 51.2; 57,155 of 26x37
+// with 8 actions, statistics, 6 / 7 34.5 / 38.3, 38.9 / 42.3).
+constexpr int kInFlightMinSteps = 6, kInFlightMinStepsTwoShifts = 16, kInFlightMinStepsLargeMaps = 10;
+constexpr size_t kInFlightLargeMap = 900;
 
 // launch geometry of the fused per-env kernel
 struct FusedPlan {
@@ -519,7 +524,9 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     const long fits = std::max<long>(kMinEnvsInFlight, (long)(kTableBytesInFlight / table_bytes));
     const bool general = !foldable || c.eps_mode == CRL_EPS_STEP_MULT;
     const bool two_shifts = p.map_kind == 1 && general && e->A == 4 && e->K < 4096 && e->N <= 2 * fits;
-    if ((size_t)e->N * table_bytes > kTableBytesInFlight && n_steps >= (two_shifts ? kInFlightMinStepsTwoShifts : kInFlightMinSteps))
+    const bool large_maps = p.map_kind == 0 && e->S >= kInFlightLargeMap && (e->A == 8 || e->N > 2 * fits);
+    const int min_steps = two_shifts ? kInFlightMinStepsTwoShifts : large_maps ? kInFlightMinStepsLargeMaps : kInFlightMinSteps;
+    if ((size_t)e->N * table_bytes > kTableBytesInFlight && n_steps >= min_steps)
       resident = fits;
     // The batch goes through the chip in shifts of that many envs; a last shift that
     // fills a fraction of the chip costs a whole one.  Even the shifts out, in whole

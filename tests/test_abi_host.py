@@ -257,6 +257,17 @@ def test_hybrid_workgroups_or_rounds_of_lane_waves(pycrl, N, W, H, A, n_steps, h
     assert name == ("k_fused_tickets<%d,fast,hbm+lds>" if hybrid else "k_fused_lanes<%d,fast>") % A
 
 
+@pytest.mark.parametrize("N,W,H,A,n_steps,grid", [
+    (105108, 43, 23, 4, 9, 410), (105108, 43, 23, 4, 10, 256),  # three shifts of maps of 900 cells and more
+    (60000, 32, 32, 4, 5, 937), (60000, 32, 32, 4, 6, 512),     # two
+    (57155, 26, 37, 8, 9, 893), (57155, 26, 37, 8, 10, 512),    # two, 8 actions
+    (150000, 20, 20, 4, 5, 585), (150000, 20, 20, 4, 6, 256),   # smaller maps
+])
+def test_envs_in_flight_of_short_launches(pycrl, N, W, H, A, n_steps, grid):
+    plan = pycrl.fused_plan_for_config(pycrl.make_config(N, W, H, n_actions=A, episode_len=128), n_steps)
+    assert (plan["name"], plan["grid"]) == ("k_fused_tickets<%d,fast,hbm>" % A, grid)
+
+
 def test_npy_agent_files_match_numpy(pycrl, tmp_path):
     """QTableAgent.save / load files (src/train.py:150-168): float64 (W, H, A)
     indexed [x, y, a], exchanged with numpy in both directions."""
