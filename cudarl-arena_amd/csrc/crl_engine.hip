@@ -405,7 +405,7 @@ constexpr int kLaneWavesMinSteps = 8;
 constexpr int kLaneRoundsMinSteps = 64, kLaneRoundsManyMinSteps = 131;
 constexpr int kLaneFewRoundsMinSteps = 48;
 constexpr long kLaneRoundsManyEnvs = 65536;
-constexpr int kLaneLateWavesMinSteps = 384, kLaneLateWavesManyMinSteps = 192;
+constexpr int kLaneUnevenMinSteps = 384, kLaneUnevenManyRoundsMinSteps = 192;
 constexpr int kLaneRoundsFourMinSteps = 64, kLaneRoundsFourLongSteps = 300;
 constexpr int kLaneDrawnMinSteps = 256, kLaneDrawnManyMinSteps = 128;
 constexpr int kLaneTouchMinSteps4 = 90, kLaneTouchMinSteps8 = 160, kLaneTouchFourRoundsMinSteps = 200;
@@ -725,19 +725,25 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
                                    : e->A == 4 && (long)e->N <= kMinEnvsInFlight     ? INT_MAX
                                    : (long)e->N <= kLaneRoundsManyEnvs               ? kLaneRoundsMinSteps
                                                                                      : kLaneRoundsManyMinSteps;
-      // (one wave more to a compute unit than fits, which runs when another has ended: 67,000 envs of 45x19 with 8
-      // actions, 131 / 400 / 800 steps, 64-env waves 380 / 1052 / 2053, lane waves 502 / 1002 / 1890, in a fourth round
-      // instead 384 / 1050 / 1977; where there are many rounds sooner, 150,000, seven, 131 / 250 / 400 steps 752 / 1411 / 2231,
-      // 760 / 1352 / 2070; 45,000, fewer than three 64-env waves to a unit, 227 / 594 / 1175, 327 / 718 / 1340)
-      const bool late_waves = lane_waves > kComputeUnits * lane_fit;
-      const bool late_pay = !p.fast || (outgrown && (long)e->N > kLaneRoundsManyEnvs && n_steps >= (rounds > 6 ? kLaneLateWavesManyMinSteps : kLaneLateWavesMinSteps));
-      const bool rounds_ok = (late_waves ? late_pay && lane_waves <= kComputeUnits * (lane_fit + 1) : true) && n_steps >= rounds_min_steps;
+      // Even rounds of one wave more to a compute unit than fits: as many as fit draw their envs instead (dealt by
+      // position, the late ones run after all others; 67,000 envs of 45x19 with 8 actions, floored maximum, 64 / 131 / 200
+      // / 425 steps late and dealt 264 / 495 / 721 / 1038, as many as fit 220 / 366 / 514 / 994; 100,000 of 40x40, 131 steps 652,
+      // 441; 39,537 of 47x42, 425 steps 881, 659).  In place of the folded loop in long launches only: 67,000 of 45x19, 131
+      // steps 64-env / lane waves 374 / 366, 100,000 of 36x26 566 / 548, but 80,000 of 45x21 404 / 453 and at 200 601 / 641;
+      // 45,000 of 45x19, fewer than three 64-env waves to a unit, 131 / 400 / 800 steps 227 / 594 / 1175, 261 / 720 / 1270;
+      // 150,000, seven rounds, 131 / 200 / 425 752 / 1111 / 2231, 742 / 1065 / 2121.
+      const bool uneven = !small && !lanes_at_once && lane_waves > kComputeUnits * lane_fit;
+      const bool uneven_pay = !p.fast || (outgrown && (long)e->N > kLaneRoundsManyEnvs &&
+                                          n_steps >= (rounds > 6 ? kLaneUnevenManyRoundsMinSteps : kLaneUnevenMinSteps));
+      const bool rounds_ok = (!uneven || (uneven_pay && lane_waves <= kComputeUnits * (lane_fit + 1))) && n_steps >= rounds_min_steps;
       if (lanes_can && (small ? lane_fit > 0 : lanes_at_once ? n_steps >= at_once_min_steps : rounds_ok)) {
         p.fast = p.moves = p.lanes = true;
         p.rich = c.eps_mode >= CRL_EPS_EPISODE_MULT || c.reward_flags != 0;
         p.log_envs = lane_log_envs;
         p.tape_steps = tape_steps_for(lane_log_envs);
-        const long most = e->resident_envs > 0 ? std::max<long>(1, resident >> lane_log_envs) : lane_waves;
+        const long most = e->resident_envs > 0 ? std::max<long>(1, resident >> lane_log_envs)
+                          : uneven               ? kComputeUnits * lane_fit
+                                                 : lane_waves;
         p.grid = (int)std::min<long>(lane_units, most);
         p.block = 64;
         const bool many_rounds = p.grid * 5L < lane_units;
@@ -762,7 +768,8 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       // dealt: 120,000 envs of 8x8, two rounds, 128 / 1000 steps 207 / 1315, 176 / 1268 us; 140,000 of 6x6
       // with 8 actions, five rounds, 128 / 300 / 1000 steps 290 / 563 / 1654, 279 / 609 / 1912; 300,000
       // of 16x16, ten rounds, 128 / 300 steps 868 / 1523, 879 / 1585; 891,000 of 20x14, 150 steps 2503, 2705.
-      const bool drawn_lanes = n_steps >= kLaneDrawnMinSteps ? e->A == 8 || p.grid * 3L < lane_units
+      const bool drawn_lanes = uneven && n_steps >= kHybridMinSteps ? true
+                               : n_steps >= kLaneDrawnMinSteps ? e->A == 8 || p.grid * 3L < lane_units
                                                              : n_steps >= kLaneDrawnManyMinSteps && p.grid * 5L < lane_units;
       p.fixed = p.lanes ? p.grid >= lane_units || !drawn_lanes : n_steps < kHybridMinSteps;
       if (!p.lanes) p.lds = waves * (p.moves ? mv_lds : map_lds);
