@@ -355,7 +355,8 @@ constexpr long kMinEnvsInFlight = kComputeUnits * 3L * 64;  // three waves per c
 // Maps of their own and of some 1000 cells, whose tables' lines a few steps meet once, lose longer by three shifts
 // and more, or two with 8 actions (105,108 envs of 43x23, 6 / 9 / 11 steps 43.1 / 56.0 / 66.9, 47.5 / 57.4 / 64.0; 200,000
 // 66.0 / 87.9 / 105.0, 78.2 / 96.0 / 107.8; 105,000 of 32x32, epsilon by episode, 6 / 8 38.9 / 46.8, 44.6 / 51.2; 57,155 of 26x37
-// with 8 actions, statistics, 6 / 7 34.5 / 38.3, 38.9 / 42.3).
+// with 8 actions, statistics, 6 / 7 34.5 / 38.3, 38.9 / 42.3; past 65,536 of these workgroups of four waves are one to a
+// unit and some late: 67,524 of 24x44, 6 steps 46.2, 35.5).
 constexpr int kInFlightMinSteps = 6, kInFlightMinStepsTwoShifts = 16, kInFlightMinStepsLargeMaps = 10;
 constexpr size_t kInFlightLargeMap = 900;
 
@@ -524,7 +525,7 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     const long fits = std::max<long>(kMinEnvsInFlight, (long)(kTableBytesInFlight / table_bytes));
     const bool general = !foldable || c.eps_mode == CRL_EPS_STEP_MULT;
     const bool two_shifts = p.map_kind == 1 && general && e->A == 4 && e->K < 4096 && e->N <= 2 * fits;
-    const bool large_maps = p.map_kind == 0 && e->S >= kInFlightLargeMap && (e->A == 8 || e->N > 2 * fits);
+    const bool large_maps = p.map_kind == 0 && e->S >= kInFlightLargeMap && (e->A == 8 ? e->N <= 4 * 64 * kComputeUnits : e->N > 2 * fits);
     const int min_steps = two_shifts ? kInFlightMinStepsTwoShifts : large_maps ? kInFlightMinStepsLargeMaps : kInFlightMinSteps;
     if ((size_t)e->N * table_bytes > kTableBytesInFlight && n_steps >= min_steps)
       resident = fits;
@@ -728,12 +729,13 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       // Even rounds of one wave more to a compute unit than fits: as many as fit draw their envs instead (dealt by
       // position, the late ones run after all others; 67,000 envs of 45x19 with 8 actions, floored maximum, 64 / 131 / 200
       // / 425 steps late and dealt 264 / 495 / 721 / 1038, as many as fit 220 / 366 / 514 / 994; 100,000 of 40x40, 131 steps 652,
-      // 441; 39,537 of 47x42, 425 steps 881, 659).  In place of the folded loop in long launches only: 67,000 of 45x19, 131
+      // 441).  With up to three 64-env waves to a unit those are faster, also by the general loop (39,537 of 47x42, floored
+      // maximum, 64 / 438 steps 101 / 492, 141 / 676; 45,000 of 45x19 with 8 actions 127 / 693, 162 / 743).  In place of the folded loop in long launches only: 67,000 of 45x19, 131
       // steps 64-env / lane waves 374 / 366, 100,000 of 36x26 566 / 548, but 80,000 of 45x21 404 / 453 and at 200 601 / 641;
       // 45,000 of 45x19, fewer than three 64-env waves to a unit, 131 / 400 / 800 steps 227 / 594 / 1175, 261 / 720 / 1270;
       // 150,000, seven rounds, 131 / 200 / 425 752 / 1111 / 2231, 742 / 1065 / 2121.
       const bool uneven = !small && !lanes_at_once && lane_waves > kComputeUnits * lane_fit;
-      const bool uneven_pay = !p.fast || (outgrown && (long)e->N > kLaneRoundsManyEnvs &&
+      const bool uneven_pay = !p.fast ? (long)e->N > kMinEnvsInFlight : (outgrown && (long)e->N > kLaneRoundsManyEnvs &&
                                           n_steps >= (rounds > 6 ? kLaneUnevenManyRoundsMinSteps : kLaneUnevenMinSteps));
       const bool rounds_ok = (!uneven || (uneven_pay && lane_waves <= kComputeUnits * (lane_fit + 1))) && n_steps >= rounds_min_steps;
       if (lanes_can && (small ? lane_fit > 0 : lanes_at_once ? n_steps >= at_once_min_steps : rounds_ok)) {

@@ -234,6 +234,7 @@ def test_every_valid_configuration_has_a_launch_plan_that_fits(pycrl):
     (67000, 45, 19, 8, 384, "k_fused_lanes<8,fast>", 2560),  # long calls: three uneven rounds
     (100000, 45, 19, 8, 131, "k_fused_lanes<8,fast>", 2500), (45000, 45, 19, 8, 800, "k_fused_tickets<8,fast,hbm>", 704),
     (150000, 45, 19, 8, 191, "k_fused_tickets<8,fast,hbm>", 256), (150000, 45, 19, 8, 192, "k_fused_lanes<8,fast>", 2560),
+    (67524, 24, 44, 8, 6, "k_fused_tickets<8,fast,hbm>", 256),
     # 8272 bytes: seven pieces, eighteen to a unit
     (73728, 21, 21, 4, 131, "k_fused_lanes<4,fast>", 4608), (73729, 21, 21, 4, 131, "k_fused_lanes<4,fast>", 1537),
 ])
@@ -255,6 +256,16 @@ def test_lane_waves_are_as_many_as_fit_a_compute_unit(pycrl, N, W, H, A, n_steps
 def test_hybrid_workgroups_or_rounds_of_lane_waves(pycrl, N, W, H, A, n_steps, hybrid):
     name = pycrl.fused_plan_for_config(pycrl.make_config(N, W, H, n_actions=A, episode_len=128), n_steps)["name"]
     assert name == ("k_fused_tickets<%d,fast,hbm+lds>" if hybrid else "k_fused_lanes<%d,fast>") % A
+
+
+@pytest.mark.parametrize("N,W,H,A,name", [
+    (39537, 47, 42, 4, "k_fused_tickets<4,general,hbm>"), (45000, 45, 19, 8, "k_fused_tickets<8,general,hbm>"),
+    (50001, 40, 40, 4, "k_fused_lanes<4,fast>"),
+])
+def test_uneven_rounds_of_a_floored_maximum(pycrl, N, W, H, A, name):
+    cfg = pycrl.make_config(N, W, H, n_actions=A, episode_len=128, max_mode=pycrl.MAX_ZERO_FLOOR)
+    for n_steps in (16, 64, 438):
+        assert pycrl.fused_plan_for_config(cfg, n_steps)["name"] == name
 
 
 @pytest.mark.parametrize("N,W,H,A,n_steps,grid", [
