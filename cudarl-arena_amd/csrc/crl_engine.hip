@@ -716,6 +716,9 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       //   others, 32 / 64 / 96 steps: 52,000 of 32x32 61 / 114 / 160, 57 / 98 / 139; 40,000 of 24x24 with
       //     8 actions 49 / 100 / 142, 57 / 97 / 136; 100,000 of 32x32 123 / 229 / 333, 119 / 206 / 291 (the
       //     larger batches keep their 64-env waves up to 130 steps, a length that their tests hold them to)
+      //   8 actions, not more than two waves of 64 envs to a compute unit: 64-env waves always, 25,161 of 28x46, 64 / 164 / 800
+      //     steps 78 / 168 / 739, 96 / 211 / 922; 30,000 of 24x24 78 / 173 / 711, 87 / 191 / 856; 32,000 of 28x28 85 / 180 / 804, 94 /
+      //     214 / 933; epsilon by episode, 400 steps 480 / 482 / 504, 501 / 473 / 512
       //   4 actions, not more than three waves of 64 envs to a compute unit: 64-env waves always, 34,000 of
       //     32x32, 128 / 1000 steps 120 / 727, 146 / 908; 49,000 176 / 1235, 174 / 1240
       const bool small = waves == 1 && tickets <= 2 * kComputeUnits;
@@ -724,6 +727,7 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       const int rounds_min_steps = !(p.fast && outgrown)                             ? kLaneWavesMinSteps
                                    : fits && e->fused_variant == 0                   ? (few_rounds ? kLaneFewRoundsMinSteps : (int)std::min<size_t>(40, std::max<size_t>(kLaneWavesMinSteps, e->K / 24)))
                                    : e->A == 4 && (long)e->N <= kMinEnvsInFlight     ? INT_MAX
+                                   : e->A == 8 && (long)e->N <= 2L * 64 * kComputeUnits ? INT_MAX
                                    : (long)e->N <= kLaneRoundsManyEnvs               ? kLaneRoundsMinSteps
                                                                                      : kLaneRoundsManyMinSteps;
       // Even rounds of one wave more to a compute unit than fits: as many as fit draw their envs instead (dealt by

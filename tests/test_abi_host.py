@@ -235,6 +235,7 @@ def test_every_valid_configuration_has_a_launch_plan_that_fits(pycrl):
     (100000, 45, 19, 8, 131, "k_fused_lanes<8,fast>", 2500), (45000, 45, 19, 8, 800, "k_fused_tickets<8,fast,hbm>", 704),
     (150000, 45, 19, 8, 191, "k_fused_tickets<8,fast,hbm>", 256), (150000, 45, 19, 8, 192, "k_fused_lanes<8,fast>", 2560),
     (67524, 24, 44, 8, 6, "k_fused_tickets<8,fast,hbm>", 256),
+    (25161, 28, 46, 8, 164, "k_fused_tickets<8,fast,hbm>", 394), (32769, 24, 24, 8, 164, "k_fused_lanes<8,fast>", 2049),
     # 8272 bytes: seven pieces, eighteen to a unit
     (73728, 21, 21, 4, 131, "k_fused_lanes<4,fast>", 4608), (73729, 21, 21, 4, 131, "k_fused_lanes<4,fast>", 1537),
 ])
