@@ -525,7 +525,8 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     const long fits = std::max<long>(kMinEnvsInFlight, (long)(kTableBytesInFlight / table_bytes));
     const bool general = !foldable || c.eps_mode == CRL_EPS_STEP_MULT;
     const bool two_shifts = p.map_kind == 1 && general && e->A == 4 && e->K < 4096 && e->N <= 2 * fits;
-    const bool large_maps = p.map_kind == 0 && e->S >= kInFlightLargeMap && (e->A == 8 ? e->N <= 4 * 64 * kComputeUnits : e->N > 2 * fits);
+    const bool large_maps = p.map_kind == 0 && e->S >= kInFlightLargeMap && e->N > (e->A == 8 ? fits : 2 * fits) &&
+                            (e->A == 4 || e->N <= 4 * 64 * kComputeUnits);
     const int min_steps = two_shifts ? kInFlightMinStepsTwoShifts : large_maps ? kInFlightMinStepsLargeMaps : kInFlightMinSteps;
     if ((size_t)e->N * table_bytes > kTableBytesInFlight && n_steps >= min_steps)
       resident = fits;
@@ -734,12 +735,13 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       // position, the late ones run after all others; 67,000 envs of 45x19 with 8 actions, floored maximum, 64 / 131 / 200
       // / 425 steps late and dealt 264 / 495 / 721 / 1038, as many as fit 220 / 366 / 514 / 994; 100,000 of 40x40, 131 steps 652,
       // 441).  With up to three 64-env waves to a unit those are faster, also by the general loop (39,537 of 47x42, floored
-      // maximum, 64 / 438 steps 101 / 492, 141 / 676; 45,000 of 45x19 with 8 actions 127 / 693, 162 / 743).  In place of the folded loop in long launches only: 67,000 of 45x19, 131
+      // maximum, 64 / 438 steps 101 / 492, 141 / 676; 45,000 of 45x19 with 8 actions 127 / 693, 162 / 743), and so they are in
+      // short launches (67,045 of 40x47, 9 steps 57, 66).  In place of the folded loop in long launches only: 67,000 of 45x19, 131
       // steps 64-env / lane waves 374 / 366, 100,000 of 36x26 566 / 548, but 80,000 of 45x21 404 / 453 and at 200 601 / 641;
       // 45,000 of 45x19, fewer than three 64-env waves to a unit, 131 / 400 / 800 steps 227 / 594 / 1175, 261 / 720 / 1270;
       // 150,000, seven rounds, 131 / 200 / 425 752 / 1111 / 2231, 742 / 1065 / 2121.
       const bool uneven = !small && !lanes_at_once && lane_waves > kComputeUnits * lane_fit;
-      const bool uneven_pay = !p.fast ? (long)e->N > kMinEnvsInFlight : (outgrown && (long)e->N > kLaneRoundsManyEnvs &&
+      const bool uneven_pay = !p.fast ? (long)e->N > kMinEnvsInFlight && n_steps >= kHybridMinSteps : (outgrown && (long)e->N > kLaneRoundsManyEnvs &&
                                           n_steps >= (rounds > 6 ? kLaneUnevenManyRoundsMinSteps : kLaneUnevenMinSteps));
       const bool rounds_ok = (!uneven || (uneven_pay && lane_waves <= kComputeUnits * (lane_fit + 1))) && n_steps >= rounds_min_steps;
       if (lanes_can && (small ? lane_fit > 0 : lanes_at_once ? n_steps >= at_once_min_steps : rounds_ok)) {
@@ -774,7 +776,7 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       // dealt: 120,000 envs of 8x8, two rounds, 128 / 1000 steps 207 / 1315, 176 / 1268 us; 140,000 of 6x6
       // with 8 actions, five rounds, 128 / 300 / 1000 steps 290 / 563 / 1654, 279 / 609 / 1912; 300,000
       // of 16x16, ten rounds, 128 / 300 steps 868 / 1523, 879 / 1585; 891,000 of 20x14, 150 steps 2503, 2705.
-      const bool drawn_lanes = uneven && n_steps >= kHybridMinSteps ? true
+      const bool drawn_lanes = uneven ? true
                                : n_steps >= kLaneDrawnMinSteps ? e->A == 8 || p.grid * 3L < lane_units
                                                              : n_steps >= kLaneDrawnManyMinSteps && p.grid * 5L < lane_units;
       p.fixed = p.lanes ? p.grid >= lane_units || !drawn_lanes : n_steps < kHybridMinSteps;

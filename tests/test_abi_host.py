@@ -235,6 +235,7 @@ def test_every_valid_configuration_has_a_launch_plan_that_fits(pycrl):
     (100000, 45, 19, 8, 131, "k_fused_lanes<8,fast>", 2500), (45000, 45, 19, 8, 800, "k_fused_tickets<8,fast,hbm>", 704),
     (150000, 45, 19, 8, 191, "k_fused_tickets<8,fast,hbm>", 256), (150000, 45, 19, 8, 192, "k_fused_lanes<8,fast>", 2560),
     (67524, 24, 44, 8, 6, "k_fused_tickets<8,fast,hbm>", 256),
+    (16810, 39, 47, 8, 7, "k_fused_tickets<8,fast,hbm>", 263),  # no envs over to begin late
     (25161, 28, 46, 8, 164, "k_fused_tickets<8,fast,hbm>", 394), (32769, 24, 24, 8, 164, "k_fused_lanes<8,fast>", 2049),
     # 8272 bytes: seven pieces, eighteen to a unit
     (73728, 21, 21, 4, 131, "k_fused_lanes<4,fast>", 4608), (73729, 21, 21, 4, 131, "k_fused_lanes<4,fast>", 1537),
@@ -265,8 +266,9 @@ def test_hybrid_workgroups_or_rounds_of_lane_waves(pycrl, N, W, H, A, n_steps, h
 ])
 def test_uneven_rounds_of_a_floored_maximum(pycrl, N, W, H, A, name):
     cfg = pycrl.make_config(N, W, H, n_actions=A, episode_len=128, max_mode=pycrl.MAX_ZERO_FLOOR)
-    for n_steps in (16, 64, 438):
+    for n_steps in (64, 438):
         assert pycrl.fused_plan_for_config(cfg, n_steps)["name"] == name
+    assert pycrl.fused_plan_for_config(cfg, 63)["name"] == "k_fused_tickets<%d,general,hbm>" % A
 
 
 @pytest.mark.parametrize("N,W,H,A,n_steps,grid", [
