@@ -374,6 +374,7 @@ struct FusedPlan {
   bool lanes;      // an env to A lanes, a wave to 2^log_envs envs, draws taped tape_steps ahead
   int log_envs, tape_steps;
   bool touch;      // ... whose tables are read ahead whole
+  bool rows;       // 64-env waves that keep their envs' rows in LDS (moves: and not their maps)
   bool rich;       // ticket kernel: the folded loop's variant with per-cell rewards / per-episode epsilon
   int tab_stride;  // floats between two tables in LDS
   bool in_lds;     // ... with all tables in LDS
@@ -414,6 +415,13 @@ constexpr int kLaneTouchMinSteps4 = 90, kLaneTouchMinSteps8 = 160, kLaneTouchFou
 constexpr int kHybridFewRoundsMinSteps = 384, kHybridOneWaveMinSteps = 96;
 constexpr long kHybridEnvStepsSmall = 18000000, kHybridEnvSteps4 = 24000000, kHybridEnvSteps8 = 28000000, kHybridEnvSteps8FewRounds = 20000000;
 constexpr size_t kTableBytesAtOnce = (size_t)512 << 20;
+// 64-env waves that keep rows in LDS.  With the maps in LDS too where eight of them and more fit a compute unit, else the move codes
+// come from HBM with the rows (20 steps, staged / not: 1M of 16x16 369 / 452 us, 100,000 of 22x22 with 8 actions 62 / 69, of
+// 32x32, six staged to a unit, 73 / 55).
+constexpr int kRowsManyEnvs = 1 << 18, kRowsHybridSteps4 = 48, kRowsHybridSteps8 = 64, kRowsFewEnvsSteps = 80;
+constexpr size_t kRowsSmallMap = 336;  // cells: eleven to a unit
+constexpr int kRowsLargeMapMinSteps = 11, kRowsLargeMapMaxSteps = 130;
+constexpr long kRowsStagedWaves = 8;
 
 // Configurations that run_lanes() steps: no goal test on the resulting cell, no sticky done,
 // no trace and no supplied stream.
@@ -667,11 +675,36 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
                                            : e->A == 4                                              ? kHybridEnvSteps4
                                            : rounds > 4                                             ? kHybridEnvSteps8
                                                                                                     : kHybridEnvSteps8FewRounds);
-    // ... (automatic) when the tables outgrow the caches: while they all fit, other plans are
+    // 64-env waves that keep rows in LDS (run_env_rows), in place of all others (us, the other plan / these; launch after launch):
+    //   64-env waves: 1M envs of 16x16, 3 / 6 / 10 / 20 / 32 steps 166 / 272 / 378 / 627 / 910, 108 / 178 / 245 / 369 / 500;
+    //     262,144 of 32x32, 8 / 80 steps 93 / 628, 58 / 405; of 22x22 with 8 actions, 8 steps 105, 69; of 48x40 3 / 200 steps
+    //     86 / 1477, 44 / 1011; 1M of 5x5, 1 / 8 steps 64 / 268, 63 / 133; 20,000 of 16x16, 1 / 4 steps 12.7 / 10.3, 7.9 / 9.8
+    //   rounds of lane waves, however long: 1M of 16x16, 64 steps 1571, 890; 300,000 of 16x16, floored maximum, 200 steps 1068, 856;
+    //     of 27x27, 300 steps 2119, 1583; 262,144 of 32x32, 250 / 800 steps 1541 / 4450, 1185 / 3777; of 16x16 with 8 actions,
+    //     150 steps 1183, 859; 300,000 of 4x4 with 8 actions, 8 / 60 steps 68 / 298, 40 / 172
+    //   hybrid workgroups, up to a length that grows with the table:
+    //     1M of 8x8, 40 / 80 / 150 steps 697 / 939 / 1422, 478 / 925 / 1877; 400,000 of 12x12, 60 / 110 / 150 470 / 658 / 785,
+    //     329 / 577 / 793; 1M of 16x16, 80 / 150 / 220 1892 / 2533 / 3217, 1101 / 2099 / 3160; 600,000 of 20x20, 200 / 450
+    //     2669 / 4689, 1703 / 4014; 8 actions: 600,000 of 8x8, 60 / 100 / 140 816 / 1095 / 1367, 616 / 1011 / 1444; 500,000
+    //     of 12x12, 150 / 250 1572 / 2202, 1535 / 2696; of 16x16, 220 / 300 2779 / 3276, 2265 / 3175; 262,144 of 22x22, 600 4262, 3805
+    // With fewer envs a step is as long as its slowest request and lane waves have fewer of those (50,000 of 16x16, 20 steps
+    // 26.6, 33.3).  What is left to the others between that and these lines are lengths and sizes that tests hold them to.
+    const bool rows_can = lanes_rules(e) && c.max_episodes == 0 && c.track_returns == 0 && c.eps_mode != CRL_EPS_STEP_MULT &&
+                          e->mv_words > 0 && e->resident_envs == 0 && e->fused_variant != 2;
+    const int rows_steps = !(fits && p.fast) ? INT_MAX
+                           : e->A == 8       ? kRowsHybridSteps8 + (int)(e->K / 16)
+                                             : kRowsHybridSteps4 + (int)(e->K / 7);
+    const bool rows_small = e->S <= kRowsSmallMap;
+    const bool rows_first =
+        rows_can && e->fused_variant == 0 &&
+        ((e->N >= kRowsManyEnvs && n_steps <= rows_steps) ||
+         (foldable && (long)e->N > kLaneRoundsManyEnvs && e->K >= 1024 && !lanes_at_once && n_steps <= kRowsFewEnvsSteps &&
+          (rows_small || n_steps >= kRowsLargeMapMinSteps)));
+    // ... hybrid workgroups (automatic) when the tables outgrow the caches: while they all fit, other plans are
     // faster (16x16 maps, 30,000 envs: 3.5e10 hybrid, 5.9e10 with lane waves); and where lane
     // waves could step what is left to the general loop, they are faster too (262,144 envs of
     // 16x16 with a zero-floored maximum: 5.1e10 general hybrid, 6.4e10)
-    p.hybrid = fits && (e->fused_variant == 2 ||
+    p.hybrid = fits && !rows_first && (e->fused_variant == 2 ||
                         (e->fused_variant == 0 && outgrown &&
                          (lanes_can && e->resident_envs == 0 ? p.fast && !lanes_at_once && hybrid_pays
                                                              : (!lanes_can || p.fast) && n_steps >= kHybridMinSteps)));
@@ -744,7 +777,7 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       const bool uneven_pay = !p.fast ? (long)e->N > kMinEnvsInFlight && n_steps >= kHybridMinSteps : (outgrown && (long)e->N > kLaneRoundsManyEnvs &&
                                           n_steps >= (rounds > 6 ? kLaneUnevenManyRoundsMinSteps : kLaneUnevenMinSteps));
       const bool rounds_ok = (!uneven || (uneven_pay && lane_waves <= kComputeUnits * (lane_fit + 1))) && n_steps >= rounds_min_steps;
-      if (lanes_can && (small ? lane_fit > 0 : lanes_at_once ? n_steps >= at_once_min_steps : rounds_ok)) {
+      if (lanes_can && !rows_first && (small ? lane_fit > 0 : lanes_at_once ? n_steps >= at_once_min_steps : rounds_ok)) {
         p.fast = p.moves = p.lanes = true;
         p.rich = c.eps_mode >= CRL_EPS_EPISODE_MULT || c.reward_flags != 0;
         p.log_envs = lane_log_envs;
@@ -781,6 +814,18 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
                                                              : n_steps >= kLaneDrawnManyMinSteps && p.grid * 5L < lane_units;
       p.fixed = p.lanes ? p.grid >= lane_units || !drawn_lanes : n_steps < kHybridMinSteps;
       if (!p.lanes) p.lds = waves * (p.moves ? mv_lds : map_lds);
+      // No more of these than rows_first, or where they are the choice that is left: waves that keep rows instead (as many
+      // as there are envs for, a workgroup each).
+      if (rows_first || (!p.lanes && rows_can && foldable &&
+                         (rows_small || (n_steps >= kRowsLargeMapMinSteps && n_steps <= kRowsLargeMapMaxSteps)))) {
+        p.rows = p.fast = p.fixed = true;
+        p.rich = c.eps_mode != CRL_EPS_FIXED || c.reward_flags != 0;
+        p.lds = map_lds + crl::RowCache<4, false>::kBytes;
+        p.moves = lds_fit(p.lds) < kRowsStagedWaves;
+        if (p.moves) p.lds = crl::RowCache<4, true>::kBytes;
+        p.block = 64;
+        p.grid = (int)(((long)e->N + 63) / 64);
+      }
     }
   }
   // (as launch_fused_a() picks the kernel)
@@ -841,8 +886,10 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
     const dim3 g(p.grid), b(p.block);
     unsigned* tk = p.fixed ? e->split.p : e->tk;
 #define CRL_LAUNCH_TICKETS(MODE, LDSW, MOVES)                                                       \
-  hipLaunchKernelGGL((crl::k_fused_tickets<A, MODE, LDSW, MOVES>), g, b, p.lds, e->stream, R, P, t0, n, \
+  hipLaunchKernelGGL((crl::k_fused_tickets<A, MODE, LDSW, MOVES, false>), g, b, p.lds, e->stream, R, P, t0, n, \
                      tk, p.tab_stride, p.fixed ? 1 : 0, p.tape_steps, p.lds_waves, p.env_bytes)
+#define CRL_LAUNCH_ROWS(MODE, MOVES)                                                                        \
+  hipLaunchKernelGGL((crl::k_fused_tickets<A, MODE, false, MOVES, true>), g, b, p.lds, e->stream, R, P, t0, n, tk, 0, 1, 0, 0, 0)
     const int events = crl::lane_events(R, P);
 #define CRL_LAUNCH_LANES(CELLS)                                                                                            \
   do {                                                                                                                     \
@@ -857,6 +904,14 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
       CRL_LAUNCH_LANES(true);
     else if (p.lanes)
       CRL_LAUNCH_LANES(false);
+    else if (p.rows && p.rich && p.moves)
+      CRL_LAUNCH_ROWS(2, true);
+    else if (p.rows && p.rich)
+      CRL_LAUNCH_ROWS(2, false);
+    else if (p.rows && p.moves)
+      CRL_LAUNCH_ROWS(1, true);
+    else if (p.rows)
+      CRL_LAUNCH_ROWS(1, false);
     else if (p.rich && p.moves)
       CRL_LAUNCH_TICKETS(2, false, true);
     else if (p.rich)
@@ -872,6 +927,7 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
     else
       CRL_LAUNCH_TICKETS(0, false, false);
 #undef CRL_LAUNCH_TICKETS
+#undef CRL_LAUNCH_ROWS
 #undef CRL_LAUNCH_LANES
     return;
   }
@@ -1709,7 +1765,7 @@ int create_engine(const crl_config* cfg, int device, crl_engine** out) {
     carve(e->Q, (size_t)e->n_tables * e->K);
     cleared = used;
     page((size_t)e->n_maps * e->mv_words * 4);
-    carve(e->moves, (size_t)e->n_maps * e->mv_words);  // move codes of every map, for the fused loops
+    carve(e->moves, (size_t)e->n_maps * e->mv_words + 1);  // move codes of every map, for the fused loops (and a word that is read, not used)
     if (cells) carve(e->cell_reward, (size_t)e->n_maps * e->S);
     carve(e->eps_tab, eps.size());
     carve(e->tr_s, N);
@@ -1827,20 +1883,20 @@ int set_cell(crl_engine* e, int32_t map_index, int32_t cell, int32_t cell_class,
   return CRL_OK;
 }
 
-// every ticket-kernel instantiation launch_fused_a can pick may use the whole LDS:
+// every ticket-kernel instantiation launch_fused_a can pick, but those that keep rows (20 KB at most), may use the whole LDS:
 // the plain ones, too, ask for more than the default 64 KB when large per-env
 // maps share a workgroup
 int opt_in_ticket_kernels(crl_engine* e) {
   if (e->hybrid_opt_in) return CRL_OK;
   const void* fns[] = {
 #define CRL_TICKET_KERNELS(A)                                                          \
-  reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 0, false, false>),            \
-      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, false, false>),        \
-      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 2, false, false>),        \
-      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 0, true, false>),         \
-      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, true, false>),         \
-      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, false, true>),         \
-      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 2, false, true>),         \
+  reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 0, false, false, false>),            \
+      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, false, false, false>),        \
+      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 2, false, false, false>),        \
+      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 0, true, false, false>),         \
+      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, true, false, false>),         \
+      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, false, true, false>),         \
+      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 2, false, true, false>),         \
       CRL_LANE_KERNELS(A, false), CRL_LANE_KERNELS(A, true),                           \
       reinterpret_cast<const void*>(&crl::k_fused_per_env<A, 1, 2>),                   \
       CRL_LDS_KERNELS(A, false), CRL_LDS_KERNELS(A, true)

@@ -434,6 +434,251 @@ __device__ __forceinline__ void run_env_fast(const Rules& R, const Ptrs& P, cons
   P.action[env] = (uint8_t)action;
 }
 
+// The folded loop for calls whose tables outgrow the caches, where what costs is the number of scattered
+// requests: the rows an env comes to are kept in LDS and written back when others take their place or the
+// call is over, so that a cell visited again costs none.
+// An env has four places, each for a run of kRun cells beside each other (cut off at the map's edge), 32 bytes
+// of the table, and a word: the run's name - first cell << 1, 1 more where it is cut off; kNone: none - and (CODES), from
+// bit 16 on, the move codes of its cells.  Which place follows from the lowest bits of x / kRun and of y, so that the runs next to each
+// other are in different ones.  Two lanes move a run together, 16 bytes each, first for one of them and then for the other.
+// [place][piece][lane], the lane mixed with the piece against bank conflicts; then the words, [place][lane].
+//
+// What bounds it: 270 vector instructions a step and, with them about half of the time, a trip to HBM for the lanes whose cell
+// is new - with 64 envs there is always one.  1M envs of 16x16, 20 steps, 627 us with a row and a value per step from and to
+// HBM (21M reads of 16 bytes that meet the L2 in 5.9M lines, 21M stores of 4 bytes); rows kept one by one, each lane moving
+// its own 474 (11.9M lines: with 16 waves to a compute unit none of it is met again in the L2); runs of two, each lane moving its own
+// 430, of four 484; runs of two moved by two lanes and only what was written put back 383, with nothing in flight at the loop's
+// entry and a word of 16 bits, so that 12 waves fit, 369; of four moved by four 474 (seven waves fit); more places would ask for
+// 10.7 rows in 20 steps where four ask for 12, and cost waves.  32 and 64 steps 910 and 1571 us -> 500 and 890.
+template <int A, bool CODES>
+struct RowCache {
+  using Word = std::conditional_t<CODES, uint32_t, uint16_t>;
+  static constexpr int kRun = 8 / A, kPlaces = 4, kBytes = 64 * kPlaces * (32 + (int)sizeof(Word));
+  static constexpr uint32_t kNone = 0xffffu, kRowBytes = 4 * A;
+  crl_f4* pieces;
+  Word* words;                  // the lane's
+  unsigned char* tables;        // of the wave's first env
+  const unsigned char* codes;
+  uint32_t table_at, codes_at;  // from there to the lane's env's
+  int lane, W;
+
+  static __device__ __forceinline__ int place(int x, int y) { return ((unsigned)x / kRun & 1) | (y & 1) << 1; }
+  static __device__ __forceinline__ int offset(int x) { return x & (kRun - 1); }
+  __device__ __forceinline__ uint32_t name(int s, int x) const {
+    return A == 4 ? (uint32_t)(s - offset(x)) << 1 | ((x | 1) == W ? 1u : 0u) : (uint32_t)s << 1;
+  }
+  __device__ __forceinline__ Word& word(int p) const { return words[p * 64]; }
+  __device__ __forceinline__ crl_f4* piece(int p, int c, int of_lane) const { return pieces + (p * 2 + c) * 64 + (of_lane ^ c); }
+  __device__ __forceinline__ Row<A> row(int p, int off) const {
+    if constexpr (A == 4) {
+      return load_row4(reinterpret_cast<const float*>(piece(p, off, lane)));
+    } else {
+      const crl_f4 t = *piece(p, 0, lane), u = *piece(p, 1, lane);
+      return Row<8>{t.x, t.y, t.z, t.w, u.x, u.y, u.z, u.w};
+    }
+  }
+  // which of a run's two pieces holds the value of that cell and action
+  static __device__ __forceinline__ int piece_of(int off, int a) { return A == 4 ? off : a >> 2; }
+  __device__ __forceinline__ float* value(int p, int off, int a) const {
+    return reinterpret_cast<float*>(piece(p, piece_of(off, a), lane)) + (a & 3);
+  }
+  // v of the even / odd one of the two lanes
+  template <int J>
+  static __device__ __forceinline__ uint32_t from(uint32_t v) {
+    constexpr int j = J, k = 2 + J;
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, j | j << 2 | k << 4 | k << 6, 0xf, 0xf, true);
+  }
+  // a run in HBM: where it starts and, in the two lowest bits, which of its pieces
+  __device__ __forceinline__ uint32_t run(uint32_t name, uint32_t pieces) const { return table_at + (name >> 1) * kRowBytes + pieces; }
+  __device__ __forceinline__ crl_f4* global(uint32_t run) const {
+    return reinterpret_cast<crl_f4*>(tables + ((run & ~15u) + (uint32_t)(lane & 1) * 16u));
+  }
+  __device__ __forceinline__ bool has(uint32_t run) const { return (run & (1u << (lane & 1))) != 0u; }
+
+  // (what comes from another lane is fetched while that is at work too: not under a condition)
+  struct Pieces {
+    crl_f4 even, odd;
+  };
+  __device__ __forceinline__ void ask(uint32_t run, Pieces& v) const {
+    const uint32_t even = from<0>(run), odd = from<1>(run);
+    if (has(even)) v.even = *global(even);
+    if (has(odd)) v.odd = *global(odd);
+  }
+  __device__ __forceinline__ Pieces take(int p) const {
+    const int even = (int)from<0>(p), odd = (int)from<1>(p);
+    return Pieces{*piece(even, lane & 1, lane & ~1), *piece(odd, lane & 1, lane | 1)};
+  }
+  __device__ __forceinline__ void put(int p, uint32_t run, const Pieces& v) const {
+    const int p_even = (int)from<0>(p), p_odd = (int)from<1>(p);
+    const uint32_t even = from<0>(run), odd = from<1>(run);
+    if (has(even)) *piece(p_even, lane & 1, lane & ~1) = v.even;
+    if (has(odd)) *piece(p_odd, lane & 1, lane | 1) = v.odd;
+  }
+  __device__ __forceinline__ void put_back(uint32_t run, const Pieces& v) const {
+    const uint32_t even = from<0>(run), odd = from<1>(run);
+    if (has(even)) *global(even) = v.even;
+    if (has(odd)) *global(odd) = v.odd;
+  }
+  __device__ __forceinline__ uint32_t codes_of(uint32_t name) const {
+    uint16_t two;  // (4 actions: a byte to a cell, at any address)
+    __builtin_memcpy(&two, codes + (codes_at + (name >> 1) * (A / 4)), 2);
+    return two;
+  }
+  static __device__ __forceinline__ uint32_t pieces_of(uint32_t name) { return A == 4 ? 3u - (name & 1u) * 2u : 3u; }
+};
+__device__ __forceinline__ void wave_fence();
+
+// All lanes of the wave call it; those without an env of their own do another's work once more, to the same effect.
+// CODES: the move codes come along with the runs, else from `moves`.
+template <int A, bool RICH, bool CODES, class Moves>
+__device__ __forceinline__ void run_env_rows(const Rules& R, const Ptrs& P, const int env, const bool live, const uint64_t t0,
+                                             const int n_steps, const Moves moves, const float* __restrict__ cr,
+                                             const RowCache<A, CODES> kept) {
+  using Cache = RowCache<A, CODES>;
+  const int W = R.W, T = R.episode_len > 0 ? R.episode_len : 0x7fffffff;
+  const float lr = R.lr, gamma = R.gamma;
+  uint32_t explore_below = explore_threshold(R.eps0);
+  float r_step = R.step_reward, r_goal = R.goal_reward, r_trap = R.trap_reward;
+  if (RICH) asm volatile("" : "+v"(r_step), "+v"(r_goal), "+v"(r_trap));
+  const bool cells = RICH && cr != nullptr;
+  const bool base_cells = cells && (R.reward_flags & 2) != 0;
+  const bool scheduled = RICH && R.eps_mode >= 2;
+  const int start = P.start[env];
+  int s = P.s[env];
+  int ep_step = P.ep_step[env];
+  int episode = P.episode[env];
+  const int sx = start % W, sy = start / W;
+  int x = s % W, y = s / W;
+  float reward = 0.0f;
+  int action = 0;
+  bool hit = false;
+  int place = Cache::place(x, y);
+  typename Cache::Pieces run;
+  const uint32_t name0 = kept.name(s, x), run0 = kept.run(name0, Cache::pieces_of(name0));
+  kept.ask(run0, run);
+  uint32_t codes = CODES ? kept.codes_of(name0) : 0u;
+#pragma unroll
+  for (int p = 0; p < Cache::kPlaces; ++p) kept.word(p) = Cache::kNone;
+  uint32_t written = 0;  // two bits for each place: the pieces of its run
+  if (scheduled) explore_below = explore_threshold(eps_of(R, P.eps_tab, t0, episode));
+  uint64_t next_block = (t0 >> 1) + 1;
+  Philox4 blk = explore_block(R.seed, (uint32_t)env, t0 >> 1);
+  bool odd = (t0 & 1) != 0;
+  kept.word(place) = (typename Cache::Word)(name0 | codes << 16);
+  kept.put(place, run0, run);
+  wave_fence();
+  Row<A> row = kept.row(place, Cache::offset(x));
+  uint32_t mv = CODES ? codes >> (8 * Cache::offset(x)) : moves.at(s, x, y);
+  // (all of these have arrived: what is in flight at the loop's entry makes every step wait for all its stores)
+  asm volatile("" : "+v"(ep_step), "+v"(episode), "+v"(mv), "+v"(explore_below));
+
+  for (int k = 0; k < n_steps; ++k) {
+    const uint32_t w0 = odd ? blk.w2 : blk.w0;
+    const uint32_t w1 = odd ? blk.w3 : blk.w1;
+    const int greedy = row_argmax(row);
+    const int a = ((w0 >> 8) < explore_below) ? (int)below(w1, (uint32_t)A) : greedy;
+
+    const uint32_t code = (mv >> (2 * a)) & 3u;
+    const bool moved = code < (uint32_t)kTrap;
+    int dx, dy;
+    action_delta(a, A, dx, dy);
+    hit = code == (uint32_t)kGoal;
+    const bool trap = code == (uint32_t)kTrap;
+    reward = hit ? r_goal : (trap ? r_trap : r_step);
+    float by_cell = 0.0f;
+    if (RICH && cells) {
+      const int tgt = s + __mul24(dy, W) + dx;
+      by_cell = cr[trap ? tgt : (moved ? tgt : s)];
+    }
+    dx = moved ? dx : 0;
+    dy = moved ? dy : 0;
+    const int s2 = s + __mul24(dy, W) + dx;
+    const int x2 = x + dx, y2 = y + dy;
+    ep_step += 1;
+    const bool ends = hit || ep_step >= T;
+
+    // the run of the cell to act from next: in its place, or asked for
+    const int s_next = ends ? start : s2;
+    const int off = Cache::offset(x);
+    x = ends ? sx : x2;
+    y = ends ? sy : y2;
+    const int place_next = Cache::place(x, y);
+    const uint32_t name_next = kept.name(s_next, x);
+    const uint32_t there = kept.word(place_next);
+    const bool miss = (there & 0xffffu) != name_next;
+    const uint32_t wanted = miss ? kept.run(name_next, Cache::pieces_of(name_next)) : 0u;
+    kept.ask(wanted, run);
+    if (CODES) {
+      codes = there >> 16;
+      if (miss) codes = kept.codes_of(name_next);
+    } else {
+      mv = moves.at(s_next, x, y);
+    }
+    if (odd) blk = explore_block(R.seed, (uint32_t)env, next_block++);  // in the loads' shadow
+    // Where the episode ends the update does not need that run: done first, because it may be the
+    // run of this step's cell that makes place.  A truncated one needs the row of the cell that the move ends on, at
+    // the goal the maximum is 0.
+    const float q_old = row_get(row, a);
+    float* const at = kept.value(place, off, a);
+    float q_new = 0.0f;
+    if (ends) {
+      float m = 0.0f;
+      if (!hit) {
+        const int place2 = Cache::place(x2, y2);
+        Row<A> row2 = kept.row(place2, Cache::offset(x2));
+        row_opaque(row2);  // (one load through a selected address otherwise)
+        if ((kept.word(place2) & 0xffffu) != kept.name(s2, x2))
+          row2 = load_row<A>(reinterpret_cast<const float*>(kept.tables + (kept.table_at + (uint32_t)s2 * Cache::kRowBytes)));
+        m = row_max(row2, false, R.max_mode);
+      }
+      if (RICH) reward = (cells && (hit || trap || base_cells)) ? by_cell : reward;
+      q_new = td_value(q_old, reward, m, lr, gamma);
+      *at = q_new;
+    }
+    written |= 1u << (place * 2 + Cache::piece_of(off, a));
+    wave_fence();
+    const typename Cache::Pieces old = kept.take(place_next);
+    const uint32_t gone = (written >> (place_next * 2)) & 3u;
+    const uint32_t leaves = miss ? kept.run(there & 0xffffu, gone) : 0u;
+    written &= miss ? ~(3u << (place_next * 2)) : ~0u;
+    if (miss) kept.word(place_next) = (typename Cache::Word)(name_next | codes << 16);
+    wave_fence();
+    kept.put(place_next, wanted, run);
+    wave_fence();
+    const Row<A> row_next = kept.row(place_next, Cache::offset(x));
+    kept.put_back(leaves, old);
+    if (!ends) {
+      if (RICH) reward = (cells && (trap || base_cells)) ? by_cell : reward;
+      q_new = td_value(q_old, reward, row_max(row_next, false, R.max_mode), lr, gamma);
+      *at = q_new;
+    }
+    row = row_set(row_next, s_next == s ? a : -1, q_new);
+    if (CODES) mv = codes >> (8 * Cache::offset(x));
+    place = place_next;
+    ep_step = ends ? 0 : ep_step;
+    episode += ends ? 1 : 0;
+    s = s_next;
+    action = a;
+    odd = !odd;
+    if (RICH && scheduled && __builtin_amdgcn_ballot_w64(ends) != 0) {
+      explore_below = explore_threshold(eps_of(R, P.eps_tab, t0, episode));
+      asm volatile("" : "+v"(explore_below));
+    }
+  }
+
+  wave_fence();
+#pragma unroll
+  for (int p = 0; p < Cache::kPlaces; ++p)
+    kept.put_back(kept.run(kept.word(p) & 0xffffu, (written >> (p * 2)) & 3u), kept.take(p));
+  if (!live) return;
+  P.s[env] = s;
+  P.ep_step[env] = ep_step;
+  P.episode[env] = episode;
+  P.reward[env] = reward;
+  P.done[env] = hit ? 1 : 0;
+  P.action[env] = (uint8_t)action;
+}
+
 // ---------------------------------------------------------------------------
 // One env to A lanes of a wave, a lane to an action, for batches that leave lanes to spare.
 // A lone wave issues an instruction every four cycles (measured: 2.4 GHz, dependent or not; a
@@ -1212,6 +1457,8 @@ __global__ __launch_bounds__(64, EVENTS == kAllEvents ? 5 : 6) void k_fused_lane
 // how many bytes of their tables - are live on the chip at once: few enough and
 // the rows an env keeps returning to are still in the last-level cache.
 //
+// ROWS: a wave to a workgroup, its envs by position, rows kept in LDS (run_env_rows; MOVES: the move codes with them, no maps).
+//
 // All waves of a workgroup but the LDS waves step 64 envs each against tables in HBM / the
 // caches, and spend most of their time waiting for one row per step.  With LDSW the last
 // `lds_waves` waves use the idle issue slots and the LDS: they stage the WHOLE tables of their
@@ -1285,8 +1532,8 @@ __device__ __forceinline__ void strided_copy(T* __restrict__ g, const int per, c
   }
 }
 
-template <int A, int MODE, bool LDSW, bool MOVES>
-__global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules R, const Ptrs P,
+template <int A, int MODE, bool LDSW, bool MOVES, bool ROWS>
+__global__ __launch_bounds__(LDSW ? 320 : ROWS ? 64 : 256) void k_fused_tickets(const Rules R, const Ptrs P,
                                                                      const uint64_t t0,
                                                                      const int n_steps,
                                                                      unsigned* __restrict__ ticket,
@@ -1301,7 +1548,7 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
   extern __shared__ __align__(16) uint32_t lds[];
   const int n_waves = (int)(blockDim.x >> 6);  // with LDSW the last `lds_waves` work on LDS tables
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = ROWS ? 0 : threadIdx.x >> 6;
   const bool lds_worker = LDSW && wave >= n_waves - lds_waves;
   // LDS: (kLaneTables) the rewards by class; one slice per table wave; then kLaneTables:
   // [LDS wave][its envs: rows, then move codes; its tape], else the LDS wave's slice, the tables
@@ -1363,12 +1610,25 @@ __global__ __launch_bounds__(LDSW ? 320 : 256) void k_fused_tickets(const Rules 
       strided_copy<false>(tables, (int)(table / 4), n_here, envs, env_bytes, lane);
       continue;
     }
-    if (codes)
+    if (codes && !ROWS)
       stage_words(P.moves + (size_t)env0 * P.mv_words, n_here, P.mv_words, cap, my_words, lane);
-    else
+    else if (!codes)
       stage_words(P.map + (size_t)env0 * P.map_words, n_here, P.map_words, 64, my_words, lane);
     const float* cr = P.cell_reward ? P.cell_reward + (size_t)env * P.S : nullptr;
 
+    if constexpr (ROWS) {
+      using Cache = RowCache<A, MOVES>;
+      wave_fence();
+      const int slot = min(lane, n_here - 1), first = __builtin_amdgcn_readfirstlane(env0);
+      crl_f4* pieces = reinterpret_cast<crl_f4*>(lds + (MOVES ? 0 : slice));
+      const Cache kept{pieces, reinterpret_cast<typename Cache::Word*>(pieces + 64 * Cache::kPlaces * 2) + lane,
+                       reinterpret_cast<unsigned char*>(P.Q + (size_t)first * table),
+                       reinterpret_cast<const unsigned char*>(P.moves + (size_t)first * P.mv_words),
+                       (uint32_t)slot * (uint32_t)table * 4u, (uint32_t)slot * (uint32_t)P.mv_words * 4u, lane, R.W};
+      run_env_rows<A, RICH, MOVES>(R, P, env0 + slot, live, t0, n_steps, MovesFromMap<A>{my_words + slot, R.W, R.H},
+                                   RICH && P.cell_reward ? P.cell_reward + (size_t)(env0 + slot) * P.S : nullptr, kept);
+      continue;
+    }
     if (!lds_worker) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
