@@ -374,7 +374,7 @@ struct FusedPlan {
   bool lanes;      // an env to A lanes, a wave to 2^log_envs envs, draws taped tape_steps ahead
   int log_envs, tape_steps;
   bool touch;      // ... whose tables are read ahead whole
-  bool rows;       // 64-env waves that keep their envs' rows in LDS (moves: and not their maps)
+  int rows;        // != 0: 64-env waves that keep their envs' rows in LDS, in so many places (moves: and not their maps)
   bool rich;       // ticket kernel: the folded loop's variant with per-cell rewards / per-episode epsilon
   int tab_stride;  // floats between two tables in LDS
   bool in_lds;     // ... with all tables in LDS
@@ -415,13 +415,20 @@ constexpr int kLaneTouchMinSteps4 = 90, kLaneTouchMinSteps8 = 160, kLaneTouchFou
 constexpr int kHybridFewRoundsMinSteps = 384, kHybridOneWaveMinSteps = 96;
 constexpr long kHybridEnvStepsSmall = 18000000, kHybridEnvSteps4 = 24000000, kHybridEnvSteps8 = 28000000, kHybridEnvSteps8FewRounds = 20000000;
 constexpr size_t kTableBytesAtOnce = (size_t)512 << 20;
-// 64-env waves that keep rows in LDS.  With the maps in LDS too where eight of them and more fit a compute unit, else the move codes
+// 64-env waves that keep rows in LDS, with the maps in LDS too where enough of them fit a compute unit, else the move codes
 // come from HBM with the rows (20 steps, staged / not: 1M of 16x16 369 / 452 us, 100,000 of 22x22 with 8 actions 62 / 69, of
-// 32x32, six staged to a unit, 73 / 55).
-constexpr int kRowsManyEnvs = 1 << 18, kRowsHybridSteps4 = 48, kRowsHybridSteps8 = 64, kRowsFewEnvsSteps = 80;
+// 32x32, six staged to a unit, 73 / 55; 262,144 of 28x28, seven, 10 / 40 / 150 steps 77 / 208 / 701, 78 / 215 / 725; of 32x32 with 8
+// actions, whose codes are twice as long, 96 / 214 / 658 at 10 / 30 / 100, 104 / 251 / 788).
+// Six places for an env's rows in place of four, in longer calls: fewer rows asked for again, fewer waves to a unit (four / six,
+// 1M of 16x16, nine waves fit, 3 / 20 / 40 / 150 / 400 steps 111 / 362 / 598 / 2262 / 5944, 114 / 355 / 570 / 1907 / 5027; of 8x8, 40 / 150
+// 487 / 2012, 438 / 1410; 300,000 of 20x20, eight, 24 / 50 / 150 126 / 236 / 681, 136 / 245 / 664; of 28x28, six, 40 / 150 208 / 701,
+// 210 / 672; of 32x32, five, 150 steps 721, 797; 300,000 of 16x16 with 8 actions, 60 / 300 392 / 1965, 390 / 1806; eight places, 300 steps of
+// 1M of 16x16 3747 -> 3967.  With epsilon by episode, where envs explore, 1M of 16x16, 24 / 60 / 200 steps 414 / 956 / 3118, 436 / 1033 / 3255).
+constexpr int kRowsManyEnvs = 1 << 18, kRowsHybridSteps4 = 64, kRowsHybridSteps8 = 96, kRowsFewEnvsSteps = 80;
 constexpr size_t kRowsSmallMap = 336;  // cells: eleven to a unit
 constexpr int kRowsLargeMapMinSteps = 11, kRowsLargeMapMaxSteps = 130;
-constexpr long kRowsStagedWaves = 8;
+constexpr long kRowsStagedWaves4 = 7, kRowsStagedWaves8 = 6, kRowsSixSoonWaves = 9, kRowsSixWaves = 6;
+constexpr int kRowsSixSoonSteps = 32, kRowsSixSteps = 100;
 
 // Configurations that run_lanes() steps: no goal test on the resulting cell, no sticky done,
 // no trace and no supplied stream.
@@ -683,17 +690,17 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     //     of 27x27, 300 steps 2119, 1583; 262,144 of 32x32, 250 / 800 steps 1541 / 4450, 1185 / 3777; of 16x16 with 8 actions,
     //     150 steps 1183, 859; 300,000 of 4x4 with 8 actions, 8 / 60 steps 68 / 298, 40 / 172
     //   hybrid workgroups, up to a length that grows with the table:
-    //     1M of 8x8, 40 / 80 / 150 steps 697 / 939 / 1422, 478 / 925 / 1877; 400,000 of 12x12, 60 / 110 / 150 470 / 658 / 785,
-    //     329 / 577 / 793; 1M of 16x16, 80 / 150 / 220 1892 / 2533 / 3217, 1101 / 2099 / 3160; 600,000 of 20x20, 200 / 450
-    //     2669 / 4689, 1703 / 4014; 8 actions: 600,000 of 8x8, 60 / 100 / 140 816 / 1095 / 1367, 616 / 1011 / 1444; 500,000
-    //     of 12x12, 150 / 250 1572 / 2202, 1535 / 2696; of 16x16, 220 / 300 2779 / 3276, 2265 / 3175; 262,144 of 22x22, 600 4262, 3805
+    //     1M of 8x8, 40 / 80 / 150 steps 697 / 939 / 1439, 438 / 780 / 1410; 400,000 of 12x12, 130 / 180 / 250 720 / 872 / 1127,
+    //     621 / 852 / 1159; 1M of 16x16, 80 / 150 / 330 / 400 1892 / 2533 / 4227 / 4861, 1000 / 1907 / 4120 / 5027; 300,000 of 20x20,
+    //     400 / 800 2156 / 3729, 1736 / 3506; 8 actions: 600,000 of 8x8, 100 / 170 1074 / 1575, 784 / 1283; 500,000 of 12x12, 160 / 200
+    //     1616 / 1911, 1411 / 1744; 300,000 of 16x16, 300 / 400 / 500 2011 / 2428 / 2854, 1806 / 2431 / 3091; 262,144 of 22x22, 600 4262, 3805
     // With fewer envs a step is as long as its slowest request and lane waves have fewer of those (50,000 of 16x16, 20 steps
     // 26.6, 33.3).  What is left to the others between that and these lines are lengths and sizes that tests hold them to.
     const bool rows_can = lanes_rules(e) && c.max_episodes == 0 && c.track_returns == 0 && c.eps_mode != CRL_EPS_STEP_MULT &&
                           e->mv_words > 0 && e->resident_envs == 0 && e->fused_variant != 2;
     const int rows_steps = !(fits && p.fast) ? INT_MAX
-                           : e->A == 8       ? kRowsHybridSteps8 + (int)(e->K / 16)
-                                             : kRowsHybridSteps4 + (int)(e->K / 7);
+                           : e->A == 8       ? kRowsHybridSteps8 + (int)(e->K / 8)
+                                             : kRowsHybridSteps4 + (int)(e->K / 4);
     const bool rows_small = e->S <= kRowsSmallMap;
     const bool rows_first =
         rows_can && e->fused_variant == 0 &&
@@ -818,11 +825,18 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       // as there are envs for, a workgroup each).
       if (rows_first || (!p.lanes && rows_can && foldable &&
                          (rows_small || (n_steps >= kRowsLargeMapMinSteps && n_steps <= kRowsLargeMapMaxSteps)))) {
-        p.rows = p.fast = p.fixed = true;
+        p.fast = p.fixed = true;
         p.rich = c.eps_mode != CRL_EPS_FIXED || c.reward_flags != 0;
-        p.lds = map_lds + crl::RowCache<4, false>::kBytes;
-        p.moves = lds_fit(p.lds) < kRowsStagedWaves;
-        if (p.moves) p.lds = crl::RowCache<4, true>::kBytes;
+        const size_t staged4 = map_lds + crl::RowCache<4, false, 4>::kBytes, staged6 = map_lds + crl::RowCache<4, false, 6>::kBytes;
+        const long fit6 = lds_fit(staged6);
+        if (!p.rich && (fit6 >= kRowsSixSoonWaves ? n_steps >= kRowsSixSoonSteps : fit6 >= kRowsSixWaves && n_steps >= kRowsSixSteps)) {
+          p.rows = 6;
+          p.lds = staged6;
+        } else {
+          p.rows = 4;
+          p.moves = lds_fit(staged4) < (e->A == 8 ? kRowsStagedWaves8 : kRowsStagedWaves4);
+          p.lds = p.moves ? crl::RowCache<4, true, 4>::kBytes : staged4;
+        }
         p.block = 64;
         p.grid = (int)(((long)e->N + 63) / 64);
       }
@@ -886,10 +900,10 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
     const dim3 g(p.grid), b(p.block);
     unsigned* tk = p.fixed ? e->split.p : e->tk;
 #define CRL_LAUNCH_TICKETS(MODE, LDSW, MOVES)                                                       \
-  hipLaunchKernelGGL((crl::k_fused_tickets<A, MODE, LDSW, MOVES, false>), g, b, p.lds, e->stream, R, P, t0, n, \
+  hipLaunchKernelGGL((crl::k_fused_tickets<A, MODE, LDSW, MOVES, 0>), g, b, p.lds, e->stream, R, P, t0, n, \
                      tk, p.tab_stride, p.fixed ? 1 : 0, p.tape_steps, p.lds_waves, p.env_bytes)
-#define CRL_LAUNCH_ROWS(MODE, MOVES)                                                                        \
-  hipLaunchKernelGGL((crl::k_fused_tickets<A, MODE, false, MOVES, true>), g, b, p.lds, e->stream, R, P, t0, n, tk, 0, 1, 0, 0, 0)
+#define CRL_LAUNCH_ROWS(MODE, MOVES, PLACES)                                                                                 \
+  hipLaunchKernelGGL((crl::k_fused_tickets<A, MODE, false, MOVES, PLACES>), g, b, p.lds, e->stream, R, P, t0, n, tk, 0, 1, 0, 0, 0)
     const int events = crl::lane_events(R, P);
 #define CRL_LAUNCH_LANES(CELLS)                                                                                            \
   do {                                                                                                                     \
@@ -904,14 +918,16 @@ void launch_fused_a(const crl_engine* e, const FusedPlan& p, uint64_t t0, int n)
       CRL_LAUNCH_LANES(true);
     else if (p.lanes)
       CRL_LAUNCH_LANES(false);
+    else if (p.rows == 6)
+      CRL_LAUNCH_ROWS(1, false, 6);
     else if (p.rows && p.rich && p.moves)
-      CRL_LAUNCH_ROWS(2, true);
+      CRL_LAUNCH_ROWS(2, true, 4);
     else if (p.rows && p.rich)
-      CRL_LAUNCH_ROWS(2, false);
+      CRL_LAUNCH_ROWS(2, false, 4);
     else if (p.rows && p.moves)
-      CRL_LAUNCH_ROWS(1, true);
+      CRL_LAUNCH_ROWS(1, true, 4);
     else if (p.rows)
-      CRL_LAUNCH_ROWS(1, false);
+      CRL_LAUNCH_ROWS(1, false, 4);
     else if (p.rich && p.moves)
       CRL_LAUNCH_TICKETS(2, false, true);
     else if (p.rich)
@@ -1890,13 +1906,13 @@ int opt_in_ticket_kernels(crl_engine* e) {
   if (e->hybrid_opt_in) return CRL_OK;
   const void* fns[] = {
 #define CRL_TICKET_KERNELS(A)                                                          \
-  reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 0, false, false, false>),            \
-      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, false, false, false>),        \
-      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 2, false, false, false>),        \
-      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 0, true, false, false>),         \
-      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, true, false, false>),         \
-      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, false, true, false>),         \
-      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 2, false, true, false>),         \
+  reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 0, false, false, 0>),            \
+      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, false, false, 0>),        \
+      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 2, false, false, 0>),        \
+      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 0, true, false, 0>),         \
+      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, true, false, 0>),         \
+      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 1, false, true, 0>),         \
+      reinterpret_cast<const void*>(&crl::k_fused_tickets<A, 2, false, true, 0>),         \
       CRL_LANE_KERNELS(A, false), CRL_LANE_KERNELS(A, true),                           \
       reinterpret_cast<const void*>(&crl::k_fused_per_env<A, 1, 2>),                   \
       CRL_LDS_KERNELS(A, false), CRL_LDS_KERNELS(A, true)

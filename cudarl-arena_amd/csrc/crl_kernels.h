@@ -450,10 +450,10 @@ __device__ __forceinline__ void run_env_fast(const Rules& R, const Ptrs& P, cons
 // 430, of four 484; runs of two moved by two lanes and only what was written put back 383, with nothing in flight at the loop's
 // entry and a word of 16 bits, so that 12 waves fit, 369; of four moved by four 474 (seven waves fit); more places would ask for
 // 10.7 rows in 20 steps where four ask for 12, and cost waves.  32 and 64 steps 910 and 1571 us -> 500 and 890.
-template <int A, bool CODES>
+template <int A, bool CODES, int PLACES>
 struct RowCache {
   using Word = std::conditional_t<CODES, uint32_t, uint16_t>;
-  static constexpr int kRun = 8 / A, kPlaces = 4, kBytes = 64 * kPlaces * (32 + (int)sizeof(Word));
+  static constexpr int kRun = 8 / A, kPlaces = PLACES, kBytes = 64 * kPlaces * (32 + (int)sizeof(Word));
   static constexpr uint32_t kNone = 0xffffu, kRowBytes = 4 * A;
   crl_f4* pieces;
   Word* words;                  // the lane's
@@ -462,7 +462,7 @@ struct RowCache {
   uint32_t table_at, codes_at;  // from there to the lane's env's
   int lane, W;
 
-  static __device__ __forceinline__ int place(int x, int y) { return ((unsigned)x / kRun & 1) | (y & 1) << 1; }
+  static __device__ __forceinline__ int place(int x, int y) { return ((unsigned)x / kRun & 1) | ((unsigned)y % (PLACES / 2)) << 1; }
   static __device__ __forceinline__ int offset(int x) { return x & (kRun - 1); }
   __device__ __forceinline__ uint32_t name(int s, int x) const {
     return A == 4 ? (uint32_t)(s - offset(x)) << 1 | ((x | 1) == W ? 1u : 0u) : (uint32_t)s << 1;
@@ -530,11 +530,11 @@ __device__ __forceinline__ void wave_fence();
 
 // All lanes of the wave call it; those without an env of their own do another's work once more, to the same effect.
 // CODES: the move codes come along with the runs, else from `moves`.
-template <int A, bool RICH, bool CODES, class Moves>
+template <int A, bool RICH, bool CODES, int PLACES, class Moves>
 __device__ __forceinline__ void run_env_rows(const Rules& R, const Ptrs& P, const int env, const bool live, const uint64_t t0,
                                              const int n_steps, const Moves moves, const float* __restrict__ cr,
-                                             const RowCache<A, CODES> kept) {
-  using Cache = RowCache<A, CODES>;
+                                             const RowCache<A, CODES, PLACES> kept) {
+  using Cache = RowCache<A, CODES, PLACES>;
   const int W = R.W, T = R.episode_len > 0 ? R.episode_len : 0x7fffffff;
   const float lr = R.lr, gamma = R.gamma;
   uint32_t explore_below = explore_threshold(R.eps0);
@@ -1532,7 +1532,7 @@ __device__ __forceinline__ void strided_copy(T* __restrict__ g, const int per, c
   }
 }
 
-template <int A, int MODE, bool LDSW, bool MOVES, bool ROWS>
+template <int A, int MODE, bool LDSW, bool MOVES, int ROWS>
 __global__ __launch_bounds__(LDSW ? 320 : ROWS ? 64 : 256) void k_fused_tickets(const Rules R, const Ptrs P,
                                                                      const uint64_t t0,
                                                                      const int n_steps,
@@ -1616,8 +1616,8 @@ __global__ __launch_bounds__(LDSW ? 320 : ROWS ? 64 : 256) void k_fused_tickets(
       stage_words(P.map + (size_t)env0 * P.map_words, n_here, P.map_words, 64, my_words, lane);
     const float* cr = P.cell_reward ? P.cell_reward + (size_t)env * P.S : nullptr;
 
-    if constexpr (ROWS) {
-      using Cache = RowCache<A, MOVES>;
+    if constexpr (ROWS != 0) {
+      using Cache = RowCache<A, MOVES, ROWS>;
       wave_fence();
       const int slot = min(lane, n_here - 1), first = __builtin_amdgcn_readfirstlane(env0);
       crl_f4* pieces = reinterpret_cast<crl_f4*>(lds + (MOVES ? 0 : slice));
@@ -1625,7 +1625,7 @@ __global__ __launch_bounds__(LDSW ? 320 : ROWS ? 64 : 256) void k_fused_tickets(
                        reinterpret_cast<unsigned char*>(P.Q + (size_t)first * table),
                        reinterpret_cast<const unsigned char*>(P.moves + (size_t)first * P.mv_words),
                        (uint32_t)slot * (uint32_t)table * 4u, (uint32_t)slot * (uint32_t)P.mv_words * 4u, lane, R.W};
-      run_env_rows<A, RICH, MOVES>(R, P, env0 + slot, live, t0, n_steps, MovesFromMap<A>{my_words + slot, R.W, R.H},
+      run_env_rows<A, RICH, MOVES, ROWS>(R, P, env0 + slot, live, t0, n_steps, MovesFromMap<A>{my_words + slot, R.W, R.H},
                                    RICH && P.cell_reward ? P.cell_reward + (size_t)(env0 + slot) * P.S : nullptr, kept);
       continue;
     }
