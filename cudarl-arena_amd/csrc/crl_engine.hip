@@ -233,6 +233,9 @@ struct crl_engine {
   bool mirror_read = false;     // ... because the state was read after the step before
   bool stepped = false;         // crl_step was the last call that changed the state
   unsigned mirror_seq = 0;      // != 0: out_page holds the state as of this launch
+  bool state_read = false;      // crl_get_state was called since the state last changed
+  bool stats_follow = false;    // the statistics were read after the state the last time: they go out with it ...
+  bool stats_here = false;      // ... and are in out_page, behind the state
 
   DevBuf<int32_t> s, ep_step, episode, start, act;
   DevBuf<float> reward;
@@ -1501,6 +1504,7 @@ int wait_seq(crl_engine* e, unsigned seq) {
 // out_page with room for `bytes`; what it held is no longer there
 int claim_out_page(crl_engine* e, size_t bytes) {
   e->mirror_seq = 0;
+  e->stats_here = false;
   if (bytes <= e->out_page.n) return CRL_OK;
   HIP_TRY(hipStreamSynchronize(e->stream));  // nobody may still be writing to the smaller one
   if (!e->out_page.ensure(bytes)) return fail(CRL_E_ALLOC, "pinned host memory: %zu bytes", bytes);
@@ -1648,6 +1652,7 @@ int state_changes(crl_engine* e) {
   if (rc) return rc;
   if (e->recorded) e->state_shared = true;
   e->mirror_seq = 0;
+  e->state_read = e->stats_here = false;
   e->stepped = false;
   return CRL_OK;
 }
@@ -2357,10 +2362,17 @@ int crl_get_state(crl_engine* e, int32_t* s, float* reward, uint8_t* done, uint8
       rc = wait_seq(e, e->mirror_seq);
       if (rc == CRL_OK) rc = check_persist(e);
     } else {
-      rc = fetch_pinned(e, e->state_at, e->state_bytes);
+      // A caller that reads the statistics after the state (a training loop, chunk after chunk) gets both with one launch:
+      // 7 us of a second launch and its answer saved, 16 bytes per env over the link added, so it stops with the first state
+      // whose statistics nobody asked for.  (One env, 500 steps, state, statistics 77.5 -> 70.3 us; 4096 100.3 -> 92.6.)
+      const size_t more = e->stats_follow && !e->state_shared && e->state_bytes + e->stats_bytes <= kLinkLimitBytes ? e->stats_bytes : 0;
+      rc = fetch_pinned(e, e->state_at, e->state_bytes + more);
+      e->stats_here = rc == CRL_OK && more != 0;
       if (rc == CRL_OK && e->stepped) e->mirror_steps = true;
     }
     if (rc) return rc;
+    e->state_read = true;
+    e->stats_follow = false;
     e->mirror_read = true;
     const crl::StateMirror M = state_mirror(e);
     if (s) std::memcpy(s, M.s, N * 4);
@@ -2409,10 +2421,16 @@ int crl_get_episode_stats(crl_engine* e, float* last_return, int32_t* last_lengt
   if (!e->cfg.track_returns) return fail(CRL_E_STATE, "the engine was created without track_returns");
   const size_t b = (size_t)e->N * 4;
   if (e->stats_bytes <= kLinkLimitBytes) {
-    rc = fetch_pinned(e, e->stats_at, e->stats_bytes);
-    if (rc) return rc;
+    const unsigned char* at = e->out_page.p + e->state_bytes;
+    if (!e->stats_here) {
+      rc = fetch_pinned(e, e->stats_at, e->stats_bytes);
+      if (rc) return rc;
+      at = e->out_page.p;
+    }
+    e->stats_here = false;
+    e->stats_follow = e->state_read;
     auto out = [&](void* to, const void* from) {
-      if (to) std::memcpy(to, e->out_page.p + (static_cast<const unsigned char*>(from) - e->stats_at), b);
+      if (to) std::memcpy(to, at + (static_cast<const unsigned char*>(from) - e->stats_at), b);
     };
     out(last_return, e->ret_last.p);
     out(last_length, e->len_last.p);
@@ -2556,6 +2574,7 @@ int crl_device_ptr(crl_engine* e, int32_t which, void** out) {
   if (which != CRL_PTR_Q) {  // the caller may write through it from now on
     e->state_shared = true;
     e->mirror_seq = 0;
+    e->stats_here = false;
   }
   return CRL_OK;
 }
