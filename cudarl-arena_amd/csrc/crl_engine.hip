@@ -427,7 +427,8 @@ constexpr size_t kTableBytesAtOnce = (size_t)512 << 20;
 // 487 / 2012, 438 / 1410; 300,000 of 20x20, eight, 24 / 50 / 150 126 / 236 / 681, 136 / 245 / 664; of 28x28, six, 40 / 150 208 / 701,
 // 210 / 672; of 32x32, five, 150 steps 721, 797; 300,000 of 16x16 with 8 actions, 60 / 300 392 / 1965, 390 / 1806; eight places, 300 steps of
 // 1M of 16x16 3747 -> 3967.  With epsilon by episode, where envs explore, 1M of 16x16, 24 / 60 / 200 steps 414 / 956 / 3118, 436 / 1033 / 3255).
-constexpr int kRowsManyEnvs = 1 << 18, kRowsHybridSteps4 = 64, kRowsHybridSteps8 = 96, kRowsFewEnvsSteps = 80;
+constexpr int kRowsManyEnvs = 1 << 18, kRowsManyLargerTables = 200000, kRowsHybridSteps4 = 48, kRowsHybridSteps8 = 96;
+constexpr int kRowsSomeEnvs = 6 * 64 * kComputeUnits, kRowsSomeEnvsSteps = 88;
 constexpr size_t kRowsSmallMap = 336;  // cells: eleven to a unit
 constexpr int kRowsLargeMapMinSteps = 11, kRowsLargeMapMaxSteps = 130;
 constexpr long kRowsStagedWaves4 = 7, kRowsStagedWaves8 = 6, kRowsSixSoonWaves = 9, kRowsSixWaves = 6;
@@ -696,20 +697,22 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     //     1M of 8x8, 40 / 80 / 150 steps 697 / 939 / 1439, 438 / 780 / 1410; 400,000 of 12x12, 130 / 180 / 250 720 / 872 / 1127,
     //     621 / 852 / 1159; 1M of 16x16, 80 / 150 / 330 / 400 1892 / 2533 / 4227 / 4861, 1000 / 1907 / 4120 / 5027; 300,000 of 20x20,
     //     400 / 800 2156 / 3729, 1736 / 3506; 8 actions: 600,000 of 8x8, 100 / 170 1074 / 1575, 784 / 1283; 500,000 of 12x12, 160 / 200
-    //     1616 / 1911, 1411 / 1744; 300,000 of 16x16, 300 / 400 / 500 2011 / 2428 / 2854, 1806 / 2431 / 3091; 262,144 of 22x22, 600 4262, 3805
-    // With fewer envs a step is as long as its slowest request and lane waves have fewer of those (50,000 of 16x16, 20 steps
-    // 26.6, 33.3).  What is left to the others between that and these lines are lengths and sizes that tests hold them to.
+    //     1616 / 1911, 1411 / 1744; 230,000 of 12x12 with 4, 150 / 180 451 / 508, 451 / 538; of 16x16, 250 / 300 869 / 975, 815 / 985; 300,000 of 16x16, 300 / 400 / 500 2011 / 2428 / 2854, 1806 / 2431 / 3091; 262,144 of 22x22, 600 4262, 3805
+    //   fewer envs, lane waves in two rounds and more: 99,000 of 9x8, 16 / 50 / 80 steps 29 / 68 / 99, 27 / 62 / 91; of 12x12, 30 / 80
+    //     69 / 151, 47 / 94; 200,000 of 5x4, 16 / 50 46 / 113, 37 / 110; of 15x15, 50 / 80 270 / 402, 175 / 261; 8 actions: 99,000 of 4x4,
+    //     8 / 50 28 / 102, 18 / 71; 130,000 of 9x9, 30 / 80 120 / 232, 79 / 140; 260,000 of 7x7, 16 / 80 141 / 435, 83 / 279
+    // With fewer envs still a step is as long as its slowest request and lane waves have fewer of those (50,000 of 16x16, 20 steps
+    // 26.6, 33.3).  Between that and these lines lie lengths and sizes that tests hold the others to.
     const bool rows_can = lanes_rules(e) && c.max_episodes == 0 && c.track_returns == 0 && c.eps_mode != CRL_EPS_STEP_MULT &&
                           e->mv_words > 0 && e->resident_envs == 0 && e->fused_variant != 2;
     const int rows_steps = !(fits && p.fast) ? INT_MAX
                            : e->A == 8       ? kRowsHybridSteps8 + (int)(e->K / 8)
-                                             : kRowsHybridSteps4 + (int)(e->K / 4);
+                                             : kRowsHybridSteps4 + (int)(3 * e->K / 16);
     const bool rows_small = e->S <= kRowsSmallMap;
-    const bool rows_first =
-        rows_can && e->fused_variant == 0 &&
-        ((e->N >= kRowsManyEnvs && n_steps <= rows_steps) ||
-         (foldable && (long)e->N > kLaneRoundsManyEnvs && e->K >= 1024 && !lanes_at_once && n_steps <= kRowsFewEnvsSteps &&
-          (rows_small || n_steps >= kRowsLargeMapMinSteps)));
+    const bool rows_many = e->N >= kRowsManyEnvs || (e->N > kRowsManyLargerTables && e->K > 256);
+    const bool rows_some = foldable && !lanes_at_once && n_steps <= kRowsSomeEnvsSteps && (rows_small || n_steps >= kRowsLargeMapMinSteps) &&
+                           (e->N > kRowsSomeEnvs ? e->N <= kRowsManyLargerTables : (long)e->N > kLaneRoundsManyEnvs && e->K >= 640);
+    const bool rows_first = rows_can && e->fused_variant == 0 && ((rows_many && n_steps <= rows_steps) || rows_some);
     // ... hybrid workgroups (automatic) when the tables outgrow the caches: while they all fit, other plans are
     // faster (16x16 maps, 30,000 envs: 3.5e10 hybrid, 5.9e10 with lane waves); and where lane
     // waves could step what is left to the general loop, they are faster too (262,144 envs of

@@ -33,7 +33,8 @@ def test_short_calls(gpu, oracle, N, W, H, A, kw):
     (262144, 5, 3, 4, 55, dict()), (262145, 4, 4, 8, 72, dict()), (262207, 1, 7, 4, 33, dict()), (262147, 2, 2, 8, 40, dict(episode_len=2)),
     (262147, 7, 2, 4, 47, dict(max_mode=1)), (262147, 3, 3, 8, 150, dict(max_mode=1, **LINEAR)),
     (262147, 6, 5, 4, 80, dict(cells=3, episode_len=3)), (262147, 3, 6, 8, 50, dict(cells=1, max_mode=1)),
-    (262147, 5, 5, 4, 40, dict(LINEAR, episode_len=1)), (262149, 4, 5, 4, 84, dict(episode_len=5)), (262149, 3, 7, 8, 110, dict(episode_len=40)),
+    (98305, 5, 4, 4, 88, dict()), (200000, 3, 3, 8, 50, dict()), (200001, 9, 8, 4, 90, dict()), (82500, 13, 13, 4, 40, dict(episode_len=30)),
+    (262147, 5, 5, 4, 40, dict(LINEAR, episode_len=1)), (262149, 4, 5, 4, 60, dict(episode_len=5)), (262149, 3, 7, 8, 110, dict(episode_len=40)),
 ])
 def test_many_envs(gpu, oracle, N, W, H, A, steps, kw):
     rows_check(gpu, oracle, N, W, H, A, (steps, 9, 31), True, lambda c: 6 if c >= 32 and not ("eps_mode" in kw or "cells" in kw) else 4, **kw)
