@@ -428,7 +428,7 @@ constexpr size_t kTableBytesAtOnce = (size_t)512 << 20;
 // 210 / 672; of 32x32, five, 150 steps 721, 797; 300,000 of 16x16 with 8 actions, 60 / 300 392 / 1965, 390 / 1806; eight places, 300 steps of
 // 1M of 16x16 3747 -> 3967.  With epsilon by episode, where envs explore, 1M of 16x16, 24 / 60 / 200 steps 414 / 956 / 3118, 436 / 1033 / 3255).
 constexpr int kRowsManyEnvs = 1 << 18, kRowsManyLargerTables = 200000, kRowsHybridSteps4 = 48, kRowsHybridSteps8 = 96;
-constexpr int kRowsSomeEnvs = 6 * 64 * kComputeUnits, kRowsSomeEnvsSteps = 88;
+constexpr int kRowsSomeEnvs = 6 * 64 * kComputeUnits, kRowsSomeEnvsRich = 1 << 17, kRowsSomeEnvsSteps = 88, kRowsLanesSteps = 500;
 constexpr size_t kRowsSmallMap = 336;  // cells: eleven to a unit
 constexpr int kRowsLargeMapMinSteps = 11, kRowsLargeMapMaxSteps = 130;
 constexpr long kRowsStagedWaves4 = 7, kRowsStagedWaves8 = 6, kRowsSixSoonWaves = 9, kRowsSixWaves = 6;
@@ -690,9 +690,14 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     //   64-env waves: 1M envs of 16x16, 3 / 6 / 10 / 20 / 32 steps 166 / 272 / 378 / 627 / 910, 108 / 178 / 245 / 369 / 500;
     //     262,144 of 32x32, 8 / 80 steps 93 / 628, 58 / 405; of 22x22 with 8 actions, 8 steps 105, 69; of 48x40 3 / 200 steps
     //     86 / 1477, 44 / 1011; 1M of 5x5, 1 / 8 steps 64 / 268, 63 / 133; 20,000 of 16x16, 1 / 4 steps 12.7 / 10.3, 7.9 / 9.8
-    //   rounds of lane waves, however long: 1M of 16x16, 64 steps 1571, 890; 300,000 of 16x16, floored maximum, 200 steps 1068, 856;
-    //     of 27x27, 300 steps 2119, 1583; 262,144 of 32x32, 250 / 800 steps 1541 / 4450, 1185 / 3777; of 16x16 with 8 actions,
-    //     150 steps 1183, 859; 300,000 of 4x4 with 8 actions, 8 / 60 steps 68 / 298, 40 / 172
+    //   rounds of lane waves: 1M of 16x16, 64 steps 1571, 890; 262,144 of 32x32, 250 / 800 steps 1541 / 4450, 1185 / 3777; of 16x16 with 8
+    //     actions, 150 steps 1183, 859; 300,000 of 4x4 with 8 actions, 8 / 60 steps 68 / 298, 40 / 172
+    //     (floored maximum, however long with 4 actions: 90,000 of 16x16, 5 / 100 / 400 steps 28 / 175 / 625, 16 / 132 / 472; of 9x9 100 / 400
+    //     112 / 402, 114 / 416; 130,000 of 12x12, 1000 steps 1604, 1125; 300,000 of 16x16, 200 / 1000 steps 1068 / 4350, 856 / 3913;
+    //     8 actions: 130,000 of 14x14, 100 / 1000 steps 433 / 2636, 256 / 2266; 200,000 400 / 700 steps 1793 / 2849, 1679 / 2968, of 20x20 1000
+    //     steps 5194, 4589; epsilon by episode, where envs explore, up to 500 steps: 300,000 of 16x16, 350 / 500 / 1000 1863 / 2575 /
+    //     4949, 1722 / 2491 / 5315; 600,000 of 9x9, 300 / 1000 2696 / 7291, 2285 / 8516; 300,000 of 30x30, 1000 steps 6580, 6034;
+    //     115,000 of 9x9, 20 / 60 steps 38 / 98, 41 / 104; 160,000 of 5x5 51 / 127, 45 / 110)
     //   hybrid workgroups, up to a length that grows with the table:
     //     1M of 8x8, 40 / 80 / 150 steps 697 / 939 / 1439, 438 / 780 / 1410; 400,000 of 12x12, 130 / 180 / 250 720 / 872 / 1127,
     //     621 / 852 / 1159; 1M of 16x16, 80 / 150 / 330 / 400 1892 / 2533 / 4227 / 4861, 1000 / 1907 / 4120 / 5027; 300,000 of 20x20,
@@ -705,14 +710,18 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     // 26.6, 33.3).  Between that and these lines lie lengths and sizes that tests hold the others to.
     const bool rows_can = lanes_rules(e) && c.max_episodes == 0 && c.track_returns == 0 && c.eps_mode != CRL_EPS_STEP_MULT &&
                           e->mv_words > 0 && e->resident_envs == 0 && e->fused_variant != 2;
-    const int rows_steps = !(fits && p.fast) ? INT_MAX
-                           : e->A == 8       ? kRowsHybridSteps8 + (int)(e->K / 8)
-                                             : kRowsHybridSteps4 + (int)(3 * e->K / 16);
+    const bool rows_rich = c.eps_mode != CRL_EPS_FIXED || c.reward_flags != 0;
+    const int rows_steps = fits && p.fast ? (e->A == 8 ? kRowsHybridSteps8 + (int)(e->K / 8) : kRowsHybridSteps4 + (int)(3 * e->K / 16))
+                           : e->A == 8 || rows_rich ? std::max(kRowsLanesSteps, (int)(e->K / 3))
+                                                    : INT_MAX;
     const bool rows_small = e->S <= kRowsSmallMap;
     const bool rows_many = e->N >= kRowsManyEnvs || (e->N > kRowsManyLargerTables && e->K > 256);
     const bool rows_some = foldable && !lanes_at_once && n_steps <= kRowsSomeEnvsSteps && (rows_small || n_steps >= kRowsLargeMapMinSteps) &&
-                           (e->N > kRowsSomeEnvs ? e->N <= kRowsManyLargerTables : (long)e->N > kLaneRoundsManyEnvs && e->K >= 640);
-    const bool rows_first = rows_can && e->fused_variant == 0 && ((rows_many && n_steps <= rows_steps) || rows_some);
+                           (e->N > kRowsSomeEnvs ? e->N <= kRowsManyLargerTables && (!rows_rich || e->A == 8 || e->K >= 512 || e->N > kRowsSomeEnvsRich)
+                                                 : (long)e->N > kLaneRoundsManyEnvs && e->K >= 640);
+    const bool rows_floored = c.max_mode != CRL_MAX_TRUE && !lanes_at_once && (long)e->N > kLaneRoundsManyEnvs &&
+                              e->K >= (e->N > kRowsSomeEnvs ? 257 : 640);
+    const bool rows_first = rows_can && e->fused_variant == 0 && (((rows_many || rows_floored) && n_steps <= rows_steps) || rows_some);
     // ... hybrid workgroups (automatic) when the tables outgrow the caches: while they all fit, other plans are
     // faster (16x16 maps, 30,000 envs: 3.5e10 hybrid, 5.9e10 with lane waves); and where lane
     // waves could step what is left to the general loop, they are faster too (262,144 envs of
@@ -832,7 +841,7 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       if (rows_first || (!p.lanes && rows_can && foldable &&
                          (rows_small || (n_steps >= kRowsLargeMapMinSteps && n_steps <= kRowsLargeMapMaxSteps)))) {
         p.fast = p.fixed = true;
-        p.rich = c.eps_mode != CRL_EPS_FIXED || c.reward_flags != 0;
+        p.rich = rows_rich;
         const size_t staged4 = map_lds + crl::RowCache<4, false, 4>::kBytes, staged6 = map_lds + crl::RowCache<4, false, 6>::kBytes;
         const long fit6 = lds_fit(staged6);
         if (!p.rich && (fit6 >= kRowsSixSoonWaves ? n_steps >= kRowsSixSoonSteps : fit6 >= kRowsSixWaves && n_steps >= kRowsSixSteps)) {

@@ -34,6 +34,7 @@ def test_short_calls(gpu, oracle, N, W, H, A, kw):
     (262147, 7, 2, 4, 47, dict(max_mode=1)), (262147, 3, 3, 8, 150, dict(max_mode=1, **LINEAR)),
     (262147, 6, 5, 4, 80, dict(cells=3, episode_len=3)), (262147, 3, 6, 8, 50, dict(cells=1, max_mode=1)),
     (98305, 5, 4, 4, 88, dict()), (200000, 3, 3, 8, 50, dict()), (200001, 9, 8, 4, 90, dict()), (82500, 13, 13, 4, 40, dict(episode_len=30)),
+    (131073, 5, 5, 4, 60, LINEAR), (98309, 9, 8, 4, 140, dict(max_mode=1)), (82501, 13, 13, 4, 101, dict(max_mode=1, **LINEAR)),
     (262147, 5, 5, 4, 40, dict(LINEAR, episode_len=1)), (262149, 4, 5, 4, 60, dict(episode_len=5)), (262149, 3, 7, 8, 110, dict(episode_len=40)),
 ])
 def test_many_envs(gpu, oracle, N, W, H, A, steps, kw):
