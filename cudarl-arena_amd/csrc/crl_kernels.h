@@ -1728,7 +1728,7 @@ __global__ __launch_bounds__(256) void k_select(const Rules R, const Ptrs P, con
     }
     const int a = (d.u < eps_of(R, P.eps_tab, t, episode)) ? d.a : greedy;
     act_out[env] = a;
-    if (host_out) host_out[env] = a;
+    if (host_out) store_host(host_out + env, a);
   }
   signal_host(sig);
 }
@@ -1744,12 +1744,12 @@ struct StateMirror {
   uint8_t* action;
   __device__ __forceinline__ void put(int env, int s_, int ep_step_, int episode_, float reward_, int done_, int action_) const {
     if (!s) return;
-    s[env] = s_;
-    ep_step[env] = ep_step_;
-    episode[env] = episode_;
-    reward[env] = reward_;
-    done[env] = (uint8_t)done_;
-    action[env] = (uint8_t)action_;
+    store_host(s + env, s_);
+    store_host(ep_step + env, ep_step_);
+    store_host(episode + env, episode_);
+    store_host(reward + env, reward_);
+    store_host(done + env, (uint8_t)done_);
+    store_host(action + env, (uint8_t)action_);
   }
 };
 
@@ -1759,8 +1759,7 @@ struct StateMirror {
 // (act null): one trip over the link less in a call of 6 us.
 // The new state also goes to `mirror` (may be null).
 __device__ __forceinline__ void step_env(const Rules& R, const Ptrs& P, const Transition& T,
-                                         const int32_t* __restrict__ act, const int act0,
-                                         const StateMirror& M, const int env) {
+                                         const int a, const StateMirror& M, const int env) {
   const uint32_t* gmap = P.map + (P.map_shared ? 0 : (size_t)env * P.map_words);
   auto cls = [&](int cell) -> int { return cell_class_of(gmap[cell >> 4], cell); };
   const float* cr = P.cell_reward ? P.cell_reward + (P.map_shared ? 0 : (size_t)env * P.S) : nullptr;
@@ -1768,7 +1767,6 @@ __device__ __forceinline__ void step_env(const Rules& R, const Ptrs& P, const Tr
   const int s0 = P.s[env], start = P.start[env], ep_step0 = P.ep_step[env];
   int episode = P.episode[env];
   const bool done0 = P.done[env] != 0;
-  const int a = act ? act[env] : act0;
   if (R.max_episodes > 0 && episode >= R.max_episodes) {
     T.s[env] = s0;  // budget used up: no move and, with action -1, no update
     T.a[env] = -1;
@@ -1818,18 +1816,26 @@ __global__ __launch_bounds__(256) void k_step(const Rules R, const Ptrs P, const
                                                const int32_t* __restrict__ act, const int act0,
                                                const StateMirror M, const HostSignal sig) {
   const int env = blockIdx.x * blockDim.x + threadIdx.x;
-  if (env < P.N) step_env(R, P, T, act, act0, M, env);
-  signal_host(sig);
+  int a = act0;
+  if (act && env < P.N) a = act[env];
+  const bool kept = M.s != nullptr;
+  if (!kept && sig.flag) {
+    asm volatile("" : "+v"(a));  // arrived
+    signal_read(sig);
+  }
+  if (env < P.N) step_env(R, P, T, a, M, env);
+  if (kept) signal_host(sig);
 }
 
-// n16 16-byte words from device memory to pinned host memory, and one word on its own
+// n16 16-byte words (at most 2 GB) from device memory to pinned host memory, and one word on its own
 // (may be null)
 __global__ __launch_bounds__(256) void k_export(const uint4* __restrict__ src, uint4* __restrict__ dst,
                                                  const size_t n16, const unsigned* __restrict__ word,
                                                  unsigned* __restrict__ word_out, const HostSignal sig) {
   const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride) dst[i] = src[i];
-  if (word && blockIdx.x == 0 && threadIdx.x == 0) *word_out = *word;
+  const DevWindow to = dev_window(dst);
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride) store_host128(to, (uint32_t)i * 16u, src[i]);
+  if (word && blockIdx.x == 0 && threadIdx.x == 0) store_host(word_out, *word);
   signal_host(sig);
 }
 

@@ -157,6 +157,15 @@ __device__ __forceinline__ void st_dev128(DevWindow w, uint32_t byte_offset, con
   t.w = v.w;
   __builtin_amdgcn_raw_buffer_store_b128(t, w, (int)byte_offset, 0, 16 /* sc1 */);
 }
+// store_host() for 16 bytes
+__device__ __forceinline__ void store_host128(DevWindow w, uint32_t byte_offset, const uint4 v) {
+  crl_u4 t;
+  t.x = v.x;
+  t.y = v.y;
+  t.z = v.z;
+  t.w = v.w;
+  __builtin_amdgcn_raw_buffer_store_b128(t, w, (int)byte_offset, 0, 17 /* sc0 sc1 */);
+}
 __device__ __forceinline__ void poll_fence() { asm volatile("" ::: "memory"); }
 
 // `Entries` = entries of the table in which the leader of a key is found: one per key of
@@ -791,7 +800,7 @@ __global__ __launch_bounds__(kBlockSamples* NB) void k_td_small(const Samples X,
       out = make_int2(k, __float_as_int(q));
     }
   }
-  if (changed && tid < n) changed[tid] = out;
+  if (changed && tid < n) store_host(reinterpret_cast<unsigned long long*>(changed) + tid, (unsigned long long)(uint32_t)out.x | (unsigned long long)(uint32_t)out.y << 32);
   signal_host(sig);
 }
 
