@@ -1360,7 +1360,7 @@ PersistPlan plan_persist(const crl_engine* e, int n_steps) {
   p.fold = c.goal_mode == CRL_GOAL_ON_TARGET && c.auto_reset == 1 && c.max_mode == CRL_MAX_TRUE && c.reward_flags == 0 &&
            e->trace_n == 0 && e->sup_n == 0 && c.max_episodes == 0 && c.track_returns == 0;
   const size_t map_bytes = (size_t)e->map_words * 4;
-  const size_t lds = p.hashed ? sizeof(crl::PersistLdsHashed) : sizeof(crl::PersistLds);
+  const size_t lds = p.hashed ? sizeof(crl::PersistLdsHashed) : e->A == 8 ? sizeof(crl::PersistLds<8>) : sizeof(crl::PersistLds<4>);
   p.lds_map = e->cfg.map_mode == CRL_MAP_SHARED && lds + map_bytes <= kLdsPerWorkgroup - kStaticLdsReserve;
   p.lds = lds + (p.lds_map ? map_bytes : 0);
   if (e->no_alloc && p.words * sizeof(unsigned long long) > kScratchExchangeBytes) return p;

@@ -69,10 +69,11 @@ constexpr uint32_t kPersistMaxTag = (1u << 17) - 1u, kPersistMaxTagHashed = (1u 
 constexpr int kPersistClockWords = 20 + 8 * 256;  // 2 workgroups x (8 phases + polls of the two waits by thread 0),
                                                   // then the wall clock of every workgroup at the 8 marks of one step
 
-// Dense form, up to 16,384 keys: an entry per key of the table in the block pass, a dense
+// Dense form, up to 16,384 keys: an entry per cell of the table in the block pass, a dense
 // [block][key] tile in the owner's.
+template <int A>
 struct alignas(16) PersistLds {
-  ReduceLds red;
+  CellReduceLds<A> red;
   alignas(16) float tile[kTileBlocks * kOwnKeys];       // the owner's [block][key] block sums: a quarter (64 blocks) to a wave, which
                                                         // clears, fills and adds up its quarter without waiting for the others
   alignas(16) unsigned long long stage[kPersistMaxGroups << kMainShift];  // the main halves of the block's cells on their way out
@@ -102,8 +103,8 @@ struct alignas(16) PersistLdsHashed {
   int o_count;
   int dead;
 };
-template <bool HASHED>
-using PersistLdsOf = std::conditional_t<HASHED, PersistLdsHashed, PersistLds>;
+template <int A, bool HASHED>
+using PersistLdsOf = std::conditional_t<HASHED, PersistLdsHashed, PersistLds<A>>;
 
 struct PersistBufs {
   unsigned long long* table;   // view [S][2 A]
@@ -333,11 +334,11 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
                                                          const int trace_row0, const int n_keys, const PersistBufs B,
                                                          const int spin_limit) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  using Lds = PersistLdsOf<HASHED>;
+  using Lds = PersistLdsOf<A, HASHED>;
   using R64 = Rec<HASHED>;
   Lds& L = *reinterpret_cast<Lds*>(lds_raw);
   static_assert(sizeof(Lds) % 16 == 0, "16-byte LDS accesses");
-  static_assert(kSortBytes <= sizeof(PersistLds::tile) / 2, "the holders' line-up borrows the upper half of the tile");
+  static_assert(kSortBytes <= sizeof(PersistLds<A>::tile) / 2, "the holders' line-up borrows the upper half of the tile");
   uint32_t* lds_map = reinterpret_cast<uint32_t*>(lds_raw + sizeof(Lds));
   // (shifts that are known here are no scalar registers to run out of)
   constexpr int kAShift = A == 8 ? 3 : 2;
@@ -440,6 +441,10 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
   };
   if (owns) publish(tag0 + 1u);
   __syncthreads();
+  if constexpr (!HASHED) {  // (of the first step; reduce_block() finds those that follow)
+    if (has_env) atomicMin(&L.red.lead[s], (uint32_t)tid);
+    __syncthreads();
+  }
 
   // What a step needs that does not depend on the table: computed at the top of the step,
   // while the values of the step before are on their way from the owners.
@@ -494,6 +499,8 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
     // (the values this workgroup published as an owner are on their way meanwhile)
     prepare(k);
     reduce_stage_init<HASHED>(L.stage, G, want);
+    int lead = 0;
+    if constexpr (!HASHED) lead = has_env ? (int)L.red.lead[s0] * A : 0;
     // (The values published at the end of the last step need about 1 us to be visible, which
     // is what the preparation above takes.  A look that comes too early costs a whole round
     // trip more; while a step was longer than now, a pause of 0.1-0.2 us here and before the
@@ -548,15 +555,15 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
       const Row<A> row = row_of_tagged<A>(rq);
       const int greedy = row_argmax(row);  // (worked out for every env: cheaper than a branch around it)
       const int a = (d.u < eps) ? d.a : greedy;
-      // (the key is known: its leader is being found while the delta is worked out)
+      // (the key is known: its holders enter themselves, or its leader is being found, while the delta is worked out)
       my_key = s0 * A + a;
       int found = -1;
       if constexpr (HASHED) {
         my_at = hash_start(kHashSlots - 1, my_key);
         found = atomicCAS(&L.keys[my_at], -1, my_key);
       } else {
-        my_at = my_key;
-        atomicMin(&L.red.lead[my_at], (uint32_t)tid);
+        my_at = lead + a;
+        atomicOr(&L.red.members[my_at][wave], 1ull << lane);
       }
       // the rule of step_rule() on the move code of the action: the class of the target
       // cell, or kWall outside the grid
@@ -609,7 +616,7 @@ __global__ __launch_bounds__(256) void k_shared_persist(const Rules R, const Ptr
     // (`sorted`: the upper half of the tile, which is free until the block sums are through)
     int* keys = nullptr;
     if constexpr (HASHED) keys = L.keys;
-    const bool over = reduce_block<HASHED>(L.red, G, wg, my_key, my_at, keys, my_delta, live, want,
+    const bool over = reduce_block<HASHED>(L.red, G, wg, my_key, has_env ? s0 : -1, s, my_at, keys, my_delta, live, want,
                                            L.tile + kTileBlocks * kOwnKeys / 2, L.stage, w_cells, (uint32_t)((size_t)half * cells_half * 8), B.cells + (2 + half) * cells_half);
     if (over && has_env)
       st_dev64(B.raw + (size_t)half * P.N + env, tagged(__float_as_uint(my_delta),

@@ -179,7 +179,20 @@ struct alignas(16) ReduceLdsT {  // (lead and members are also accessed 16 bytes
   int over;                                      // some owner was handed more than a cell holds
   int none;                                      // (written by the others; nobody reads it)
 };
-using ReduceLds = ReduceLdsT<kDenseKeys>;
+
+// The same where each key of the table has its place: a cell's lowest thread is found before the actions are
+// chosen, while the step before is under way (cell_sums), and the holders of its A keys have a set each, by
+// that thread's number.
+template <int A>
+struct alignas(16) CellReduceLds {
+  static constexpr int kCells = kDenseKeys / A;
+  alignas(16) uint32_t lead[kCells];                             // lowest thread of the block in the cell; kNoLead between uses
+  alignas(16) unsigned long long members[kBlockSamples * A][4];  // [lead][action]; zero between uses
+  float delta[kBlockSamples];
+  int handed[256];
+  int over;
+  int none;
+};
 
 // Besides ReduceLds, reduce_block() needs kSortBytes of LDS for `sorted`: the deltas of a
 // key's further holders, lined up for its leader ([place among the holders][leader]).
@@ -199,12 +212,41 @@ __device__ __forceinline__ void reduce_block_init(ReduceLdsT<Entries>& L) {
   if (tid == 0) L.over = 0;
 }
 
+// acc and the deltas of a leader's further holders (those in mw), in thread order = sample order
+__device__ __forceinline__ float add_holders(const float* delta, const float* sorted, const unsigned long long (&mw)[4], const int holders,
+                                             float acc) {
+  const int tid = threadIdx.x;
+  const int lined = holders < kSortRows ? holders : kSortRows;
+  for (int r0 = 0; r0 < lined; r0 += 4) {
+    float d[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = sorted[(r0 + i < kSortRows ? r0 + i : kSortRows - 1) * kBlockSamples + tid];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (r0 + i < lined) acc = acc + d[i];
+  }
+  if (holders > kSortRows) {  // more holders than places: the rest one by one
+    int seen = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      unsigned long long m = mw[w];
+      while (m != 0ull) {
+        const int j = __builtin_ctzll(m);
+        if (seen >= kSortRows) acc = acc + delta[w * 64 + j];
+        ++seen;
+        m &= m - 1ull;
+      }
+    }
+  }
+  return acc;
+}
+
 // What both forms of pass 1 share: the ordered sum of each distinct key of a block, in its
 // leader.  All 256 threads call it with their sample (valid = false: none); `at` is the
 // key's entry of L.lead, where the caller has entered its thread with an atomic min.  On
 // return (behind a barrier that only the last lines of the function follow) *sum is the
-// leader's block sum, and L.lead and L.members are as reduce_block_init() left them, so it
-// can be called again and again.  -> whether this thread is a leader.
+// leader's block sum.  L.lead[at] and the leader's member set are as they were used: who calls
+// it again clears them first, when nobody waits for it.  -> whether this thread is a leader.
 // (Written without branches: one wave to a SIMD has nothing to hide them behind.  A thread
 // without a sample reads its own, empty member set; a thread that has nothing to line up
 // writes its delta where it already is.)
@@ -249,33 +291,67 @@ __device__ __forceinline__ bool block_sums(ReduceLdsT<Entries>& L, const int at,
   float acc = 0.0f;
   if (leader) {
     acc = acc + delta;  // the leader is the key's first sample; the other holders come after it
+    if (holders != 0) acc = add_holders(L.delta, sorted, mw, holders, acc);
+  }
+  *sum = acc;
+  return leader;
+}
+
+template <int A>
+__device__ __forceinline__ void reduce_block_init(CellReduceLds<A>& L) {
+  const int tid = threadIdx.x;
+  uint4* lead4 = reinterpret_cast<uint4*>(L.lead);
+  for (int i = tid; i < CellReduceLds<A>::kCells / 4; i += kBlockSamples) lead4[i] = make_uint4(kNoLead, kNoLead, kNoLead, kNoLead);
+  for (int i = tid; i < kBlockSamples * A; i += kBlockSamples) {
+    *reinterpret_cast<ulonglong2*>(&L.members[i][0]) = make_ulonglong2(0ull, 0ull);
+    *reinterpret_cast<ulonglong2*>(&L.members[i][2]) = make_ulonglong2(0ull, 0ull);
+  }
+  if (tid == 0) L.over = 0;
+}
+
+// block_sums() where the threads of a cell know the lowest of them: all of a key's holders have entered themselves in
+// `set` = lead * A + action, and a barrier later each of them sees its place, the first of them that it leads - one
+// barrier and two trips to LDS fewer than finding the key's lowest thread first.  What makes it pay is that nothing else is done between
+// the barriers: 65,536 envs, 200 steps, 64x64x4 / 32x32x4 1357 / 1267 us with keys' leaders, 1345 / 1242 with the next leads
+// found and the sets cleared between the second barrier and the third, 1324 / 1228 behind the third; found in the same step,
+// behind a barrier of their own, 1416 / 1316.
+template <int A, class Between>
+__device__ __forceinline__ bool cell_sums(CellReduceLds<A>& L, const int cell, const int set, const float delta, const bool valid, float* sorted,
+                                          Between between, float* sum) {
+  const int tid = threadIdx.x, w = tid >> 6;
+  L.delta[tid] = delta;
+  __syncthreads();
+  between();
+  unsigned long long mw[4];
+  {
+    const ulonglong2 lo = *reinterpret_cast<const ulonglong2*>(&L.members[set][0]);
+    const ulonglong2 hi = *reinterpret_cast<const ulonglong2*>(&L.members[set][2]);
+    mw[0] = lo.x;
+    mw[1] = lo.y;
+    mw[2] = hi.x;
+    mw[3] = hi.y;
+  }
+  const int p0 = __popcll(mw[0]), p1 = __popcll(mw[1]), p2 = __popcll(mw[2]), p3 = __popcll(mw[3]);
+  const unsigned long long mine = w == 0 ? mw[0] : w == 1 ? mw[1] : w == 2 ? mw[2] : mw[3];
+  const int place = (w > 0 ? p0 : 0) + (w > 1 ? p1 : 0) + (w > 2 ? p2 : 0) + __popcll(mine & ((1ull << (tid & 63)) - 1ull));
+  const bool leader = valid && place == 0;
+  const int holders = leader ? p0 + p1 + p2 + p3 - 1 : 0;  // the key's further holders
+  {
+    const unsigned long long first = mw[0] != 0ull ? mw[0] : mw[1] != 0ull ? mw[1] : mw[2] != 0ull ? mw[2] : mw[3];
+    const int ld = (mw[0] != 0ull ? 0 : mw[1] != 0ull ? 64 : mw[2] != 0ull ? 128 : 192) + __builtin_ctzll(first | (1ull << 63));
+    const bool lines_up = valid && place > 0 && place <= kSortRows;
+    *(lines_up ? &sorted[(place - 1) * kBlockSamples + ld] : &L.delta[tid]) = delta;
+  }
+  if (cell >= 0) L.lead[cell] = kNoLead;  // (read before the barrier above)
+  __syncthreads();
+  float acc = 0.0f;
+  if (leader) {
+    acc = acc + delta;
     if (holders != 0) {
-      *reinterpret_cast<ulonglong2*>(&L.members[tid][0]) = make_ulonglong2(0ull, 0ull);
-      *reinterpret_cast<ulonglong2*>(&L.members[tid][2]) = make_ulonglong2(0ull, 0ull);
-      const int lined = holders < kSortRows ? holders : kSortRows;
-      for (int r0 = 0; r0 < lined; r0 += 4) {
-        float d[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) d[i] = sorted[(r0 + i < kSortRows ? r0 + i : kSortRows - 1) * kBlockSamples + tid];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (r0 + i < lined) acc = acc + d[i];  // thread order = sample order
-      }
-      if (holders > kSortRows) {  // more holders than places: the rest one by one
-        int seen = 0;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          unsigned long long m = mw[w];
-          while (m != 0ull) {
-            const int j = __builtin_ctzll(m);
-            if (seen >= kSortRows) acc = acc + L.delta[w * 64 + j];
-            ++seen;
-            m &= m - 1ull;
-          }
-        }
-      }
+      for (int i = 0; i < 4; ++i) mw[i] &= w == i ? ~(1ull << (tid & 63)) : ~0ull;
+      acc = add_holders(L.delta, sorted, mw, holders, acc);
     }
-    L.lead[at] = kNoLead;
   }
   *sum = acc;
   return leader;
@@ -293,9 +369,9 @@ __device__ __forceinline__ void reduce_stage_init(unsigned long long* stage, con
 }
 
 // One-launch kernel: pass 1 for one block.  All 256 threads of the workgroup call it with
-// their sample (valid = false: no sample / no delta), having entered their thread number in
-// L.lead[at] with an atomic min: `at` is the key itself, or (hashed form) its entry in `keys`,
-// which is cleared again.  The main halves of all cells of the
+// their sample (valid = false: no sample / no delta).  Hashed form: having entered their thread number in
+// L.lead[at] with an atomic min, `at` the key's entry in `keys`, which is cleared again.  Dense form: in the set
+// at = (lead of the cell) * A + action; cell and next_cell: where the env stands now and next, -1 without one.  The main halves of all cells of the
 // block are put together in LDS (`stage`, owners << main_shift records, free again
 // on return) and go out as whole lines (that of (block, owner) at (block * owners + owner)
 // << main_shift behind `window_offset`), 16 bytes to a store and lane, every record
@@ -306,9 +382,9 @@ __device__ __forceinline__ void reduce_stage_init(unsigned long long* stage, con
 // Returns (to every thread) whether some owner was handed more distinct keys than a
 // cell has records: its cell then says kSlotOverflow and the owner needs the block's
 // raw samples.
-template <bool HASHED, int Entries>
-__device__ __forceinline__ bool reduce_block(ReduceLdsT<Entries>& L, const ReduceGeom G, const int block,
-                                             const int key, const int at, int* keys, const float delta,
+template <bool HASHED, class Lds>
+__device__ __forceinline__ bool reduce_block(Lds& L, const ReduceGeom G, const int block, const int key, const int cell, const int next_cell,
+                                             const int at, int* keys, const float delta,
                                              const bool valid, const uint32_t tag, float* sorted,
                                              unsigned long long* stage, const DevWindow window,
                                              const uint32_t window_offset, unsigned long long* ext) {
@@ -317,16 +393,18 @@ __device__ __forceinline__ bool reduce_block(ReduceLdsT<Entries>& L, const Reduc
   const int cap = 1 << G.cell_shift;  // records of a cell
   const int cap_main = 1 << G.main_shift;  // of its main half
   float acc;
-  const bool leader = block_sums(L, at, delta, valid, sorted, [&] {
+  auto clear = [&] {
     L.handed[tid] = 0;  // (256 owners)
     if (tid == 0) L.over = 0;
-  }, &acc);
+  };
+  bool leader;
+  if constexpr (HASHED) leader = block_sums(L, at, delta, valid, sorted, clear, &acc);
+  else leader = cell_sums(L, cell, at, delta, valid, sorted, clear, &acc);
   int slot = 0, owner = 0;
   if (leader) {
     owner = owner_of(key, G);
     slot = atomicAdd(&L.handed[owner], 1);  // slot order is free: records carry the key
     *(slot >= cap ? &L.over : &L.none) = 1;
-    if (HASHED) keys[at] = -1;
     // (record 0's count is added on the way out, when every leader has drawn its slot)
     if (slot < cap_main) stage[(owner << G.main_shift) + slot] = Rec<HASHED>::make((uint32_t)slot_of(key, G), tag, acc);
   }
@@ -359,6 +437,21 @@ __device__ __forceinline__ bool reduce_block(ReduceLdsT<Entries>& L, const Reduc
     if (i < pieces)
       st_dev128(window, window_offset + (uint32_t)((((size_t)block * n_own) << (G.main_shift + 3)) + (size_t)i * 16),
                 make_uint4((uint32_t)v[j].x, (uint32_t)(v[j].x >> 32), (uint32_t)v[j].y, (uint32_t)(v[j].y >> 32)));
+  }
+  // For the next call, while the cells travel (the caller has a barrier before that): nobody waits for it here, where
+  // between the barriers above it is in the way of the sums (hashed: 20,000 envs on 101x99x8, 50 steps 440 us there, 437 here).
+  if (leader) {
+    unsigned long long* set = L.members[HASHED ? tid : at];
+    *reinterpret_cast<ulonglong2*>(set) = make_ulonglong2(0ull, 0ull);
+    *reinterpret_cast<ulonglong2*>(set + 2) = make_ulonglong2(0ull, 0ull);
+  }
+  if constexpr (HASHED) {
+    if (leader) {
+      L.lead[at] = kNoLead;
+      keys[at] = -1;
+    }
+  } else if (cell >= 0) {
+    atomicMin(&L.lead[next_cell], (uint32_t)tid);
   }
   return over;
 }
