@@ -2621,14 +2621,30 @@ int crl_fused_kernel_info(crl_engine* e, int32_t n_steps, char* name, size_t nam
   return CRL_OK;
 }
 
-int crl_fused_plan_for_config(const crl_config* cfg, int32_t n_steps, char* name, size_t name_len,
-                              int32_t* grid, int32_t* block, int32_t* lds_bytes) {
+static int plan_for_config(const crl_config* cfg, int32_t n_steps, FusedPlan* p) {
   int rc = crl::validate_config(cfg, crl::last_error());
   if (rc != CRL_OK) return rc;
   if (cfg->table_mode != CRL_TABLE_PER_ENV) return fail(CRL_E_ARG, "only per-env tables have a fused launch plan");
   crl_engine shell;  // sizes only: nothing is allocated and no device is touched
   set_geometry(&shell, *cfg);
-  const FusedPlan p = plan_fused(&shell, n_steps > 0 ? n_steps : 1 << 20);
+  *p = plan_fused(&shell, n_steps > 0 ? n_steps : 1 << 20);
+  return CRL_OK;
+}
+
+int crl_fused_plan_rows_for_config(const crl_config* cfg, int32_t n_steps, int32_t* rows, int32_t* codes) {
+  FusedPlan p;
+  int rc = plan_for_config(cfg, n_steps, &p);
+  if (rc != CRL_OK) return rc;
+  if (rows) *rows = p.rows;
+  if (codes) *codes = p.moves ? 1 : 0;
+  return CRL_OK;
+}
+
+int crl_fused_plan_for_config(const crl_config* cfg, int32_t n_steps, char* name, size_t name_len,
+                              int32_t* grid, int32_t* block, int32_t* lds_bytes) {
+  FusedPlan p;
+  int rc = plan_for_config(cfg, n_steps, &p);
+  if (rc != CRL_OK) return rc;
   if (name && name_len) snprintf(name, name_len, "%s", p.name);
   if (grid) *grid = p.grid;
   if (block) *block = p.block;

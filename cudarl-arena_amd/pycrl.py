@@ -89,7 +89,7 @@ EXPORTS = [
     "crl_step", "crl_select", "crl_update", "crl_td_update", "crl_td_update_collect", "crl_run_fused", "crl_run_fused_noalloc", "crl_get_state",
     "crl_set_state", "crl_get_episode_stats", "crl_get_step_count", "crl_set_step_count", "crl_q_get", "crl_q_set",
     "crl_q_get_range", "crl_set_trace", "crl_get_trace", "crl_set_exploration_stream", "crl_set_persist_spin_limit",
-    "crl_device_ptr", "crl_fused_kernel_info", "crl_fused_plan_for_config", "crl_philox4x32_10", "crl_explore_draw",
+    "crl_device_ptr", "crl_fused_kernel_info", "crl_fused_plan_for_config", "crl_fused_plan_rows_for_config", "crl_philox4x32_10", "crl_explore_draw",
     "crl_eps_table", "crl_gen_maps_bernoulli", "crl_gen_maps_noise", "crl_probe_copy", "crl_probe_barrier", "crl_get_persist_clocks", "crl_set_persist_clocks",
 ]
 
@@ -141,6 +141,7 @@ def load():
                                           C.POINTER(i32)]
     lib.crl_fused_plan_for_config.argtypes = [C.POINTER(Config), i32, C.c_char_p, C.c_size_t, C.POINTER(i32),
                                               C.POINTER(i32), C.POINTER(i32)]
+    lib.crl_fused_plan_rows_for_config.argtypes = [C.POINTER(Config), i32, C.POINTER(i32), C.POINTER(i32)]
     lib.crl_philox4x32_10.argtypes = [vp, vp, vp]
     lib.crl_philox4x32_10.restype = None
     lib.crl_explore_draw.argtypes = [u64, C.c_uint32, u64, i32, C.POINTER(f32), C.POINTER(i32)]
@@ -202,6 +203,14 @@ def fused_plan_for_config(cfg, n_steps=0):
     g, b, l = C.c_int32(), C.c_int32(), C.c_int32()
     _check(load().crl_fused_plan_for_config(C.byref(cfg), n_steps, name, 128, C.byref(g), C.byref(b), C.byref(l)))
     return dict(name=name.value.decode(), grid=g.value, block=b.value, lds_bytes=l.value)
+
+
+def fused_plan_rows(cfg, n_steps=0):
+    """(rows, codes) of that plan: places that a 64-env wave has in LDS for each env's table rows
+    (0: it keeps none), and whether its waves read move codes or class maps."""
+    rows, codes = C.c_int32(), C.c_int32()
+    _check(load().crl_fused_plan_rows_for_config(C.byref(cfg), n_steps, C.byref(rows), C.byref(codes)))
+    return rows.value, codes.value
 
 
 def probe_barrier(pattern, n_groups=256, rounds=2000):

@@ -305,6 +305,11 @@ int crl_fused_kernel_info(crl_engine* e, int32_t n_steps, char* name, size_t nam
 int crl_fused_plan_for_config(const crl_config* cfg, int32_t n_steps, char* name, size_t name_len,
                               int32_t* grid, int32_t* block, int32_t* lds_bytes);
 
+/* What that plan keeps in LDS, where kernels of one name differ in it: rows = the places
+ * a 64-env wave has for each env's table rows (0: it keeps none), codes = 1 if its waves
+ * read move codes (staged, or coming with the rows), 0 if they read staged class maps. */
+int crl_fused_plan_rows_for_config(const crl_config* cfg, int32_t n_steps, int32_t* rows, int32_t* codes);
+
 /* -- diagnostics (no reference counterpart; not part of the drop-in surface) -- */
 
 /* One launch of a plain copy kernel `k_probe_copy` moving n_bytes from one device

@@ -66,7 +66,8 @@ def test_hybrid_workgroups(gpu, oracle, N, W, H, A, lds_waves):
 
 
 # waves of 64 envs, which short calls of more envs than lane waves are for take, and longer calls on
-# tables past the caches, then with their move codes staged; the general loop's hybrid workgroups
+# tables past the caches (most of these keep rows in LDS: those that keep none are below); the general
+# loop's hybrid workgroups
 LINEAR = dict(eps_mode=3, eps0=0.9, eps_end=0.1, eps_span=4)
 
 
@@ -84,3 +85,15 @@ LINEAR = dict(eps_mode=3, eps0=0.9, eps_end=0.1, eps_span=4)
 ])
 def test_waves_of_64_envs(gpu, oracle, N, W, H, A, chunks, variant, kernel, kw):
     check(gpu, oracle, N, W, H, A, chunks, variant=variant, hybrid="hbm+lds" in kernel, kernel=kernel, **kw)
+
+
+# those that keep no rows in LDS: class maps staged, move codes staged (from 128 steps on)
+@pytest.mark.parametrize("N,W,H,A,steps,codes,kw", [
+    (17003, 31, 33, 4, 7, 0, dict()), (34001, 20, 20, 4, 5, 0, LINEAR), (34001, 20, 20, 8, 5, 0, dict()), (17003, 31, 33, 8, 7, 0, dict(cells=3)),
+    (48001, 29, 29, 4, 131, 1, dict()), (48001, 29, 29, 4, 131, 1, LINEAR), (30001, 24, 24, 8, 131, 1, dict()), (30001, 24, 24, 8, 131, 1, dict(cells=1)),
+])
+def test_waves_of_64_envs_without_rows(gpu, oracle, N, W, H, A, steps, codes, kw):
+    kernel = "k_fused_tickets<%d,fast%s,hbm>" % (A, "+" if kw else "")
+    check(gpu, oracle, N, W, H, A, (steps, 1), kernel=kernel, **kw)
+    cfg = gpu.make_config(N, W, H, n_actions=A, reward_flags=kw.get("cells", 0), eps_mode=kw.get("eps_mode", 0), eps_span=9)
+    assert gpu.fused_plan_rows(cfg, steps) == (0, codes) and gpu.fused_plan_rows(cfg, 1)[0] == 0

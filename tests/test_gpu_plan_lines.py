@@ -1,6 +1,6 @@
 """Both sides of the lines where a fused launch changes its kernel: tables in LDS or behind lane
 waves, lane waves in rounds dealt or drawn, hybrid workgroups or rounds of lane waves, waves of 64
-envs with and without staged move codes.  Against the oracle bit for bit."""
+envs that keep rows in LDS or none.  Against the oracle bit for bit."""
 import numpy as np
 import pytest
 
@@ -9,6 +9,7 @@ from test_gpu_lane_waves import STATE, check
 pytestmark = pytest.mark.gpu
 
 LDS, LANES, PLAIN, HYBRID = "k_fused_tickets_lds<%d,fast>", "k_fused_lanes<%d,fast>", "k_fused_tickets<%d,fast,hbm>", "k_fused_tickets<%d,fast,hbm+lds>"
+ROWS = PLAIN + ", rows kept"  # which go by the name of the plain ones
 
 
 @pytest.mark.parametrize("N,W,H,A,steps,kernel", [
@@ -16,13 +17,13 @@ LDS, LANES, PLAIN, HYBRID = "k_fused_tickets_lds<%d,fast>", "k_fused_lanes<%d,fa
     (4090, 16, 16, 4, 39, LANES), (4090, 16, 16, 4, 40, LDS),        # 16 KB to a wave
     (15001, 8, 8, 4, 40, LDS), (30001, 8, 8, 4, 117, LANES), (30001, 8, 8, 4, 119, LDS),  # four and eight such waves
     (70, 47, 49, 8, 143, LANES), (70, 47, 49, 8, 144, LDS),          # 72 KB to a wave
-    (33001, 32, 32, 4, 130, PLAIN),                                  # codes staged: fewer waves at once
-    (50001, 32, 32, 4, 63, PLAIN), (50001, 32, 32, 4, 64, LANES),    # rounds, of at most 65,536 envs
-    (66001, 28, 28, 4, 130, PLAIN), (66001, 28, 28, 4, 131, LANES),  # of more
-    (250001, 8, 8, 4, 9, PLAIN), (250001, 8, 8, 4, 10, LANES),       # in place of hybrid workgroups
+    (33001, 32, 32, 4, 130, ROWS), (33001, 32, 32, 4, 131, PLAIN),   # large maps
+    (50001, 32, 32, 4, 63, ROWS), (50001, 32, 32, 4, 64, LANES),     # rounds, of at most 65,536 envs
+    (66001, 28, 28, 4, 130, ROWS), (66001, 28, 28, 4, 131, LANES),   # of more
+    (250001, 8, 8, 4, 9, ROWS), (250001, 8, 8, 4, 10, LANES),        # in place of hybrid workgroups
     (250001, 8, 8, 4, 71, LANES), (250001, 8, 8, 4, 72, HYBRID),
-    (94001, 12, 12, 4, 47, PLAIN), (94001, 12, 12, 4, 48, LANES),    # ... where they are few rounds
-    (200001, 8, 8, 4, 5, PLAIN), (200001, 8, 8, 4, 6, PLAIN),        # all envs in flight, a limit on them
+    (94001, 12, 12, 4, 47, ROWS), (94001, 12, 12, 4, 48, LANES),     # ... where they are few rounds
+    (200001, 8, 8, 4, 5, ROWS), (200001, 8, 8, 4, 6, ROWS),
 ])
 def test_lines(gpu, oracle, N, W, H, A, steps, kernel):
     cls, start = gpu.gen_maps_bernoulli(7, N, N, W, H, 0.12, 0.08)
@@ -31,7 +32,8 @@ def test_lines(gpu, oracle, N, W, H, A, steps, kernel):
     oracle.run(cfg, cls, None, start, Q, want, 0, steps)
     with gpu.Engine(cfg, 0) as eng:
         eng.set_maps(cls, start)
-        assert eng.fused_kernel_info(steps)["name"] == kernel % A
+        kept = gpu.fused_plan_rows(cfg, steps)[0] != 0
+        assert eng.fused_kernel_info(steps)["name"] + (", rows kept" if kept else "") == kernel % A
         eng.run_fused(steps)
         state = eng.get_state()
         assert all(np.array_equal(state[k], want[k]) for k in STATE)

@@ -18,6 +18,7 @@ def rows_check(gpu, oracle, N, W, H, A, chunks, staged, places=lambda steps: 4, 
         plan = gpu.fused_plan_for_config(cfg, c)
         assert plan["lds_bytes"] == places(c) * (PLACE + 64 * (2 if staged else 4)) + (W * H + 15) // 16 * 256 * staged, plan
         assert (plan["grid"], plan["block"]) == (-(-N // 64), 64), plan
+        assert gpu.fused_plan_rows(cfg, c)[0] == places(c), plan
     rich = kw.get("cells") or "eps_mode" in kw
     check(gpu, oracle, N, W, H, A, chunks, kernel="k_fused_tickets<%d,fast%s,hbm>" % (A, "+" if rich else ""), **kw)
 
