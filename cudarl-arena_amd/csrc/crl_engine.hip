@@ -846,6 +846,7 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
         const long fit6 = lds_fit(staged6);
         if (!p.rich && (fit6 >= kRowsSixSoonWaves ? n_steps >= kRowsSixSoonSteps : fit6 >= kRowsSixWaves && n_steps >= kRowsSixSteps)) {
           p.rows = 6;
+          p.moves = false;
           p.lds = staged6;
         } else {
           p.rows = 4;

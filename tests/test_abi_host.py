@@ -282,6 +282,17 @@ def test_envs_in_flight_of_short_launches(pycrl, N, W, H, A, n_steps, grid):
     assert (plan["name"], plan["grid"]) == ("k_fused_tickets<%d,fast,hbm>" % A, grid)
 
 
+@pytest.mark.parametrize("N,W,H,A,n_steps,rows,codes", [
+    (1 << 20, 16, 16, 4, 20, 4, 0), (1 << 20, 16, 16, 4, 31, 4, 0), (1 << 20, 16, 16, 4, 32, 6, 0),
+    (66001, 28, 28, 4, 99, 4, 0), (66001, 28, 28, 4, 100, 6, 0), (66001, 28, 28, 4, 130, 6, 0),  # (plain waves would have move codes staged)
+    (100000, 32, 32, 4, 130, 4, 1), (1 << 20, 16, 16, 4, 1000, 0, 0),
+])
+def test_rows_that_a_plan_keeps(pycrl, N, W, H, A, n_steps, rows, codes):
+    """64-env waves that keep rows in LDS: four places and six, their maps staged or their move codes coming with the rows."""
+    cfg = pycrl.make_config(N, W, H, n_actions=A, episode_len=128)
+    assert pycrl.fused_plan_rows(cfg, n_steps) == (rows, codes)
+
+
 def test_npy_agent_files_match_numpy(pycrl, tmp_path):
     """QTableAgent.save / load files (src/train.py:150-168): float64 (W, H, A)
     indexed [x, y, a], exchanged with numpy in both directions."""
