@@ -273,8 +273,8 @@ def test_uneven_rounds_of_a_floored_maximum(pycrl, N, W, H, A, name):
 
 @pytest.mark.parametrize("N,W,H,A,n_steps,grid", [
     (105108, 43, 23, 4, 9, 410), (105108, 43, 23, 4, 10, 256),  # three shifts of maps of 900 cells and more
-    (60000, 32, 32, 4, 5, 937), (60000, 32, 32, 4, 6, 512),     # two
-    (57155, 26, 37, 8, 9, 893), (57155, 26, 37, 8, 10, 512),    # two, 8 actions
+    (60000, 32, 32, 4, 5, 938), (60000, 32, 32, 4, 6, 512),     # two
+    (57155, 26, 37, 8, 9, 894), (57155, 26, 37, 8, 10, 512),    # two, 8 actions
     (150000, 20, 20, 4, 5, 585), (150000, 20, 20, 4, 6, 256),   # smaller maps
 ])
 def test_envs_in_flight_of_short_launches(pycrl, N, W, H, A, n_steps, grid):
@@ -291,6 +291,14 @@ def test_rows_that_a_plan_keeps(pycrl, N, W, H, A, n_steps, rows, codes):
     """64-env waves that keep rows in LDS: four places and six, their maps staged or their move codes coming with the rows."""
     cfg = pycrl.make_config(N, W, H, n_actions=A, episode_len=128)
     assert pycrl.fused_plan_rows(cfg, n_steps) == (rows, codes)
+
+
+@pytest.mark.parametrize("N,W,H,A,n_steps", [(19895, 40, 40, 8, 1), (24961, 16, 16, 4, 5), (58545, 20, 20, 8, 2), (16385, 3, 3, 4, 1)])
+def test_all_envs_in_flight_at_once(pycrl, N, W, H, A, n_steps):
+    """A wave for the last, part-filled 64 envs too."""
+    for kw in (dict(), dict(track_returns=1)):
+        plan = pycrl.fused_plan_for_config(pycrl.make_config(N, W, H, n_actions=A, episode_len=128, **kw), n_steps)
+        assert "lanes" in plan["name"] or plan["grid"] * plan["block"] >= N, plan
 
 
 def test_npy_agent_files_match_numpy(pycrl, tmp_path):
