@@ -430,6 +430,9 @@ constexpr size_t kTableBytesAtOnce = (size_t)512 << 20;
 constexpr int kRowsManyEnvs = 1 << 18, kRowsManyLargerTables = 200000, kRowsHybridSteps4 = 48, kRowsHybridSteps8 = 96;
 constexpr int kRowsSomeEnvs = 6 * 64 * kComputeUnits, kRowsSomeEnvsRich = 1 << 17, kRowsSomeEnvsSteps = 88, kRowsLanesSteps = 500;
 constexpr size_t kRowsSmallMap = 336;  // cells: eleven to a unit
+constexpr long kRowsCells4 = 80, kRowsCells4Rich = 60, kRowsCells4Fixed = 40, kRowsCells8 = 96, kRowsCells8Rich = 80, kRowsFixedEnvs = 11L * 16 * kComputeUnits;
+constexpr int kRowsFixedMinSteps = 3;
+constexpr size_t kRowsFixedMap8 = 1300;
 constexpr int kRowsLargeMapMinSteps = 11, kRowsLargeMapMaxSteps = 130;
 constexpr long kRowsStagedWaves4 = 7, kRowsStagedWaves8 = 6, kRowsSixSoonWaves = 9, kRowsSixWaves = 6;
 constexpr int kRowsSixSoonSteps = 32, kRowsSixSteps = 100;
@@ -721,6 +724,30 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
                                                  : (long)e->N > kLaneRoundsManyEnvs && e->K >= 640);
     const bool rows_floored = c.max_mode != CRL_MAX_TRUE && !lanes_at_once && (long)e->N > kLaneRoundsManyEnvs &&
                               e->K >= (e->N > kRowsSomeEnvs ? 257 : 640);
+    const size_t rows_lds4 = map_lds + crl::RowCache<4, false, 4>::kBytes;
+    const bool rows_staged = lds_fit(rows_lds4) >= (e->A == 8 ? kRowsStagedWaves8 : kRowsStagedWaves4);
+    // Up to three of them to a compute unit plain 64-env waves are faster (plain / rows: 40,960 of 8x8, 2 / 5 steps 7.1 / 9.0, 8.2 /
+    // 11.1; 40,000 of 16x16 with 8 actions, 4 steps 12.0, 13.3; 40,960 of 32x32, 128 steps 141, 159; 24,576 of 40x40 with 8 actions 171,
+    // 210; 44,866 of 4x38 with 8 actions, 43 steps 55, 68), and four in calls too short for a limit on the envs in flight (62,848 of
+    // 4x4, 5 steps 9.9, 11.6; 49,984 of 8x8 with 8 actions, 6 steps 14.6, 16.6; 57,984 of 4x4, 3 steps 6.6, 8.0).  Rows are where
+    //   plain waves go in shifts or their maps do not all fit LDS (56,000 envs and more, 16 steps and more 1.2 to 1.6 times as fast;
+    //     35,968 of 64x64, 112 steps 203, 144);
+    //   a map costs more to stage than the steps then save, some cells to a step: with two 64-env waves to a unit 80 (32,768 of 64x64, 20 /
+    //     32 / 50 steps 41.3 / 52.1 / 70.2, 31.9 / 48.0 / 72.5; 30,000 of 48x48, 16 / 32 steps 30.5 / 45.0, 26.7 / 48.6), with three 60 while
+    //     envs explore and 40 with epsilon fixed (40,960 of 32x32, 12 / 16 / 64 steps 24.1 / 28.0 / 83.1, 21.1 / 26.3 / 83.5); 8 actions 80
+    //     and 96 (24,576 of 40x40, 16 / 20 steps 28.5 / 37.7, 27.9 / 36.5); not where the maps are staged for rows too (17,042 of 20x55
+    //     with 8 actions, 11 steps 23.0, 27.0);
+    //   epsilon is fixed: more than three, tables past the caches, from three steps on (65,536 of 16x16, 4 steps 14.2, 12.9; 61,803 of 42x7
+    //     with 8 actions 15.5, 14.7); more than 2.75, large maps (48,000 of 32x32, 20 / 64 / 100 steps 35.5 / 99.5 / 136, 33.5 / 88.7 / 135; 8
+    //     actions up to 1300 cells: 46,298 of 46x36, 125 steps 222, 253).
+    const long rows_cells = e->A == 8                               ? (rows_rich ? kRowsCells8Rich : kRowsCells8)
+                            : (long)e->N <= 2L * 64 * kComputeUnits ? kRowsCells4
+                            : rows_rich                             ? kRowsCells4Rich
+                                                                    : kRowsCells4Fixed;
+    const bool rows_pay = (long)e->N > 4L * 64 * kComputeUnits || resident < e->N || ((long)e->N + 63) / 64 > kComputeUnits * lds_fit(map_lds) ||
+                          (!rows_staged && n_steps >= kRowsLargeMapMinSteps && (long)e->S >= n_steps * rows_cells) ||
+                          (!rows_rich && outgrown && (long)e->N > kMinEnvsInFlight && n_steps >= kRowsFixedMinSteps) ||
+                          (!rows_rich && (long)e->N > kRowsFixedEnvs && !rows_small && (e->A == 4 || e->S <= kRowsFixedMap8));
     const bool rows_first = rows_can && e->fused_variant == 0 && (((rows_many || rows_floored) && n_steps <= rows_steps) || rows_some);
     // ... hybrid workgroups (automatic) when the tables outgrow the caches: while they all fit, other plans are
     // faster (16x16 maps, 30,000 envs: 3.5e10 hybrid, 5.9e10 with lane waves); and where lane
@@ -840,11 +867,11 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
       if (!p.lanes) p.lds = waves * (p.moves ? mv_lds : map_lds);
       // No more of these than rows_first, or where they are the choice that is left: waves that keep rows instead (as many
       // as there are envs for, a workgroup each).
-      if (rows_first || (!p.lanes && rows_can && foldable &&
+      if (rows_first || (!p.lanes && rows_can && foldable && rows_pay &&
                          (rows_small || (n_steps >= kRowsLargeMapMinSteps && n_steps <= kRowsLargeMapMaxSteps)))) {
         p.fast = p.fixed = true;
         p.rich = rows_rich;
-        const size_t staged4 = map_lds + crl::RowCache<4, false, 4>::kBytes, staged6 = map_lds + crl::RowCache<4, false, 6>::kBytes;
+        const size_t staged6 = map_lds + crl::RowCache<4, false, 6>::kBytes;
         const long fit6 = lds_fit(staged6);
         if (!p.rich && (fit6 >= kRowsSixSoonWaves ? n_steps >= kRowsSixSoonSteps : fit6 >= kRowsSixWaves && n_steps >= kRowsSixSteps)) {
           p.rows = 6;
@@ -852,8 +879,8 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
           p.lds = staged6;
         } else {
           p.rows = 4;
-          p.moves = lds_fit(staged4) < (e->A == 8 ? kRowsStagedWaves8 : kRowsStagedWaves4);
-          p.lds = p.moves ? crl::RowCache<4, true, 4>::kBytes : staged4;
+          p.moves = !rows_staged;
+          p.lds = p.moves ? crl::RowCache<4, true, 4>::kBytes : rows_lds4;
         }
         p.block = 64;
         p.grid = (int)(((long)e->N + 63) / 64);

@@ -293,6 +293,27 @@ def test_rows_that_a_plan_keeps(pycrl, N, W, H, A, n_steps, rows, codes):
     assert pycrl.fused_plan_rows(cfg, n_steps) == (rows, codes)
 
 
+@pytest.mark.parametrize("N,W,H,A,n_steps,rows,kw", [
+    # up to three 64-env waves to a compute unit none, on any map, ragged or not
+    (40960, 8, 8, 4, 5, 0, 0), (49152, 12, 12, 4, 7, 0, 0), (17003, 13, 11, 8, 7, 0, 1), (44866, 4, 38, 8, 43, 0, 1),
+    (40960, 32, 32, 4, 128, 0, 0), (24576, 40, 40, 8, 128, 0, 1),
+    # ... but where a map costs more to stage than it saves in so few steps
+    (32768, 64, 64, 4, 51, 4, 1), (32768, 64, 64, 4, 52, 0, 1), (40960, 32, 32, 4, 25, 4, 0), (40960, 32, 32, 4, 26, 0, 0),
+    (40960, 32, 32, 4, 17, 4, 1), (40960, 32, 32, 4, 18, 0, 1), (24576, 40, 40, 8, 16, 4, 0), (24576, 40, 40, 8, 17, 0, 0),
+    (24576, 40, 40, 8, 20, 4, 1), (24576, 40, 40, 8, 21, 0, 1), (17042, 20, 55, 8, 11, 0, 1),
+    (35968, 64, 64, 4, 112, 4, 0), (32768, 64, 64, 4, 112, 0, 0),  # two of 64 KB of maps to a unit
+    (45056, 32, 32, 4, 64, 0, 0), (45057, 32, 32, 4, 64, 4, 0), (46298, 46, 36, 8, 125, 0, 0),
+    # four in calls of some steps
+    (65536, 16, 16, 4, 2, 0, 0), (65536, 16, 16, 4, 3, 4, 0), (65536, 16, 16, 4, 5, 0, 1), (65536, 16, 16, 4, 6, 4, 1), (57984, 4, 4, 4, 7, 0, 0),
+    (65537, 8, 8, 4, 4, 4, 1),
+])
+def test_rows_or_plain_waves(pycrl, N, W, H, A, n_steps, rows, kw):
+    linear = dict(eps_mode=pycrl.EPS_EPISODE_LINEAR, eps0=1.0, eps_end=0.1, eps_span=10) if kw else dict()
+    cfg = pycrl.make_config(N, W, H, n_actions=A, episode_len=128, **linear)
+    assert "lanes" not in pycrl.fused_plan_for_config(cfg, n_steps)["name"]
+    assert pycrl.fused_plan_rows(cfg, n_steps)[0] == rows
+
+
 @pytest.mark.parametrize("N,W,H,A,n_steps", [(19895, 40, 40, 8, 1), (24961, 16, 16, 4, 5), (58545, 20, 20, 8, 2), (16385, 3, 3, 4, 1)])
 def test_all_envs_in_flight_at_once(pycrl, N, W, H, A, n_steps):
     """A wave for the last, part-filled 64 envs too."""

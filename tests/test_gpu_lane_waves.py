@@ -66,8 +66,8 @@ def test_hybrid_workgroups(gpu, oracle, N, W, H, A, lds_waves):
 
 
 # waves of 64 envs, which short calls of more envs than lane waves are for take, and longer calls on
-# tables past the caches (most of these keep rows in LDS: those that keep none are below); the general
-# loop's hybrid workgroups
+# tables past the caches (which keep rows in LDS: with staged move codes below); the general loop's
+# hybrid workgroups
 LINEAR = dict(eps_mode=3, eps0=0.9, eps_end=0.1, eps_span=4)
 
 

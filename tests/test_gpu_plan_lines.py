@@ -17,7 +17,8 @@ ROWS = PLAIN + ", rows kept"  # which go by the name of the plain ones
     (4090, 16, 16, 4, 39, LANES), (4090, 16, 16, 4, 40, LDS),        # 16 KB to a wave
     (15001, 8, 8, 4, 40, LDS), (30001, 8, 8, 4, 117, LANES), (30001, 8, 8, 4, 119, LDS),  # four and eight such waves
     (70, 47, 49, 8, 143, LANES), (70, 47, 49, 8, 144, LDS),          # 72 KB to a wave
-    (33001, 32, 32, 4, 130, ROWS), (33001, 32, 32, 4, 131, PLAIN),   # large maps
+    (33001, 32, 32, 4, 130, PLAIN), (33001, 32, 32, 4, 25, ROWS), (33001, 32, 32, 4, 26, PLAIN),  # a map costs more to stage
+    (40001, 8, 8, 4, 7, PLAIN), (62001, 16, 16, 4, 2, PLAIN), (62001, 16, 16, 4, 3, ROWS),  # few envs; a part-filled last wave
     (50001, 32, 32, 4, 63, ROWS), (50001, 32, 32, 4, 64, LANES),     # rounds, of at most 65,536 envs
     (66001, 28, 28, 4, 130, ROWS), (66001, 28, 28, 4, 131, LANES),   # of more
     (250001, 8, 8, 4, 9, ROWS), (250001, 8, 8, 4, 10, LANES),        # in place of hybrid workgroups

@@ -25,7 +25,7 @@ def rows_check(gpu, oracle, N, W, H, A, chunks, staged, places=lambda steps: 4, 
 
 @pytest.mark.parametrize("kw", [dict(), LINEAR, dict(cells=1), dict(cells=3, **LINEAR), dict(episode_len=1), dict(episode_len=2),
                                 dict(episode_len=0)])
-@pytest.mark.parametrize("N,W,H,A", [(17003, 13, 11, 4), (16449, 16, 21, 4), (16385, 9, 10, 8)])
+@pytest.mark.parametrize("N,W,H,A", [(65603, 13, 11, 4), (65601, 16, 21, 4), (65537, 9, 10, 8)])
 def test_short_calls(gpu, oracle, N, W, H, A, kw):
     rows_check(gpu, oracle, N, W, H, A, (1, 7, 2, 5, 7, 7, 7), True, **kw)
 
@@ -42,12 +42,14 @@ def test_many_envs(gpu, oracle, N, W, H, A, steps, kw):
     rows_check(gpu, oracle, N, W, H, A, (steps, 9, 31), True, lambda c: 6 if c >= 32 and not ("eps_mode" in kw or "cells" in kw) else 4, **kw)
 
 
-@pytest.mark.parametrize("N,W,H,A,kw", [(33001, 33, 31, 4, dict()), (33001, 31, 33, 4, LINEAR), (17003, 35, 33, 8, dict()),
-                                        (17003, 34, 34, 8, dict(cells=3, **LINEAR))])
-def test_codes_with_the_rows(gpu, oracle, N, W, H, A, kw):
-    rows_check(gpu, oracle, N, W, H, A, (101, 12), False, episode_len=17, **kw)
+@pytest.mark.parametrize("N,W,H,A,chunks,kw", [
+    (50003, 33, 31, 4, (63, 12), dict()), (65701, 31, 33, 4, (101, 12), LINEAR), (17003, 35, 33, 8, (12, 11, 12), dict()),
+    (17003, 34, 34, 8, (12, 14, 11), dict(cells=3, **LINEAR)), (33001, 33, 31, 4, (25, 11), dict()), (16449, 61, 45, 4, (33, 20), LINEAR),
+])
+def test_codes_with_the_rows(gpu, oracle, N, W, H, A, chunks, kw):
+    rows_check(gpu, oracle, N, W, H, A, chunks, False, episode_len=17, **kw)
 
 
-@pytest.mark.parametrize("N,W,H,A,steps", [(66001, 27, 29, 4, 99), (66001, 27, 29, 4, 100), (30001, 31, 24, 8, 130)])
+@pytest.mark.parametrize("N,W,H,A,steps", [(66001, 27, 29, 4, 99), (66001, 27, 29, 4, 100), (66001, 31, 24, 8, 130)])
 def test_six_places_on_larger_maps(gpu, oracle, N, W, H, A, steps):
     rows_check(gpu, oracle, N, W, H, A, (steps,), True, lambda c: 6 if c >= 100 else 4, episode_len=30)
