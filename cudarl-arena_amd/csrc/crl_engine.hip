@@ -432,7 +432,7 @@ constexpr int kRowsSomeEnvs = 6 * 64 * kComputeUnits, kRowsSomeEnvsRich = 1 << 1
 constexpr size_t kRowsSmallMap = 336;  // cells: eleven to a unit
 constexpr long kRowsCells4 = 80, kRowsCells4Rich = 60, kRowsCells4Fixed = 40, kRowsCells8 = 96, kRowsCells8Rich = 80, kRowsFixedEnvs = 11L * 16 * kComputeUnits;
 constexpr int kRowsFixedMinSteps = 3;
-constexpr size_t kRowsFixedMap8 = 1300;
+constexpr size_t kRowsFixedMap8 = 1300, kRowsTwoStepsMap = 600;
 constexpr int kRowsLargeMapMinSteps = 11, kRowsLargeMapMaxSteps = 130;
 constexpr long kRowsStagedWaves4 = 7, kRowsStagedWaves8 = 6, kRowsSixSoonWaves = 9, kRowsSixWaves = 6;
 constexpr int kRowsSixSoonSteps = 32, kRowsSixSteps = 100;
@@ -744,11 +744,19 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
                             : (long)e->N <= 2L * 64 * kComputeUnits ? kRowsCells4
                             : rows_rich                             ? kRowsCells4Rich
                                                                     : kRowsCells4Fixed;
-    const bool rows_pay = (long)e->N > 4L * 64 * kComputeUnits || resident < e->N || ((long)e->N + 63) / 64 > kComputeUnits * lds_fit(map_lds) ||
+    // More envs than are at work at once, 4 actions, staged maps of more than 336 cells: not a call of one step (plain / rows: 262,144 of
+    // 16x32 25.2, 27.9; 315,185 of 33x18 31.8, 38.0; 252,160 of 20x40 29.4, 34.4; 524,288 of 20x20 39.6, 39.4; 258,311 of 12x48, epsilon by
+    // episode, 26.6, 30.5; with 8 actions 254,259 of 26x15 24.0, 24.1, 303,488 of 7x54 28.2, 27.0), on more than 600 while envs explore
+    // nor one of two (274,538 of 24x26 39.4, 44.4; 339,243 of 16x46 48.4, 52.4; but 281,664 of 24x24 38.5, 37.1).  Where codes come with the
+    // rows they pay at once (256,271 of 40x24, one step 38.8, 23.6), and in place of the general loop (505,664 of 29x13 39.6, 37.5).
+    const int rows_from = e->A == 8 || !foldable || !rows_staged || rows_small || e->N <= kRowsManyLargerTables ? 1
+                          : rows_rich && e->S > kRowsTwoStepsMap                                                 ? 3
+                                                                                                                 : 2;
+    const bool rows_pay = n_steps >= rows_from && ((long)e->N > 4L * 64 * kComputeUnits || resident < e->N || ((long)e->N + 63) / 64 > kComputeUnits * lds_fit(map_lds) ||
                           (!rows_staged && n_steps >= kRowsLargeMapMinSteps && (long)e->S >= n_steps * rows_cells) ||
                           (!rows_rich && outgrown && (long)e->N > kMinEnvsInFlight && n_steps >= kRowsFixedMinSteps) ||
-                          (!rows_rich && (long)e->N > kRowsFixedEnvs && !rows_small && (e->A == 4 || e->S <= kRowsFixedMap8));
-    const bool rows_first = rows_can && e->fused_variant == 0 && (((rows_many || rows_floored) && n_steps <= rows_steps) || rows_some);
+                          (!rows_rich && (long)e->N > kRowsFixedEnvs && !rows_small && (e->A == 4 || e->S <= kRowsFixedMap8)));
+    const bool rows_first = rows_can && rows_pay && e->fused_variant == 0 && (((rows_many || rows_floored) && n_steps <= rows_steps) || rows_some);
     // ... hybrid workgroups (automatic) when the tables outgrow the caches: while they all fit, other plans are
     // faster (16x16 maps, 30,000 envs: 3.5e10 hybrid, 5.9e10 with lane waves); and where lane
     // waves could step what is left to the general loop, they are faster too (262,144 envs of

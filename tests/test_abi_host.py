@@ -306,6 +306,9 @@ def test_rows_that_a_plan_keeps(pycrl, N, W, H, A, n_steps, rows, codes):
     # four in calls of some steps
     (65536, 16, 16, 4, 2, 0, 0), (65536, 16, 16, 4, 3, 4, 0), (65536, 16, 16, 4, 5, 0, 1), (65536, 16, 16, 4, 6, 4, 1), (57984, 4, 4, 4, 7, 0, 0),
     (65537, 8, 8, 4, 4, 4, 1),
+    # many envs: one step, and two while envs explore, on staged maps
+    (262144, 16, 32, 4, 1, 0, 0), (262144, 16, 32, 4, 2, 4, 0), (262144, 16, 21, 4, 1, 4, 0), (262144, 32, 32, 4, 1, 4, 1), (262144, 22, 22, 8, 1, 4, 1),
+    (262144, 17, 20, 4, 1, 0, 1), (262144, 17, 20, 4, 2, 4, 1), (300000, 24, 26, 4, 2, 0, 1), (300000, 24, 26, 4, 3, 4, 1), (300000, 24, 26, 4, 2, 4, 0),
 ])
 def test_rows_or_plain_waves(pycrl, N, W, H, A, n_steps, rows, kw):
     linear = dict(eps_mode=pycrl.EPS_EPISODE_LINEAR, eps0=1.0, eps_end=0.1, eps_span=10) if kw else dict()
