@@ -431,7 +431,9 @@ constexpr int kRowsManyEnvs = 1 << 18, kRowsManyLargerTables = 200000, kRowsHybr
 constexpr int kRowsSomeEnvs = 6 * 64 * kComputeUnits, kRowsSomeEnvsRich = 1 << 17, kRowsSomeEnvsSteps = 88, kRowsLanesSteps = 500;
 constexpr size_t kRowsSmallMap = 336;  // cells: eleven to a unit
 constexpr long kRowsCells4 = 80, kRowsCells4Rich = 60, kRowsCells4Fixed = 40, kRowsCells8 = 96, kRowsCells8Rich = 80, kRowsFixedEnvs = 11L * 16 * kComputeUnits;
-constexpr int kRowsFixedMinSteps = 3;
+constexpr int kRowsFixedMinSteps = 3, kRowsTwoRoundsSteps = 20, kRowsLateSteps = 240, kRowsSmallestTablesSteps = 64;
+constexpr long kRowsTwoRoundsWaves = 27, kRowsLateWaves = 12;
+constexpr size_t kRowsSmallestTables = 40;
 constexpr size_t kRowsFixedMap8 = 1300, kRowsTwoStepsMap = 600;
 constexpr int kRowsLargeMapMinSteps = 11, kRowsLargeMapMaxSteps = 130;
 constexpr long kRowsStagedWaves4 = 7, kRowsStagedWaves8 = 6, kRowsSixSoonWaves = 9, kRowsSixWaves = 6;
@@ -756,7 +758,22 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
                           (!rows_staged && n_steps >= kRowsLargeMapMinSteps && (long)e->S >= n_steps * rows_cells) ||
                           (!rows_rich && outgrown && (long)e->N > kMinEnvsInFlight && n_steps >= kRowsFixedMinSteps) ||
                           (!rows_rich && (long)e->N > kRowsFixedEnvs && !rows_small && (e->A == 4 || e->S <= kRowsFixedMap8)));
-    const bool rows_first = rows_can && rows_pay && e->fused_variant == 0 && (((rows_many || rows_floored) && n_steps <= rows_steps) || rows_some);
+    // Floored maximum, 4 actions: rounds of lane waves stay (us, these / rows)
+    //   epsilon by episode, tables that the caches hold and not two full rounds: 100,000 of 10x10, 100 / 400 steps 150 / 537, 157 / 580;
+    //     102,577 of 17x4, 211 steps 254, 289; 106,471 of 6x12, 72 steps 103, 111; 117,792 of 13x8, 48 steps 100, 93;
+    //   epsilon by episode, tables past them, long calls, where up to a quarter more waves with rows than are at work at once would begin
+    //     when the others are through: 200,882 of 11x19 (12.3 to a unit, 12 fit), 315 steps 1175, 1317; 213,000 of 14x15, 358 steps 1317, 1421;
+    //     172,032 of 22x20, 464 steps 1633, 1831; not with as many as fit (208,724 of 22x7, 265 steps 968, 778), smaller maps, of which
+    //     more than twelve fit (305,000 of 20x4, 17.3 and 16 to a unit, 455 steps 1887, 1530) or shorter calls (240,442 of 17x11, 131 steps 652, 599);
+    //   epsilon fixed, the smallest tables: 300,000 of 3x3, 20 / 100 / 400 / 1000 steps 66 / 250 / 935 / 2356, 55 / 254 / 977 / 2410; 376,832 of 2x3,
+    //     197 steps 530, 584; of 4x4 400 steps 982, 991; 358,000 of 3x5, 151 steps 469, 436; 563,274 of 4x3, 850 steps 3816, 3357.
+    const long rows_waves = ((long)e->N + 63) / 64, rows_at_once = kComputeUnits * lds_fit(rows_lds4);
+    const bool rows_late = c.max_mode != CRL_MAX_TRUE && e->A == 4 &&
+                           (!by_episode ? !outgrown && rounds <= 6 && e->K <= kRowsSmallestTables && n_steps >= kRowsSmallestTablesSteps
+                            : outgrown  ? rows_staged && rows_at_once <= kRowsLateWaves * kComputeUnits && rows_waves > rows_at_once &&
+                                             4 * rows_waves <= 5 * rows_at_once && n_steps >= kRowsLateSteps
+                                        : lane_units <= kRowsTwoRoundsWaves * kComputeUnits && n_steps >= kRowsTwoRoundsSteps);
+    const bool rows_first = rows_can && rows_pay && !rows_late && e->fused_variant == 0 && (((rows_many || rows_floored) && n_steps <= rows_steps) || rows_some);
     // ... hybrid workgroups (automatic) when the tables outgrow the caches: while they all fit, other plans are
     // faster (16x16 maps, 30,000 envs: 3.5e10 hybrid, 5.9e10 with lane waves); and where lane
     // waves could step what is left to the general loop, they are faster too (262,144 envs of

@@ -317,6 +317,24 @@ def test_rows_or_plain_waves(pycrl, N, W, H, A, n_steps, rows, kw):
     assert pycrl.fused_plan_rows(cfg, n_steps)[0] == rows
 
 
+@pytest.mark.parametrize("N,W,H,A,n_steps,rows,kw", [
+    # two rounds of lane waves that are not full, tables that the caches hold
+    (100000, 10, 10, 4, 400, 0, 1), (100000, 10, 10, 4, 19, 4, 1), (100000, 10, 10, 4, 400, 6, 0), (110592, 5, 15, 4, 400, 0, 1), (110608, 5, 15, 4, 400, 4, 1),
+    (100000, 16, 16, 4, 400, 4, 1),
+    # a few more waves with rows than the twelve to a unit that fit, tables past the caches
+    (196608, 11, 19, 4, 240, 4, 1), (196672, 11, 19, 4, 240, 0, 1), (196672, 11, 19, 4, 239, 4, 1), (196672, 11, 19, 4, 240, 6, 0), (196672, 11, 19, 8, 240, 4, 1),
+    (245760, 11, 19, 4, 240, 0, 1), (245824, 11, 19, 4, 240, 4, 1), (240000, 22, 7, 4, 240, 4, 1), (305000, 20, 4, 4, 455, 4, 1),
+    # the smallest tables
+    (300000, 3, 3, 4, 63, 6, 0), (300000, 3, 3, 4, 64, 0, 0), (300000, 3, 4, 4, 400, 6, 0), (300000, 3, 3, 4, 400, 4, 1), (400000, 3, 3, 4, 400, 6, 0),
+    (300000, 2, 2, 8, 400, 6, 0),
+])
+def test_rows_or_lane_waves_of_a_floored_maximum(pycrl, N, W, H, A, n_steps, rows, kw):
+    linear = dict(eps_mode=pycrl.EPS_EPISODE_LINEAR, eps0=1.0, eps_end=0.1, eps_span=10) if kw else dict()
+    cfg = pycrl.make_config(N, W, H, n_actions=A, episode_len=128, max_mode=pycrl.MAX_ZERO_FLOOR, **linear)
+    assert pycrl.fused_plan_rows(cfg, n_steps)[0] == rows
+    assert ("lanes" in pycrl.fused_plan_for_config(cfg, n_steps)["name"]) == (rows == 0)
+
+
 @pytest.mark.parametrize("N,W,H,A,n_steps", [(19895, 40, 40, 8, 1), (24961, 16, 16, 4, 5), (58545, 20, 20, 8, 2), (16385, 3, 3, 4, 1)])
 def test_all_envs_in_flight_at_once(pycrl, N, W, H, A, n_steps):
     """A wave for the last, part-filled 64 envs too."""
