@@ -427,17 +427,27 @@ constexpr size_t kTableBytesAtOnce = (size_t)512 << 20;
 // 487 / 2012, 438 / 1410; 300,000 of 20x20, eight, 24 / 50 / 150 126 / 236 / 681, 136 / 245 / 664; of 28x28, six, 40 / 150 208 / 701,
 // 210 / 672; of 32x32, five, 150 steps 721, 797; 300,000 of 16x16 with 8 actions, 60 / 300 392 / 1965, 390 / 1806; eight places, 300 steps of
 // 1M of 16x16 3747 -> 3967.  With epsilon by episode, where envs explore, 1M of 16x16, 24 / 60 / 200 steps 414 / 956 / 3118, 436 / 1033 / 3255).
-constexpr int kRowsManyEnvs = 1 << 18, kRowsManyLargerTables = 200000, kRowsHybridSteps4 = 48, kRowsHybridSteps8 = 96;
-constexpr int kRowsSomeEnvs = 6 * 64 * kComputeUnits, kRowsSomeEnvsRich = 1 << 17, kRowsSomeEnvsSteps = 88, kRowsLanesSteps = 500;
-constexpr size_t kRowsSmallMap = 336;  // cells: eleven to a unit
-constexpr long kRowsCells4 = 80, kRowsCells4Rich = 60, kRowsCells4Fixed = 40, kRowsCells8 = 96, kRowsCells8Rich = 80, kRowsFixedEnvs = 11L * 16 * kComputeUnits;
-constexpr int kRowsFixedMinSteps = 3, kRowsTwoRoundsSteps = 20, kRowsLateSteps = 240, kRowsSmallestTablesSteps = 64;
+// (which of plan_fused's figures each line comes from)
+constexpr int kRowsManyEnvs = 1 << 18;           // in place of every other plan, whatever the table ...
+constexpr int kRowsManyLargerTables = 200000;    // ... of more than 256 values
+constexpr int kRowsHybridSteps4 = 48, kRowsHybridSteps8 = 96;  // up to so many steps, and some for each key, before hybrid workgroups
+constexpr int kRowsLanesSteps = 500;             // up to so many, 8 actions or epsilon by episode, before rounds of lane waves
+constexpr int kRowsSomeEnvs = 6 * 64 * kComputeUnits, kRowsSomeEnvsRich = 1 << 17, kRowsSomeEnvsSteps = 88;  // fewer envs: in place of lane waves in two rounds and more
+constexpr size_t kRowsSmallMap = 336;            // cells: eleven to a unit
+constexpr int kRowsLargeMapMinSteps = 11, kRowsLargeMapMaxSteps = 130;  // larger maps, fewer envs: where plain 64-env waves are the other choice
+constexpr long kRowsStagedWaves4 = 7, kRowsStagedWaves8 = 6;  // maps in LDS if so many waves then fit a unit (above)
+constexpr long kRowsSixSoonWaves = 9, kRowsSixWaves = 6;      // six places if so many waves fit (above) ...
+constexpr int kRowsSixSoonSteps = 32, kRowsSixSteps = 100;    // ... in calls of so many steps
+// against plain waves (rows_pay):
+constexpr long kRowsCells4 = 80, kRowsCells4Rich = 60, kRowsCells4Fixed = 40, kRowsCells8 = 96, kRowsCells8Rich = 80;  // cells to a step
+constexpr long kRowsFixedEnvs = 11L * 16 * kComputeUnits;     // epsilon fixed, large maps: 2.75 waves to a unit ...
+constexpr size_t kRowsFixedMap8 = 1300;                       // ... with 8 actions up to so many cells
+constexpr int kRowsFixedMinSteps = 3;                         // epsilon fixed, four waves to a unit
+constexpr size_t kRowsTwoStepsMap = 600;                      // many envs, epsilon by episode: two steps are too few on more cells
+// against lane waves with a floored maximum (rows_late):
+constexpr int kRowsTwoRoundsSteps = 20, kRowsLateSteps = 240, kRowsSmallestTablesSteps = 64;
 constexpr long kRowsTwoRoundsWaves = 27, kRowsLateWaves = 12;
 constexpr size_t kRowsSmallestTables = 40;
-constexpr size_t kRowsFixedMap8 = 1300, kRowsTwoStepsMap = 600;
-constexpr int kRowsLargeMapMinSteps = 11, kRowsLargeMapMaxSteps = 130;
-constexpr long kRowsStagedWaves4 = 7, kRowsStagedWaves8 = 6, kRowsSixSoonWaves = 9, kRowsSixWaves = 6;
-constexpr int kRowsSixSoonSteps = 32, kRowsSixSteps = 100;
 
 // Configurations that run_lanes() steps: no goal test on the resulting cell, no sticky done,
 // no trace and no supplied stream.
@@ -712,7 +722,9 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     //     69 / 151, 47 / 94; 200,000 of 5x4, 16 / 50 46 / 113, 37 / 110; of 15x15, 50 / 80 270 / 402, 175 / 261; 8 actions: 99,000 of 4x4,
     //     8 / 50 28 / 102, 18 / 71; 130,000 of 9x9, 30 / 80 120 / 232, 79 / 140; 260,000 of 7x7, 16 / 80 141 / 435, 83 / 279
     // With fewer envs still a step is as long as its slowest request and lane waves have fewer of those (50,000 of 16x16, 20 steps
-    // 26.6, 33.3).  Between that and these lines lie lengths and sizes that tests hold the others to.
+    // 26.6, 33.3).  Not all of these lines lie where the two sides cross: 200,001 to 262,143 envs with tables of up to 256 values, up to
+    // 200,000 on maps of up to 336 cells past 88 steps (at 80 steps rows are still 1.5 times as fast), and on larger ones below 11 and
+    // above 130, keep the other plans although their neighbours in size are the faster ones with rows.
     const bool rows_can = lanes_rules(e) && c.max_episodes == 0 && c.track_returns == 0 && c.eps_mode != CRL_EPS_STEP_MULT &&
                           e->mv_words > 0 && e->resident_envs == 0 && e->fused_variant != 2;
     const bool rows_rich = c.eps_mode != CRL_EPS_FIXED || c.reward_flags != 0;
@@ -1971,9 +1983,10 @@ int set_cell(crl_engine* e, int32_t map_index, int32_t cell, int32_t cell_class,
   return CRL_OK;
 }
 
-// every ticket-kernel instantiation launch_fused_a can pick, but those that keep rows (20 KB at most), may use the whole LDS:
+// every ticket-kernel instantiation launch_fused_a can pick may use the whole LDS:
 // the plain ones, too, ask for more than the default 64 KB when large per-env
-// maps share a workgroup
+// maps share a workgroup (those that keep rows do not: six of them fit a compute
+// unit where their maps are staged, 26,880 bytes at most)
 int opt_in_ticket_kernels(crl_engine* e) {
   if (e->hybrid_opt_in) return CRL_OK;
   const void* fns[] = {

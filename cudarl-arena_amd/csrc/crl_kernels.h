@@ -443,8 +443,10 @@ __device__ __forceinline__ void run_env_fast(const Rules& R, const Ptrs& P, cons
 // other are in different ones.  Two lanes move a run together, 16 bytes each, first for one of them and then for the other.
 // [place][piece][lane], the lane mixed with the piece against bank conflicts; then the words, [place][lane].
 //
-// What bounds it: 270 vector instructions a step and, with them about half of the time, a trip to HBM for the lanes whose cell
-// is new - with 64 envs there is always one.  1M envs of 16x16, 20 steps, 627 us with a row and a value per step from and to
+// What bounds it: memory, in requests of 128 bytes of which an env wants 32 and in partial writes, and that these and the steps overlap
+// but in part: 1M envs of 16x16, 20 steps, 369 us, without loads and stores 169, with the stores only 187, the loads only 271.  A step
+// waits for the lanes whose cell is new - with 64 envs there is always one.  257 vector instructions a step are not the bound (a
+// variant with 14 % fewer took the same time).  What it came from: 627 us with a row and a value per step from and to
 // HBM (21M reads of 16 bytes that meet the L2 in 5.9M lines, 21M stores of 4 bytes); rows kept one by one, each lane moving
 // its own 474 (11.9M lines: with 16 waves to a compute unit none of it is met again in the L2); runs of two, each lane moving its own
 // 430, of four 484; runs of two moved by two lanes and only what was written put back 383, with nothing in flight at the loop's

@@ -211,6 +211,8 @@ def test_every_valid_configuration_has_a_launch_plan_that_fits(pycrl):
                         plan = pycrl.fused_plan_for_config(cfg, n_steps)  # raises on a plan that does not fit
                         assert 0 <= plan["lds_bytes"] <= 160 * 1024, (N, W, H, A, n_steps, plan)
                         assert plan["grid"] >= 1 and plan["block"] in (64, 128, 192, 256, 320), plan
+                        # (kernels that keep rows are launched without asking for more than the default 64 KB)
+                        assert pycrl.fused_plan_rows(cfg, n_steps)[0] == 0 or plan["lds_bytes"] <= 64 * 1024, plan
                         checked += 1
     assert checked > 2000
     # the two cases that used to ask for 192 KB and 256 KB

@@ -43,3 +43,12 @@ def test_lane_waves_to_a_simd(kernels):
     for name, got in lanes.items():
         assert got["vgpr_count"] <= (96 if "ELi2EEE" in name else 80), (name, got)
         assert got["private_segment_fixed_size"] == 0 and got["vgpr_spill_count"] == 0, (name, got)
+
+
+def test_waves_that_keep_rows(kernels):
+    """Up to sixteen 64-env waves that keep rows in LDS to a compute unit: 512 / 4 registers, and nothing in scratch."""
+    rows = {k: v for k, v in kernels.items() if re.search(r"k_fused_ticketsILi[48]ELi[012]ELb0ELb[01]ELi[1-9]EE", k)}
+    assert len(rows) == 10
+    for name, got in rows.items():
+        assert got["vgpr_count"] <= 128, (name, got)
+        assert got["private_segment_fixed_size"] == 0 and got["vgpr_spill_count"] == 0, (name, got)
