@@ -439,10 +439,12 @@ constexpr long kRowsStagedWaves4 = 7, kRowsStagedWaves8 = 6;  // maps in LDS if 
 constexpr long kRowsSixSoonWaves = 9, kRowsSixWaves = 6;      // six places if so many waves fit (above) ...
 constexpr int kRowsSixSoonSteps = 32, kRowsSixSteps = 100;    // ... in calls of so many steps
 // against plain waves (rows_pay):
-constexpr long kRowsCells4 = 80, kRowsCells4Rich = 60, kRowsCells4Fixed = 40, kRowsCells8 = 96, kRowsCells8Rich = 80;  // cells to a step
+constexpr long kRowsCells4 = 80, kRowsCells4Rich = 60, kRowsCells4Fixed = 40, kRowsCells8 = 96, kRowsCells8Rich = 80;  // cells to a step ...
+constexpr long kRowsCells4Rewards = 32, kRowsCells8Rewards = 16;  // ... with rewards per cell and more than two waves to a unit
+constexpr long kRowsRewardsEnvs = 10L * 16 * kComputeUnits;   // rewards per cell, large maps: 2.5 waves to a unit
 constexpr long kRowsFixedEnvs = 11L * 16 * kComputeUnits;     // epsilon fixed, large maps: 2.75 waves to a unit ...
 constexpr size_t kRowsFixedMap8 = 1300;                       // ... with 8 actions up to so many cells
-constexpr int kRowsFixedMinSteps = 3;                         // epsilon fixed, four waves to a unit
+constexpr int kRowsFixedMinSteps = 3;                         // epsilon fixed or rewards per cell, four waves to a unit
 constexpr size_t kRowsTwoStepsMap = 600;                      // many envs, epsilon by episode: two steps are too few on more cells
 // against lane waves with a floored maximum (rows_late):
 constexpr int kRowsTwoRoundsSteps = 20, kRowsLateSteps = 240, kRowsSmallestTablesSteps = 64;
@@ -727,7 +729,7 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     // above 130, keep the other plans although their neighbours in size are the faster ones with rows.
     const bool rows_can = lanes_rules(e) && c.max_episodes == 0 && c.track_returns == 0 && c.eps_mode != CRL_EPS_STEP_MULT &&
                           e->mv_words > 0 && e->resident_envs == 0 && e->fused_variant != 2;
-    const bool rows_rich = c.eps_mode != CRL_EPS_FIXED || c.reward_flags != 0;
+    const bool cells = c.reward_flags != 0, rows_rich = c.eps_mode != CRL_EPS_FIXED || cells;
     const int rows_steps = fits && p.fast ? (e->A == 8 ? kRowsHybridSteps8 + (int)(e->K / 8) : kRowsHybridSteps4 + (int)(3 * e->K / 16))
                            : e->A == 8 || rows_rich ? std::max(kRowsLanesSteps, (int)(e->K / 3))
                                                     : INT_MAX;
@@ -753,23 +755,29 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     //     with 8 actions, 11 steps 23.0, 27.0);
     //   epsilon is fixed: more than three, tables past the caches, from three steps on (65,536 of 16x16, 4 steps 14.2, 12.9; 61,803 of 42x7
     //     with 8 actions 15.5, 14.7); more than 2.75, large maps (48,000 of 32x32, 20 / 64 / 100 steps 35.5 / 99.5 / 136, 33.5 / 88.7 / 135; 8
-    //     actions up to 1300 cells: 46,298 of 46x36, 125 steps 222, 253).
-    const long rows_cells = e->A == 8                               ? (rows_rich ? kRowsCells8Rich : kRowsCells8)
-                            : (long)e->N <= 2L * 64 * kComputeUnits ? kRowsCells4
-                            : rows_rich                             ? kRowsCells4Rich
-                                                                    : kRowsCells4Fixed;
+    //     actions up to 1300 cells: 46,298 of 46x36, 125 steps 222, 253);
+    //   cells have rewards, whatever epsilon: the same with more than three waves, on large maps with more than 2.5 (45,825 of 57x44 with 8
+    //     actions, 32 steps 70, 52; 48,448 of 58x28, epsilon by episode, 74 steps 152, 126), and with more than two 32 and 16 cells to a step (41,216
+    //     of 32x59, 64 steps 92.1, 82.5; 33,904 of 49x30 with 8 actions, 20 steps 38.2, 31.7).
+    const bool two_waves = (long)e->N <= 2L * 64 * kComputeUnits;
+    const long rows_cells = cells && !two_waves ? (e->A == 8 ? kRowsCells8Rewards : kRowsCells4Rewards)
+                            : e->A == 8         ? (rows_rich ? kRowsCells8Rich : kRowsCells8)
+                            : two_waves         ? kRowsCells4
+                            : rows_rich         ? kRowsCells4Rich
+                                                : kRowsCells4Fixed;
     // More envs than are at work at once, 4 actions, staged maps of more than 336 cells: not a call of one step (plain / rows: 262,144 of
     // 16x32 25.2, 27.9; 315,185 of 33x18 31.8, 38.0; 252,160 of 20x40 29.4, 34.4; 524,288 of 20x20 39.6, 39.4; 258,311 of 12x48, epsilon by
     // episode, 26.6, 30.5; with 8 actions 254,259 of 26x15 24.0, 24.1, 303,488 of 7x54 28.2, 27.0), on more than 600 while envs explore
     // nor one of two (274,538 of 24x26 39.4, 44.4; 339,243 of 16x46 48.4, 52.4; but 281,664 of 24x24 38.5, 37.1).  Where codes come with the
     // rows they pay at once (256,271 of 40x24, one step 38.8, 23.6), and in place of the general loop (505,664 of 29x13 39.6, 37.5).
-    const int rows_from = e->A == 8 || !foldable || !rows_staged || rows_small || e->N <= kRowsManyLargerTables ? 1
+    const int rows_from = e->A == 8 || cells || !foldable || !rows_staged || rows_small || e->N <= kRowsManyLargerTables ? 1
                           : rows_rich && e->S > kRowsTwoStepsMap                                                 ? 3
                                                                                                                  : 2;
     const bool rows_pay = n_steps >= rows_from && ((long)e->N > 4L * 64 * kComputeUnits || resident < e->N || ((long)e->N + 63) / 64 > kComputeUnits * lds_fit(map_lds) ||
                           (!rows_staged && n_steps >= kRowsLargeMapMinSteps && (long)e->S >= n_steps * rows_cells) ||
-                          (!rows_rich && outgrown && (long)e->N > kMinEnvsInFlight && n_steps >= kRowsFixedMinSteps) ||
-                          (!rows_rich && (long)e->N > kRowsFixedEnvs && !rows_small && (e->A == 4 || e->S <= kRowsFixedMap8)));
+                          ((!rows_rich || cells) && outgrown && (long)e->N > kMinEnvsInFlight && n_steps >= kRowsFixedMinSteps) ||
+                          ((!rows_rich || cells) && (long)e->N > (cells ? kRowsRewardsEnvs : kRowsFixedEnvs) && !rows_small &&
+                           (e->A == 4 || cells || e->S <= kRowsFixedMap8)));
     // Floored maximum, 4 actions: rounds of lane waves stay (us, these / rows)
     //   epsilon by episode, tables that the caches hold and not two full rounds: 100,000 of 10x10, 100 / 400 steps 150 / 537, 157 / 580;
     //     102,577 of 17x4, 211 steps 254, 289; 106,471 of 6x12, 72 steps 103, 111; 117,792 of 13x8, 48 steps 100, 93;

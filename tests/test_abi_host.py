@@ -319,6 +319,19 @@ def test_rows_or_plain_waves(pycrl, N, W, H, A, n_steps, rows, kw):
     assert pycrl.fused_plan_rows(cfg, n_steps)[0] == rows
 
 
+@pytest.mark.parametrize("N,W,H,A,n_steps,rows,linear", [
+    (40960, 57, 44, 8, 32, 4, 0), (40960, 32, 32, 8, 65, 0, 0), (40961, 32, 32, 8, 120, 4, 0), (40961, 58, 28, 4, 74, 4, 1), (32768, 49, 30, 8, 20, 0, 0),
+    (32769, 49, 30, 8, 20, 4, 1), (40960, 32, 59, 4, 59, 4, 0), (40960, 32, 59, 4, 60, 0, 0), (40961, 8, 8, 4, 5, 0, 0),
+    (65536, 16, 16, 8, 2, 0, 1), (65536, 16, 16, 8, 3, 4, 1), (331526, 30, 23, 4, 1, 4, 1),
+])
+def test_rows_or_plain_waves_with_cell_rewards(pycrl, N, W, H, A, n_steps, rows, linear):
+    kw = dict(eps_mode=pycrl.EPS_EPISODE_LINEAR, eps0=1.0, eps_end=0.1, eps_span=10) if linear else dict()
+    for flags in (1, 3):
+        cfg = pycrl.make_config(N, W, H, n_actions=A, episode_len=128, reward_flags=flags, **kw)
+        assert "lanes" not in pycrl.fused_plan_for_config(cfg, n_steps)["name"]
+        assert pycrl.fused_plan_rows(cfg, n_steps)[0] == rows
+
+
 @pytest.mark.parametrize("N,W,H,A,n_steps,rows,kw", [
     # two rounds of lane waves that are not full, tables that the caches hold
     (100000, 10, 10, 4, 400, 0, 1), (100000, 10, 10, 4, 19, 4, 1), (100000, 10, 10, 4, 400, 6, 0), (110592, 5, 15, 4, 400, 0, 1), (110608, 5, 15, 4, 400, 4, 1),
