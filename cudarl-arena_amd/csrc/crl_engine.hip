@@ -433,6 +433,8 @@ constexpr int kRowsManyLargerTables = 200000;    // ... of more than 256 values
 constexpr int kRowsHybridSteps4 = 48, kRowsHybridSteps8 = 96;  // up to so many steps, and some for each key, before hybrid workgroups
 constexpr int kRowsLanesSteps = 500;             // up to so many, 8 actions or epsilon by episode, before rounds of lane waves
 constexpr int kRowsSomeEnvs = 6 * 64 * kComputeUnits, kRowsSomeEnvsRich = 1 << 17, kRowsSomeEnvsSteps = 88;  // fewer envs: in place of lane waves in two rounds and more
+constexpr size_t kRowsRewardsSmallest = 25, kRowsRewardsMiddle = 100, kRowsRewardsLarge = 256;  // cells: with rewards per cell ...
+constexpr int kRowsRewardsMiddleSteps = 200, kRowsRewardsLargeSteps = 240;             // ... up to so many steps (cells_steps)
 constexpr size_t kRowsSmallMap = 336;            // cells: eleven to a unit
 constexpr int kRowsLargeMapMinSteps = 11, kRowsLargeMapMaxSteps = 130;  // larger maps, fewer envs: where plain 64-env waves are the other choice
 constexpr long kRowsStagedWaves4 = 7, kRowsStagedWaves8 = 6;  // maps in LDS if so many waves then fit a unit (above)
@@ -729,8 +731,28 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     // above 130, keep the other plans although their neighbours in size are the faster ones with rows.
     const bool rows_can = lanes_rules(e) && c.max_episodes == 0 && c.track_returns == 0 && c.eps_mode != CRL_EPS_STEP_MULT &&
                           e->mv_words > 0 && e->resident_envs == 0 && e->fused_variant != 2;
+    const size_t rows_lds4 = map_lds + crl::RowCache<4, false, 4>::kBytes;
+    const bool rows_staged = lds_fit(rows_lds4) >= (e->A == 8 ? kRowsStagedWaves8 : kRowsStagedWaves4);
     const bool cells = c.reward_flags != 0, rows_rich = c.eps_mode != CRL_EPS_FIXED || cells;
+    // (rewards per cell: lane waves, which take over from plain ones at 131 steps, are the faster ones then on most tables, the more so where
+    // envs wander; lane waves / rows: rewards of goals and traps only, epsilon fixed, 357,632 of 4x12, 245 steps 1157, 2299; 910,400 of 4x17, 182
+    // steps 2470, 4554; 247,808 of 24x5, 339 steps 1558, 2393; 8 actions, 278,651 of 10x33, 324 steps 2931, 3284; rewards of all cells, epsilon by
+    // episode, 8 actions, 597,376 of 29x4, 197 steps 3306, 3499.  Rows go on on the smallest maps (974,336 of 5x3, 254 steps 3161, 1683; 682,624,
+    // epsilon fixed, 308 steps 2040, 1310; 578,368 of 5x5 with 8 actions, 312 steps 2688, 2136); with 4 actions on 256 cells and more whose maps are staged (1.05 to 1.2
+    // times as fast; not where codes come with the rows, 236,650 of 37x30, epsilon by episode, 532 steps 3837, 4715, unless lane waves have no even rounds
+    // either, 104,006 of 61x33, floored maximum, 320 steps 1652 by the general loop, 1147; 8 actions, epsilon by episode, 296,064 of 13x30, 134 steps 1510, 1396, past 240 0.96 times); with rewards of all cells and
+    // epsilon fixed (417,152 of 22x6, 363 steps 2197, 1597; 889,344 of 5x16 with 8 actions, 182 steps 3220, 2704; 896,384 of 15x3, 252 steps 2772,
+    // 1980; not all of 30 to 100 cells, 229,376 of 4x20, 273 steps 823, 976); for a while with 4 actions, epsilon by episode, on 100 and more (861,017 of 30x8, 178 steps
+    // 4179, 3594; 362,432 of 24x5, 230 steps 1860, 1676).)
+    const bool base_cells = (c.reward_flags & CRL_REWARD_BASE_CELLS) != 0;
+    const bool cells_long = e->S <= kRowsRewardsSmallest || (e->A == 4 && e->S >= kRowsRewardsLarge && rows_staged) || (base_cells && !by_episode) ||
+                            kComputeUnits * lane_fit < per_round;  // (no even rounds)
+    const int cells_steps = !by_episode || !rows_staged                     ? kLaneRoundsManyMinSteps - 1
+                            : e->S >= kRowsRewardsLarge                     ? kRowsRewardsLargeSteps
+                            : e->A == 4 && e->S >= kRowsRewardsMiddle       ? kRowsRewardsMiddleSteps
+                                                                            : kLaneRoundsManyMinSteps - 1;
     const int rows_steps = fits && p.fast ? (e->A == 8 ? kRowsHybridSteps8 + (int)(e->K / 8) : kRowsHybridSteps4 + (int)(3 * e->K / 16))
+                           : cells && !cells_long   ? cells_steps
                            : e->A == 8 || rows_rich ? std::max(kRowsLanesSteps, (int)(e->K / 3))
                                                     : INT_MAX;
     const bool rows_small = e->S <= kRowsSmallMap;
@@ -740,8 +762,6 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
                                                  : (long)e->N > kLaneRoundsManyEnvs && e->K >= 640);
     const bool rows_floored = c.max_mode != CRL_MAX_TRUE && !lanes_at_once && (long)e->N > kLaneRoundsManyEnvs &&
                               e->K >= (e->N > kRowsSomeEnvs ? 257 : 640);
-    const size_t rows_lds4 = map_lds + crl::RowCache<4, false, 4>::kBytes;
-    const bool rows_staged = lds_fit(rows_lds4) >= (e->A == 8 ? kRowsStagedWaves8 : kRowsStagedWaves4);
     // Up to three of them to a compute unit plain 64-env waves are faster (plain / rows: 40,960 of 8x8, 2 / 5 steps 7.1 / 9.0, 8.2 /
     // 11.1; 40,000 of 16x16 with 8 actions, 4 steps 12.0, 13.3; 40,960 of 32x32, 128 steps 141, 159; 24,576 of 40x40 with 8 actions 171,
     // 210; 44,866 of 4x38 with 8 actions, 43 steps 55, 68), and four in calls too short for a limit on the envs in flight (62,848 of
