@@ -433,7 +433,8 @@ constexpr int kRowsManyLargerTables = 200000;    // ... of more than 256 values
 constexpr int kRowsHybridSteps4 = 48, kRowsHybridSteps8 = 96;  // up to so many steps, and some for each key, before hybrid workgroups
 constexpr int kRowsLanesSteps = 500;             // up to so many, 8 actions or epsilon by episode, before rounds of lane waves
 constexpr int kRowsSomeEnvs = 6 * 64 * kComputeUnits, kRowsSomeEnvsRich = 1 << 17, kRowsSomeEnvsSteps = 88;  // fewer envs: in place of lane waves in two rounds and more
-constexpr size_t kRowsRewardsSmallest = 25, kRowsRewardsMiddle = 100, kRowsRewardsLarge = 256;  // cells: with rewards per cell ...
+constexpr long kRowsRewardsSmallEnvs = 22L * 64 * kComputeUnits;  // with rewards of all cells
+constexpr size_t kRowsRewardsSmallest = 25, kRowsRewardsSmaller = 26, kRowsRewardsSmall = 28, kRowsRewardsMiddle = 100, kRowsRewardsLarge = 256;  // cells: with rewards per cell ...
 constexpr int kRowsRewardsMiddleSteps = 200, kRowsRewardsLargeSteps = 240;             // ... up to so many steps (cells_steps)
 constexpr size_t kRowsSmallMap = 336;            // cells: eleven to a unit
 constexpr int kRowsLargeMapMinSteps = 11, kRowsLargeMapMaxSteps = 130;  // larger maps, fewer envs: where plain 64-env waves are the other choice
@@ -745,7 +746,12 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
     // 1980; not all of 30 to 100 cells, 229,376 of 4x20, 273 steps 823, 976); for a while with 4 actions, epsilon by episode, on 100 and more (861,017 of 30x8, 178 steps
     // 4179, 3594; 362,432 of 24x5, 230 steps 1860, 1676).)
     const bool base_cells = (c.reward_flags & CRL_REWARD_BASE_CELLS) != 0;
-    const bool cells_long = e->S <= kRowsRewardsSmallest || (e->A == 4 && e->S >= kRowsRewardsLarge && rows_staged) || (base_cells && !by_episode) ||
+    // (the smallest maps with rewards of all cells, 4 actions, epsilon by episode, 20 to 300 steps, rows so many times as fast as lane waves: 26 cells,
+    // 270,001 / 360,001 / 520,001 envs 0.98 to 1.06 / 1.09 to 1.17 / 1.3 and more; 27, 270,001 / 360,001 / 430,001 0.82 to 0.93 / 0.94 to 1.07 / 1.00 to
+    // 1.15; 28, 0.90 to 1.07 / 1.00 to 1.14 / 1.08 to 1.28; 30 cells 0.77 to 0.85 / 0.90 to 1.00, 390,001 0.92 to 1.06.)
+    const bool smallest = e->S <= kRowsRewardsSmallest ||
+                          (e->A == 4 && base_cells && (e->S <= kRowsRewardsSmaller || (e->S <= kRowsRewardsSmall && (long)e->N > kRowsRewardsSmallEnvs)));
+    const bool cells_long = smallest || (e->A == 4 && e->S >= kRowsRewardsLarge && rows_staged) || (base_cells && !by_episode) ||
                             kComputeUnits * lane_fit < per_round;  // (no even rounds)
     const int cells_steps = !by_episode || !rows_staged                     ? kLaneRoundsManyMinSteps - 1
                             : e->S >= kRowsRewardsLarge                     ? kRowsRewardsLargeSteps

@@ -336,10 +336,11 @@ def test_rows_or_plain_waves_with_cell_rewards(pycrl, N, W, H, A, n_steps, rows,
 @pytest.mark.parametrize("N,W,H,A,n_steps,rows,linear", [
     (300000, 4, 17, 4, 130, (4, 4), 0), (300000, 4, 17, 4, 131, (0, 4), 0), (300000, 4, 17, 4, 500, (0, 4), 0), (300000, 4, 17, 4, 501, (0, 0), 0),
     (300000, 9, 11, 4, 131, (0, 0), 1), (300000, 10, 10, 4, 200, (4, 4), 1), (300000, 10, 10, 4, 201, (0, 0), 1), (300000, 10, 10, 8, 131, (0, 0), 1),
-    (300000, 5, 5, 4, 500, (4, 4), 0), (300000, 5, 5, 8, 500, (4, 4), 1), (300000, 13, 2, 4, 131, (0, 0), 1),
+    (300000, 5, 5, 4, 500, (4, 4), 0), (300000, 5, 5, 8, 500, (4, 4), 1), (300000, 13, 2, 4, 131, (0, 4), 1), (300000, 13, 2, 8, 131, (0, 0), 1),
     (300000, 15, 17, 4, 131, (0, 4), 0), (300000, 16, 16, 4, 131, (4, 4), 0), (300000, 16, 16, 4, 500, (4, 4), 1), (300000, 16, 16, 4, 501, (0, 0), 1),
     (236650, 37, 30, 4, 130, (4, 4), 1), (236650, 37, 30, 4, 131, (0, 4), 0), (236650, 37, 30, 4, 131, (0, 0), 1),
     (300000, 16, 16, 8, 130, (4, 4), 0), (300000, 16, 16, 8, 131, (0, 4), 0), (300000, 16, 16, 8, 240, (4, 4), 1), (300000, 16, 16, 8, 241, (0, 0), 1),
+    (451269, 4, 7, 4, 283, (0, 4), 1), (519060, 2, 13, 4, 172, (0, 4), 1), (360448, 4, 7, 4, 283, (0, 0), 1),
 ])
 def test_rows_or_lane_waves_with_cell_rewards(pycrl, N, W, H, A, n_steps, rows, linear, flags):
     kw = dict(eps_mode=pycrl.EPS_EPISODE_LINEAR, eps0=1.0, eps_end=0.1, eps_span=10) if linear else dict()
