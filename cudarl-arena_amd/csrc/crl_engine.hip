@@ -753,7 +753,15 @@ FusedPlan plan_fused(const crl_engine* e, int n_steps) {
                           (e->A == 4 && base_cells && (e->S <= kRowsRewardsSmaller || (e->S <= kRowsRewardsSmall && (long)e->N > kRowsRewardsSmallEnvs)));
     const bool cells_long = smallest || (e->A == 4 && e->S >= kRowsRewardsLarge && rows_staged) || (base_cells && !by_episode) ||
                             kComputeUnits * lane_fit < per_round;  // (no even rounds)
-    const int cells_steps = !by_episode || !rows_staged                     ? kLaneRoundsManyMinSteps - 1
+    // (while the caches hold the tables lane waves take over from plain ones from 8 steps on, and are the faster ones then with 4 actions but on
+    // the smallest maps; lane waves / rows, launches of 262,144 envs and more: rewards of goals and traps, 270,845 of 5x9, epsilon by episode,
+    // 47 steps 217, 332; 274,286 of 5x9, 15 steps 78, 118; 298,062 of 2x20, by episode, 8 steps 50, 65; 422,354 of 3x9, 75 steps 425, 524;
+    // 371,959 of 2x13, 96 steps 458, 559; but 408,508 of 3x4, by episode, 60 steps 290, 222; rewards of all cells, by episode, 336,159 of 4x8, 28
+    // steps 152, 199; 274,212 of 6x7, 9 steps 53, 72; with epsilon fixed 281,012 of 6x6, 38 steps 149, 113; in calls that plain waves
+    // would take, 312,999 of 3x9, 2 steps 33.7, 30.6.)
+    const bool cells_cached = e->A == 4 && !outgrown && e->N >= kRowsManyEnvs && !smallest;
+    const int cells_steps = cells_cached                                    ? kLaneWavesMinSteps - 1
+                            : !by_episode || !rows_staged                   ? kLaneRoundsManyMinSteps - 1
                             : e->S >= kRowsRewardsLarge                     ? kRowsRewardsLargeSteps
                             : e->A == 4 && e->S >= kRowsRewardsMiddle       ? kRowsRewardsMiddleSteps
                                                                             : kLaneRoundsManyMinSteps - 1;

@@ -340,7 +340,10 @@ def test_rows_or_plain_waves_with_cell_rewards(pycrl, N, W, H, A, n_steps, rows,
     (300000, 15, 17, 4, 131, (0, 4), 0), (300000, 16, 16, 4, 131, (4, 4), 0), (300000, 16, 16, 4, 500, (4, 4), 1), (300000, 16, 16, 4, 501, (0, 0), 1),
     (236650, 37, 30, 4, 130, (4, 4), 1), (236650, 37, 30, 4, 131, (0, 4), 0), (236650, 37, 30, 4, 131, (0, 0), 1),
     (300000, 16, 16, 8, 130, (4, 4), 0), (300000, 16, 16, 8, 131, (0, 4), 0), (300000, 16, 16, 8, 240, (4, 4), 1), (300000, 16, 16, 8, 241, (0, 0), 1),
-    (451269, 4, 7, 4, 283, (0, 4), 1), (519060, 2, 13, 4, 172, (0, 4), 1), (360448, 4, 7, 4, 283, (0, 0), 1),
+    # tables that the caches hold: lane waves in shorter calls too (270,845 of 5x9 are 195 MB, 280,000 past the 192 MiB)
+    (270845, 5, 9, 4, 7, (4, 4), 1), (270845, 5, 9, 4, 8, (0, 0), 1), (270845, 5, 9, 4, 47, (0, 4), 0), (280000, 5, 9, 4, 47, (4, 4), 1),
+    (371959, 2, 13, 4, 96, (0, 4), 0), (382977, 2, 13, 4, 53, (0, 4), 1), (360448, 4, 7, 4, 65, (0, 0), 1), (360449, 4, 7, 4, 65, (0, 4), 1), (451269, 4, 7, 4, 283, (0, 4), 1), (519060, 2, 13, 4, 172, (0, 4), 1), (330000, 4, 8, 4, 28, (0, 0), 1),
+    (425835, 5, 5, 4, 40, (4, 4), 1), (262144, 4, 6, 8, 40, (4, 4), 1),
 ])
 def test_rows_or_lane_waves_with_cell_rewards(pycrl, N, W, H, A, n_steps, rows, linear, flags):
     kw = dict(eps_mode=pycrl.EPS_EPISODE_LINEAR, eps0=1.0, eps_end=0.1, eps_span=10) if linear else dict()
